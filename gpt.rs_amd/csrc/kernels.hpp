@@ -282,9 +282,9 @@ struct MfmaLinearArgs {
     // the k-grouped CODE copies (mfma_pack_codes) and scale / scale2 the matrices' scale tensors
     int quant;
     const void* scale; const void* scale2;
-    // tail split: when the last round of 128 x 128 tiles would leave most CUs idle, those tiles are split over k between
-    // 2 or 4 workgroups that meet through `part` (mfma_workspace_bytes() of scratch) and `tickets` (kSkinnyTickets
-    // counters, zero before and after every launch); without them every tile runs whole
+    // `part`: mfma_workspace_bytes() of scratch for the partial sums of tiles that are split over k; `tickets`
+    // (kSkinnyTickets counters, zero before and after every launch) is where the register-staged kernel's splits of a tile
+    // meet; without them every tile runs whole
     void* part = nullptr; size_t part_bytes = 0; unsigned* tickets = nullptr;
     int out_f32 = 0;   // bf16 only: y and residual are f32
     EpiExtra extra;    // unquantised only

@@ -504,27 +504,37 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
 
 // ---------------------------------------------------------------------------------------------------------------
 // bf16 GEMM whose tiles go memory -> LDS without passing through registers (global_load_lds_dwordx4), for unquantised
-// bf16 operands.  Against the kernel above: no staging registers and no LDS store instructions, a ring of NST staged
-// tiles (loads run NST - 1 tiles ahead), and tile shapes chosen per launch so that the tiles fill the 256 CUs in whole
-// rounds (128 x 192 and 128 x 96 as well as 128 x 128).
+// bf16 operands: no staging registers, no LDS store instructions, loads run NST - 1 k tiles ahead through a ring.
 //
-// Workgroup: KW groups of WM x WN waves.  A wave owns 64 x (32 TN) outputs as 2 x TN fragments of 32 x 32; the tile is
-// (64 WM) x (32 TN WN).  All groups share the staged tiles; group g multiplies k-steps [g KSW, (g + 1) KSW) of every
-// tile (KSW = 4 / KW k-steps of 16) and the groups' sums meet through LDS before the epilogue, so a launch of one tile
-// per CU still has 8 waves per CU.
+// Workgroup: WM x WN waves; a wave owns (32 TM) x (32 TN) outputs as TM x TN fragments of 32 x 32, the tile is
+// BM x BN = (32 TM WM) x (32 TN WN).  A launch takes one of six tiles and a number of splits over k, see tile_plan().
 //
-// LDS, per stage: A as rows of 128 bytes (64 k), B k-group-major ([k-group][column][8 k]).  One load instruction moves
+// What bounds it.  256 x 256 tiles, all CUs busy: the matrix pipes at the clock that random operands allow.  A tile's 32 k
+// take 0.54 us on a quarter of the CUs and 0.8 us on all of them; over all-zero operands the same launch runs at 1.35 times
+// the rate (M = 8188, K = 3072, N = 6144: 1680 against 1240 TFLOP/s), so it is power and not data that paces it.  Why 256 x
+// 256: a k tile moves 1 / (2 BM) + 1 / (2 BN) bytes per flop from the L2s into LDS and as many fragments from LDS into
+// registers, 5/6 of what 128 x 192 needs twice over; 8 waves of 128 x 64 read 6 fragments for 8 MFMAs (64 x 96: 5 for 6,
+// each k-group its own).  Against the 128 x 192 tiles (two k-groups of 2 x 2 waves) that ran here before, us in a traced
+// 26-layer prompt: M = 8188 qkv 340 -> 263, gate/up pair 1010 -> 771, out and down 337 (mean) -> 215 and 413; M = 333 (few tiles,
+// weights from memory) qkv 32 -> 28, out and down 51 (mean) -> 29 with the launch that adds the splits, pair 81 -> 49.  k tiles of 32 in a ring of four beat k tiles of 64 in
+// a ring of two there (1035 -> 1239 TFLOP/s: loads have three k tiles of time, not one); 4 waves of 128 x 128 lose (1090).
+// Smaller tiles are for launches whose 256 x 256 tiles would leave CUs without work; they stage 64 k, the memory's lines.
+//
+// LDS, per stage: A as rows of 2 BK bytes, B k-group-major ([k-group][column][8 k]).  One load instruction moves
 // 64 x 16 bytes to 1 KiB of consecutive LDS, lane l to byte 16 l, so the layout is fixed by WHICH 16 bytes of memory a
-// lane asks for: in A, position p of row r holds k-group p ^ ((r >> 1) & 7); eight lanes still read one row's 128
-// contiguous bytes, and a fragment read (32 rows x 2 k-groups) touches every bank once per 16 lanes.  B fragments are
-// contiguous as they are.
+// lane asks for: in A, position p of row r holds k-group p ^ swz(r), with swz(r) such that 16 consecutive rows of a
+// fragment read (32 rows x 2 k-groups) touch every bank once; BK / 8 lanes still read one row's 2 BK contiguous bytes.
+// B fragments are contiguous as they are.
 //
 // Order of issue, fixed by hand with scheduling barriers: the fragments of the next k-step are requested before the
 // MFMAs of this one; in a tile's last k-step half the MFMAs are issued, then the wave waits for its own loads of the
 // next tile (vmcnt, which counts only LDS-direct loads here), passes the barrier that makes that tile complete and this
 // one free, requests the next tile's first fragments, issues the other half and, behind it, requests the tile NST
-// ahead into the freed stage.  Loads past the last tile repeat it into a stage nobody reads, so the count the wait relies on never changes.
-// DUAL (SwiGLU pair): the tile's first BN / 2 columns are columns of W, the others the same columns of W2.
+// ahead into the freed stage.  Nothing is requested past the last tile; from there on the wave waits for everything.
+// MFMAs run at raised wave priority, so that the two waves of a SIMD take turns instead of stalling on each other's LDS
+// reads (k tiles of 64: 1035 -> 1167 TFLOP/s; of 32: within the noise).
+// DUAL (SwiGLU pair): the tile's first BN / 2 columns are columns of W, the others the same columns of W2, and a wave
+// multiplies the same 16 TN columns of both, so gate and up of an output meet in one lane.
 // One load instruction: lane l asks for the 16 bytes at base + offset(l) (a scalar base and a 32-bit offset per lane, so
 // stepping to the next k tile is scalar arithmetic; vector instructions in the step loop cost the matrix pipe issue
 // slots: per-lane 64-bit addresses were 5-10 % slower) and they land at LDS byte lds_addr + 16 l.
@@ -537,71 +547,138 @@ __device__ __forceinline__ unsigned long long gemm_uniform64(unsigned long long 
 }
 template <int N> __device__ __forceinline__ void gemm_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-template <int NST, int WM, int WN, int TN, int KW, bool DUAL>
-__global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wk,
-                                                                   const bf16_t* __restrict__ wk2, const bf16_t* __restrict__ bias,
-                                                                   const bf16_t* __restrict__ residual, bf16_t* __restrict__ y,
-                                                                   int M, int K, int N, int Npad, int act, int NT, int MT, int out_f32,
-                                                                   int splits, float* __restrict__ part, unsigned* __restrict__ tickets, EpiExtra extra) {
-    constexpr int BK = 64, KG = 8, ROWB = 128;
-    constexpr int BM = 64 * WM, BN = 32 * TN * WN, NW = WM * WN * KW;
+// What happens to a sum on its way out (a pair has been combined before).
+struct TileEpilogue {
+    const bf16_t* bias; const void* residual; void* y;
+    int64_t N;
+    int act, out_f32;
+    EpiExtra extra;
+};
+// Eight neighbours of row m, columns n .. n + 7, from LDS: bias, GELU, column factor and residual, then one 16-byte store (two
+// for f32 results; element by element when N is not a multiple of 8).  Kept short: with every output's options unrolled the
+// epilogue was 13 000 to 18 000 instructions, more than the instruction cache holds (M = 8188, see gemm_tile_kernel).
+__device__ __forceinline__ void gemm_finish8(const TileEpilogue& p, int64_t m, int64_t n, const float* at_lds) {
+    const int64_t at = m * p.N + n;
+    if ((p.N & 7) != 0) {
+#pragma unroll 1
+        for (int e = 0; e < 8; ++e) {
+            if (n + e >= p.N) break;
+            const float bv = p.bias ? bf16_to_f32(p.bias[n + e]) : 0.f;
+            const float rv = p.residual ? (p.out_f32 ? static_cast<const float*>(p.residual)[at + e] : bf16_to_f32(static_cast<const bf16_t*>(p.residual)[at + e])) : 0.f;
+            const float f = mfma_finish(at_lds[e], 0.f, false, p.act, bv, p.residual != nullptr, rv, p.extra.glu, p.extra.colscale ? p.extra.colscale[n + e] : 1.0f);
+            if (p.out_f32) static_cast<float*>(p.y)[at + e] = f;
+            else static_cast<bf16_t*>(p.y)[at + e] = f32_to_bf16(f);
+        }
+        return;
+    }
+    float o[8];
+    *reinterpret_cast<f32x4_t*>(o) = *reinterpret_cast<const f32x4_t*>(at_lds);
+    *reinterpret_cast<f32x4_t*>(o + 4) = *reinterpret_cast<const f32x4_t*>(at_lds + 4);
+    if (p.bias) {
+        const u32x4_t bw = *reinterpret_cast<const u32x4_t*>(p.bias + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[2 * e] += __uint_as_float(bw[e] << 16);            // tensor_ops.rs:42-56
+            o[2 * e + 1] += __uint_as_float(bw[e] & 0xFFFF0000u);
+        }
+    }
+    if (p.act == 1) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (o[e] * 0.5f) * (erff(o[e] / 1.41421354f) + 1.0f);   // activation.rs:96-113
+    }
+    if (p.extra.colscale) {
+        const f32x4_t c0 = *reinterpret_cast<const f32x4_t*>(p.extra.colscale + n), c1 = *reinterpret_cast<const f32x4_t*>(p.extra.colscale + n + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { o[e] *= c0[e]; o[4 + e] *= c1[e]; }
+    }
+    if (p.residual) {
+        if (p.out_f32) {
+            const f32x4_t r0 = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(p.residual) + at);
+            const f32x4_t r1 = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(p.residual) + at + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { o[e] += r0[e]; o[4 + e] += r1[e]; }
+        } else {
+            const u32x4_t rw = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(p.residual) + at);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o[2 * e] += __uint_as_float(rw[e] << 16);
+                o[2 * e + 1] += __uint_as_float(rw[e] & 0xFFFF0000u);
+            }
+        }
+    }
+    if (p.out_f32) {
+        *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.y) + at) = *reinterpret_cast<const f32x4_t*>(o);
+        *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.y) + at + 4) = *reinterpret_cast<const f32x4_t*>(o + 4);
+    } else {
+        u32x4_t w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = mfma_pack_bf16(o[2 * e], o[2 * e + 1]);
+        *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(p.y) + at) = w;
+    }
+}
+// The pair's gate on the hardware's exp2 and reciprocal (1 ulp each of f32; the result goes on as bf16): the exact division
+// and expf of glu_combine are 40 instructions an output, 9 us of a 256 x 256 tile's 85.
+__device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) {
+    const float alpha = p.kind == 1 ? p.alpha : 1.0f;
+    if (p.kind == 1) {
+        g = fminf(g, p.limit);
+        u = fminf(fmaxf(u, -p.limit), p.limit) + p.shift;
+    }
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.44269504f * alpha))) * u;
+}
+
+template <int BK, int NST, int WM, int WN, int TM, int TN, bool DUAL>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wk, const bf16_t* __restrict__ wk2,
+                                                                 int M, int K, int Npad, int NT, int MT, int splits, float* __restrict__ part, TileEpilogue epi) {
+    static_assert(BK == 32 || BK == 64, "k tile");
+    constexpr int KG = BK / 8, ROWB = BK * 2, KS = BK / 16;            // k-groups, bytes of an A row, k-steps
+    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NW = WM * WN;
     constexpr int NREAL = DUAL ? BN / 2 : BN;                          // output columns per tile
+    constexpr int TNO = DUAL ? TN / 2 : TN;                            // output fragments per wave and row
     constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, STAGE = A_BYTES + B_BYTES;
     constexpr int LAI = A_BYTES / 1024, LBI = B_BYTES / 1024;          // load instructions per tile
-    constexpr int LA = (LAI + NW - 1) / NW, LB = (LBI + NW - 1) / NW;  // per wave (a wave past the end repeats an earlier one)
-    constexpr int LPT = LA + LB;
-    constexpr int KSW = 4 / KW;
-    static_assert(KSW == 2 || KSW == 4, "an even number of k-steps per wave and tile: the last one's fragments sit in slot 1");
-    static_assert(!DUAL || WN == 2, "pair tiles: wave column 0 multiplies W, wave column 1 the same columns of W2");
+    constexpr int LA = LAI / NW, LB = LBI / NW, LPT = LA + LB;         // per wave
+    static_assert(LA * NW == LAI && LB * NW == LBI, "whole load instructions per wave");
+    static_assert(KS % 2 == 0, "the last k-step's fragments sit in slot 1, the next tile's first in slot 0");
+    static_assert(!DUAL || (TN % 2 == 0 && BN % 128 == 0), "a load instruction's 64 columns belong to one matrix of the pair");
     static_assert((NST - 2) * LPT < 64, "vmcnt is a 6-bit counter");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wg = wave / (WM * WN), wq = wave % (WM * WN);
-    const int wm = wq / WN, wn = wq % WN;
-    int bx, by, tile, sidx;
+    const int wm = wave / WN, wn = wave % WN;
+    int bx, by, sidx;
     {
-        // XCD c takes a contiguous range of a grouped tile order (see gemm_mfma_kernel)
-        // splits > 1: `splits` neighbours of that order share a tile and take a contiguous range of its k tiles each
+        // XCD c takes a contiguous range of a grouped tile order (see gemm_mfma_kernel: 8 row blocks by 4 column tiles run on
+        // an XCD at a time; groups of 4 or 32 row blocks are 3-10 % slower at M = 8188); `splits` neighbours of that order
+        // share a tile and take a contiguous range of its k tiles each
         const int total = NT * MT * splits, per = (total + 7) / 8;
         const int u = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
         if (u >= total) return;
-        tile = u / splits;
+        const int v = u / splits;
         sidx = u % splits;
-        const int v = tile;
         const int gsz = 8 * NT, g = v / gsz, first = g * 8;
         const int gm = MT - first < 8 ? MT - first : 8;
         by = first + (v % gsz) % gm;
         bx = (v % gsz) / gm;
     }
     const int m0 = by * BM, n0 = bx * NREAL;
-    // what each of this wave's load instructions fetches (per lane) and where its KiB goes
+    auto swz = [](int row) { return BK == 64 ? (row >> 1) & 7 : (row >> 2) & 3; };
+    // what each of this wave's load instructions fetches, per lane
     unsigned a_off[LA], b_off[LB];
-    unsigned a_dst[LA], b_dst[LB];
+    unsigned long long b_base[LB];
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
-        const int q = (wave * LA + j) % LAI;
-        const int sl = q * 64 + lane, row = sl / KG, pos = sl % KG;
+        const int sl = (wave * LA + j) * 64 + lane, row = sl / KG, pos = sl % KG;
         int m = m0 + row;
         if (m > M - 1) m = M - 1;
-        a_off[j] = (unsigned)((m - m0) * K * 2 + ((pos ^ ((row >> 1) & 7)) * 16));   // under 128 rows of K bf16: fits 32 bits (K < 2^23)
-        a_dst[j] = q * 1024;
+        a_off[j] = (unsigned)((m - m0) * K * 2 + ((pos ^ swz(row)) * 16));   // under 256 rows of K bf16: fits 32 bits (K <= 2^22)
     }
-    // DUAL: both matrices are addressed from the lower of the two pointers (the launcher has checked that the other
-    // lies less than 2^32 bytes above it, a k tile included)
-    const unsigned long long w_lo = DUAL && (unsigned long long)wk2 < (unsigned long long)wk ? (unsigned long long)wk2 : (unsigned long long)wk;
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
-        const int q = (wave * LB + j) % LBI;
-        const int sl = q * 64 + lane, kg = sl / BN, bc = sl % BN;
-        int col = n0 + bc;
-        unsigned long long src = (unsigned long long)wk;
-        if (DUAL) {
-            col = n0 + bc % NREAL;
-            src = bc >= NREAL ? (unsigned long long)wk2 : (unsigned long long)wk;
-        }
+        const int q = wave * LB + j, kg = q * 64 / BN, bc = q * 64 % BN;
+        int col = n0 + (DUAL ? bc % NREAL : bc) + lane;
         if (col > Npad - 1) col = Npad - 1;
-        b_off[j] = (unsigned)(src - w_lo) + (unsigned)(((unsigned long long)kg * Npad + col) * 16);
-        b_dst[j] = A_BYTES + q * 1024;
+        b_base[j] = (unsigned long long)(DUAL && bc >= NREAL ? wk2 : wk);
+        b_off[j] = (unsigned)(((unsigned long long)kg * Npad + col) * 16);
     }
     const unsigned long long a_base = (unsigned long long)(x + (int64_t)m0 * K);
     const int64_t b_tile_step = (int64_t)KG * Npad * 16;
@@ -609,282 +686,231 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(const bf16_
     const int kt_all = K / BK, kt0 = (int)((int64_t)sidx * kt_all / splits);
     const int nt = (int)((int64_t)(sidx + 1) * kt_all / splits) - kt0;   // this workgroup's k tiles: [kt0, kt0 + nt)
     auto issue = [&](int t, int st) {
-        if (t > nt - 1) t = nt - 1;
-        t += kt0;
-        const unsigned long long ab = gemm_uniform64(a_base + (unsigned long long)t * (BK * 2));
-        const unsigned long long bb = gemm_uniform64(w_lo + (unsigned long long)(t * b_tile_step));
+        if (t >= nt) return;
+        const unsigned long long ab = gemm_uniform64(a_base + (unsigned long long)(t + kt0) * (BK * 2));
+        const unsigned long long bt = (unsigned long long)((t + kt0) * b_tile_step);
         const unsigned sbase = lds0 + st * STAGE;
 #pragma unroll
-        for (int j = 0; j < LA; ++j) gemm_lds_load16(a_off[j], ab, (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + a_dst[j])));
+        for (int j = 0; j < LA; ++j) gemm_lds_load16(a_off[j], ab, (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + (wave * LA + j) * 1024)));
 #pragma unroll
-        for (int j = 0; j < LB; ++j) gemm_lds_load16(b_off[j], bb, (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + b_dst[j])));
+        for (int j = 0; j < LB; ++j) gemm_lds_load16(b_off[j], gemm_uniform64(b_base[j] + bt), (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + A_BYTES + (wave * LB + j) * 1024)));
     };
-    f32x16_t acc[2][TN];
+    f32x16_t acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
     const int fsel = lane >> 5;
-    const int b_rd = A_BYTES + (wn * 32 * TN + (lane & 31)) * 16;
-    bf16x8_t af[2][2], bfr[2][TN];
+    const int b_rd = A_BYTES + (wn * 32 * TNO + (lane & 31)) * 16;
+    bf16x8_t af[2][TM], bfr[2][TN];
     auto fread = [&](int st, int kk, int slot) {   // kk: k-step of the tile
         const unsigned char* base = lds + st * STAGE;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int row = wm * 64 + i * 32 + (lane & 31), kg = 2 * kk + fsel;
-            af[slot][i] = *reinterpret_cast<const bf16x8_t*>(base + row * ROWB + ((kg ^ ((row >> 1) & 7)) * 16));
+        for (int i = 0; i < TM; ++i) {
+            const int row = wm * 32 * TM + i * 32 + (lane & 31), kg = 2 * kk + fsel;
+            af[slot][i] = *reinterpret_cast<const bf16x8_t*>(base + row * ROWB + ((kg ^ swz(row)) * 16));
         }
 #pragma unroll
-        for (int j = 0; j < TN; ++j) bfr[slot][j] = *reinterpret_cast<const bf16x8_t*>(base + b_rd + (2 * kk + fsel) * (BN * 16) + j * 512);
+        for (int j = 0; j < TN; ++j)
+            bfr[slot][j] = *reinterpret_cast<const bf16x8_t*>(base + b_rd + (2 * kk + fsel) * (BN * 16) + (DUAL ? (j / TNO) * (NREAL * 16) : 0) + (j % TNO) * 512);
     };
     for (int st = 0; st < NST - 1; ++st) issue(st, st);
-    gemm_wait_loads<(NST - 2) * LPT>();
+    if (nt >= NST - 1) gemm_wait_loads<(NST - 2) * LPT>();
+    else gemm_wait_loads<0>();
     __syncthreads();
     issue(NST - 1, NST - 1);
-    fread(0, wg * KSW, 0);
+    fread(0, 0, 0);
     // One k tile; the ring position is a compile-time constant (the tile loop below is unrolled over the ring), so every
-    // LDS address of the step loop is a register plus an immediate: with the position in a register the six address
-    // additions per tile cost 3 % on the 8-wave tiles and 8-10 % on the 4-wave ones.
+    // LDS address of the step loop is a register plus an immediate.
     auto tile_step = [&](auto ring_pos, int t) {
         constexpr int ST = decltype(ring_pos)::value, ST1 = ST + 1 == NST ? 0 : ST + 1;
-#pragma unroll
-        for (int kk = 0; kk < KSW; ++kk) {
-            if (kk + 1 < KSW) fread(ST, wg * KSW + kk + 1, (kk + 1) & 1);
+        auto mul = [&](int slot, int i0, int i1) {
             __builtin_amdgcn_sched_barrier(0);
-            if (kk + 1 < KSW) {
+            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk & 1][i], bfr[kk & 1][j], acc[i][j], 0, 0, 0);
-            } else {
-#pragma unroll
-                for (int j = 0; j < TN; ++j) acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk & 1][0], bfr[kk & 1][j], acc[0][j], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                gemm_wait_loads<(NST - 2) * LPT>();
-                __syncthreads();
-                fread(ST1, wg * KSW, 0);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) acc[1][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk & 1][1], bfr[kk & 1][j], acc[1][j], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                issue(t + NST, ST);   // behind the MFMAs: the address arithmetic and the requests run under them (6 % faster than ahead of them)
-            }
+                for (int j = 0; j < TN; ++j)
+                    if (i * TN + j >= i0 && i * TN + j < i1) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[slot][i], bfr[slot][j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int kk = 0; kk + 1 < KS; ++kk) {
+            fread(ST, kk + 1, (kk + 1) & 1);
+            mul(kk & 1, 0, TM * TN);
         }
+        mul(1, 0, TM * TN / 2);
+        if (t + NST - 1 < nt) gemm_wait_loads<(NST - 2) * LPT>();   // the loads of tiles t + 2 .. t + NST - 1 may be on their way
+        else gemm_wait_loads<0>();
+        __syncthreads();
+        fread(ST1, 0, 0);
+        mul(1, TM * TN / 2, TM * TN);
+        issue(t + NST, ST);   // behind the MFMAs: the address arithmetic and the requests run under them (6 % faster than ahead of them)
+        __builtin_amdgcn_sched_barrier(0);
     };
-    static_assert(NST == 3, "the tile loop is unrolled over a ring of three");
+    static_assert(NST >= 2 && NST <= 4, "the tile loop is unrolled over the ring");
     {
+        constexpr std::integral_constant<int, 0> R0{};
+        constexpr std::integral_constant<int, 1> R1{};
+        constexpr std::integral_constant<int, NST == 2 ? 0 : 2> R2{};
+        constexpr std::integral_constant<int, NST - 1> R3{};
         int t = 0;
-        for (; t + 3 <= nt; t += 3) {
-            tile_step(std::integral_constant<int, 0>{}, t);
-            tile_step(std::integral_constant<int, 1>{}, t + 1);
-            tile_step(std::integral_constant<int, 2>{}, t + 2);
+        for (; t + NST <= nt; t += NST) {
+            tile_step(R0, t);
+            tile_step(R1, t + 1);
+            if constexpr (NST > 2) tile_step(R2, t + 2);
+            if constexpr (NST > 3) tile_step(R3, t + 3);
         }
-        if (t < nt) tile_step(std::integral_constant<int, 0>{}, t);
-        if (t + 1 < nt) tile_step(std::integral_constant<int, 1>{}, t + 1);
+        if (t < nt) tile_step(R0, t);
+        if constexpr (NST > 2)
+            if (t + 1 < nt) tile_step(R1, t + 1);
+        if constexpr (NST > 3)
+            if (t + 2 < nt) tile_step(R2, t + 2);
     }
-    gemm_wait_loads<0>();   // the repeated loads of the last tile have landed before LDS is used for anything else
-    // The two k-groups swap halves through LDS (the staged tiles are dead behind the barrier): group g gives the sums of
-    // fragment row 1 - g and keeps row g, so all 8 waves take part in the epilogue, 32 rows each.
-    static_assert(KW == 2, "two k-groups");
-    f32x16_t mine[TN];
-    {
-        float* give = reinterpret_cast<float*>(lds) + (wg * (WM * WN) + wq) * (TN * 16 * 64) + lane;
-        const float* take = reinterpret_cast<const float*>(lds) + ((1 - wg) * (WM * WN) + wq) * (TN * 16 * 64) + lane;
-        __syncthreads();
-        if (wg == 0) {
+    if (splits > 1) {
+        // partial sums, [split][row][columns padded to 8] f32 (a pair: W's columns, then W2's); gemm_reduce_kernel adds them
+        const int np = ((int)epi.N + 7) & ~7, width = DUAL ? 2 * np : np;
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) give[(j * 16 + v) * 64] = acc[1][j][v];
-        } else {
+            for (int j = 0; j < TN; ++j) {
+                const int n = n0 + (wn * TNO + j % TNO) * 32 + (lane & 31);
+                if (n >= np) continue;
+                float* to = part + (int64_t)sidx * M * width + (DUAL ? (j / TNO) * np : 0) + n;
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) give[(j * 16 + v) * 64] = acc[0][j][v];
-        }
-        __syncthreads();
-        if (wg == 0) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) mine[j][v] = acc[0][j][v] + take[(j * 16 + v) * 64];
-        } else {
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) mine[j][v] = acc[1][j][v] + take[(j * 16 + v) * 64];
-        }
-        __syncthreads();   // every wave has taken its half before the area is written again
-    }
-    if (!DUAL && splits > 1) {
-        // Split over k: the workgroups of a tile leave their sums in the workspace, [tile][split][wave][value][lane],
-        // through device-scope stores (coherent across the XCDs' L2s without cache maintenance); once they are
-        // acknowledged the workgroup draws the tile's ticket.  The one that draws the last ticket adds all partial sums
-        // in split order, its own included, so the result does not depend on which workgroup that is, leaves the ticket
-        // at zero and runs the epilogue.
-        float* mine_at = part + ((int64_t)(tile * splits + sidx) * NW + wave) * (TN * 16 * 64) + lane;
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) __hip_atomic_store(mine_at + (j * 16 + v) * 64, mine[j][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0)
-        asm volatile("" ::: "memory");
-        unsigned* flag = reinterpret_cast<unsigned*>(lds);
-        __syncthreads();
-        if (tid == 0) *flag = __hip_atomic_fetch_add(&tickets[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        const unsigned drawn = *flag;
-        __syncthreads();                                            // the flag has been read before its bytes are used again
-        if (drawn != (unsigned)(splits - 1)) return;
-        asm volatile("" ::: "memory");                              // the partial sums are read after the ticket is known
-        if (tid == 0) __hip_atomic_store(&tickets[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) mine[j][v] = 0.f;
-        for (int q = 0; q < splits; ++q) {
-            const float* src = part + ((int64_t)(tile * splits + q) * NW + wave) * (TN * 16 * 64) + lane;
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) mine[j][v] += __hip_atomic_load(src + (j * 16 + v) * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    // Rows of 8 outputs: a wave's 32 x (32 TN) sums go through an LDS area of its own (a lane holds one column of
-    // four-row groups, memory wants runs along a row); then bias, GELU and the residual are applied to 8 neighbours at a
-    // time and leave in one 16-byte store (two for f32 results; element by element when N is not a multiple of 8).
-    // DUAL: the wave columns are the two matrices (wn = 0: x.W, wn = 1: x.W2, same output columns), so the pair of
-    // waves meets here: each takes half of the pair's chunks and reads both areas.
-    constexpr int RSF = 32 * TN + 4;     // floats per row of an area
-    constexpr int CH = 32 * TN / 8;      // chunks of 8 per row
-    constexpr int PASSES = 32 * CH / 64 / (DUAL ? 2 : 1);
-    static_assert((32 * CH) % (DUAL ? 128 : 64) == 0, "whole passes of the wave");
-    {
-        float* tr = reinterpret_cast<float*>(lds) + wave * (32 * RSF);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) tr[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * RSF + j * 32 + (lane & 31)] = mine[j][v];
-    }
-    if (DUAL) __syncthreads();
-    const float* area = reinterpret_cast<const float*>(lds) + (DUAL ? wave - wn : wave) * (32 * RSF);
-    const int mrow0 = m0 + wm * 64 + wg * 32, ncol0 = DUAL ? n0 : n0 + wn * 32 * TN;
-    const bool vec = (N & 7) == 0;
-#pragma unroll
-    for (int it = 0; it < PASSES; ++it) {
-        const int c = (DUAL ? wn * PASSES + it : it) * 64 + lane, r = c / CH, cc = c % CH;
-        const int m = mrow0 + r, n = ncol0 + cc * 8;
-        if (m >= M || n >= N) continue;
-        float o[8];
-        *reinterpret_cast<f32x4_t*>(o) = *reinterpret_cast<const f32x4_t*>(area + r * RSF + cc * 8);
-        *reinterpret_cast<f32x4_t*>(o + 4) = *reinterpret_cast<const f32x4_t*>(area + r * RSF + cc * 8 + 4);
-        if (DUAL) {
-            float u[8];
-            *reinterpret_cast<f32x4_t*>(u) = *reinterpret_cast<const f32x4_t*>(area + 32 * RSF + r * RSF + cc * 8);
-            *reinterpret_cast<f32x4_t*>(u + 4) = *reinterpret_cast<const f32x4_t*>(area + 32 * RSF + r * RSF + cc * 8 + 4);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = glu_combine(o[e], u[e], extra.glu.kind, extra.glu.limit, extra.glu.alpha, extra.glu.shift);   // activation.rs:141-162
-        }
-        const int64_t at = (int64_t)m * N + n;
-        if (vec) {
-            if (bias) {
-                const u32x4_t bw = *reinterpret_cast<const u32x4_t*>(bias + n);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    o[2 * e] += __uint_as_float(bw[e] << 16);            // tensor_ops.rs:42-56
-                    o[2 * e + 1] += __uint_as_float(bw[e] & 0xFFFF0000u);
+                for (int v = 0; v < 16; ++v) {
+                    const int m = m0 + (wm * TM + i) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                    if (m < M) to[(int64_t)m * width] = acc[i][j][v];
                 }
             }
-            if (act == 1) {
+        return;
+    }
+    // Rows of 8 outputs: 32 x (32 TNO) sums at a time go through an LDS area of the wave's own (a lane holds one column of
+    // four-row groups, memory wants runs along a row).  The staged tiles are dead: nothing is in flight, and every wave has
+    // read its last fragments in front of the last step's barrier.
+    constexpr int RSF = 32 * TNO + 4;    // floats per row of an area
+    constexpr int CH = 4 * TNO;          // chunks of 8 per row
+    float* area = reinterpret_cast<float*>(lds) + wave * (32 * RSF);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o[e] = (o[e] * 0.5f) * (erff(o[e] / 1.41421354f) + 1.0f);   // activation.rs:96-113
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TNO; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                float o = acc[i][j][v];
+                if (DUAL) o = gemm_glu(o, acc[i][DUAL ? j + TNO : j][v], epi.extra.glu);   // activation.rs:141-162
+                area[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * RSF + j * 32 + (lane & 31)] = o;
             }
-            if (extra.colscale) {
-                const f32x4_t c0 = *reinterpret_cast<const f32x4_t*>(extra.colscale + n), c1 = *reinterpret_cast<const f32x4_t*>(extra.colscale + n + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { o[e] *= c0[e]; o[4 + e] *= c1[e]; }
-            }
-            if (residual) {
-                if (out_f32) {
-                    const f32x4_t r0 = *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(residual) + at);
-                    const f32x4_t r1 = *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(residual) + at + 4);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) { o[e] += r0[e]; o[4 + e] += r1[e]; }
-                } else {
-                    const u32x4_t rw = *reinterpret_cast<const u32x4_t*>(residual + at);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        o[2 * e] += __uint_as_float(rw[e] << 16);
-                        o[2 * e + 1] += __uint_as_float(rw[e] & 0xFFFF0000u);
-                    }
-                }
-            }
-            if (out_f32) {
-                *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(y) + at) = *reinterpret_cast<const f32x4_t*>(o);
-                *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(y) + at + 4) = *reinterpret_cast<const f32x4_t*>(o + 4);
-            } else {
-                u32x4_t w;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = (uint32_t)f32_to_bf16(o[2 * e]) | ((uint32_t)f32_to_bf16(o[2 * e + 1]) << 16);
-                *reinterpret_cast<u32x4_t*>(y + at) = w;
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (n + e >= N) break;
-                const float bv = bias ? bf16_to_f32(bias[n + e]) : 0.f;
-                const float rv = residual ? (out_f32 ? reinterpret_cast<const float*>(residual)[at + e] : bf16_to_f32(residual[at + e])) : 0.f;
-                const float f = mfma_finish(o[e], 0.f, false, act, bv, residual != nullptr, rv, extra.glu, extra.colscale ? extra.colscale[n + e] : 1.0f);
-                if (out_f32) reinterpret_cast<float*>(y)[at + e] = f;
-                else y[at + e] = f32_to_bf16(f);
-            }
+#pragma unroll 1
+        for (int it = 0; it < CH / 2; ++it) {
+            const int c = it * 64 + lane, r = c / CH, cc = c % CH;
+            const int m = m0 + (wm * TM + i) * 32 + r, n = n0 + wn * 32 * TNO + cc * 8;
+            if (m < M && n < epi.N) gemm_finish8(epi, m, n, area + r * RSF + cc * 8);
         }
     }
 }
 
-template <int NST, int WM, int WN, int TN, int KW, bool DUAL>
-static void launch_dma(hipStream_t s, const MfmaLinearArgs& a, int splits = 1) {
-    constexpr int BM = 64 * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
-    constexpr int stage = (BM + BN) * 128, xch = WM * WN * KW * TN * 16 * 64 * 4, rows = WM * WN * KW * 32 * (32 * TN + 4) * 4;
-    constexpr int lds_bytes = NST * stage > (xch > rows ? xch : rows) ? NST * stage : (xch > rows ? xch : rows);
+// Adds the partial sums of a launch whose tiles were split over k, in split order (the result does not depend on which
+// workgroup ended first), and finishes the outputs.  One thread per 8 outputs.  A launch of its own over the whole chip:
+// with the last workgroup of a tile adding them, 48 tiles of M = 333 kept 48 CUs busy reading while 208 waited.
+template <bool DUAL>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int M, int splits, TileEpilogue epi) {
+    const int np = ((int)epi.N + 7) & ~7, chunks = np / 8, width = DUAL ? 2 * np : np;
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (id >= (int64_t)M * chunks) return;
+    const int64_t m = id / chunks;
+    const int n = (int)(id % chunks) * 8;
+    auto sum8 = [&](const float* p, float* o) {
+        f32x4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
+        for (int s = 0; s < splits; ++s, p += (int64_t)M * width) {
+            a += *reinterpret_cast<const f32x4_t*>(p);
+            b += *reinterpret_cast<const f32x4_t*>(p + 4);
+        }
+        *reinterpret_cast<f32x4_t*>(o) = a;
+        *reinterpret_cast<f32x4_t*>(o + 4) = b;
+    };
+    __shared__ __attribute__((aligned(16))) float rows[256][12];   // finish8 reads its eight from LDS; each thread its own
+    float* o = rows[threadIdx.x];
+    sum8(part + m * width + n, o);
+    if (DUAL) {
+        float u[8];
+        sum8(part + m * width + np + n, u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = gemm_glu(o[e], u[e], epi.extra.glu);   // activation.rs:141-162
+    }
+    gemm_finish8(epi, m, n, o);
+}
+
+// The tiles, in the order of tile_cost's table.
+enum TileId { kT256x256, kT256x192, kT128x256, kT128x128, kT64x256, kT64x128, kTiles };
+struct TilePlan { int tile; int splits; };
+
+template <int BK, int NST, int WM, int WN, int TM, int TN, bool DUAL>
+static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
+    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
+    constexpr int ring = NST * (BM + BN) * BK * 2, rows = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4;
+    constexpr int lds_bytes = ring > rows ? ring : rows;
     static_assert(lds_bytes <= 160 * 1024, "LDS of one CU");
-    auto kern = gemm_dma_kernel<NST, WM, WN, TN, KW, DUAL>;
-    static bool configured = false;
+    auto kern = gemm_tile_kernel<BK, NST, WM, WN, TM, TN, DUAL>;
+    static bool configured = false;  // the attribute is per function, not per stream or device state
     if (!configured) {
         (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         configured = true;
     }
     const int64_t nt = cdiv(a.n, NREAL), mt = cdiv(a.m, BM);
-    if (splits > 1 && (DUAL || !a.part || !a.tickets || nt * mt > (int64_t)kSkinnyTickets ||
-                       a.part_bytes < (size_t)(nt * mt) * splits * BM * BN * sizeof(float)))
-        splits = 1;
-    const unsigned grid = (unsigned)(cdiv(nt * mt * splits, 8) * 8);
-    kern<<<grid, 64 * WM * WN * KW, lds_bytes, s>>>((const bf16_t*)a.x, (const bf16_t*)a.wk, (const bf16_t*)a.wk2, (const bf16_t*)a.bias,
-                                                   (const bf16_t*)a.residual, (bf16_t*)a.y, (int)a.m, (int)a.k, (int)a.n,
-                                                   (int)mfma_padded_n(a.n), a.act, (int)nt, (int)mt, a.out_f32, splits, (float*)a.part,
-                                                   a.tickets, a.extra);
+    TileEpilogue epi{(const bf16_t*)a.bias, a.residual, a.y, a.n, a.act, a.out_f32, a.extra};
+    kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN, lds_bytes, s>>>((const bf16_t*)a.x, (const bf16_t*)a.wk, (const bf16_t*)a.wk2, (int)a.m, (int)a.k,
+                                                                                   (int)mfma_padded_n(a.n), (int)nt, (int)mt, splits, (float*)a.part, epi);
+    if (splits > 1) gemm_reduce_kernel<DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
+}
+static size_t tile_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
+    return splits > 1 ? (size_t)splits * m * cdiv(n, 8) * 8 * (dual ? 2 : 1) * sizeof(float) : 0;
 }
 
-// Which tiles an unquantised bf16 launch of the LDS-direct kernel takes: 128 x 192 (`wide`), 128 x 96, or 128 x 192 with
-// every tile split two ways over k.  Estimated from what the kernels measure at M = 1024 (us): a round of wide tiles
-// 8 + 0.72 per k tile, of narrow ones 7 + 0.45 (28 KB per k tile against 40 KB, for half the flops), of split wide ones
-// 15 + 0.36 (half the k tiles; 7 us for 25 MB of partial sums out and in again).  N = 6144: 256 wide tiles; N = 3072:
-// 256 narrow tiles at K = 4096 (36.7 us; split 38.5), 128 wide tiles split in two at K = 9216 (66.7 us; narrow 72.8);
-// the 9216-wide pair: 768 tiles of 128 x 96 outputs.
-struct DmaPlan { bool wide; int splits; };
-static DmaPlan dma_plan(int64_t m, int64_t k, int64_t n) {
-    const int64_t mt = cdiv(m, 128), kt = k / 64;
-    const int64_t tw = mt * cdiv(n, 192), tn = mt * cdiv(n, 96);
-    const double wide = (double)cdiv(tw, 256) * (8.0 + 0.72 * kt);
-    const double narrow = (double)cdiv(tn, 256) * (7.0 + 0.45 * kt);
+// Which tile a launch takes, and over how many workgroups a tile's k is split.  Estimated time in us of every choice, from a
+// linear fit (within 6 % rms) to measurements at M = 40 .. 1500 of the 3072-wide layers (K = 3072, 4096, 9216; N = 3072, 6144,
+// a pair of 9216; weights from memory): rounds of workgroups x (fixed + per k tile of 64) + what a k tile costs more with the
+// chip full, and for a split the second launch plus its bytes.  What it picks is 1 % slower than the best measured choice,
+// over all of those shapes.
+struct TileCost { int bm, bn, slots; double fixed, per_kt, full_kt, split, split_mb; };
+static const TileCost kTileCost[kTiles] = {
+    {256, 256, 256, 5.45, 1.237, 0.379, 2.8, 0.30}, {256, 192, 256, 1.16, 1.206, 0.122, 4.7, 0.35}, {128, 256, 256, 6.87, 0.661, 0.171, 3.1, 0.26},
+    {128, 128, 256, 4.48, 0.425, 0.055, 3.9, 0.31}, {64, 256, 256, 4.59, 0.572, 0.0, 5.4, 0.13}, {64, 128, 512, 2.58, 0.361, 0.143, 5.0, 0.34},
+};
+static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual) {
     static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
-    const bool can_split = allow_split && kt >= 32 && tw <= (int64_t)kSkinnyTickets;
-    const double split = can_split ? (double)cdiv(2 * tw, 256) * (15.0 + 0.36 * kt) : 1e30;
-    if (split < wide && split < narrow) return {true, 2};
-    return {wide <= narrow, 1};
+    TilePlan best{kT256x256, 1};
+    double least = 1e300;
+    for (int t = 0; t < kTiles; ++t) {
+        const TileCost& c = kTileCost[t];
+        if (dual && c.bn == 192) continue;   // a pair's tile holds whole 64-column loads of either matrix
+        const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
+        for (int sp : {1, 2, 3, 4, 6, 8}) {
+            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > (64u << 20))) break;
+            const double kt = (double)k / 64 / sp, wg = (double)(tiles * sp);
+            double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
+            if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
+            if (us < least) { least = us; best = {t, sp}; }
+        }
+    }
+    return best;
+}
+template <bool DUAL>
+static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p) {
+    if (p.splits > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, DUAL, p.splits))) p.splits = 1;
+    switch (p.tile) {
+        case kT256x256: return launch_tile<32, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits);
+        case kT256x192: if constexpr (!DUAL) return launch_tile<64, 2, 4, 2, 2, 3, false>(s, a, p.splits); else return;
+        case kT128x256: return launch_tile<64, 3, 2, 4, 2, 2, DUAL>(s, a, p.splits);
+        case kT128x128:
+            if constexpr (DUAL) return launch_tile<64, 4, 4, 2, 1, 2, true>(s, a, p.splits);
+            else return launch_tile<64, 4, 2, 4, 2, 1, false>(s, a, p.splits);
+        case kT64x256: return launch_tile<64, 3, 2, 4, 1, 2, DUAL>(s, a, p.splits);
+        default: return launch_tile<64, 3, 2, 2, 1, 2, DUAL>(s, a, p.splits);
+    }
 }
 
 bool mfma_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n, int quant) {
@@ -921,20 +947,19 @@ static int mfma_few_tiles_split(int64_t tiles64, int64_t k_tiles) {
 }
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant) {
     if (!mfma_gemm_supported(dtype, m, k, n, quant)) return 0;
-    const int64_t tiles = cdiv(m, 128) * cdiv(mfma_padded_n(n), dual ? 64 : 128);
     const int64_t k_tiles = k / (kKb * kpc_of(dtype));
+    int sp = 1;
+    size_t bytes = 0;
     if (!dual && cdiv(m, 128) * cdiv(n, 128) < 128) {   // the 64 x 64 kernel runs (see mfma_gemm)
         const int64_t t64 = cdiv(m, 64) * cdiv(mfma_padded_n(n), 64);
-        const int sp = mfma_few_tiles_split(t64, k_tiles);
-        return sp > 1 ? (size_t)t64 * sp * 64 * 64 * sizeof(float) : 0;
+        sp = mfma_few_tiles_split(t64, k_tiles);
+        if (sp > 1) bytes = (size_t)t64 * sp * 64 * 64 * sizeof(float);
+    } else {
+        const int64_t tiles = cdiv(m, 128) * cdiv(mfma_padded_n(n), dual ? 64 : 128);
+        const int64_t full = mfma_tail_plan(tiles, k_tiles, &sp);
+        if (sp > 1) bytes = (size_t)(tiles - full) * sp * 128 * 128 * sizeof(float);
     }
-    int sp = 1;
-    const int64_t full = mfma_tail_plan(tiles, k_tiles, &sp);
-    size_t bytes = sp > 1 ? (size_t)(tiles - full) * sp * 128 * 128 * sizeof(float) : 0;
-    if (dtype == 2 && quant == 0 && !dual) {   // the LDS-direct kernel may split its 128 x 192 tiles over k
-        const DmaPlan p = dma_plan(m, k, n);
-        if (p.wide && p.splits > 1) bytes = std::max(bytes, (size_t)(cdiv(m, 128) * cdiv(n, 192)) * p.splits * 128 * 192 * sizeof(float));
-    }
+    if (dtype == 2 && quant == 0) bytes = std::max(bytes, tile_part_bytes(m, n, dual, tile_plan(m, k, n, dual).splits));   // the LDS-direct kernel
     return bytes;
 }
 
@@ -991,17 +1016,12 @@ void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
         else if (split) launch_mfma<float, 128, 128, false, 0, 2>(s, a);
         else launch_mfma<float, 128, 128, false>(s, a);
     } else {
-        // unquantised bf16: the LDS-direct kernel, on the tiles dma_plan() picks
-        const bool allow_dma = a.lds_direct != 0;
-        // its loads address a k tile with 32-bit offsets from one scalar base: 128 rows of x, 8 k-groups of the padded
-        // weights, and for a pair the distance between the two matrices
-        const uint64_t w_span = (uint64_t)mfma_padded_n(a.n) * 128;
-        const uint64_t w_dist = !a.wk2 ? 0 : (a.wk2 > a.wk ? (uint64_t)((const char*)a.wk2 - (const char*)a.wk) : (uint64_t)((const char*)a.wk - (const char*)a.wk2));
-        const bool reach = a.k <= (1 << 22) && w_span < (1ull << 31) && w_dist + w_span < (1ull << 32);
-        if (allow_dma && reach && !small && a.wk2) return launch_dma<3, 2, 2, 3, 2, true>(s, a);
-        if (allow_dma && reach && !small) {
-            const DmaPlan p = dma_plan(a.m, a.k, a.n);
-            return p.wide ? launch_dma<3, 2, 2, 3, 2, false>(s, a, p.splits) : launch_dma<3, 2, 1, 3, 2, false>(s, a);
+        // unquantised bf16: the LDS-direct kernel, on the tiles tile_plan() picks; its loads address a k tile with 32-bit
+        // offsets from one scalar base: 256 rows of x, 8 k-groups of the padded weights
+        const bool reach = a.k <= (1 << 22) && (uint64_t)mfma_padded_n(a.n) * 128 < (1ull << 31);
+        if (a.lds_direct != 0 && reach) {
+            const TilePlan p = tile_plan(a.m, a.k, a.n, a.wk2 != nullptr);
+            return a.wk2 ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);
         }
         if (a.wk2) launch_mfma<bf16_t, 128, 128, true>(s, a);
         else if (small) launch_mfma<bf16_t, 64, 64, false>(s, a);
