@@ -1270,7 +1270,7 @@ int gptrs_hip_fusion_report(const char* program_json, size_t json_len, const int
                 if (in.softcap != 0.f) text += "+softcap";
                 text += in.mfma ? " [gemm]" : in.tiled ? " [stream]" : " [generic]";
             }
-            if (in.op == gptrs::OpKind::FAttnDecode && in.rot_half > 0) text += "+rope";
+            if ((in.op == gptrs::OpKind::FAttnDecode || in.op == gptrs::OpKind::FAttnPrefill) && in.rot_half > 0) text += "+rope";
             text += '\n';
         }
         *needed = text.size() + 1;

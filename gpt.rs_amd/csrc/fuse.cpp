@@ -881,6 +881,120 @@ struct Fuser {
         }
     }
 
+    // A prompt's attention with everything between the projection and the caches: [the rotation of its packed rows,] the attention
+    // and the updates of the two caches with its K and V rows, for every sequence of a batch of stacked rows, become one
+    // instruction (ops/functional/attention.rs:443-522, model/gpt.rs:712-730).
+    void pass_prefill_caches() {
+        std::map<int, std::vector<std::array<int64_t, 3>>> updates;   // packed tensor -> (instruction, first column, columns)
+        for (size_t i = 0; i < fn.body.size(); ++i) {
+            const Instr& du = fn.body[i];
+            if (du.dead || du.op != OpKind::DynamicUpdateSlice || !du.view_dims.empty() || du.operands[1].value < 0) continue;
+            int packed;
+            int64_t col, width;
+            if (m_qkv_block(du.operands[1].value, true, packed, col, width)) updates[packed].push_back({(int64_t)i, col, width});
+        }
+        const std::vector<int> uses = count_uses();
+        auto attention = [&](int v) -> const Instr* {
+            const Instr* p = producer(v);
+            return p && !p->dead && p->op == OpKind::FAttnPrefill && p->batch == 0 ? p : nullptr;
+        };
+        auto input = [&](int v) { return v >= 0 && def[v] < 0; };
+        struct Part { int x = -1, cos = -1, sin = -1, starts = -1, du[2] = {-1, -1}; int64_t rot = 0; };
+        auto part_of = [&](const Instr& at, int64_t T, Part& p) {
+            const int rows = at.operands[0].value;
+            p.x = rows;
+            const Instr* rp = producer(rows);
+            if (rp && !rp->dead && rp->op == OpKind::FRope && rp->n_q == at.n_q && rp->n_kv == at.n_kv && rp->head_dim == at.head_dim) {
+                p.x = rp->operands[0].value; p.cos = rp->operands[1].value; p.sin = rp->operands[2].value; p.rot = rp->rot_half;
+            }
+            if (p.x < 0 || (p.rot && (p.cos < 0 || p.sin < 0))) return false;
+            for (int from : {rows, p.x}) {
+                auto it = updates.find(from);
+                if (it == updates.end()) continue;
+                for (const auto& u : it->second) {
+                    const Instr& du = fn.body[u[0]];
+                    const int kv = u[1] == at.n_q * at.head_dim ? 0 : u[1] == (at.n_q + at.n_kv) * at.head_dim ? 1 : -1;
+                    if (du.dead || kv < 0 || u[2] != at.n_kv * at.head_dim || (kv == 0 && from != rows)) continue;   // cached keys are the rotated ones
+                    if (p.du[kv] == (int)u[0]) continue;
+                    if (p.du[kv] >= 0 || du.a != std::vector<int64_t>{at.n_kv, T, at.head_dim}) return false;
+                    if (!input(du.operands[0].value) || !input(du.operands[2].value)) return false;   // nothing of the program in front of them
+                    if (p.starts >= 0 && du.operands[2].value != p.starts) return false;
+                    p.starts = du.operands[2].value;
+                    p.du[kv] = (int)u[0];
+                }
+            }
+            return p.du[0] >= 0 && p.du[1] >= 0;
+        };
+        // the stacked attentions of a batch first, then whatever stands alone
+        for (size_t at_ci = 0; at_ci < 2 * fn.body.size(); ++at_ci) {
+            const size_t ci = at_ci % fn.body.size();
+            const Instr root = fn.body[ci];
+            if (root.dead) continue;
+            std::vector<const Instr*> ats;
+            if (at_ci < fn.body.size()) {
+                if (root.op != OpKind::Concat || root.axis != 0 || root.operands.size() > (size_t)k::kAttnBatch) continue;
+                for (const Operand& o : root.operands) {
+                    const Instr* at = o.value >= 0 && uses[o.value] == 1 ? attention(o.value) : nullptr;
+                    if (!at) { ats.clear(); break; }
+                    ats.push_back(at);
+                }
+            } else if (root.op == OpKind::FAttnPrefill && root.batch == 0) {
+                ats.push_back(&fn.body[ci]);
+            }
+            if (ats.empty()) continue;
+            const int64_t B = (int64_t)ats.size(), T = ats[0]->out_specs[0].dims[0];
+            const Instr& a0 = *ats[0];
+            if (!k::attn_prefill_batch_ok((int)a0.out_specs[0].dtype, a0.n_q, a0.n_kv, a0.head_dim, 0)) continue;
+            std::vector<Part> parts(B);
+            int src = -1;
+            bool ok = true;
+            for (int64_t b = 0; b < B && ok; ++b) {
+                const Instr& at = *ats[b];
+                ok = at.n_q == a0.n_q && at.n_kv == a0.n_kv && at.head_dim == a0.head_dim && at.scale == a0.scale && at.out_specs == a0.out_specs && part_of(at, T, parts[b]);
+                if (!ok) break;
+                const Part &p = parts[b], &p0 = parts[0];
+                ok = p.cos == p0.cos && p.sin == p0.sin && p.rot == p0.rot && p.starts == p0.starts;
+                for (int kv = 0; kv < 2 && ok; ++kv) {
+                    const Spec& c = fn.body[p.du[kv]].out_specs[0];
+                    ok = c == fn.body[p0.du[0]].out_specs[0] && c.dtype == a0.out_specs[0].dtype;
+                }
+                if (B == 1) { src = p.x; continue; }
+                const Instr* sl = ok ? producer(p.x) : nullptr;
+                const Spec* ss = sl && !sl->dead && sl->op == OpKind::Slice ? spec_of(sl->operands[0].value) : nullptr;
+                ok = ss && ss->rank() == 2 && ss->dims[0] == B * T && sl->a == std::vector<int64_t>{b * T, 0} && sl->b == std::vector<int64_t>{T, ss->dims[1]};
+                if (!ok) break;
+                if (b == 0) src = sl->operands[0].value;
+                ok = sl->operands[0].value == src;
+            }
+            ok = ok && k::attn_prefill_batch_ok((int)a0.out_specs[0].dtype, a0.n_q, a0.n_kv, a0.head_dim, parts[0].rot);
+            if (ok && parts[0].rot) {   // tables of the rows' type, one row per position
+                const Spec *cs = spec_of(parts[0].cos), *ss = spec_of(parts[0].sin);
+                ok = cs && ss && *cs == *ss && cs->dims == std::vector<int64_t>{T, parts[0].rot} && cs->dtype == a0.out_specs[0].dtype;
+            }
+            if (!ok) continue;
+            Instr ni = make(OpKind::FAttnPrefill, "fused.attention_prefill_caches", {src, parts[0].starts}, root.out_ids[0], root.out_specs[0]);
+            ni.n_q = a0.n_q; ni.n_kv = a0.n_kv; ni.head_dim = a0.head_dim; ni.scale = a0.scale;
+            ni.rot_half = parts[0].rot;
+            ni.batch = B;
+            auto add = [&](int v) { Operand o; o.value = v; ni.operands.push_back(o); };
+            if (ni.rot_half) { add(parts[0].cos); add(parts[0].sin); }
+            std::vector<int> dead;
+            for (const Part& p : parts)
+                for (int kv = 0; kv < 2; ++kv) {
+                    const Instr& du = fn.body[p.du[kv]];
+                    add(du.operands[0].value);
+                    add_out(ni, du.out_ids[0], du.out_specs[0]);
+                    dead.push_back(du.out_ids[0]);
+                }
+            if (B > 1)
+                for (const Instr* at : ats) dead.push_back(at->out_ids[0]);
+            for (int v : dead) kill(v);
+            fn.body[ci] = ni;
+            ++fused;
+            reindex();
+        }
+    }
+
     // ---------------------------------------------------------------- sequence mixers
     // The calls of one mixer layer, for one sequence or for every sequence of a batch, become one instruction.
     const Instr* mixer(int v, Mix mix) const {
@@ -1798,6 +1912,8 @@ int fuse_function(Function& fn) {
     f.pass_rope_into_attention();
     f.dce();
     f.pass_attention_batch();
+    f.dce();
+    f.pass_prefill_caches();
     f.dce();
     f.pass_ssm();
     f.pass_latent();

@@ -327,16 +327,27 @@ struct AttnDecodeArgs {
 size_t attn_decode_workspace_bytes(int64_t n_q, int64_t head_dim, int64_t capacity);
 int attn_decode(hipStream_t s, const AttnDecodeArgs& a);   // returns the number of launches it made
 
-// Prefill causal attention (ops/functional/attention.rs:443-522): packed qkv [T, P] ->
-// ctx [T, n_q*head_dim], and K/V in cache layout [n_kv, T, head_dim].
+// Prefill causal attention (ops/functional/attention.rs:443-522): packed qkv [T, P] -> ctx [T, n_q*head_dim], for up to
+// kAttnBatch sequences of one length in one launch, and the sequences' K / V rows into their caches.
+constexpr int kAttnBatch = 16;
 struct AttnPrefillArgs {
     int dtype;
-    const void* qkv;
-    void* ctx; void* k_out; void* v_out;
-    int64_t t, n_q, n_kv, head_dim;
+    const void* qkv;      // [batch * t, P]: the sequences' rows stacked
+    void* ctx;
+    int64_t t, n_q, n_kv, head_dim;   // t: rows of every sequence
     float scale;
+    int batch = 1;
+    // with `starts` (attn_prefill_batch_ok() shapes): sequence b's key and value rows go into its caches [n_kv, capacity,
+    // head_dim] first, at row clamp(starts[1], 0, capacity - t) as a DynamicUpdateSlice places them; with rot_half =
+    // head_dim / 2 the queries and the cached keys are rotated by cos / sin [t, rot_half]
+    const int32_t* starts = nullptr;
+    int64_t capacity = 0;
+    void* k_caches[kAttnBatch] = {}; void* v_caches[kAttnBatch] = {};
+    const void* cos = nullptr; const void* sin = nullptr;
+    int64_t rot_half = 0;
 };
-void attn_prefill(hipStream_t s, const AttnPrefillArgs& a);
+bool attn_prefill_batch_ok(int dtype, int64_t n_q, int64_t n_kv, int64_t head_dim, int64_t rot_half);
+int attn_prefill(hipStream_t s, const AttnPrefillArgs& a);   // returns the number of launches
 
 // Causal attention over a growing cache (ops/functional/attention.rs:359-437, the `cache = Some` branch): T new rows of
 // packed qkv [T, P] behind caches [n_kv, C, head_dim]: k_all / v_all [n_kv, C + T, head_dim] = the caches with the new

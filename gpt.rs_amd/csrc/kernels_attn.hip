@@ -6,6 +6,8 @@
 // <= the query position are visited.  GQA: query head h reads kv head h / group.
 #include <cstdlib>
 
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "device_utils.hpp"
 
@@ -604,6 +606,62 @@ int attn_decode(hipStream_t s, const AttnDecodeArgs& a) {
     return a.dtype == 0 ? attn_decode_t<float>(s, a) : attn_decode_t<bf16_t>(s, a);
 }
 
+// Where the K / V rows of a prefill's sequences lie: in the caches attn_prefill_kv_kernel has put them into, or (no `starts`)
+// in the packed rows themselves.
+template <typename T> struct PrefillKv {
+    const T* k[kAttnBatch];
+    const T* v[kAttnBatch];
+    const int32_t* starts;
+    int64_t capacity;
+    const T* cos;
+    const T* sin;
+};
+template <typename T>
+__device__ __forceinline__ const T* prefill_rows(const T* const* caches, const PrefillKv<T>& kv, const T* rows, int seq, int kvh, int dh, int t, int64_t row_pitch,
+                                                 int64_t col, int64_t& pitch) {
+    if (!kv.starts) { pitch = row_pitch; return rows + col; }
+    pitch = dh;
+    const int64_t at = min(max((int64_t)kv.starts[1], (int64_t)0), kv.capacity - t);
+    return caches[seq] + (kvh * kv.capacity + at) * dh;
+}
+
+// The K and V columns of stacked packed rows [batch * t, P] -> the sequences' caches [n_kv, capacity, dh] at the row the update
+// names, the keys rotated on the way (the arithmetic and rounding of rope_kernel).  One thread per 16 bytes; bound by memory: a
+// third of the projection read once and written once, where a rotation of all rows, a copy of every sequence's rows and two
+// cache updates per sequence took 164 us a layer at 4 x 2047 tokens of 32 + 2 x 8 heads of 128.
+template <typename T>
+__global__ __launch_bounds__(256) void attn_prefill_kv_kernel(const T* __restrict__ qkv, int64_t chunks, int t, int n_q, int n_kv, int dh, PrefillKv<T> kv) {
+    constexpr int VEC = 16 / sizeof(T);
+    typedef T vec_t __attribute__((ext_vector_type(VEC)));
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (id >= chunks) return;
+    const int hc = dh / VEC, rc = 2 * n_kv * hc;        // chunks of a head, of a row's K and V
+    const int64_t row = id / rc;
+    const int c = (int)(id % rc), head = c / hc, d = c % hc * VEC;
+    const int seq = (int)(row / t), pos = (int)(row % t);
+    const T* src = qkv + row * ((int64_t)(n_q + 2 * n_kv) * dh) + (int64_t)(n_q + head) * dh;
+    vec_t x = *reinterpret_cast<const vec_t*>(src + d);
+    const bool key = head < n_kv;
+    if (key && kv.cos) {
+        const int h2 = dh / 2;
+        const bool second = d >= h2;
+        const int j = second ? d - h2 : d;
+        const vec_t y = *reinterpret_cast<const vec_t*>(src + (second ? j : d + h2));
+        const vec_t cv = *reinterpret_cast<const vec_t*>(kv.cos + (int64_t)pos * h2 + j), sv = *reinterpret_cast<const vec_t*>(kv.sin + (int64_t)pos * h2 + j);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const T xe = x[e], ye = y[e], ce = cv[e], se = sv[e];
+            const float xf = ldf(&xe, 0), yf = ldf(&ye, 0), cf = ldf(&ce, 0), sf = ldf(&se, 0);
+            T out;
+            stf(&out, 0, second ? xf * cf + yf * sf : xf * cf - yf * sf);
+            x[e] = out;
+        }
+    }
+    const int64_t at = min(max((int64_t)kv.starts[1], (int64_t)0), kv.capacity - t) + pos;
+    T* to = const_cast<T*>(key ? kv.k[seq] : kv.v[seq]) + ((int64_t)(key ? head : head - n_kv) * kv.capacity + at) * dh + d;
+    *reinterpret_cast<vec_t*>(to) = x;
+}
+
 // ------------------------------------------------------------------------------ prefill
 // grid (ceil(T/4), n_q), 256 threads: one wave per query row.  Keys are visited 64 at a time
 // (one per lane) with an online softmax; the P.V update then walks the chunk with the lanes
@@ -676,7 +734,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const T* __restrict__
 // (the launch has one wave-sized task per SIMD otherwise).
 template <int DH, int KG>
 __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ ctx, int T,
-                                                                int n_q, int n_kv, float scale_log2e) {
+                                                                int n_q, int n_kv, float scale_log2e, int zgroups, PrefillKv<bf16_t> kv) {
     constexpr int KT = 32;            // keys per tile
     constexpr int KS = DH + 8;        // K tile row stride in elements (16 bytes of padding)
     // V^T rows: stride VS elements, row d starts 8 * ((d / 8) % 8) elements in.  Two access patterns must spread over
@@ -708,12 +766,17 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
     const int gw = G >= 4 ? 4 : G;                 // query heads of the group in this workgroup
     const int rtpb = 4 / gw;                       // 32-row tiles per workgroup
     const int kvh = blockIdx.y;
-    const int head = kvh * G + blockIdx.z * gw + wave % gw;
-    const int q0 = (blockIdx.x * rtpb + wave / gw) * 32;
+    const int seq = blockIdx.z / zgroups, zg = blockIdx.z % zgroups;
+    const int bx = gridDim.x - 1 - blockIdx.x;     // rows that see many keys first: the last workgroups to start are the short ones
+    const int head = kvh * G + zg * gw + wave % gw;
+    const int q0 = (bx * rtpb + wave / gw) * 32;
     const int64_t P = (int64_t)(n_q + 2 * n_kv) * DH;
-    const int64_t koff = (int64_t)n_q * DH + (int64_t)kvh * DH;
-    const int64_t voff = (int64_t)(n_q + n_kv) * DH + (int64_t)kvh * DH;
-    const int kend = min(T, (blockIdx.x * rtpb + rtpb) * 32);   // keys any row of the workgroup may see
+    qkv += (int64_t)seq * T * P;
+    ctx += (int64_t)seq * T * n_q * DH;
+    int64_t kpitch;
+    const auto* kp = prefill_rows(kv.k, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + kvh) * DH, kpitch);
+    const auto* vp = prefill_rows(kv.v, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + n_kv + kvh) * DH, kpitch);
+    const int kend = min(T, (bx * rtpb + rtpb) * 32);   // keys any row of the workgroup may see
     const int ntiles = (kend + KT - 1) / KT;
     const bool active = q0 < T;
     const int my_tiles = active ? min(ntiles, (q0 + 31) / KT + 1) : 0;   // tiles holding a key <= this wave's last row
@@ -725,6 +788,19 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
         const bf16_t* qp = qkv + (int64_t)row * P + (int64_t)head * DH + 8 * half;
 #pragma unroll
         for (int kk = 0; kk < NK; ++kk) qf[kk] = *reinterpret_cast<const bf16x8_v*>(qp + 16 * kk);
+        if (kv.cos) {   // the rotated row, rounded to bf16 as the projection's rows are (rope_kernel); partners sit in one lane
+#pragma unroll
+            for (int kk = 0; kk < NK / 2; ++kk) {
+                const bf16x8_v cv = *reinterpret_cast<const bf16x8_v*>(kv.cos + (int64_t)row * (DH / 2) + 16 * kk + 8 * half);
+                const bf16x8_v sv = *reinterpret_cast<const bf16x8_v*>(kv.sin + (int64_t)row * (DH / 2) + 16 * kk + 8 * half);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = (float)qf[kk][e], y = (float)qf[kk + NK / 2][e], c = (float)cv[e], sn = (float)sv[e];
+                    qf[kk][e] = (__bf16)(x * c - y * sn);
+                    qf[kk + NK / 2][e] = (__bf16)(y * c + x * sn);
+                }
+            }
+        }
     }
     f32x16_v acc_o[ND];
 #pragma unroll
@@ -743,8 +819,8 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
             const int c = min(tid + 256 * j, CH - 1);
             const int r = c / (DH / 8), ch = c % (DH / 8);
             const int64_t key = min(t * KT + r, T - 1);
-            kreg[j] = *reinterpret_cast<const u32x4_s*>(qkv + key * P + koff + ch * 8);
-            vreg[j] = *reinterpret_cast<const u32x4_s*>(qkv + key * P + voff + ch * 8);
+            kreg[j] = *reinterpret_cast<const u32x4_s*>(kp + key * kpitch + ch * 8);
+            vreg[j] = *reinterpret_cast<const u32x4_s*>(vp + key * kpitch + ch * 8);
         }
     };
     auto lwrite = [&](int buf) {
@@ -894,7 +970,7 @@ __device__ __forceinline__ f32x16_v mma_f32x4(const f32x4_v& a, const f32x4_v& b
 
 template <int DH>
 __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const float* __restrict__ qkv, float* __restrict__ ctx, int T,
-                                                                    int n_q, int n_kv, float scale_log2e) {
+                                                                    int n_q, int n_kv, float scale_log2e, int zgroups, PrefillKv<float> kv) {
     constexpr int KT = 32;            // keys per tile
     constexpr int KS = DH + 4;        // K tile row stride in elements (16 bytes of padding)
     // V^T row stride in elements; row d starts 4 * ((d / 4) % 8) elements in, which spreads the lanes that scatter one
@@ -913,12 +989,17 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
     const int gw = G >= 4 ? 4 : G;
     const int rtpb = 4 / gw;
     const int kvh = blockIdx.y;
-    const int head = kvh * G + blockIdx.z * gw + wave % gw;
-    const int q0 = (blockIdx.x * rtpb + wave / gw) * 32;
+    const int seq = blockIdx.z / zgroups, zg = blockIdx.z % zgroups;
+    const int bx = gridDim.x - 1 - blockIdx.x;     // rows that see many keys first: the last workgroups to start are the short ones
+    const int head = kvh * G + zg * gw + wave % gw;
+    const int q0 = (bx * rtpb + wave / gw) * 32;
     const int64_t P = (int64_t)(n_q + 2 * n_kv) * DH;
-    const int64_t koff = (int64_t)n_q * DH + (int64_t)kvh * DH;
-    const int64_t voff = (int64_t)(n_q + n_kv) * DH + (int64_t)kvh * DH;
-    const int kend = min(T, (blockIdx.x * rtpb + rtpb) * 32);
+    qkv += (int64_t)seq * T * P;
+    ctx += (int64_t)seq * T * n_q * DH;
+    int64_t kpitch;
+    const auto* kp = prefill_rows(kv.k, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + kvh) * DH, kpitch);
+    const auto* vp = prefill_rows(kv.v, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + n_kv + kvh) * DH, kpitch);
+    const int kend = min(T, (bx * rtpb + rtpb) * 32);
     const int ntiles = (kend + KT - 1) / KT;
     const bool active = q0 < T;
     const int my_tiles = active ? min(ntiles, (q0 + 31) / KT + 1) : 0;
@@ -929,6 +1010,19 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
         const float* qp = qkv + (int64_t)row * P + (int64_t)head * DH + 4 * half;
 #pragma unroll
         for (int kk = 0; kk < NK; ++kk) qf[kk] = *reinterpret_cast<const f32x4_v*>(qp + 8 * kk);
+        if (kv.cos) {   // see the bf16 kernel
+#pragma unroll
+            for (int kk = 0; kk < NK / 2; ++kk) {
+                const f32x4_v cv = *reinterpret_cast<const f32x4_v*>(kv.cos + (int64_t)row * (DH / 2) + 8 * kk + 4 * half);
+                const f32x4_v sv = *reinterpret_cast<const f32x4_v*>(kv.sin + (int64_t)row * (DH / 2) + 8 * kk + 4 * half);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float x = qf[kk][e], y = qf[kk + NK / 2][e];
+                    qf[kk][e] = x * cv[e] - y * sv[e];
+                    qf[kk + NK / 2][e] = y * cv[e] + x * sv[e];
+                }
+            }
+        }
     }
     f32x16_v acc_o[ND];
 #pragma unroll
@@ -944,8 +1038,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
             const int c = min(tid + 256 * j, CH - 1);   // unconditional loads: see the bf16 kernel
             const int r = c / (DH / 4), ch = c % (DH / 4);
             const int64_t key = min(t * KT + r, T - 1);
-            kreg[j] = *reinterpret_cast<const f32x4_v*>(qkv + key * P + koff + ch * 4);
-            vreg[j] = *reinterpret_cast<const f32x4_v*>(qkv + key * P + voff + ch * 4);
+            kreg[j] = *reinterpret_cast<const f32x4_v*>(kp + key * kpitch + ch * 4);
+            vreg[j] = *reinterpret_cast<const f32x4_v*>(vp + key * kpitch + ch * 4);
         }
     };
     auto lwrite = [&](int buf) {
@@ -1039,46 +1133,65 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
     }
 }
 
-static bool attn_prefill_mfma_ok(const AttnPrefillArgs& a) {
-    if ((a.dtype != 2 && a.dtype != 0) || a.n_kv <= 0 || a.n_q % a.n_kv != 0 || a.t >= (1ll << 30)) return false;
-    if (a.head_dim != 32 && a.head_dim != 64 && a.head_dim != 128) return false;
-    const int64_t g = a.n_q / a.n_kv;
+static bool attn_prefill_mfma_ok(int dtype, int64_t n_q, int64_t n_kv, int64_t head_dim) {
+    static const bool use_mfma = [] { const char* e = getenv("GPTRS_HIP_MFMA_ATTN"); return !(e && e[0] == '0'); }();
+    if (!use_mfma || (dtype != 2 && dtype != 0) || n_kv <= 0 || n_q % n_kv != 0) return false;
+    if (head_dim != 32 && head_dim != 64 && head_dim != 128) return false;
+    const int64_t g = n_q / n_kv;
     return g == 1 || g == 2 || g % 4 == 0;
 }
+bool attn_prefill_batch_ok(int dtype, int64_t n_q, int64_t n_kv, int64_t head_dim, int64_t rot_half) {
+    return attn_prefill_mfma_ok(dtype, n_q, n_kv, head_dim) && (rot_half == 0 || 2 * rot_half == head_dim);
+}
 
-void attn_prefill(hipStream_t s, const AttnPrefillArgs& a) {
-    if (a.t <= 0) return;
-    static const bool use_mfma = [] { const char* e = getenv("GPTRS_HIP_MFMA_ATTN"); return !(e && e[0] == '0'); }();
-    if (use_mfma && attn_prefill_mfma_ok(a)) {
-        const int g = (int)(a.n_q / a.n_kv), gw = g >= 4 ? 4 : g;
-        dim3 grid((unsigned)cdiv(cdiv(a.t, 32), 4 / gw), (unsigned)a.n_kv, (unsigned)(g >= 4 ? g / 4 : 1));
-        const float sl = a.scale * 1.44269504088896f;
-        if (a.dtype == 0) {
-            if (a.head_dim == 32) attn_prefill_mfma_f32_kernel<32><<<grid, 256, 0, s>>>((const float*)a.qkv, (float*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl);
-            else if (a.head_dim == 64) attn_prefill_mfma_f32_kernel<64><<<grid, 256, 0, s>>>((const float*)a.qkv, (float*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl);
-            else attn_prefill_mfma_f32_kernel<128><<<grid, 256, 0, s>>>((const float*)a.qkv, (float*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl);
-            return;
-        }
+template <typename T>
+static int attn_prefill_mfma(hipStream_t s, const AttnPrefillArgs& a) {
+    PrefillKv<T> kv{};
+    for (int b = 0; b < a.batch && a.starts; ++b) { kv.k[b] = (const T*)a.k_caches[b]; kv.v[b] = (const T*)a.v_caches[b]; }
+    kv.starts = a.starts;
+    kv.capacity = a.capacity;
+    if (a.rot_half) { kv.cos = (const T*)a.cos; kv.sin = (const T*)a.sin; }
+    int launches = 1;
+    if (a.starts) {
+        const int64_t chunks = a.batch * a.t * 2 * a.n_kv * a.head_dim / (16 / (int64_t)sizeof(T));
+        attn_prefill_kv_kernel<T><<<(unsigned)cdiv(chunks, 256), 256, 0, s>>>((const T*)a.qkv, chunks, (int)a.t, (int)a.n_q, (int)a.n_kv, (int)a.head_dim, kv);
+        ++launches;
+    }
+    const int g = (int)(a.n_q / a.n_kv), gw = g >= 4 ? 4 : g, zg = g >= 4 ? g / 4 : 1;
+    const dim3 grid((unsigned)cdiv(cdiv(a.t, 32), 4 / gw), (unsigned)a.n_kv, (unsigned)(zg * a.batch));
+    const float sl = a.scale * 1.44269504088896f;
+    if constexpr (std::is_same<T, float>::value) {
+        auto go = [&](auto dh) { attn_prefill_mfma_f32_kernel<decltype(dh)::value><<<grid, 256, 0, s>>>((const float*)a.qkv, (float*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv); };
+        if (a.head_dim == 32) go(std::integral_constant<int, 32>{});
+        else if (a.head_dim == 64) go(std::integral_constant<int, 64>{});
+        else go(std::integral_constant<int, 128>{});
+    } else {
         // two key groups per workgroup once the launch is smaller than three workgroups per CU and rows are long
         // enough to split
         static const bool allow_kg = [] { const char* e = getenv("GPTRS_HIP_ATTN_KEYGROUPS"); return !(e && e[0] == '0'); }();
         const bool kg2 = allow_kg && a.t >= 128 && (int64_t)grid.x * grid.y * grid.z < 768;
-#define GPTRS_PREFILL(DHV)                                                                                                   \
-        do {                                                                                                                 \
-            if (kg2) attn_prefill_mfma_kernel<DHV, 2><<<grid, 512, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl); \
-            else attn_prefill_mfma_kernel<DHV, 1><<<grid, 256, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl);     \
-        } while (0)
-        if (a.head_dim == 32) GPTRS_PREFILL(32);
-        else if (a.head_dim == 64) GPTRS_PREFILL(64);
-        else GPTRS_PREFILL(128);
-#undef GPTRS_PREFILL
-        return;
+        auto go = [&](auto dh) {
+            constexpr int D = decltype(dh)::value;
+            if (kg2) attn_prefill_mfma_kernel<D, 2><<<grid, 512, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv);
+            else attn_prefill_mfma_kernel<D, 1><<<grid, 256, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv);
+        };
+        if (a.head_dim == 32) go(std::integral_constant<int, 32>{});
+        else if (a.head_dim == 64) go(std::integral_constant<int, 64>{});
+        else go(std::integral_constant<int, 128>{});
     }
+    return launches;
+}
+
+int attn_prefill(hipStream_t s, const AttnPrefillArgs& a) {
+    if (a.t <= 0) return 0;
+    if (attn_prefill_mfma_ok(a.dtype, a.n_q, a.n_kv, a.head_dim) && a.t < (1ll << 30))
+        return a.dtype == 0 ? attn_prefill_mfma<float>(s, a) : attn_prefill_mfma<bf16_t>(s, a);
     dim3 grid((unsigned)cdiv(a.t, 4), (unsigned)a.n_q);
     if (a.dtype == 0)
         attn_prefill_kernel<float><<<grid, 256, 0, s>>>((const float*)a.qkv, (float*)a.ctx, a.t, (int)a.n_q, (int)a.n_kv, (int)a.head_dim, a.scale);
     else
         attn_prefill_kernel<bf16_t><<<grid, 256, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.ctx, a.t, (int)a.n_q, (int)a.n_kv, (int)a.head_dim, a.scale);
+    return 1;
 }
 
 // ------------------------------------------------------------------------------ attention over a growing cache

@@ -711,6 +711,9 @@ void Builder::build() {
                 pairs.push_back({(int)attn_cache_operand(st.in, b), (int)attn_cache_output(b)});
                 pairs.push_back({(int)attn_cache_operand(st.in, b) + 1, (int)attn_cache_output(b) + 1});
             }
+        if (st.in.op == OpKind::FAttnPrefill && prefill_cached(st.in))
+            for (int64_t b = 0; b < st.in.batch; ++b)
+                for (int kv = 0; kv < 2; ++kv) pairs.push_back({(int)prefill_cache_operand(st.in, b) + kv, (int)attn_cache_output(b) + kv});
         if (st.in.op == OpKind::FMixer) pairs = mixer_inplace_pairs(st.in);
         bool all_inplace = !pairs.empty();
         for (auto& pr : pairs) {
@@ -1442,10 +1445,23 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
             a.dtype = (int)out.dtype;
             a.qkv = src_ptr(st, cx, 0);
             a.ctx = dst;
-            a.t = x.dims[0]; a.n_q = in.n_q; a.n_kv = in.n_kv; a.head_dim = in.head_dim;
+            a.batch = (int)std::max<int64_t>(in.batch, 1);
+            a.t = x.dims[0] / a.batch; a.n_q = in.n_q; a.n_kv = in.n_kv; a.head_dim = in.head_dim;
             a.scale = in.scale;
-            k::attn_prefill(s, a);
-            ++cx.launches;
+            if (prefill_cached(in)) {
+                const Spec& ck = in_spec(prefill_cache_operand(in, 0));
+                for (int64_t b = 0; b < a.batch; ++b)   // caches that were not donated are copied first
+                    for (size_t kv = 0; kv < 2; ++kv) {
+                        void* to = cx.ptr[st.dst[attn_cache_output(b) + kv]];
+                        const void* from = src_ptr(st, cx, prefill_cache_operand(in, b) + kv);
+                        if (to != from) { GPTRS_HIP_CHECK(hipMemcpyAsync(to, from, ck.bytes(), hipMemcpyDeviceToDevice, s)); ++cx.launches; }
+                        (kv ? a.v_caches : a.k_caches)[b] = to;
+                    }
+                a.capacity = ck.dims[1];
+                a.starts = (const int32_t*)src_ptr(st, cx, 1);
+                if (in.rot_half > 0) { a.cos = src_ptr(st, cx, 2); a.sin = src_ptr(st, cx, 3); a.rot_half = in.rot_half; }
+            }
+            cx.launches += k::attn_prefill(s, a);
             break;
         }
         case OpKind::FAttnConcat: {

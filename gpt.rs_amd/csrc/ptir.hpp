@@ -167,6 +167,10 @@ struct Instr {
 // FAttnDecode: operand slots of the K / V cache of sequence b, output slot of its updated K cache (V follows)
 inline size_t attn_cache_operand(const Instr& in, int64_t b) { return b == 0 ? 1 : (size_t)(5 + (in.rot_half > 0 ? 2 : 0) + 2 * (b - 1)); }
 inline size_t attn_cache_output(int64_t b) { return (size_t)(1 + 2 * b); }
+// FAttnPrefill with caches (Fuser::pass_prefill_caches): (qkv [batch * T, P], starts, [cos, sin,] k_0, v_0, k_1, ..) ->
+// (ctx, k'_0, v'_0, ..); without: (qkv) -> (ctx)
+inline bool prefill_cached(const Instr& in) { return in.out_ids.size() > 1; }
+inline size_t prefill_cache_operand(const Instr& in, int64_t b) { return (size_t)(2 + (in.rot_half > 0 ? 2 : 0) + 2 * b); }
 
 // operand position of the SwiGLU partner's weights / of the first epilogue operand of an FLinear
 inline size_t linear_w2_pos(const Instr& in) { return in.quant ? 3 : 2; }

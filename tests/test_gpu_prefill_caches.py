@@ -1,0 +1,89 @@
+"""A prompt's attention fused with the rotation of its rows and the updates of the caches (Fuser::pass_prefill_caches): one sequence
+and stacked batches, against the oracle and against float64."""
+import numpy as np
+import pytest
+
+from parity import assert_close, check_program, hip_run, oracle_run
+from gptrs_amd import functional as F
+from gptrs_amd.backend import fusion_report
+from gptrs_amd.ptir import FunctionBuilder, Program, Tensor, bf16_bits_to_f32, f32_to_bf16_bits
+
+CASES = [  # sequences, rows, query heads, key heads, head size, rotated, cache rows, first row that the update names
+    (1, 2, 2, 2, 32, True, 2, 0), (1, 33, 4, 1, 32, True, 64, 5), (2, 32, 2, 2, 64, False, 32, 0), (3, 31, 8, 2, 64, True, 40, 100),
+    (16, 3, 4, 4, 32, False, 8, -2), (2, 129, 8, 1, 128, True, 160, 7), (1, 200, 4, 2, 128, False, 256, 0), (2, 65, 6, 3, 64, True, 65, 0),
+    (3, 5, 3, 1, 32, False, 6, 1),     # three query heads to a key head: the unfused series
+]
+
+
+def program(dt, B, T, hq, hkv, dh, rot, cap):
+    fb = FunctionBuilder("main", dt)
+    cfg = F.AttentionConfig(hq * dh, hq, hkv, dh)
+    qkv = fb.param(dt, [B * T, (hq + 2 * hkv) * dh])
+    tabs = [fb.param(dt, [T, dh // 2]) for _ in range(2)] if rot else []
+    starts = fb.param("Si32", [3])
+    caches = [fb.param(dt, [hkv, cap, dh]) for _ in range(2 * B)]
+    ctxs, outs = [], []
+    for b in range(B):
+        rows = qkv if B == 1 else qkv.slice([b * T, 0], [T, qkv.dims[1]])
+        if rot:
+            rows = F.apply_rope_qkv_packed(cfg, rows, *tabs)
+        ctx, k, v = F.attention(cfg, rows, None)
+        ctxs.append(ctx)
+        outs += [F.dynamic_update_slice_into(caches[2 * b], k, starts), F.dynamic_update_slice_into(caches[2 * b + 1], v, starts)]
+    fb.set_results([ctxs[0] if B == 1 else Tensor.concat(0, ctxs)] + outs)
+    return Program(fb)
+
+
+def inputs(B, T, hq, hkv, dh, rot, cap, first, seed):
+    rng = np.random.default_rng(seed)
+    out = [rng.standard_normal((B * T, (hq + 2 * hkv) * dh), dtype=np.float32)]
+    if rot:
+        ang = np.arange(T)[:, None] * 100.0 ** (-np.arange(dh // 2) / (dh // 2))
+        out += [np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)]
+    return out + [np.array([0, first, 0], np.int32)] + [rng.standard_normal((hkv, cap, dh), dtype=np.float32) for _ in range(2 * B)]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_is_one_instruction(case):
+    B, T, hq, hkv, dh, rot, cap, _ = case
+    rep = fusion_report(program("F32", B, T, hq, hkv, dh, rot, cap))
+    if hq // hkv == 3:
+        assert "DynamicUpdateSlice" in rep
+    else:
+        assert rep == ["fused.attention_prefill_caches" + ("+rope" if rot else "")]
+
+
+def test_a_cache_that_the_program_computes_stays_apart():
+    """The update's base depends on the attention: taking both up in one instruction would make a cycle."""
+    fb = FunctionBuilder("main", "F32")
+    qkv, starts = fb.param("F32", [8, 96]), fb.param("Si32", [3])
+    cfg = F.AttentionConfig(32, 1, 1, 32)
+    ctx, k, v = F.attention(cfg, qkv, None)
+    base = ctx.reshape([1, 8, 32])
+    fb.set_results([ctx, F.dynamic_update_slice_into(base, k, starts), F.dynamic_update_slice_into(base, v, starts)])
+    assert fusion_report(Program(fb)).count("DynamicUpdateSlice") == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES)
+def test_f32(hip, case):
+    B, T, hq, hkv, dh, rot, cap, first = case
+    check_program(hip, program("F32", B, T, hq, hkv, dh, rot, cap), inputs(B, T, hq, hkv, dh, rot, cap, first, 3), what=str(case))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("donate", [False, True])
+@pytest.mark.parametrize("case", CASES[:-1])
+def test_bf16(hip, case, donate):
+    B, T, hq, hkv, dh, rot, cap, first = case
+    args = [a if a.dtype == np.int32 else bf16_bits_to_f32(f32_to_bf16_bits(a)) for a in inputs(B, T, hq, hkv, dh, rot, cap, first, 4)]
+    n_in = 4 if rot else 2
+    got = hip_run(hip, program("Bf16", B, T, hq, hkv, dh, rot, cap), args, [False] * n_in + [donate] * (2 * B))
+    want = oracle_run(program("F32", B, T, hq, hkv, dh, rot, cap), args)
+    # values between -5 and 5: rotated rows rounded once (2^-9 of up to 7), probabilities and the context once more
+    assert_close(got[0], want[0], atol=3e-2, rtol=2.0 ** -7, what=f"context {case}")
+    for i, (g, w) in enumerate(zip(got[1:], want[1:])):
+        if i % 2 == 0 and rot:
+            assert_close(g, w, atol=1e-6, rtol=2.0 ** -8, what=f"keys {case}")
+        else:
+            assert np.array_equal(g, w), f"cache {i} {case}"
