@@ -503,13 +503,14 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// bf16 GEMM whose tiles go memory -> LDS without passing through registers (global_load_lds_dwordx4), for unquantised
-// bf16 operands: no staging registers, no LDS store instructions, loads run NST - 1 k tiles ahead through a ring.
+// GEMM whose tiles go memory -> LDS without passing through registers (global_load_lds_dwordx4), for unquantised bf16 and f32
+// operands: no staging registers, no LDS store instructions, loads run NST - 1 k tiles ahead through a ring.  Sizes below are
+// those of bf16; f32 has 4 k where bf16 has 8 and moves the same bytes.
 //
 // Workgroup: WM x WN waves; a wave owns (32 TM) x (32 TN) outputs as TM x TN fragments of 32 x 32, the tile is
-// BM x BN = (32 TM WM) x (32 TN WN).  A launch takes one of six tiles and a number of splits over k, see tile_plan().
+// BM x BN = (32 TM WM) x (32 TN WN).  A bf16 launch takes one of six tiles and a number of splits over k, see tile_plan().
 //
-// What bounds it.  256 x 256 tiles, all CUs busy: the matrix pipes at the clock that random operands allow.  A tile's 32 k
+// What bounds it (bf16).  256 x 256 tiles, all CUs busy: the matrix pipes at the clock that random operands allow.  A tile's 32 k
 // take 0.54 us on a quarter of the CUs and 0.8 us on all of them; over all-zero operands the same launch runs at 1.35 times
 // the rate (M = 8188, K = 3072, N = 6144: 1680 against 1240 TFLOP/s), so it is power and not data that paces it.  Why 256 x
 // 256: a k tile moves 1 / (2 BM) + 1 / (2 BN) bytes per flop from the L2s into LDS and as many fragments from LDS into
@@ -548,8 +549,9 @@ __device__ __forceinline__ unsigned long long gemm_uniform64(unsigned long long 
 template <int N> __device__ __forceinline__ void gemm_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
 // What happens to a sum on its way out (a pair has been combined before).
+template <typename T>
 struct TileEpilogue {
-    const bf16_t* bias; const void* residual; void* y;
+    const T* bias; const void* residual; void* y;
     int64_t N;
     int act, out_f32;
     EpiExtra extra;
@@ -557,30 +559,41 @@ struct TileEpilogue {
 // Eight neighbours of row m, columns n .. n + 7, from LDS: bias, GELU, column factor and residual, then one 16-byte store (two
 // for f32 results; element by element when N is not a multiple of 8).  Kept short: with every output's options unrolled the
 // epilogue was 13 000 to 18 000 instructions, more than the instruction cache holds (M = 8188, see gemm_tile_kernel).
-__device__ __forceinline__ void gemm_finish8(const TileEpilogue& p, int64_t m, int64_t n, const float* at_lds) {
+template <typename T>
+__device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m, int64_t n, const float* at_lds) {
     const int64_t at = m * p.N + n;
+    const bool f32 = std::is_same<T, float>::value || p.out_f32;     // y and residual
     if ((p.N & 7) != 0) {
 #pragma unroll 1
         for (int e = 0; e < 8; ++e) {
             if (n + e >= p.N) break;
-            const float bv = p.bias ? bf16_to_f32(p.bias[n + e]) : 0.f;
-            const float rv = p.residual ? (p.out_f32 ? static_cast<const float*>(p.residual)[at + e] : bf16_to_f32(static_cast<const bf16_t*>(p.residual)[at + e])) : 0.f;
+            const float bv = p.bias ? Mma<T>::ld(p.bias, n + e) : 0.f;
+            const float rv = p.residual ? (f32 ? static_cast<const float*>(p.residual)[at + e] : Mma<T>::ld(static_cast<const T*>(p.residual), at + e)) : 0.f;
             const float f = mfma_finish(at_lds[e], 0.f, false, p.act, bv, p.residual != nullptr, rv, p.extra.glu, p.extra.colscale ? p.extra.colscale[n + e] : 1.0f);
-            if (p.out_f32) static_cast<float*>(p.y)[at + e] = f;
-            else static_cast<bf16_t*>(p.y)[at + e] = f32_to_bf16(f);
+            if (f32) static_cast<float*>(p.y)[at + e] = f;
+            else Mma<T>::st(static_cast<T*>(p.y), at + e, f);
         }
         return;
     }
     float o[8];
     *reinterpret_cast<f32x4_t*>(o) = *reinterpret_cast<const f32x4_t*>(at_lds);
     *reinterpret_cast<f32x4_t*>(o + 4) = *reinterpret_cast<const f32x4_t*>(at_lds + 4);
-    if (p.bias) {
-        const u32x4_t bw = *reinterpret_cast<const u32x4_t*>(p.bias + n);
+    auto add_f32 = [&](const float* v) {
+        const f32x4_t r0 = *reinterpret_cast<const f32x4_t*>(v), r1 = *reinterpret_cast<const f32x4_t*>(v + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { o[e] += r0[e]; o[4 + e] += r1[e]; }
+    };
+    auto add_bf16 = [&](const void* v) {
+        const u32x4_t w = *static_cast<const u32x4_t*>(v);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            o[2 * e] += __uint_as_float(bw[e] << 16);            // tensor_ops.rs:42-56
-            o[2 * e + 1] += __uint_as_float(bw[e] & 0xFFFF0000u);
+            o[2 * e] += __uint_as_float(w[e] << 16);
+            o[2 * e + 1] += __uint_as_float(w[e] & 0xFFFF0000u);
         }
+    };
+    if (p.bias) {                                                    // tensor_ops.rs:42-56
+        if constexpr (std::is_same<T, float>::value) add_f32(p.bias + n);
+        else add_bf16(p.bias + n);
     }
     if (p.act == 1) {
 #pragma unroll
@@ -592,21 +605,10 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue& p, int64_t m, i
         for (int e = 0; e < 4; ++e) { o[e] *= c0[e]; o[4 + e] *= c1[e]; }
     }
     if (p.residual) {
-        if (p.out_f32) {
-            const f32x4_t r0 = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(p.residual) + at);
-            const f32x4_t r1 = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(p.residual) + at + 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { o[e] += r0[e]; o[4 + e] += r1[e]; }
-        } else {
-            const u32x4_t rw = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(p.residual) + at);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                o[2 * e] += __uint_as_float(rw[e] << 16);
-                o[2 * e + 1] += __uint_as_float(rw[e] & 0xFFFF0000u);
-            }
-        }
+        if (f32) add_f32(static_cast<const float*>(p.residual) + at);
+        else add_bf16(static_cast<const bf16_t*>(p.residual) + at);
     }
-    if (p.out_f32) {
+    if (f32) {
         *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.y) + at) = *reinterpret_cast<const f32x4_t*>(o);
         *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.y) + at + 4) = *reinterpret_cast<const f32x4_t*>(o + 4);
     } else {
@@ -618,7 +620,9 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue& p, int64_t m, i
 }
 // The pair's gate on the hardware's exp2 and reciprocal (1 ulp each of f32; the result goes on as bf16): the exact division
 // and expf of glu_combine are 40 instructions an output, 9 us of a 256 x 256 tile's 85.
+template <typename T>
 __device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) {
+    if (std::is_same<T, float>::value) return glu_combine(g, u, p.kind, p.limit, p.alpha, p.shift);
     const float alpha = p.kind == 1 ? p.alpha : 1.0f;
     if (p.kind == 1) {
         g = fminf(g, p.limit);
@@ -627,11 +631,12 @@ __device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) 
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.44269504f * alpha))) * u;
 }
 
-template <int BK, int NST, int WM, int WN, int TM, int TN, bool DUAL>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wk, const bf16_t* __restrict__ wk2,
-                                                                 int M, int K, int Npad, int NT, int MT, int splits, float* __restrict__ part, TileEpilogue epi) {
-    static_assert(BK == 32 || BK == 64, "k tile");
-    constexpr int KG = BK / 8, ROWB = BK * 2, KS = BK / 16;            // k-groups, bytes of an A row, k-steps
+template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __restrict__ x, const T* __restrict__ wk, const T* __restrict__ wk2,
+                                                                 int M, int K, int Npad, int NT, int MT, int splits, float* __restrict__ part, TileEpilogue<T> epi) {
+    static_assert(KG == 4 || KG == 8, "k-groups of a k tile");
+    typedef typename Mma<T>::frag frag_t;
+    constexpr int BK = KG * Mma<T>::KPC, ROWB = KG * 16, KS = KG / 2;  // k of a tile, bytes of an A row, k-steps
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NW = WM * WN;
     constexpr int NREAL = DUAL ? BN / 2 : BN;                          // output columns per tile
     constexpr int TNO = DUAL ? TN / 2 : TN;                            // output fragments per wave and row
@@ -661,7 +666,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* _
         bx = (v % gsz) / gm;
     }
     const int m0 = by * BM, n0 = bx * NREAL;
-    auto swz = [](int row) { return BK == 64 ? (row >> 1) & 7 : (row >> 2) & 3; };
+    auto swz = [](int row) { return KG == 8 ? (row >> 1) & 7 : (row >> 2) & 3; };
     // what each of this wave's load instructions fetches, per lane
     unsigned a_off[LA], b_off[LB];
     unsigned long long b_base[LB];
@@ -670,7 +675,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* _
         const int sl = (wave * LA + j) * 64 + lane, row = sl / KG, pos = sl % KG;
         int m = m0 + row;
         if (m > M - 1) m = M - 1;
-        a_off[j] = (unsigned)((m - m0) * K * 2 + ((pos ^ swz(row)) * 16));   // under 256 rows of K bf16: fits 32 bits (K <= 2^22)
+        a_off[j] = (unsigned)(m - m0) * (unsigned)(K * sizeof(T)) + (unsigned)((pos ^ swz(row)) * 16);   // under 256 rows: fits 32 bits (K <= 2^21)
     }
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
@@ -687,7 +692,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* _
     const int nt = (int)((int64_t)(sidx + 1) * kt_all / splits) - kt0;   // this workgroup's k tiles: [kt0, kt0 + nt)
     auto issue = [&](int t, int st) {
         if (t >= nt) return;
-        const unsigned long long ab = gemm_uniform64(a_base + (unsigned long long)(t + kt0) * (BK * 2));
+        const unsigned long long ab = gemm_uniform64(a_base + (unsigned long long)(t + kt0) * ROWB);
         const unsigned long long bt = (unsigned long long)((t + kt0) * b_tile_step);
         const unsigned sbase = lds0 + st * STAGE;
 #pragma unroll
@@ -704,17 +709,17 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* _
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
     const int fsel = lane >> 5;
     const int b_rd = A_BYTES + (wn * 32 * TNO + (lane & 31)) * 16;
-    bf16x8_t af[2][TM], bfr[2][TN];
+    frag_t af[2][TM], bfr[2][TN];
     auto fread = [&](int st, int kk, int slot) {   // kk: k-step of the tile
         const unsigned char* base = lds + st * STAGE;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             const int row = wm * 32 * TM + i * 32 + (lane & 31), kg = 2 * kk + fsel;
-            af[slot][i] = *reinterpret_cast<const bf16x8_t*>(base + row * ROWB + ((kg ^ swz(row)) * 16));
+            af[slot][i] = *reinterpret_cast<const frag_t*>(base + row * ROWB + ((kg ^ swz(row)) * 16));
         }
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-            bfr[slot][j] = *reinterpret_cast<const bf16x8_t*>(base + b_rd + (2 * kk + fsel) * (BN * 16) + (DUAL ? (j / TNO) * (NREAL * 16) : 0) + (j % TNO) * 512);
+            bfr[slot][j] = *reinterpret_cast<const frag_t*>(base + b_rd + (2 * kk + fsel) * (BN * 16) + (DUAL ? (j / TNO) * (NREAL * 16) : 0) + (j % TNO) * 512);
     };
     for (int st = 0; st < NST - 1; ++st) issue(st, st);
     if (nt >= NST - 1) gemm_wait_loads<(NST - 2) * LPT>();
@@ -733,7 +738,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* _
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    if (i * TN + j >= i0 && i * TN + j < i1) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[slot][i], bfr[slot][j], acc[i][j], 0, 0, 0);
+                    if (i * TN + j >= i0 && i * TN + j < i1) acc[i][j] = Mma<T>::mma(af[slot][i], bfr[slot][j], acc[i][j]);
             __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -801,7 +806,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* _
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 float o = acc[i][j][v];
-                if (DUAL) o = gemm_glu(o, acc[i][DUAL ? j + TNO : j][v], epi.extra.glu);   // activation.rs:141-162
+                if (DUAL) o = gemm_glu<T>(o, acc[i][DUAL ? j + TNO : j][v], epi.extra.glu);   // activation.rs:141-162
                 area[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * RSF + j * 32 + (lane & 31)] = o;
             }
 #pragma unroll 1
@@ -816,8 +821,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const bf16_t* _
 // Adds the partial sums of a launch whose tiles were split over k, in split order (the result does not depend on which
 // workgroup ended first), and finishes the outputs.  One thread per 8 outputs.  A launch of its own over the whole chip:
 // with the last workgroup of a tile adding them, 48 tiles of M = 333 kept 48 CUs busy reading while 208 waited.
-template <bool DUAL>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int M, int splits, TileEpilogue epi) {
+template <typename T, bool DUAL>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int M, int splits, TileEpilogue<T> epi) {
     const int np = ((int)epi.N + 7) & ~7, chunks = np / 8, width = DUAL ? 2 * np : np;
     const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (id >= (int64_t)M * chunks) return;
@@ -839,7 +844,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
         float u[8];
         sum8(part + m * width + np + n, u);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = gemm_glu(o[e], u[e], epi.extra.glu);   // activation.rs:141-162
+        for (int e = 0; e < 8; ++e) o[e] = gemm_glu<T>(o[e], u[e], epi.extra.glu);   // activation.rs:141-162
     }
     gemm_finish8(epi, m, n, o);
 }
@@ -848,23 +853,23 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
 enum TileId { kT256x256, kT256x192, kT128x256, kT128x128, kT64x256, kT64x128, kTiles };
 struct TilePlan { int tile; int splits; };
 
-template <int BK, int NST, int WM, int WN, int TM, int TN, bool DUAL>
+template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL>
 static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
-    constexpr int ring = NST * (BM + BN) * BK * 2, rows = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4;
+    constexpr int ring = NST * (BM + BN) * KG * 16, rows = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4;
     constexpr int lds_bytes = ring > rows ? ring : rows;
     static_assert(lds_bytes <= 160 * 1024, "LDS of one CU");
-    auto kern = gemm_tile_kernel<BK, NST, WM, WN, TM, TN, DUAL>;
+    auto kern = gemm_tile_kernel<T, KG, NST, WM, WN, TM, TN, DUAL>;
     static bool configured = false;  // the attribute is per function, not per stream or device state
     if (!configured) {
         (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         configured = true;
     }
     const int64_t nt = cdiv(a.n, NREAL), mt = cdiv(a.m, BM);
-    TileEpilogue epi{(const bf16_t*)a.bias, a.residual, a.y, a.n, a.act, a.out_f32, a.extra};
-    kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN, lds_bytes, s>>>((const bf16_t*)a.x, (const bf16_t*)a.wk, (const bf16_t*)a.wk2, (int)a.m, (int)a.k,
+    TileEpilogue<T> epi{(const T*)a.bias, a.residual, a.y, a.n, a.act, a.out_f32, a.extra};
+    kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (int)a.m, (int)a.k,
                                                                                    (int)mfma_padded_n(a.n), (int)nt, (int)mt, splits, (float*)a.part, epi);
-    if (splits > 1) gemm_reduce_kernel<DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
+    if (splits > 1) gemm_reduce_kernel<T, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
 }
 static size_t tile_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
     return splits > 1 ? (size_t)splits * m * cdiv(n, 8) * 8 * (dual ? 2 : 1) * sizeof(float) : 0;
@@ -900,17 +905,36 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual) {
 }
 template <bool DUAL>
 static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p) {
+    typedef bf16_t T;
     if (p.splits > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, DUAL, p.splits))) p.splits = 1;
     switch (p.tile) {
-        case kT256x256: return launch_tile<32, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits);
-        case kT256x192: if constexpr (!DUAL) return launch_tile<64, 2, 4, 2, 2, 3, false>(s, a, p.splits); else return;
-        case kT128x256: return launch_tile<64, 3, 2, 4, 2, 2, DUAL>(s, a, p.splits);
+        case kT256x256: return launch_tile<T, 4, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits);
+        case kT256x192: if constexpr (!DUAL) return launch_tile<T, 8, 2, 4, 2, 2, 3, false>(s, a, p.splits); else return;
+        case kT128x256: return launch_tile<T, 8, 3, 2, 4, 2, 2, DUAL>(s, a, p.splits);
         case kT128x128:
-            if constexpr (DUAL) return launch_tile<64, 4, 4, 2, 1, 2, true>(s, a, p.splits);
-            else return launch_tile<64, 4, 2, 4, 2, 1, false>(s, a, p.splits);
-        case kT64x256: return launch_tile<64, 3, 2, 4, 1, 2, DUAL>(s, a, p.splits);
-        default: return launch_tile<64, 3, 2, 2, 1, 2, DUAL>(s, a, p.splits);
+            if constexpr (DUAL) return launch_tile<T, 8, 4, 4, 2, 1, 2, true>(s, a, p.splits);
+            else return launch_tile<T, 8, 4, 2, 4, 2, 1, false>(s, a, p.splits);
+        case kT64x256: return launch_tile<T, 8, 3, 2, 4, 1, 2, DUAL>(s, a, p.splits);
+        default: return launch_tile<T, 8, 3, 2, 2, 1, 2, DUAL>(s, a, p.splits);
     }
+}
+
+// f32: one tile, 64 x 64 outputs in 4 waves of 32 x 32 (a pair: 64 x 64 of each matrix), three workgroups to a CU.  The f32
+// products are paced by the matrix pipes alone, 0.43 us for a k tile of 32 on a CU, one wave per SIMD is enough to keep them
+// busy, and the small tile divides best among the CUs: M = 8192, K = 768, N = 3072 297 us = 130 TFLOP/s (64 x 128 304, 128 x 128
+// 316, 256 x 256 396), K = 3072, N = 768 273 = 141 (274, 354, 350); the register-staged 128 x 128 tiles took 366 and 354.
+// M = 400 (K = 768, N = 2304): 18 us (64 x 128 26).  Splits over k: rounds of 256 workgroups, a launch more and its bytes.
+static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual) {
+    const int64_t tiles = cdiv(m, 64) * cdiv(n, 64);
+    int best = 1;
+    double least = 1e300;
+    for (int sp : {1, 2, 3, 4, 6, 8}) {
+        if (sp > 1 && (k < 128 * sp || tile_part_bytes(m, n, dual, sp) > (64u << 20))) break;
+        double us = 5.0 + (dual ? 0.88 : 0.44) * ((double)k / 32 / sp) * (double)cdiv(tiles * sp, 256);
+        if (sp > 1) us += 3.5 + 0.4 * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
+        if (us < least) { least = us; best = sp; }
+    }
+    return best;
 }
 
 bool mfma_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n, int quant) {
@@ -947,6 +971,7 @@ static int mfma_few_tiles_split(int64_t tiles64, int64_t k_tiles) {
 }
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant) {
     if (!mfma_gemm_supported(dtype, m, k, n, quant)) return 0;
+    if (dtype == 0) return tile_part_bytes(m, n, dual, tile_splits_f32(m, k, n, dual));
     const int64_t k_tiles = k / (kKb * kpc_of(dtype));
     int sp = 1;
     size_t bytes = 0;
@@ -959,7 +984,7 @@ size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dua
         const int64_t full = mfma_tail_plan(tiles, k_tiles, &sp);
         if (sp > 1) bytes = (size_t)(tiles - full) * sp * 128 * 128 * sizeof(float);
     }
-    if (dtype == 2 && quant == 0) bytes = std::max(bytes, tile_part_bytes(m, n, dual, tile_plan(m, k, n, dual).splits));   // the LDS-direct kernel
+    if (quant == 0) bytes = std::max(bytes, tile_part_bytes(m, n, dual, tile_plan(m, k, n, dual).splits));   // the LDS-direct kernel
     return bytes;
 }
 
@@ -1000,6 +1025,9 @@ void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
     const bool small = tiles < 128;
     static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_KSPLIT"); return !(e && e[0] == '0'); }();
     const bool split = allow_split && !a.wk2 && !small && tiles <= 256;
+    // the LDS-direct kernel's loads address a k tile with 32-bit offsets from one scalar base: 256 rows of x, 8 k-groups of
+    // the padded weights
+    const bool reach = a.k <= (1 << 21) && (uint64_t)mfma_padded_n(a.n) * 128 < (1ull << 31);
     if (a.quant == 1) {
         if (a.wk2) launch_mfma<bf16_t, 128, 128, true, 1>(s, a);
         else if (small) launch_mfma<bf16_t, 64, 64, false, 1>(s, a);
@@ -1011,14 +1039,13 @@ void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
         else if (split) launch_mfma<bf16_t, 128, 128, false, 2, 2>(s, a);
         else launch_mfma<bf16_t, 128, 128, false, 2>(s, a);
     } else if (a.dtype == 0) {
-        if (a.wk2) launch_mfma<float, 128, 128, true>(s, a);
-        else if (small) launch_mfma<float, 64, 64, false>(s, a);
-        else if (split) launch_mfma<float, 128, 128, false, 0, 2>(s, a);
-        else launch_mfma<float, 128, 128, false>(s, a);
+        if (!reach) return a.wk2 ? launch_mfma<float, 128, 128, true>(s, a) : launch_mfma<float, 128, 128, false>(s, a);
+        int sp = tile_splits_f32(a.m, a.k, a.n, a.wk2 != nullptr);
+        if (sp > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, a.wk2 != nullptr, sp))) sp = 1;
+        if (a.wk2) launch_tile<float, 8, 3, 2, 2, 1, 2, true>(s, a, sp);
+        else launch_tile<float, 8, 3, 2, 2, 1, 1, false>(s, a, sp);
     } else {
-        // unquantised bf16: the LDS-direct kernel, on the tiles tile_plan() picks; its loads address a k tile with 32-bit
-        // offsets from one scalar base: 256 rows of x, 8 k-groups of the padded weights
-        const bool reach = a.k <= (1 << 22) && (uint64_t)mfma_padded_n(a.n) * 128 < (1ull << 31);
+        // unquantised bf16: the LDS-direct kernel, on the tiles tile_plan() picks
         if (a.lds_direct != 0 && reach) {
             const TilePlan p = tile_plan(a.m, a.k, a.n, a.wk2 != nullptr);
             return a.wk2 ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);

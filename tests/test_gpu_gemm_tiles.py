@@ -58,3 +58,33 @@ def test_tiles_and_splits(hip, m, k, n):
     assert (np.abs(got[2][rows] - s * sig * t) <= pair).all()
     for a, b in zip(got, staged):           # two orders of the same sums, one rounding apart in bf16
         assert (np.abs(a - b) <= 2.0 ** -6 * np.maximum(np.abs(a), np.abs(b)) + 4e-4 * np.sqrt(k) / 16).all()
+
+
+# the same kernel in f32 (64 x 64 tiles): tile edges, columns that are no multiple of 8, one k tile, splits that do not divide k
+@pytest.mark.parametrize("m,k,n", [(17, 32, 8), (40, 768, 41), (63, 96, 130), (65, 3072, 768), (129, 800, 2307), (300, 4096, 192), (700, 256, 3072)])
+def test_f32_tiles_and_splits(hip, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    x, w, w2 = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (k, n), (k, n)))
+    w, w2 = w * np.float32(k ** -0.5), w2 * np.float32(k ** -0.5)
+    bias, res = rng.standard_normal(n, dtype=np.float32), rng.standard_normal((m, n), dtype=np.float32)
+    f32, mat = "F32", ("F32", [k, n])
+
+    def run(specs, body, args):
+        fb = FunctionBuilder("main", f32)
+        fb.set_results([body(*[fb.param(dt, dims) for dt, dims in specs])])
+        p = Program(fb)
+        got = hip_run(hip, p, args)[0]
+        assert np.array_equal(got, hip_run(hip, p, args)[0])
+        return got
+
+    plain = run([(f32, [m, k]), mat, (f32, [m, n])], lambda a, b, r: F.linear(a, b) + r, [x, w, res])
+    biased = run([(f32, [m, k]), mat, (f32, [n])], lambda a, b, c: F.linear(a, b, c), [x, w, bias])
+    pair = run([(f32, [m, k]), mat, mat], lambda a, b, c: F.swiglu(F.linear(a, b), F.linear(a, c)), [x, w, w2])
+    x64, w64, v64 = x.astype(np.float64), w.astype(np.float64), w2.astype(np.float64)
+    s, t = x64 @ w64, x64 @ v64
+    # as above: 2 sqrt(k) roundings of the sum of magnitudes, and one for each operation behind the sum
+    bs, bt = (2 * np.sqrt(k) * 2.0 ** -24 * (np.abs(x64) @ np.abs(v)) + 1e-6 for v in (w64, v64))
+    assert (np.abs(plain - (s + res)) <= bs + 2.0 ** -23 * np.abs(s + res)).all()
+    assert (np.abs(biased - (s + bias)) <= bs + 2.0 ** -23 * np.abs(s + bias)).all()
+    g = s / (1 + np.exp(-s))
+    assert (np.abs(pair - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + 2.0 ** -20 * np.abs(g * t) + 1e-6).all()
