@@ -22,7 +22,7 @@ TAG_DTYPE = {v: k for k, v in DTYPE_TAG.items()}
 NP_OF = {"F32": np.float32, "Si32": np.int32, "I1": np.uint8, "Bf16": np.uint16, "Si8": np.int8, "Ui8": np.uint8}
 
 EXPORTS = [
-    "gptrs_hip_create", "gptrs_hip_destroy", "gptrs_hip_backend_name", "gptrs_hip_materialize",
+    "gptrs_hip_create", "gptrs_hip_destroy", "gptrs_hip_backend_name", "gptrs_hip_materialize", "gptrs_hip_materialize_zeros",
     "gptrs_hip_to_literal", "gptrs_hip_tensor_retain", "gptrs_hip_tensor_release", "gptrs_hip_tensor_spec",
     "gptrs_hip_run_program", "gptrs_hip_run_program_donate", "gptrs_hip_execute_instruction",
     "gptrs_hip_param_get", "gptrs_hip_param_set", "gptrs_hip_supports_decode_sampling",
@@ -65,6 +65,7 @@ def load_library(path: str = LIB_PATH):
     lib.gptrs_hip_backend_name.argtypes = [vp]
     lib.gptrs_hip_backend_name.restype = cp
     lib.gptrs_hip_materialize.argtypes = [vp, ctypes.POINTER(_Desc), vp, sz, pvp]
+    lib.gptrs_hip_materialize_zeros.argtypes = [vp, ctypes.POINTER(_Desc), sz, pvp]
     lib.gptrs_hip_to_literal.argtypes = [vp, vp, vp, sz]
     lib.gptrs_hip_tensor_retain.argtypes = [vp]
     lib.gptrs_hip_tensor_retain.restype = None
@@ -199,6 +200,13 @@ class HipBackend:
                 buf = bytes(data)
                 self._check(self._lib.gptrs_hip_materialize(self._handle, ctypes.byref(desc), buf, len(buf), ctypes.byref(out)))
         return TensorHandle(self, out.value, spec)
+
+    def materialize_zeros(self, spec: TensorSpec, n: int) -> List[TensorHandle]:
+        """`n` tensors of zeros of one spec (TensorInit::Zeroed n times, in one call)."""
+        dims = (ctypes.c_int64 * max(len(spec.dims), 1))(*spec.dims)
+        outs = (ctypes.c_void_p * max(n, 1))()
+        self._check(self._lib.gptrs_hip_materialize_zeros(self._handle, ctypes.byref(_Desc(DTYPE_TAG[spec.dtype], len(spec.dims), dims)), n, outs))
+        return [TensorHandle(self, p, spec) for p in outs[:n]]
 
     def to_literal(self, handle: TensorHandle) -> bytes:
         n = handle.spec.byte_len()

@@ -112,6 +112,7 @@ Backend::Backend(int dev) : device(dev) {
 
 Backend::~Backend() {
     (void)hipSetDevice(device);
+    n_fresh_zero_ = n_fresh_small_ = 0;
     if (stream) (void)hipStreamSynchronize(stream);
     try { profile_collect(); } catch (...) {}
     for (auto& kv : params_) release_handle_locked(kv.second);
@@ -292,6 +293,7 @@ void Backend::evict_packed_sources(const Plan& plan, gptrs_hip_tensor* const* in
 // family (the prefill copies once a server only decodes) gets their memory back here, the layouts still in use are
 // rebuilt by the next call that needs them.
 void Backend::drop_derived_weights() {
+    flush_fresh();
     GPTRS_HIP_CHECK(hipStreamSynchronize(stream));
     for (auto& kv : plan_lru_) {
         Plan& p = *kv.second;
@@ -348,6 +350,28 @@ const k::ChainPhase* Backend::chain_table(const std::vector<k::ChainPhase>& phas
     return (const k::ChainPhase*)chain_tables_.back().dev->ptr;
 }
 
+void Backend::flush_fresh() {
+    const int zeros = n_fresh_zero_, smalls = n_fresh_small_;
+    n_fresh_zero_ = n_fresh_small_ = 0;
+    k::fill_zero_many(stream, fresh_zero_, zeros);
+    k::store_small(stream, fresh_small_, smalls);
+}
+void Backend::forget_fresh(const void* p) {
+    for (int i = 0; i < n_fresh_zero_;) {
+        if (fresh_zero_.dst[i] != p) { ++i; continue; }
+        --n_fresh_zero_;
+        fresh_zero_.dst[i] = fresh_zero_.dst[n_fresh_zero_];
+        fresh_zero_.bytes[i] = fresh_zero_.bytes[n_fresh_zero_];
+    }
+    for (int i = 0; i < n_fresh_small_;) {
+        if (fresh_small_.dst[i] != p) { ++i; continue; }
+        --n_fresh_small_;
+        fresh_small_.payload[i] = fresh_small_.payload[n_fresh_small_];
+        fresh_small_.dst[i] = fresh_small_.dst[n_fresh_small_];
+        fresh_small_.bytes[i] = fresh_small_.bytes[n_fresh_small_];
+    }
+}
+
 gptrs_hip_tensor* Backend::materialize(const Spec& spec, const void* host, size_t nbytes) {
     GPTRS_HIP_CHECK(hipSetDevice(device));
     const size_t want = spec.bytes();
@@ -358,12 +382,14 @@ gptrs_hip_tensor* Backend::materialize(const Spec& spec, const void* host, size_
         t->buf = new_buffer(want);
         if (!want) return t;
         if (!host) {
-            k::fill_zero(stream, t->buf->ptr, want);
+            fresh_zero_.dst[n_fresh_zero_] = (uint8_t*)t->buf->ptr;
+            fresh_zero_.bytes[n_fresh_zero_] = want;
+            if (++n_fresh_zero_ == k::ZeroBatch::kMost) flush_fresh();
         } else if (want <= sizeof(k::SmallPayload)) {
-            k::SmallPayload p;
-            memset(&p, 0, sizeof(p));
-            memcpy(p.w, host, want);
-            k::store_small(stream, t->buf->ptr, p, (int)want);
+            memcpy(fresh_small_.payload[n_fresh_small_].w, host, want);
+            fresh_small_.dst[n_fresh_small_] = (uint8_t*)t->buf->ptr;
+            fresh_small_.bytes[n_fresh_small_] = (int)want;
+            if (++n_fresh_small_ == k::SmallBatch::kMost) flush_fresh();
         } else {
             // pageable source: the copy is staged by the runtime; wait so the caller may reuse `host`
             GPTRS_HIP_CHECK(hipMemcpyAsync(t->buf->ptr, host, want, hipMemcpyHostToDevice, stream));
@@ -401,8 +427,9 @@ void Backend::check_device_errors() {
 }
 
 void Backend::to_literal(const gptrs_hip_tensor* t, void* dst, size_t cap) {
-    realize(t);
     GPTRS_HIP_CHECK(hipSetDevice(device));
+    flush_fresh();
+    realize(t);
     if (t->consumed) fail_exec("tensor handle was donated to run_program and can no longer be read");
     const size_t n = t->spec.bytes();
     if (cap < n) fail_exec("to_literal destination too small");
@@ -414,6 +441,7 @@ void Backend::to_literal(const gptrs_hip_tensor* t, void* dst, size_t cap) {
 
 void Backend::synchronize() {
     GPTRS_HIP_CHECK(hipSetDevice(device));
+    flush_fresh();
     GPTRS_HIP_CHECK(hipStreamSynchronize(stream));
     check_device_errors();
 }
@@ -437,6 +465,7 @@ void Backend::param_set(const std::array<uint8_t, 16>& id, gptrs_hip_tensor* t) 
 
 bool Backend::queue_sampling(const gptrs_hip_tensor* logits, float temperature, bool has_top_k, bool has_u, float u) {
     GPTRS_HIP_CHECK(hipSetDevice(device));
+    flush_fresh();
     if (logits->consumed) fail_exec("tensor handle was donated to run_program and can no longer be read");
     realize(logits);
     const Spec& s = logits->spec;
@@ -478,6 +507,7 @@ int64_t Backend::sample_begin(const gptrs_hip_tensor* logits, float temperature,
 
 int64_t Backend::sample_rows_begin(const gptrs_hip_tensor* logits) {
     GPTRS_HIP_CHECK(hipSetDevice(device));
+    flush_fresh();
     if (logits->consumed) fail_exec("tensor handle was donated to run_program and can no longer be read");
     realize(logits);
     const Spec& s = logits->spec;
@@ -499,6 +529,7 @@ int64_t Backend::sample_rows_begin(const gptrs_hip_tensor* logits) {
 // The allocation-free variant of sample_rows_begin: kernels only, partial maxima in the library's fixed device array.
 void Backend::sample_rows_into(const gptrs_hip_tensor* logits, gptrs_hip_tensor* tokens_out) {
     GPTRS_HIP_CHECK(hipSetDevice(device));
+    flush_fresh();
     if (logits->consumed || tokens_out->consumed) fail_exec("tensor handle was donated to run_program and can no longer be used");
     realize(logits);
     realize(tokens_out);
@@ -941,6 +972,7 @@ void Backend::tag_broadcast_result(const Plan& plan, size_t r, gptrs_hip_tensor*
 void Backend::run_program(const char* json, size_t len, uint64_t key, gptrs_hip_tensor* const* inputs,
                           const uint8_t* donate, size_t n_in, gptrs_hip_tensor** outputs, size_t n_out) {
     GPTRS_HIP_CHECK(hipSetDevice(device));
+    flush_fresh();
     auto plan = get_plan(json, len, key, inputs, donate, n_in);
     if (plan->fn.result_ids.size() != n_out)
         fail_exec("program produces " + std::to_string(plan->fn.result_ids.size()) + " results but " + std::to_string(n_out) + " were requested");
@@ -1029,6 +1061,21 @@ int gptrs_hip_materialize(gptrs_hip_backend* b, const gptrs_hip_tensor_desc* des
         const gptrs::Spec s = spec_from_desc(desc);
         std::lock_guard<std::mutex> g(b->impl.mu);
         *out = b->impl.materialize(s, host_bytes, nbytes);
+    });
+}
+
+int gptrs_hip_materialize_zeros(gptrs_hip_backend* b, const gptrs_hip_tensor_desc* desc, size_t n, gptrs_hip_tensor** outs) {
+    return guarded([&] {
+        if (!b || (n && !outs)) gptrs::fail_exec("null argument");
+        const gptrs::Spec s = spec_from_desc(desc);
+        std::lock_guard<std::mutex> g(b->impl.mu);
+        size_t done = 0;
+        try {
+            for (; done < n; ++done) outs[done] = b->impl.materialize(s, nullptr, 0);
+        } catch (...) {
+            while (done > 0) gptrs::release_handle_locked(outs[--done]);
+            throw;
+        }
     });
 }
 

@@ -30,8 +30,11 @@ void copy_strided(hipStream_t s, void* dst, const void* src, int elem_size, cons
 // Up to 256 payload bytes travel as kernel arguments: an upload with no staging buffer and
 // no host synchronisation (token ids, positions, update_starts, RoPE rows).
 struct SmallPayload { uint32_t w[64]; };
-void store_small(hipStream_t s, void* dst, const SmallPayload& p, int nbytes);
+struct SmallBatch { static constexpr int kMost = 8; SmallPayload payload[kMost]; uint8_t* dst[kMost]; int bytes[kMost]; };
+void store_small(hipStream_t s, const SmallBatch& b, int count);
 void fill_zero(hipStream_t s, void* dst, size_t nbytes);
+struct ZeroBatch { static constexpr int kMost = 64; uint8_t* dst[kMost]; size_t bytes[kMost]; };
+void fill_zero_many(hipStream_t s, const ZeroBatch& b, int count);
 
 // dtype: 0 f32, 2 bf16 (tags of include/gptrs_hip.h).  Math in f32, output rounded to dtype.
 void unary(hipStream_t s, int dtype, int op, const void* x, void* y, int64_t n);

@@ -65,25 +65,39 @@ void copy_strided(hipStream_t s, void* dst, const void* src, int elem_size, cons
     }
 }
 
-__global__ void store_small_kernel(uint8_t* dst, SmallPayload p, int nbytes) {
-    const int i = threadIdx.x;
-    if (i < nbytes) dst[i] = ((const uint8_t*)p.w)[i];
+__global__ void store_small_kernel(SmallBatch b) {
+    const int e = blockIdx.x, i = threadIdx.x;
+    if (i < b.bytes[e]) b.dst[e][i] = ((const uint8_t*)b.payload[e].w)[i];
 }
-void store_small(hipStream_t s, void* dst, const SmallPayload& p, int nbytes) {
-    if (nbytes <= 0) return;
-    store_small_kernel<<<1, 256, 0, s>>>((uint8_t*)dst, p, nbytes);
+void store_small(hipStream_t s, const SmallBatch& b, int count) {
+    if (count > 0) store_small_kernel<<<count, 256, 0, s>>>(b);
 }
 
-__global__ void fill_zero_kernel(uint4* dst, int64_t n16, uint8_t* tail, int ntail) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i] = make_uint4(0, 0, 0, 0);
-    if (blockIdx.x == 0 && (int)threadIdx.x < ntail) tail[threadIdx.x] = 0;
+__device__ __forceinline__ void fill_zero_range(uint8_t* dst, size_t nbytes, int64_t first, int64_t step) {
+    uint4* d16 = reinterpret_cast<uint4*>(dst);
+    const int64_t n16 = (int64_t)(nbytes / 16);
+    for (int64_t i = first; i < n16; i += step) d16[i] = make_uint4(0, 0, 0, 0);
+    const int64_t tail = (int64_t)(nbytes % 16);
+    if (first < tail) dst[n16 * 16 + first] = 0;
+}
+__global__ void fill_zero_kernel(uint8_t* dst, size_t nbytes) {
+    fill_zero_range(dst, nbytes, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int64_t)gridDim.x * blockDim.x);
 }
 void fill_zero(hipStream_t s, void* dst, size_t nbytes) {
     if (!nbytes) return;
-    const int64_t n16 = (int64_t)(nbytes / 16);
-    fill_zero_kernel<<<grid_for(n16 ? n16 : 1, 256, 8192), 256, 0, s>>>((uint4*)dst, n16, (uint8_t*)dst + n16 * 16,
-                                                                          (int)(nbytes % 16));
+    fill_zero_kernel<<<grid_for(nbytes / 16 ? (int64_t)(nbytes / 16) : 1, 256, 8192), 256, 0, s>>>((uint8_t*)dst, nbytes);
+}
+// Many fresh tensors in one launch (grid.y = tensor): a prompt of 16 sequences through 12 layers starts from 384 zeroed caches,
+// 2.2 us each as launches of their own and more than that for the host to queue them.
+__global__ void fill_zero_many_kernel(ZeroBatch b) {
+    fill_zero_range(b.dst[blockIdx.y], b.bytes[blockIdx.y], (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int64_t)gridDim.x * blockDim.x);
+}
+void fill_zero_many(hipStream_t s, const ZeroBatch& b, int count) {
+    if (count <= 0) return;
+    size_t most = 0;
+    for (int i = 0; i < count; ++i) most = b.bytes[i] > most ? b.bytes[i] : most;
+    const int64_t blocks = (int64_t)(most / 16 + 1023) / 1024;   // four stores a thread
+    fill_zero_many_kernel<<<dim3((unsigned)(blocks < 1 ? 1 : blocks > 1024 ? 1024 : blocks), (unsigned)count), 256, 0, s>>>(b);
 }
 
 // ------------------------------------------------------------------------------ elementwise

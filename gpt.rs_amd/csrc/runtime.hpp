@@ -241,7 +241,14 @@ class Backend {
     bool chain_stall_fired = false;   // such a launch has been queued and its time-out not yet reported
     int64_t n_chain_launches = 0, n_chain_phases = 0;
     int64_t n_tiled_built = 0;
-    void release_block(void* p, size_t cap) { pool_.release(p, cap); }
+    void release_block(void* p, size_t cap) {
+        if (n_fresh_zero_ + n_fresh_small_) forget_fresh(p);   // the block may have another owner before the next flush
+        pool_.release(p, cap);
+    }
+    // Fresh tensors of zeros and small uploads are written by one launch for many of them: materialize() notes them here, and
+    // whatever puts other work on the stream (or waits for it) flushes first.
+    void flush_fresh();
+    void forget_fresh(const void* p);
     void note_dead_source() { dead_sources_.fetch_add(1, std::memory_order_relaxed); }
 
     std::mutex mu;
@@ -273,6 +280,9 @@ class Backend {
     bool run_graphed(Plan& plan, ExecCtx& cx, const std::vector<BufferP>& out_bufs);
 
     DevicePool pool_;
+    k::ZeroBatch fresh_zero_;
+    k::SmallBatch fresh_small_;
+    int n_fresh_zero_ = 0, n_fresh_small_ = 0;
     std::unordered_map<std::array<uint8_t, 16>, gptrs_hip_tensor*, IdHash> params_;
     std::list<std::pair<uint64_t, std::shared_ptr<Plan>>> plan_lru_;
     std::unordered_map<uint64_t, std::list<std::pair<uint64_t, std::shared_ptr<Plan>>>::iterator> plan_index_;

@@ -260,6 +260,12 @@ class _ModelBase:
     def _zeros(self, dims, dtype: Optional[str] = None):
         return self.backend.materialize(TensorSpec(dtype or self.dtype, dims), None)
 
+    def _zeros_many(self, dims, n: int) -> list:
+        """n zero tensors in the model dtype."""
+        spec = TensorSpec(self.dtype, dims)
+        many = getattr(self.backend, "materialize_zeros", None)
+        return many(spec, n) if many is not None else [self.backend.materialize(spec, None) for _ in range(n)]
+
     def _grow_rows(self, handle, dims, capacity: int):
         """A cache tensor of shape `dims` = [heads, old capacity, width] copied into a zero tensor of `capacity` rows
         (model/gpt.rs:626-657)."""
@@ -575,7 +581,7 @@ class Gpt(_ModelBase):
         else:
             hkv, dh = self.attn.num_key_value_heads, self.attn.kv_head_dim
             args.append(self._upload_i32([0, 0, 0]))
-            kv = [self._zeros([hkv, capacity, dh]) for _ in range(2 * L * batch)]
+            kv = self._zeros_many([hkv, capacity, dh], 2 * L * batch)
         donate = [False] * len(args) + [True] * len(kv)       # old caches are dropped (gpt.rs:738-747)
         outs = self._run(prog, args + kv, donate)
         it = iter(outs[:-1])
@@ -907,7 +913,7 @@ class Ministral(_ModelBase):
         else:
             hkv, dh = self.attn.num_key_value_heads, self.attn.kv_head_dim
             args.append(self._upload_i32([0, 0, 0]))
-            kv = [self._zeros([hkv, capacity, dh]) for _ in range(2 * L * batch)]
+            kv = self._zeros_many([hkv, capacity, dh], 2 * L * batch)
         donate = [False] * len(args) + [True] * len(kv)
         outs = self._run(prog, args + kv, donate)
         it = iter(outs[:-1])

@@ -64,6 +64,8 @@ const char* gptrs_hip_backend_name(const gptrs_hip_backend* b);
  * TensorInit::Zeroed when it is NULL. */
 int gptrs_hip_materialize(gptrs_hip_backend* b, const gptrs_hip_tensor_desc* desc,
                           const void* host_bytes, size_t nbytes, gptrs_hip_tensor** out);
+/* n tensors of one spec, all zeros: what n calls with host_bytes NULL give (the caches a prompt starts from). */
+int gptrs_hip_materialize_zeros(gptrs_hip_backend* b, const gptrs_hip_tensor_desc* desc, size_t n, gptrs_hip_tensor** outs);
 
 /* PortableBackend::to_literal (spec.rs:1314): copies the tensor to host memory.
  * cap must be at least the tensor's byte length. */
