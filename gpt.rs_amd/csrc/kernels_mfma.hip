@@ -81,8 +81,8 @@ void mfma_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int64
 }
 
 // Weight-only quantised weights (bf16 activations): the GEMM reads the CODES, in the same k-grouped order, and turns
-// them into the bf16 values of the dequantised matrix, bf16(code * scale), on the way into LDS; no dequantised copy
-// exists.  Ck[kb][n] holds the 8 codes of k-group kb of column n with the sign bias added (int8: 8 bytes of q + 128;
+// them into the bf16 values of the dequantised matrix, bf16(code * scale), on the way to the matrix pipes; no dequantised
+// copy exists.  Ck[kb][n] holds the 8 codes of k-group kb of column n with the sign bias added (int8: 8 bytes of q + 128;
 // int4: one dword, nibble i = q(k = 8 kb + i) + 8), so a code converts with one unsigned-byte / bit-field instruction
 // and one fma (u * s - bias * s is exactly (u - bias) * s, rounded once like the product the dequantiser forms).
 // Padding (n >= N, k >= K) holds the code of zero.
@@ -133,8 +133,20 @@ __device__ __forceinline__ uint32_t mfma_pack_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));   // round to nearest even
 }
 
-__device__ __forceinline__ float mfma_finish(float v, float v2, bool dual, int act, float bias, bool has_res, float res, const GluParams& glu, float colscale) {
-    if (dual) v = glu_combine(v, v2, glu.kind, glu.limit, glu.alpha, glu.shift);   // activation.rs:141-162
+// The pair's gate on the hardware's exp2 and reciprocal (1 ulp each of f32; the result goes on as bf16): the exact division
+// and expf of glu_combine are 40 instructions an output, 9 us of a 256 x 256 tile's 85.
+template <typename T>
+__device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) {
+    if (std::is_same<T, float>::value) return glu_combine(g, u, p.kind, p.limit, p.alpha, p.shift);
+    const float alpha = p.kind == 1 ? p.alpha : 1.0f;
+    if (p.kind == 1) {
+        g = fminf(g, p.limit);
+        u = fminf(fmaxf(u, -p.limit), p.limit) + p.shift;
+    }
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.44269504f * alpha))) * u;
+}
+
+__device__ __forceinline__ float mfma_finish(float v, int act, float bias, bool has_res, float res, float colscale) {
     v += bias;                                                // tensor_ops.rs:42-56
     if (act == 1) v = (v * 0.5f) * (erff(v / 1.41421354f) + 1.0f);  // activation.rs:96-113
     v *= colscale;
@@ -163,12 +175,8 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 // QF: 0 = wk / wk2 hold values; 1 / 2 = they hold int8 / int4 codes (see k8_codes_kernel) and `scale` / `scale2` the
 // scale tensors of the two matrices ([N] per column, or [K / 128, N] per group of 128 k), T = bf16 only.
-// KW: wave groups per workgroup.  With KW = 2 a workgroup has 8 waves: both groups of four own the same 2 x 2 layout of
-// outputs, group g multiplies k-steps [2 g, 2 g + 2) of every tile, and the second group's accumulators reach the
-// first through LDS before the epilogue.  A launch with fewer tiles than two per CU then still has 8 waves per CU to
-// cover LDS and barrier waits (what two co-resident workgroups do for the launches with many tiles).
-template <typename T, int BM, int BN, bool DUAL, int QF, int KW>
-__global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict__ x, const T* __restrict__ wk,
+template <typename T, int BM, int BN, bool DUAL, int QF>
+__global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x, const T* __restrict__ wk,
                                                         const T* __restrict__ wk2, const T* __restrict__ bias,
                                                         const T* __restrict__ residual, T* __restrict__ y,
                                                         int M, int K, int N, int Npad, int act, int NT, int MT,
@@ -181,17 +189,15 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
     constexpr int SA = (BM + 1) * 16, SB = (BN + 1) * 16;     // bytes between k-groups
     constexpr int STAGE = kKb * (SA + SB);
     constexpr int TM = BM / 64, TN = BN / 64;
-    constexpr int NTH = 256 * KW;
-    constexpr int KSTEPS = kKb / 2 / KW;                      // k-steps (2 k-groups each) per wave and tile
+    constexpr int NTH = 256;
+    constexpr int KSTEPS = kKb / 2;                           // k-steps (2 k-groups each) per wave and tile
     constexpr int CA = BM * kKb / NTH, CB = BN * kKb / NTH;   // 16-byte chunks per thread per tile
-    static_assert(KW == 1 || (!DUAL && KSTEPS >= 1 && CA >= 1 && CB >= 1), "k-split layout");
     constexpr int WN = BN / 2;                                // B-tile columns per wave column
     constexpr int NREAL = DUAL ? BN / 2 : BN;                 // output columns per block
     static_assert(!DUAL || TN % 2 == 0, "dual tiles need an even number of column fragments");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wg = wave >> 2;               // wave group
     const int wm = (wave >> 1) & 1, wn = wave & 1;
     // Tile order.  Consecutive workgroup ids go to the 8 XCDs in turn and each XCD has its own L2, so XCD c takes
     // the contiguous range [c * per, (c + 1) * per) of a grouped order in which up to 8 row blocks of one column
@@ -199,9 +205,9 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
     // weight tile is fetched from memory once for all its row blocks (with row-major ids the 1024 column tiles of an
     // lm_head were each fetched once per row block) and an activation tile once per 4 column tiles.
     //
-    // Tail split: tiles [full_tiles, total) of that order are the last, partly filled round of the launch; each is
-    // taken by `splits` workgroups (ids behind the whole tiles' ids, so the XCDs share them) that multiply a contiguous
-    // range of k tiles each and meet through `part` and a ticket per tile, see the end of the kernel.
+    // Split over k: tiles [full_tiles, total) of that order are each taken by `splits` workgroups (ids behind the whole
+    // tiles' ids, so the XCDs share them) that multiply a contiguous range of k tiles each and meet through `part` and a
+    // ticket per tile, see the end of the kernel.
     int bx, by;
     int t_begin = 0, t_end = K / kBK, tail = -1, split = 0;
     {
@@ -355,7 +361,7 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
     lwrite(0, 0, 1);
     gload(t_begin + 1 < nt ? t_begin + 1 : t_begin, 0, 1);
     __syncthreads();
-    fread(0, wg * KSTEPS, 0);
+    fread(0, 0, 0);
     // The order of issue inside a k-step is fixed by hand (the scheduling barriers): the fragments of the NEXT k-step
     // are requested before the MFMAs of this one, so their LDS latency runs under the matrix work; left to itself the
     // compiler sinks the reads below the MFMAs into the same registers and the matrix pipe waits for every fragment.
@@ -369,7 +375,7 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
         const int cur = stage;
 #pragma unroll
         for (int kk = 0; kk < KSTEPS; ++kk) {
-            if (kk + 1 < KSTEPS) fread(cur, wg * KSTEPS + kk + 1, (kk + 1) & 1);
+            if (kk + 1 < KSTEPS) fread(cur, kk + 1, (kk + 1) & 1);
             // tile t+1 goes registers -> LDS (codes are converted on the way) and tile t+2 memory -> registers a quarter
             // of the chunks per k-step, between the MFMAs; past the last tile this stores a copy nobody reads
             if (QF == 2 && kk == 0) q_scale = q_scale_next;   // the scale that came with tile t+1
@@ -391,7 +397,7 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
                         acc[i][j] = Mma<T>::mma(af[kk & 1][i], bfr[kk & 1][j], acc[i][j]);
                 __builtin_amdgcn_sched_barrier(0);
                 __syncthreads();
-                fread(cur ^ 1, wg * KSTEPS, 0);
+                fread(cur ^ 1, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
@@ -413,28 +419,7 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
         for (int t = t_begin; t < nt; ++t) tile_step((t - t_begin) & 1, t);
     }
 
-    if (KW == 2) {
-        // the second wave group hands its sums over through LDS (the tiles in it are dead: the loop ended on a barrier)
-        float* xch = reinterpret_cast<float*>(lds) + (wave & 3) * (TM * TN * 16 * 64);
-        static_assert(KW == 1 || 4 * TM * TN * 16 * 64 * 4 <= 2 * STAGE, "exchange area fits the staging buffers");
-        if (wg == 1) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) xch[((i * TN + j) * 16 + v) * 64 + lane] = acc[i][j][v];
-        }
-        __syncthreads();
-        if (wg == 1) return;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] += xch[((i * TN + j) * 16 + v) * 64 + lane];
-    }
-    if (KW == 1 && tail >= 0) {
+    if (tail >= 0) {
         // Partial sums of a split tile go to the workspace, [item][value][thread], through device-scope stores (coherent
         // across the L2s of the XCDs without cache maintenance); once they are acknowledged the workgroup draws the
         // tile's ticket.  The one that draws the last ticket adds all partials in split order, its own included, so
@@ -493,9 +478,8 @@ __global__ __launch_bounds__(256 * KW) void gemm_mfma_kernel(const T* __restrict
                 // out_f32: the f32 accumulator (plus an f32 residual) is stored as it is
                 const float r = residual ? (out_f32 ? reinterpret_cast<const float*>(residual)[(int64_t)m * N + n]
                                                     : Mma<T>::ld(residual, (int64_t)m * N + n)) : 0.f;
-                const float g = acc[i][j][v];
-                const float u = DUAL ? acc[i][DUAL ? j + TN / 2 : j][v] : 0.f;
-                const float o = mfma_finish(g, u, DUAL, act, bv, residual != nullptr, r, extra.glu, cs);
+                const float g = DUAL ? gemm_glu<T>(acc[i][j][v], acc[i][DUAL ? j + TN / 2 : j][v], extra.glu) : acc[i][j][v];   // activation.rs:141-162
+                const float o = mfma_finish(g, act, bv, residual != nullptr, r, cs);
                 if (out_f32) reinterpret_cast<float*>(y)[(int64_t)m * N + n] = o;
                 else Mma<T>::st(y, (int64_t)m * N + n, o);
             }
@@ -569,7 +553,7 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m
             if (n + e >= p.N) break;
             const float bv = p.bias ? Mma<T>::ld(p.bias, n + e) : 0.f;
             const float rv = p.residual ? (f32 ? static_cast<const float*>(p.residual)[at + e] : Mma<T>::ld(static_cast<const T*>(p.residual), at + e)) : 0.f;
-            const float f = mfma_finish(at_lds[e], 0.f, false, p.act, bv, p.residual != nullptr, rv, p.extra.glu, p.extra.colscale ? p.extra.colscale[n + e] : 1.0f);
+            const float f = mfma_finish(at_lds[e], p.act, bv, p.residual != nullptr, rv, p.extra.colscale ? p.extra.colscale[n + e] : 1.0f);
             if (f32) static_cast<float*>(p.y)[at + e] = f;
             else Mma<T>::st(static_cast<T*>(p.y), at + e, f);
         }
@@ -618,34 +602,24 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m
         *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(p.y) + at) = w;
     }
 }
-// The pair's gate on the hardware's exp2 and reciprocal (1 ulp each of f32; the result goes on as bf16): the exact division
-// and expf of glu_combine are 40 instructions an output, 9 us of a 256 x 256 tile's 85.
-template <typename T>
-__device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) {
-    if (std::is_same<T, float>::value) return glu_combine(g, u, p.kind, p.limit, p.alpha, p.shift);
-    const float alpha = p.kind == 1 ? p.alpha : 1.0f;
-    if (p.kind == 1) {
-        g = fminf(g, p.limit);
-        u = fminf(fmaxf(u, -p.limit), p.limit) + p.shift;
-    }
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.44269504f * alpha))) * u;
-}
-
-template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL>
+template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL, int QF>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __restrict__ x, const T* __restrict__ wk, const T* __restrict__ wk2,
-                                                                 int M, int K, int Npad, int NT, int MT, int splits, float* __restrict__ part, TileEpilogue<T> epi) {
+                                                                 int M, int K, int Npad, int NT, int MT, int splits, float* __restrict__ part, const T* __restrict__ scale, const T* __restrict__ scale2,
+                                                                 TileEpilogue<T> epi) {
     static_assert(KG == 4 || KG == 8, "k-groups of a k tile");
     typedef typename Mma<T>::frag frag_t;
     constexpr int BK = KG * Mma<T>::KPC, ROWB = KG * 16, KS = KG / 2;  // k of a tile, bytes of an A row, k-steps
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NW = WM * WN;
     constexpr int NREAL = DUAL ? BN / 2 : BN;                          // output columns per tile
     constexpr int TNO = DUAL ? TN / 2 : TN;                            // output fragments per wave and row
-    constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, STAGE = A_BYTES + B_BYTES;
+    constexpr int CB = QF == 0 ? 16 : QF == 1 ? 8 : 4;                 // bytes of a column's k-group
+    constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * KG * CB, STAGE = A_BYTES + B_BYTES;
     constexpr int LAI = A_BYTES / 1024, LBI = B_BYTES / 1024;          // load instructions per tile
-    constexpr int LA = LAI / NW, LB = LBI / NW, LPT = LA + LB;         // per wave
-    static_assert(LA * NW == LAI && LB * NW == LBI, "whole load instructions per wave");
+    constexpr int LA = LAI / NW, LB = (LBI + NW - 1) / NW, LPT = LA + LB;   // per wave (with fewer instructions than waves, two waves bring the same)
+    static_assert(LA * NW == LAI && LBI * 1024 == B_BYTES && (LB * NW == LBI || NW % LBI == 0), "whole load instructions per wave");
+    static_assert(QF == 0 || (KG == 8 && std::is_same<T, bf16_t>::value), "codes: bf16 activations, k tiles of 64");
     static_assert(KS % 2 == 0, "the last k-step's fragments sit in slot 1, the next tile's first in slot 0");
-    static_assert(!DUAL || (TN % 2 == 0 && BN % 128 == 0), "a load instruction's 64 columns belong to one matrix of the pair");
+    static_assert(!DUAL || (TN % 2 == 0 && NREAL * KG * CB % 1024 == 0), "a load instruction belongs to one matrix of the pair");
     static_assert((NST - 2) * LPT < 64, "vmcnt is a 6-bit counter");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -679,14 +653,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
     }
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
-        const int q = wave * LB + j, kg = q * 64 / BN, bc = q * 64 % BN;
-        int col = n0 + (DUAL ? bc % NREAL : bc) + lane;
-        if (col > Npad - 1) col = Npad - 1;
-        b_base[j] = (unsigned long long)(DUAL && bc >= NREAL ? wk2 : wk);
-        b_off[j] = (unsigned)(((unsigned long long)kg * Npad + col) * 16);
+        const int q = (wave * LB + j) % LBI, half = q * 1024 / (NREAL * KG * CB), at = q * 1024 - half * (NREAL * KG * CB) + lane * 16;
+        const int kg = at / (NREAL * CB);
+        int col = n0 + at % (NREAL * CB) / CB;                           // first of the 16 / CB columns that 16 bytes hold
+        if (col > Npad - 16 / CB) col = Npad - 16 / CB;
+        b_base[j] = (unsigned long long)(DUAL && half ? wk2 : wk);
+        b_off[j] = (unsigned)(((unsigned long long)kg * Npad + col) * CB);
     }
     const unsigned long long a_base = (unsigned long long)(x + (int64_t)m0 * K);
-    const int64_t b_tile_step = (int64_t)KG * Npad * 16;
+    const int64_t b_tile_step = (int64_t)KG * Npad * CB;
     const unsigned lds0 = (unsigned)(uintptr_t)lds;
     const int kt_all = K / BK, kt0 = (int)((int64_t)sidx * kt_all / splits);
     const int nt = (int)((int64_t)(sidx + 1) * kt_all / splits) - kt0;   // this workgroup's k tiles: [kt0, kt0 + nt)
@@ -698,7 +673,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
 #pragma unroll
         for (int j = 0; j < LA; ++j) gemm_lds_load16(a_off[j], ab, (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + (wave * LA + j) * 1024)));
 #pragma unroll
-        for (int j = 0; j < LB; ++j) gemm_lds_load16(b_off[j], gemm_uniform64(b_base[j] + bt), (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + A_BYTES + (wave * LB + j) * 1024)));
+        for (int j = 0; j < LB; ++j) gemm_lds_load16(b_off[j], gemm_uniform64(b_base[j] + bt), (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + A_BYTES + (wave * LB + j) % LBI * 1024)));
     };
     f32x16_t acc[TM][TN];
 #pragma unroll
@@ -708,8 +683,30 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
     const int fsel = lane >> 5;
-    const int b_rd = A_BYTES + (wn * 32 * TNO + (lane & 31)) * 16;
-    frag_t af[2][TM], bfr[2][TN];
+    const int b_rd = A_BYTES + (wn * 32 * TNO + (lane & 31)) * CB;
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    typedef typename std::conditional<QF == 0, frag_t, typename std::conditional<QF == 1, u32x2_t, uint32_t>::type>::type raw_t;
+    frag_t af[2][TM], bq[QF == 0 ? 1 : TN];
+    raw_t bfr[2][TN];
+    // the codes' scales: one per column (int8), or one per column and 128 k (int4), the latter for all of this workgroup's k in LDS
+    float sc[QF == 0 ? 1 : TN];
+    bf16_t* sc_lds = reinterpret_cast<bf16_t*>(lds + NST * STAGE);
+    if constexpr (QF == 1) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int col = n0 + (wn * TNO + j % TNO) * 32 + (lane & 31);
+            sc[j] = Mma<T>::ld(DUAL && j >= TNO ? scale2 : scale, col < (int)epi.N ? col : (int)epi.N - 1);
+            asm volatile("" : : "v"(sc[j]));                             // arrived before the ring's loads are counted
+        }
+    }
+    if constexpr (QF == 2) {
+        const int groups = (kt0 + nt - 1) / 2 - kt0 / 2 + 1;
+#pragma unroll 4
+        for (int e = tid; e < groups * BN; e += 64 * NW) {
+            const int g = kt0 / 2 + e / BN, c = e % BN, col = n0 + (DUAL ? c % NREAL : c);
+            sc_lds[e] = (DUAL && c >= NREAL ? scale2 : scale)[(int64_t)g * epi.N + (col < epi.N ? col : epi.N - 1)];
+        }
+    }
     auto fread = [&](int st, int kk, int slot) {   // kk: k-step of the tile
         const unsigned char* base = lds + st * STAGE;
 #pragma unroll
@@ -719,7 +716,27 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
         }
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-            bfr[slot][j] = *reinterpret_cast<const frag_t*>(base + b_rd + (2 * kk + fsel) * (BN * 16) + (DUAL ? (j / TNO) * (NREAL * 16) : 0) + (j % TNO) * 512);
+            bfr[slot][j] = *reinterpret_cast<const raw_t*>(base + b_rd + (2 * kk + fsel) * (NREAL * CB) + (j / TNO) * (NREAL * KG * CB) + (j % TNO) * 32 * CB);
+    };
+    // codes -> the bf16 values of the dequantised matrix, bf16(code * scale): u * s - bias * s is exactly (u - bias) * s, rounded
+    // once like the product the dequantiser forms
+    auto dequantise = [&](int slot) {
+        if constexpr (QF != 0) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                float f[8];
+                const float nb = (QF == 1 ? -128.0f : -8.0f) * sc[j];
+                uint32_t w[2];
+                if constexpr (QF == 1) { w[0] = bfr[slot][j].x; w[1] = bfr[slot][j].y; }
+                else { w[0] = bfr[slot][j] & 0x0F0F0F0Fu; w[1] = (bfr[slot][j] >> 4) & 0x0F0F0F0Fu; }   // codes 0, 2, 4, 6 and 1, 3, 5, 7
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[QF == 1 ? e : 2 * (e & 3) + (e >> 2)] = __builtin_fmaf((float)((w[e >> 2] >> (8 * (e & 3))) & 0xFFu), sc[j], nb);
+                u32x4_t v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = mfma_pack_bf16(f[2 * e], f[2 * e + 1]);
+                bq[j] = __builtin_bit_cast(frag_t, v);
+            }
+        }
     };
     for (int st = 0; st < NST - 1; ++st) issue(st, st);
     if (nt >= NST - 1) gemm_wait_loads<(NST - 2) * LPT>();
@@ -738,15 +755,25 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    if (i * TN + j >= i0 && i * TN + j < i1) acc[i][j] = Mma<T>::mma(af[slot][i], bfr[slot][j], acc[i][j]);
+                    if (i * TN + j >= i0 && i * TN + j < i1) {
+                        if constexpr (QF == 0) acc[i][j] = Mma<T>::mma(af[slot][i], bfr[slot][j], acc[i][j]);
+                        else acc[i][j] = Mma<T>::mma(af[slot][i], bq[j], acc[i][j]);
+                    }
             __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
         };
+        if constexpr (QF == 2) {
+            const int g = (t + kt0) / 2 - kt0 / 2;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) sc[j] = bf16_to_f32(sc_lds[g * BN + (j / TNO) * NREAL + (wn * TNO + j % TNO) * 32 + (lane & 31)]);
+        }
 #pragma unroll
         for (int kk = 0; kk + 1 < KS; ++kk) {
             fread(ST, kk + 1, (kk + 1) & 1);
+            dequantise(kk & 1);
             mul(kk & 1, 0, TM * TN);
         }
+        dequantise(1);
         mul(1, 0, TM * TN / 2);
         if (t + NST - 1 < nt) gemm_wait_loads<(NST - 2) * LPT>();   // the loads of tiles t + 2 .. t + NST - 1 may be on their way
         else gemm_wait_loads<0>();
@@ -852,23 +879,27 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
 // The tiles, in the order of tile_cost's table.
 enum TileId { kT256x256, kT256x192, kT128x256, kT128x128, kT64x256, kT64x128, kTiles };
 struct TilePlan { int tile; int splits; };
+constexpr int kTileLds = 160 * 1024;   // LDS of one CU
 
-template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL>
+template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL, int QF = 0>
 static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
-    constexpr int ring = NST * (BM + BN) * KG * 16, rows = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4;
-    constexpr int lds_bytes = ring > rows ? ring : rows;
-    static_assert(lds_bytes <= 160 * 1024, "LDS of one CU");
-    auto kern = gemm_tile_kernel<T, KG, NST, WM, WN, TM, TN, DUAL>;
+    constexpr int ring = NST * (BM * KG * 16 + BN * KG * (QF == 0 ? 16 : QF == 1 ? 8 : 4)), rows = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4;
+    constexpr int lds_most = QF == 2 ? kTileLds : ring > rows ? ring : rows;
+    static_assert(ring <= kTileLds && lds_most <= kTileLds, "LDS of one CU");
+    // int4: behind the ring the scales of the groups of 128 k that a workgroup's share of K touches
+    const int lds_bytes = QF == 2 ? std::max(rows, ring + (int)(cdiv(cdiv(a.k, 64), splits) / 2 + 2) * BN * 2) : lds_most;
+    auto kern = gemm_tile_kernel<T, KG, NST, WM, WN, TM, TN, DUAL, QF>;
     static bool configured = false;  // the attribute is per function, not per stream or device state
     if (!configured) {
-        (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+        (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_most);
         configured = true;
     }
     const int64_t nt = cdiv(a.n, NREAL), mt = cdiv(a.m, BM);
     TileEpilogue<T> epi{(const T*)a.bias, a.residual, a.y, a.n, a.act, a.out_f32, a.extra};
     kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (int)a.m, (int)a.k,
-                                                                                   (int)mfma_padded_n(a.n), (int)nt, (int)mt, splits, (float*)a.part, epi);
+                                                                                   (int)mfma_padded_n(a.n), (int)nt, (int)mt, splits, (float*)a.part,
+                                                                                   (const T*)a.scale, (const T*)a.scale2, epi);
     if (splits > 1) gemm_reduce_kernel<T, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
 }
 static size_t tile_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
@@ -937,6 +968,39 @@ static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual) {
     return best;
 }
 
+// Quantised: which tile converts the codes of which columns.  Every wave converts the B fragments it multiplies, 20 (int8) or
+// 23 (int4) vector instructions for 8 codes, so the tiles give a wave as many rows per column as fit: one wave row (128 x 256 in 8
+// waves of 128 x 32, 128 x 128 and 64 x 128 in 4) has no column converted twice; a pair, whose waves hold both matrices, has two
+// wave rows and runs 256 x 256 where it is large.  Measured with int8 at M = 40 .. 4000 of the 3072-wide layers, fitted as above
+// (7 % rms, the pick 1.5 % slower than the best measured); int4 is 0-15 % slower and takes the same plan.  Against the
+// register-staged tiles that ran here before (64 x 64 below half a chip of 128 x 128), M = 200, int8, us: out and down 65 (mean)
+// -> 21 and 29, qkv 35 -> 24, pair 58 -> 58.
+enum QuantTileId { kQ256x256, kQ128x256, kQ128x128, kQ64x128, kQTiles };
+static const TileCost kQuantCost[2][kQTiles] = {
+    {{256, 256, 0, 0, 0, 0, 0, 0}, {128, 256, 256, 4.87, 0.719, 0.337, 5.5, 0.15}, {128, 128, 512, 4.72, 0.486, 0.283, 6.3, 0.12}, {64, 128, 768, 4.25, 0.311, 0.207, 6.3, 0.09}},
+    {{256, 256, 256, 3.15, 1.197, 1.059, 0.2, 0.24}, {128, 256, 256, 4.88, 0.870, 0.480, 3.9, 0.17}, {128, 128, 0, 0, 0, 0, 0, 0}, {64, 128, 768, 3.0, 0.524, 0.30, 4.0, 0.0}},
+};
+static TilePlan quant_plan(int64_t m, int64_t k, int64_t n, bool dual) {
+    static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
+    TilePlan best{-1, 1};
+    double least = 1e300;
+    for (int t = 0; t < kQTiles; ++t) {
+        const TileCost& c = kQuantCost[dual][t];
+        if (c.slots == 0) continue;
+        const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
+        for (int sp : {1, 2, 3, 4, 6, 8}) {
+            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > (64u << 20))) break;
+            // an int4 ring of three and the scales behind it, see launch_tile()
+            if (3 * (c.bm * 128 + c.bn * 32) + (cdiv(cdiv(k, 64), sp) / 2 + 2) * c.bn * 2 > kTileLds) continue;
+            const double kt = (double)k / 64 / sp, wg = (double)(tiles * sp);
+            double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
+            if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
+            if (us < least) { least = us; best = {t, sp}; }
+        }
+    }
+    return best;
+}
+
 bool mfma_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n, int quant) {
     if (dtype != 0 && dtype != 2) return false;
     if (quant != 0 && (dtype != 2 || (quant == 2 && k % 128 != 0))) return false;
@@ -945,53 +1009,22 @@ bool mfma_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n, int quant) 
            cdiv(m, 128) * cdiv(n, 64) < (1ll << 30);   // tile ids are ints
 }
 
-// Tail split of a launch of 128 x 128 tiles on a chip of 256 CUs: the tiles beyond the last multiple of 256 would run
-// as a round of their own on a few CUs (576 pair tiles: 64 CUs work, 192 wait); split 2 or 4 ways over k they give
-// every CU a share.  Returns the number of whole tiles; `splits` = 1 means no split.
-static int64_t mfma_tail_plan(int64_t tiles, int64_t k_tiles, int* splits) {
-    *splits = 1;
-    static const bool allow = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
-    const int64_t tail = tiles % 256;
-    if (!allow || tiles <= 256 || tail == 0 || tail > 128 || tail > (int64_t)kSkinnyTickets) return tiles;
-    int sp = tail <= 64 ? 4 : 2;
-    while (sp > 1 && k_tiles < 4 * sp) sp /= 2;
-    if (sp < 2) return tiles;
-    *splits = sp;
-    return tiles - tail;
-}
-// A launch of few 64 x 64 tiles (under a quarter of the CUs) splits EVERY tile over k between up to 16 workgroups, the
-// same way (partial sums through the workspace, a ticket per tile, the last ticket adds them in split order): twelve
-// tiles with 96 k-tiles each otherwise keep twelve CUs busy for 96 steps while 244 wait.  Returns the split (1: none).
-static int mfma_few_tiles_split(int64_t tiles64, int64_t k_tiles) {
-    static const bool allow = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
-    if (!allow || tiles64 > 64 || tiles64 > (int64_t)kSkinnyTickets) return 1;
-    int sp = 16;
-    while (sp > 1 && (tiles64 * sp > 256 || k_tiles < 4 * sp)) sp /= 2;
-    return sp;
+// Partial sums of the register-staged kernel's 128 x 128 tiles when they are split.
+static size_t staged_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
+    return splits > 1 ? (size_t)(cdiv(m, 128) * cdiv(mfma_padded_n(n), dual ? 64 : 128)) * splits * 128 * 128 * sizeof(float) : 0;
 }
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant) {
     if (!mfma_gemm_supported(dtype, m, k, n, quant)) return 0;
     if (dtype == 0) return tile_part_bytes(m, n, dual, tile_splits_f32(m, k, n, dual));
-    const int64_t k_tiles = k / (kKb * kpc_of(dtype));
-    int sp = 1;
-    size_t bytes = 0;
-    if (!dual && cdiv(m, 128) * cdiv(n, 128) < 128) {   // the 64 x 64 kernel runs (see mfma_gemm)
-        const int64_t t64 = cdiv(m, 64) * cdiv(mfma_padded_n(n), 64);
-        sp = mfma_few_tiles_split(t64, k_tiles);
-        if (sp > 1) bytes = (size_t)t64 * sp * 64 * 64 * sizeof(float);
-    } else {
-        const int64_t tiles = cdiv(m, 128) * cdiv(mfma_padded_n(n), dual ? 64 : 128);
-        const int64_t full = mfma_tail_plan(tiles, k_tiles, &sp);
-        if (sp > 1) bytes = (size_t)(tiles - full) * sp * 128 * 128 * sizeof(float);
-    }
-    if (quant == 0) bytes = std::max(bytes, tile_part_bytes(m, n, dual, tile_plan(m, k, n, dual).splits));   // the LDS-direct kernel
-    return bytes;
+    const int qsp = quant_plan(m, k, n, dual).splits;
+    if (quant) return tile_part_bytes(m, n, dual, qsp);
+    return std::max(tile_part_bytes(m, n, dual, tile_plan(m, k, n, dual).splits), staged_part_bytes(m, n, dual, qsp));
 }
 
-template <typename T, int BM, int BN, bool DUAL, int QF = 0, int KW = 1>
-static void launch_mfma(hipStream_t s, const MfmaLinearArgs& a) {
-    constexpr int lds_bytes = 2 * kKb * ((BM + 1) * 16 + (BN + 1) * 16);
-    auto kern = gemm_mfma_kernel<T, BM, BN, DUAL, QF, KW>;
+template <typename T, bool DUAL, int QF = 0>
+static void launch_staged(hipStream_t s, const MfmaLinearArgs& a, int splits = 1) {
+    constexpr int BM = 128, BN = 128, lds_bytes = 2 * kKb * ((BM + 1) * 16 + (BN + 1) * 16);
+    auto kern = gemm_mfma_kernel<T, BM, BN, DUAL, QF>;
     static bool configured = false;  // the attribute is per function, not per stream or device state
     if (!configured) {
         (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
@@ -1000,61 +1033,56 @@ static void launch_mfma(hipStream_t s, const MfmaLinearArgs& a) {
     const int64_t npad = mfma_padded_n(a.n);
     constexpr int nreal = DUAL ? BN / 2 : BN;
     const int64_t nt = cdiv(npad, nreal), mt = cdiv(a.m, BM);
-    int64_t full = nt * mt;
-    int splits = 1;
-    if (KW == 1 && BM == 128 && BN == 128 && a.part && a.tickets) {
-        int sp = 1;
-        const int64_t f = mfma_tail_plan(nt * mt, a.k / (kKb * Mma<T>::KPC), &sp);
-        if (sp > 1 && a.part_bytes >= (size_t)(nt * mt - f) * sp * BM * BN * sizeof(float)) { full = f; splits = sp; }
-    }
-    if (KW == 1 && BM == 64 && BN == 64 && !DUAL && a.part && a.tickets) {
-        const int sp = mfma_few_tiles_split(nt * mt, a.k / (kKb * Mma<T>::KPC));
-        if (sp > 1 && a.part_bytes >= (size_t)(nt * mt) * sp * BM * BN * sizeof(float)) { full = 0; splits = sp; }
-    }
+    if (splits > 1 && (!a.part || !a.tickets || nt * mt > (int64_t)kSkinnyTickets || a.part_bytes < staged_part_bytes(a.m, a.n, DUAL, splits))) splits = 1;
+    const int64_t full = splits > 1 ? 0 : nt * mt;
     const unsigned grid = (unsigned)(cdiv(full, 8) * 8 + (nt * mt - full) * splits);
-    kern<<<grid, 256 * KW, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (const T*)a.bias, (const T*)a.residual, (T*)a.y,
+    kern<<<grid, 256, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (const T*)a.bias, (const T*)a.residual, (T*)a.y,
                                       (int)a.m, (int)a.k, (int)a.n, (int)npad, a.act, (int)nt, (int)mt, (const T*)a.scale, (const T*)a.scale2,
                                       (int)full, splits, (float*)a.part, a.tickets, a.dtype == 2 ? a.out_f32 : 0, a.extra);
 }
 
+template <bool DUAL, int QF>
+static void launch_quant(hipStream_t s, const MfmaLinearArgs& a) {
+    const TilePlan p = quant_plan(a.m, a.k, a.n, DUAL);
+    typedef bf16_t T;
+    const int sp = p.splits > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, DUAL, p.splits)) ? 1 : p.splits;
+    switch (p.tile) {
+        case kQ256x256: if constexpr (DUAL) return launch_tile<T, 8, 3, 2, 4, 4, 2, true, QF>(s, a, sp); else return;
+        case kQ128x256:
+            if constexpr (DUAL) return launch_tile<T, 8, 3, 2, 4, 2, 2, true, QF>(s, a, sp);
+            else return launch_tile<T, 8, 3, 1, 8, 4, 1, false, QF>(s, a, sp);
+        case kQ128x128: if constexpr (!DUAL) return launch_tile<T, 8, 3, 1, 4, 4, 1, false, QF>(s, a, sp); else return;
+        case kQ64x128:
+            if constexpr (DUAL) return launch_tile<T, 8, 3, 2, 2, 1, 2, true, QF>(s, a, sp);
+            else return launch_tile<T, 8, 3, 1, 4, 2, 1, false, QF>(s, a, sp);
+        default: return launch_staged<T, DUAL, QF>(s, a);   // K too long for the scales of an int4 tile in LDS
+    }
+}
+
 void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
-    // a problem with fewer 128 x 128 tiles than half the CUs runs on 64 x 64 tiles (four times the workgroups); one
-    // with at most one tile per CU on 8-wave workgroups that split every tile's k-steps between two wave groups
-    // (M = 1024, bf16: 192 tiles 46 -> 40 us at K = 4096 and 87 -> 72 us at K = 9216; 384 tiles 54 -> 56 us, not taken)
-    const int64_t tiles = cdiv(a.m, 128) * cdiv(a.n, a.wk2 ? 64 : 128);
-    const bool small = tiles < 128;
-    static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_KSPLIT"); return !(e && e[0] == '0'); }();
-    const bool split = allow_split && !a.wk2 && !small && tiles <= 256;
+    const bool dual = a.wk2 != nullptr;
     // the LDS-direct kernel's loads address a k tile with 32-bit offsets from one scalar base: 256 rows of x, 8 k-groups of
     // the padded weights
     const bool reach = a.k <= (1 << 21) && (uint64_t)mfma_padded_n(a.n) * 128 < (1ull << 31);
-    if (a.quant == 1) {
-        if (a.wk2) launch_mfma<bf16_t, 128, 128, true, 1>(s, a);
-        else if (small) launch_mfma<bf16_t, 64, 64, false, 1>(s, a);
-        else if (split) launch_mfma<bf16_t, 128, 128, false, 1, 2>(s, a);
-        else launch_mfma<bf16_t, 128, 128, false, 1>(s, a);
-    } else if (a.quant == 2) {
-        if (a.wk2) launch_mfma<bf16_t, 128, 128, true, 2>(s, a);
-        else if (small) launch_mfma<bf16_t, 64, 64, false, 2>(s, a);
-        else if (split) launch_mfma<bf16_t, 128, 128, false, 2, 2>(s, a);
-        else launch_mfma<bf16_t, 128, 128, false, 2>(s, a);
-    } else if (a.dtype == 0) {
-        if (!reach) return a.wk2 ? launch_mfma<float, 128, 128, true>(s, a) : launch_mfma<float, 128, 128, false>(s, a);
-        int sp = tile_splits_f32(a.m, a.k, a.n, a.wk2 != nullptr);
-        if (sp > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, a.wk2 != nullptr, sp))) sp = 1;
-        if (a.wk2) launch_tile<float, 8, 3, 2, 2, 1, 2, true>(s, a, sp);
-        else launch_tile<float, 8, 3, 2, 2, 1, 1, false>(s, a, sp);
-    } else {
-        // unquantised bf16: the LDS-direct kernel, on the tiles tile_plan() picks
-        if (a.lds_direct != 0 && reach) {
-            const TilePlan p = tile_plan(a.m, a.k, a.n, a.wk2 != nullptr);
-            return a.wk2 ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);
-        }
-        if (a.wk2) launch_mfma<bf16_t, 128, 128, true>(s, a);
-        else if (small) launch_mfma<bf16_t, 64, 64, false>(s, a);
-        else if (split) launch_mfma<bf16_t, 128, 128, false, 0, 2>(s, a);
-        else launch_mfma<bf16_t, 128, 128, false>(s, a);
+    if (a.quant && !reach) {
+        if (a.quant == 1) return dual ? launch_staged<bf16_t, true, 1>(s, a) : launch_staged<bf16_t, false, 1>(s, a);
+        return dual ? launch_staged<bf16_t, true, 2>(s, a) : launch_staged<bf16_t, false, 2>(s, a);
     }
+    if (a.quant == 1) return dual ? launch_quant<true, 1>(s, a) : launch_quant<false, 1>(s, a);
+    if (a.quant == 2) return dual ? launch_quant<true, 2>(s, a) : launch_quant<false, 2>(s, a);
+    if (a.dtype == 0) {
+        if (!reach) return dual ? launch_staged<float, true>(s, a) : launch_staged<float, false>(s, a);
+        int sp = tile_splits_f32(a.m, a.k, a.n, dual);
+        if (sp > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, dual, sp))) sp = 1;
+        return dual ? launch_tile<float, 8, 3, 2, 2, 1, 2, true>(s, a, sp) : launch_tile<float, 8, 3, 2, 2, 1, 1, false>(s, a, sp);
+    }
+    if (a.lds_direct != 0 && reach) {
+        const TilePlan p = tile_plan(a.m, a.k, a.n, dual);
+        return dual ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);
+    }
+    // the splits of a quantised layer of this shape: its sums, in the same order over the dequantised matrix
+    const int sp = reach ? quant_plan(a.m, a.k, a.n, dual).splits : 1;
+    return dual ? launch_staged<bf16_t, true>(s, a, sp) : launch_staged<bf16_t, false>(s, a, sp);
 }
 
 }  // namespace k

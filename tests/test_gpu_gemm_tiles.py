@@ -88,3 +88,27 @@ def test_f32_tiles_and_splits(hip, m, k, n):
     assert (np.abs(biased - (s + bias)) <= bs + 2.0 ** -23 * np.abs(s + bias)).all()
     g = s / (1 + np.exp(-s))
     assert (np.abs(pair - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + 2.0 ** -20 * np.abs(g * t) + 1e-6).all()
+
+
+# codes converted on the way to the matrix pipes: odd columns, one k tile pair, k tiles that split in the middle of an int4 group, rows
+# around the tiles' 64 and 128
+@pytest.mark.parametrize("scheme", ["w8", "w4g128"])
+@pytest.mark.parametrize("m,k,n", [(17, 128, 9), (63, 384, 130), (65, 640, 137), (129, 1920, 391), (200, 2176, 260), (257, 9216, 72)])
+def test_codes_equal_the_dequantised_matrix(hip, scheme, m, k, n):
+    from test_gpu_quant import code_spec, dequantize_host, quantize, scale_dims
+    rng = np.random.default_rng(m + k + n)
+    x = bf16(rng.standard_normal((m, k), dtype=np.float32))
+    (q, s), (q2, s2) = (quantize(rng.standard_normal((k, n), dtype=np.float32) * np.float32(k ** -0.5), scheme) for _ in range(2))
+    rows, cs, ss, mat = ("Bf16", [m, k]), code_spec(scheme, k, n), ("Bf16", scale_dims(scheme, k, n)), ("Bf16", [k, n])
+    codes = [program([rows, cs, ss], lambda a, b, c: [F.linear_quantized(a, b, c)]),
+             program([rows, cs, ss, cs, ss], lambda a, b, bs, c, cs_: [F.swiglu(F.linear_quantized(a, b, bs), F.linear_quantized(a, c, cs_))])]
+    plain = [program([rows, mat], lambda a, b: [F.linear(a, b)]), program([rows, mat, mat], lambda a, b, c: [F.swiglu(F.linear(a, b), F.linear(a, c))])]
+    got = [hip_run(hip, p, a)[0] for p, a in zip(codes, ([x, q, s], [x, q, s, q2, s2]))]
+    w, w2 = dequantize_host(q, s, scheme), dequantize_host(q2, s2, scheme)
+    hip.set_option("gemm_lds_direct", 0)
+    try:
+        want = [hip_run(hip, p, a)[0] for p, a in zip(plain, ([x, w], [x, w, w2]))]
+    finally:
+        hip.set_option("gemm_lds_direct", 1)
+    for g, v in zip(got, want):
+        assert np.array_equal(g, v)      # the same products, added in the same order
