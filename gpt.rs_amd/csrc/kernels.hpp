@@ -167,7 +167,6 @@ bool skinny_quant_supported(int dtype, int64_t m, int64_t k, int64_t n, int qf);
 size_t skinny_codes_bytes(int64_t k, int64_t n, int qf);
 void skinny_pack_codes(hipStream_t s, const void* codes, void* out, int64_t k, int64_t n, int qf);
 constexpr size_t kSkinnyTickets = 1024;
-int skinny_ksplit(int64_t k, int64_t n);
 size_t skinny_workspace_bytes(int64_t k, int64_t n, bool dual);
 bool skinny_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n);
 size_t skinny_weight_bytes(int dtype, int64_t k, int64_t n);

@@ -7,8 +7,8 @@
 //
 // Weights are read from a derived copy Ws[tile][K/8][16 columns][8 k] (tile = 16 output columns): the 64 lanes of
 // a wave fetch 32 consecutive k of the tile's 16 columns as ONE contiguous KiB in exactly the B-operand layout
-// (lane = 16 * k-group + column holds 8 consecutive k of its column).  A workgroup owns one tile; its 4 waves take
-// the 32-k steps round-robin (so the workgroup reads 4 consecutive KiB per round) and add their partial products
+// (lane = 16 * k-group + column holds 8 consecutive k of its column).  A workgroup owns one tile; its 4, 8 or 16 waves
+// (skinny_plan) take the 32-k steps round-robin (so the workgroup reads consecutive KiB) and add their partial products
 // through LDS.  The A operand (lane = 16 * k-group + row) comes straight from x, which is small and stays in L2.
 // DUAL computes silu(x.W) * (x.W2) (ops/functional/activation.rs:141-162) from two weight copies.
 // f32 takes the same route with 4 k per 16-byte lane word (Ws[tile][K/4][16][4], 16-k steps) on four
@@ -21,8 +21,7 @@
 // sum_k x[row, k], which takes the bias out again (x.(q + b) - b.sum x).  int8 scales (per column) are applied in the
 // epilogue, int4 group scales when a group's sums are added to the running total.
 //
-// A layer with few tiles (N = 3072 has 192, fewer than there are CUs) is split along K over gridDim.y workgroups per
-// tile so the whole chip streams: each writes its 16 x 16 partial sums to a workspace and takes a ticket; the
+// A layer with few tiles (under 96) is split along K over gridDim.y workgroups per tile so that more of the chip streams: each writes its 16 x 16 partial sums to a workspace and takes a ticket; the
 // workgroup that draws the last ticket of a tile adds the partials in split order (so the result does not depend on
 // which one that is), applies the epilogue and resets the ticket for the next launch.
 #include "kernels.hpp"
@@ -91,15 +90,14 @@ __device__ __forceinline__ float skinny_finish(float v, float v2, bool dual, int
     return v;
 }
 
-template <typename T, bool DUAL>
-__global__ __launch_bounds__(256) void skinny_gemm_kernel(const T* __restrict__ x, const T* __restrict__ ws,
+template <typename T, bool DUAL, int NW, int U>
+__global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const T* __restrict__ x, const T* __restrict__ ws,
                                                           const T* __restrict__ ws2, const T* __restrict__ bias,
                                                           const T* __restrict__ residual, T* __restrict__ y, int M, int K,
                                                           int N, int act, float* __restrict__ part, unsigned* __restrict__ tickets,
                                                           int out_f32, EpiExtra extra) {
-    constexpr int U = 4;                         // steps per wave and round, all requested before the first is used
     constexpr int KPC = SkinnyT<T>::KPC, KSTEP = 4 * KPC;
-    __shared__ float red[4][DUAL ? 2 : 1][64][4];
+    __shared__ float red[NW][DUAL ? 2 : 1][64][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, kg = lane >> 4;     // B: column c, k-group kg; A: row c, k-group kg
     const int tile = blockIdx.x;
@@ -111,18 +109,18 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const T* __restrict__ 
     const u32x4_s* asrc = reinterpret_cast<const u32x4_s*>(x + (int64_t)arow * K + KPC * kg);
 
     f32x4_s acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = s_begin + wave; s0 < nsteps; s0 += 4 * U) {
+    for (int s0 = s_begin + wave; s0 < nsteps; s0 += NW * U) {
         u32x4_s b[U], b2[DUAL ? U : 1], a[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int s = s0 + 4 * u < nsteps ? s0 + 4 * u : s0;   // a step past the end repeats the first, weight zero below
-            b[u] = bsrc[(int64_t)s * 64];
-            if (DUAL) b2[u] = bsrc2[(int64_t)s * 64];
+            const int s = s0 + NW * u < nsteps ? s0 + NW * u : s0;   // a step past the end repeats the first, weight zero below
+            b[u] = __builtin_nontemporal_load(bsrc + (int64_t)s * 64);
+            if (DUAL) b2[u] = __builtin_nontemporal_load(bsrc2 + (int64_t)s * 64);
             a[u] = asrc[s * 4];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (s0 + 4 * u < nsteps) {
+            if (s0 + NW * u < nsteps) {
                 acc = SkinnyT<T>::mma(a[u], b[u], acc);
                 if (DUAL) acc2 = SkinnyT<T>::mma(a[u], b2[DUAL ? u : 0], acc2);
             }
@@ -141,7 +139,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const T* __restrict__ 
     for (int i = 0; i < 4; ++i) {
         g[i] = up[i] = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < NW; ++w) {
             g[i] += red[w][0][lane][i];
             if (DUAL) up[i] += red[w][DUAL ? 1 : 0][lane][i];
         }
@@ -241,19 +239,18 @@ __device__ __forceinline__ bf16x8_s nibbles_to_bf16(uint32_t w) {
 }
 
 // QF 1: int8, per-column scales [N]; QF 2: int4 in groups of 128, scales [K/128, N].  A word covers KPW = 64 / 128 k.
-template <int QF, bool DUAL>
-__global__ __launch_bounds__(256) void skinny_gemm_quant_kernel(const bf16_t* __restrict__ x, const uint8_t* __restrict__ qs,
+template <int QF, bool DUAL, int NW, int U>
+__global__ __launch_bounds__(64 * NW) void skinny_gemm_quant_kernel(const bf16_t* __restrict__ x, const uint8_t* __restrict__ qs,
                                                                 const uint8_t* __restrict__ qs2, const bf16_t* __restrict__ sc,
                                                                 const bf16_t* __restrict__ sc2, const bf16_t* __restrict__ bias,
                                                                 const bf16_t* __restrict__ residual, bf16_t* __restrict__ y, int M, int K,
                                                                 int N, int act, float* __restrict__ part, unsigned* __restrict__ tickets,
                                                                 int out_f32) {
-    constexpr int U = 4;                         // words per wave and round, all requested before the first is used
     constexpr int KPW = QF == 1 ? 64 : 128;      // k per word
     constexpr int SPW = KPW / 32;                // MFMA steps per word
     constexpr int NP = DUAL ? 2 : 1;
     constexpr float BIAS = QF == 1 ? 128.0f : 8.0f;
-    __shared__ float red[4][NP][64][4];
+    __shared__ float red[NW][NP][64][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, kg = lane >> 4;
     const int tile = blockIdx.x;
@@ -270,14 +267,14 @@ __global__ __launch_bounds__(256) void skinny_gemm_quant_kernel(const bf16_t* __
     for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
 
     f32x4_s tot = {0.f, 0.f, 0.f, 0.f}, tot2 = {0.f, 0.f, 0.f, 0.f}, xsum = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = s_begin + wave; s0 < s_end; s0 += 4 * U) {
+    for (int s0 = s_begin + wave; s0 < s_end; s0 += NW * U) {
         u32x4_s b[U], b2[DUAL ? U : 1], a[U][SPW];
         float gs[U], gs2[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int s = s0 + 4 * u < s_end ? s0 + 4 * u : s0;   // a word past the end repeats the first and is skipped below
-            b[u] = bsrc[(int64_t)s * 64];
-            if (DUAL) b2[u] = bsrc2[(int64_t)s * 64];
+            const int s = s0 + NW * u < s_end ? s0 + NW * u : s0;   // a word past the end repeats the first and is skipped below
+            b[u] = __builtin_nontemporal_load(bsrc + (int64_t)s * 64);
+            if (DUAL) b2[u] = __builtin_nontemporal_load(bsrc2 + (int64_t)s * 64);
 #pragma unroll
             for (int t = 0; t < SPW; ++t) a[u][t] = *reinterpret_cast<const u32x4_s*>(arowp + (int64_t)s * KPW + 8 * t);
             if (QF == 2) {
@@ -287,7 +284,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_quant_kernel(const bf16_t* __
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (s0 + 4 * u < s_end) {
+            if (s0 + NW * u < s_end) {
                 f32x4_s acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f}, xs = {0.f, 0.f, 0.f, 0.f};
                 const uint32_t bw[4] = {b[u].x, b[u].y, b[u].z, b[u].w};
                 const uint32_t bw2[4] = {DUAL ? b2[DUAL ? u : 0].x : 0u, DUAL ? b2[DUAL ? u : 0].y : 0u, DUAL ? b2[DUAL ? u : 0].z : 0u,
@@ -335,7 +332,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_quant_kernel(const bf16_t* __
     for (int i = 0; i < 4; ++i) {
         g[i] = up[i] = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < NW; ++w) {
             g[i] += red[w][0][lane][i];
             if (DUAL) up[i] += red[w][DUAL ? 1 : 0][lane][i];
         }
@@ -401,19 +398,29 @@ void skinny_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int
     if (dtype == 0) skinny_pack_kernel<float><<<g, 256, 0, s>>>((const float*)w, (float*)out, k, n, kb, ntiles);
     else skinny_pack_kernel<bf16_t><<<g, 256, 0, s>>>((const bf16_t*)w, (bf16_t*)out, k, n, kb, ntiles);
 }
-// Workgroups per tile: doubled while the launch has fewer than two workgroups per CU and each split keeps at least 16
-// steps of 32 k (measured on Ministral-3B shapes at 8 rows: 192 tiles x 4 takes 13.8 us where 192 x 1 took 18.7; at
-// 576 tiles a split no longer pays).
-int skinny_ksplit(int64_t k, int64_t n) {
+// How a launch shares out the steps (words of codes) of a tile: waves per workgroup, workgroups per tile.  Every layer is one pass over its weights; what is left beside HBM's pace are the rounds of a wave (a request and its
+// answer, about 1.5 us each) and, with several workgroups to a tile, their meeting (3 us).  So a layer of at most one tile per CU
+// takes 16 waves to a tile and none of the splits that kept the chip busy with four (8 rows, bf16, us: K = 4096, N = 3072 10.4 ->
+// 8.6, K = 9216 16.0 -> 14.6, f32 K = 768, N = 2304 6.8 -> 5.7; int8 9.0 -> 6.8, 12.6 -> 10.6); up to three tiles per CU, and pairs
+// and codes (which a wave also has to convert) beyond, 8 waves (K = 3072: N = 6144 11.3 -> 10.7, pair of 9216 23.6 -> 20.3, int8
+// N = 6144 11.8 -> 8.2, int4 N = 32768 29.4 -> 20.5); plain layers with more tiles 4 waves with four steps in flight (N = 14432 18.7;
+// 8 waves 19.8, 16 waves 21.1).  Two requests at a time, not four, where 8 or 16 waves share the CU's memory pipeline (pair 20.3
+// against 23.2; at 16 rows K = 9216 16.2 against 19.6).  Only layers of a few tiles still split (f32 K = 3072, N = 768: 10.6 -> 9.1).
+// Weights are read past the caches (nontemporal): 4-5 % on every shape.
+struct SkinnyPlan { int nw, ks; };
+static SkinnyPlan skinny_plan(int64_t steps, int64_t n, bool dual, bool codes) {
     const int64_t tiles = cdiv_s(n, 16);
-    if (tiles > (int64_t)kSkinnyTickets) return 1;
-    int ks = 1;
-    while (ks < 8 && tiles * ks < 512 && k / 32 / (ks * 2) >= 16) ks *= 2;
-    return ks;
+    if (tiles <= 256) {
+        int ks = 1;
+        while (tiles * ks < 96 && steps / (32 * ks) >= 3) ks *= 2;
+        return {16, ks};
+    }
+    if (dual || codes || tiles < 768) return {8, 1};
+    return {4, 1};
 }
+static size_t skinny_part_bytes(int64_t n, bool dual, int ks) { return ks > 1 ? (size_t)cdiv_s(n, 16) * ks * (dual ? 2 : 1) * 256 * sizeof(float) : 0; }
 size_t skinny_workspace_bytes(int64_t k, int64_t n, bool dual) {
-    const int ks = skinny_ksplit(k, n);
-    return ks > 1 ? (size_t)cdiv_s(n, 16) * ks * (dual ? 2 : 1) * 256 * sizeof(float) : 0;
+    return skinny_part_bytes(n, dual, skinny_plan(k / 16, n, dual, false).ks);   // f32 has the most steps, so the most splits
 }
 bool skinny_quant_supported(int dtype, int64_t m, int64_t k, int64_t n, int qf) {
     if ((qf != 1 && qf != 2) || dtype != 2) return false;
@@ -430,27 +437,34 @@ void skinny_pack_codes(hipStream_t s, const void* codes, void* out, int64_t k, i
 }
 
 void skinny_gemm(hipStream_t s, const SkinnyLinearArgs& a) {
+    const bool dual = a.ws2 != nullptr;
+    const int64_t steps = a.k / (a.quant == 1 ? 64 : a.quant == 2 ? 128 : a.dtype == 0 ? 16 : 32);
+    SkinnyPlan p = skinny_plan(steps, a.n, dual, a.quant != 0);
+    if (p.ks > 1 && (!a.part || !a.tickets || a.part_bytes < skinny_part_bytes(a.n, dual, p.ks))) p.ks = 1;
+    const dim3 grid((unsigned)cdiv_s(a.n, 16), (unsigned)p.ks);
     if (a.quant) {
-        int ks = skinny_ksplit(a.k / (a.quant == 1 ? 2 : 4), a.n);   // half / a quarter of the bytes per k
-        if (!a.part || !a.tickets || a.part_bytes < (size_t)cdiv_s(a.n, 16) * ks * (a.ws2 ? 2 : 1) * 256 * sizeof(float)) ks = 1;
-        const dim3 grid((unsigned)cdiv_s(a.n, 16), (unsigned)ks);
-#define GPTRS_LAUNCH(QF, DUAL)                                                                                              \
-        skinny_gemm_quant_kernel<QF, DUAL><<<grid, 256, 0, s>>>((const bf16_t*)a.x, (const uint8_t*)a.ws, (const uint8_t*)a.ws2,  \
+#define GPTRS_LAUNCH(QF, DUAL, NW)                                                                                          \
+        skinny_gemm_quant_kernel<QF, DUAL, NW, 1><<<grid, 64 * NW, 0, s>>>((const bf16_t*)a.x, (const uint8_t*)a.ws, (const uint8_t*)a.ws2,  \
             (const bf16_t*)a.scale, (const bf16_t*)a.scale2, (const bf16_t*)a.bias, (const bf16_t*)a.residual, (bf16_t*)a.y,   \
             (int)a.m, (int)a.k, (int)a.n, a.act, (float*)a.part, a.tickets, a.out_f32)
-        if (a.quant == 1) { if (a.ws2) GPTRS_LAUNCH(1, true); else GPTRS_LAUNCH(1, false); }
-        else { if (a.ws2) GPTRS_LAUNCH(2, true); else GPTRS_LAUNCH(2, false); }
+#define GPTRS_LAUNCH_W(QF, DUAL) do { if (p.nw == 16) GPTRS_LAUNCH(QF, DUAL, 16); else GPTRS_LAUNCH(QF, DUAL, 8); } while (0)
+        if (a.quant == 1) { if (dual) GPTRS_LAUNCH_W(1, true); else GPTRS_LAUNCH_W(1, false); }
+        else { if (dual) GPTRS_LAUNCH_W(2, true); else GPTRS_LAUNCH_W(2, false); }
+#undef GPTRS_LAUNCH_W
 #undef GPTRS_LAUNCH
         return;
     }
-    int ks = skinny_ksplit(a.k, a.n);
-    if (!a.part || !a.tickets || a.part_bytes < skinny_workspace_bytes(a.k, a.n, a.ws2 != nullptr)) ks = 1;
-    const dim3 grid((unsigned)cdiv_s(a.n, 16), (unsigned)ks);
-#define GPTRS_LAUNCH(T, DUAL)                                                                                               \
-    skinny_gemm_kernel<T, DUAL><<<grid, 256, 0, s>>>((const T*)a.x, (const T*)a.ws, (const T*)a.ws2, (const T*)a.bias,          \
+#define GPTRS_LAUNCH(T, DUAL, NW, U)                                                                                        \
+    skinny_gemm_kernel<T, DUAL, NW, U><<<grid, 64 * NW, 0, s>>>((const T*)a.x, (const T*)a.ws, (const T*)a.ws2, (const T*)a.bias, \
         (const T*)a.residual, (T*)a.y, (int)a.m, (int)a.k, (int)a.n, a.act, (float*)a.part, a.tickets, a.dtype == 2 ? a.out_f32 : 0, a.extra)
-    if (a.dtype == 0) { if (a.ws2) GPTRS_LAUNCH(float, true); else GPTRS_LAUNCH(float, false); }
-    else { if (a.ws2) GPTRS_LAUNCH(bf16_t, true); else GPTRS_LAUNCH(bf16_t, false); }
+    if (dual) {
+        if (a.dtype == 0) { if (p.nw == 16) GPTRS_LAUNCH(float, true, 16, 2); else GPTRS_LAUNCH(float, true, 8, 2); }
+        else { if (p.nw == 16) GPTRS_LAUNCH(bf16_t, true, 16, 2); else GPTRS_LAUNCH(bf16_t, true, 8, 2); }
+    } else if (a.dtype == 0) {
+        if (p.nw == 16) GPTRS_LAUNCH(float, false, 16, 2); else if (p.nw == 8) GPTRS_LAUNCH(float, false, 8, 2); else GPTRS_LAUNCH(float, false, 4, 4);
+    } else {
+        if (p.nw == 16) GPTRS_LAUNCH(bf16_t, false, 16, 2); else if (p.nw == 8) GPTRS_LAUNCH(bf16_t, false, 8, 2); else GPTRS_LAUNCH(bf16_t, false, 4, 4);
+    }
 #undef GPTRS_LAUNCH
 }
 
