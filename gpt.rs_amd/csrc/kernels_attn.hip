@@ -44,6 +44,7 @@ constexpr int kMaxDecodeSplits = 512;
 
 typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef float f32x16_v __attribute__((ext_vector_type(16)));
+typedef unsigned u32x4_v __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int64_t clamp_i64(int64_t v, int64_t lo, int64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
@@ -260,8 +261,10 @@ __device__ __forceinline__ float half_sum(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 // bf16 decode attention with the scores on the matrix cores.  grid (n_kv, nsplit, batch), 256 threads; wave w of a
-// workgroup takes the 32-key tiles w, w+4, ... of the workgroup's chunk.  Per tile
-//   S^T[key, q] = K[key, :] . Q[q, :]   v_mfma_f32_32x32x16_bf16, A = cache rows straight from memory (lane = key row),
+// workgroup takes the 32-key tiles w, w+4, ... of the workgroup's share, the rows of its next tile in flight while it works on one.
+// Bound by the caches' rows; 8 sequences of 1000 positions of 8 kv heads of 128 (33 MB), capacity 2048: 18.1 -> 14.5 us since the
+// attended tiles, not the capacity, are shared out and all workgroups are resident at once.  Per tile
+//   S^T[key, q] = K[key, :] . Q[q, :]   v_mfma_f32_32x32x16_bf16, A = cache rows, read whole and turned in LDS (lane = key row),
 //                                       B = the group's G query heads in columns 0..G-1 (other columns repeat them)
 // so a lane owns ONE query: its 16 scores, the running maximum and sum (log2 domain) are per-lane values and the
 // softmax costs a few instructions per key instead of a cross-lane reduction per key and head.  The probabilities go
@@ -270,22 +273,22 @@ __device__ __forceinline__ float half_sum(float x) {
 // lane-groups by shuffles, across waves through LDS, across splits by attn_decode_combine_kernel (same records as
 // attn_decode_kernel, maxima in natural-log units).
 template <int DH, int G>
-__global__ __launch_bounds__(256) void attn_decode_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ kc,
+__global__ __launch_bounds__(256, DH * G == 1024 ? 1 : 2) void attn_decode_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ kc,
                                                                bf16_t* __restrict__ vc, const int32_t* __restrict__ us,
                                                                const int32_t* __restrict__ qs, bf16_t* __restrict__ ctx,
                                                                float* __restrict__ ws, int n_q, int n_kv, int64_t cap,
-                                                               float scale_log2e, int64_t chunk, int nsplit,
+                                                               float scale_log2e, int nsplit,
                                                                const bf16_t* __restrict__ cs, const bf16_t* __restrict__ sn,
                                                                int half_rot, int batched, DecodeCaches caches) {
     constexpr int NK = DH / 16;        // k-steps of the score product
     constexpr int LPR = DH / 8;        // lanes per V row
     constexpr int NSUB = 64 / LPR;     // lane-groups per wave
     constexpr int NV = 32 / NSUB;      // keys of a tile per lane-group
-    __shared__ __align__(16) float p_lds[2][4][G][32];
-    __shared__ float corr_lds[2][4][G];
+    __shared__ __align__(16) float p_lds[4][G][32];
+    __shared__ float corr_lds[4][G];
     __shared__ float sm[4][G], sl[4][G];
     __shared__ float so[4][G][DH];
-    __shared__ __align__(16) bf16_t q_lds[G][DH];
+    __shared__ __align__(16) bf16_t q_lds[G][DH], k_lds[DH], kt_lds[4][32][DH];
     if (batched) {
         const int b = blockIdx.z;
         kc = (bf16_t*)caches.k[b];
@@ -305,40 +308,70 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(const bf16_t* __r
     bf16_t* kbase = kc + (int64_t)kvh * cap * DH;
     bf16_t* vbase = vc + (int64_t)kvh * cap * DH;
 
-    // append this step's row (one workgroup per kv head owns position `upd`); the rows are read back below, by this
-    // workgroup only, after the barrier
-    if (upd / chunk == split) {
-        for (int d = tid; d < DH; d += 256) {
-            kbase[upd * DH + d] = cs ? roped_elem<bf16_t>(knew, d, half_rot, cs, sn) : knew[d];
-            vbase[upd * DH + d] = vnew[d];
-        }
-        __threadfence_block();
-    }
-    // the group's query heads, rotated once per workgroup (16 bytes per thread)
-    for (int c = tid; c < G * LPR; c += 256) {
-        const int g = c / LPR, c0 = (c % LPR) * 8;
-        const bf16_t* qh = qkv + (int64_t)(kvh * G + g) * DH;
-        if (cs) {
-            float f[8];
-            load_roped<bf16_t>(qh, c0, half_rot, cs, sn, f);
-            bf16x8_v r;
+    // the tiles that are attended at this position, shared out evenly: shares of the capacity left the workgroups behind the position
+    // idle in front of the others (half of the chip at half the capacity)
+    const unsigned tiles = (unsigned)(qpos / 32) + 1, share = (tiles + nsplit - 1) / nsplit, own_split = (unsigned)(upd / 32) / share;
+    const bool owner = (own_split < (unsigned)nsplit ? own_split : nsplit - 1) == split;
+    const int64_t p0 = (int64_t)split * share * 32;
+    const int left = qpos + 1 - p0 < (int64_t)share * 32 ? (int)(qpos + 1 - p0) : (int)(share * 32);   // keys of this split
+    const int ntiles = left > 0 ? (left + 31) / 32 : 0;
+    const int fresh = upd - p0 >= 0 && upd - p0 < left ? (int)(upd - p0) : -1;                        // this step's row among them
+    // the cache rows of a wave's first tile are requested before anything else is waited for, whole rows at a time (a lane group to a
+    // row).  Rows past the last attended position re-read that position and get probability zero; this step's row, which the caches do
+    // not hold yet, comes from LDS (K) and from the projection itself (V)
+    const int64_t base = left > 0 ? p0 : 0;
+    kbase += base * DH;
+    vbase += base * DH;
+    u32x4_v kreg[NV], vreg[NV];
+    const auto load_k = [&](int k0) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) r[e] = (__bf16)f[e];   // exact: f holds bf16 values
-            *reinterpret_cast<bf16x8_v*>(&q_lds[g][c0]) = r;
-        } else {
-            *reinterpret_cast<uint4*>(&q_lds[g][c0]) = *reinterpret_cast<const uint4*>(qh + c0);
+        for (int j = 0; j < NV; ++j) {
+            const int r = max(min(k0 + NV * sub + j, left - 1), 0);
+            kreg[j] = *reinterpret_cast<const u32x4_v*>(kbase + (unsigned)(r * DH + li * 8));
         }
+    };
+    const auto load_v = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int r = max(min(k0 + NV * sub + j, left - 1), 0);
+            vreg[j] = *reinterpret_cast<const u32x4_v*>(r == fresh ? vnew + li * 8 : vbase + (unsigned)(r * DH + li * 8));
+        }
+    };
+    // this step's rows first, since loads are answered in order: LPR threads to each of the group's query heads, to the K row and to the
+    // V row.  Dims below half_rot pair with dim + half_rot and the next half_rot with dim - half_rot, a thread's 8 all alike
+    const int hd = tid / LPR, c0 = li * 8;
+    const bool rot = cs && hd <= G && c0 < 2 * half_rot, first = c0 < half_rot;
+    const bf16_t* src = hd < G ? qkv + (int64_t)(kvh * G + hd) * DH : hd == G ? knew : vnew;
+    const int other = rot ? (first ? c0 + half_rot : c0 - half_rot) : c0, cj = first ? c0 : c0 - half_rot;
+    // every thread loads, and every wave a tile: under a branch the waits for these rows would wait for the caches as well
+    u32x4_v own = *reinterpret_cast<const u32x4_v*>(src + c0);
+    const u32x4_v oth = *reinterpret_cast<const u32x4_v*>(src + other);
+    const u32x4_v cosv = *reinterpret_cast<const u32x4_v*>(rot ? cs + cj : src + c0);
+    const u32x4_v sinv = *reinterpret_cast<const u32x4_v*>(rot ? sn + cj : src + c0);
+    load_k(wave * 32);
+    load_v(wave * 32);
+    if (hd < G + 2 && (hd < G || owner)) {
+        if (rot) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a0 = bf16lo(own[e]), a1 = bf16hi(own[e]), b0 = bf16lo(oth[e]), b1 = bf16hi(oth[e]);
+                const float x0 = a0 * bf16lo(cosv[e]), x1 = a1 * bf16hi(cosv[e]), y0 = b0 * bf16lo(sinv[e]), y1 = b1 * bf16hi(sinv[e]);
+                own[e] = (unsigned)f32_to_bf16(first ? x0 - y0 : x0 + y0) | (unsigned)f32_to_bf16(first ? x1 - y1 : x1 + y1) << 16;
+            }
+        }
+        if (hd <= G) *reinterpret_cast<u32x4_v*>(hd < G ? &q_lds[hd][c0] : &k_lds[c0]) = own;
+        // one workgroup per kv head owns position `upd`, and no other reads it
+        if (hd >= G) *reinterpret_cast<u32x4_v*>((hd == G ? kbase : vbase) + (upd - base) * DH + c0) = own;
+    }
+    if (ntiles == 0) {   // a split behind the position: an empty record (split 0 always has a key)
+        for (int idx = tid; idx < G * (DH + 2); idx += 256) {
+            const int g = idx / (DH + 2), d = idx % (DH + 2);
+            ws[((int64_t)(kvh * G + g) * nsplit + split) * (DH + 2) + d] = d == 0 ? -INFINITY : 0.f;
+        }
+        return;
     }
     __syncthreads();
 
-    const int64_t p0 = (int64_t)split * chunk;
-    int64_t p1 = p0 + chunk;
-    if (p1 > qpos + 1) p1 = qpos + 1;
-
-    // query fragments: column = query head col % G, 8 consecutive d per lane and k-step
-    bf16x8_v qf[NK];
-#pragma unroll
-    for (int kk = 0; kk < NK; ++kk) qf[kk] = *reinterpret_cast<const bf16x8_v*>(&q_lds[col % G][16 * kk + 8 * half]);
     float o[G][8];
 #pragma unroll
     for (int g = 0; g < G; ++g)
@@ -346,77 +379,76 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(const bf16_t* __r
         for (int e = 0; e < 8; ++e) o[g][e] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;
 
-    const int ntiles = p1 > p0 ? (int)((p1 - p0 + 31) / 32) : 0;
-    const int iters = (ntiles + 3) / 4;   // uniform over the workgroup
-    for (int it = 0; it < iters; ++it) {
-        const int buf = it & 1;
-        const int64_t kb = p0 + (int64_t)(it * 4 + wave) * 32;
-        const bool active = kb < p1;
-        uint4 vreg[NV];
-        if (active) {
-            // rows past the last attended position re-read that position and get probability zero
-            const bf16_t* krow = kbase + (kb + col < p1 ? kb + col : p1 - 1) * DH + 8 * half;
-            bf16x8_v kf[NK];
+    for (int t = wave; t < ntiles; t += 4) {   // waves are on their own: LDS of one wave, in the order of its instructions
+        const int k0 = t * 32;
+        // 16-byte pieces moved about by their row so that neither side meets bank conflicts
 #pragma unroll
-            for (int kk = 0; kk < NK; ++kk) kf[kk] = *reinterpret_cast<const bf16x8_v*>(krow + 16 * kk);
-#pragma unroll
-            for (int j = 0; j < NV; ++j) {
-                const int64_t key = kb + NV * sub + j;
-                vreg[j] = *reinterpret_cast<const uint4*>(vbase + (key < p1 ? key : p1 - 1) * DH + li * 8);
-            }
-            f32x16_v sc;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) sc[v] = 0.f;
-#pragma unroll
-            for (int kk = 0; kk < NK; ++kk) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[kk], sc, 0, 0, 0);
-            float mx = -INFINITY;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int64_t key = kb + 8 * (v >> 2) + (v & 3) + 4 * half;
-                const float x = key < p1 ? sc[v] * scale_log2e : -INFINITY;
-                sc[v] = x;
-                mx = fmaxf(mx, x);
-            }
-            mx = half_max(mx);
-            const float m_new = fmaxf(m_run, mx);   // finite: the tile holds at least one attended key
-            const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
-            float ls = 0.f;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                sc[v] = __builtin_amdgcn_exp2f(sc[v] - m_new);
-                ls += sc[v];
-            }
-            ls = half_sum(ls);
-            l_run = l_run * corr + ls;
-            m_run = m_new;
-            if (col < G) {
-#pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4)
-                    *reinterpret_cast<float4*>(&p_lds[buf][wave][col][8 * q4 + 4 * half]) =
-                        make_float4(sc[4 * q4], sc[4 * q4 + 1], sc[4 * q4 + 2], sc[4 * q4 + 3]);
-                if (half == 0) corr_lds[buf][wave][col] = corr;
-            }
+        for (int j = 0; j < NV; ++j) {
+            const int r = NV * sub + j;
+            *reinterpret_cast<u32x4_v*>(&kt_lds[wave][r][(li ^ (r & (LPR - 1))) * 8]) = kreg[j];
         }
-        __syncthreads();
-        if (active) {
+        if ((unsigned)(fresh - k0) < 32u && lane < LPR)
+            *reinterpret_cast<u32x4_v*>(&kt_lds[wave][fresh - k0][(lane ^ ((fresh - k0) & (LPR - 1))) * 8]) = *reinterpret_cast<const u32x4_v*>(&k_lds[lane * 8]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (t + 4 < ntiles) load_k(k0 + 128);
+        f32x16_v sc;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sc[v] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {   // A: key `col`; B: query head col % G, 8 consecutive d per lane and k-step
+            const bf16x8_v kf = *reinterpret_cast<const bf16x8_v*>(&kt_lds[wave][col][((2 * kk + half) ^ (col & (LPR - 1))) * 8]);
+            const bf16x8_v qf = *reinterpret_cast<const bf16x8_v*>(&q_lds[col % G][16 * kk + 8 * half]);
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf, sc, 0, 0, 0);
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const float x = k0 + 8 * (v >> 2) + (v & 3) + 4 * half < left ? sc[v] * scale_log2e : -INFINITY;
+            sc[v] = x;
+            mx = fmaxf(mx, x);
+        }
+        mx = half_max(mx);
+        const float m_new = fmaxf(m_run, mx);   // finite: the tile holds at least one attended key
+        const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
+        float ls = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            sc[v] = __builtin_amdgcn_exp2f(sc[v] - m_new);
+            ls += sc[v];
+        }
+        ls = half_sum(ls);
+        l_run = l_run * corr + ls;
+        m_run = m_new;
+        if (col < G) {
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4)
+                *reinterpret_cast<float4*>(&p_lds[wave][col][8 * q4 + 4 * half]) =
+                    make_float4(sc[4 * q4], sc[4 * q4 + 1], sc[4 * q4 + 2], sc[4 * q4 + 3]);
+            if (half == 0) corr_lds[wave][col] = corr;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float c = corr_lds[wave][g];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[g][e] *= c;
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const float vf[8] = {bf16lo(vreg[j][0]), bf16hi(vreg[j][0]), bf16lo(vreg[j][1]), bf16hi(vreg[j][1]),
+                                 bf16lo(vreg[j][2]), bf16hi(vreg[j][2]), bf16lo(vreg[j][3]), bf16hi(vreg[j][3])};
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const float c = corr_lds[buf][wave][g];
+                const float pj = p_lds[wave][g][NV * sub + j];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o[g][e] *= c;
-            }
-#pragma unroll
-            for (int j = 0; j < NV; ++j) {
-                const float vf[8] = {bf16lo(vreg[j].x), bf16hi(vreg[j].x), bf16lo(vreg[j].y), bf16hi(vreg[j].y),
-                                     bf16lo(vreg[j].z), bf16hi(vreg[j].z), bf16lo(vreg[j].w), bf16hi(vreg[j].w)};
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    const float pj = p_lds[buf][wave][g][NV * sub + j];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) o[g][e] += pj * vf[e];
-                }
+                for (int e = 0; e < 8; ++e) o[g][e] += pj * vf[e];
             }
         }
+        if (t + 4 < ntiles) load_v(k0 + 128);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 
     // merge the lane-groups of this wave (they share the wave's maximum), then the four waves through LDS
@@ -462,31 +494,36 @@ __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, T* __re
     // grid (n_q, batch): sequence blockIdx.y owns gridDim.x heads of records and of the context
     ws += (int64_t)blockIdx.y * gridDim.x * nsplit * (dh + 2);
     ctx += (int64_t)blockIdx.y * gridDim.x * dh;
-    // per-split weights exp(m_s - max) are computed once into LDS; the slice loads of the output
-    // loop are then independent of each other
-    __shared__ float wgt[kMaxDecodeSplits];
-    __shared__ float red[16];
+    // eight records at a time, all of their loads independent: every thread keeps the running maximum and sum for itself (LDS
+    // reductions of the two, with their four barriers and three rounds of dependent loads, took 4.8 us for 16 splits)
     const int h = blockIdx.x;
     const float* base = ws + (int64_t)h * nsplit * (dh + 2);
-    float mn = -INFINITY;
-    for (int s = threadIdx.x; s < nsplit; s += blockDim.x) {
-        const float ms = base[(int64_t)s * (dh + 2)];
-        wgt[s] = ms;
-        mn = fmaxf(mn, ms);
-    }
-    mn = block_max(mn, red);
-    float lsum = 0.f;
-    for (int s = threadIdx.x; s < nsplit; s += blockDim.x) {
-        const float ms = wgt[s];
-        const float c = ms == -INFINITY ? 0.f : expf(ms - mn);
-        wgt[s] = c;
-        lsum += base[(int64_t)s * (dh + 2) + 1] * c;
-    }
-    const float L = block_sum(lsum, red);  // also orders the wgt[] writes before the reads below
     for (int d = threadIdx.x; d < dh; d += blockDim.x) {
-        float O = 0.f;
-#pragma unroll 8
-        for (int s = 0; s < nsplit; ++s) O += base[(int64_t)s * (dh + 2) + 2 + d] * wgt[s];
+        float mn = -INFINITY, L = 0.f, O = 0.f;
+        for (int s0 = 0; s0 < nsplit; s0 += 8) {
+            float m[8], l[8], o[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float* rec = base + (int64_t)(s0 + j < nsplit ? s0 + j : nsplit - 1) * (dh + 2);
+                m[j] = rec[0]; l[j] = rec[1]; o[j] = rec[2 + d];
+            }
+            float mx = mn;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) if (s0 + j < nsplit) mx = fmaxf(mx, m[j]);
+            if (mx == -INFINITY) mx = 0.f;     // nothing but empty records so far
+            const float c0 = expf(mn - mx);
+            L *= c0;
+            O *= c0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (s0 + j < nsplit) {
+                    const float c = expf(m[j] - mx);
+                    L += l[j] * c;
+                    O += o[j] * c;
+                }
+            }
+            mn = mx;
+        }
         stf(ctx, (int64_t)h * dh + d, O / L);
     }
 }
@@ -526,15 +563,10 @@ static int attn_decode_mfma(hipStream_t s, const AttnDecodeArgs& a) {
     int64_t chunk;
     decode_geometry(a.dtype, a.head_dim, a.capacity, &nsplit, &chunk);   // the workspace holds this many splits
     const int nb = a.batch > 1 ? a.batch : 1;
-    // chunks of whole 32-key tiles, never shorter than the workspace geometry's; lengthened until the launch is
-    // near four workgroups per CU (each wave then walks several tiles)
-    const int64_t step = chunk > 32 ? chunk : 32;
-    chunk = step;
-    nsplit = (int)cdiv(a.capacity, chunk);
-    while (nsplit > 1 && (int64_t)a.n_kv * nb * nsplit > 1024) {
-        chunk += step;
-        nsplit = (int)cdiv(a.capacity, chunk);
-    }
+    // at most the two workgroups per CU that its registers hold (one with 8 heads of 128): one round whose waves have their loads in flight together
+    const int64_t most = (a.head_dim * a.n_q == 1024 * a.n_kv ? 256 : 512) / ((int64_t)a.n_kv * nb), tiles = cdiv(a.capacity, 32);
+    if (nsplit > tiles) nsplit = (int)tiles;
+    if (nsplit > most) nsplit = most > 1 ? (int)most : 1;
     dim3 grid((unsigned)a.n_kv, (unsigned)nsplit, (unsigned)nb);
     DecodeCaches caches{};
     for (int b = 0; b < nb && b < 16; ++b) { caches.k[b] = a.k_caches[b]; caches.v[b] = a.v_caches[b]; }
@@ -542,8 +574,8 @@ static int attn_decode_mfma(hipStream_t s, const AttnDecodeArgs& a) {
     const int g = (int)(a.n_q / a.n_kv);
 #define GPTRS_LAUNCH(DH, G)                                                                                          \
     attn_decode_mfma_kernel<DH, G><<<grid, 256, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.k_cache, (bf16_t*)a.v_cache, \
-        a.update_starts, a.query_start, (bf16_t*)a.ctx, (float*)a.ws, (int)a.n_q, (int)a.n_kv, a.capacity, sl, chunk, \
-        nsplit, (const bf16_t*)a.cos, (const bf16_t*)a.sin, (int)a.rot_half, a.batch > 1 ? 1 : 0, caches)
+        a.update_starts, a.query_start, (bf16_t*)a.ctx, (float*)a.ws, (int)a.n_q, (int)a.n_kv, a.capacity, sl, nsplit, \
+        (const bf16_t*)a.cos, (const bf16_t*)a.sin, (int)a.rot_half, a.batch > 1 ? 1 : 0, caches)
 #define GPTRS_LAUNCH_G(DH)                                                                                           \
     switch (g) {                                                                                                     \
         case 1: GPTRS_LAUNCH(DH, 1); break;                                                                          \
