@@ -167,8 +167,9 @@ __device__ __forceinline__ float block_sum(float v, float* smem16) {
     __syncthreads();
     if ((threadIdx.x & 63) == 0) smem16[w] = v;
     __syncthreads();
-    float r = 0.f;
-    for (int i = 0; i < nw; ++i) r += smem16[i];
+    float r = 0.f;   // all reads at once, added in the order of the waves (a loop up to nw waited for every read)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) { const float s = smem16[i]; r += i < nw ? s : 0.f; }
     return r;
 }
 __device__ __forceinline__ float block_max(float v, float* smem16) {
@@ -178,7 +179,8 @@ __device__ __forceinline__ float block_max(float v, float* smem16) {
     if ((threadIdx.x & 63) == 0) smem16[w] = v;
     __syncthreads();
     float r = -INFINITY;
-    for (int i = 0; i < nw; ++i) r = fmaxf(r, smem16[i]);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) { const float s = smem16[i]; r = fmaxf(r, i < nw ? s : -INFINITY); }
     return r;
 }
 
