@@ -184,5 +184,25 @@ __device__ __forceinline__ float block_max(float v, float* smem16) {
     return r;
 }
 
+// The tile of a workgroup of a prompt's attention, grid (row tiles, heads, sequences).  Workgroups go to the 8 XCDs in turn, so
+// with the plain indices every XCD reads the keys and values of every head through its own 4 MiB of L2 (4 sequences of 2047 rows of
+// 8 kv heads of 128: 8 MiB at a time).  Here an XCD takes an eighth of the heads of each sequence (heads that share keys lie side by
+// side), all of their row tiles in turn, or, where the heads do not divide, an eighth of the pairs of head and sequence.  Those
+// prompts 313 -> 236 us per layer; latent attention of 4 sequences, 3064 rows, 32 heads 136 -> 94; chunked of 3000 rows, 32 heads,
+// 126 -> 116.
+struct XcdTile { unsigned x, y, z; };
+__device__ __forceinline__ XcdTile xcd_tile() {
+    const unsigned gx = gridDim.x, gy = gridDim.y, lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), xcd = lin & 7, slot = lin >> 3;
+    if (gy % 8 == 0) {
+        const unsigned per = gy / 8, r = slot / per;
+        return {r % gx, xcd * per + slot % per, r / gx};
+    }
+    if (gy * gridDim.z % 8 == 0) {
+        const unsigned pair = xcd + 8 * (slot / gx);
+        return {slot % gx, pair % gy, pair / gy};
+    }
+    return {blockIdx.x, blockIdx.y, blockIdx.z};
+}
+
 }  // namespace k
 }  // namespace gptrs

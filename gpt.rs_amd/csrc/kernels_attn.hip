@@ -797,9 +797,10 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
     const int G = n_q / n_kv;
     const int gw = G >= 4 ? 4 : G;                 // query heads of the group in this workgroup
     const int rtpb = 4 / gw;                       // 32-row tiles per workgroup
-    const int kvh = blockIdx.y;
-    const int seq = blockIdx.z / zgroups, zg = blockIdx.z % zgroups;
-    const int bx = gridDim.x - 1 - blockIdx.x;     // rows that see many keys first: the last workgroups to start are the short ones
+    const XcdTile at = xcd_tile();
+    const int kvh = at.y;
+    const int seq = at.z / zgroups, zg = at.z % zgroups;
+    const int bx = gridDim.x - 1 - at.x;     // rows that see many keys first: the last workgroups to start are the short ones
     const int head = kvh * G + zg * gw + wave % gw;
     const int q0 = (bx * rtpb + wave / gw) * 32;
     const int64_t P = (int64_t)(n_q + 2 * n_kv) * DH;
@@ -1020,9 +1021,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
     const int G = n_q / n_kv;
     const int gw = G >= 4 ? 4 : G;
     const int rtpb = 4 / gw;
-    const int kvh = blockIdx.y;
-    const int seq = blockIdx.z / zgroups, zg = blockIdx.z % zgroups;
-    const int bx = gridDim.x - 1 - blockIdx.x;     // rows that see many keys first: the last workgroups to start are the short ones
+    const XcdTile at = xcd_tile();
+    const int kvh = at.y;
+    const int seq = at.z / zgroups, zg = at.z % zgroups;
+    const int bx = gridDim.x - 1 - at.x;     // rows that see many keys first: the last workgroups to start are the short ones
     const int head = kvh * G + zg * gw + wave % gw;
     const int q0 = (bx * rtpb + wave / gw) * 32;
     const int64_t P = (int64_t)(n_q + 2 * n_kv) * DH;

@@ -454,8 +454,9 @@ __global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, cons
     bf16_t* kt = reinterpret_cast<bf16_t*>(chk_smem);                 // [64][KSTR]
     bf16_t* vt = kt + kKTile * KSTR;                                  // [64][VSTR]
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 15, kg = lane >> 4;
-    const int b = blockIdx.z, h = blockIdx.y, T = a.len[b], r0 = a.row0[b];
-    const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kQTile;
+    const XcdTile at = xcd_tile();
+    const int b = at.z, h = at.y, T = a.len[b], r0 = a.row0[b];
+    const int q0 = ((int)gridDim.x - 1 - (int)at.x) * kQTile;
     if (q0 >= T) return;
     const int H = (int)a.heads, G = (int)a.kv_heads, D = (int)a.dim, V = (int)a.vdim, rot = (int)a.rot, g = h / (H / G);
     const int chunk = a.chunk > 0 && a.chunk < T ? (int)a.chunk : T;

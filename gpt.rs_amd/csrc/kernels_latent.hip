@@ -489,8 +489,9 @@ __global__ __launch_bounds__(512) void latent_prefill_kernel(LatentPrefillArgs a
     bf16_t* kt = reinterpret_cast<bf16_t*>(lat_smem);                 // [64][KSTR]
     bf16_t* vt = kt + kKTile * KSTR;                                  // [64][VSTR]
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 15, kg = lane >> 4;
-    const int b = blockIdx.z, h = blockIdx.y, T = a.len[b], r0 = a.row0[b];
-    const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kQTile;   // the longest workgroups first
+    const XcdTile at = xcd_tile();
+    const int b = at.z, h = at.y, T = a.len[b], r0 = a.row0[b];
+    const int q0 = ((int)gridDim.x - 1 - (int)at.x) * kQTile;   // the longest workgroups first
     if (q0 >= T) return;
     const int dim = (int)a.dim, rot = (int)a.rot, hd = dim + rot, vdim = (int)a.vdim, H = (int)a.heads, w = (int)(a.rank + a.rot);
     const int kend = min(q0 + kQTile, T);
