@@ -204,9 +204,31 @@ __global__ void rms_norm_f32_bf16_kernel(const float* __restrict__ x, const floa
         }
         return;
     }
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) { const float v = row[i]; q += v * v; }
+    const bool wide = n % 8 == 0 && ((((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)y) & 15u) == 0);   // longer rows, read twice
+    if (wide) {
+        for (int64_t c = threadIdx.x; c * 8 < n; c += blockDim.x) {
+            const float4 a = *reinterpret_cast<const float4*>(row + c * 8), b = *reinterpret_cast<const float4*>(row + c * 8 + 4);
+            q += a.x * a.x; q += a.y * a.y; q += a.z * a.z; q += a.w * a.w;
+            q += b.x * b.x; q += b.y * b.y; q += b.z * b.z; q += b.w * b.w;
+        }
+    } else {
+        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) { const float v = row[i]; q += v * v; }
+    }
     const float inv_rms = 1.0f / sqrtf(block_sum(q, red) * inv_n + eps);
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) out[i] = f32_to_bf16((row[i] * inv_rms) * gamma[i]);
+    if (wide) {
+        for (int64_t c = threadIdx.x; c * 8 < n; c += blockDim.x) {
+            const float4 a = *reinterpret_cast<const float4*>(row + c * 8), b = *reinterpret_cast<const float4*>(row + c * 8 + 4);
+            const float4 ga = *reinterpret_cast<const float4*>(gamma + c * 8), gb = *reinterpret_cast<const float4*>(gamma + c * 8 + 4);
+            fused_u32x4_t o;
+            o[0] = pack_bf16x2((a.x * inv_rms) * ga.x, (a.y * inv_rms) * ga.y);
+            o[1] = pack_bf16x2((a.z * inv_rms) * ga.z, (a.w * inv_rms) * ga.w);
+            o[2] = pack_bf16x2((b.x * inv_rms) * gb.x, (b.y * inv_rms) * gb.y);
+            o[3] = pack_bf16x2((b.z * inv_rms) * gb.z, (b.w * inv_rms) * gb.w);
+            *reinterpret_cast<fused_u32x4_t*>(out + c * 8) = o;
+        }
+    } else {
+        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) out[i] = f32_to_bf16((row[i] * inv_rms) * gamma[i]);
+    }
 }
 // out = x + mult * (y * inv_rms(y) * gain), f32 rows; the sum in bf16 as well when out16 is given.  ONE: a thread holds all it
 // handles (n <= 8 per thread), so y is read once and x and the gains are requested ahead of the statistic.
