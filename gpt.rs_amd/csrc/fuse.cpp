@@ -955,8 +955,10 @@ struct Fuser {
                 const Part &p = parts[b], &p0 = parts[0];
                 ok = p.cos == p0.cos && p.sin == p0.sin && p.rot == p0.rot && p.starts == p0.starts;
                 for (int kv = 0; kv < 2 && ok; ++kv) {
+                    // a cache is [n_kv, capacity, head_dim]: of an update's start only the row is left to say.  Taller or wider bases (several
+                    // layers' heads in one tensor, say) keep their updates
                     const Spec& c = fn.body[p.du[kv]].out_specs[0];
-                    ok = c == fn.body[p0.du[0]].out_specs[0] && c.dtype == a0.out_specs[0].dtype;
+                    ok = c == fn.body[p0.du[0]].out_specs[0] && c.dtype == a0.out_specs[0].dtype && c.rank() == 3 && c.dims[0] == a0.n_kv && c.dims[2] == a0.head_dim;
                 }
                 if (B == 1) { src = p.x; continue; }
                 const Instr* sl = ok ? producer(p.x) : nullptr;

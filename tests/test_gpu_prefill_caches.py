@@ -15,13 +15,13 @@ CASES = [  # sequences, rows, query heads, key heads, head size, rotated, cache 
 ]
 
 
-def program(dt, B, T, hq, hkv, dh, rot, cap):
+def program(dt, B, T, hq, hkv, dh, rot, cap, base=None):
     fb = FunctionBuilder("main", dt)
     cfg = F.AttentionConfig(hq * dh, hq, hkv, dh)
     qkv = fb.param(dt, [B * T, (hq + 2 * hkv) * dh])
     tabs = [fb.param(dt, [T, dh // 2]) for _ in range(2)] if rot else []
     starts = fb.param("Si32", [3])
-    caches = [fb.param(dt, [hkv, cap, dh]) for _ in range(2 * B)]
+    caches = [fb.param(dt, base or [hkv, cap, dh]) for _ in range(2 * B)]
     ctxs, outs = [], []
     for b in range(B):
         rows = qkv if B == 1 else qkv.slice([b * T, 0], [T, qkv.dims[1]])
@@ -62,6 +62,41 @@ def test_a_cache_that_the_program_computes_stays_apart():
     base = ctx.reshape([1, 8, 32])
     fb.set_results([ctx, F.dynamic_update_slice_into(base, k, starts), F.dynamic_update_slice_into(base, v, starts)])
     assert fusion_report(Program(fb)).count("DynamicUpdateSlice") == 2
+
+
+# tensors that hold more than the keys (or values) of one layer: more heads, wider rows, both; where the update goes
+BASES = [((1, 8, 4, 2, 32, False), [6, 16, 32], (4, 3, 0)), ((1, 33, 2, 2, 32, True), [2, 64, 64], (0, 5, 32)), ((2, 9, 4, 2, 64, True), [4, 12, 72], (1, 2, 8)),
+         ((3, 5, 2, 1, 32, False), [2, 5, 33], (7, -1, 1)), ((1, 17, 4, 4, 64, False), [5, 17, 64], (1, 0, 0))]
+
+
+def test_wider_and_taller_bases_keep_their_updates():
+    for (B, T, hq, hkv, dh, rot), base, _ in BASES:
+        for dt in ("F32", "Bf16"):
+            rep = fusion_report(program(dt, B, T, hq, hkv, dh, rot, 1, base))
+            assert sum("DynamicUpdateSlice" in line for line in rep) == 2 * B, (base, rep)
+            assert not any("prefill_caches" in line for line in rep), (base, rep)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["F32", "Bf16"])
+def test_wider_and_taller_bases(hip, dt):
+    """Heads, rows and columns of the start all count; what the update does not name stays."""
+    for (B, T, hq, hkv, dh, rot), base, at in BASES:
+        args = inputs(B, T, hq, hkv, dh, rot, 1, 0, 5)[:3 if rot else 1] + [np.array(at, np.int32)]
+        rng = np.random.default_rng(6)
+        args += [rng.standard_normal(base, dtype=np.float32) for _ in range(2 * B)]
+        if dt == "F32":
+            check_program(hip, program(dt, B, T, hq, hkv, dh, rot, 1, base), args, what=f"{base} at {at}")
+            continue
+        args = [a if a.dtype == np.int32 else bf16_bits_to_f32(f32_to_bf16_bits(a)) for a in args]
+        got = hip_run(hip, program(dt, B, T, hq, hkv, dh, rot, 1, base), args)
+        want = oracle_run(program("F32", B, T, hq, hkv, dh, rot, 1, base), args)
+        assert_close(got[0], want[0], atol=3e-2, rtol=2.0 ** -7, what=f"context {base}")      # as in test_bf16
+        for i, (g, w) in enumerate(zip(got[1:], want[1:])):
+            if i % 2 == 0 and rot:
+                assert_close(g, w, atol=1e-6, rtol=2.0 ** -8, what=f"keys {base}")
+            else:
+                assert np.array_equal(g, w), f"cache {i} {base}"
 
 
 @pytest.mark.gpu
