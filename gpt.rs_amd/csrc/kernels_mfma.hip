@@ -133,18 +133,10 @@ __device__ __forceinline__ uint32_t mfma_pack_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));   // round to nearest even
 }
 
-// The pair's gate on the hardware's exp2 and reciprocal (1 ulp each of f32; the result goes on as bf16): the exact division
-// and expf of glu_combine are 40 instructions an output, 9 us of a 256 x 256 tile's 85.
-template <typename T>
-__device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) {
-    if (std::is_same<T, float>::value) return glu_combine(g, u, p.kind, p.limit, p.alpha, p.shift);
-    const float alpha = p.kind == 1 ? p.alpha : 1.0f;
-    if (p.kind == 1) {
-        g = fminf(g, p.limit);
-        u = fminf(fmaxf(u, -p.limit), p.limit) + p.shift;
-    }
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.44269504f * alpha))) * u;
-}
+// A pair's output, the function that the decode kernels form (activation.rs:141-162): 28 instructions, 4 us of a 256 x 256 tile's 86 more than exp2 and a
+// reciprocal alone would take (M = 8188, pair of 9216: 773 us against 737), but those are off by up to 65 ulp of f32 where g is far below
+// zero, against 3, and lose the result altogether from -87.4 on, where the reciprocal is subnormal.
+__device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) { return glu_combine(g, u, p.kind, p.limit, p.alpha, p.shift); }
 
 __device__ __forceinline__ float mfma_finish(float v, int act, float bias, bool has_res, float res, float colscale) {
     v += bias;                                                // tensor_ops.rs:42-56
@@ -478,7 +470,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
                 // out_f32: the f32 accumulator (plus an f32 residual) is stored as it is
                 const float r = residual ? (out_f32 ? reinterpret_cast<const float*>(residual)[(int64_t)m * N + n]
                                                     : Mma<T>::ld(residual, (int64_t)m * N + n)) : 0.f;
-                const float g = DUAL ? gemm_glu<T>(acc[i][j][v], acc[i][DUAL ? j + TN / 2 : j][v], extra.glu) : acc[i][j][v];   // activation.rs:141-162
+                const float g = DUAL ? gemm_glu(acc[i][j][v], acc[i][DUAL ? j + TN / 2 : j][v], extra.glu) : acc[i][j][v];
                 const float o = mfma_finish(g, act, bv, residual != nullptr, r, cs);
                 if (out_f32) reinterpret_cast<float*>(y)[(int64_t)m * N + n] = o;
                 else Mma<T>::st(y, (int64_t)m * N + n, o);
@@ -833,7 +825,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 float o = acc[i][j][v];
-                if (DUAL) o = gemm_glu<T>(o, acc[i][DUAL ? j + TNO : j][v], epi.extra.glu);   // activation.rs:141-162
+                if (DUAL) o = gemm_glu(o, acc[i][DUAL ? j + TNO : j][v], epi.extra.glu);
                 area[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * RSF + j * 32 + (lane & 31)] = o;
             }
 #pragma unroll 1
@@ -871,7 +863,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
         float u[8];
         sum8(part + m * width + np + n, u);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = gemm_glu<T>(o[e], u[e], epi.extra.glu);   // activation.rs:141-162
+        for (int e = 0; e < 8; ++e) o[e] = gemm_glu(o[e], u[e], epi.extra.glu);
     }
     gemm_finish8(epi, m, n, o);
 }

@@ -112,3 +112,26 @@ def test_codes_equal_the_dequantised_matrix(hip, scheme, m, k, n):
         hip.set_option("gemm_lds_direct", 1)
     for g, v in zip(got, want):
         assert np.array_equal(g, v)      # the same products, added in the same order
+
+
+# a pair's gate is one function for prompts and for decode steps (kernels_skinny.hip), also far below zero, where e^-g nears the largest
+# f32.  Each sum has two exact products, so both kernels combine the same gates; a split over k meets in gemm_reduce_kernel
+@pytest.mark.parametrize("kind", ["silu", "clamped"])
+@pytest.mark.parametrize("m,k", [(17, 64), (300, 64), (300, 3072)])
+def test_pair_is_the_decode_steps_function(hip, kind, m, k):
+    rng = np.random.default_rng(k + m)
+    n = 4096
+    glu = F.swiglu if kind == "silu" else lambda a, b: F.clamped_glu(a, b, 60.0, 1.25)
+    w, w2 = np.zeros((k, n), np.float32), np.zeros((k, n), np.float32)
+    at = (0, k - 1)                                       # the two products of a sum lie as far apart as k allows
+    w[at[0]], w[at[1]] = bf16(np.linspace(-100, 100, n)), bf16(rng.uniform(-1, 1, n))
+    w2[at[0]] = bf16(rng.standard_normal(n) * 2.0 ** rng.uniform(-4, 60, n))
+    x = np.zeros((m, k), np.float32)
+    x[:, at[0]], x[:, at[1]] = bf16(np.linspace(1.0, 0.25, m)), 2.0 ** -8
+    mat = ("Bf16", [k, n])
+    run = lambda rows: hip_run(hip, program([("Bf16", [len(rows), k]), mat, mat], lambda a, b, c: [glu(F.linear(a, b), F.linear(a, c))]), [rows, w, w2])[0]
+    got = run(x)
+    for r in range(0, m, 16):
+        rows = x[r:r + 16] if r + 16 <= m else x[m - 16:]
+        first = r if r + 16 <= m else m - 16
+        assert np.array_equal(got[first:first + 16], run(rows)), first
