@@ -90,6 +90,20 @@ def test_f32_tiles_and_splits(hip, m, k, n):
     assert (np.abs(pair - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + 2.0 ** -20 * np.abs(g * t) + 1e-6).all()
 
 
+def test_f32_sums_in_two_chains(hip):
+    """An f32 rounding is off by 0.42 * 2^-24 of its value in the mean square (uniform over half an ulp, an ulp being 2^-23 to 2^-24 of it), and
+    a chain of n terms of one size rounds partial sums of sqrt(i): sqrt(n / 2) of that over the sum's own sqrt(n).  Two chains of k / 2:
+    sqrt(k / 4).  A fifth is left for the sample of rows; one chain would be 1.41 times the value."""
+    m, k, n = 1500, 768, 3072
+    rng = np.random.default_rng(11)
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    fb = FunctionBuilder("main", "F32")
+    fb.set_results([F.linear(fb.param("F32", [m, k]), fb.param("F32", [k, n]))])
+    rows = np.arange(0, m, 71)
+    got, want = hip_run(hip, Program(fb), [x, w])[0][rows], x[rows].astype(np.float64) @ w.astype(np.float64)
+    assert np.linalg.norm(got - want) <= 1.2 * 0.42 * 2.0 ** -24 * np.sqrt(k / 4) * np.linalg.norm(want)
+
+
 # codes converted on the way to the matrix pipes: odd columns, one k tile pair, k tiles that split in the middle of an int4 group, rows
 # around the tiles' 64 and 128
 @pytest.mark.parametrize("scheme", ["w8", "w4g128"])
