@@ -510,14 +510,14 @@ __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, T* __re
             float mx = mn;
 #pragma unroll
             for (int j = 0; j < 8; ++j) if (s0 + j < nsplit) mx = fmaxf(mx, m[j]);
-            if (mx == -INFINITY) mx = 0.f;     // nothing but empty records so far
-            const float c0 = expf(mn - mx);
+            const float at = mx == -INFINITY ? 0.f : mx;     // nothing but empty records so far: any finite stand-in, for these eight alone
+            const float c0 = expf(mn - at);
             L *= c0;
             O *= c0;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 if (s0 + j < nsplit) {
-                    const float c = expf(m[j] - mx);
+                    const float c = expf(m[j] - at);
                     L += l[j] * c;
                     O += o[j] * c;
                 }
