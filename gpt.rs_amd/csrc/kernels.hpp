@@ -286,7 +286,7 @@ struct MfmaLinearArgs {
     const void* scale; const void* scale2;
     // `part`: mfma_workspace_bytes() of scratch for the partial sums of tiles that are split over k; `tickets`
     // (kSkinnyTickets counters, zero before and after every launch) is where the register-staged kernel's splits of a tile
-    // meet; without them every tile runs whole
+    // meet; tiles are split as far as there is room, without any every tile runs whole
     void* part = nullptr; size_t part_bytes = 0; unsigned* tickets = nullptr;
     int out_f32 = 0;   // bf16 only: y and residual are f32
     EpiExtra extra;    // unquantised only
@@ -298,6 +298,9 @@ void mfma_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int64
 size_t mfma_codes_bytes(int64_t k, int64_t n, int quant);
 void mfma_pack_codes(hipStream_t s, const void* q, void* out, int64_t k, int64_t n, int quant);
 bool mfma_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n, int quant = 0);
+// Dynamic LDS that mfma_gemm() asks for int4 codes when `room` bytes of workspace are there (0: the register-staged kernel runs):
+// never more than a CU has, however little room there is.
+size_t mfma_int4_lds_bytes(int64_t m, int64_t k, int64_t n, bool dual, size_t room);
 void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a);
 
 // Rotate-half RoPE on packed [T, Q|K|V] rows (ops/functional/rotary.rs:430-536).

@@ -886,14 +886,17 @@ enum TileId { kT256x256, kT256x192, kT128x256, kT128x128, kT64x256, kT64x128, kT
 struct TilePlan { int tile; int splits; };
 constexpr int kTileLds = 160 * 1024;   // LDS of one CU
 
+// LDS of an int4 tile: a ring of three and, behind it, the scales of the groups of 128 k that a workgroup's share of K touches.
+static int64_t int4_lds_bytes(int64_t bm, int64_t bn, int64_t k, int64_t splits) { return 3 * (bm * 128 + bn * 32) + (cdiv(cdiv(k, 64), splits) / 2 + 2) * bn * 2; }
+
 template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL, int QF = 0>
 static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
     constexpr int ring = NST * (BM * KG * 16 + BN * KG * (QF == 0 ? 16 : QF == 1 ? 8 : 4)), rows = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4;
     constexpr int lds_most = QF == 2 ? kTileLds : ring > rows ? ring : rows;
     static_assert(ring <= kTileLds && lds_most <= kTileLds, "LDS of one CU");
-    // int4: behind the ring the scales of the groups of 128 k that a workgroup's share of K touches
-    const int lds_bytes = QF == 2 ? std::max(rows, ring + (int)(cdiv(cdiv(a.k, 64), splits) / 2 + 2) * BN * 2) : lds_most;
+    static_assert(QF != 2 || (NST == 3 && KG == 8), "int4_lds_bytes()");
+    const int lds_bytes = QF == 2 ? std::max(rows, (int)int4_lds_bytes(BM, BN, a.k, splits)) : lds_most;
     auto kern = gemm_tile_kernel<T, KG, NST, WM, WN, TM, TN, DUAL, QF>;
     static bool configured = false;  // the attribute is per function, not per stream or device state
     if (!configured) {
@@ -911,7 +914,9 @@ static size_t tile_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
     return splits > 1 ? (size_t)splits * m * cdiv(n, 8) * 8 * (dual ? 2 : 1) * sizeof(float) : 0;
 }
 
-// Which tile a launch takes, and over how many workgroups a tile's k is split.  Estimated time in us of every choice, from a
+constexpr size_t kMostPart = 64u << 20;   // bytes of partial sums that a plan may take
+
+// Which tile a launch takes, and over how many workgroups a tile's k is split, with `room` bytes for their partial sums.  Estimated time in us of every choice, from a
 // linear fit (within 6 % rms) to measurements at M = 40 .. 1500 of the 3072-wide layers (K = 3072, 4096, 9216; N = 3072, 6144,
 // a pair of 9216; weights from memory): rounds of workgroups x (fixed + per k tile of 64) + what a k tile costs more with the
 // chip full, and for a split the second launch plus its bytes.  What it picks is 1 % slower than the best measured choice,
@@ -921,7 +926,7 @@ static const TileCost kTileCost[kTiles] = {
     {256, 256, 256, 5.45, 1.237, 0.379, 2.8, 0.30}, {256, 192, 256, 1.16, 1.206, 0.122, 4.7, 0.35}, {128, 256, 256, 6.87, 0.661, 0.171, 3.1, 0.26},
     {128, 128, 256, 4.48, 0.425, 0.055, 3.9, 0.31}, {64, 256, 256, 4.59, 0.572, 0.0, 5.4, 0.13}, {64, 128, 512, 2.58, 0.361, 0.143, 5.0, 0.34},
 };
-static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual) {
+static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
     static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
     TilePlan best{kT256x256, 1};
     double least = 1e300;
@@ -930,7 +935,7 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual) {
         if (dual && c.bn == 192) continue;   // a pair's tile holds whole 64-column loads of either matrix
         const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
         for (int sp : {1, 2, 3, 4, 6, 8}) {
-            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > (64u << 20))) break;
+            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
             const double kt = (double)k / 64 / sp, wg = (double)(tiles * sp);
             double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
             if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
@@ -942,7 +947,6 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual) {
 template <bool DUAL>
 static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p) {
     typedef bf16_t T;
-    if (p.splits > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, DUAL, p.splits))) p.splits = 1;
     switch (p.tile) {
         case kT256x256: return launch_tile<T, 4, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits);
         case kT256x192: if constexpr (!DUAL) return launch_tile<T, 8, 2, 4, 2, 2, 3, false>(s, a, p.splits); else return;
@@ -960,12 +964,12 @@ static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p)
 // busy, and the small tile divides best among the CUs: M = 8192, K = 768, N = 3072 297 us = 130 TFLOP/s (64 x 128 304, 128 x 128
 // 316, 256 x 256 396), K = 3072, N = 768 273 = 141 (274, 354, 350); the register-staged 128 x 128 tiles took 366 and 354.
 // M = 400 (K = 768, N = 2304): 18 us (64 x 128 26).  Splits over k: rounds of 256 workgroups, a launch more and its bytes.
-static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual) {
+static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
     const int64_t tiles = cdiv(m, 64) * cdiv(n, 64);
     int best = 1;
     double least = 1e300;
     for (int sp : {1, 2, 3, 4, 6, 8}) {
-        if (sp > 1 && (k < 128 * sp || tile_part_bytes(m, n, dual, sp) > (64u << 20))) break;
+        if (sp > 1 && (k < 128 * sp || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
         double us = 5.0 + (dual ? 0.88 : 0.44) * ((double)k / 32 / sp) * (double)cdiv(tiles * sp, 256);
         if (sp > 1) us += 3.5 + 0.4 * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
         if (us < least) { least = us; best = sp; }
@@ -985,7 +989,7 @@ static const TileCost kQuantCost[2][kQTiles] = {
     {{256, 256, 0, 0, 0, 0, 0, 0}, {128, 256, 256, 4.87, 0.719, 0.337, 5.5, 0.15}, {128, 128, 512, 4.72, 0.486, 0.283, 6.3, 0.12}, {64, 128, 768, 4.25, 0.311, 0.207, 6.3, 0.09}},
     {{256, 256, 256, 3.15, 1.197, 1.059, 0.2, 0.24}, {128, 256, 256, 4.88, 0.870, 0.480, 3.9, 0.17}, {128, 128, 0, 0, 0, 0, 0, 0}, {64, 128, 768, 3.0, 0.524, 0.30, 4.0, 0.0}},
 };
-static TilePlan quant_plan(int64_t m, int64_t k, int64_t n, bool dual) {
+static TilePlan quant_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
     static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
     TilePlan best{-1, 1};
     double least = 1e300;
@@ -994,9 +998,8 @@ static TilePlan quant_plan(int64_t m, int64_t k, int64_t n, bool dual) {
         if (c.slots == 0) continue;
         const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
         for (int sp : {1, 2, 3, 4, 6, 8}) {
-            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > (64u << 20))) break;
-            // an int4 ring of three and the scales behind it, see launch_tile()
-            if (3 * (c.bm * 128 + c.bn * 32) + (cdiv(cdiv(k, 64), sp) / 2 + 2) * c.bn * 2 > kTileLds) continue;
+            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+            if (int4_lds_bytes(c.bm, c.bn, k, sp) > kTileLds) continue;   // int8 takes the same plan
             const double kt = (double)k / 64 / sp, wg = (double)(tiles * sp);
             double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
             if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
@@ -1046,11 +1049,17 @@ static void launch_staged(hipStream_t s, const MfmaLinearArgs& a, int splits = 1
                                       (int)full, splits, (float*)a.part, a.tickets, a.dtype == 2 ? a.out_f32 : 0, a.extra);
 }
 
+static size_t room_of(const MfmaLinearArgs& a) { return a.part ? a.part_bytes : 0; }
+size_t mfma_int4_lds_bytes(int64_t m, int64_t k, int64_t n, bool dual, size_t room) {
+    const TilePlan p = quant_plan(m, k, n, dual, room);
+    return p.tile < 0 ? 0 : (size_t)int4_lds_bytes(kQuantCost[dual][p.tile].bm, kQuantCost[dual][p.tile].bn, k, p.splits);
+}
+
 template <bool DUAL, int QF>
 static void launch_quant(hipStream_t s, const MfmaLinearArgs& a) {
-    const TilePlan p = quant_plan(a.m, a.k, a.n, DUAL);
+    const TilePlan p = quant_plan(a.m, a.k, a.n, DUAL, room_of(a));
     typedef bf16_t T;
-    const int sp = p.splits > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, DUAL, p.splits)) ? 1 : p.splits;
+    const int sp = p.splits;
     switch (p.tile) {
         case kQ256x256: if constexpr (DUAL) return launch_tile<T, 8, 3, 2, 4, 4, 2, true, QF>(s, a, sp); else return;
         case kQ128x256:
@@ -1077,12 +1086,11 @@ void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
     if (a.quant == 2) return dual ? launch_quant<true, 2>(s, a) : launch_quant<false, 2>(s, a);
     if (a.dtype == 0) {
         if (!reach) return dual ? launch_staged<float, true>(s, a) : launch_staged<float, false>(s, a);
-        int sp = tile_splits_f32(a.m, a.k, a.n, dual);
-        if (sp > 1 && (!a.part || a.part_bytes < tile_part_bytes(a.m, a.n, dual, sp))) sp = 1;
+        const int sp = tile_splits_f32(a.m, a.k, a.n, dual, room_of(a));
         return dual ? launch_tile<float, 8, 3, 2, 2, 1, 2, true>(s, a, sp) : launch_tile<float, 8, 3, 2, 2, 1, 1, false>(s, a, sp);
     }
     if (a.lds_direct != 0 && reach) {
-        const TilePlan p = tile_plan(a.m, a.k, a.n, dual);
+        const TilePlan p = tile_plan(a.m, a.k, a.n, dual, room_of(a));
         return dual ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);
     }
     // the splits of a quantised layer of this shape: its sums, in the same order over the dequantised matrix

@@ -1,0 +1,36 @@
+"""The plans of the MFMA GEMM that the host makes (kernels_mfma.hip), without a device."""
+import ctypes
+
+import pytest
+
+import __graft_entry__ as entry
+
+entry.load_package()
+from gptrs_amd import backend  # noqa: E402
+
+LDS = 160 * 1024   # of one CU
+
+
+def lib():
+    lib = backend.load_library()
+    lds, part = lib._ZN5gptrs1k19mfma_int4_lds_bytesElllbm, lib._ZN5gptrs1k20mfma_workspace_bytesEilllbi   # mfma_int4_lds_bytes, mfma_workspace_bytes
+    lds.argtypes, lds.restype = [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_size_t], ctypes.c_size_t
+    part.argtypes, part.restype = [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_int], ctypes.c_size_t
+    return lds, part
+
+
+@pytest.mark.parametrize("dual", [False, True])
+def test_int4_tiles_fit_whatever_the_workspace(dual):
+    """The scales of a workgroup's share of K lie in LDS: with the splits given up for want of room the share is all of K, and the tile has to be
+    one that holds them."""
+    lds, part = lib()
+    split = 0
+    for m in (17, 64, 200, 513, 1025, 4000):
+        for k in (128, 3072, 9216, 12288, 20480, 32768, 65536, 131072, 262144):
+            for n in (64, 1024, 3072, 9216):
+                need = part(2, m, k, n, dual, 2)
+                split += need > 0
+                for room in (need, need // 2, need - 1 if need else 0, 4096, 0):
+                    assert lds(m, k, n, dual, room) <= LDS, (m, k, n, room)
+                assert lds(m, k, n, dual, need) == lds(m, k, n, dual, 1 << 40)      # what the planner hands in is enough for its plan
+    assert split > 20
