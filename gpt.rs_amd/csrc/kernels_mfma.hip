@@ -915,6 +915,10 @@ static size_t tile_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
 }
 
 constexpr size_t kMostPart = 64u << 20;   // bytes of partial sums that a plan may take
+static bool splits_allowed() {
+    static const bool on = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
+    return on;
+}
 
 // Which tile a launch takes, and over how many workgroups a tile's k is split, with `room` bytes for their partial sums.  Estimated time in us of every choice, from a
 // linear fit (within 6 % rms) to measurements at M = 40 .. 1500 of the 3072-wide layers (K = 3072, 4096, 9216; N = 3072, 6144,
@@ -927,7 +931,6 @@ static const TileCost kTileCost[kTiles] = {
     {128, 128, 256, 4.48, 0.425, 0.055, 3.9, 0.31}, {64, 256, 256, 4.59, 0.572, 0.0, 5.4, 0.13}, {64, 128, 512, 2.58, 0.361, 0.143, 5.0, 0.34},
 };
 static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
-    static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
     TilePlan best{kT256x256, 1};
     double least = 1e300;
     for (int t = 0; t < kTiles; ++t) {
@@ -935,7 +938,7 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t roo
         if (dual && c.bn == 192) continue;   // a pair's tile holds whole 64-column loads of either matrix
         const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
         for (int sp : {1, 2, 3, 4, 6, 8}) {
-            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+            if (sp > 1 && (!splits_allowed() || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
             const double kt = (double)k / 64 / sp, wg = (double)(tiles * sp);
             double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
             if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
@@ -969,7 +972,7 @@ static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
     int best = 1;
     double least = 1e300;
     for (int sp : {1, 2, 3, 4, 6, 8}) {
-        if (sp > 1 && (k < 128 * sp || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+        if (sp > 1 && (!splits_allowed() || k < 128 * sp || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
         double us = 5.0 + (dual ? 0.88 : 0.44) * ((double)k / 32 / sp) * (double)cdiv(tiles * sp, 256);
         if (sp > 1) us += 3.5 + 0.4 * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
         if (us < least) { least = us; best = sp; }
@@ -990,7 +993,6 @@ static const TileCost kQuantCost[2][kQTiles] = {
     {{256, 256, 256, 3.15, 1.197, 1.059, 0.2, 0.24}, {128, 256, 256, 4.88, 0.870, 0.480, 3.9, 0.17}, {128, 128, 0, 0, 0, 0, 0, 0}, {64, 128, 768, 3.0, 0.524, 0.30, 4.0, 0.0}},
 };
 static TilePlan quant_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
-    static const bool allow_split = [] { const char* e = getenv("GPTRS_HIP_GEMM_TAILSPLIT"); return !(e && e[0] == '0'); }();
     TilePlan best{-1, 1};
     double least = 1e300;
     for (int t = 0; t < kQTiles; ++t) {
@@ -998,7 +1000,7 @@ static TilePlan quant_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
         if (c.slots == 0) continue;
         const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
         for (int sp : {1, 2, 3, 4, 6, 8}) {
-            if (sp > 1 && (!allow_split || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+            if (sp > 1 && (!splits_allowed() || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
             if (int4_lds_bytes(c.bm, c.bn, k, sp) > kTileLds) continue;   // int8 takes the same plan
             const double kt = (double)k / 64 / sp, wg = (double)(tiles * sp);
             double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;

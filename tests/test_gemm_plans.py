@@ -1,5 +1,8 @@
 """The plans of the MFMA GEMM that the host makes (kernels_mfma.hip), without a device."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -34,3 +37,14 @@ def test_int4_tiles_fit_whatever_the_workspace(dual):
                     assert lds(m, k, n, dual, room) <= LDS, (m, k, n, room)
                 assert lds(m, k, n, dual, need) == lds(m, k, n, dual, 1 << 40)      # what the planner hands in is enough for its plan
     assert split > 20
+
+
+def test_the_split_switch_reaches_every_type():
+    """GPTRS_HIP_GEMM_TAILSPLIT=0 (read once per process): no tile of f32, bf16 or codes is split, so none has partial sums."""
+    sizes = [(d, 100, k, 768, dual, q) for d, q in ((0, 0), (2, 0), (2, 1), (2, 2)) for k in (3072, 9216) for dual in (False, True)]
+    _, part = lib()
+    assert all(part(*s) > 0 for s in sizes)
+    code = f"import sys; sys.path[:0] = {sys.path!r}\nimport test_gemm_plans as t; part = t.lib()[1]\nprint([part(*s) for s in {sizes!r}])"
+    out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, GPTRS_HIP_GEMM_TAILSPLIT="0"), cwd=os.path.dirname(os.path.abspath(__file__)),
+                         stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert out.strip() == str([0] * len(sizes))
