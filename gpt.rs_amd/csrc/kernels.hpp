@@ -290,7 +290,7 @@ struct MfmaLinearArgs {
     void* part = nullptr; size_t part_bytes = 0; unsigned* tickets = nullptr;
     int out_f32 = 0;   // bf16 only: y and residual are f32
     EpiExtra extra;    // unquantised only
-    int lds_direct = 1;   // unquantised bf16: the LDS-direct kernel where it applies (0: the register-staged one)
+    int lds_direct = 1;   // the LDS-direct kernel where it applies (0: the register-staged one)
 };
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant);
 size_t mfma_weight_bytes(int dtype, int64_t k, int64_t n);

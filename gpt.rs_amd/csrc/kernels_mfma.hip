@@ -1027,8 +1027,7 @@ size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dua
     if (!mfma_gemm_supported(dtype, m, k, n, quant)) return 0;
     if (dtype == 0) return tile_part_bytes(m, n, dual, tile_splits_f32(m, k, n, dual));
     const int qsp = quant_plan(m, k, n, dual).splits;
-    if (quant) return tile_part_bytes(m, n, dual, qsp);
-    return std::max(tile_part_bytes(m, n, dual, tile_plan(m, k, n, dual).splits), staged_part_bytes(m, n, dual, qsp));
+    return std::max(tile_part_bytes(m, n, dual, quant ? qsp : tile_plan(m, k, n, dual).splits), staged_part_bytes(m, n, dual, qsp));
 }
 
 template <typename T, bool DUAL, int QF = 0>
@@ -1080,24 +1079,22 @@ void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
     // the LDS-direct kernel's loads address a k tile with 32-bit offsets from one scalar base: 256 rows of x, 8 k-groups of
     // the padded weights
     const bool reach = a.k <= (1 << 21) && (uint64_t)mfma_padded_n(a.n) * 128 < (1ull << 31);
-    if (a.quant && !reach) {
-        if (a.quant == 1) return dual ? launch_staged<bf16_t, true, 1>(s, a) : launch_staged<bf16_t, false, 1>(s, a);
-        return dual ? launch_staged<bf16_t, true, 2>(s, a) : launch_staged<bf16_t, false, 2>(s, a);
+    if (a.lds_direct == 0 || !reach) {
+        // the splits of a layer of codes of this shape, for them and for the matrix that they stand for: the same sums in the same order
+        const int sp = reach && a.dtype == 2 ? quant_plan(a.m, a.k, a.n, dual).splits : 1;
+        if (a.dtype == 0) return dual ? launch_staged<float, true>(s, a) : launch_staged<float, false>(s, a);
+        if (a.quant == 1) return dual ? launch_staged<bf16_t, true, 1>(s, a, sp) : launch_staged<bf16_t, false, 1>(s, a, sp);
+        if (a.quant == 2) return dual ? launch_staged<bf16_t, true, 2>(s, a, sp) : launch_staged<bf16_t, false, 2>(s, a, sp);
+        return dual ? launch_staged<bf16_t, true>(s, a, sp) : launch_staged<bf16_t, false>(s, a, sp);
     }
     if (a.quant == 1) return dual ? launch_quant<true, 1>(s, a) : launch_quant<false, 1>(s, a);
     if (a.quant == 2) return dual ? launch_quant<true, 2>(s, a) : launch_quant<false, 2>(s, a);
     if (a.dtype == 0) {
-        if (!reach) return dual ? launch_staged<float, true>(s, a) : launch_staged<float, false>(s, a);
         const int sp = tile_splits_f32(a.m, a.k, a.n, dual, room_of(a));
         return dual ? launch_tile<float, 8, 3, 2, 2, 1, 2, true>(s, a, sp) : launch_tile<float, 8, 3, 2, 2, 1, 1, false>(s, a, sp);
     }
-    if (a.lds_direct != 0 && reach) {
-        const TilePlan p = tile_plan(a.m, a.k, a.n, dual, room_of(a));
-        return dual ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);
-    }
-    // the splits of a quantised layer of this shape: its sums, in the same order over the dequantised matrix
-    const int sp = reach ? quant_plan(a.m, a.k, a.n, dual).splits : 1;
-    return dual ? launch_staged<bf16_t, true>(s, a, sp) : launch_staged<bf16_t, false>(s, a, sp);
+    const TilePlan p = tile_plan(a.m, a.k, a.n, dual, room_of(a));
+    return dual ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);
 }
 
 }  // namespace k

@@ -196,9 +196,9 @@ int gptrs_hip_synchronize(gptrs_hip_backend* b);
  * persistent launch only when they stream at least this many KiB of weights each on average: a phase of the launch costs
  * what a small stand-alone kernel costs; GPT-2 small (7 MB per layer) runs on the launch (its steady decode step takes the
  * same time either way, a whole generate call of 64 tokens is 7 % shorter), narrower f32 models on stand-alone kernels; 0 = always.
- * "gemm_lds_direct" (default 1) = unquantised bf16 linear layers of more than 16 rows run on the GEMM whose tiles go from
- * memory to LDS without passing through registers; 0 = on the register-staged GEMM that serves f32 and quantised weights
- * (the two sum in different orders: results agree to bf16 rounding, not bit for bit).
+ * "gemm_lds_direct" (default 1) = linear layers of more than 16 rows run on the GEMM whose tiles go from memory to LDS
+ * without passing through registers; 0 = on the register-staged GEMM (quantised weights: the same sums in the same order;
+ * unquantised: another order, results agree to rounding, not bit for bit).
  * "chain_stall_phase" (default -1; a test hook) = value >= 1: the next persistent launch expects, at that phase's grid
  * barrier, one arrival more than its workgroups can deliver, so that its bounded wait gives up: the call that next
  * synchronises reports an Execution error and the option returns to -1.

@@ -77,17 +77,27 @@ def test_f32_tiles_and_splits(hip, m, k, n):
         assert np.array_equal(got, hip_run(hip, p, args)[0])
         return got
 
-    plain = run([(f32, [m, k]), mat, (f32, [m, n])], lambda a, b, r: F.linear(a, b) + r, [x, w, res])
-    biased = run([(f32, [m, k]), mat, (f32, [n])], lambda a, b, c: F.linear(a, b, c), [x, w, bias])
-    pair = run([(f32, [m, k]), mat, mat], lambda a, b, c: F.swiglu(F.linear(a, b), F.linear(a, c)), [x, w, w2])
+    def all_three():
+        return (run([(f32, [m, k]), mat, (f32, [m, n])], lambda a, b, r: F.linear(a, b) + r, [x, w, res]),
+                run([(f32, [m, k]), mat, (f32, [n])], lambda a, b, c: F.linear(a, b, c), [x, w, bias]),
+                run([(f32, [m, k]), mat, mat], lambda a, b, c: F.swiglu(F.linear(a, b), F.linear(a, c)), [x, w, w2]))
+
+    tiles = all_three()
+    hip.set_option("gemm_lds_direct", 0)
+    try:
+        staged = all_three()
+    finally:
+        hip.set_option("gemm_lds_direct", 1)
+    assert not np.array_equal(tiles[0], staged[0]) or k <= 32      # another order of the sums: the switch has taken the other kernel
     x64, w64, v64 = x.astype(np.float64), w.astype(np.float64), w2.astype(np.float64)
     s, t = x64 @ w64, x64 @ v64
     # as above: 2 sqrt(k) roundings of the sum of magnitudes, and one for each operation behind the sum
     bs, bt = (2 * np.sqrt(k) * 2.0 ** -24 * (np.abs(x64) @ np.abs(v)) + 1e-6 for v in (w64, v64))
-    assert (np.abs(plain - (s + res)) <= bs + 2.0 ** -23 * np.abs(s + res)).all()
-    assert (np.abs(biased - (s + bias)) <= bs + 2.0 ** -23 * np.abs(s + bias)).all()
     g = s / (1 + np.exp(-s))
-    assert (np.abs(pair - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + 2.0 ** -20 * np.abs(g * t) + 1e-6).all()
+    for plain, biased, pair in (tiles, staged):
+        assert (np.abs(plain - (s + res)) <= bs + 2.0 ** -23 * np.abs(s + res)).all()
+        assert (np.abs(biased - (s + bias)) <= bs + 2.0 ** -23 * np.abs(s + bias)).all()
+        assert (np.abs(pair - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + 2.0 ** -20 * np.abs(g * t) + 1e-6).all()
 
 
 def test_f32_sums_in_two_chains(hip):
@@ -122,10 +132,12 @@ def test_codes_equal_the_dequantised_matrix(hip, scheme, m, k, n):
     hip.set_option("gemm_lds_direct", 0)
     try:
         want = [hip_run(hip, p, a)[0] for p, a in zip(plain, ([x, w], [x, w, w2]))]
+        staged = [hip_run(hip, p, a)[0] for p, a in zip(codes, ([x, q, s], [x, q, s, q2, s2]))]
     finally:
         hip.set_option("gemm_lds_direct", 1)
-    for g, v in zip(got, want):
+    for g, v, r in zip(got, want, staged):
         assert np.array_equal(g, v)      # the same products, added in the same order
+        assert np.array_equal(r, v)      # so does the register-staged kernel over codes
 
 
 # a pair's gate is one function for prompts and for decode steps (kernels_skinny.hip), also far below zero, where e^-g nears the largest
