@@ -133,10 +133,20 @@ __device__ __forceinline__ uint32_t mfma_pack_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));   // round to nearest even
 }
 
-// A pair's output, the function that the decode kernels form (activation.rs:141-162): 28 instructions, 4 us of a 256 x 256 tile's 86 more than exp2 and a
-// reciprocal alone would take (M = 8188, pair of 9216: 773 us against 737), but those are off by up to 65 ulp of f32 where g is far below
-// zero, against 3, and lose the result altogether from -87.4 on, where the reciprocal is subnormal.
-__device__ __forceinline__ float gemm_glu(float g, float u, const GluParams& p) { return glu_combine(g, u, p.kind, p.limit, p.alpha, p.shift); }
+// Pairs' outputs from their N gates and up sums, the function that the decode kernels form (activation.rs:141-162): 28 instructions each, 4 us of a
+// 256 x 256 tile's 86 more than exp2 and a reciprocal alone would take (pair of 9216, M = 8188: 789 us against 756), but those are off by up
+// to 65 ulp of f32 where the gate is far below zero, against 3, and lose the result altogether from -87.4 on, where the
+// reciprocal is subnormal.  The kind is looked at once, not at every output (420 us against 423 at M = 4000).
+template <int N, typename G, typename U>
+__device__ __forceinline__ void gemm_glu(G&& g, const U& u, const GluParams& p) {
+    if (p.kind == 1) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) g[e] = glu_combine(g[e], u[e], 1, p.limit, p.alpha, p.shift);
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) g[e] = glu_combine(g[e], u[e], 0, p.limit, p.alpha, p.shift);
+    }
+}
 
 __device__ __forceinline__ float mfma_finish(float v, int act, float bias, bool has_res, float res, float colscale) {
     v += bias;                                                // tensor_ops.rs:42-56
@@ -455,6 +465,12 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
     // through LDS to store rows of 8, as the LDS-direct kernel below does, changed nothing here: 19.0 against 19.1 us at
     // K = 192, M = 1024, N = 6144)
     constexpr int TNO = DUAL ? TN / 2 : TN;
+    if constexpr (DUAL) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TNO; ++j) gemm_glu<16>(acc[i][j], acc[i][j + TNO], extra.glu);
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -470,8 +486,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
                 // out_f32: the f32 accumulator (plus an f32 residual) is stored as it is
                 const float r = residual ? (out_f32 ? reinterpret_cast<const float*>(residual)[(int64_t)m * N + n]
                                                     : Mma<T>::ld(residual, (int64_t)m * N + n)) : 0.f;
-                const float g = DUAL ? gemm_glu(acc[i][j][v], acc[i][DUAL ? j + TN / 2 : j][v], extra.glu) : acc[i][j][v];
-                const float o = mfma_finish(g, act, bv, residual != nullptr, r, cs);
+                const float o = mfma_finish(acc[i][j][v], act, bv, residual != nullptr, r, cs);
                 if (out_f32) reinterpret_cast<float*>(y)[(int64_t)m * N + n] = o;
                 else Mma<T>::st(y, (int64_t)m * N + n, o);
             }
@@ -484,7 +499,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
 // those of bf16; f32 has 4 k where bf16 has 8 and moves the same bytes.
 //
 // Workgroup: WM x WN waves; a wave owns (32 TM) x (32 TN) outputs as TM x TN fragments of 32 x 32, the tile is
-// BM x BN = (32 TM WM) x (32 TN WN).  A bf16 launch takes one of six tiles and a number of splits over k, see tile_plan().
+// BM x BN = (32 TM WM) x (32 TN WN).  KW = 2: two such groups of waves share the staged tiles, each multiplies half of every k tile, and
+// their sums meet through LDS in front of the epilogue.  A bf16 launch takes one of seven tiles and a number of splits over k, see tile_plan().
 //
 // What bounds it (bf16).  256 x 256 tiles, all CUs busy: the matrix pipes at the clock that random operands allow.  A tile's 32 k
 // take 0.54 us on a quarter of the CUs and 0.8 us on all of them; over all-zero operands the same launch runs at 1.35 times
@@ -496,6 +512,9 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
 // weights from memory) qkv 32 -> 28, out and down 51 (mean) -> 29 with the launch that adds the splits, pair 81 -> 49.  k tiles of 32 in a ring of four beat k tiles of 64 in
 // a ring of two there (1035 -> 1239 TFLOP/s: loads have three k tiles of time, not one); 4 waves of 128 x 128 lose (1090).
 // Smaller tiles are for launches whose 256 x 256 tiles would leave CUs without work; they stage 64 k, the memory's lines.
+// 128 x 192 in two k-groups of 2 x 2 waves: 8 waves that still read 5 fragments for 6 MFMAs (8 waves of 32 x 96 read 4 for 3, more than LDS
+// delivers), for launches that its tiles fill in whole rounds: M = 1000, weights from memory, us against the best of the other six: N = 6144
+// 44.6 -> 40.5, pair of 9216 153 -> 129, K = 9216 68 -> 64; M = 2047, K = 9216 117 -> 105; M = 6000, K = 9216 359 -> 304.
 //
 // LDS, per stage: A as rows of 2 BK bytes, B k-group-major ([k-group][column][8 k]).  One load instruction moves
 // 64 x 16 bytes to 1 KiB of consecutive LDS, lane l to byte 16 l, so the layout is fixed by WHICH 16 bytes of memory a
@@ -511,7 +530,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
 // MFMAs run at raised wave priority, so that the two waves of a SIMD take turns instead of stalling on each other's LDS
 // reads (k tiles of 64: 1035 -> 1167 TFLOP/s; of 32: within the noise).
 // DUAL (SwiGLU pair): the tile's first BN / 2 columns are columns of W, the others the same columns of W2, and a wave
-// multiplies the same 16 TN columns of both, so gate and up of an output meet in one lane.
+// multiplies the same 16 TN columns of both, so gate and up of an output meet in one lane; with an odd TN wave column 0 multiplies
+// W and wave column 1 W2, and they meet in the epilogue's LDS.
 // One load instruction: lane l asks for the 16 bytes at base + offset(l) (a scalar base and a 32-bit offset per lane, so
 // stepping to the next k tile is scalar arithmetic; vector instructions in the step loop cost the matrix pipe issue
 // slots: per-lane 64-bit addresses were 5-10 % slower) and they land at LDS byte lds_addr + 16 l.
@@ -535,8 +555,9 @@ struct TileEpilogue {
 // Eight neighbours of row m, columns n .. n + 7, from LDS: bias, GELU, column factor and residual, then one 16-byte store (two
 // for f32 results; element by element when N is not a multiple of 8).  Kept short: with every output's options unrolled the
 // epilogue was 13 000 to 18 000 instructions, more than the instruction cache holds (M = 8188, see gemm_tile_kernel).
-template <typename T>
-__device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m, int64_t n, const float* at_lds) {
+// PAIR: `at_lds` holds gates and `up_lds` the up sums, still to be combined.
+template <typename T, bool PAIR>
+__device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m, int64_t n, const float* at_lds, const float* up_lds) {
     const int64_t at = m * p.N + n;
     const bool f32 = std::is_same<T, float>::value || p.out_f32;     // y and residual
     if ((p.N & 7) != 0) {
@@ -545,7 +566,9 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m
             if (n + e >= p.N) break;
             const float bv = p.bias ? Mma<T>::ld(p.bias, n + e) : 0.f;
             const float rv = p.residual ? (f32 ? static_cast<const float*>(p.residual)[at + e] : Mma<T>::ld(static_cast<const T*>(p.residual), at + e)) : 0.f;
-            const float f = mfma_finish(at_lds[e], p.act, bv, p.residual != nullptr, rv, p.extra.colscale ? p.extra.colscale[n + e] : 1.0f);
+            float sum[1] = {at_lds[e]};
+            if constexpr (PAIR) gemm_glu<1>(sum, up_lds + e, p.extra.glu);
+            const float f = mfma_finish(sum[0], p.act, bv, p.residual != nullptr, rv, p.extra.colscale ? p.extra.colscale[n + e] : 1.0f);
             if (f32) static_cast<float*>(p.y)[at + e] = f;
             else Mma<T>::st(static_cast<T*>(p.y), at + e, f);
         }
@@ -554,6 +577,12 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m
     float o[8];
     *reinterpret_cast<f32x4_t*>(o) = *reinterpret_cast<const f32x4_t*>(at_lds);
     *reinterpret_cast<f32x4_t*>(o + 4) = *reinterpret_cast<const f32x4_t*>(at_lds + 4);
+    if constexpr (PAIR) {
+        float u[8];
+        *reinterpret_cast<f32x4_t*>(u) = *reinterpret_cast<const f32x4_t*>(up_lds);
+        *reinterpret_cast<f32x4_t*>(u + 4) = *reinterpret_cast<const f32x4_t*>(up_lds + 4);
+        gemm_glu<8>(o, u, p.extra.glu);
+    }
     auto add_f32 = [&](const float* v) {
         const f32x4_t r0 = *reinterpret_cast<const f32x4_t*>(v), r1 = *reinterpret_cast<const f32x4_t*>(v + 4);
 #pragma unroll
@@ -594,28 +623,34 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m
         *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(p.y) + at) = w;
     }
 }
-template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL, int QF>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __restrict__ x, const T* __restrict__ wk, const T* __restrict__ wk2,
+template <typename T, int KG, int NST, int WM, int WN, int KW, int TM, int TN, bool DUAL, int QF>
+__global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* __restrict__ x, const T* __restrict__ wk, const T* __restrict__ wk2,
                                                                  int M, int K, int Npad, int NT, int MT, int splits, float* __restrict__ part, const T* __restrict__ scale, const T* __restrict__ scale2,
                                                                  TileEpilogue<T> epi) {
     static_assert(KG == 4 || KG == 8, "k-groups of a k tile");
     typedef typename Mma<T>::frag frag_t;
     constexpr int BK = KG * Mma<T>::KPC, ROWB = KG * 16, KS = KG / 2;  // k of a tile, bytes of an A row, k-steps
-    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NW = WM * WN;
+    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NW = WM * WN * KW;
     constexpr int NREAL = DUAL ? BN / 2 : BN;                          // output columns per tile
-    constexpr int TNO = DUAL ? TN / 2 : TN;                            // output fragments per wave and row
+    constexpr bool ACROSS = DUAL && TN % 2 != 0;                       // a pair's matrices are the two wave columns, not halves of a wave's fragments
+    constexpr int TNO = DUAL && !ACROSS ? TN / 2 : TN;                 // output fragments per wave and row
+    constexpr int KSW = KS / KW, TMO = TM / KW;                        // k-steps of a k-group of waves; rows of fragments that a wave finishes
     constexpr int CB = QF == 0 ? 16 : QF == 1 ? 8 : 4;                 // bytes of a column's k-group
     constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * KG * CB, STAGE = A_BYTES + B_BYTES;
     constexpr int LAI = A_BYTES / 1024, LBI = B_BYTES / 1024;          // load instructions per tile
     constexpr int LA = LAI / NW, LB = (LBI + NW - 1) / NW, LPT = LA + LB;   // per wave (with fewer instructions than waves, two waves bring the same)
     static_assert(LA * NW == LAI && LBI * 1024 == B_BYTES && (LB * NW == LBI || NW % LBI == 0), "whole load instructions per wave");
     static_assert(QF == 0 || (KG == 8 && std::is_same<T, bf16_t>::value), "codes: bf16 activations, k tiles of 64");
-    static_assert(KS % 2 == 0, "the last k-step's fragments sit in slot 1, the next tile's first in slot 0");
-    static_assert(!DUAL || (TN % 2 == 0 && NREAL * KG * CB % 1024 == 0), "a load instruction belongs to one matrix of the pair");
+    static_assert(KSW % 2 == 0, "the last k-step's fragments sit in slot 1, the next tile's first in slot 0");
+    static_assert(!DUAL || NREAL * KG * CB % 1024 == 0, "a load instruction belongs to one matrix of the pair");
+    static_assert(KW == 1 || (KW == 2 && TM % 2 == 0 && QF == 0 && std::is_same<T, bf16_t>::value), "two k-groups halve the rows of their sums");
+    static_assert(!DUAL || ACROSS || KW == 1, "a wave's own pairs are combined where they were summed");
+    static_assert(!ACROSS || (WN == 2 && TMO == 1 && QF == 0), "wave column 0 multiplies W, wave column 1 the same columns of W2");
     static_assert((NST - 2) * LPT < 64, "vmcnt is a 6-bit counter");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
+    const int wg = KW == 1 ? 0 : wave / (WM * WN), wq = KW == 1 ? wave : wave % (WM * WN);   // k-group; place in it
+    const int wm = wq / WN, wn = wq % WN;
     int bx, by, sidx;
     {
         // XCD c takes a contiguous range of a grouped tile order (see gemm_mfma_kernel: 8 row blocks by 4 column tiles run on
@@ -681,7 +716,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
 #pragma unroll
                 for (int v = 0; v < 16; ++v) sums[c][i][j][v] = 0.f;
     const int fsel = lane >> 5;
-    const int b_rd = A_BYTES + (wn * 32 * TNO + (lane & 31)) * CB;
+    const int b_rd = A_BYTES + (ACROSS ? wn * (NREAL * KG * CB) : wn * 32 * TNO * CB) + (lane & 31) * CB;
     typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
     typedef typename std::conditional<QF == 0, frag_t, typename std::conditional<QF == 1, u32x2_t, uint32_t>::type>::type raw_t;
     frag_t af[2][TM], bq[QF == 0 ? 1 : TN];
@@ -705,7 +740,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
             sc_lds[e] = (DUAL && c >= NREAL ? scale2 : scale)[(int64_t)g * epi.N + (col < epi.N ? col : epi.N - 1)];
         }
     }
-    auto fread = [&](int st, int kk, int slot) {   // kk: k-step of the tile
+    auto fread = [&](int st, int kw, int slot) {   // kw: k-step of the k-group
+        const int kk = wg * KSW + kw;
         const unsigned char* base = lds + st * STAGE;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -714,7 +750,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
         }
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-            bfr[slot][j] = *reinterpret_cast<const raw_t*>(base + b_rd + (2 * kk + fsel) * (NREAL * CB) + (j / TNO) * (NREAL * KG * CB) + (j % TNO) * 32 * CB);
+            bfr[slot][j] = *reinterpret_cast<const raw_t*>(base + b_rd + (2 * kk + fsel) * (NREAL * CB) + (j / TNO) * (NREAL * KG * CB) + (j % TNO) * 32 * CB);   // ACROSS: j < TNO
     };
     // codes -> the bf16 values of the dequantised matrix, bf16(code * scale): u * s - bias * s is exactly (u - bias) * s, rounded
     // once like the product the dequantiser forms
@@ -767,10 +803,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
             for (int j = 0; j < TN; ++j) sc[j] = bf16_to_f32(sc_lds[g * BN + (j / TNO) * NREAL + (wn * TNO + j % TNO) * 32 + (lane & 31)]);
         }
 #pragma unroll
-        for (int kk = 0; kk + 1 < KS; ++kk) {
+        for (int kk = 0; kk + 1 < KSW; ++kk) {
             fread(ST, kk + 1, (kk + 1) & 1);
             dequantise(kk & 1);
-            mul(kk & 1, 0, TM * TN, 2 * kk / KS);
+            mul(kk & 1, 0, TM * TN, 2 * kk / KSW);
         }
         dequantise(1);
         mul(1, 0, TM * TN / 2, 1);
@@ -807,45 +843,82 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const T* __rest
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) acc[i][j] += sums[c][i][j];
+    // two k-groups: group g gives the sums of the other half of its rows of fragments away and keeps half g, through LDS (the staged tiles
+    // are dead: nothing is in flight, and every wave has read its last fragments in front of the last step's barrier)
+    f32x16_t kept[KW == 1 ? 1 : TMO][KW == 1 ? 1 : TN];
+    if constexpr (KW == 2) {
+        constexpr int XCH = TMO * TN * 16 * 64;
+        float* give = reinterpret_cast<float*>(lds) + wave * XCH + lane;
+        const float* take = reinterpret_cast<const float*>(lds) + (wg == 0 ? wave + WM * WN : wave - WM * WN) * XCH + lane;
+        auto hand_over = [&](int from) {
+#pragma unroll
+            for (int i = 0; i < TMO; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) give[((i * TN + j) * 16 + v) * 64] = acc[from + i][j][v];
+        };
+        auto keep = [&](int from) {
+#pragma unroll
+            for (int i = 0; i < TMO; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) kept[i][j][v] = acc[from + i][j][v] + take[((i * TN + j) * 16 + v) * 64];
+        };
+        if (wg == 0) hand_over(TMO);
+        else hand_over(0);
+        __syncthreads();
+        if (wg == 0) keep(0);
+        else keep(TMO);
+        __syncthreads();   // every wave has taken its half before the area is written again
+    }
+    auto sum = [&](int i, int j, int v) {
+        if constexpr (KW == 1) return acc[i][j][v];
+        else return kept[i][j][v];
+    };
+    const int mw = m0 + (wm * TM + wg * TMO) * 32, nw = n0 + (ACROSS ? 0 : wn * 32 * TNO);   // the wave's first output
     if (splits > 1) {
         // partial sums, [split][row][columns padded to 8] f32 (a pair: W's columns, then W2's); gemm_reduce_kernel adds them
         const int np = ((int)epi.N + 7) & ~7, width = DUAL ? 2 * np : np;
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TMO; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                const int n = n0 + (wn * TNO + j % TNO) * 32 + (lane & 31);
+                const int n = nw + (j % TNO) * 32 + (lane & 31);
                 if (n >= np) continue;
-                float* to = part + (int64_t)sidx * M * width + (DUAL ? (j / TNO) * np : 0) + n;
+                float* to = part + (int64_t)sidx * M * width + (ACROSS ? wn * np : DUAL ? (j / TNO) * np : 0) + n;
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
-                    const int m = m0 + (wm * TM + i) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                    if (m < M) to[(int64_t)m * width] = acc[i][j][v];
+                    const int m = mw + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                    if (m < M) to[(int64_t)m * width] = sum(i, j, v);
                 }
             }
         return;
     }
     // Rows of 8 outputs: 32 x (32 TNO) sums at a time go through an LDS area of the wave's own (a lane holds one column of
-    // four-row groups, memory wants runs along a row).  The staged tiles are dead: nothing is in flight, and every wave has
-    // read its last fragments in front of the last step's barrier.
+    // four-row groups, memory wants runs along a row).  ACROSS: the two waves of a pair meet here, each takes half of the chunks and reads both areas.
     constexpr int RSF = 32 * TNO + 4;    // floats per row of an area
     constexpr int CH = 4 * TNO;          // chunks of 8 per row
+    constexpr int PASSES = ACROSS ? CH / 4 : CH / 2;
+    static_assert(!ACROSS || CH % 4 == 0, "whole passes of either wave");
     float* area = reinterpret_cast<float*>(lds) + wave * (32 * RSF);
+    const float* gates = ACROSS ? area - wn * (32 * RSF) : area;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i = 0; i < TMO; ++i) {
 #pragma unroll
-        for (int j = 0; j < TNO; ++j)
+        for (int j = 0; j < TNO; ++j) {
+            if constexpr (DUAL && !ACROSS) gemm_glu<16>(acc[i][j], acc[i][j + TNO], epi.extra.glu);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                float o = acc[i][j][v];
-                if (DUAL) o = gemm_glu(o, acc[i][DUAL ? j + TNO : j][v], epi.extra.glu);
-                area[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * RSF + j * 32 + (lane & 31)] = o;
+            for (int v = 0; v < 16; ++v)
+                area[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * RSF + j * 32 + (lane & 31)] = sum(i, j, v);
             }
+        if (ACROSS) __syncthreads();
 #pragma unroll 1
-        for (int it = 0; it < CH / 2; ++it) {
-            const int c = it * 64 + lane, r = c / CH, cc = c % CH;
-            const int m = m0 + (wm * TM + i) * 32 + r, n = n0 + wn * 32 * TNO + cc * 8;
-            if (m < M && n < epi.N) gemm_finish8(epi, m, n, area + r * RSF + cc * 8);
+        for (int it = 0; it < PASSES; ++it) {
+            const int c = (ACROSS ? wn * PASSES + it : it) * 64 + lane, r = c / CH, cc = c % CH;
+            const int m = mw + i * 32 + r, n = nw + cc * 8;
+            if (m < M && n < epi.N) gemm_finish8<T, ACROSS>(epi, m, n, gates + r * RSF + cc * 8, gates + 32 * RSF + r * RSF + cc * 8);
         }
     }
 }
@@ -875,29 +948,29 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
     if (DUAL) {
         float u[8];
         sum8(part + m * width + np + n, u);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = gemm_glu(o[e], u[e], epi.extra.glu);
+        gemm_glu<8>(o, u, epi.extra.glu);
     }
-    gemm_finish8(epi, m, n, o);
+    gemm_finish8<T, false>(epi, m, n, o, nullptr);
 }
 
 // The tiles, in the order of tile_cost's table.
-enum TileId { kT256x256, kT256x192, kT128x256, kT128x128, kT64x256, kT64x128, kTiles };
+enum TileId { kT256x256, kT256x192, kT128x256, kT128x192, kT128x128, kT64x256, kT64x128, kTiles };
 struct TilePlan { int tile; int splits; };
 constexpr int kTileLds = 160 * 1024;   // LDS of one CU
 
 // LDS of an int4 tile: a ring of three and, behind it, the scales of the groups of 128 k that a workgroup's share of K touches.
 static int64_t int4_lds_bytes(int64_t bm, int64_t bn, int64_t k, int64_t splits) { return 3 * (bm * 128 + bn * 32) + (cdiv(cdiv(k, 64), splits) / 2 + 2) * bn * 2; }
 
-template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL, int QF = 0>
+template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL, int QF = 0, int KW = 1>
 static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
-    constexpr int ring = NST * (BM * KG * 16 + BN * KG * (QF == 0 ? 16 : QF == 1 ? 8 : 4)), rows = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4;
+    constexpr int ring = NST * (BM * KG * 16 + BN * KG * (QF == 0 ? 16 : QF == 1 ? 8 : 4)), area = WM * WN * KW * 32 * (32 * (DUAL && TN % 2 == 0 ? TN / 2 : TN) + 4) * 4;
+    constexpr int rows = KW == 1 ? area : std::max(area, WM * WN * KW * (TM / KW) * TN * 16 * 64 * 4);   // what the epilogue puts where the ring was
     constexpr int lds_most = QF == 2 ? kTileLds : ring > rows ? ring : rows;
     static_assert(ring <= kTileLds && lds_most <= kTileLds, "LDS of one CU");
     static_assert(QF != 2 || (NST == 3 && KG == 8), "int4_lds_bytes()");
     const int lds_bytes = QF == 2 ? std::max(rows, (int)int4_lds_bytes(BM, BN, a.k, splits)) : lds_most;
-    auto kern = gemm_tile_kernel<T, KG, NST, WM, WN, TM, TN, DUAL, QF>;
+    auto kern = gemm_tile_kernel<T, KG, NST, WM, WN, KW, TM, TN, DUAL, QF>;
     static bool configured = false;  // the attribute is per function, not per stream or device state
     if (!configured) {
         (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_most);
@@ -905,7 +978,7 @@ static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
     }
     const int64_t nt = cdiv(a.n, NREAL), mt = cdiv(a.m, BM);
     TileEpilogue<T> epi{(const T*)a.bias, a.residual, a.y, a.n, a.act, a.out_f32, a.extra};
-    kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (int)a.m, (int)a.k,
+    kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN * KW, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (int)a.m, (int)a.k,
                                                                                    (int)mfma_padded_n(a.n), (int)nt, (int)mt, splits, (float*)a.part,
                                                                                    (const T*)a.scale, (const T*)a.scale2, epi);
     if (splits > 1) gemm_reduce_kernel<T, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
@@ -921,13 +994,13 @@ static bool splits_allowed() {
 }
 
 // Which tile a launch takes, and over how many workgroups a tile's k is split, with `room` bytes for their partial sums.  Estimated time in us of every choice, from a
-// linear fit (within 6 % rms) to measurements at M = 40 .. 1500 of the 3072-wide layers (K = 3072, 4096, 9216; N = 3072, 6144,
+// linear fit (within 6 % rms, 128 x 192 10 %) to measurements at M = 40 .. 1500 of the 3072-wide layers (K = 3072, 4096, 9216; N = 3072, 6144,
 // a pair of 9216; weights from memory): rounds of workgroups x (fixed + per k tile of 64) + what a k tile costs more with the
-// chip full, and for a split the second launch plus its bytes.  What it picks is 1 % slower than the best measured choice,
-// over all of those shapes.
+// chip full, and for a split the second launch plus its bytes.  Over 158 shapes (M = 20 .. 8188 of those layers and of K = 768 .. 6144,
+// N = 512 .. 14432) what it picks is 3.0 % slower than the best measured choice in the mean (4.8 % without the 128 x 192 tiles).
 struct TileCost { int bm, bn, slots; double fixed, per_kt, full_kt, split, split_mb; };
 static const TileCost kTileCost[kTiles] = {
-    {256, 256, 256, 5.45, 1.237, 0.379, 2.8, 0.30}, {256, 192, 256, 1.16, 1.206, 0.122, 4.7, 0.35}, {128, 256, 256, 6.87, 0.661, 0.171, 3.1, 0.26},
+    {256, 256, 256, 5.45, 1.237, 0.379, 2.8, 0.30}, {256, 192, 256, 1.16, 1.206, 0.122, 4.7, 0.35}, {128, 256, 256, 6.87, 0.661, 0.171, 3.1, 0.26}, {128, 192, 256, 7.9, 0.48, 0.266, 5.1, 0.10},
     {128, 128, 256, 4.48, 0.425, 0.055, 3.9, 0.31}, {64, 256, 256, 4.59, 0.572, 0.0, 5.4, 0.13}, {64, 128, 512, 2.58, 0.361, 0.143, 5.0, 0.34},
 };
 static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
@@ -935,7 +1008,7 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t roo
     double least = 1e300;
     for (int t = 0; t < kTiles; ++t) {
         const TileCost& c = kTileCost[t];
-        if (dual && c.bn == 192) continue;   // a pair's tile holds whole 64-column loads of either matrix
+        if (dual && t == kT256x192) continue;   // a wave's three fragments do not divide between the matrices
         const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
         for (int sp : {1, 2, 3, 4, 6, 8}) {
             if (sp > 1 && (!splits_allowed() || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
@@ -954,6 +1027,7 @@ static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p)
         case kT256x256: return launch_tile<T, 4, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits);
         case kT256x192: if constexpr (!DUAL) return launch_tile<T, 8, 2, 4, 2, 2, 3, false>(s, a, p.splits); else return;
         case kT128x256: return launch_tile<T, 8, 3, 2, 4, 2, 2, DUAL>(s, a, p.splits);
+        case kT128x192: return launch_tile<T, 8, 3, 2, 2, 2, 3, DUAL, 0, 2>(s, a, p.splits);
         case kT128x128:
             if constexpr (DUAL) return launch_tile<T, 8, 4, 4, 2, 1, 2, true>(s, a, p.splits);
             else return launch_tile<T, 8, 4, 2, 4, 2, 1, false>(s, a, p.splits);

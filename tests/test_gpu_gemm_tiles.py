@@ -23,7 +23,9 @@ def program(specs, body):
 # one row over and under the tiles' 64, 128 and 256 rows; columns that end inside a fragment, a tile and a group of 8; one
 # k tile, fewer k tiles than the ring holds, k that does not divide among the splits; the layer sizes on each tile and split
 @pytest.mark.parametrize("m,k,n", [(17, 64, 8), (33, 128, 41), (64, 192, 130), (65, 3072, 1000), (127, 4096, 3072), (129, 1088, 3075), (200, 9216, 1536),
-                                   (255, 3072, 6144), (257, 320, 520), (333, 3072, 6176), (513, 2048, 4100), (1000, 9216, 768), (1025, 448, 9216), (2049, 256, 3008)])
+                                   (255, 3072, 6144), (257, 320, 520), (333, 3072, 6176), (513, 2048, 4100), (1000, 9216, 768), (1025, 448, 9216), (2049, 256, 3008),
+                                   # 128 x 192 tiles, whole and in 2, 4 and 8 splits, then for the pair whole and in 2, 3 and 4: ragged rows and columns
+                                   (1227, 1536, 3985), (913, 9216, 2673), (230, 9216, 5883), (2025, 9216, 368), (687, 3072, 3335), (615, 9216, 1602)])
 def test_tiles_and_splits(hip, m, k, n):
     rng = np.random.default_rng(m * 7 + k + n)
     x = bf16(rng.standard_normal((m, k), dtype=np.float32))
