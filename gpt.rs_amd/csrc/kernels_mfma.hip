@@ -1058,7 +1058,9 @@ static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
 // 23 (int4) vector instructions for 8 codes, so the tiles give a wave as many rows per column as fit: one wave row (128 x 256 in 8
 // waves of 128 x 32, 128 x 128 and 64 x 128 in 4) has no column converted twice; a pair, whose waves hold both matrices, has two
 // wave rows and runs 256 x 256 where it is large.  Measured with int8 at M = 40 .. 4000 of the 3072-wide layers, fitted as above
-// (7 % rms, the pick 1.5 % slower than the best measured); int4 is 0-15 % slower and takes the same plan.  Against the
+// (7 % rms).  Int4 takes the same plan, so that a layer's sums do not depend on its codes: 7 % slower than int8 in the median (-6 .. 16 %), and
+// over 60 of those shapes the pick is 2.1 % slower than the best measured choice for int4, 2.8 % for int8; worst for int4 at M = 3000, K =
+// 9216 (288 us against 229: a long K's scales leave a CU two workgroups of 64 x 128; counting them so would cost int8 229 -> 255).  Against the
 // register-staged tiles that ran here before (64 x 64 below half a chip of 128 x 128), M = 200, int8, us: out and down 65 (mean)
 // -> 21 and 29, qkv 35 -> 24, pair 58 -> 58.
 enum QuantTileId { kQ256x256, kQ128x256, kQ128x128, kQ64x128, kQTiles };
