@@ -881,6 +881,21 @@ struct Fuser {
         }
     }
 
+    // does value `v` come out of instruction `from`, directly or through others
+    bool depends_on(int v, int from) const {
+        std::vector<int> todo{v};
+        std::vector<bool> seen(fn.body.size(), false);
+        while (!todo.empty()) {
+            const int i = todo.back() < 0 ? -1 : def[todo.back()];
+            todo.pop_back();
+            if (i < 0 || seen[i]) continue;
+            if (i == from) return true;
+            seen[i] = true;
+            for (const Operand& o : fn.body[i].operands) todo.push_back(o.value);
+        }
+        return false;
+    }
+
     // A prompt's attention with everything between the projection and the caches: [the rotation of its packed rows,] the attention
     // and the updates of the two caches with its K and V rows, for every sequence of a batch of stacked rows, become one
     // instruction (ops/functional/attention.rs:443-522, model/gpt.rs:712-730).
@@ -972,6 +987,8 @@ struct Fuser {
             if (ok && parts[0].rot) {   // tables of the rows' type, one row per position
                 const Spec *cs = spec_of(parts[0].cos), *ss = spec_of(parts[0].sin);
                 ok = cs && ss && *cs == *ss && cs->dims == std::vector<int64_t>{T, parts[0].rot} && cs->dtype == a0.out_specs[0].dtype;
+                for (const Part& p : parts)                // nor made of the values that the instruction is to store
+                    ok = ok && !depends_on(p.cos, p.du[1]) && !depends_on(p.sin, p.du[1]);
             }
             if (!ok) continue;
             Instr ni = make(OpKind::FAttnPrefill, "fused.attention_prefill_caches", {src, parts[0].starts}, root.out_ids[0], root.out_specs[0]);

@@ -64,6 +64,40 @@ def test_a_cache_that_the_program_computes_stays_apart():
     assert fusion_report(Program(fb)).count("DynamicUpdateSlice") == 2
 
 
+def tables_of_values(B):
+    """The rotation's tables are read back from the values that one of the updates has stored."""
+    T, hd, cap = 8, 32, 16
+    fb = FunctionBuilder("main", "F32")
+    cfg = F.AttentionConfig(hd, 1, 1, hd)
+    qkv, starts, sin = fb.param("F32", [B * T, 3 * hd]), fb.param("Si32", [3]), fb.param("F32", [T, hd // 2])
+    caches = [fb.param("F32", [1, cap, hd]) for _ in range(2 * B)]
+    parts = [qkv if B == 1 else qkv.slice([b * T, 0], [T, 3 * hd]) for b in range(B)]
+    new_v = [F.dynamic_update_slice_into(caches[2 * b + 1], parts[b].slice([0, 2 * hd], [T, hd]).reshape([T, 1, hd]).transpose([1, 0, 2]), starts) for b in range(B)]
+    cos = new_v[-1].reshape([cap, hd]).slice([0, 0], [T, hd // 2])
+    ctxs, outs = [], []
+    for b in range(B):
+        ctx, k, _ = F.attention(cfg, F.apply_rope_qkv_packed(cfg, parts[b], cos, sin), None)
+        ctxs.append(ctx)
+        outs += [F.dynamic_update_slice_into(caches[2 * b], k, starts), new_v[b]]
+    fb.set_results([ctxs[0] if B == 1 else Tensor.concat(0, ctxs)] + outs)
+    return Program(fb)
+
+
+@pytest.mark.parametrize("B", [1, 2])
+def test_tables_made_of_stored_values_stay_apart(B):
+    """The tables depend on the update of the values: taking both up in one instruction would make a cycle."""
+    assert sum("DynamicUpdateSlice" in line for line in fusion_report(tables_of_values(B))) >= 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [1, 2])
+def test_tables_made_of_stored_values(hip, B):
+    rng = np.random.default_rng(8)
+    args = [rng.standard_normal((8 * B, 96), dtype=np.float32), np.array([0, 3, 0], np.int32), rng.standard_normal((8, 16), dtype=np.float32)]
+    args += [rng.standard_normal((1, 16, 32), dtype=np.float32) for _ in range(2 * B)]
+    check_program(hip, tables_of_values(B), args, what=f"{B} sequences")
+
+
 # tensors that hold more than the keys (or values) of one layer: more heads, wider rows, both; where the update goes
 BASES = [((1, 8, 4, 2, 32, False), [6, 16, 32], (4, 3, 0)), ((1, 33, 2, 2, 32, True), [2, 64, 64], (0, 5, 32)), ((2, 9, 4, 2, 64, True), [4, 12, 72], (1, 2, 8)),
          ((3, 5, 2, 1, 32, False), [2, 5, 33], (7, -1, 1)), ((1, 17, 4, 4, 64, False), [5, 17, 64], (1, 0, 0))]
