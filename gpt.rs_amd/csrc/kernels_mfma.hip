@@ -508,8 +508,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
 // 256: a k tile moves 1 / (2 BM) + 1 / (2 BN) bytes per flop from the L2s into LDS and as many fragments from LDS into
 // registers, 5/6 of what 128 x 192 needs twice over; 8 waves of 128 x 64 read 6 fragments for 8 MFMAs (64 x 96: 5 for 6,
 // each k-group its own).  Against the 128 x 192 tiles (two k-groups of 2 x 2 waves) that ran here before, us in a traced
-// 26-layer prompt: M = 8188 qkv 340 -> 263, gate/up pair 1010 -> 771, out and down 337 (mean) -> 215 and 413; M = 333 (few tiles,
-// weights from memory) qkv 32 -> 28, out and down 51 (mean) -> 29 with the launch that adds the splits, pair 81 -> 49.  k tiles of 32 in a ring of four beat k tiles of 64 in
+// 26-layer prompt: M = 8188 qkv 340 -> 263, gate/up pair 1010 -> 798, out and down 337 (mean) -> 208 and 414; M = 333 (few tiles,
+// weights from memory) qkv 32 -> 28, out and down 51 (mean) -> 29 with the launch that adds the splits, pair 81 -> 51.  k tiles of 32 in a ring of four beat k tiles of 64 in
 // a ring of two there (1035 -> 1239 TFLOP/s: loads have three k tiles of time, not one); 4 waves of 128 x 128 lose (1090).
 // Smaller tiles are for launches whose 256 x 256 tiles would leave CUs without work; they stage 64 k, the memory's lines.
 // 128 x 192 in two k-groups of 2 x 2 waves: 8 waves that still read 5 fragments for 6 MFMAs (8 waves of 32 x 96 read 4 for 3, more than LDS
@@ -1038,9 +1038,11 @@ static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p)
 
 // f32: one tile, 64 x 64 outputs in 4 waves of 32 x 32 (a pair: 64 x 64 of each matrix), three workgroups to a CU.  The f32
 // products are paced by the matrix pipes alone, 0.43 us for a k tile of 32 on a CU, one wave per SIMD is enough to keep them
-// busy, and the small tile divides best among the CUs: M = 8192, K = 768, N = 3072 297 us = 130 TFLOP/s (64 x 128 304, 128 x 128
-// 316, 256 x 256 396), K = 3072, N = 768 273 = 141 (274, 354, 350); the register-staged 128 x 128 tiles took 366 and 354.
-// M = 400 (K = 768, N = 2304): 18 us (64 x 128 26).  Splits over k: rounds of 256 workgroups, a launch more and its bytes.
+// busy, and the small tile divides best among the CUs: in a lab program 64 x 128 takes 0-2 % longer at M = 8192 (K = 768, N = 3072 and K =
+// 3072, N = 768), 128 x 128 6 and 30 %, 256 x 256 33 and 28 %, and 64 x 128 44 % at M = 400.  As a program of one layer, M = 8192, against the
+// register-staged 128 x 128 tiles: K = 768, N = 3072 361 -> 344 us = 112 TFLOP/s, with bias and GELU (an erff and two divisions per output)
+// 389 -> 380; N = 2304 298 -> 254; N = 768 99 -> 87; K = 3072, N = 768 346 -> 321 .. 366 (medians of nine; clocks move it by that).  The same
+// layers inside 16 prompts of 512 take 354 (with GELU) and 253.  The two chains of sums cost nothing there: 338, 378, 249 and 86 with one.  Splits over k: rounds of 256 workgroups, a launch more and its bytes.
 static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
     const int64_t tiles = cdiv(m, 64) * cdiv(n, 64);
     int best = 1;

@@ -406,7 +406,10 @@ void skinny_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int
 // N = 6144 11.8 -> 8.2, int4 N = 32768 29.4 -> 20.5); plain layers with more tiles 4 waves with four steps in flight (N = 14432 18.7;
 // 8 waves 19.8, 16 waves 21.1).  Two requests at a time, not four, where 8 or 16 waves share the CU's memory pipeline (pair 20.3
 // against 23.2; at 16 rows K = 9216 16.2 against 19.6).  Only layers of a few tiles still split (f32 K = 3072, N = 768: 10.6 -> 9.1).
-// Weights are read past the caches (nontemporal): 4-5 % on every shape.
+// Weights are read past the caches (nontemporal): 4-5 % of a layer whose weights come from memory.  Models that the 256 MB last-level cache
+// holds gain or lose: whole f32 decode steps of 2 to 16 rows, against plain loads, take 0-15 % less with 16 MB of weights (5 % more at 2
+// rows), 2-9 % more with 100 to 180 MB (13 % at 16 rows of three layers of 1024), the same with 210, up to 5 % less with 240 to 270 and 1-7 %
+// less from 300 MB on.  None takes longer than with the four waves and the splits that ran here before; one rule for all.
 struct SkinnyPlan { int nw, ks; };
 static SkinnyPlan skinny_plan(int64_t steps, int64_t n, bool dual, bool codes) {
     const int64_t tiles = cdiv_s(n, 16);
