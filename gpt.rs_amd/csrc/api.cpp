@@ -206,6 +206,9 @@ BufferP Backend::derived_weights(const BufferP& src, int kind, DType dtype, int6
     } else if (kind == 9 || kind == 10) {               // batched decode: int8 / int4 codes in the 16-column tiled word order
         t = new_buffer(k::skinny_codes_bytes(k, n, kind - 8));
         k::skinny_pack_codes(stream, src->ptr, t->ptr, k, n, kind - 8);
+    } else if (kind == 12) {                            // prefill GEMM: f32 as three bf16 planes, k-grouped (kernels_mfma.hip)
+        t = new_buffer(k::mfma_split_bytes(k, n));
+        k::mfma_split_weights(stream, src->ptr, t->ptr, k, n);
     } else {                                            // 6 / 7: prefill GEMM: int8 / int4 codes, k-grouped (kernels_mfma.hip)
         t = new_buffer(k::mfma_codes_bytes(k, n, kind - 5));
         k::mfma_pack_codes(stream, src->ptr, t->ptr, k, n, kind - 5);

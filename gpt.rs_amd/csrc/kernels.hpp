@@ -295,6 +295,10 @@ struct MfmaLinearArgs {
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant);
 size_t mfma_weight_bytes(int dtype, int64_t k, int64_t n);
 void mfma_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int64_t k, int64_t n);
+// f32 weights as three bf16 planes, Ws[K/8][3][Npad][8]: what `wk` / `wk2` hold where mfma_takes_split_weights() says so
+size_t mfma_split_bytes(int64_t k, int64_t n);
+void mfma_split_weights(hipStream_t s, const void* w, void* out, int64_t k, int64_t n);
+bool mfma_takes_split_weights(int dtype, int64_t m, int64_t k, int64_t n, int lds_direct);
 size_t mfma_codes_bytes(int64_t k, int64_t n, int quant);
 void mfma_pack_codes(hipStream_t s, const void* q, void* out, int64_t k, int64_t n, int quant);
 bool mfma_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n, int quant = 0);

@@ -1,5 +1,5 @@
 // MFMA tile GEMM for prefill-sized linear layers (M > 16): bf16 in / f32 accumulate / bf16 out on
-// v_mfma_f32_32x32x16_bf16, and f32 throughout on v_mfma_f32_32x32x2_f32.
+// v_mfma_f32_32x32x16_bf16; f32 throughout on v_mfma_f32_32x32x2_f32, and from 129 rows on as six bf16 products (gemm_split_kernel).
 //
 // Per lane the matrix cores want consecutive k of ONE row (A) or ONE column (B).  Activations x[M,K] are row-major,
 // so A fragments are plain 16-byte loads.  Weights are stored [in,out] row-major (nn/layers/linear.rs:50-71), the
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* _
 #pragma unroll
         for (int j = 0; j < LB; ++j) gemm_lds_load16(b_off[j], gemm_uniform64(b_base[j] + bt), (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + A_BYTES + (wave * LB + j) % LBI * 1024)));
     };
-    // f32 adds the two halves of every k tile apart: half as many roundings in a row, and the registers are there (M = 8192, K = 3072, N = 768:
+    // f32 adds the two halves of every k tile apart: half as many roundings in a row, and the registers are there (K = 3072:
     // 7.0e-7 of the result's norm away from 64 bits, in one chain 9.9e-7; K = 768 3.5e-7 and 5.0e-7)
     constexpr int CHAINS = std::is_same<T, float>::value ? 2 : 1;
     f32x16_t sums[CHAINS][TM][TN];
@@ -923,11 +923,302 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* _
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// f32 layers of more than 128 rows, on the bf16 matrix cores.  An f32 value is the sum of three bf16 values, a = a1 + a2 + a3 exactly (8 bits of
+// its 24 each, rounded to nearest, so |a2| <= 2^-8 |a| and |a3| <= 2^-17 |a|; the last bits of values under 2^-109 are lost), and a product is
+//   a b = a1 b1 + (a1 b2 + a2 b1) + (a2 b2 + a1 b3 + a3 b1) + what is left out: a2 b3 + a3 b2 + a3 b3 < 2^-23.9 |a b|,
+// six bf16 products, each exact in f32.  The bf16 cores are 16 times as fast as the f32 cores, so six cost 0.375 of one f32 product.
+//
+// Precision.  What is left out is 2^-27 of a product in the mean square, far below the roundings of the sum.  a1 b1 and the five small products are
+// summed apart (the small sum's roundings are 2^-8 of the large one's), and a sum of K terms is rounded about K / 8 times, where the f32
+// cores round it K / 2 times.  Distance from 64 bits over the result's norm, normal operands: K = 768 1.6e-7 (f32 cores, two chains of sums: 3.5e-7; all
+// six products in one chain: 4.2e-7), K = 3072 3.4e-7 (7.0e-7; 9.0e-7).  Infinities and NaN, and operands that round to infinity in bf16, leave a
+// sum that is not finite (a2 of an infinity is a NaN); such a sum is formed again, with one f32 product per term, before anything is made of it.
+//
+// The weights are split once, into Ws[K/8][plane][Npad][8] (6 bytes a weight); the rows are staged in f32 and every wave splits the fragments it
+// multiplies, 44 vector instructions for 8 values, so a wave takes one row of fragments and all of a large tile's columns: 256 x 96 in 8 waves of 32 x 96
+// (18 MFMAs per 44), two k-steps of 16 to a staged tile; 128 x 96 in 4, one k-step, two workgroups to a CU; and 64 x 64 in 4 waves of 32 x 32 for
+// launches of few rows (two k-steps: one barrier for 12 MFMAs, not 6; K = 768 in one round 19 -> 14.5 us).
+// What bounds it: with the chip full, the matrix pipes at the clock that random operands allow (256 x 96 at M = 8192, K = 3072, N = 768: 218
+// TFLOP/s = 1310 of bf16, the rate of the bf16 tiles); with K = 768 the tile's first loads and its epilogue.  us, M = 8192, weights from memory, f32 cores
+// and this: K = 768, N = 3072 288 -> 199, N = 2304 218 -> 151, N = 768 83 -> 51; K = 3072, N = 768 301 -> 177; M = 1000, K = 768, N = 3072 44 -> 35;
+// M = 512, N = 2304 27 -> 21; 16 prompts of 512 through GPT-2 small 13.9 -> 10.7 ms.  Dropped: 64 x 64 per wave (88 vector
+// instructions per 24 MFMAs: 177 TFLOP/s against 193), 32 x 128 (the small products' own sums no longer fit the registers), fragments split a k tile
+// ahead of their use, a ring of six (no change).
+__global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ w, bf16_t* __restrict__ out, int64_t K, int64_t N, int64_t Npad) {
+    const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t kb = blockIdx.y;
+    if (n >= Npad) return;
+    alignas(16) bf16_t r[3][8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int64_t kx = kb * 8 + i;
+        const float v = n < N && kx < K ? w[kx * N + n] : 0.f;
+        bf16_t p[3] = {f32_to_bf16(v), 0, 0};
+        if (__builtin_isfinite(v)) {
+            if (!__builtin_isfinite(bf16_to_f32(p[0]))) p[0] = (bf16_t)(__float_as_uint(v) >> 16);   // next to the largest f32: cut off instead
+            const float rest = v - bf16_to_f32(p[0]);
+            p[1] = f32_to_bf16(rest);
+            p[2] = f32_to_bf16(rest - bf16_to_f32(p[1]));
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) r[q][i] = p[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4*>(out + ((kb * 3 + q) * Npad + n) * 8) = *reinterpret_cast<const uint4*>(r[q]);
+}
+size_t mfma_split_bytes(int64_t k, int64_t n) { return (size_t)cdiv(k, 8) * 3 * (size_t)mfma_padded_n(n) * 16; }
+void mfma_split_weights(hipStream_t s, const void* w, void* out, int64_t k, int64_t n) {
+    const int64_t npad = mfma_padded_n(n);
+    split_weights_kernel<<<dim3((unsigned)cdiv(npad, 256), (unsigned)cdiv(k, 8)), 256, 0, s>>>((const float*)w, (bf16_t*)out, k, n, npad);
+}
+// What a sum that is not finite is formed from again: x[M, K] and the split weights.
+struct SplitOperands {
+    const float* x; const bf16_t* wp; const bf16_t* wp2;
+    int K, Npad;
+};
+__device__ __forceinline__ float split_dot(const float* row, const bf16_t* w, int K, int Npad, int64_t col) {
+    float s = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < K; ++k) {
+        const bf16_t* p = w + ((int64_t)(k >> 3) * 3 * Npad + col) * 8 + (k & 7);
+        s += row[k] * ((bf16_to_f32(p[0]) + bf16_to_f32(p[(int64_t)Npad * 8])) + bf16_to_f32(p[(int64_t)Npad * 16]));   // w again, exactly
+    }
+    return s;
+}
+__device__ __forceinline__ void split_rows8(const f32x4_t& r0, const f32x4_t& r1, bf16x8_t* out) {
+    u32x4_t p[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float lo = e < 2 ? r0[2 * e] : r1[2 * e - 4], hi = e < 2 ? r0[2 * e + 1] : r1[2 * e - 3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            p[q][e] = mfma_pack_bf16(lo, hi);
+            if (q < 2) {
+                lo -= __uint_as_float(p[q][e] << 16);
+                hi -= __uint_as_float(p[q][e] & 0xFFFF0000u);
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) out[q] = __builtin_bit_cast(bf16x8_t, p[q]);
+}
+
+// WM x WN waves of 32 x (32 TN) outputs; order of issue, tile order, partial sums and epilogue as in gemm_tile_kernel.  DUAL: half of a wave's
+// fragments are columns of W, the others the same columns of W2.
+template <int WM, int WN, int TN, int KS, int NST, bool DUAL>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(int M, int NT, int MT, int splits, float* __restrict__ part, SplitOperands of, TileEpilogue<float> epi) {
+    constexpr int BK = 16 * KS, ROWB = BK * 4;
+    constexpr int BM = 32 * WM, BN = 32 * TN * WN, NW = WM * WN;
+    constexpr int NREAL = DUAL ? BN / 2 : BN, TNO = DUAL ? TN / 2 : TN;
+    constexpr int PLANE = NREAL * 16, MAT = 6 * KS * PLANE;            // bytes of a plane's k-group of 8 in LDS; of a matrix, [k-group][plane][column]
+    constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * 96 * KS, STAGE = A_BYTES + B_BYTES;
+    constexpr int LAI = A_BYTES / 1024, LBI = B_BYTES / 1024, LA = LAI / NW, LB = (LBI + NW - 1) / NW, LPT = LA + LB;   // load instructions of a tile; of a wave
+    constexpr bool EVEN = LBI % NW == 0;                               // otherwise the first LBI % NW waves bring one more than the others
+    static_assert(LA * NW == LAI && LBI * 1024 == B_BYTES, "whole load instructions");
+    static_assert(!DUAL || (TN % 2 == 0 && MAT % 1024 == 0), "a load instruction belongs to one matrix of the pair");
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN, K = of.K, Npad = of.Npad;
+    int bx, by, sidx;
+    {
+        const int total = NT * MT * splits, per = (total + 7) / 8;
+        const int u = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+        if (u >= total) return;
+        const int v = u / splits;
+        sidx = u % splits;
+        const int gsz = 8 * NT, g = v / gsz, first = g * 8;
+        const int gm = MT - first < 8 ? MT - first : 8;
+        by = first + (v % gsz) % gm;
+        bx = (v % gsz) / gm;
+    }
+    const int m0 = by * BM, n0 = bx * NREAL;
+    auto swz = [](int row) { return KS == 2 ? (row >> 1) & 7 : (row >> 2) & 3; };   // position p of a row holds its 4 k of chunk p ^ swz(row)
+    unsigned a_off[LA], b_off[LB];
+    unsigned long long b_base[LB];
+#pragma unroll
+    for (int j = 0; j < LA; ++j) {
+        const int sl = (wave * LA + j) * 64 + lane, row = sl / (4 * KS), pos = sl % (4 * KS);
+        int m = m0 + row;
+        if (m > M - 1) m = M - 1;
+        a_off[j] = (unsigned)(m - m0) * (unsigned)(K * 4) + (unsigned)((pos ^ swz(row)) * 16);   // under 256 rows: fits 32 bits (K <= 2^21)
+    }
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+        const int q = wave + j * NW < LBI ? wave + j * NW : wave, half = q * 1024 / MAT, at = q * 1024 + lane * 16 - half * MAT;
+        int col = n0 + at % PLANE / 16;
+        if (col > Npad - 1) col = Npad - 1;
+        b_base[j] = (unsigned long long)(DUAL && half ? of.wp2 : of.wp);
+        b_off[j] = (unsigned)(((unsigned long long)(at / PLANE) * Npad + col) * 16);
+    }
+    const unsigned long long a_base = (unsigned long long)(of.x + (int64_t)m0 * K);
+    const int64_t b_tile_step = (int64_t)6 * KS * Npad * 16;
+    const unsigned lds0 = (unsigned)(uintptr_t)lds;
+    const int kt_all = K / BK, kt0 = (int)((int64_t)sidx * kt_all / splits);
+    const int nt = (int)((int64_t)(sidx + 1) * kt_all / splits) - kt0;   // this workgroup's k tiles: [kt0, kt0 + nt)
+    const bool all_loads = EVEN || wave < LBI % NW;
+    auto issue = [&](int t, int st) {
+        if (t >= nt) return;
+        const unsigned long long ab = gemm_uniform64(a_base + (unsigned long long)(t + kt0) * ROWB);
+        const unsigned long long bt = (unsigned long long)((t + kt0) * b_tile_step);
+        const unsigned sbase = lds0 + st * STAGE;
+#pragma unroll
+        for (int j = 0; j < LA; ++j) gemm_lds_load16(a_off[j], ab, (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + (wave * LA + j) * 1024)));
+#pragma unroll
+        for (int j = 0; j < LB; ++j)
+            if (j + 1 < LB || all_loads) gemm_lds_load16(b_off[j], gemm_uniform64(b_base[j] + bt), (unsigned)__builtin_amdgcn_readfirstlane((int)(sbase + A_BYTES + (wave + j * NW) * 1024)));
+    };
+    f32x16_t acc[TN], small[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[j][v] = small[j][v] = 0.f;
+    const int fsel = lane >> 5, r32 = lane & 31;
+    int a_rd[KS][2];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) a_rd[kk][c] = (wm * 32 + r32) * ROWB + (((4 * kk + 2 * fsel + c) ^ swz(r32)) * 16);
+    const int b_rd = A_BYTES + fsel * 3 * PLANE + (wn * 32 * TNO + r32) * 16;
+    f32x4_t ar[2];
+    bf16x8_t as[2][3], bs[2][TN][3];
+    auto fread = [&](int st, int kk, int slot) {
+        const unsigned char* base = lds + st * STAGE;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) ar[c] = *reinterpret_cast<const f32x4_t*>(base + a_rd[kk][c]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) bs[slot][j][p] = *reinterpret_cast<const bf16x8_t*>(base + b_rd + (6 * kk + p) * PLANE + (j / TNO) * MAT + (j % TNO) * 32 * 16);
+    };
+    auto wait_for = [&](int t) {   // tile t has landed; those up to t + NST - 2 may be on their way
+        if (t + NST - 2 < nt) {
+            if (all_loads) gemm_wait_loads<(NST - 2) * LPT>();
+            else gemm_wait_loads<(NST - 2) * (LPT - 1)>();
+        } else {
+            gemm_wait_loads<0>();
+        }
+    };
+    for (int st = 0; st < NST - 1; ++st) issue(st, st);
+    wait_for(0);
+    __syncthreads();
+    issue(NST - 1, NST - 1);
+    fread(0, 0, 0);
+    split_rows8(ar[0], ar[1], as[0]);
+    auto tile_step = [&](auto ring_pos, int t) {
+        constexpr int ST = decltype(ring_pos)::value, ST1 = (ST + 1) % NST;
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+            const int slot = KS == 2 ? kk : ST & 1;
+            auto mul = [&](int pa, int pb, f32x16_t* to) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j) to[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as[slot][pa], bs[slot][j][pb], to[j], 0, 0, 0);
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            if (kk + 1 < KS) fread(ST, kk + 1, slot ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+            mul(2, 0, small);
+            mul(1, 1, small);
+            mul(0, 2, small);
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (kk + 1 == KS) {
+                wait_for(t + 1);
+                __syncthreads();
+                fread(ST1, 0, slot ^ 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+            mul(1, 0, small);
+            mul(0, 1, small);
+            mul(0, 0, acc);
+            split_rows8(ar[0], ar[1], as[slot ^ 1]);
+            if (kk + 1 == KS) issue(t + NST, ST);
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    static_assert(KS == 1 || KS == 2, "");
+    static_assert((KS == 2 && NST == 3) || NST == 4, "a k-step's fragments alternate between two slots; the tile loop is unrolled over the ring");
+    {
+        constexpr std::integral_constant<int, 0> R0{};
+        constexpr std::integral_constant<int, 1> R1{};
+        constexpr std::integral_constant<int, 2> R2{};
+        constexpr std::integral_constant<int, NST - 1> R3{};
+        int t = 0;
+        for (; t + NST <= nt; t += NST) {
+            tile_step(R0, t);
+            tile_step(R1, t + 1);
+            tile_step(R2, t + 2);
+            if constexpr (NST > 3) tile_step(R3, t + 3);
+        }
+        if (t < nt) tile_step(R0, t);
+        if (t + 1 < nt) tile_step(R1, t + 1);
+        if constexpr (NST > 3)
+            if (t + 2 < nt) tile_step(R2, t + 2);
+    }
+    float odd = 0.f;                                                   // a NaN once any sum is not finite
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        acc[j] += small[j];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) odd += acc[j][v] * 0.f;
+    }
+    const int mw = m0 + wm * 32, nw = n0 + wn * 32 * TNO;              // the wave's first output
+    const int r0 = 4 * fsel;                                           // value v of a lane: row 8 (v / 4) + r0 + v % 4, column r32
+    if (splits > 1) {
+        const int np = ((int)epi.N + 7) & ~7, width = DUAL ? 2 * np : np;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = nw + (j % TNO) * 32 + r32;
+            if (n >= np) continue;
+            float* to = part + (int64_t)sidx * M * width + (j / TNO) * np + n;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int m = mw + 8 * (v >> 2) + r0 + (v & 3);
+                if (m < M) to[(int64_t)m * width] = acc[j][v];
+            }
+        }
+        return;
+    }
+    constexpr int RSF = 32 * TNO + 4, CH = 4 * TNO, PASSES = CH / 2;   // as in gemm_tile_kernel
+    float* area = reinterpret_cast<float*>(lds) + wave * (32 * RSF);
+    if (__any(!(odd == 0.f))) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            float* mine = area + lane;                                 // 16 x 64 floats, a fragment at a time; each lane its own column of it
+#pragma unroll
+            for (int v = 0; v < 16; ++v) mine[v * 64] = acc[j][v];
+            const int n = nw + (j % TNO) * 32 + r32;
+#pragma unroll 1
+            for (int v = 0; v < 16; ++v) {
+                const int m = mw + 8 * (v >> 2) + r0 + (v & 3);
+                if (m < M && n < (int)epi.N && !__builtin_isfinite(mine[v * 64])) mine[v * 64] = split_dot(of.x + (int64_t)m * K, j >= TNO ? of.wp2 : of.wp, K, Npad, n);
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[j][v] = mine[v * 64];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < TNO; ++j) {
+        if constexpr (DUAL) gemm_glu<16>(acc[j], acc[j + TNO], epi.extra.glu);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) area[(8 * (v >> 2) + r0 + (v & 3)) * RSF + j * 32 + r32] = acc[j][v];
+    }
+#pragma unroll 1
+    for (int it = 0; it < PASSES; ++it) {
+        const int c = it * 64 + lane, r = c / CH, cc = c % CH;
+        const int m = mw + r, n = nw + cc * 8;
+        if (m < M && n < epi.N) gemm_finish8<float, false>(epi, m, n, area + r * RSF + cc * 8, nullptr);
+    }
+}
+
 // Adds the partial sums of a launch whose tiles were split over k, in split order (the result does not depend on which
 // workgroup ended first), and finishes the outputs.  One thread per 8 outputs.  A launch of its own over the whole chip:
 // with the last workgroup of a tile adding them, 48 tiles of M = 333 kept 48 CUs busy reading while 208 waited.
-template <typename T, bool DUAL>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int M, int splits, TileEpilogue<T> epi) {
+template <typename T, bool DUAL, bool SPLIT = false>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int M, int splits, TileEpilogue<T> epi, SplitOperands of) {
     const int np = ((int)epi.N + 7) & ~7, chunks = np / 8, width = DUAL ? 2 * np : np;
     const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (id >= (int64_t)M * chunks) return;
@@ -942,12 +1233,23 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
         *reinterpret_cast<f32x4_t*>(o) = a;
         *reinterpret_cast<f32x4_t*>(o + 4) = b;
     };
-    __shared__ __attribute__((aligned(16))) float rows[256][12];   // finish8 reads its eight from LDS; each thread its own
-    float* o = rows[threadIdx.x];
+    auto again = [&](float* p, const bf16_t* w) {   // SPLIT: gemm_split_kernel's sums
+        float odd = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) odd += p[e] * 0.f;
+        if (odd == 0.f) return;
+#pragma unroll 1
+        for (int e = 0; e < 8 && n + e < (int)epi.N; ++e)
+            if (!__builtin_isfinite(p[e])) p[e] = split_dot(of.x + m * of.K, w, of.K, of.Npad, n + e);
+    };
+    __shared__ __attribute__((aligned(16))) float rows[DUAL ? 2 : 1][256][12];   // finish8 reads its eight from LDS; each thread its own
+    float* o = rows[0][threadIdx.x];
     sum8(part + m * width + n, o);
-    if (DUAL) {
-        float u[8];
+    if constexpr (SPLIT) again(o, of.wp);
+    if constexpr (DUAL) {
+        float* u = rows[1][threadIdx.x];
         sum8(part + m * width + np + n, u);
+        if constexpr (SPLIT) again(u, of.wp2);
         gemm_glu<8>(o, u, epi.extra.glu);
     }
     gemm_finish8<T, false>(epi, m, n, o, nullptr);
@@ -981,7 +1283,7 @@ static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
     kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN * KW, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (int)a.m, (int)a.k,
                                                                                    (int)mfma_padded_n(a.n), (int)nt, (int)mt, splits, (float*)a.part,
                                                                                    (const T*)a.scale, (const T*)a.scale2, epi);
-    if (splits > 1) gemm_reduce_kernel<T, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
+    if (splits > 1) gemm_reduce_kernel<T, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi, SplitOperands{});
 }
 static size_t tile_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
     return splits > 1 ? (size_t)splits * m * cdiv(n, 8) * 8 * (dual ? 2 : 1) * sizeof(float) : 0;
@@ -1036,13 +1338,9 @@ static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p)
     }
 }
 
-// f32: one tile, 64 x 64 outputs in 4 waves of 32 x 32 (a pair: 64 x 64 of each matrix), three workgroups to a CU.  The f32
-// products are paced by the matrix pipes alone, 0.43 us for a k tile of 32 on a CU, one wave per SIMD is enough to keep them
-// busy, and the small tile divides best among the CUs: in a lab program 64 x 128 takes 0-2 % longer at M = 8192 (K = 768, N = 3072 and K =
-// 3072, N = 768), 128 x 128 6 and 30 %, 256 x 256 33 and 28 %, and 64 x 128 44 % at M = 400.  As a program of one layer, M = 8192, against the
-// register-staged 128 x 128 tiles: K = 768, N = 3072 361 -> 344 us = 112 TFLOP/s, with bias and GELU (an erff and two divisions per output)
-// 389 -> 380; N = 2304 298 -> 254; N = 768 99 -> 87; K = 3072, N = 768 346 -> 321 .. 366 (medians of nine; clocks move it by that).  The same
-// layers inside 16 prompts of 512 take 354 (with GELU) and 253.  The two chains of sums cost nothing there: 338, 378, 249 and 86 with one.  Splits over k: rounds of 256 workgroups, a launch more and its bytes.
+// f32 of up to 128 rows (more: split_plan()): one tile, 64 x 64 outputs in 4 waves of 32 x 32 (a pair: 64 x 64 of each matrix), three workgroups to a CU.  The f32
+// products are paced by the matrix pipes alone, 0.43 us for a k tile of 32 on a CU, one wave per SIMD is enough to keep them busy, and the small
+// tile divides best among the CUs (64 x 128 takes 44 % longer at M = 400).  Splits over k: rounds of 256 workgroups, a launch more and its bytes.
 static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
     const int64_t tiles = cdiv(m, 64) * cdiv(n, 64);
     int best = 1;
@@ -1054,6 +1352,46 @@ static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
         if (us < least) { least = us; best = sp; }
     }
     return best;
+}
+
+// The split kernel's tiles and splits, fitted as above to measurements at M = 65 .. 8192 of GPT-2's layers (K = 768 with N = 768, 2304, 3072 and K = 3072, N = 768;
+// weights from memory, 1 to 8 splits; k tiles of 16): within 6 % rms, worst 16 %; over those 44 shapes the pick is 2.1 % slower than the best choice in
+// the mean.  Up to two rows of 64 x 64 tiles the f32 cores keep up on 4 bytes a weight instead of 6 (M = 128, us, f32 and split: 11.8 and 12.9, 9.8 and 10.0, 14.0 and
+// 13.4, K = 3072 15.1 and 14.6; M = 200: 16.2 and 15.3, 10.4 and 10.5, 17.2 and 15.7, 19.9 and 18.4).
+static bool mfma_splits_f32(int64_t m) { return m > 128; }
+enum SplitTileId { kS256x96, kS128x96, kS64x64, kSTiles };
+static const TileCost kSplitCost[kSTiles] = {{256, 96, 256, 6.0, 0.576, 0.289, 2.6, 0.29}, {128, 96, 512, 4.9, 0.497, 0.186, 2.8, 0.33}, {64, 64, 512, 2.8, 0.203, 0.10, 4.1, 0.19}};
+static TilePlan split_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
+    TilePlan best{kS64x64, 1};
+    double least = 1e300;
+    for (int t = dual ? kS64x64 : 0; t < kSTiles; ++t) {   // a pair: 64 x 64 of each matrix
+        const TileCost& c = kSplitCost[t];
+        const int64_t tiles = cdiv(m, c.bm) * cdiv(n, c.bn);
+        for (int sp : {1, 2, 3, 4, 6, 8, 12}) {
+            if (sp > 1 && (!splits_allowed() || k < 128 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+            const double kt = (dual ? 2.0 : 1.0) * (double)k / 16 / sp, wg = (double)(tiles * sp);
+            double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
+            if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
+            if (us < least) { least = us; best = {t, sp}; }
+        }
+    }
+    return best;
+}
+template <int WM, int WN, int TN, int KS, int NST, bool DUAL>
+static void launch_split(hipStream_t s, const MfmaLinearArgs& a, int splits) {
+    constexpr int BM = 32 * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
+    constexpr int ring = NST * KS * (BM * 64 + BN * 96), area = WM * WN * 32 * (32 * (DUAL ? TN / 2 : TN) + 4) * 4, lds_bytes = ring > area ? ring : area;
+    auto kern = gemm_split_kernel<WM, WN, TN, KS, NST, DUAL>;
+    static bool configured = false;  // the attribute is per function, not per stream or device state
+    if (!configured) {
+        (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+        configured = true;
+    }
+    const int64_t nt = cdiv(a.n, NREAL), mt = cdiv(a.m, BM);
+    TileEpilogue<float> epi{(const float*)a.bias, a.residual, a.y, a.n, a.act, 0, a.extra};
+    const SplitOperands of{(const float*)a.x, (const bf16_t*)a.wk, (const bf16_t*)a.wk2, (int)a.k, (int)mfma_padded_n(a.n)};
+    kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN, lds_bytes, s>>>((int)a.m, (int)nt, (int)mt, splits, (float*)a.part, of, epi);
+    if (splits > 1) gemm_reduce_kernel<float, DUAL, true><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi, of);
 }
 
 // Quantised: which tile converts the codes of which columns.  Every wave converts the B fragments it multiplies, 20 (int8) or
@@ -1103,7 +1441,7 @@ static size_t staged_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
 }
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant) {
     if (!mfma_gemm_supported(dtype, m, k, n, quant)) return 0;
-    if (dtype == 0) return tile_part_bytes(m, n, dual, tile_splits_f32(m, k, n, dual));
+    if (dtype == 0) return tile_part_bytes(m, n, dual, mfma_splits_f32(m) ? split_plan(m, k, n, dual).splits : tile_splits_f32(m, k, n, dual));
     const int qsp = quant_plan(m, k, n, dual).splits;
     return std::max(tile_part_bytes(m, n, dual, quant ? qsp : tile_plan(m, k, n, dual).splits), staged_part_bytes(m, n, dual, qsp));
 }
@@ -1134,6 +1472,11 @@ size_t mfma_int4_lds_bytes(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
     return p.tile < 0 ? 0 : (size_t)int4_lds_bytes(kQuantCost[dual][p.tile].bm, kQuantCost[dual][p.tile].bn, k, p.splits);
 }
 
+// The LDS-direct kernels' loads address a k tile with 32-bit offsets from one scalar base: 256 rows of x, 8 k-groups of
+// the padded weights (6 of the split ones).
+static bool mfma_lds_direct_reach(int64_t k, int64_t n) { return k <= (1 << 21) && (uint64_t)mfma_padded_n(n) * 128 < (1ull << 31); }
+bool mfma_takes_split_weights(int dtype, int64_t m, int64_t k, int64_t n, int lds_direct) { return dtype == 0 && lds_direct != 0 && mfma_splits_f32(m) && mfma_lds_direct_reach(k, n); }
+
 template <bool DUAL, int QF>
 static void launch_quant(hipStream_t s, const MfmaLinearArgs& a) {
     const TilePlan p = quant_plan(a.m, a.k, a.n, DUAL, room_of(a));
@@ -1154,9 +1497,7 @@ static void launch_quant(hipStream_t s, const MfmaLinearArgs& a) {
 
 void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
     const bool dual = a.wk2 != nullptr;
-    // the LDS-direct kernel's loads address a k tile with 32-bit offsets from one scalar base: 256 rows of x, 8 k-groups of
-    // the padded weights
-    const bool reach = a.k <= (1 << 21) && (uint64_t)mfma_padded_n(a.n) * 128 < (1ull << 31);
+    const bool reach = mfma_lds_direct_reach(a.k, a.n);
     if (a.lds_direct == 0 || !reach) {
         // the splits of a layer of codes of this shape, for them and for the matrix that they stand for: the same sums in the same order
         const int sp = reach && a.dtype == 2 ? quant_plan(a.m, a.k, a.n, dual).splits : 1;
@@ -1167,6 +1508,13 @@ void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
     }
     if (a.quant == 1) return dual ? launch_quant<true, 1>(s, a) : launch_quant<false, 1>(s, a);
     if (a.quant == 2) return dual ? launch_quant<true, 2>(s, a) : launch_quant<false, 2>(s, a);
+    if (a.dtype == 0 && mfma_splits_f32(a.m)) {
+        const TilePlan p = split_plan(a.m, a.k, a.n, dual, room_of(a));
+        if (dual) return launch_split<2, 2, 2, 2, 3, true>(s, a, p.splits);
+        if (p.tile == kS256x96) return launch_split<8, 1, 3, 2, 3, false>(s, a, p.splits);
+        if (p.tile == kS128x96) return launch_split<4, 1, 3, 1, 4, false>(s, a, p.splits);
+        return launch_split<2, 2, 1, 2, 3, false>(s, a, p.splits);
+    }
     if (a.dtype == 0) {
         const int sp = tile_splits_f32(a.m, a.k, a.n, dual, room_of(a));
         return dual ? launch_tile<float, 8, 3, 2, 2, 1, 2, true>(s, a, sp) : launch_tile<float, 8, 3, 2, 2, 1, 1, false>(s, a, sp);

@@ -1158,7 +1158,7 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
                 ma.x = src_ptr(st, cx, 0);
                 ma.m = x.dims[0]; ma.k = x.dims[1]; ma.n = w.dims[1];
                 // quantised weights: the k-grouped copy holds the codes; the kernel applies the scales on the way into LDS
-                const int kind = in.quant == 0 ? 1 : (in.quant == 1 ? 6 : 7);
+                const int kind = k::mfma_takes_split_weights(ma.dtype, ma.m, ma.k, ma.n, ma.lds_direct) ? 12 : in.quant == 0 ? 1 : (in.quant == 1 ? 6 : 7);
                 BufferP wk = cx.be->derived_weights(cx.input_bufs[st.tiled_w_input], kind, ldt, ma.k, ma.n);
                 BufferP wk2;
                 ma.wk = wk->ptr;

@@ -116,6 +116,73 @@ def test_f32_sums_in_two_chains(hip):
     assert np.linalg.norm(got - want) <= 1.2 * 0.42 * 2.0 ** -24 * np.sqrt(k / 4) * np.linalg.norm(want)
 
 
+def f32_layers(hip, x, w, w2, bias, res):
+    """x.w + res, x.w + bias and silu(x.w) * (x.w2), each run twice"""
+    def run(specs, body, args):
+        fb = FunctionBuilder("main", "F32")
+        fb.set_results([body(*[fb.param("F32", dims) for dims in specs])])
+        got = [hip_run(hip, Program(fb), args)[0] for _ in range(2)]
+        assert np.array_equal(got[0], got[1], equal_nan=True)
+        return got[0]
+
+    (m, k), n = x.shape, w.shape[1]
+    return (run([(m, k), (k, n), (m, n)], lambda a, b, r: F.linear(a, b) + r, [x, w, res]), run([(m, k), (k, n), (n,)], lambda a, b, c: F.linear(a, b, c), [x, w, bias]),
+            run([(m, k), (k, n), (k, n)], lambda a, b, c: F.swiglu(F.linear(a, b), F.linear(a, c)), [x, w, w2]))
+
+
+# f32 of more than 128 rows as six bf16 products (fewer: f32 products): rows around the tiles' 64, 128 and 256, columns around 64 and 96 and no multiples of 8, two k tiles,
+# fewer and more than the ring, whole and in splits.  `scale` takes the rows far from 1, up and down
+@pytest.mark.parametrize("m,k,n,scale", [(129, 32, 8, 1.0), (130, 96, 63, 1e18), (160, 3072, 97, 1.0), (191, 64, 193, 1.0), (193, 800, 770, 1e-29), (255, 768, 2304, 1.0), (511, 3072, 767, 1.0),
+                                         (700, 736, 3070, 1e-18), (1025, 1536, 1000, 1.0), (2047, 768, 3073, 1.0), (2305, 3104, 769, 1.0)])
+def test_f32_as_bf16_products(hip, m, k, n, scale):
+    rng = np.random.default_rng(m + k + n)
+    x, w, w2 = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (k, n), (k, n)))
+    x, w, w2 = x * np.float32(scale), w * np.float32(k ** -0.5), w2 * np.float32(k ** -0.5)
+    bias, res = (rng.standard_normal(s, dtype=np.float32) * np.float32(scale) for s in ((n,), (m, n)))
+    plain, biased, pair = f32_layers(hip, x, w, w2, bias, res)
+    rows = sorted({r for r in (0, 31, 63, 64, 95, 96, 127, 128, 255, 256, 1000, m - 2, m - 1) if r < m})
+    x64, w64, v64 = x[rows].astype(np.float64), w.astype(np.float64), w2.astype(np.float64)
+    s, t = x64 @ w64, x64 @ v64
+    # every term is off by 2^-23.9 at the most, and 2 sqrt(k) roundings of the sum of magnitudes as above
+    bs, bt = (2 * (np.sqrt(k) + 1) * 2.0 ** -24 * (np.abs(x64) @ np.abs(v)) for v in (w64, v64))
+    assert (np.abs(plain[rows] - (s + res[rows])) <= bs + 2.0 ** -23 * np.abs(s + res[rows])).all()
+    assert (np.abs(biased[rows] - (s + bias)) <= bs + 2.0 ** -23 * np.abs(s + bias)).all()
+    if scale == 1.0:
+        g = s / (1 + np.exp(-s))
+        assert (np.abs(pair[rows] - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + 2.0 ** -20 * np.abs(g * t) + 1e-12).all()
+    # in the mean: a chain of n = k / 8 roundings of 0.42 * 2^-24 each is (n + 1) / 2 of their squares away (see test_f32_sums_in_two_chains), the sum
+    # of the large and the small products 1 and the residual, which doubles the value's square, 2.  A quotient of two norms of so many values is itself
+    # 1 / sqrt(values) uncertain: three of those, beside that test's fifth
+    far = np.linalg.norm(plain[rows] - (s + res[rows])) / np.linalg.norm(s)
+    assert far <= (1.2 + 3 / np.sqrt(s.size)) * 0.42 * 2.0 ** -24 * np.sqrt((k / 8 + 1) / 2 + 3)
+
+
+# infinities, NaN and values that round to infinity in bf16: what f32 products give, whole tiles and splits, both matrices of a pair
+@pytest.mark.parametrize("m,k,n", [(129, 64, 40), (140, 3072, 100), (300, 96, 193), (2100, 64, 3000)])
+def test_f32_as_bf16_products_not_finite(hip, m, k, n):
+    rng = np.random.default_rng(m)
+    x, w, w2 = (rng.uniform(0.5, 1, s).astype(np.float32) * rng.choice([-1, 1], s).astype(np.float32) for s in ((m, k), (k, n), (k, n)))
+    w, w2 = w / np.float32(k), w2 / np.float32(k)
+    x[3, 5], x[7, k - 1], x[m - 1, 0], x[20, 3], x[20, 4], x[33] = np.inf, np.nan, -np.inf, np.inf, -np.inf, np.float32(3.4e38)
+    w[11, 2], w[k - 1, n - 1], w2[5, 6], w[9, 8] = -np.inf, np.nan, np.inf, np.float32(3.4e38)
+    x[33, 1::2] *= -1                                      # terms of 3.4e38 / k, a sum that no order takes out of range
+    x[33, [9, 11, k - 1]] = 0.0
+    plain, biased, pair = f32_layers(hip, x, w, w2, np.zeros(n, np.float32), np.zeros((m, n), np.float32))
+    with np.errstate(all="ignore"):
+        s, t = ((x.astype(np.float64) @ v.astype(np.float64)).astype(np.float32) for v in (w, w2))
+        both = (s.astype(np.float64) / (1 + np.exp(-s.astype(np.float64))) * t).astype(np.float32)
+    odd = ~np.isfinite(s)
+    scale = np.abs(np.where(np.isfinite(x), x, 0)).max(1, keepdims=True) * np.ones(n)
+    scale[:, 8] = 3.4e38
+    for got in (plain, biased):
+        assert np.array_equal(got[odd], s[odd], equal_nan=True)
+        assert (np.abs(got[~odd].astype(np.float64) - s[~odd]) <= 1e-5 * scale[~odd]).all()
+    clear = np.isfinite(s) & np.isfinite(t) & np.isfinite(both)
+    assert odd.sum() > 2 * n and np.isfinite(pair[clear]).all()
+    gone = np.isnan(both)
+    assert gone.any() and np.isnan(pair[gone & ~np.isneginf(s)]).all()      # (silu of an infinite negative gate: either zero or NaN)
+
+
 # codes converted on the way to the matrix pipes: odd columns, one k tile pair, k tiles that split in the middle of an int4 group, rows
 # around the tiles' 64 and 128
 @pytest.mark.parametrize("scheme", ["w8", "w4g128"])
