@@ -146,8 +146,8 @@ void tile_weights(hipStream_t s, int dtype, const void* w, void* wt, int64_t k, 
 bool gemv_tiled_supported(int dtype, int64_t m, int64_t k, int64_t n);
 void gemv_tiled(hipStream_t s, const TiledLinearArgs& a);
 
-// Batched-decode linear layers (2 <= M <= 16, bf16 or f32) on the matrix cores over a 16-column tiled, k-grouped copy
-// of the weights, Ws[tile][K/KPC][16][KPC] with KPC = 8 (bf16) or 4 (f32) k per 16 bytes (kernels_skinny.hip).  ws2 != nullptr: SwiGLU pair.  act: 0 none, 1 gelu.
+// Batched-decode linear layers (2 <= M <= 16, bf16 or f32) on the matrix cores over a tiled, k-grouped copy
+// of the weights, Ws[tile][K/KPC][12 or 16 columns][KPC] with KPC = 8 (bf16) or 4 (f32) k per 16 bytes (kernels_skinny.hip).  ws2 != nullptr: SwiGLU pair.  act: 0 none, 1 gelu.
 struct SkinnyLinearArgs {
     int dtype;   // 0 f32, 2 bf16
     const void* x; const void* ws; const void* ws2; const void* bias; const void* residual;

@@ -5,13 +5,13 @@
 // until the vector ALUs, not memory, set the pace.  One v_mfma_f32_16x16x32_bf16 multiplies 16 rows by a
 // 32 x 16 block of W at a cost that does not depend on M, so the kernel below only has to stream W.
 //
-// Weights are read from a derived copy Ws[tile][K/8][16 columns][8 k] (tile = 16 output columns): the 64 lanes of
-// a wave fetch 32 consecutive k of the tile's 16 columns as ONE contiguous KiB in exactly the B-operand layout
-// (lane = 16 * k-group + column holds 8 consecutive k of its column).  A workgroup owns one tile; its 4, 8 or 16 waves
+// Weights are read from a derived copy Ws[tile][K/8][16 columns][8 k] (tile = 16 output columns, or 12: skinny_cols): the 64 lanes of
+// a wave fetch 32 consecutive k of the tile's columns as ONE contiguous KiB in exactly the B-operand layout
+// (lane = 16 * k-group + column holds 8 consecutive k of its column).  A workgroup owns one tile; its 8 or 16 waves
 // (skinny_plan) take the 32-k steps round-robin (so the workgroup reads consecutive KiB) and add their partial products
 // through LDS.  The A operand (lane = 16 * k-group + row) comes straight from x, which is small and stays in L2.
 // DUAL computes silu(x.W) * (x.W2) (ops/functional/activation.rs:141-162) from two weight copies.
-// f32 takes the same route with 4 k per 16-byte lane word (Ws[tile][K/4][16][4], 16-k steps) on four
+// f32 takes the same route with 4 k per 16-byte lane word (Ws[tile][K/4][16 or 12][4], 16-k steps) on four
 // v_mfma_f32_16x16x4_f32 per word.
 //
 // Weight-only quantised layers (skinny_gemm_quant_kernel<QF, DUAL>) stream the CODES: a lane's 16-byte word holds 16
@@ -21,9 +21,12 @@
 // sum_k x[row, k], which takes the bias out again (x.(q + b) - b.sum x).  int8 scales (per column) are applied in the
 // epilogue, int4 group scales when a group's sums are added to the running total.
 //
-// A layer with few tiles (under 96) is split along K over gridDim.y workgroups per tile so that more of the chip streams: each writes its 16 x 16 partial sums to a workspace and takes a ticket; the
-// workgroup that draws the last ticket of a tile adds the partials in split order (so the result does not depend on
-// which one that is), applies the epilogue and resets the ticket for the next launch.
+// A layer with few tiles is split along K over gridDim.y workgroups per tile so that more of the chip streams: each writes its
+// 16 x 16 partial sums to a workspace and takes a ticket; the workgroup that draws the last ticket of a tile adds the partials in split
+// order (so the result does not depend on which one that is), applies the epilogue and resets the ticket for the next launch.
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "device_utils.hpp"
 
@@ -61,16 +64,16 @@ template <> struct SkinnyT<float> {
     static __device__ __forceinline__ void st(float* p, int64_t i, float v) { p[i] = v; }
 };
 
-// Ws[tile][kb][c][i] = W[KPC kb + i][16 tile + c], zero outside [K) x [N); one thread per 16-byte group
+// Ws[tile][kb][c][i] = W[KPC kb + i][cols tile + c], zero outside [K) x [N); one thread per 16-byte group
 template <typename T>
 __global__ __launch_bounds__(256) void skinny_pack_kernel(const T* __restrict__ w, T* __restrict__ out, int64_t K, int64_t N,
-                                                          int64_t KB, int64_t ntiles) {
+                                                          int64_t KB, int64_t ntiles, int cols) {
     constexpr int KPC = SkinnyT<T>::KPC;
-    const int64_t total = ntiles * KB * 16;
+    const int64_t total = ntiles * KB * cols;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(g & 15);
-        const int64_t kb = (g >> 4) % KB, tile = (g >> 4) / KB;
-        const int64_t col = tile * 16 + c;
+        const int c = (int)(g % cols);
+        const int64_t kb = g / cols % KB, tile = g / cols / KB;
+        const int64_t col = tile * cols + c;
         alignas(16) T r[KPC];
 #pragma unroll
         for (int i = 0; i < KPC; ++i) {
@@ -90,39 +93,112 @@ __device__ __forceinline__ float skinny_finish(float v, float v2, bool dual, int
     return v;
 }
 
-template <typename T, bool DUAL, int NW, int U>
+// The way out, shared by both kernels: the workgroup's first 256 threads add an output each, thread 16 m + c row m of the tile's column
+// c, so a wave's LDS reads meet no bank twice and a row's stores are neighbours.  What an output needs besides its sum is requested
+// before the first weight (the constructor) and has long arrived.  One output's code instead of four per lane of one wave, and no
+// round trip to memory at the end: 8 rows, us: K = 9216,
+// N = 3072 13.4 -> 12.8, N = 6144 9.9 -> 9.4, f32 K = 768, N = 768 4.7 -> 4.3; int4 pair of 9216 17 -> 12.
+template <typename T, bool DUAL, int NW, int COLS>
+struct SkinnyOut {
+    static constexpr int NP = DUAL ? 2 : 1;
+    const int m, c, n;
+    const bool in;
+    int64_t at;
+    float bias, res, colscale;
+    __device__ __forceinline__ SkinnyOut(int tile, int M, int N, const T* pbias, const void* residual, int out_f32, const float* pscale)
+        : m((int)threadIdx.x >> 4), c((int)threadIdx.x & 15), n(tile * COLS + c), in(m < M && c < COLS && n < N), at((int64_t)m * N + n), bias(0.f), res(0.f), colscale(1.0f) {
+        if (!in) return;
+        if (pbias) bias = SkinnyT<T>::ld(pbias, n);
+        if (pscale) colscale = pscale[n];
+        if (residual) res = out_f32 ? static_cast<const float*>(residual)[at] : SkinnyT<T>::ld(static_cast<const T*>(residual), at);
+    }
+    // Behind a barrier after the waves' sums.  False: another workgroup finishes the tile, or the thread has no output.
+    __device__ __forceinline__ bool sum(const float (*red)[NP][64][4], int tile, float* part, unsigned* tickets, unsigned* ticket_lds, float (&v)[2]) {
+        asm volatile("" : "+v"(bias), "+v"(res), "+v"(colscale));       // requested up there, not here
+        if (threadIdx.x >= 256) return false;
+        const int lane = 16 * (m >> 2) + c, i = m & 3;                   // D: lane holds rows 4 kg .. 4 kg + 3 of column c
+        v[0] = v[1] = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            v[0] += red[w][0][lane][i];
+            if (DUAL) v[1] += red[w][NP - 1][lane][i];
+        }
+        const int ksplit = gridDim.y;
+        if (ksplit > 1) {
+            // partials and tickets cross workgroups through device-scope accesses only (coherent across the L2s of the
+            // XCDs without cache maintenance): stores acknowledged, then the ticket
+            float* mine = part + ((int64_t)tile * ksplit + blockIdx.y) * NP * 256 + threadIdx.x;
+            __hip_atomic_store(mine, v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (DUAL) __hip_atomic_store(mine + 256, v[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0)
+            __syncthreads();                                            // (the waves that are left: 256 threads)
+            if (threadIdx.x == 0) *ticket_lds = __hip_atomic_fetch_add(&tickets[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();                                            // the partials are read after the ticket is known
+            if (*ticket_lds != (unsigned)(ksplit - 1)) return false;
+            // every ticket of this launch has been drawn: leave the counter at zero for the next one
+            if (threadIdx.x == 0) __hip_atomic_store(&tickets[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v[0] = v[1] = 0.f;
+            for (int q = 0; q < ksplit; ++q) {                           // device-scope loads: the partials come from other CUs
+                const float* src = part + ((int64_t)tile * ksplit + q) * NP * 256 + threadIdx.x;
+                v[0] += __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (DUAL) v[1] += __hip_atomic_load(src + 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        return in;
+    }
+    // out_f32: the f32 accumulator (plus an f32 residual) is stored as it is
+    __device__ __forceinline__ void store(T* y, int out_f32, float o) {
+        if (out_f32) reinterpret_cast<float*>(y)[at] = o;
+        else SkinnyT<T>::st(y, at, o);
+    }
+};
+
+template <typename T, bool DUAL, int NW, int U, int COLS>
 __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const T* __restrict__ x, const T* __restrict__ ws,
                                                           const T* __restrict__ ws2, const T* __restrict__ bias,
                                                           const T* __restrict__ residual, T* __restrict__ y, int M, int K,
                                                           int N, int act, float* __restrict__ part, unsigned* __restrict__ tickets,
                                                           int out_f32, EpiExtra extra) {
+    static_assert(COLS == 12 || COLS == 16, "columns of a tile");
     constexpr int KPC = SkinnyT<T>::KPC, KSTEP = 4 * KPC;
     __shared__ float red[NW][DUAL ? 2 : 1][64][4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ unsigned ticket;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));   // uniform: a matrix instruction does not look at the lane mask, so the tests of a step must be branches
     const int c = lane & 15, kg = lane >> 4;     // B: column c, k-group kg; A: row c, k-group kg
     const int tile = blockIdx.x;
+    SkinnyOut<T, DUAL, NW, COLS> out(tile, M, N, bias, residual, out_f32, extra.colscale);
     const int ksplit = gridDim.y, ks = blockIdx.y;
     const int s_begin = (int)((int64_t)(K / KSTEP) * ks / ksplit), nsteps = (int)((int64_t)(K / KSTEP) * (ks + 1) / ksplit);
-    const u32x4_s* bsrc = reinterpret_cast<const u32x4_s*>(ws) + (int64_t)tile * (K / KPC) * 16 + lane;
-    const u32x4_s* bsrc2 = DUAL ? reinterpret_cast<const u32x4_s*>(ws2) + (int64_t)tile * (K / KPC) * 16 + lane : nullptr;
+    const int bcol = c < COLS ? c : COLS - 1;    // columns beyond the tile re-read its last one; their sums are never stored
+    const int64_t b0 = (int64_t)tile * (K / KPC) * COLS + kg * COLS + bcol;
+    const u32x4_s* bsrc = reinterpret_cast<const u32x4_s*>(ws) + b0;
+    const u32x4_s* bsrc2 = DUAL ? reinterpret_cast<const u32x4_s*>(ws2) + b0 : nullptr;
     const int arow = c < M ? c : M - 1;          // rows beyond M re-read the last one; their products are never stored
     const u32x4_s* asrc = reinterpret_cast<const u32x4_s*>(x + (int64_t)arow * K + KPC * kg);
 
+    // A ring of U steps: a step's registers are asked to fetch the wave's next but U - 1 as soon as they have been multiplied, so
+    // a wave has U - 1 or U requests on their way all the time.  (Rounds of U requests, all awaited before the next were made, left the memory
+    // pipeline empty once a round: K = 9216, N = 3072, 8 rows 17.0 us; this 14.9, with tiles of 12 columns 11.8.)
     f32x4_s acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = s_begin + wave; s0 < nsteps; s0 += NW * U) {
-        u32x4_s b[U], b2[DUAL ? U : 1], a[U];
+    u32x4_s b[U], b2[DUAL ? U : 1], a[U];
+    auto fetch = [&](int u, int s) {
+        b[u] = __builtin_nontemporal_load(bsrc + (int64_t)s * (4 * COLS));
+        if (DUAL) b2[DUAL ? u : 0] = __builtin_nontemporal_load(bsrc2 + (int64_t)s * (4 * COLS));
+        a[u] = asrc[s * 4];
+    };
+    if (s_begin + wave < nsteps) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int s = s0 + NW * u < nsteps ? s0 + NW * u : s0;   // a step past the end repeats the first, weight zero below
-            b[u] = __builtin_nontemporal_load(bsrc + (int64_t)s * 64);
-            if (DUAL) b2[u] = __builtin_nontemporal_load(bsrc2 + (int64_t)s * 64);
-            a[u] = asrc[s * 4];
-        }
+        for (int u = 0; u < U; ++u) fetch(u, s_begin + wave + NW * u < nsteps ? s_begin + wave + NW * u : s_begin + wave);   // (a step past the end is not multiplied)
+        for (int s0 = s_begin + wave; s0 < nsteps; s0 += NW * U) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (s0 + NW * u < nsteps) {
-                acc = SkinnyT<T>::mma(a[u], b[u], acc);
-                if (DUAL) acc2 = SkinnyT<T>::mma(a[u], b2[DUAL ? u : 0], acc2);
+            for (int u = 0; u < U; ++u) {
+                const int s = s0 + NW * u;
+                if (s < nsteps) {
+                    acc = SkinnyT<T>::mma(a[u], b[u], acc);
+                    if (DUAL) acc2 = SkinnyT<T>::mma(a[u], b2[DUAL ? u : 0], acc2);
+                }
+                if (s + NW * U < nsteps) fetch(u, s + NW * U);
             }
         }
     }
@@ -132,63 +208,11 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const T* __restric
         if (DUAL) red[wave][DUAL ? 1 : 0][lane][i] = acc2[i];
     }
     __syncthreads();
-    if (wave != 0) return;
-    constexpr int NP = DUAL ? 2 : 1;
-    float g[4], up[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        g[i] = up[i] = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            g[i] += red[w][0][lane][i];
-            if (DUAL) up[i] += red[w][DUAL ? 1 : 0][lane][i];
-        }
-    }
-    if (ksplit > 1) {
-        // partials and tickets cross workgroups through device-scope accesses only (coherent across the L2s of the
-        // XCDs without cache maintenance): stores acknowledged, then the ticket
-        float* mine = part + ((int64_t)tile * ksplit + ks) * NP * 256 + lane * 4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __hip_atomic_store(mine + i, g[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (DUAL) __hip_atomic_store(mine + 256 + i, up[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0)
-        asm volatile("" ::: "memory");
-        unsigned t = 0;
-        if (lane == 0) t = __hip_atomic_fetch_add(&tickets[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        t = __shfl(t, 0, 64);
-        if (t != (unsigned)(ksplit - 1)) return;
-        asm volatile("" ::: "memory");                              // the partials are read after the ticket is known
-        // every ticket of this launch has been drawn: leave the counter at zero for the next one
-        if (lane == 0) __hip_atomic_store(&tickets[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) g[i] = up[i] = 0.f;
-        for (int q = 0; q < ksplit; ++q) {
-            const float* src = part + ((int64_t)tile * ksplit + q) * NP * 256 + lane * 4;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {                           // device-scope loads: the partials come from other CUs
-                g[i] += __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (DUAL) up[i] += __hip_atomic_load(src + 256 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-    }
-    const int n = tile * 16 + c;
-    if (n >= N) return;
-    const float bv = bias ? SkinnyT<T>::ld(bias, n) : 0.f;
-    const float cs = extra.colscale ? extra.colscale[n] : 1.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = 4 * kg + i;                // D: lane holds rows 4 kg .. 4 kg + 3 of column c
-        if (m >= M) continue;
-        // out_f32: the f32 accumulator (plus an f32 residual) is stored as it is
-        const float r = residual ? (out_f32 ? reinterpret_cast<const float*>(residual)[(int64_t)m * N + n]
-                                            : SkinnyT<T>::ld(residual, (int64_t)m * N + n)) : 0.f;
-        float o = skinny_finish(g[i], up[i], DUAL, act, bv, residual != nullptr, r, extra.glu, cs);
-        if (extra.softcap != 0.f) o = softcap_f32(o, extra.softcap);
-        if (out_f32) reinterpret_cast<float*>(y)[(int64_t)m * N + n] = o;
-        else SkinnyT<T>::st(y, (int64_t)m * N + n, o);
-    }
+    float v[2];
+    if (!out.sum(red, tile, part, tickets, &ticket, v)) return;
+    float o = skinny_finish(v[0], v[1], DUAL, act, out.bias, residual != nullptr, out.res, extra.glu, out.colscale);
+    if (extra.softcap != 0.f) o = softcap_f32(o, extra.softcap);
+    out.store(y, out_f32, o);
 }
 
 // Qs[tile][S][lane = 16 kg + c][16 bytes]: byte i = code row (RPW S + RPL kg + i) of column 16 tile + c, xor flip.  int8:
@@ -251,9 +275,12 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_quant_kernel(const bf16_t
     constexpr int NP = DUAL ? 2 : 1;
     constexpr float BIAS = QF == 1 ? 128.0f : 8.0f;
     __shared__ float red[NW][NP][64][4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ unsigned ticket;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));   // uniform: a matrix instruction does not look at the lane mask, so the tests of a step must be branches
     const int c = lane & 15, kg = lane >> 4;
     const int tile = blockIdx.x;
+    SkinnyOut<bf16_t, DUAL, NW, 16> out(tile, M, N, bias, residual, out_f32, nullptr);
     const int ksplit = gridDim.y, ks = blockIdx.y;
     const int nwords = K / KPW;
     const int s_begin = (int)((int64_t)nwords * ks / ksplit), s_end = (int)((int64_t)nwords * (ks + 1) / ksplit);
@@ -326,58 +353,10 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_quant_kernel(const bf16_t
         if (DUAL) red[wave][DUAL ? 1 : 0][lane][i] = tot2[i];
     }
     __syncthreads();
-    if (wave != 0) return;
-    float g[4], up[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        g[i] = up[i] = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            g[i] += red[w][0][lane][i];
-            if (DUAL) up[i] += red[w][DUAL ? 1 : 0][lane][i];
-        }
-    }
-    if (ksplit > 1) {   // as in skinny_gemm_kernel
-        float* mine = part + ((int64_t)tile * ksplit + ks) * NP * 256 + lane * 4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __hip_atomic_store(mine + i, g[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (DUAL) __hip_atomic_store(mine + 256 + i, up[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0)
-        asm volatile("" ::: "memory");
-        unsigned t = 0;
-        if (lane == 0) t = __hip_atomic_fetch_add(&tickets[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        t = __shfl(t, 0, 64);
-        if (t != (unsigned)(ksplit - 1)) return;
-        asm volatile("" ::: "memory");
-        if (lane == 0) __hip_atomic_store(&tickets[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) g[i] = up[i] = 0.f;
-        for (int q = 0; q < ksplit; ++q) {
-            const float* src = part + ((int64_t)tile * ksplit + q) * NP * 256 + lane * 4;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                g[i] += __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (DUAL) up[i] += __hip_atomic_load(src + 256 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-    }
-    const int n = tile * 16 + c;
-    if (n >= N) return;
-    const float bv = bias ? bf16_to_f32(bias[n]) : 0.f;
-    const float s1 = QF == 1 ? bf16_to_f32(sc[n]) : 1.0f;
-    const float s2 = QF == 1 && DUAL ? bf16_to_f32(sc2[n]) : 1.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = 4 * kg + i;
-        if (m >= M) continue;
-        const float r = residual ? (out_f32 ? reinterpret_cast<const float*>(residual)[(int64_t)m * N + n]
-                                            : bf16_to_f32(residual[(int64_t)m * N + n])) : 0.f;
-        const float o = skinny_finish(g[i] * s1, up[i] * s2, DUAL, act, bv, residual != nullptr, r);
-        if (out_f32) reinterpret_cast<float*>(y)[(int64_t)m * N + n] = o;
-        else y[(int64_t)m * N + n] = f32_to_bf16(o);
-    }
+    float v[2];
+    if (!out.sum(red, tile, part, tickets, &ticket, v)) return;
+    const float s1 = QF == 1 ? bf16_to_f32(sc[out.n]) : 1.0f, s2 = QF == 1 && DUAL ? bf16_to_f32(sc2[out.n]) : 1.0f;
+    out.store(y, out_f32, skinny_finish(v[0] * s1, v[1] * s2, DUAL, act, out.bias, residual != nullptr, out.res));
 }
 
 }  // namespace
@@ -387,43 +366,58 @@ bool skinny_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n) {
     const int64_t kstep = dtype == 0 ? 16 : 32;
     return m >= 2 && m <= 16 && k >= kstep && k % kstep == 0 && n >= 1 && k < (1ll << 31) && n < (1ll << 31) - 16;
 }
+// Columns of a tile of the copy.  A workgroup is one tile, and while there are few of them the CU with the most columns sets the
+// time: tiles of 12 where they leave fewer columns on it (N = 3072: 256 tiles, one for every CU, instead of 192; N = 9216 three a CU instead
+// of three on some and two on others).  The MFMA's other four columns are wasted, which costs nothing here; from 768 tiles of 16 on
+// the CUs are evenly loaded either way and whole instructions are the better use of the memory pipeline.  us with 16 and with 12 columns, 8
+// rows: K = 9216, N = 3072 14.9 and 11.8, K = 4096 7.8 and 6.7, K = 3072 N = 6144 10.0 and 8.6, pair of 9216 23.0 and 19.7; N = 32768 35.7
+// and 38.6.
+static int skinny_cols(int64_t n) {
+    const int64_t t16 = cdiv_s(n, 16), t12 = cdiv_s(n, 12);
+    return t16 < 768 && cdiv_s(t12, 256) * 12 < cdiv_s(t16, 256) * 16 ? 12 : 16;
+}
 size_t skinny_weight_bytes(int dtype, int64_t k, int64_t n) {
-    const int64_t kpc = dtype == 0 ? 4 : 8;
-    return (size_t)(cdiv_s(n, 16) * cdiv_s(k, kpc) * 16) * 16;
+    const int64_t kpc = dtype == 0 ? 4 : 8, cols = skinny_cols(n);
+    return (size_t)(cdiv_s(n, cols) * cdiv_s(k, kpc) * cols) * 16;
 }
 void skinny_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int64_t k, int64_t n) {
-    const int64_t ntiles = cdiv_s(n, 16), kb = cdiv_s(k, dtype == 0 ? 4 : 8), total = ntiles * kb * 16;
+    const int64_t cols = skinny_cols(n), ntiles = cdiv_s(n, cols), kb = cdiv_s(k, dtype == 0 ? 4 : 8), total = ntiles * kb * cols;
     if (total <= 0) return;
     const unsigned g = (unsigned)(cdiv_s(total, 256) > 65536 ? 65536 : cdiv_s(total, 256));
-    if (dtype == 0) skinny_pack_kernel<float><<<g, 256, 0, s>>>((const float*)w, (float*)out, k, n, kb, ntiles);
-    else skinny_pack_kernel<bf16_t><<<g, 256, 0, s>>>((const bf16_t*)w, (bf16_t*)out, k, n, kb, ntiles);
+    if (dtype == 0) skinny_pack_kernel<float><<<g, 256, 0, s>>>((const float*)w, (float*)out, k, n, kb, ntiles, (int)cols);
+    else skinny_pack_kernel<bf16_t><<<g, 256, 0, s>>>((const bf16_t*)w, (bf16_t*)out, k, n, kb, ntiles, (int)cols);
 }
-// How a launch shares out the steps (words of codes) of a tile: waves per workgroup, workgroups per tile.  Every layer is one pass over its weights; what is left beside HBM's pace are the rounds of a wave (a request and its
-// answer, about 1.5 us each) and, with several workgroups to a tile, their meeting (3 us).  So a layer of at most one tile per CU
-// takes 16 waves to a tile and none of the splits that kept the chip busy with four (8 rows, bf16, us: K = 4096, N = 3072 10.4 ->
-// 8.6, K = 9216 16.0 -> 14.6, f32 K = 768, N = 2304 6.8 -> 5.7; int8 9.0 -> 6.8, 12.6 -> 10.6); up to three tiles per CU, and pairs
-// and codes (which a wave also has to convert) beyond, 8 waves (K = 3072: N = 6144 11.3 -> 10.7, pair of 9216 23.6 -> 20.3, int8
-// N = 6144 11.8 -> 8.2, int4 N = 32768 29.4 -> 20.5); plain layers with more tiles 4 waves with four steps in flight (N = 14432 18.7;
-// 8 waves 19.8, 16 waves 21.1).  Two requests at a time, not four, where 8 or 16 waves share the CU's memory pipeline (pair 20.3
-// against 23.2; at 16 rows K = 9216 16.2 against 19.6).  Only layers of a few tiles still split (f32 K = 3072, N = 768: 10.6 -> 9.1).
+// How a launch shares out the steps (words of codes) of a tile: waves per workgroup, requests of a wave, workgroups per tile.  Every layer
+// is one pass over its weights; what is left beside HBM's pace are a wave's waits for its answers (1 to 1.5 us each) and, with
+// several workgroups to a tile, their meeting (3 us).
+//   up to 8 rows     16 waves with two steps in flight while there is at most one tile per CU; beyond, 8 waves, two steps over tiles of 12
+//                    columns, four over tiles of 16 (8 rows, us: N = 6144 9.4, with 4 waves of four 9.7, 16 of one 10.2; N = 32768 34.8, 36.1, 33.8)
+//   9 to 16 rows     one step in flight: a step's 16 rows take more of the memory pipeline than its weights, and more requests only wait
+//                    for one another; 16 waves, 8 where several tiles of 12 columns share a CU (16 rows, us: K = 9216, N = 3072 14.6, 8
+//                    waves of three 16.5; pair of 9216 8 waves of one 22.1, of two 24.8, 16 of one 29.2; N = 32768 43.3, 8 of four 45.5;
+//                    f32 N = 50257 36.2 and 36.8)
+//   few tiles        split while the launch stays within one workgroup per CU and a wave keeps six steps (8 rows, us: f32 K = 3072, N = 768
+//                    8.5 -> 7.1, K = 12288 27.2 -> 12.1; bf16 K = 3072, N = 576, six steps already, 5.3, in two 5.7)
+//   codes            16 waves to a tile up to one tile per CU, else 8, one word in flight (a wave also has to convert it)
 // Weights are read past the caches (nontemporal): 4-5 % of a layer whose weights come from memory.  Models that the 256 MB last-level cache
 // holds gain or lose: whole f32 decode steps of 2 to 16 rows, against plain loads, take 0-15 % less with 16 MB of weights (5 % more at 2
 // rows), 2-9 % more with 100 to 180 MB (13 % at 16 rows of three layers of 1024), the same with 210, up to 5 % less with 240 to 270 and 1-7 %
 // less from 300 MB on.  None takes longer than with the four waves and the splits that ran here before; one rule for all.
-struct SkinnyPlan { int nw, ks; };
-static SkinnyPlan skinny_plan(int64_t steps, int64_t n, bool dual, bool codes) {
-    const int64_t tiles = cdiv_s(n, 16);
-    if (tiles <= 256) {
-        int ks = 1;
-        while (tiles * ks < 96 && steps / (32 * ks) >= 3) ks *= 2;
-        return {16, ks};
-    }
-    if (dual || codes || tiles < 768) return {8, 1};
-    return {4, 1};
+struct SkinnyPlan { int nw, depth, ks; };
+static SkinnyPlan skinny_plan(int64_t m, int64_t steps, int64_t n, bool codes) {
+    const int64_t cols = codes ? 16 : skinny_cols(n), tiles = cdiv_s(n, cols);
+    int ks = 1;
+    if (codes) while (tiles * ks < 96 && steps / (32 * ks) >= 3) ks *= 2;
+    else while (tiles * ks <= 128 && steps / (16 * ks) >= 12) ks *= 2;
+    if (codes) return {tiles <= 256 ? 16 : 8, 1, ks};
+    if (tiles <= 256) return {16, m > 8 ? 1 : 2, ks};
+    if (m > 8) return {cols == 12 ? 8 : 16, 1, 1};
+    return {8, cols == 12 ? 2 : 4, 1};
 }
-static size_t skinny_part_bytes(int64_t n, bool dual, int ks) { return ks > 1 ? (size_t)cdiv_s(n, 16) * ks * (dual ? 2 : 1) * 256 * sizeof(float) : 0; }
+static size_t skinny_part_bytes(int64_t n, bool dual, int cols, int ks) { return ks > 1 ? (size_t)cdiv_s(n, cols) * ks * (dual ? 2 : 1) * 256 * sizeof(float) : 0; }
 size_t skinny_workspace_bytes(int64_t k, int64_t n, bool dual) {
-    return skinny_part_bytes(n, dual, skinny_plan(k / 16, n, dual, false).ks);   // f32 has the most steps, so the most splits
+    // whichever of rows and codes splits more (f32 has the most steps), over the narrower tiles
+    return skinny_part_bytes(n, dual, 12, std::max(skinny_plan(1, k / 16, n, false).ks, skinny_plan(1, k / 64, n, true).ks));
 }
 bool skinny_quant_supported(int dtype, int64_t m, int64_t k, int64_t n, int qf) {
     if ((qf != 1 && qf != 2) || dtype != 2) return false;
@@ -442,9 +436,10 @@ void skinny_pack_codes(hipStream_t s, const void* codes, void* out, int64_t k, i
 void skinny_gemm(hipStream_t s, const SkinnyLinearArgs& a) {
     const bool dual = a.ws2 != nullptr;
     const int64_t steps = a.k / (a.quant == 1 ? 64 : a.quant == 2 ? 128 : a.dtype == 0 ? 16 : 32);
-    SkinnyPlan p = skinny_plan(steps, a.n, dual, a.quant != 0);
-    if (p.ks > 1 && (!a.part || !a.tickets || a.part_bytes < skinny_part_bytes(a.n, dual, p.ks))) p.ks = 1;
-    const dim3 grid((unsigned)cdiv_s(a.n, 16), (unsigned)p.ks);
+    const int cols = a.quant ? 16 : skinny_cols(a.n);
+    SkinnyPlan p = skinny_plan(a.m, steps, a.n, a.quant != 0);
+    if (p.ks > 1 && (!a.part || !a.tickets || a.part_bytes < skinny_part_bytes(a.n, dual, cols, p.ks))) p.ks = 1;
+    const dim3 grid((unsigned)cdiv_s(a.n, cols), (unsigned)p.ks);
     if (a.quant) {
 #define GPTRS_LAUNCH(QF, DUAL, NW)                                                                                          \
         skinny_gemm_quant_kernel<QF, DUAL, NW, 1><<<grid, 64 * NW, 0, s>>>((const bf16_t*)a.x, (const uint8_t*)a.ws, (const uint8_t*)a.ws2,  \
@@ -457,18 +452,32 @@ void skinny_gemm(hipStream_t s, const SkinnyLinearArgs& a) {
 #undef GPTRS_LAUNCH
         return;
     }
-#define GPTRS_LAUNCH(T, DUAL, NW, U)                                                                                        \
-    skinny_gemm_kernel<T, DUAL, NW, U><<<grid, 64 * NW, 0, s>>>((const T*)a.x, (const T*)a.ws, (const T*)a.ws2, (const T*)a.bias, \
-        (const T*)a.residual, (T*)a.y, (int)a.m, (int)a.k, (int)a.n, a.act, (float*)a.part, a.tickets, a.dtype == 2 ? a.out_f32 : 0, a.extra)
-    if (dual) {
-        if (a.dtype == 0) { if (p.nw == 16) GPTRS_LAUNCH(float, true, 16, 2); else GPTRS_LAUNCH(float, true, 8, 2); }
-        else { if (p.nw == 16) GPTRS_LAUNCH(bf16_t, true, 16, 2); else GPTRS_LAUNCH(bf16_t, true, 8, 2); }
-    } else if (a.dtype == 0) {
-        if (p.nw == 16) GPTRS_LAUNCH(float, false, 16, 2); else if (p.nw == 8) GPTRS_LAUNCH(float, false, 8, 2); else GPTRS_LAUNCH(float, false, 4, 4);
-    } else {
-        if (p.nw == 16) GPTRS_LAUNCH(bf16_t, false, 16, 2); else if (p.nw == 8) GPTRS_LAUNCH(bf16_t, false, 8, 2); else GPTRS_LAUNCH(bf16_t, false, 4, 4);
-    }
-#undef GPTRS_LAUNCH
+    auto go = [&](auto type, auto pair, auto nw, auto depth, auto columns) {
+        typedef decltype(type) T;
+        constexpr int NW = decltype(nw)::value;
+        skinny_gemm_kernel<T, decltype(pair)::value, NW, decltype(depth)::value, decltype(columns)::value><<<grid, 64 * NW, 0, s>>>(
+            (const T*)a.x, (const T*)a.ws, (const T*)a.ws2, (const T*)a.bias, (const T*)a.residual, (T*)a.y, (int)a.m, (int)a.k, (int)a.n, a.act,
+            (float*)a.part, a.tickets, a.dtype == 2 ? a.out_f32 : 0, a.extra);
+    };
+    auto shape = [&](auto type, auto pair) {
+        constexpr std::integral_constant<int, 1> I1{};
+        constexpr std::integral_constant<int, 2> I2{};
+        constexpr std::integral_constant<int, 4> I4{};
+        constexpr std::integral_constant<int, 8> I8{};
+        constexpr std::integral_constant<int, 12> I12{};
+        constexpr std::integral_constant<int, 16> I16{};
+        if (cols == 12) {
+            if (p.nw == 16) { if (p.depth == 1) go(type, pair, I16, I1, I12); else go(type, pair, I16, I2, I12); }
+            else { if (p.depth == 1) go(type, pair, I8, I1, I12); else go(type, pair, I8, I2, I12); }
+        } else {
+            if (p.depth == 1) go(type, pair, I16, I1, I16);
+            else if (p.nw == 16) go(type, pair, I16, I2, I16);
+            else go(type, pair, I8, I4, I16);
+        }
+    };
+    auto types = [&](auto pair) { if (a.dtype == 0) shape(float(), pair); else shape(bf16_t(), pair); };
+    if (dual) types(std::true_type{});
+    else types(std::false_type{});
 }
 
 }  // namespace k

@@ -214,7 +214,7 @@ class Backend {
     // src2 the SwiGLU pair (gate = src, up = src2) interleaved column by column in one copy.
     // Quantised weights: kind 3 / 4: chain copies of int8 / int4 codes (src2: the partner's codes); kind 5:
     // chain copy of int4 group scales (src2: the partner's); kind 6 / 7: k-grouped copy of the int8 / int4
-    // codes for the MFMA GEMM, which applies the scales itself; kind 8: 16-column tiled k-grouped copy for batched decode
+    // codes for the MFMA GEMM, which applies the scales itself; kind 8: k-grouped copy in tiles of 12 or 16 columns for batched decode
     // (kernels_skinny.hip); kind 9 / 10: int8 / int4 codes in that tile order; kind 11: chain copy of f32 weights.
     BufferP derived_weights(const BufferP& src, int kind, DType dtype, int64_t k, int64_t n, const BufferP& src2 = nullptr);
     void drop_derived_weights();

@@ -1,5 +1,5 @@
 """Linear layers of 2 to 16 rows (kernels_skinny.hip) at the edges of their launch rule: layers of at most 256 column tiles, of up to
-768 and beyond; few tiles, whose steps are split over workgroups; steps that do not divide among the waves, and fewer steps than
+768 and beyond; tiles of 12 and of 16 columns, 8 rows and more; few tiles, whose steps are split over workgroups; steps that do not divide among the waves, and fewer steps than
 waves.  Rows against float64 sums of the same values, codes against the dequantised matrix."""
 import numpy as np
 import pytest
@@ -19,7 +19,9 @@ def bounds(x, w, dtype):
     return s, 2 * np.sqrt(x.shape[1]) * 2.0 ** -24 * mags + (2.0 ** -8 if dtype == "Bf16" else 2.0 ** -23) * np.abs(s) + 1e-6
 
 
-SIZES = [(2, 32, 16), (3, 96, 130), (7, 3072, 40), (16, 1568, 700), (8, 9216, 304), (5, 288, 4096), (16, 544, 4112), (9, 160, 12272), (4, 192, 12304)]
+SIZES = [(2, 32, 16), (3, 96, 130), (7, 3072, 40), (16, 1568, 700), (8, 9216, 304), (5, 288, 4096), (16, 544, 4112), (9, 160, 12272), (4, 192, 12304),
+         # tiles of 12 columns: one to a CU, a last tile of 4, two to a CU; splits of 12 steps and more
+         (8, 96, 3072), (9, 64, 3064), (16, 224, 6144), (3, 352, 4108), (2, 12288, 36)]
 
 
 @pytest.mark.parametrize("dtype", ["Bf16", "F32"])
