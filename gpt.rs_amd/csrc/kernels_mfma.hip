@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const T* __restrict__ x,
 //
 // Workgroup: WM x WN waves; a wave owns (32 TM) x (32 TN) outputs as TM x TN fragments of 32 x 32, the tile is
 // BM x BN = (32 TM WM) x (32 TN WN).  KW = 2: two such groups of waves share the staged tiles, each multiplies half of every k tile, and
-// their sums meet through LDS in front of the epilogue.  A bf16 launch takes one of seven tiles and a number of splits over k, see tile_plan().
+// their sums meet through LDS in front of the epilogue.  A bf16 launch takes one of eight tiles and a number of splits over k, see tile_plan().
 //
 // What bounds it (bf16).  256 x 256 tiles, all CUs busy: the matrix pipes at the clock that random operands allow.  A tile's 32 k
 // take 0.54 us on a quarter of the CUs and 0.8 us on all of them; over all-zero operands the same launch runs at 1.35 times
@@ -1256,7 +1256,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
 }
 
 // The tiles, in the order of tile_cost's table.
-enum TileId { kT256x256, kT256x192, kT128x256, kT128x192, kT128x128, kT64x256, kT64x128, kTiles };
+enum TileId { kT256x256, kT256x192, kT192x192, kT128x256, kT128x192, kT128x128, kT64x256, kT64x128, kTiles };
 struct TilePlan { int tile; int splits; };
 constexpr int kTileLds = 160 * 1024;   // LDS of one CU
 
@@ -1300,9 +1300,13 @@ static bool splits_allowed() {
 // a pair of 9216; weights from memory): rounds of workgroups x (fixed + per k tile of 64) + what a k tile costs more with the
 // chip full, and for a split the second launch plus its bytes.  Over 158 shapes (M = 20 .. 8188 of those layers and of K = 768 .. 6144,
 // N = 512 .. 14432) what it picks is 3.0 % slower than the best measured choice in the mean (4.8 % without the 128 x 192 tiles).
+// 192 x 192 (4 waves of 96 x 96, plain layers) is for one round of long sums that the 256-wide tiles leave a quarter of the CUs out of: M = 3064,
+// N = 3072 is 256 of them, 192 of 256 x 192.  us, against the best of the others: K = 9216 157 and 178 (M = 2900 155 and 161), K = 6144 107 and
+// 117; below 80 k tiles its long start and way out cost what it gains (K = 4096 72 and 70), and in two rounds 128 x 192 is better
+// (M = 5500, K = 9216 296 and 278).
 struct TileCost { int bm, bn, slots; double fixed, per_kt, full_kt, split, split_mb; };
 static const TileCost kTileCost[kTiles] = {
-    {256, 256, 256, 5.45, 1.237, 0.379, 2.8, 0.30}, {256, 192, 256, 1.16, 1.206, 0.122, 4.7, 0.35}, {128, 256, 256, 6.87, 0.661, 0.171, 3.1, 0.26}, {128, 192, 256, 7.9, 0.48, 0.266, 5.1, 0.10},
+    {256, 256, 256, 5.45, 1.237, 0.379, 2.8, 0.30}, {256, 192, 256, 1.16, 1.206, 0.122, 4.7, 0.35}, {192, 192, 256, 12.0, 0.86, 0.14, 0.0, 0.0}, {128, 256, 256, 6.87, 0.661, 0.171, 3.1, 0.26}, {128, 192, 256, 7.9, 0.48, 0.266, 5.1, 0.10},
     {128, 128, 256, 4.48, 0.425, 0.055, 3.9, 0.31}, {64, 256, 256, 4.59, 0.572, 0.0, 5.4, 0.13}, {64, 128, 512, 2.58, 0.361, 0.143, 5.0, 0.34},
 };
 static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
@@ -1310,10 +1314,11 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t roo
     double least = 1e300;
     for (int t = 0; t < kTiles; ++t) {
         const TileCost& c = kTileCost[t];
-        if (dual && t == kT256x192) continue;   // a wave's three fragments do not divide between the matrices
+        if (dual && (t == kT256x192 || t == kT192x192)) continue;   // a wave's three fragments do not divide between the matrices
         const int64_t tiles = cdiv(m, c.bm) * cdiv(n, dual ? c.bn / 2 : c.bn);
+        if (t == kT192x192 && (tiles > c.slots || k < 80 * 64)) continue;
         for (int sp : {1, 2, 3, 4, 6, 8}) {
-            if (sp > 1 && (!splits_allowed() || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+            if (sp > 1 && (!splits_allowed() || t == kT192x192 || k < 256 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
             const double kt = (double)k / 64 / sp, wg = (double)(tiles * sp);
             double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
             if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
@@ -1328,6 +1333,7 @@ static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p)
     switch (p.tile) {
         case kT256x256: return launch_tile<T, 4, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits);
         case kT256x192: if constexpr (!DUAL) return launch_tile<T, 8, 2, 4, 2, 2, 3, false>(s, a, p.splits); else return;
+        case kT192x192: if constexpr (!DUAL) return launch_tile<T, 8, 3, 2, 2, 3, 3, false>(s, a, p.splits); else return;
         case kT128x256: return launch_tile<T, 8, 3, 2, 4, 2, 2, DUAL>(s, a, p.splits);
         case kT128x192: return launch_tile<T, 8, 3, 2, 2, 2, 3, DUAL, 0, 2>(s, a, p.splits);
         case kT128x128:

@@ -24,6 +24,8 @@ def program(specs, body):
 # k tile, fewer k tiles than the ring holds, k that does not divide among the splits; the layer sizes on each tile and split
 @pytest.mark.parametrize("m,k,n", [(17, 64, 8), (33, 128, 41), (64, 192, 130), (65, 3072, 1000), (127, 4096, 3072), (129, 1088, 3075), (200, 9216, 1536),
                                    (255, 3072, 6144), (257, 320, 520), (333, 3072, 6176), (513, 2048, 4100), (1000, 9216, 768), (1025, 448, 9216), (2049, 256, 3008),
+                                   # 192 x 192 tiles: one round, ragged rows and columns, k tiles that divide by the ring and that do not
+                                   (2881, 9216, 2900), (2753, 5120, 3050), (3072, 5184, 3072),
                                    # 128 x 192 tiles, whole and in 2, 4 and 8 splits, then for the pair whole and in 2, 3 and 4: ragged rows and columns
                                    (1227, 1536, 3985), (913, 9216, 2673), (230, 9216, 5883), (2025, 9216, 368), (687, 3072, 3335), (615, 9216, 1602)])
 def test_tiles_and_splits(hip, m, k, n):
@@ -230,3 +232,4 @@ def test_pair_is_the_decode_steps_function(hip, kind, m, k):
         rows = x[r:r + 16] if r + 16 <= m else x[m - 16:]
         first = r if r + 16 <= m else m - 16
         assert np.array_equal(got[first:first + 16], run(rows)), first
+
