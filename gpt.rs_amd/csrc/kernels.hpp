@@ -291,6 +291,9 @@ struct MfmaLinearArgs {
     int out_f32 = 0;   // bf16 only: y and residual are f32
     EpiExtra extra;    // unquantised only
     int lds_direct = 1;   // the LDS-direct kernel where it applies (0: the register-staged one)
+    // an RMS norm of the f32 result, rounded to bf16, wanted next: the launch that adds the splits of a tile writes it along with y where it can,
+    // and says so in *normed
+    const void* norm_gamma = nullptr; void* norm_y = nullptr; float norm_inv_n = 0.f, norm_eps = 0.f; bool* normed = nullptr;
 };
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant);
 size_t mfma_weight_bytes(int dtype, int64_t k, int64_t n);

@@ -772,14 +772,26 @@ void Builder::build() {
     for (int v = 0; v < nv; ++v)
         if (plan.values[v].defined && plan.values[v].root == v && def_step[v] >= 0 && plan.storage[v].kind == Storage::Temp)
             dying[std::max(last_use[v], def_step[v])].push_back(v);
+    // prefill linears whose f32 result goes into an RMS norm with the next step (Step::norm_next)
+    for (int s = 0; s + 1 < n_steps; ++s) {
+        Step& st = plan.steps[s];
+        const Step& nx = plan.steps[s + 1];
+        st.norm_next = st.in.op == OpKind::FLinear && st.in.mfma && st.in.out_f32 && st.dst.size() == 1 && nx.in.op == OpKind::FRmsNorm && nx.src[0] >= 0 &&
+                       root(nx.src[0]) == st.dst[0] && nx.in.out_specs[0].dtype == DType::BF16 && nx.dst.size() == 1 &&
+                       plan.values[nx.src[0]].spec.dims.back() == plan.values[st.dst[0]].spec.dims.back();
+    }
     for (int s = 0; s < n_steps; ++s) {
         Step& st = plan.steps[s];
-        for (int v : st.dst) {
-            RootStorage& rs = plan.storage[v];
-            if (rs.kind != Storage::Temp) continue;
-            rs.bytes = std::max<size_t>(plan.values[v].spec.bytes(), 1);
-            rs.offset = ws_alloc(rs.bytes);
-        }
+        auto place = [&](const Step& of) {
+            for (int v : of.dst) {
+                RootStorage& rs = plan.storage[v];
+                if (rs.kind != Storage::Temp) continue;
+                rs.bytes = std::max<size_t>(plan.values[v].spec.bytes(), 1);
+                rs.offset = ws_alloc(rs.bytes);
+            }
+        };
+        if (s == 0 || !plan.steps[s - 1].norm_next) place(st);
+        if (st.norm_next) place(plan.steps[s + 1]);   // beside everything that this step still reads
         if (st.scratch_bytes) {
             st.scratch_off = ws_alloc(st.scratch_bytes);
             ws_free(st.scratch_off, st.scratch_bytes);
@@ -1010,6 +1022,7 @@ static bool run_chain(const Plan& plan, const Step& head, ExecCtx& cx) {
 }
 
 void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
+    if (cx.done_ahead == &st) { cx.done_ahead = nullptr; return; }
     const Instr& in = st.in;
     const Spec& out = in.out_specs[0];
     void* dst = cx.ptr[st.dst[0]];
@@ -1181,6 +1194,14 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
                     ma.part_bytes = st.scratch_bytes;
                     ma.tickets = cx.be->skinny_tickets();
                 }
+                bool normed = false;
+                if (st.norm_next && in.softcap == 0.f) {
+                    const Step& nx = (&st)[1];   // (steps are in order; norm_next says that there is one)
+                    ma.norm_gamma = src_ptr(nx, cx, 1);
+                    ma.norm_y = cx.ptr[nx.dst[0]];
+                    ma.norm_inv_n = nx.in.scale; ma.norm_eps = nx.in.eps;
+                    ma.normed = &normed;
+                }
                 hipEvent_t e0 = nullptr, e1 = nullptr;
                 if (cx.profile) {
                     GPTRS_HIP_CHECK(hipEventCreate(&e0));
@@ -1188,6 +1209,7 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
                     GPTRS_HIP_CHECK(hipEventRecord(e0, s));
                 }
                 k::mfma_gemm(s, ma);
+                if (normed) cx.done_ahead = &st + 1;
                 if (in.softcap != 0.f) { k::softcap(s, (const float*)dst, (float*)dst, out.count(), in.softcap); ++cx.launches; }
                 if (cx.profile) {
                     GPTRS_HIP_CHECK(hipEventRecord(e1, s));

@@ -120,6 +120,9 @@ struct Step {
     // first step of the run carries its length, the others are marked as members.
     int chain_len = 0;
     bool chain_member = false;
+    // Prefill linear: the next step is an RMS norm of its f32 result, which the launch that adds its splits may do; the norm's result is then
+    // given its storage together with this step's own.
+    bool norm_next = false;
     k::CopyDesc pack_l{}, pack_r{};
     size_t pack_l_off = 0, pack_r_off = 0;
 };
@@ -361,6 +364,7 @@ struct ExecCtx {
     bool profile = false;
     bool chain = false;               // run decode linears as persistent chain launches
     std::vector<BufferP> input_bufs;  // per input position
+    const Step* done_ahead = nullptr; // a step whose work the step before it has done
 };
 void run_step(const Plan& plan, const Step& st, ExecCtx& cx);
 

@@ -233,3 +233,36 @@ def test_pair_is_the_decode_steps_function(hip, kind, m, k):
         first = r if r + 16 <= m else m - 16
         assert np.array_equal(got[first:first + 16], run(rows)), first
 
+
+# the launch that adds a layer's splits takes the RMS norm behind it along: the same bits as the norm by itself, with every value of the
+# program between its ends in reused memory; widths under and over a thread's 8 values, 64, 256 and 512 threads; more rows than splits are made for
+@pytest.mark.parametrize("m,k,n", [(17, 1088, 264), (64, 9216, 3072), (129, 4096, 4160), (333, 9216, 3072), (333, 9216, 3084), (40, 2048, 8192), (40, 2048, 8200), (2100, 512, 3072)])
+def test_norm_behind_splits(hip, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    x, w = bf16(rng.standard_normal((m, k), dtype=np.float32)), bf16(rng.standard_normal((k, n), dtype=np.float32) * np.float32(k ** -0.5))
+    w2 = bf16(rng.standard_normal((n, 256), dtype=np.float32) * np.float32(n ** -0.5))
+    res, gain = rng.standard_normal((m, n), dtype=np.float32), 1 + rng.standard_normal(n, dtype=np.float32) / 8
+    rows, mat, f32, vec = ("Bf16", [m, k]), ("Bf16", [k, n]), ("F32", [m, n]), ("F32", [n])
+
+    def norm(y, g):
+        return F.rms_norm(y, g, 1e-5)[0].cast("Bf16")
+
+    def block(a, b, r, g, c):
+        y = F.linear(a, b, out_dtype="F32") + r
+        return [F.linear(norm(y, g), c), y]
+
+    layer = program([rows, mat, f32], lambda a, b, r: [F.linear(a, b, out_dtype="F32") + r])
+    alone = program([f32, vec], lambda y, g: [norm(y, g)])
+    head = program([("Bf16", [m, n]), ("Bf16", [n, 256])], lambda a, b: [F.linear(a, b)])
+    both = program([rows, mat, f32, vec], lambda a, b, r, g: (lambda y: [norm(y, g), y])(F.linear(a, b, out_dtype="F32") + r))
+    whole = program([rows, mat, f32, vec, ("Bf16", [n, 256])], block)
+    no_res = program([rows, mat, vec], lambda a, b, g: [norm(F.linear(a, b, out_dtype="F32"), g)])
+    y = hip_run(hip, layer, [x, w, res])[0]
+    z = hip_run(hip, alone, [y, gain])[0]
+    for _ in range(2):
+        got = hip_run(hip, both, [x, w, res, gain])
+        assert np.array_equal(got[1], y) and np.array_equal(got[0], z)
+        got = hip_run(hip, whole, [x, w, res, gain, w2])
+        assert np.array_equal(got[1], y) and np.array_equal(got[0], hip_run(hip, head, [z, w2])[0])
+    plain = hip_run(hip, program([rows, mat], lambda a, b: [F.linear(a, b, out_dtype="F32")]), [x, w])[0]
+    assert np.array_equal(hip_run(hip, no_res, [x, w, gain])[0], hip_run(hip, alone, [plain, gain])[0])
