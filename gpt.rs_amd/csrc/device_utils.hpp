@@ -187,21 +187,27 @@ __device__ __forceinline__ float block_max(float v, float* smem16) {
 // The tile of a workgroup of a prompt's attention, grid (row tiles, heads, sequences).  Workgroups go to the 8 XCDs in turn, so
 // with the plain indices every XCD reads the keys and values of every head through its own 4 MiB of L2 (4 sequences of 2047 rows of
 // 8 kv heads of 128: 8 MiB at a time).  Here an XCD takes an eighth of the heads of each sequence (heads that share keys lie side by
-// side), all of their row tiles in turn, or, where the heads do not divide, an eighth of the pairs of head and sequence.  Those
-// prompts 313 -> 236 us per layer; latent attention of 4 sequences, 3064 rows, 32 heads 136 -> 94; chunked of 3000 rows, 32 heads,
-// 126 -> 116.
+// side), or, where the heads do not divide, an eighth of the pairs of head and sequence.  Those prompts 313 -> 236 us per layer;
+// latent attention of 4 sequences, 3064 rows, 32 heads 136 -> 94; chunked of 3000 rows, 32 heads, 126 -> 116.
+// Within an XCD all pairs of head and sequence come before the next row tile: a row tile is as long as the keys it sees, the tiles that
+// see most go first, and the short ones fill up behind them.  With a pair's row tiles in a row, workgroup i and i + 32 of an XCD, which
+// land on one CU, were tiles of one length wherever the number of row tiles divides 32, so some CUs had the long ones only.  us a layer,
+// before and after: f32, 12 heads of 64, 16 x 512 rows 126 -> 103, 16 x 1000 380 -> 264, 8 x 900 193 -> 150; bf16, 32 / 8 heads of 128, 4 x 2047
+// 226 -> 218, 8 x 1000 146 -> 135, 3 x 500 38.6 -> 34.9; one sequence as before.
 struct XcdTile { unsigned x, y, z; };
 __device__ __forceinline__ XcdTile xcd_tile() {
     const unsigned gx = gridDim.x, gy = gridDim.y, lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), xcd = lin & 7, slot = lin >> 3;
     if (gy % 8 == 0) {
-        const unsigned per = gy / 8, r = slot / per;
-        return {r % gx, xcd * per + slot % per, r / gx};
+        const unsigned per = gy / 8, pairs = per * gridDim.z, p = slot % pairs;
+        return {slot / pairs, xcd * per + p % per, p / per};
     }
-    if (gy * gridDim.z % 8 == 0) {
-        const unsigned pair = xcd + 8 * (slot / gx);
-        return {slot % gx, pair % gy, pair / gy};
+    const unsigned all = gy * gridDim.z;
+    if (all % 8 == 0) {
+        const unsigned pairs = all / 8, pair = xcd + 8 * (slot % pairs);
+        return {slot / pairs, pair % gy, pair / gy};
     }
-    return {blockIdx.x, blockIdx.y, blockIdx.z};
+    const unsigned pair = lin % all;
+    return {lin / all, pair % gy, pair / gy};
 }
 
 }  // namespace k
