@@ -694,6 +694,22 @@ __global__ __launch_bounds__(256) void attn_prefill_kv_kernel(const T* __restric
     *reinterpret_cast<vec_t*>(to) = x;
 }
 
+// Prompts of one row tile (at most 32 rows where 4 query heads share keys, 128 where one has them alone): the one workgroup of a kv head that sees all
+// of its keys puts them into the caches itself, on their way to LDS, and the launch of attn_prefill_kv_kernel is saved.  One 16-byte chunk of
+// a K row, rotated as that kernel does it; T: element, `second`: the chunk lies in the rotated half that adds.
+template <typename T, typename V>
+__device__ __forceinline__ V rotated_chunk(const V& own, const V& other, const V& c, const V& s, bool second) {
+    constexpr int VEC = 16 / sizeof(T);
+    alignas(16) T x[VEC], y[VEC], cv[VEC], sv[VEC];
+    *reinterpret_cast<V*>(x) = own; *reinterpret_cast<V*>(y) = other; *reinterpret_cast<V*>(cv) = c; *reinterpret_cast<V*>(sv) = s;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        const float xf = ldf(x, e), yf = ldf(y, e), cf = ldf(cv, e), sf = ldf(sv, e);
+        stf(x, e, second ? xf * cf + yf * sf : xf * cf - yf * sf);
+    }
+    return *reinterpret_cast<const V*>(x);
+}
+
 // ------------------------------------------------------------------------------ prefill
 // grid (ceil(T/4), n_q), 256 threads: one wave per query row.  Keys are visited 64 at a time
 // (one per lane) with an online softmax; the P.V update then walks the chunk with the lanes
@@ -764,7 +780,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const T* __restrict__
 // 2 s + g (it stages them itself, into its own LDS buffers), and the two online-softmax states meet through LDS at the
 // end.  A row tile then takes half as many steps, and a SIMD holds two waves whose matrix and vector phases overlap
 // (the launch has one wave-sized task per SIMD otherwise).
-template <int DH, int KG>
+template <int DH, int KG, bool FILL>
 __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ ctx, int T,
                                                                 int n_q, int n_kv, float scale_log2e, int zgroups, PrefillKv<bf16_t> kv) {
     constexpr int KT = 32;            // keys per tile
@@ -809,6 +825,8 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
     int64_t kpitch;
     const auto* kp = prefill_rows(kv.k, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + kvh) * DH, kpitch);
     const auto* vp = prefill_rows(kv.v, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + n_kv + kvh) * DH, kpitch);
+    bf16_t *kout = const_cast<bf16_t*>(kp), *vout = const_cast<bf16_t*>(vp);   // FILL: the caches' rows
+    if (FILL) { kp = qkv + (int64_t)(n_q + kvh) * DH; vp = qkv + (int64_t)(n_q + n_kv + kvh) * DH; kpitch = P; }
     const int kend = min(T, (bx * rtpb + rtpb) * 32);   // keys any row of the workgroup may see
     const int ntiles = (kend + KT - 1) / KT;
     const bool active = q0 < T;
@@ -845,7 +863,7 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
     // native vectors and unconditional loads (the chunk index is clamped instead): with HIP's uint4 struct and a
     // guarded load the compiler keeps these in scratch memory and waits for every load right where it is issued
     typedef uint32_t u32x4_s __attribute__((ext_vector_type(4)));
-    u32x4_s kreg[CPT], vreg[CPT];
+    u32x4_s kreg[CPT], vreg[CPT], kother[FILL ? CPT : 1], kcos[FILL ? CPT : 1], ksin[FILL ? CPT : 1];
     auto gload = [&](int t) {
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
@@ -854,14 +872,27 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
             const int64_t key = min(t * KT + r, T - 1);
             kreg[j] = *reinterpret_cast<const u32x4_s*>(kp + key * kpitch + ch * 8);
             vreg[j] = *reinterpret_cast<const u32x4_s*>(vp + key * kpitch + ch * 8);
+            if (FILL && kv.cos) {
+                const int first = ch % (DH / 16);
+                kother[FILL ? j : 0] = *reinterpret_cast<const u32x4_s*>(kp + key * kpitch + (ch < DH / 16 ? ch + DH / 16 : first) * 8);
+                kcos[FILL ? j : 0] = *reinterpret_cast<const u32x4_s*>(kv.cos + key * (DH / 2) + first * 8);
+                ksin[FILL ? j : 0] = *reinterpret_cast<const u32x4_s*>(kv.sin + key * (DH / 2) + first * 8);
+            }
         }
     };
-    auto lwrite = [&](int buf) {
+    auto lwrite = [&](int buf, int t) {
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
             const int c = tid + 256 * j;
             if (CH % 256 == 0 || c < CH) {
                 const int r = c / (DH / 8), ch = c % (DH / 8);
+                if (FILL) {
+                    if (kv.cos) kreg[j] = rotated_chunk<bf16_t>(kreg[j], kother[FILL ? j : 0], kcos[FILL ? j : 0], ksin[FILL ? j : 0], ch >= DH / 16);
+                    if (zg == 0 && t * KT + r < T) {
+                        *reinterpret_cast<u32x4_s*>(kout + (int64_t)(t * KT + r) * DH + ch * 8) = kreg[j];
+                        *reinterpret_cast<u32x4_s*>(vout + (int64_t)(t * KT + r) * DH + ch * 8) = vreg[j];
+                    }
+                }
                 *reinterpret_cast<u32x4_s*>(&ksm[buf][r * KS + ch * 8]) = kreg[j];
                 // key r goes to k-slot position p: bits 2 and 3 of r swapped
                 const int pos = (r & 0x13) | ((r & 4) << 1) | ((r & 8) >> 1);
@@ -876,7 +907,7 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
 
     // group kg visits tiles kg, kg + KG, ...; the step count is uniform over the workgroup (barriers)
     const int nsteps = (ntiles + KG - 1) / KG;
-    if (kg < ntiles) { gload(kg); lwrite(0); }
+    if (kg < ntiles) { gload(kg); lwrite(0, kg); }
     // The Q fragments are used here, once, so that they have arrived on EVERY path into the step loop.  A workgroup whose
     // group has no first tile skips the wait above; the compiler then assumes the eight Q loads may still be in flight at
     // the loop's head and puts `s_waitcnt vmcnt(7) .. vmcnt(0)` in front of the eight score MFMAs of every step, which in
@@ -947,7 +978,7 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
                 }
             }
         }
-        if (t + KG < ntiles) lwrite(buf ^ 1);
+        if (t + KG < ntiles) lwrite(buf ^ 1, t + KG);
         __syncthreads();
     }
     if (KG == 2) {
@@ -1001,7 +1032,7 @@ __device__ __forceinline__ f32x16_v mma_f32x4(const f32x4_v& a, const f32x4_v& b
     return c;
 }
 
-template <int DH>
+template <int DH, bool FILL>
 __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const float* __restrict__ qkv, float* __restrict__ ctx, int T,
                                                                     int n_q, int n_kv, float scale_log2e, int zgroups, PrefillKv<float> kv) {
     constexpr int KT = 32;            // keys per tile
@@ -1033,6 +1064,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
     int64_t kpitch;
     const auto* kp = prefill_rows(kv.k, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + kvh) * DH, kpitch);
     const auto* vp = prefill_rows(kv.v, kv, qkv, seq, kvh, DH, T, P, (int64_t)(n_q + n_kv + kvh) * DH, kpitch);
+    float *kout = const_cast<float*>(kp), *vout = const_cast<float*>(vp);   // FILL: the caches' rows
+    if (FILL) { kp = qkv + (int64_t)(n_q + kvh) * DH; vp = qkv + (int64_t)(n_q + n_kv + kvh) * DH; kpitch = P; }
     const int kend = min(T, (bx * rtpb + rtpb) * 32);
     const int ntiles = (kend + KT - 1) / KT;
     const bool active = q0 < T;
@@ -1065,7 +1098,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
         for (int v = 0; v < 16; ++v) acc_o[db][v] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;
 
-    f32x4_v kreg[CPT], vreg[CPT];
+    f32x4_v kreg[CPT], vreg[CPT], kother[FILL ? CPT : 1], kcos[FILL ? CPT : 1], ksin[FILL ? CPT : 1];
     auto gload = [&](int t) {
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
@@ -1074,14 +1107,27 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
             const int64_t key = min(t * KT + r, T - 1);
             kreg[j] = *reinterpret_cast<const f32x4_v*>(kp + key * kpitch + ch * 4);
             vreg[j] = *reinterpret_cast<const f32x4_v*>(vp + key * kpitch + ch * 4);
+            if (FILL && kv.cos) {
+                const int first = ch % (DH / 8);
+                kother[FILL ? j : 0] = *reinterpret_cast<const f32x4_v*>(kp + key * kpitch + (ch < DH / 8 ? ch + DH / 8 : first) * 4);
+                kcos[FILL ? j : 0] = *reinterpret_cast<const f32x4_v*>(kv.cos + key * (DH / 2) + first * 4);
+                ksin[FILL ? j : 0] = *reinterpret_cast<const f32x4_v*>(kv.sin + key * (DH / 2) + first * 4);
+            }
         }
     };
-    auto lwrite = [&](int buf) {
+    auto lwrite = [&](int buf, int t) {
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
             const int c = tid + 256 * j;
             if (CH % 256 == 0 || c < CH) {
                 const int r = c / (DH / 4), ch = c % (DH / 4);
+                if (FILL) {
+                    if (kv.cos) kreg[j] = rotated_chunk<float>(kreg[j], kother[FILL ? j : 0], kcos[FILL ? j : 0], ksin[FILL ? j : 0], ch >= DH / 8);
+                    if (zg == 0 && t * KT + r < T) {
+                        *reinterpret_cast<f32x4_v*>(kout + (int64_t)(t * KT + r) * DH + ch * 4) = kreg[j];
+                        *reinterpret_cast<f32x4_v*>(vout + (int64_t)(t * KT + r) * DH + ch * 4) = vreg[j];
+                    }
+                }
                 *reinterpret_cast<f32x4_v*>(&ksm[buf][r * KS + ch * 4]) = kreg[j];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) vsm[buf][(ch * 4 + e) * VS + 4 * (ch & 7) + r] = vreg[j][e];
@@ -1090,7 +1136,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
     };
 
     gload(0);
-    lwrite(0);
+    lwrite(0, 0);
     // the Q fragments have arrived before the step loop on every path (see attn_prefill_mfma_kernel)
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk) asm volatile("" : : "v"(qf[kk]));
@@ -1150,7 +1196,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_f32_kernel(const flo
                 }
             }
         }
-        if (t + 1 < ntiles) lwrite(buf ^ 1);
+        if (t + 1 < ntiles) lwrite(buf ^ 1, t + 1);
         __syncthreads();
     }
     if (active && q0 + col < T) {
@@ -1185,34 +1231,36 @@ static int attn_prefill_mfma(hipStream_t s, const AttnPrefillArgs& a) {
     kv.starts = a.starts;
     kv.capacity = a.capacity;
     if (a.rot_half) { kv.cos = (const T*)a.cos; kv.sin = (const T*)a.sin; }
+    const int g = (int)(a.n_q / a.n_kv), gw = g >= 4 ? 4 : g, zg = g >= 4 ? g / 4 : 1;
+    const dim3 grid((unsigned)cdiv(cdiv(a.t, 32), 4 / gw), (unsigned)a.n_kv, (unsigned)(zg * a.batch));
+    const float sl = a.scale * 1.44269504088896f;
+    // two key groups per workgroup once the launch is smaller than three workgroups per CU and rows are long
+    // enough to split (bf16)
+    static const bool allow_kg = [] { const char* e = getenv("GPTRS_HIP_ATTN_KEYGROUPS"); return !(e && e[0] == '0'); }();
+    const bool kg2 = std::is_same<T, bf16_t>::value && allow_kg && a.t >= 128 && (int64_t)grid.x * grid.y * grid.z < 768;
+    // one row tile: the attention fills the caches itself (us: 7 rows, 12 heads of 64 in f32 8.9 -> 6.4, 16 x 100 rows 22.7 -> 17.9; 20 rows, 32 / 8 heads of 128 in bf16 11.5 -> 9.4)
+    const bool fill = a.starts && grid.x == 1 && !kg2;
     int launches = 1;
-    if (a.starts) {
+    if (a.starts && !fill) {
         const int64_t chunks = a.batch * a.t * 2 * a.n_kv * a.head_dim / (16 / (int64_t)sizeof(T));
         attn_prefill_kv_kernel<T><<<(unsigned)cdiv(chunks, 256), 256, 0, s>>>((const T*)a.qkv, chunks, (int)a.t, (int)a.n_q, (int)a.n_kv, (int)a.head_dim, kv);
         ++launches;
     }
-    const int g = (int)(a.n_q / a.n_kv), gw = g >= 4 ? 4 : g, zg = g >= 4 ? g / 4 : 1;
-    const dim3 grid((unsigned)cdiv(cdiv(a.t, 32), 4 / gw), (unsigned)a.n_kv, (unsigned)(zg * a.batch));
-    const float sl = a.scale * 1.44269504088896f;
-    if constexpr (std::is_same<T, float>::value) {
-        auto go = [&](auto dh) { attn_prefill_mfma_f32_kernel<decltype(dh)::value><<<grid, 256, 0, s>>>((const float*)a.qkv, (float*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv); };
-        if (a.head_dim == 32) go(std::integral_constant<int, 32>{});
-        else if (a.head_dim == 64) go(std::integral_constant<int, 64>{});
-        else go(std::integral_constant<int, 128>{});
-    } else {
-        // two key groups per workgroup once the launch is smaller than three workgroups per CU and rows are long
-        // enough to split
-        static const bool allow_kg = [] { const char* e = getenv("GPTRS_HIP_ATTN_KEYGROUPS"); return !(e && e[0] == '0'); }();
-        const bool kg2 = allow_kg && a.t >= 128 && (int64_t)grid.x * grid.y * grid.z < 768;
-        auto go = [&](auto dh) {
-            constexpr int D = decltype(dh)::value;
-            if (kg2) attn_prefill_mfma_kernel<D, 2><<<grid, 512, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv);
-            else attn_prefill_mfma_kernel<D, 1><<<grid, 256, 0, s>>>((const bf16_t*)a.qkv, (bf16_t*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv);
-        };
-        if (a.head_dim == 32) go(std::integral_constant<int, 32>{});
-        else if (a.head_dim == 64) go(std::integral_constant<int, 64>{});
-        else go(std::integral_constant<int, 128>{});
-    }
+    auto go = [&](auto dh) {
+        constexpr int D = decltype(dh)::value;
+        auto launch = [&](auto kernel, int threads) { kernel<<<grid, threads, 0, s>>>((const T*)a.qkv, (T*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv); };
+        if constexpr (std::is_same<T, float>::value) {
+            if (fill) launch(attn_prefill_mfma_f32_kernel<D, true>, 256);
+            else launch(attn_prefill_mfma_f32_kernel<D, false>, 256);
+        } else {
+            if (kg2) launch(attn_prefill_mfma_kernel<D, 2, false>, 512);
+            else if (fill) launch(attn_prefill_mfma_kernel<D, 1, true>, 256);
+            else launch(attn_prefill_mfma_kernel<D, 1, false>, 256);
+        }
+    };
+    if (a.head_dim == 32) go(std::integral_constant<int, 32>{});
+    else if (a.head_dim == 64) go(std::integral_constant<int, 64>{});
+    else go(std::integral_constant<int, 128>{});
     return launches;
 }
 

@@ -11,6 +11,8 @@ from gptrs_amd.ptir import FunctionBuilder, Program, Tensor, bf16_bits_to_f32, f
 CASES = [  # sequences, rows, query heads, key heads, head size, rotated, cache rows, first row that the update names
     (1, 2, 2, 2, 32, True, 2, 0), (1, 33, 4, 1, 32, True, 64, 5), (2, 32, 2, 2, 64, False, 32, 0), (3, 31, 8, 2, 64, True, 40, 100),
     (16, 3, 4, 4, 32, False, 8, -2), (2, 129, 8, 1, 128, True, 160, 7), (1, 200, 4, 2, 128, False, 256, 0), (2, 65, 6, 3, 64, True, 65, 0),
+    # one row tile, whose workgroups fill the caches: 32, 64 and 128 rows by query heads to a key head, two workgroups to a key head, and one row more
+    (2, 32, 8, 1, 128, True, 33, 1), (1, 64, 4, 2, 128, True, 64, 0), (2, 128, 2, 2, 64, False, 130, 2), (1, 127, 2, 2, 32, True, 128, 0), (1, 65, 4, 2, 64, False, 70, 3),
     (3, 5, 3, 1, 32, False, 6, 1),     # three query heads to a key head: the unfused series
 ]
 
