@@ -466,7 +466,10 @@ void Backend::param_set(const std::array<uint8_t, 16>& id, gptrs_hip_tensor* t) 
     }
 }
 
-bool Backend::queue_sampling(const gptrs_hip_tensor* logits, float temperature, bool has_top_k, bool has_u, float u) {
+k::ArgmaxScratch Backend::argmax_scratch() const { return {d_argmax_val_, d_argmax_idx_, 1024, skinny_tickets(), (const int64_t*)d_err_flag_}; }
+
+// Queues the sampling of a token and its way into `host`, a pinned slot: [0] the token, [1] the device's error flags.
+bool Backend::queue_sampling(const gptrs_hip_tensor* logits, float temperature, bool has_top_k, bool has_u, float u, int64_t* host) {
     GPTRS_HIP_CHECK(hipSetDevice(device));
     flush_fresh();
     if (logits->consumed) fail_exec("tensor handle was donated to run_program and can no longer be read");
@@ -477,33 +480,33 @@ bool Backend::queue_sampling(const gptrs_hip_tensor* logits, float temperature, 
     const int64_t vocab = s.dims.back(), rows = s.rank() == 2 ? s.dims[0] : 1;
     if (has_top_k) return false;  // Ok(None): host sampler handles top-k
     if (temperature <= 0.0f) {
-        k::argmax_last_row(stream, (int)s.dtype, logits->data(), rows, vocab, d_token_, d_argmax_val_, d_argmax_idx_, 1024);
-        n_launches += 2;
+        const char* last = (const char*)logits->data() + (size_t)(rows - 1) * vocab * dtype_size(s.dtype);
+        k::argmax_tokens(stream, (int)s.dtype, last, 1, vocab, d_token_, nullptr, argmax_scratch(), host);
+        n_launches += 1;
     } else {
         if (!has_u) return false;
         k::sample_temperature_last_row(stream, (int)s.dtype, logits->data(), rows, vocab, temperature, u, d_token_);
+        GPTRS_HIP_CHECK(hipMemcpyAsync(host, d_token_, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+        GPTRS_HIP_CHECK(hipMemcpyAsync(host + 1, d_err_flag_, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
         n_launches += 1;
     }
     return true;
 }
 
 int64_t Backend::sample(const gptrs_hip_tensor* logits, float temperature, bool has_top_k, bool has_u, float u) {
-    if (!queue_sampling(logits, temperature, has_top_k, has_u, u)) return -1;
     int64_t* host = (int64_t*)h_pinned_;
-    GPTRS_HIP_CHECK(hipMemcpyAsync(host, d_token_, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
+    if (!queue_sampling(logits, temperature, has_top_k, has_u, u, host)) return -1;
     GPTRS_HIP_CHECK(hipStreamSynchronize(stream));
     check_device_errors();
     return *host;
 }
 
 int64_t Backend::sample_begin(const gptrs_hip_tensor* logits, float temperature, bool has_top_k, bool has_u, float u) {
-    if (!queue_sampling(logits, temperature, has_top_k, has_u, u)) return -1;
+    const int slot = (int)(next_ticket_ % kTokenRing);
+    if (!queue_sampling(logits, temperature, has_top_k, has_u, u, h_token_ring_ + kRingSlot * slot)) return -1;
     const int64_t ticket = next_ticket_++;
-    const int slot = (int)(ticket % kTokenRing);
     if (!token_events_[slot]) GPTRS_HIP_CHECK(hipEventCreateWithFlags(&token_events_[slot], hipEventDisableTiming));
     ring_rows_[slot] = 0;
-    GPTRS_HIP_CHECK(hipMemcpyAsync(h_token_ring_ + kRingSlot * slot, d_token_, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
-    GPTRS_HIP_CHECK(hipMemcpyAsync(h_token_ring_ + kRingSlot * slot + 1, d_err_flag_, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
     GPTRS_HIP_CHECK(hipEventRecord(token_events_[slot], stream));
     return ticket;
 }
@@ -516,15 +519,12 @@ int64_t Backend::sample_rows_begin(const gptrs_hip_tensor* logits) {
     const Spec& s = logits->spec;
     if (!dtype_is_float(s.dtype) || s.rank() != 2 || s.count() == 0 || s.dims[0] > kMaxTokenRows)
         fail_exec("sample_decode_rows expects non-empty f32/bf16 logits [rows <= 64, vocab]");
-    k::argmax_rows(stream, (int)s.dtype, logits->data(), s.dims[0], s.dims[1], (int32_t*)rows_buf_->ptr, d_argmax_val_, d_argmax_idx_, 1024);
-    n_launches += 2;
     const int64_t ticket = next_ticket_++;
     const int slot = (int)(ticket % kTokenRing);
+    k::argmax_tokens(stream, (int)s.dtype, logits->data(), s.dims[0], s.dims[1], nullptr, (int32_t*)rows_buf_->ptr, argmax_scratch(), h_token_ring_ + kRingSlot * slot);
+    n_launches += 1;
     if (!token_events_[slot]) GPTRS_HIP_CHECK(hipEventCreateWithFlags(&token_events_[slot], hipEventDisableTiming));
     ring_rows_[slot] = (int)s.dims[0];
-    GPTRS_HIP_CHECK(hipMemcpyAsync(h_token_ring_ + kRingSlot * slot + 2, rows_buf_->ptr, (size_t)s.dims[0] * sizeof(int32_t),
-                                   hipMemcpyDeviceToHost, stream));
-    GPTRS_HIP_CHECK(hipMemcpyAsync(h_token_ring_ + kRingSlot * slot + 1, d_err_flag_, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
     GPTRS_HIP_CHECK(hipEventRecord(token_events_[slot], stream));
     return ticket;
 }

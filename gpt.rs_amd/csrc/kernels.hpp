@@ -62,12 +62,14 @@ struct DotDesc {
 // dtype: of A and B; out_f32: bf16 operands, the f32 accumulator is stored as f32 (DotGeneralSpec.out_dtype)
 void dot_generic(hipStream_t s, int dtype, const void* a, const void* b, void* c, const DotDesc& d, bool out_f32 = false);
 
-// last row of [rows][vocab] logits; ties -> smallest index; result (int64) written to *out
-// greedy token of every row (rows * partial blocks <= scratch_cap), ties to the smallest index; out: si32[rows]
+// Greedy token of every row of logits [rows, vocab], ties to the smallest index.  One row into out64, or each into out32 (si32[rows]); with `host`, a
+// pinned slot, also there: [0] the token of out64, [1] the eight bytes at err_flags, from [2] on the tokens of out32.  Scratch: `parts` partial
+// results (rows <= parts), a ticket per row that is zero before and after; the launch has them to itself.
+struct ArgmaxScratch { float* val; int32_t* idx; int parts; unsigned* tickets; const int64_t* err_flags; };
+void argmax_tokens(hipStream_t s, int dtype, const void* logits, int64_t rows, int64_t vocab, int64_t* out64, int32_t* out32, const ArgmaxScratch& w, int64_t* host);
+// the same in two launches without tickets (rows * partial blocks <= scratch_cap); out: si32[rows]
 void argmax_rows(hipStream_t s, int dtype, const void* logits, int64_t rows, int64_t vocab, int32_t* out, float* scratch_val,
                  int32_t* scratch_idx, int scratch_cap);
-void argmax_last_row(hipStream_t s, int dtype, const void* logits, int64_t rows, int64_t vocab, int64_t* out,
-                     float* scratch_val, int32_t* scratch_idx, int scratch_cap);
 // argmax_rows over a fixed device array of the library instead of caller scratch: no allocation anywhere.
 // argmax_noalloc_init: once per device, with that device current (resolves the array's address on that GPU).
 // argmax_rows_noalloc: false when the device was not initialised or rows is outside [1, argmax_noalloc_max_rows()].

@@ -381,59 +381,78 @@ void dot_generic(hipStream_t s, int dtype, const void* a, const void* b, void* c
 }
 
 // ------------------------------------------------------------------------------ sampling
-// argmax of the last row: stage 1 = per-block (value, smallest index) partials, stage 2 = one
-// block combines.  Ties -> smallest index (docs/backend.md:270).
+// Greedy token of every row of logits [gridDim.y, n], in one launch: a workgroup leaves the (value, smallest index) of its share, and the one
+// that draws a row's last ticket combines them.  Ties -> smallest index (docs/backend.md:270).  The token goes where the next step reads it
+// (out64, one row, or out32) and, with `host`, straight into the pinned slot that the caller waits for, with the device's error flags beside
+// it: host[0] the token of a single row, host[1] the flags, from host + 2 on the tokens of several.  Between two decode steps
+// that is one launch of 6 us where two stages and two copies took 19.  A ticket is zero before and after every launch.
 template <typename T>
-__global__ void argmax_stage1(const T* __restrict__ row, int64_t n, float* pv, int32_t* pi) {
+__global__ __launch_bounds__(256) void argmax_kernel(const T* __restrict__ logits, int64_t n, float* pv, int32_t* pi, unsigned* tickets, int64_t* out64, int32_t* out32,
+                                                     int64_t* host, const int64_t* err_flags) {
+    constexpr int U = 4;
     __shared__ float sv[4];
     __shared__ int32_t si[4];
+    __shared__ unsigned ticket;
+    const T* row = logits + (int64_t)blockIdx.y * n;
     float best = -INFINITY;
     int32_t bidx = 0x7fffffff;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float v = ldf(row, i);
-        if (v > best || (v == best && (int32_t)i < bidx)) { best = v; bidx = (int32_t)i; }
+    auto better = [&](float v, int32_t i) { if (v > best || (v == best && i < bidx)) { best = v; bidx = i; } };
+    auto over_wave = [&]() {
+        for (int off = 32; off > 0; off >>= 1) {
+            const float ov = __shfl_down(best, off, 64);
+            const int32_t oi = __shfl_down(bidx, off, 64);
+            better(ov, oi);
+        }
+    };
+    const int64_t stride = (int64_t)gridDim.x * 256;
+    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += U * stride) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = ldf(row, i0 + u * stride < n ? i0 + u * stride : i0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) better(v[u], (int32_t)(i0 + u * stride < n ? i0 + u * stride : i0));
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        const float ov = __shfl_down(best, off, 64);
-        const int32_t oi = __shfl_down(bidx, off, 64);
-        if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
-    }
+    over_wave();
     if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = best; si[threadIdx.x >> 6] = bidx; }
     __syncthreads();
+    const int part = blockIdx.y * gridDim.x;
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; ++w)
-            if (sv[w] > best || (sv[w] == best && si[w] < bidx)) { best = sv[w]; bidx = si[w]; }
-        pv[blockIdx.x] = best;
-        pi[blockIdx.x] = bidx;
+        for (int w = 1; w < 4; ++w) better(sv[w], si[w]);
+        __hip_atomic_store(pv + part + blockIdx.x, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (other XCDs read them)
+        __hip_atomic_store(pi + part + blockIdx.x, bidx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(0x0F70);                                                             // vmcnt(0)
+        asm volatile("" ::: "memory");
+        ticket = __hip_atomic_fetch_add(tickets + blockIdx.y, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    __syncthreads();
+    if (ticket != gridDim.x - 1 || threadIdx.x >= 64) return;
+    best = -INFINITY;
+    bidx = 0x7fffffff;
+    for (int i = threadIdx.x; i < (int)gridDim.x; i += 64)
+        better(__hip_atomic_load(pv + part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), __hip_atomic_load(pi + part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    over_wave();
+    if (threadIdx.x != 0) return;
+    const int32_t token = bidx == 0x7fffffff ? 0 : bidx;
+    if (out64) *out64 = token;
+    if (out32) out32[blockIdx.y] = token;
+    if (host) {
+        if (out64) __hip_atomic_store(host, (int64_t)token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (out32) __hip_atomic_store(reinterpret_cast<int32_t*>(host + 2) + blockIdx.y, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (blockIdx.y == 0) __hip_atomic_store(host + 1, *err_flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __hip_atomic_store(tickets + blockIdx.y, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__global__ void argmax_stage2(const float* pv, const int32_t* pi, int nparts, int64_t* out) {
-    float best = -INFINITY;
-    int32_t bidx = 0x7fffffff;
-    for (int i = threadIdx.x; i < nparts; i += 64) {
-        const float v = pv[i];
-        const int32_t id = pi[i];
-        if (v > best || (v == best && id < bidx)) { best = v; bidx = id; }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const float ov = __shfl_down(best, off, 64);
-        const int32_t oi = __shfl_down(bidx, off, 64);
-        if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
-    }
-    if (threadIdx.x == 0) *out = bidx == 0x7fffffff ? 0 : (int64_t)bidx;
-}
-void argmax_last_row(hipStream_t s, int dtype, const void* logits, int64_t rows, int64_t vocab, int64_t* out,
-                     float* scratch_val, int32_t* scratch_idx, int scratch_cap) {
-    int nb = (int)cdiv(vocab, 256 * 8);
+void argmax_tokens(hipStream_t s, int dtype, const void* logits, int64_t rows, int64_t vocab, int64_t* out64, int32_t* out32, const ArgmaxScratch& w, int64_t* host) {
+    if (rows <= 0) return;
+    int64_t nb = cdiv(vocab, 256 * 4);
+    if (nb > w.parts / rows) nb = w.parts / rows;
     if (nb < 1) nb = 1;
-    if (nb > scratch_cap) nb = scratch_cap;
-    const size_t off = (size_t)(rows - 1) * vocab;
-    if (dtype == 0) argmax_stage1<float><<<nb, 256, 0, s>>>((const float*)logits + off, vocab, scratch_val, scratch_idx);
-    else argmax_stage1<bf16_t><<<nb, 256, 0, s>>>((const bf16_t*)logits + off, vocab, scratch_val, scratch_idx);
-    argmax_stage2<<<1, 64, 0, s>>>(scratch_val, scratch_idx, nb, out);
+    const dim3 grid((unsigned)nb, (unsigned)rows);
+    if (dtype == 0) argmax_kernel<float><<<grid, 256, 0, s>>>((const float*)logits, vocab, w.val, w.idx, w.tickets, out64, out32, host, w.err_flags);
+    else argmax_kernel<bf16_t><<<grid, 256, 0, s>>>((const bf16_t*)logits, vocab, w.val, w.idx, w.tickets, out64, out32, host, w.err_flags);
 }
 
-// Greedy token of EVERY row (batched decode): the same two stages with the row in blockIdx.y; out[r] as si32.
+// The same in two stages without tickets, for callers that may overlap (argmax_rows_noalloc): per-block partials, then one block per row; out[r] as si32.
 template <typename T>
 __global__ void argmax_rows_stage1(const T* __restrict__ logits, int64_t n, float* pv, int32_t* pi) {
     __shared__ float sv[4];

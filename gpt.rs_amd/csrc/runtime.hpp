@@ -302,7 +302,8 @@ class Backend {
     int ring_rows_[kTokenRing] = {};   // rows behind each ticket (0: a single-token ticket)
     hipEvent_t token_events_[kTokenRing] = {};
     int64_t next_ticket_ = 0;
-    bool queue_sampling(const gptrs_hip_tensor* logits, float temperature, bool has_top_k, bool has_u, float u);
+    bool queue_sampling(const gptrs_hip_tensor* logits, float temperature, bool has_top_k, bool has_u, float u, int64_t* host);
+    k::ArgmaxScratch argmax_scratch() const;
     void* h_pinned_ = nullptr;  // 64 bytes of pinned host memory for readbacks
     struct Derived { std::weak_ptr<Buffer> src, src2; BufferP tiled; int64_t k = 0, n = 0; };
     std::map<std::array<uint64_t, 3>, Derived> tiled_cache_;

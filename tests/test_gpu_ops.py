@@ -701,3 +701,31 @@ def test_few_tile_gemm_splits_k_and_is_reproducible(hip, dtype, m, k, n):
         assert_close(got, want, atol=2e-4, rtol=1e-4, what="few-tile f32 linear")
     else:
         assert_close(got, want, atol=1e-2, rtol=2.0 ** -7, what="few-tile bf16 linear")
+
+
+@pytest.mark.parametrize("dt", ["F32", "Bf16"])
+@pytest.mark.parametrize("rows,vocab", [(1, 1), (1, 255), (1, 1024), (1, 1025), (1, 50257), (1, 1200000), (3, 4097), (8, 131072), (64, 20000), (2, 2)])
+def test_greedy_tokens_of_rows(hip, dt, rows, vocab):
+    """One launch: shares of a row meet by ticket, and the tokens reach the host without a copy.  Ties to the smallest index, also across
+    shares; rows without a largest value; the same scratch again and again."""
+    from gptrs_amd.ptir import TensorSpec
+    rng = np.random.default_rng(rows + vocab)
+    for trial in range(3):
+        x = rng.standard_normal((rows, vocab), dtype=np.float32)
+        for r in range(rows):
+            at = rng.integers(0, vocab, 3)
+            x[r, at] = 9.0                                   # a tie of up to three, anywhere
+        if trial == 1:
+            x[0] = -np.inf                                   # the first index
+        if trial == 2:
+            x[-1, ::2] = np.nan                              # never the largest
+            if vocab == 1:
+                x[-1] = np.nan                               # no index at all: 0
+        y = bf16_bits_to_f32(f32_to_bf16_bits(x)).reshape(x.shape) if dt == "Bf16" else x
+        want = [int(np.argmax(np.where(np.isnan(v), -np.inf, v))) if not np.isnan(v).all() else 0 for v in y]
+        h = hip.materialize(TensorSpec(dt, [rows, vocab]), to_bytes(x, dt))
+        assert hip.sample_decode_token(h, temperature=0.0) == want[-1]
+        assert hip.sample_decode_token_wait(hip.sample_decode_token_begin(h, temperature=0.0)) == want[-1]
+        assert hip.sample_decode_rows_wait(hip.sample_decode_rows_begin(h), rows) == want
+        assert hip.to_numpy(hip.decode_rows_tensor(rows)).tolist() == want
+        assert hip.to_numpy(hip.decode_token_tensor()).tolist() == [want[-1]]
