@@ -51,6 +51,9 @@ void reduce(hipStream_t s, int dtype, int kind, const void* x, void* y, int64_t 
 // zero-fills the row and raises *err_flag (checked at the next synchronising call)
 void take(hipStream_t s, int elem_size, const void* table, const int32_t* idx, void* y, int64_t n_idx,
           int64_t vocab, int64_t inner, int* err_flag);
+// y[r] = ta[ia[r]] + tb[ib[r]], rows of `inner` values (dtype 0 f32, 2 bf16: rounded once)
+void take_add(hipStream_t s, int dtype, const void* ta, const int32_t* ia, int64_t rows_a, const void* tb, const int32_t* ib, int64_t rows_b, void* y, int64_t n_idx, int64_t inner,
+              int* err_flag);
 
 // C[b][m][n] = sum_k A[b][m][k] * B[b][k][n]; element strides given per operand; f32 accumulate.
 struct DotDesc {

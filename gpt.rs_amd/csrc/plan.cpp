@@ -772,6 +772,24 @@ void Builder::build() {
     for (int v = 0; v < nv; ++v)
         if (plan.values[v].defined && plan.values[v].root == v && def_step[v] >= 0 && plan.storage[v].kind == Storage::Temp)
             dying[std::max(last_use[v], def_step[v])].push_back(v);
+    // sums of two gathers (Step::take_a)
+    for (int s = 0; s < n_steps; ++s) {
+        Step& st = plan.steps[s];
+        if (st.in.op != OpKind::Binary || st.in.scalar_rhs || st.in.binary != BinaryOp::Add || !dtype_is_float(st.in.out_specs[0].dtype)) continue;
+        auto gather = [&](int v) {   // the step that makes operand v, if nothing but this sum needs its result
+            const int r = v >= 0 ? root(v) : -1;
+            if (r < 0 || def_step[r] < 0 || use_count[r] != 1 || root_is_result[r]) return -1;
+            const Step& t = plan.steps[def_step[r]];
+            if (t.in.op != OpKind::Take || t.axis_len < 1 || t.in.out_specs[0].count() != st.in.out_specs[0].count()) return -1;
+            for (int o = 0; o < 2; ++o)
+                if (t.src[o] < 0 || plan.storage[root(t.src[o])].kind != Storage::Input) return -1;
+            return def_step[r];
+        };
+        const int a = gather(st.src[0]), b = gather(st.src[1]);
+        if (a < 0 || b < 0 || a == b || plan.steps[a].inner != plan.steps[b].inner || plan.steps[a].outer != plan.steps[b].outer) continue;
+        st.take_a = a; st.take_b = b;
+        plan.steps[a].left_out = plan.steps[b].left_out = true;
+    }
     // prefill linears whose f32 result goes into an RMS norm with the next step (Step::norm_next)
     for (int s = 0; s + 1 < n_steps; ++s) {
         Step& st = plan.steps[s];
@@ -1023,6 +1041,7 @@ static bool run_chain(const Plan& plan, const Step& head, ExecCtx& cx) {
 
 void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
     if (cx.done_ahead == &st) { cx.done_ahead = nullptr; return; }
+    if (st.left_out) return;
     const Instr& in = st.in;
     const Spec& out = in.out_specs[0];
     void* dst = cx.ptr[st.dst[0]];
@@ -1062,7 +1081,11 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
             ++cx.launches;
             break;
         case OpKind::Binary:
-            if (in.scalar_rhs) k::binary_scalar(s, (int)out.dtype, (int)in.binary, src_ptr(st, cx, 0), in.scalar_val, dst, out.count());
+            if (st.take_a >= 0) {
+                const Step &a = plan.steps[st.take_a], &b = plan.steps[st.take_b];
+                k::take_add(s, (int)out.dtype, src_ptr(a, cx, 0), (const int32_t*)src_ptr(a, cx, 1), a.axis_len, src_ptr(b, cx, 0), (const int32_t*)src_ptr(b, cx, 1), b.axis_len, dst,
+                            a.outer, a.inner, cx.err_flag);
+            } else if (in.scalar_rhs) k::binary_scalar(s, (int)out.dtype, (int)in.binary, src_ptr(st, cx, 0), in.scalar_val, dst, out.count());
             else k::binary(s, (int)out.dtype, (int)in.binary, src_ptr(st, cx, 0), src_ptr(st, cx, 1), dst, out.count());
             ++cx.launches;
             break;

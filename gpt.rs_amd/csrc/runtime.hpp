@@ -123,6 +123,9 @@ struct Step {
     // Prefill linear: the next step is an RMS norm of its f32 result, which the launch that adds its splits may do; the norm's result is then
     // given its storage together with this step's own.
     bool norm_next = false;
+    // Sum of two gathers of program inputs: the gathers' steps are left out and this step reads the tables itself.
+    int take_a = -1, take_b = -1;
+    bool left_out = false;
     k::CopyDesc pack_l{}, pack_r{};
     size_t pack_l_off = 0, pack_r_off = 0;
 };

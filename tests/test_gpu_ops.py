@@ -729,3 +729,29 @@ def test_greedy_tokens_of_rows(hip, dt, rows, vocab):
         assert hip.sample_decode_rows_wait(hip.sample_decode_rows_begin(h), rows) == want
         assert hip.to_numpy(hip.decode_rows_tensor(rows)).tolist() == want
         assert hip.to_numpy(hip.decode_token_tensor()).tolist() == [want[-1]]
+
+
+@pytest.mark.parametrize("dt", ["F32", "Bf16"])
+@pytest.mark.parametrize("rows,inner", [(1, 768), (7, 768), (3, 5), (1, 1), (300, 24), (2, 1028)])
+def test_sum_of_two_gathers(hip, dt, rows, inner):
+    """One launch where nothing else needs the gathered rows; the same values either way, and an index outside its table is reported either way."""
+    rng = np.random.default_rng(rows + inner)
+    ta, tb = (to_bytes(rng.standard_normal((n, inner), dtype=np.float32), dt) for n in (50, 9))
+    ta, tb = (np.frombuffer(t, "<u2" if dt == "Bf16" else "<f4").reshape(-1, inner) for t in (ta, tb))
+    fa, fb_ = (bf16_bits_to_f32(t).reshape(t.shape) if dt == "Bf16" else t for t in (ta, tb))
+    ia, ib = rng.integers(0, 50, rows).astype(np.int32), rng.integers(0, 9, rows).astype(np.int32)
+    specs = [(dt, [50, inner]), ("Si32", [rows]), (dt, [9, inner]), ("Si32", [rows])]
+    p = prog(lambda fb, a, i, b, j: a.take(i) + b.take(j), specs)
+    got = hip_run(hip, p, [fa, ia, fb_, ib])[0]
+    assert hip.counter("last_program_launches") == 1
+    want = fa[ia] + fb_[ib]
+    assert np.array_equal(got, bf16_bits_to_f32(f32_to_bf16_bits(want)).reshape(want.shape) if dt == "Bf16" else want)
+    kept = prog(lambda fb, a, i, b, j: (lambda r: [r + b.take(j), r])(a.take(i)), specs)
+    both = hip_run(hip, kept, [fa, ia, fb_, ib])
+    assert np.array_equal(both[0], got) and np.array_equal(both[1], fa[ia])
+    for bad in ([fa, np.full(rows, 50, np.int32), fb_, ib], [fa, ia, fb_, np.full(rows, -1, np.int32)]):
+        for q in (p, kept):
+            with pytest.raises(Exception):
+                hip_run(hip, q, bad)
+                hip.synchronize()
+    assert np.array_equal(hip_run(hip, p, [fa, ia, fb_, ib])[0], got)
