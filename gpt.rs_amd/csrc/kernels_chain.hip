@@ -592,16 +592,15 @@ struct Patience {
         return now - t0 > ticks;
     }
 };
-// Where the compute waves of a workgroup wait until the control wave has seen the grid barrier of a phase that the workgroup takes part in, and where
-// the control wave lets them go: a workgroup barrier, which costs the waiting waves no instructions and releases them at once (polling a
-// word of LDS took them 0.3 us to notice, and issue slots from the control wave on their SIMD).  The control wave comes here
-// whether the barrier was seen or it has given up (its waits are bounded), or it has ended, and a wave that has ended is not waited
-// for: so every wave gets past, and False says that the launch is being abandoned.
+// compute waves wait here until the control wave has seen the grid barrier of `phase`
 template <typename IP>
-__device__ __forceinline__ bool phase_opens(IP abort) {
-    wg_barrier();
-    asm volatile("" ::: "memory");
-    return uni(lds_ld(abort)) == 0;
+__device__ __forceinline__ bool wait_go(IP go, IP abort, int phase, unsigned long long budget) {
+    Patience pat(8 * budget);
+    while (uni(lds_ld(go)) < phase) {
+        __builtin_amdgcn_s_sleep(1);
+        if (uni(lds_ld(abort)) || pat.spent()) return false;
+    }
+    return true;
 }
 
 // exp through v_exp_f32 (2^x): softmax weights only, about one ulp, exp(-inf) = 0
@@ -643,7 +642,8 @@ __device__ __forceinline__ void lane_pair(float v, int off, float& a, float& b) 
 // the waves of different heads re-read the same rows out of the caches.  Cache rows older than
 // this launch are requested BEFORE the grid barrier is awaited (they do not depend on the
 // previous phase); only the query row and this step's K/V row are read after it.
-__device__ bool attn_partial(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int unit) {
+__device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int unit, int phase,
+                             unsigned long long budget) {
     constexpr int PP = 5;   // positions per lane group requested ahead of the barrier (32 chunks x 8 lane groups x 5 = 1280 positions)
     const int t = local_tid(), lane = t & 63, wave = uni(t >> 6);
     const bool control = wave == NWS;
@@ -681,7 +681,7 @@ __device__ bool attn_partial(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LD
             vraw[j] = make_uint4(0, 0, 0, 0);
         }
     }
-    if (!phase_opens(abort)) return false;
+    if (!control && !wait_go(go, abort, phase, budget)) return false;
 
     float m = -INFINITY, l = 0.f, o[8];
 #pragma unroll
@@ -827,11 +827,12 @@ __device__ bool attn_partial(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LD
 // unit = query head: softmax-merge of its nch chunk records into the context row.  Thread
 // (sg, d2) reads the records of the chunks s = sg, sg + NW, ... for the dims (2 d2, 2 d2 + 1) in
 // one round of loads and merges them locally; the NW subsets meet in LDS.
-__device__ bool attn_combine(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq) {
+__device__ bool attn_combine(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq, int phase,
+                             unsigned long long budget) {
     constexpr int MAXC = 8;   // chunks per thread: nch <= MAXC * NW
     const int t = local_tid(), wave = uni(t >> 6);
     const int dh = P.head_dim, nch = P.nch;
-    if (!phase_opens(abort)) return false;
+    if (wave != NWS && !wait_go(go, abort, phase, budget)) return false;
     const float* base = P.part + (long)hq * nch * (dh + 2);
     bf16_t* ctx = (bf16_t*)P.y;
     const int h2 = dh / 2;
@@ -887,7 +888,8 @@ __device__ bool attn_combine(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LD
 // lane's 8 values are then two 16-byte words; no RoPE): written this way the bf16 phases above lost a microsecond each
 // to the compiler, so they keep their own text.
 template <bool F32>
-__device__ bool attn_partial_t(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int unit) {
+__device__ bool attn_partial_t(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int unit, int phase,
+                             unsigned long long budget) {
     typedef typename std::conditional<F32, float, bf16_t>::type E;
     constexpr int PP = F32 ? 2 : 4;   // positions per lane group requested ahead of the barrier
     constexpr int RW = F32 ? 2 : 1;   // 16-byte words of a lane's 8 values
@@ -953,7 +955,7 @@ __device__ bool attn_partial_t(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_
             unpack8(w[0], w[1], f);
         }
     };
-    if (!phase_opens(abort)) return false;
+    if (!control && !wait_go(go, abort, phase, budget)) return false;
 
     float m = -INFINITY, l = 0.f, o[8];
 #pragma unroll
@@ -1113,11 +1115,12 @@ __device__ bool attn_partial_t(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_
 // (sg, d2) reads the records of the chunks s = sg, sg + NW, ... for the dims (2 d2, 2 d2 + 1) in
 // one round of loads and merges them locally; the NW subsets meet in LDS.
 template <bool F32>
-__device__ bool attn_combine_t(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq) {
+__device__ bool attn_combine_t(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq, int phase,
+                             unsigned long long budget) {
     constexpr int MAXC = 8;   // chunks per thread: nch <= MAXC * NW
     const int t = local_tid(), wave = uni(t >> 6);
     const int dh = P.head_dim, nch = P.nch;
-    if (!phase_opens(abort)) return false;
+    if (wave != NWS && !wait_go(go, abort, phase, budget)) return false;
     const float* base = P.part + (long)hq * nch * (dh + 2);
     bf16_t* ctx = (bf16_t*)P.y;
     const int h2 = dh / 2;
@@ -1176,7 +1179,8 @@ __device__ bool attn_combine_t(GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_
 // The descriptor comes straight from the table in memory (scalar loads): the compute waves enter an attention phase, and
 // request the cache rows it needs, before the control wave has seen the barrier and filled the LDS copy.
 template <bool F32>
-__device__ __forceinline__ bool run_attn_phase(const GPTRS_CONST ChainPhase* php, GPTRS_LDS float* lds, GPTRS_LDS int* abort) {
+__device__ __forceinline__ bool run_attn_phase(const GPTRS_CONST ChainPhase* php, GPTRS_LDS float* lds, GPTRS_LDS int* go, GPTRS_LDS int* abort, int phase,
+                                               unsigned long long budget) {
     ChainPhase P;
     {
         int* dst = reinterpret_cast<int*>(&P);
@@ -1188,11 +1192,11 @@ __device__ __forceinline__ bool run_attn_phase(const GPTRS_CONST ChainPhase* php
     for (int u = blockIdx.x; u < units; u += gridDim.x) {
         bool ok;
         if (F32) {
-            if (kind == kChainAttnCombine) ok = attn_combine_t<true>(abort, P, lds, u);
-            else ok = attn_partial_t<true>(abort, P, lds, u);
+            if (kind == kChainAttnCombine) ok = attn_combine_t<true>(go, abort, P, lds, u, phase, budget);
+            else ok = attn_partial_t<true>(go, abort, P, lds, u, phase, budget);
         } else {
-            if (kind == kChainAttnCombine) ok = attn_combine(abort, P, lds, u);
-            else ok = attn_partial(abort, P, lds, u);
+            if (kind == kChainAttnCombine) ok = attn_combine(go, abort, P, lds, u, phase, budget);
+            else ok = attn_partial(go, abort, P, lds, u, phase, budget);
         }
         if (!ok) return false;
     }
@@ -1239,18 +1243,17 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
             if (!ok) {
                 __hip_atomic_store(as_global(abort_flag), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 lds_st(&sh.abort, 1);
-                __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): there before this wave's end lets the others past their barrier
                 return;
             }
         }
         // the compute waves hold their own copy of the descriptor: the phase opens the moment the barrier is seen
         if (kind != kChainLinear) {
             if (blk < units) {
-                run_attn_phase<FMT == kChainW32>(table + ph, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.abort);
+                if (lane == 0) lds_st(&sh.go, ph);
+                run_attn_phase<FMT == kChainW32>(table + ph, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.go, (GPTRS_LDS int*)&sh.abort, ph, budget);
             }
         } else if (u0 < u1) {
-            if (lane == 0) lds_st(&sh.go, ph);   // (compute waves that are about to park another step look at it)
-            phase_opens(&sh.abort);
+            if (lane == 0) lds_st(&sh.go, ph);
             PhaseRegs P;
             regs_from_lanes<FMT == kChainW32 || FMT == kChainW16, FMT == kChainW16>(P, pd);
             const int flags = P.flags, ntiles = P.ntiles, N = P.N;
@@ -1347,7 +1350,6 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
                     __builtin_amdgcn_s_sleep(1);
                     if (pat.spent()) {
                         lds_st(&sh.abort, 1);
-                        __builtin_amdgcn_s_waitcnt(0xC07F);   // as above
                         __hip_atomic_store(as_global(abort_flag), 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         return;
                     }
@@ -1591,7 +1593,8 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
             const int units = uni(D->units);
             if (uni(D->kind) != kChainLinear) {
                 if (blk >= units) continue;
-                if (!run_attn_phase<FMT == kChainW32>(table + c_phase, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.abort)) return false;
+                if (!run_attn_phase<FMT == kChainW32>(table + c_phase, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.go, (GPTRS_LDS int*)&sh.abort, c_phase,
+                                    budget)) return false;
                 continue;
             }
             const int upb = uni(D->upb);
@@ -1629,9 +1632,9 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
       // back first; the registers are free again before the next phase is looked for.
       constexpr int PARKN = FMT == kChainW4 ? PARK_W4 : (FMT == kChainW8 ? PARK_W8 : PARK);   // (the int4 kernel stages its group scales through registers as well)
       u32x4 park[PARKN][TP];
-      int n_parked = 0;
+      int n_parked = 0, park_rd = 0;
       {
-        const int want = min(PARKN, min(c_wpt, inflight));   // of the phase's first unit
+        const int want = min(PARKN, min(c_wpt * (c_unit_end - c_unit), inflight));
 #pragma unroll
         for (int i = 0; i < PARKN; ++i) {
             if (i < want && uni(lds_ld(&sh.go)) < c_phase) {
@@ -1654,97 +1657,24 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
             }
         }
       }
-      if (!phase_opens(&sh.abort)) break;
+      if (!wait_go(&sh.go, &sh.abort, c_phase, budget)) break;
       if (FMT == kChainW32) stage_block_f32(R, const_cast<unsigned*>(xs), sh.ssq);
       else stage_block<FMT>(R, const_cast<unsigned*>(xs), sh.ssq);
-      auto multiply = [&](u32x4 (&cur)[TP], int j) {   // j-step j of the unit
-          if ((j + 1) * NS > c_Kv) {   // the stream's last step: lanes whose words are padding count as zeros
-              if (j * NS + t >= c_Kv) {
-#pragma unroll
-                  for (int p = 0; p < TP; ++p) { cur[p].x = 0u; cur[p].y = 0u; cur[p].z = 0u; cur[p].w = 0u; }
-              }
-          }
-          // element reads go through scalars: __builtin_bit_cast applied directly to `vec.y` of an
-          // ext-vector reads element 0 with this compiler
-          if (c_fmt == kChainW16) {
-              const bf16x2 xv = __builtin_bit_cast(bf16x2, xs[j * NS + t]);
-#pragma unroll
-              for (int p = 0; p < TP; ++p) {
-                  const unsigned q0 = cur[p].x, q1 = cur[p].y, q2 = cur[p].z, q3 = cur[p].w;
-                  acc[p][0] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q0), xv, acc[p][0], false);
-                  acc[p][1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q1), xv, acc[p][1], false);
-                  acc[p][2] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q2), xv, acc[p][2], false);
-                  acc[p][3] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q3), xv, acc[p][3], false);
-              }
-          } else if (c_fmt == kChainW32) {
-              const float xv = __uint_as_float(xs[j * NS + t]);
-#pragma unroll
-              for (int p = 0; p < TP; ++p) {
-                  const unsigned q0 = cur[p].x, q1 = cur[p].y, q2 = cur[p].z, q3 = cur[p].w;
-                  acc[p][0] = __builtin_fmaf(__uint_as_float(q0), xv, acc[p][0]);
-                  acc[p][1] = __builtin_fmaf(__uint_as_float(q1), xv, acc[p][1]);
-                  acc[p][2] = __builtin_fmaf(__uint_as_float(q2), xv, acc[p][2]);
-                  acc[p][3] = __builtin_fmaf(__uint_as_float(q3), xv, acc[p][3]);
-              }
-          } else if (c_fmt == kChainW8) {
-              const u32x2 xw = *reinterpret_cast<const u32x2*>(&xs[2 * (j * NS + t)]);
-              const unsigned xa = xw.x, xb = xw.y;
-              const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
-              const float corr = -128.0f * ((x0 + x1) + (x2 + x3));
-#pragma unroll
-              for (int p = 0; p < TP; ++p) {
-                  const unsigned q[4] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w};
-#pragma unroll
-                  for (int c = 0; c < 4; ++c) {
-                      float a = acc[p][c] + corr;
-                      a = __builtin_fmaf((float)(q[c] & 0xFFu), x0, a);
-                      a = __builtin_fmaf((float)((q[c] >> 8) & 0xFFu), x1, a);
-                      a = __builtin_fmaf((float)((q[c] >> 16) & 0xFFu), x2, a);
-                      a = __builtin_fmaf((float)(q[c] >> 24), x3, a);
-                      acc[p][c] = a;
-                  }
-              }
-          } else {
-              const u32x4 xw = *reinterpret_cast<const u32x4*>(&xs[4 * (j * NS + t)]);
-              const unsigned xa = xw.x, xb = xw.y, xc = xw.z, xd = xw.w;
-              const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
-              const float x4 = bf16lo(xc), x5 = bf16hi(xc), x6 = bf16lo(xd), x7 = bf16hi(xd);
-              const float corr = -8.0f * (((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7)));
-#pragma unroll
-              for (int p = 0; p < TP; ++p) {
-                  const unsigned q[4] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w};
-                  const u32x2 sw = *reinterpret_cast<const u32x2*>(&xs[c_soff + 2 * (c_sidx + p * c_G + j * (NS / 16) + (t >> 4))]);
-                  const unsigned sa = sw.x, sb = sw.y;
-                  const float sc[4] = {bf16lo(sa), bf16hi(sa), bf16lo(sb), bf16hi(sb)};
-#pragma unroll
-                  for (int c = 0; c < 4; ++c) {
-                      // byte i of a column's dword: k = 2i in the low nibble, k = 2i + 1 in the high one
-                      const unsigned lo = q[c] & 0x0F0F0F0Fu, hi = (q[c] >> 4) & 0x0F0F0F0Fu;
-                      float a = corr;
-                      a = __builtin_fmaf((float)(lo & 0xFFu), x0, a);
-                      a = __builtin_fmaf((float)(hi & 0xFFu), x1, a);
-                      a = __builtin_fmaf((float)((lo >> 8) & 0xFFu), x2, a);
-                      a = __builtin_fmaf((float)((hi >> 8) & 0xFFu), x3, a);
-                      a = __builtin_fmaf((float)((lo >> 16) & 0xFFu), x4, a);
-                      a = __builtin_fmaf((float)((hi >> 16) & 0xFFu), x5, a);
-                      a = __builtin_fmaf((float)(lo >> 24), x6, a);
-                      a = __builtin_fmaf((float)(hi >> 24), x7, a);
-                      acc[p][c] = __builtin_fmaf(sc[c], a, acc[p][c]);
-                  }
-              }
-          }
-      };
+      bool from_park = false;
       for (; c_unit < c_unit_end; ++c_unit) {
-        // Parked steps one after another in straight code, their activations' LDS reads ahead of them: picked out of the registers by a
-        // switch, step by step, they took 0.37 us each.
-        const bool ring_steps = n_parked < c_wpt;
-        c_j = n_parked;
-#pragma unroll
-        for (int i = 0; i < PARKN; ++i)
-            if (i < n_parked) multiply(park[i], i);
-        n_parked = 0;
-        for (; c_j < c_wpt; ++c_j) {
+        for (c_j = 0; c_j < c_wpt; ++c_j) {
         u32x4 cur[TP];
+        from_park = park_rd < n_parked;
+        if (from_park) {
+            switch (park_rd) {
+#define GPTRS_PARK(k) case k: _Pragma("unroll") for (int p = 0; p < TP; ++p) cur[p] = park[k < PARKN ? k : 0][p]; break;
+                GPTRS_PARK(0) GPTRS_PARK(1)
+                default: _Pragma("unroll") for (int p = 0; p < TP; ++p) cur[p] = park[PARKN - 1][p]; break;
+#undef GPTRS_PARK
+            }
+            static_assert(PARK >= 1 && PARK <= 3 && PARK_W4 >= 1 && PARK_W4 <= 3 && PARK_W8 >= 1 && PARK_W8 <= 3, "cases above");
+            ++park_rd;
+        } else {
         const GPTRS_LDS u32x4* wp = mine + slot * (SLOT_BYTES / 16);
         // the loads of this j-step are the oldest in flight: they have landed once no more than the younger ones remain
         {
@@ -1761,8 +1691,83 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
         for (int p = 0; p < TP; ++p) cur[p] = wp[p * NS];
         --inflight;
         if (++slot == RING_D) slot = 0;
-        multiply(cur, c_j);
-        if (c_j + 1 < c_wpt && r_more) request();   // (the unit's last step: after the hand-over below; a parked step's slot was refilled when it was parked)
+        }
+        if ((c_j + 1) * NS > c_Kv) {   // the stream's last step: lanes whose words are padding count as zeros
+            if (c_j * NS + t >= c_Kv) {
+#pragma unroll
+                for (int p = 0; p < TP; ++p) { cur[p].x = 0u; cur[p].y = 0u; cur[p].z = 0u; cur[p].w = 0u; }
+            }
+        }
+        // element reads go through scalars: __builtin_bit_cast applied directly to `vec.y` of an
+        // ext-vector reads element 0 with this compiler
+        if (c_fmt == kChainW16) {
+            const bf16x2 xv = __builtin_bit_cast(bf16x2, xs[c_j * NS + t]);
+#pragma unroll
+            for (int p = 0; p < TP; ++p) {
+                const unsigned q0 = cur[p].x, q1 = cur[p].y, q2 = cur[p].z, q3 = cur[p].w;
+                acc[p][0] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q0), xv, acc[p][0], false);
+                acc[p][1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q1), xv, acc[p][1], false);
+                acc[p][2] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q2), xv, acc[p][2], false);
+                acc[p][3] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q3), xv, acc[p][3], false);
+            }
+        } else if (c_fmt == kChainW32) {
+            const float xv = __uint_as_float(xs[c_j * NS + t]);
+#pragma unroll
+            for (int p = 0; p < TP; ++p) {
+                const unsigned q0 = cur[p].x, q1 = cur[p].y, q2 = cur[p].z, q3 = cur[p].w;
+                acc[p][0] = __builtin_fmaf(__uint_as_float(q0), xv, acc[p][0]);
+                acc[p][1] = __builtin_fmaf(__uint_as_float(q1), xv, acc[p][1]);
+                acc[p][2] = __builtin_fmaf(__uint_as_float(q2), xv, acc[p][2]);
+                acc[p][3] = __builtin_fmaf(__uint_as_float(q3), xv, acc[p][3]);
+            }
+        } else if (c_fmt == kChainW8) {
+            const u32x2 xw = *reinterpret_cast<const u32x2*>(&xs[2 * (c_j * NS + t)]);
+            const unsigned xa = xw.x, xb = xw.y;
+            const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
+            const float corr = -128.0f * ((x0 + x1) + (x2 + x3));
+#pragma unroll
+            for (int p = 0; p < TP; ++p) {
+                const unsigned q[4] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    float a = acc[p][c] + corr;
+                    a = __builtin_fmaf((float)(q[c] & 0xFFu), x0, a);
+                    a = __builtin_fmaf((float)((q[c] >> 8) & 0xFFu), x1, a);
+                    a = __builtin_fmaf((float)((q[c] >> 16) & 0xFFu), x2, a);
+                    a = __builtin_fmaf((float)(q[c] >> 24), x3, a);
+                    acc[p][c] = a;
+                }
+            }
+        } else {
+            const u32x4 xw = *reinterpret_cast<const u32x4*>(&xs[4 * (c_j * NS + t)]);
+            const unsigned xa = xw.x, xb = xw.y, xc = xw.z, xd = xw.w;
+            const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
+            const float x4 = bf16lo(xc), x5 = bf16hi(xc), x6 = bf16lo(xd), x7 = bf16hi(xd);
+            const float corr = -8.0f * (((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7)));
+#pragma unroll
+            for (int p = 0; p < TP; ++p) {
+                const unsigned q[4] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w};
+                const u32x2 sw = *reinterpret_cast<const u32x2*>(&xs[c_soff + 2 * (c_sidx + p * c_G + c_j * (NS / 16) + (t >> 4))]);
+                const unsigned sa = sw.x, sb = sw.y;
+                const float sc[4] = {bf16lo(sa), bf16hi(sa), bf16lo(sb), bf16hi(sb)};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    // byte i of a column's dword: k = 2i in the low nibble, k = 2i + 1 in the high one
+                    const unsigned lo = q[c] & 0x0F0F0F0Fu, hi = (q[c] >> 4) & 0x0F0F0F0Fu;
+                    float a = corr;
+                    a = __builtin_fmaf((float)(lo & 0xFFu), x0, a);
+                    a = __builtin_fmaf((float)(hi & 0xFFu), x1, a);
+                    a = __builtin_fmaf((float)((lo >> 8) & 0xFFu), x2, a);
+                    a = __builtin_fmaf((float)((hi >> 8) & 0xFFu), x3, a);
+                    a = __builtin_fmaf((float)((lo >> 16) & 0xFFu), x4, a);
+                    a = __builtin_fmaf((float)((hi >> 16) & 0xFFu), x5, a);
+                    a = __builtin_fmaf((float)(lo >> 24), x6, a);
+                    a = __builtin_fmaf((float)(hi >> 24), x7, a);
+                    acc[p][c] = __builtin_fmaf(sc[c], a, acc[p][c]);
+                }
+            }
+        }
+        if (!from_park && c_j + 1 < c_wpt && r_more) request();   // (the unit's last step: after the hand-over below; a parked step's slot was refilled when it was parked)
         }   // j-steps
         {
             const int hslot = ucount % NSLOT;
@@ -1791,7 +1796,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
             if (lane == 0) __hip_atomic_fetch_add(&sh.red_cnt[hslot], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             ++ucount;
             c_sidx += TP * c_G;
-            if (ring_steps && r_more) request();
+            if (!from_park && r_more) request();
         }
       }   // units
     }
