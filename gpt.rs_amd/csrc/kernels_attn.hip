@@ -774,41 +774,45 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const T* __restrict__
 // Both products are taken transposed so that a lane always owns ONE query (column lane % 32): the 16 scores a lane
 // holds belong to its query, the online-softmax state (running maximum and sum, in the log2 domain) is a per-lane
 // scalar, the rescaling of O^T is a per-lane multiply, and P^T needs no cross-lane movement to become the B operand:
-// the k-slots of the second product are simply numbered in the order the lane holds its keys, and V^T is written to
-// LDS in that order (key bits 2 and 3 swapped).
+// the k-slots of the second product are simply numbered in the order the lane holds its keys, and V^T is read out of V's rows in LDS in
+// that order by transposing reads.  (Writing V^T into LDS, two bytes at a time, took 16 stores a thread and tile and 53 KB of
+// it; without, three workgroups share a CU instead of two.  us a layer, 32 / 8 heads of 128: 4 x 2047 rows 234 -> 199, 1 x 4000 198 -> 176,
+// 8 x 1000 137 -> 120, 1 x 1024 37.0 -> 36.2.)
 // KG = 2: the workgroup has two groups of four waves; both serve the same queries, group g takes the key tiles
 // 2 s + g (it stages them itself, into its own LDS buffers), and the two online-softmax states meet through LDS at the
 // end.  A row tile then takes half as many steps, and a SIMD holds two waves whose matrix and vector phases overlap
 // (the launch has one wave-sized task per SIMD otherwise).
+// V^T as the A operand of a 32 x 32 x 16 product, out of 16 rows of V from v on (keys down, 32 d across): lane 32 h + c holds, of d = c, the
+// keys 4 h .. 4 h + 3 and 8 + 4 h .. 8 + 4 h + 3, the order in which the scores' lanes hold theirs.  Two transposing reads: lane i of 16 gets
+// column i of four rows, lane 4 e + j of the 16 names columns 4 j .. 4 j + 3 of row e.
+__device__ __forceinline__ bf16x8_v v_fragment(const bf16_t* v, int stride, int lane) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* lds_p;
+    const int c = lane & 15;
+    const bf16_t* p = v + (4 * (lane >> 5) + (c >> 2)) * stride + (lane & 16) + 4 * (c & 3);
+    const u32x2_m lo = __builtin_bit_cast(u32x2_m, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_p)(p)));
+    const u32x2_m hi = __builtin_bit_cast(u32x2_m, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_p)(p + 8 * stride)));
+    u32x4_m r;
+    r.x = lo.x; r.y = lo.y; r.z = hi.x; r.w = hi.y;
+    return __builtin_bit_cast(bf16x8_v, r);
+}
+
 template <int DH, int KG, bool FILL>
-__global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ ctx, int T,
+__global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ ctx, int T,
                                                                 int n_q, int n_kv, float scale_log2e, int zgroups, PrefillKv<bf16_t> kv) {
     constexpr int KT = 32;            // keys per tile
     constexpr int KS = DH + 8;        // K tile row stride in elements (16 bytes of padding)
-    // V^T rows: stride VS elements, row d starts 8 * ((d / 8) % 8) elements in.  Two access patterns must spread over
-    // the 32 banks: a fragment read (8 lanes = 8 consecutive rows, 16 bytes each) wants the row stride to be an odd
-    // multiple of 16 bytes modulo 128 (104 elements = 208 bytes: rows land 20 banks apart), and the scatter of one key's
-    // d-chunks (16 lanes, 8 rows apart, same position) would hit a single bank whatever the stride (8 rows are a
-    // multiple of 128 bytes apart), which the skew spreads over 8 groups of 4 banks.  Measured at 1024 tokens: no skew
-    // 88 us per layer, skew with 128-byte rows (reads 8-way conflicting) 68 us.
-    // Two key groups: rows of 88 elements (176 bytes: consecutive rows 44 banks apart, so the 8 rows of one d-chunk fall
-    // into 8 different groups of 4 banks, and a chunk's first row starts 32 banks from its neighbour's) and a skew of
-    // 16 bytes x (chunk / 2): the 16 chunks of one key then scatter into 16 different groups of 4 banks (with 72-element
-    // rows and 4 skews they shared 4, an 8-way conflict on every 2-byte store: 2.7 M conflict cycles per launch).
-    constexpr int VS = KG == 1 ? 104 : 88;
-    constexpr int SKEW = 7;
-    constexpr int SKSH = KG == 1 ? 0 : 1;     // the skew index is (chunk >> SKSH) & SKEW
+    constexpr int VS = DH + 16;       // V tile row stride: four rows of 16 d, which a transposing read takes at a time, lie in 32 different banks
     constexpr int ND = DH / 32;       // 32-row blocks of d in O^T
     constexpr int NK = DH / 16;       // k-steps of the score product
     constexpr int CH = KT * DH / 8;   // 16-byte chunks of a K (or V) tile
     constexpr int CPT = (CH + 255) / 256;
-    __shared__ __align__(16) bf16_t ksm_all[KG][2][KT * KS];
-    __shared__ __align__(16) bf16_t vsm_all[KG][2][DH * VS];
+    __shared__ __align__(16) bf16_t smem[KG * 2 * KT * (KS + VS)];
 
     const int kg = threadIdx.x / 256;                     // key group of this wave
     const int tid = threadIdx.x % 256, lane = tid & 63, wave = tid >> 6;
-    bf16_t (*ksm)[KT * KS] = ksm_all[kg];
-    bf16_t (*vsm)[DH * VS] = vsm_all[kg];
+    bf16_t (*ksm)[KT * KS] = reinterpret_cast<bf16_t (*)[KT * KS]>(smem + kg * 2 * KT * KS);
+    bf16_t (*vsm)[KT * VS] = reinterpret_cast<bf16_t (*)[KT * VS]>(smem + KG * 2 * KT * KS + kg * 2 * KT * VS);
     const int col = lane & 31, half = lane >> 5;
     const int G = n_q / n_kv;
     const int gw = G >= 4 ? 4 : G;                 // query heads of the group in this workgroup
@@ -894,13 +898,7 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
                     }
                 }
                 *reinterpret_cast<u32x4_s*>(&ksm[buf][r * KS + ch * 8]) = kreg[j];
-                // key r goes to k-slot position p: bits 2 and 3 of r swapped
-                const int pos = (r & 0x13) | ((r & 4) << 1) | ((r & 8) >> 1);
-                const uint32_t w0 = vreg[j].x, w1 = vreg[j].y, w2 = vreg[j].z, w3 = vreg[j].w;
-                const uint32_t w[4] = {w0, w1, w2, w3};
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    vsm[buf][(ch * 8 + e) * VS + 8 * ((ch >> SKSH) & SKEW) + pos] = (bf16_t)((w[e >> 1] >> ((e & 1) * 16)) & 0xFFFFu);
+                *reinterpret_cast<u32x4_s*>(&vsm[buf][r * VS + ch * 8]) = vreg[j];
             }
         }
     };
@@ -973,7 +971,7 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
             for (int db = 0; db < ND; ++db) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    const bf16x8_v vf = *reinterpret_cast<const bf16x8_v*>(&vsm[buf][(db * 32 + col) * VS + 8 * (((db * 4 + (col >> 3)) >> SKSH) & SKEW) + 16 * i + 8 * half]);
+                    const bf16x8_v vf = v_fragment(&vsm[buf][16 * i * VS + db * 32], VS, lane);
                     acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pb[i], acc_o[db], 0, 0, 0);
                 }
             }
@@ -985,8 +983,8 @@ __global__ __launch_bounds__(256 * KG, 2 / KG) void attn_prefill_mfma_kernel(con
         // merge the two groups' states: O = O0 c0 + O1 c1, l = l0 c0 + l1 c1 with c_g = 2^(m_g - max(m0, m1)); a group
         // that saw no tile has m = -inf, l = 0, O = 0 and drops out.  The tiles in LDS are dead (the loop ended on a
         // barrier); the exchange area is 66 floats per lane of the second group.
-        float* xch = reinterpret_cast<float*>(&vsm_all[0][0][0]) + (wave * 64 + lane);
-        static_assert(KG == 1 || (ND * 16 + 2) * 256 * 4 <= (int)sizeof(vsm_all), "exchange area fits the V buffers");
+        float* xch = reinterpret_cast<float*>(smem) + (wave * 64 + lane);
+        static_assert(KG == 1 || (ND * 16 + 2) * 256 * 4 <= (int)sizeof(smem), "exchange area fits the tiles");
         if (kg == 1) {
 #pragma unroll
             for (int db = 0; db < ND; ++db)
