@@ -296,6 +296,7 @@ struct MfmaLinearArgs {
     int out_f32 = 0;   // bf16 only: y and residual are f32
     EpiExtra extra;    // unquantised only
     int lds_direct = 1;   // the LDS-direct kernel where it applies (0: the register-staged one)
+    const void* w = nullptr; const void* w2 = nullptr;   // split f32 weights: row-major [k, n], for sums that are not finite
     // an RMS norm of the f32 result, rounded to bf16, wanted next: the launch that adds the splits of a tile writes it along with y where it can,
     // and says so in *normed
     const void* norm_gamma = nullptr; void* norm_y = nullptr; float norm_inv_n = 0.f, norm_eps = 0.f; bool* normed = nullptr;
@@ -303,7 +304,8 @@ struct MfmaLinearArgs {
 size_t mfma_workspace_bytes(int dtype, int64_t m, int64_t k, int64_t n, bool dual, int quant);
 size_t mfma_weight_bytes(int dtype, int64_t k, int64_t n);
 void mfma_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int64_t k, int64_t n);
-// f32 weights as three bf16 planes, Ws[K/8][3][Npad][8]: what `wk` / `wk2` hold where mfma_takes_split_weights() says so
+// f32 weights as three bf16 planes, Ws[K/8][3][Npad][8]: what `wk` / `wk2` hold where mfma_takes_split_weights() says so; `w` / `w2` are then the
+// matrices themselves
 size_t mfma_split_bytes(int64_t k, int64_t n);
 void mfma_split_weights(hipStream_t s, const void* w, void* out, int64_t k, int64_t n);
 bool mfma_takes_split_weights(int dtype, int64_t m, int64_t k, int64_t n, int lds_direct);

@@ -972,20 +972,11 @@ void mfma_split_weights(hipStream_t s, const void* w, void* out, int64_t k, int6
     const int64_t npad = mfma_padded_n(n);
     split_weights_kernel<<<dim3((unsigned)cdiv(npad, 256), (unsigned)cdiv(k, 8)), 256, 0, s>>>((const float*)w, (bf16_t*)out, k, n, npad);
 }
-// What a sum that is not finite is formed from again: x[M, K] and the split weights.
 struct SplitOperands {
     const float* x; const bf16_t* wp; const bf16_t* wp2;
     int K, Npad;
+    const float* w; const float* w2;   // the same weights row-major, [K, N]
 };
-__device__ __forceinline__ float split_dot(const float* row, const bf16_t* w, int K, int Npad, int64_t col) {
-    float s = 0.f;
-#pragma unroll 1
-    for (int k = 0; k < K; ++k) {
-        const bf16_t* p = w + ((int64_t)(k >> 3) * 3 * Npad + col) * 8 + (k & 7);
-        s += row[k] * ((bf16_to_f32(p[0]) + bf16_to_f32(p[(int64_t)Npad * 8])) + bf16_to_f32(p[(int64_t)Npad * 16]));   // w again, exactly
-    }
-    return s;
-}
 __device__ __forceinline__ void split_rows8(const f32x4_t& r0, const f32x4_t& r1, bf16x8_t* out) {
     u32x4_t p[3];
 #pragma unroll
@@ -1158,6 +1149,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(int M, int 
         if constexpr (NST > 3)
             if (t + 2 < nt) tile_step(R2, t + 2);
     }
+    const int mw = m0 + wm * 32, nw = n0 + wn * 32 * TNO;              // the wave's first output
     float odd = 0.f;                                                   // a NaN once any sum is not finite
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
@@ -1165,7 +1157,48 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(int M, int 
 #pragma unroll
         for (int v = 0; v < 16; ++v) odd += acc[j][v] * 0.f;
     }
-    const int mw = m0 + wm * 32, nw = n0 + wn * 32 * TNO;              // the wave's first output
+    if (__any(!(odd == 0.f))) {
+        // Sums that are not finite are formed again over this workgroup's k, on the f32 cores: x and the row-major weights straight from memory, a lane's four k of
+        // every 8 in two chains as in gemm_tile_kernel.  All of the wave's fragments at once, so that a round trip to memory brings 16 k of each; rows and columns
+        // past the end repeat the last one.
+        const float* xr = of.x + (int64_t)(mw + r32 < M ? mw + r32 : M - 1) * K + 4 * fsel;
+        const float* wc[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = nw + (j % TNO) * 32 + r32;
+            wc[j] = (j >= TNO ? of.w2 : of.w) + (n < (int)epi.N ? n : (int)epi.N - 1);
+        }
+        f32x16_t sums[2][TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sums[0][j][v] = sums[1][j][v] = 0.f;
+#pragma unroll 1
+        for (int k0 = kt0 * BK; k0 < (kt0 + nt) * BK; k0 += 16) {
+            f32x4_t a[2];
+            float b[2][TN][4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                a[h] = *reinterpret_cast<const f32x4_t*>(xr + k0 + 8 * h);
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) b[h][j][e] = wc[j][(int64_t)(k0 + 8 * h + 4 * fsel + e) * epi.N];
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) sums[e >> 1][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[h][e], b[h][j][e], sums[e >> 1][j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            sums[0][j] += sums[1][j];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[j][v] = __builtin_isfinite(acc[j][v]) ? acc[j][v] : sums[0][j][v];
+        }
+    }
     const int r0 = 4 * fsel;                                           // value v of a lane: row 8 (v / 4) + r0 + v % 4, column r32
     if (splits > 1) {
         const int np = ((int)epi.N + 7) & ~7, width = DUAL ? 2 * np : np;
@@ -1184,22 +1217,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(int M, int 
     }
     constexpr int RSF = 32 * TNO + 4, CH = 4 * TNO, PASSES = CH / 2;   // as in gemm_tile_kernel
     float* area = reinterpret_cast<float*>(lds) + wave * (32 * RSF);
-    if (__any(!(odd == 0.f))) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            float* mine = area + lane;                                 // 16 x 64 floats, a fragment at a time; each lane its own column of it
-#pragma unroll
-            for (int v = 0; v < 16; ++v) mine[v * 64] = acc[j][v];
-            const int n = nw + (j % TNO) * 32 + r32;
-#pragma unroll 1
-            for (int v = 0; v < 16; ++v) {
-                const int m = mw + 8 * (v >> 2) + r0 + (v & 3);
-                if (m < M && n < (int)epi.N && !__builtin_isfinite(mine[v * 64])) mine[v * 64] = split_dot(of.x + (int64_t)m * K, j >= TNO ? of.wp2 : of.wp, K, Npad, n);
-            }
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[j][v] = mine[v * 64];
-        }
-    }
 #pragma unroll
     for (int j = 0; j < TNO; ++j) {
         if constexpr (DUAL) gemm_glu<16>(acc[j], acc[j + TNO], epi.extra.glu);
@@ -1217,8 +1234,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(int M, int 
 // Adds the partial sums of a launch whose tiles were split over k, in split order (the result does not depend on which
 // workgroup ended first), and finishes the outputs.  One thread per 8 outputs.  A launch of its own over the whole chip:
 // with the last workgroup of a tile adding them, 48 tiles of M = 333 kept 48 CUs busy reading while 208 waited.
-template <typename T, bool DUAL, bool SPLIT = false>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int M, int splits, TileEpilogue<T> epi, SplitOperands of) {
+template <typename T, bool DUAL>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int M, int splits, TileEpilogue<T> epi) {
     const int np = ((int)epi.N + 7) & ~7, chunks = np / 8, width = DUAL ? 2 * np : np;
     const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (id >= (int64_t)M * chunks) return;
@@ -1233,23 +1250,12 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
         *reinterpret_cast<f32x4_t*>(o) = a;
         *reinterpret_cast<f32x4_t*>(o + 4) = b;
     };
-    auto again = [&](float* p, const bf16_t* w) {   // SPLIT: gemm_split_kernel's sums
-        float odd = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) odd += p[e] * 0.f;
-        if (odd == 0.f) return;
-#pragma unroll 1
-        for (int e = 0; e < 8 && n + e < (int)epi.N; ++e)
-            if (!__builtin_isfinite(p[e])) p[e] = split_dot(of.x + m * of.K, w, of.K, of.Npad, n + e);
-    };
-    __shared__ __attribute__((aligned(16))) float rows[DUAL ? 2 : 1][256][12];   // finish8 reads its eight from LDS; each thread its own
-    float* o = rows[0][threadIdx.x];
+    __shared__ __attribute__((aligned(16))) float rows[256][12];   // finish8 reads its eight from LDS; each thread its own
+    float* o = rows[threadIdx.x];
     sum8(part + m * width + n, o);
-    if constexpr (SPLIT) again(o, of.wp);
-    if constexpr (DUAL) {
-        float* u = rows[1][threadIdx.x];
+    if (DUAL) {
+        float u[8];
         sum8(part + m * width + np + n, u);
-        if constexpr (SPLIT) again(u, of.wp2);
         gemm_glu<8>(o, u, epi.extra.glu);
     }
     gemm_finish8<T, false>(epi, m, n, o, nullptr);
@@ -1346,7 +1352,7 @@ static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
                                                                                    (const T*)a.scale, (const T*)a.scale2, epi);
     if constexpr (std::is_same<T, bf16_t>::value && !DUAL)
         if (splits > 1 && norm_fits(a)) return launch_reduce_norm(s, a, splits);
-    if (splits > 1) gemm_reduce_kernel<T, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi, SplitOperands{});
+    if (splits > 1) gemm_reduce_kernel<T, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
 }
 static size_t tile_part_bytes(int64_t m, int64_t n, bool dual, int splits) {
     return splits > 1 ? (size_t)splits * m * cdiv(n, 8) * 8 * (dual ? 2 : 1) * sizeof(float) : 0;
@@ -1458,9 +1464,9 @@ static void launch_split(hipStream_t s, const MfmaLinearArgs& a, int splits) {
     }
     const int64_t nt = cdiv(a.n, NREAL), mt = cdiv(a.m, BM);
     TileEpilogue<float> epi{(const float*)a.bias, a.residual, a.y, a.n, a.act, 0, a.extra};
-    const SplitOperands of{(const float*)a.x, (const bf16_t*)a.wk, (const bf16_t*)a.wk2, (int)a.k, (int)mfma_padded_n(a.n)};
+    const SplitOperands of{(const float*)a.x, (const bf16_t*)a.wk, (const bf16_t*)a.wk2, (int)a.k, (int)mfma_padded_n(a.n), (const float*)a.w, (const float*)a.w2};
     kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN, lds_bytes, s>>>((int)a.m, (int)nt, (int)mt, splits, (float*)a.part, of, epi);
-    if (splits > 1) gemm_reduce_kernel<float, DUAL, true><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi, of);
+    if (splits > 1) gemm_reduce_kernel<float, DUAL><<<(unsigned)cdiv(a.m * cdiv(a.n, 8), 256), 256, 0, s>>>((const float*)a.part, (int)a.m, splits, epi);
 }
 
 // Quantised: which tile converts the codes of which columns.  Every wave converts the B fragments it multiplies, 20 (int8) or

@@ -1194,7 +1194,13 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
                 ma.x = src_ptr(st, cx, 0);
                 ma.m = x.dims[0]; ma.k = x.dims[1]; ma.n = w.dims[1];
                 // quantised weights: the k-grouped copy holds the codes; the kernel applies the scales on the way into LDS
-                const int kind = k::mfma_takes_split_weights(ma.dtype, ma.m, ma.k, ma.n, ma.lds_direct) ? 12 : in.quant == 0 ? 1 : (in.quant == 1 ? 6 : 7);
+                const bool split = k::mfma_takes_split_weights(ma.dtype, ma.m, ma.k, ma.n, ma.lds_direct);
+                const int kind = split ? 12 : in.quant == 0 ? 1 : (in.quant == 1 ? 6 : 7);
+                auto row_major = [&](int input) -> const void* {   // read beside the split copy
+                    cx.be->ensure_resident(cx.input_bufs[input]);
+                    return cx.input_bufs[input]->ptr;
+                };
+                if (split) ma.w = row_major(st.tiled_w_input);
                 BufferP wk = cx.be->derived_weights(cx.input_bufs[st.tiled_w_input], kind, ldt, ma.k, ma.n);
                 BufferP wk2;
                 ma.wk = wk->ptr;
@@ -1204,6 +1210,7 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
                 if (in.act == 2) {
                     wk2 = cx.be->derived_weights(cx.input_bufs[st.tiled_w2_input], kind, ldt, ma.k, ma.n);
                     ma.wk2 = wk2->ptr;
+                    if (split) ma.w2 = row_major(st.tiled_w2_input);
                     if (in.quant) ma.scale2 = cx.input_bufs[st.tiled_s2_input]->ptr;
                 }
                 if (in.has_bias) ma.bias = src_ptr(st, cx, oi++);

@@ -1,9 +1,11 @@
 """The LDS-direct bf16 GEMM (kernels_mfma.hip, gemm_tile_kernel) at the edges of its tiles and splits over k: rows against
 float64 sums of the same bf16 values, every output against the register-staged kernel."""
+import time
+
 import numpy as np
 import pytest
 
-from parity import hip_run
+from parity import hip_run, to_bytes
 from gptrs_amd import functional as F
 from gptrs_amd.ptir import FunctionBuilder, Program, bf16_bits_to_f32, f32_to_bf16_bits
 
@@ -183,6 +185,36 @@ def test_f32_as_bf16_products_not_finite(hip, m, k, n):
     assert odd.sum() > 2 * n and np.isfinite(pair[clear]).all()
     gone = np.isnan(both)
     assert gone.any() and np.isnan(pair[gone & ~np.isneginf(s)]).all()      # (silu of an infinite negative gate: either zero or NaN)
+
+
+# such sums are formed again by whole fragments on the f32 cores: all of a layer's take 2.7 times the layer, one row's 2.6 (one lane a sum, a term after
+# another: 200 and 180 times)
+@pytest.mark.parametrize("m,k,n", [(2048, 768, 3072), (512, 3072, 768)])
+def test_f32_sums_not_finite_are_formed_again_quickly(hip, m, k, n):
+    rng = np.random.default_rng(m)
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    fb = FunctionBuilder("main", "F32")
+    fb.set_results([F.linear(fb.param("F32", [m, k]), fb.param("F32", [k, n]))])
+    p = Program(fb)
+    row, every = x.copy(), np.full_like(x, np.nan)
+    row[5, 7] = np.nan
+    weights = hip.materialize(p.param_specs[1], to_bytes(w, "F32"))
+
+    def us(rows):
+        args = [hip.materialize(p.param_specs[0], to_bytes(rows, "F32")), weights]
+        out, took = hip.to_numpy(hip.run_program(p, args)[0]), []
+        for _ in range(5):
+            hip.synchronize()
+            t = time.perf_counter()
+            for _ in range(8):
+                hip.run_program(p, args)
+            hip.synchronize()
+            took.append(time.perf_counter() - t)
+        return min(took) / 8 * 1e6, out
+
+    (plain, a), (one, b), (all_nan, c) = (us(rows) for rows in (x, row, every))
+    assert np.isnan(b[5]).all() and np.array_equal(np.delete(a, 5, 0), np.delete(b, 5, 0)) and np.isnan(c).all()
+    assert max(one, all_nan) <= 5 * plain, (plain, one, all_nan)
 
 
 # codes converted on the way to the matrix pipes: odd columns, one k tile pair, k tiles that split in the middle of an int4 group, rows
