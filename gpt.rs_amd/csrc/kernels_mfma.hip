@@ -925,19 +925,24 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* _
 
 // ---------------------------------------------------------------------------------------------------------------
 // f32 layers of more than 128 rows, on the bf16 matrix cores.  An f32 value is the sum of three bf16 values, a = a1 + a2 + a3 exactly (8 bits of
-// its 24 each, rounded to nearest, so |a2| <= 2^-8 |a| and |a3| <= 2^-17 |a|; the last bits of values under 2^-109 are lost), and a product is
+// its 24 each, rounded to nearest, so |a2| <= 2^-8 |a| and |a3| <= 2^-17 |a|), and a product is
 //   a b = a1 b1 + (a1 b2 + a2 b1) + (a2 b2 + a1 b3 + a3 b1) + what is left out: a2 b3 + a3 b2 + a3 b3 < 2^-23.9 |a b|,
 // six bf16 products, each exact in f32.  The bf16 cores are 16 times as fast as the f32 cores, so six cost 0.375 of one f32 product.
 //
 // Precision.  What is left out is 2^-27 of a product in the mean square, far below the roundings of the sum.  a1 b1 and the five small products are
 // summed apart (the small sum's roundings are 2^-8 of the large one's), and a sum of K terms is rounded about K / 8 times, where the f32
 // cores round it K / 2 times.  Distance from 64 bits over the result's norm, normal operands: K = 768 1.6e-7 (f32 cores, two chains of sums: 3.5e-7; all
-// six products in one chain: 4.2e-7), K = 3072 3.4e-7 (7.0e-7; 9.0e-7).  Infinities and NaN, and operands that round to infinity in bf16, leave a
-// sum that is not finite (a2 of an infinity is a NaN); such a sum is formed again, with one f32 product per term, before anything is made of it.
+// six products in one chain: 4.2e-7), K = 3072 3.4e-7 (7.0e-7; 9.0e-7).
+// Range.  bf16 has f32's exponents, so the second and third values of a small f32 value run out of them (below 2^-103 bits go, at 2^-120 eleven of 24
+// or more).  Both operands are therefore split times 2^24, where every bit of every f32 value, subnormals too, is a normal bf16 value's, and the sums are
+// divided by 2^48: powers of two, no rounding but a subnormal result's.  The eight multiplications more for a fragment's 8 values take 16 prompts of 512 through
+// GPT-2 small from 11.01 to 11.13 ms (the matrix cores would flush subnormal pieces: without the scale rows or weights of 2^-135 were multiplied as zeros).
+// Infinities, NaN, values from 2^104 on and sums from 2^80 on leave a scaled sum that is not finite (an infinity's second value is a NaN); such a sum is formed
+// again, on the f32 cores, before anything is made of it.
 //
 // The weights are split once, into Ws[K/8][plane][Npad][8] (6 bytes a weight); the rows are staged in f32 and every wave splits the fragments it
-// multiplies, 44 vector instructions for 8 values, so a wave takes one row of fragments and all of a large tile's columns: 256 x 96 in 8 waves of 32 x 96
-// (18 MFMAs per 44), two k-steps of 16 to a staged tile; 128 x 96 in 4, one k-step, two workgroups to a CU; and 64 x 64 in 4 waves of 32 x 32 for
+// multiplies, 52 vector instructions for 8 values, so a wave takes one row of fragments and all of a large tile's columns: 256 x 96 in 8 waves of 32 x 96
+// (18 MFMAs per 52), two k-steps of 16 to a staged tile; 128 x 96 in 4, one k-step, two workgroups to a CU; and 64 x 64 in 4 waves of 32 x 32 for
 // launches of few rows (two k-steps: one barrier for 12 MFMAs, not 6; K = 768 in one round 19 -> 14.5 us).
 // What bounds it: with the chip full, the matrix pipes at the clock that random operands allow (256 x 96 at M = 8192, K = 3072, N = 768: 218
 // TFLOP/s = 1310 of bf16, the rate of the bf16 tiles); with K = 768 the tile's first loads and its epilogue.  us, M = 8192, weights from memory, f32 cores
@@ -945,6 +950,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* _
 // M = 512, N = 2304 27 -> 21; 16 prompts of 512 through GPT-2 small 13.9 -> 10.7 ms.  Dropped: 64 x 64 per wave (88 vector
 // instructions per 24 MFMAs: 177 TFLOP/s against 193), 32 x 128 (the small products' own sums no longer fit the registers), fragments split a k tile
 // ahead of their use, a ring of six (no change).
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
 __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ w, bf16_t* __restrict__ out, int64_t K, int64_t N, int64_t Npad) {
     const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t kb = blockIdx.y;
@@ -953,16 +959,12 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restr
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int64_t kx = kb * 8 + i;
-        const float v = n < N && kx < K ? w[kx * N + n] : 0.f;
-        bf16_t p[3] = {f32_to_bf16(v), 0, 0};
-        if (__builtin_isfinite(v)) {
-            if (!__builtin_isfinite(bf16_to_f32(p[0]))) p[0] = (bf16_t)(__float_as_uint(v) >> 16);   // next to the largest f32: cut off instead
-            const float rest = v - bf16_to_f32(p[0]);
-            p[1] = f32_to_bf16(rest);
-            p[2] = f32_to_bf16(rest - bf16_to_f32(p[1]));
-        }
+        float v = n < N && kx < K ? w[kx * N + n] * kSplitScale : 0.f;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) r[q][i] = p[q];
+        for (int q = 0; q < 3; ++q) {
+            r[q][i] = f32_to_bf16(v);
+            v -= bf16_to_f32(r[q][i]);
+        }
     }
 #pragma unroll
     for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4*>(out + ((kb * 3 + q) * Npad + n) * 8) = *reinterpret_cast<const uint4*>(r[q]);
@@ -981,7 +983,7 @@ __device__ __forceinline__ void split_rows8(const f32x4_t& r0, const f32x4_t& r1
     u32x4_t p[3];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float lo = e < 2 ? r0[2 * e] : r1[2 * e - 4], hi = e < 2 ? r0[2 * e + 1] : r1[2 * e - 3];
+        float lo = (e < 2 ? r0[2 * e] : r1[2 * e - 4]) * kSplitScale, hi = (e < 2 ? r0[2 * e + 1] : r1[2 * e - 3]) * kSplitScale;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             p[q][e] = mfma_pack_bf16(lo, hi);
@@ -1150,12 +1152,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(int M, int 
             if (t + 2 < nt) tile_step(R2, t + 2);
     }
     const int mw = m0 + wm * 32, nw = n0 + wn * 32 * TNO;              // the wave's first output
-    float odd = 0.f;                                                   // a NaN once any sum is not finite
+    float odd = 0.f;                                                   // a NaN once any scaled sum is not finite
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         acc[j] += small[j];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) odd += acc[j][v] * 0.f;
+        for (int v = 0; v < 16; ++v) {
+            odd += acc[j][v] * 0.f;
+            acc[j][v] *= kSplitUnscale;
+        }
     }
     if (__any(!(odd == 0.f))) {
         // Sums that are not finite are formed again over this workgroup's k, on the f32 cores: x and the row-major weights straight from memory, a lane's four k of

@@ -161,6 +161,24 @@ def test_f32_as_bf16_products(hip, m, k, n, scale):
     assert far <= (1.2 + 3 / np.sqrt(s.size)) * 0.42 * 2.0 ** -24 * np.sqrt((k / 8 + 1) / 2 + 3)
 
 
+# rows and weights of any size: subnormal values and up to where the split kernel's scaled sums leave f32's range (from 2^80 on), which f32 products then form.
+# What f32 products hold, and no bits less
+@pytest.mark.parametrize("m,k,n", [(129, 96, 70), (300, 3072, 130), (1100, 768, 1500)])
+@pytest.mark.parametrize("sx,sw", [(-120, 0), (-112, 100), (-104, 0), (-140, 60), (0, -124), (90, -135), (-60, -50), (60, 0), (50, 40), (110, -100), (-90, 105)])
+def test_f32_as_bf16_products_of_any_size(hip, m, k, n, sx, sw):
+    rng = np.random.default_rng(m + 200 + sx)
+    x, w = (rng.uniform(0.5, 1, s).astype(np.float32) * rng.choice([-1, 1], s).astype(np.float32) for s in ((m, k), (k, n)))
+    x, w = np.ldexp(x, sx), np.ldexp(w, sw)
+    fb = FunctionBuilder("main", "F32")
+    fb.set_results([F.linear(fb.param("F32", [m, k]), fb.param("F32", [k, n]))])
+    rows = sorted({0, 31, 32, 63, 64, 127, 128, m // 2, m - 1})
+    got, x64, w64 = hip_run(hip, Program(fb), [x, w])[0][rows].astype(np.float64), x[rows].astype(np.float64), w.astype(np.float64)
+    s = x64 @ w64
+    assert (np.abs(got - s) <= 2 * (np.sqrt(k) + 1) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64)) + 2.0 ** -149).all()
+    # in the mean as two chains of f32 sums (see test_f32_sums_in_two_chains); the split kernel's sums are nearer
+    assert np.linalg.norm(got - s) <= (1.2 + 3 / np.sqrt(s.size)) * 0.42 * 2.0 ** -24 * np.sqrt(k / 4 + 3) * np.linalg.norm(s)
+
+
 # infinities, NaN and values that round to infinity in bf16: what f32 products give, whole tiles and splits, both matrices of a pair
 @pytest.mark.parametrize("m,k,n", [(129, 64, 40), (140, 3072, 100), (300, 96, 193), (2100, 64, 3000)])
 def test_f32_as_bf16_products_not_finite(hip, m, k, n):
