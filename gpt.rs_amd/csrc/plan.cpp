@@ -801,6 +801,7 @@ void Builder::build() {
     for (int s = 0; s < n_steps; ++s) {
         Step& st = plan.steps[s];
         auto place = [&](const Step& of) {
+            if (of.left_out) return;   // nothing is written
             for (int v : of.dst) {
                 RootStorage& rs = plan.storage[v];
                 if (rs.kind != Storage::Temp) continue;
@@ -814,7 +815,8 @@ void Builder::build() {
             st.scratch_off = ws_alloc(st.scratch_bytes);
             ws_free(st.scratch_off, st.scratch_bytes);
         }
-        for (int v : dying[s]) ws_free(plan.storage[v].offset, plan.storage[v].bytes);
+        for (int v : dying[s])
+            if (!plan.steps[def_step[v]].left_out) ws_free(plan.storage[v].offset, plan.storage[v].bytes);
     }
     plan.workspace_bytes = high;
 

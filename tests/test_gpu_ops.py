@@ -7,6 +7,7 @@ import pytest
 
 from parity import FunctionBuilder, Program, assert_close, check_program, hip_run, oracle_run, to_bytes
 from gptrs_amd import functional as F
+from gptrs_amd.backend import HipBackend
 from gptrs_amd.ptir import Tensor, bf16_bits_to_f32, f32_to_bf16_bits
 
 pytestmark = pytest.mark.gpu
@@ -755,3 +756,15 @@ def test_sum_of_two_gathers(hip, dt, rows, inner):
                 hip_run(hip, q, bad)
                 hip.synchronize()
     assert np.array_equal(hip_run(hip, p, [fa, ia, fb_, ib])[0], got)
+
+
+def test_gathers_left_out_take_no_memory():
+    be = HipBackend(0)
+    rows, inner = 8192, 768
+    specs = [("F32", [50, inner]), ("Si32", [rows]), ("F32", [9, inner]), ("Si32", [rows])]
+    p = prog(lambda fb, a, i, b, j: a.take(i) + b.take(j), specs)
+    args = [be.materialize(s, bytes(s.byte_len())) for s in p.param_specs]
+    before = be.counter("bytes_allocated")
+    out = be.run_program(p, args)
+    assert be.counter("bytes_allocated") - before < 1.5 * rows * inner * 4, "the sum alone"
+    del out
