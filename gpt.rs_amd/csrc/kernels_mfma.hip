@@ -1434,24 +1434,36 @@ static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
     return best;
 }
 
-// The split kernel's tiles and splits, fitted as above to measurements at M = 65 .. 8192 of GPT-2's layers (K = 768 with N = 768, 2304, 3072 and K = 3072, N = 768;
-// weights from memory, 1 to 8 splits; k tiles of 16): within 6 % rms, worst 16 %; over those 44 shapes the pick is 2.1 % slower than the best choice in
-// the mean.  Up to two rows of 64 x 64 tiles the f32 cores keep up on 4 bytes a weight instead of 6 (M = 128, us, f32 and split: 11.8 and 12.9, 9.8 and 10.0, 14.0 and
-// 13.4, K = 3072 15.1 and 14.6; M = 200: 16.2 and 15.3, 10.4 and 10.5, 17.2 and 15.7, 19.9 and 18.4).
+// Up to two rows of 64 x 64 tiles the f32 cores keep up on 4 bytes a weight instead of 6 (M = 128, us, f32 and split: K = 768 and N = 2304, 768, 3072 11.8 and 12.9, 9.8 and 10.0,
+// 14.0 and 13.4, K = 3072, N = 768 15.1 and 14.6; M = 200: 16.2 and 15.3, 10.4 and 10.5, 17.2 and 15.7, 19.9 and 18.4).
 static bool mfma_splits_f32(int64_t m) { return m > 128; }
-enum SplitTileId { kS256x96, kS128x96, kS64x64, kSTiles };
-static const TileCost kSplitCost[kSTiles] = {{256, 96, 256, 6.0, 0.576, 0.289, 2.6, 0.29}, {128, 96, 512, 4.9, 0.497, 0.186, 2.8, 0.33}, {64, 64, 512, 2.8, 0.203, 0.10, 4.1, 0.19}};
+// The split kernel's tiles and splits, by a cost fitted to measurements at M = 129 .. 8192 of 21 plain layers (K = 64 .. 5120, N = 256 .. 6144) and M = 129 .. 3000 of nine
+// pairs (K = 512 .. 4096, N = 768 .. 8192), 1 to 12 splits, weights from memory: rounds of workgroups, at one price where two share a CU and another
+// where each has one to itself, x (fixed + per k tile of 16) + what a k tile costs more with the chip full, and for a split the launch that adds them, by their bytes and their
+// number (a thread reads one after another).  What it picks is 0.7 % (plain, 233 shapes) and 0.3 % (pairs, 99) slower than the best measured choice in the mean, at most
+// 13 %.  (Fitted to four layers alone, and a pair, whose ring leaves room for one workgroup on a CU, priced as if there were two: 2.3 and 8.8 %, and layers of 200 to
+// 640 rows, K = N = 768, slower than f32 products.)  A plain layer of 64 x 64 tiles has two workgroups on a CU by its splits only where
+// each of them keeps 512 k (K = N = 768, us, 333 rows in 3 and in 6 splits 11.5 and 13.0, 640 rows in 2 and in 4 14.0 and 15.5); no split is under 160 k.
+struct SplitCost { int bm, bn, slots; double fixed, per_kt, alone_fixed, alone_per_kt, full_kt, split, split_mb, per_split; };
+enum SplitTileId { kS256x96, kS128x96, kS64x64, kSPair, kSTiles };   // a pair: 64 x 64 of each matrix
+static const SplitCost kSplitCost[kSTiles] = {
+    {256, 96, 256, 6.66, 0.473, 0.0, 0.0, 0.514, 4.14, 0.122, 0.254}, {128, 96, 512, 6.30, 0.558, 4.73, 0.439, 0.242, 4.33, 0.139, 0.225},
+    {64, 64, 512, 4.93, 0.295, 4.80, 0.180, 0.090, 2.94, 0.0, 0.131}, {64, 64, 256, 4.96, 0.180, 0.0, 0.0, 0.033, 3.02, 0.0, 0.248},
+};
 static TilePlan split_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t room = SIZE_MAX) {
-    TilePlan best{kS64x64, 1};
+    TilePlan best{dual ? kSPair : kS64x64, 1};
     double least = 1e300;
-    for (int t = dual ? kS64x64 : 0; t < kSTiles; ++t) {   // a pair: 64 x 64 of each matrix
-        const TileCost& c = kSplitCost[t];
+    for (int t = dual ? kSPair : 0; t < (dual ? kSTiles : kSPair); ++t) {
+        const SplitCost& c = kSplitCost[t];
         const int64_t tiles = cdiv(m, c.bm) * cdiv(n, c.bn);
         for (int sp : {1, 2, 3, 4, 6, 8, 12}) {
-            if (sp > 1 && (!splits_allowed() || k < 128 * sp || tiles * sp > 2 * c.slots || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+            if (sp > 1 && (!splits_allowed() || k < 160 * sp || tiles * sp > 1024 || tile_part_bytes(m, n, dual, sp) > std::min(room, kMostPart))) break;
+            if (sp > 1 && t == kS64x64 && tiles * sp > 256 && k < 512 * sp) break;
             const double kt = (dual ? 2.0 : 1.0) * (double)k / 16 / sp, wg = (double)(tiles * sp);
-            double us = (double)cdiv(tiles * sp, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * wg / 256;
-            if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6;
+            const int64_t last = tiles * sp % c.slots;
+            const bool alone = c.slots == 512 && last > 0 && last <= 256;   // in the last round
+            double us = (double)(cdiv(tiles * sp, c.slots) - alone) * (c.fixed + c.per_kt * kt) + alone * (c.alone_fixed + c.alone_per_kt * kt) + c.full_kt * kt * wg / 256;
+            if (sp > 1) us += c.split + c.split_mb * (double)tile_part_bytes(m, n, dual, sp) / 1e6 + c.per_split * sp;
             if (us < least) { least = us; best = {t, sp}; }
         }
     }

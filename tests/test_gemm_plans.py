@@ -48,3 +48,13 @@ def test_the_split_switch_reaches_every_type():
     out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, GPTRS_HIP_GEMM_TAILSPLIT="0"), cwd=os.path.dirname(os.path.abspath(__file__)),
                          stdout=subprocess.PIPE, text=True, check=True).stdout
     assert out.strip() == str([0] * len(sizes))
+
+
+# us, measured in this many splits and in those that a plan gave which took a pair for two workgroups to a CU and a second workgroup on a CU for nothing
+@pytest.mark.parametrize("m,k,n,dual,splits", [(333, 768, 768, False, 3),     # 11.5, in 6 13.0
+                                               (640, 768, 768, False, 2),     # 14.0, in 4 15.5
+                                               (200, 1024, 1024, False, 4),   # 12.7, in 8 14.1
+                                               (200, 768, 3072, True, 1),     # 26.1, in 2 32.9
+                                               (200, 1024, 2816, True, 1)])   # 31.9, in 2 38.7
+def test_f32_as_bf16_products_is_split_where_it_pays(m, k, n, dual, splits):
+    assert lib()[1](0, m, k, n, dual, 0) == (splits > 1) * splits * m * n * 4 * (1 + dual)

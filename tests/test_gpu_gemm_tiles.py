@@ -137,7 +137,7 @@ def f32_layers(hip, x, w, w2, bias, res):
 # f32 of more than 128 rows as six bf16 products (fewer: f32 products): rows around the tiles' 64, 128 and 256, columns around 64 and 96 and no multiples of 8, two k tiles,
 # fewer and more than the ring, whole and in splits.  `scale` takes the rows far from 1, up and down
 @pytest.mark.parametrize("m,k,n,scale", [(129, 32, 8, 1.0), (130, 96, 63, 1e18), (160, 3072, 97, 1.0), (191, 64, 193, 1.0), (193, 800, 770, 1e-29), (255, 768, 2304, 1.0), (511, 3072, 767, 1.0),
-                                         (700, 736, 3070, 1e-18), (1025, 1536, 1000, 1.0), (2047, 768, 3073, 1.0), (2305, 3104, 769, 1.0)])
+                                         (700, 736, 3070, 1e-18), (1025, 1536, 1000, 1.0), (1473, 768, 2309, 1.0), (2047, 768, 3073, 1.0), (2305, 3104, 769, 1.0)])
 def test_f32_as_bf16_products(hip, m, k, n, scale):
     rng = np.random.default_rng(m + k + n)
     x, w, w2 = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (k, n), (k, n)))
