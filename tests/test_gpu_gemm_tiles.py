@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from parity import hip_run, to_bytes
+from test_gemm_plans import lib
 from gptrs_amd import functional as F
 from gptrs_amd.ptir import FunctionBuilder, Program, bf16_bits_to_f32, f32_to_bf16_bits
 
@@ -66,8 +67,10 @@ def test_tiles_and_splits(hip, m, k, n):
         assert (np.abs(a - b) <= 2.0 ** -6 * np.maximum(np.abs(a), np.abs(b)) + 4e-4 * np.sqrt(k) / 16).all()
 
 
-# the same kernel in f32 (64 x 64 tiles): tile edges, columns that are no multiple of 8, one k tile, splits that do not divide k
-@pytest.mark.parametrize("m,k,n", [(17, 32, 8), (40, 768, 41), (63, 96, 130), (65, 3072, 768), (129, 800, 2307), (300, 4096, 192), (700, 256, 3072)])
+# the same kernel in f32, of up to 128 rows (64 x 64 tiles): tile edges, columns that are no multiple of 8, one k tile, k tiles that do not divide among
+# the splits (13 in 3, 25 in 6 and in 3, 35 in 6, 65 in 8, 97 in 4); three layers of more rows, which gemm_split_kernel takes, against the same bounds
+@pytest.mark.parametrize("m,k,n", [(17, 32, 8), (40, 768, 41), (63, 96, 130), (65, 3072, 768), (66, 416, 130), (97, 1120, 1290), (100, 2080, 1000), (127, 800, 2307), (128, 800, 700),
+                                   (128, 3104, 2000), (129, 800, 2307), (300, 4096, 192), (700, 256, 3072)])
 def test_f32_tiles_and_splits(hip, m, k, n):
     rng = np.random.default_rng(m + k + n)
     x, w, w2 = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (k, n), (k, n)))
@@ -109,14 +112,15 @@ def test_f32_tiles_and_splits(hip, m, k, n):
 def test_f32_sums_in_two_chains(hip):
     """An f32 rounding is off by 0.42 * 2^-24 of its value in the mean square (uniform over half an ulp, an ulp being 2^-23 to 2^-24 of it), and
     a chain of n terms of one size rounds partial sums of sqrt(i): sqrt(n / 2) of that over the sum's own sqrt(n).  Two chains of k / 2:
-    sqrt(k / 4).  A fifth is left for the sample of rows; one chain would be 1.41 times the value."""
-    m, k, n = 1500, 768, 3072
+    sqrt(k / 4).  A fifth is left for the sample of values; one chain would be 1.41 times the value.  128 rows are the most that f32 products take, and
+    this layer's tiles fill the chip without splits, which would be chains of their own."""
+    m, k, n = 128, 768, 8192
+    assert lib()[1](0, m, k, n, False, 0) == 0      # no partial sums
     rng = np.random.default_rng(11)
     x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
     fb = FunctionBuilder("main", "F32")
     fb.set_results([F.linear(fb.param("F32", [m, k]), fb.param("F32", [k, n]))])
-    rows = np.arange(0, m, 71)
-    got, want = hip_run(hip, Program(fb), [x, w])[0][rows], x[rows].astype(np.float64) @ w.astype(np.float64)
+    got, want = hip_run(hip, Program(fb), [x, w])[0], x.astype(np.float64) @ w.astype(np.float64)
     assert np.linalg.norm(got - want) <= 1.2 * 0.42 * 2.0 ** -24 * np.sqrt(k / 4) * np.linalg.norm(want)
 
 
