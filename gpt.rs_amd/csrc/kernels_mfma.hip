@@ -1564,8 +1564,8 @@ size_t mfma_int4_lds_bytes(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
     return p.tile < 0 ? 0 : (size_t)int4_lds_bytes(kQuantCost[dual][p.tile].bm, kQuantCost[dual][p.tile].bn, k, p.splits);
 }
 
-// The LDS-direct kernels' loads address a k tile with 32-bit offsets from one scalar base: 256 rows of x, 8 k-groups of
-// the padded weights (6 of the split ones).
+// The LDS-direct kernels' loads address a k tile with unsigned 32-bit offsets from one scalar base: 256 rows of x (K * 1024 bytes at most), and 8 k-groups of
+// 16 bytes of the padded weights, of the split ones 12 in a tile of two k-steps.  The bound is for the 8; the 12 stay under 1.5 * 2^31.
 static bool mfma_lds_direct_reach(int64_t k, int64_t n) { return k <= (1 << 21) && (uint64_t)mfma_padded_n(n) * 128 < (1ull << 31); }
 bool mfma_takes_split_weights(int dtype, int64_t m, int64_t k, int64_t n, int lds_direct) { return dtype == 0 && lds_direct != 0 && mfma_splits_f32(m) && mfma_lds_direct_reach(k, n); }
 

@@ -221,7 +221,8 @@ class Backend {
     // Quantised weights: kind 3 / 4: chain copies of int8 / int4 codes (src2: the partner's codes); kind 5:
     // chain copy of int4 group scales (src2: the partner's); kind 6 / 7: k-grouped copy of the int8 / int4
     // codes for the MFMA GEMM, which applies the scales itself; kind 8: k-grouped copy in tiles of 12 or 16 columns for batched decode
-    // (kernels_skinny.hip); kind 9 / 10: int8 / int4 codes in that tile order; kind 11: chain copy of f32 weights.
+    // (kernels_skinny.hip); kind 9 / 10: int8 / int4 codes in that tile order; kind 11: chain copy of f32 weights.  kind 12: f32 weights as three
+    // bf16 planes, k-grouped (kernels_mfma.hip, prompts of more than 128 rows; 6 bytes a weight, beside the 4 of kind 1 where a program has shorter prompts too).
     BufferP derived_weights(const BufferP& src, int kind, DType dtype, int64_t k, int64_t n, const BufferP& src2 = nullptr);
     void drop_derived_weights();
     // Row-major weights that a chain copy duplicates: evict_packed_sources frees those among `inputs` that `plan`
