@@ -389,35 +389,44 @@ void skinny_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int
 }
 // How a launch shares out the steps (words of codes) of a tile: waves per workgroup, requests of a wave, workgroups per tile.  Every layer
 // is one pass over its weights; what is left beside HBM's pace are a wave's waits for its answers (1 to 1.5 us each) and, with
-// several workgroups to a tile, their meeting (3 us).
-//   up to 8 rows     16 waves with two steps in flight while there is at most one tile per CU; beyond, 8 waves, two steps over tiles of 12
-//                    columns, four over tiles of 16 (8 rows, us: N = 6144 9.4, with 4 waves of four 9.7, 16 of one 10.2; N = 32768 34.8, 36.1, 33.8)
-//   9 to 16 rows     one step in flight: a step's 16 rows take more of the memory pipeline than its weights, and more requests only wait
-//                    for one another; 16 waves, 8 where several tiles of 12 columns share a CU (16 rows, us: K = 9216, N = 3072 14.6, 8
-//                    waves of three 16.5; pair of 9216 8 waves of one 22.1, of two 24.8, 16 of one 29.2; N = 32768 43.3, 8 of four 45.5;
-//                    f32 N = 50257 36.2 and 36.8)
-//   few tiles        split while the launch stays within one workgroup per CU and a wave keeps six steps (8 rows, us: f32 K = 3072, N = 768
-//                    8.5 -> 7.1, K = 12288 27.2 -> 12.1; bf16 K = 3072, N = 576, six steps already, 5.3, in two 5.7)
+// several workgroups to a tile, their meeting (3 us).  Fitted to 45 layers (K = 256 .. 14336, N = 512 .. 50257, f32 and bf16, plain and pairs, 2 to 16 rows, weights from
+// memory): of 711 that take over 8 us the rule's choice is 3.1 % from the best of 14 in the mean.  us:
+//   one tile per CU or less   plain layers 16 waves with two steps in flight, from 9 rows on one: a step's 16 rows take more of the memory pipeline than its
+//                    weights (16 rows, K = 9216, N = 3072 14.6, 8 waves of three 16.5).  Pairs, whose step is two requests and the rows', 8 waves of two (bf16, 12
+//                    rows, K = 4096, N = 1024 8.2, 16 of one 9.5); of f32 only over tiles of 16 columns, over those of 12 as plain ones
+//   tiles of 12 columns beyond   8 waves of two, from 9 rows on of one (8 rows, N = 6144 9.4, with 4 waves of four 9.7, 16 of one 10.2; 16 rows, pair of 9216 8 waves of one
+//                    22.1, of two 24.8, 16 of one 29.2)
+//   tiles of 16 columns, under three a CU   16 waves of two, from 9 rows on 8 of one (12 rows, bf16 pair of 11008 over K = 4096 29.6, 16 of one 36.9; f32 K = 2048, N = 8192
+//                    14.9 and 16.9); pairs of f32 16 of one (the same pair 67.3 and 62.3)
+//   three and more a CU   8 waves of two (8 rows, bf16, K = 512, N = 32000 8.5, 8 of four 11.0; 12 rows, pair of 50257 over K = 768 26.2, 16 of one 32.2); plain f32 up to
+//                    8 rows of four (2 rows, K = 3072, N = 14432 30.4 and 31.9); plain layers of 9 rows and more whose sums are long enough for 16 waves those, of one (12 rows,
+//                    K = 3072, N = 32768 40.4 and 37.1, K = 768, N = 50257 16.8 and 21.1)
+//   few tiles        split while the launch stays within one workgroup per CU and a wave keeps six steps, of a pair three (8 rows: f32 K = 3072, N = 768
+//                    8.5 -> 7.1, K = 12288 27.2 -> 12.1; bf16 K = 3072, N = 576, six steps already, 5.3, in two 5.7; 12 rows, pair K = 4096, N = 1024 11.9 -> 8.2)
 //   codes            16 waves to a tile up to one tile per CU, else 8, one word in flight (a wave also has to convert it)
 // Weights are read past the caches (nontemporal): 4-5 % of a layer whose weights come from memory.  Models that the 256 MB last-level cache
 // holds gain or lose: whole f32 decode steps of 2 to 16 rows, against plain loads, take 0-15 % less with 16 MB of weights (5 % more at 2
 // rows), 2-9 % more with 100 to 180 MB (13 % at 16 rows of three layers of 1024), the same with 210, up to 5 % less with 240 to 270 and 1-7 %
-// less from 300 MB on.  None takes longer than with the four waves and the splits that ran here before; one rule for all.
-struct SkinnyPlan { int nw, depth, ks; };
-static SkinnyPlan skinny_plan(int64_t m, int64_t steps, int64_t n, bool codes) {
+// less from 300 MB on.  One rule for all.
+SkinnyPlan skinny_plan(int dtype, int64_t m, int64_t steps, int64_t n, bool dual, bool codes) {
     const int64_t cols = codes ? 16 : skinny_cols(n), tiles = cdiv_s(n, cols);
     int ks = 1;
-    if (codes) while (tiles * ks < 96 && steps / (32 * ks) >= 3) ks *= 2;
-    else while (tiles * ks <= 128 && steps / (16 * ks) >= 12) ks *= 2;
-    if (codes) return {tiles <= 256 ? 16 : 8, 1, ks};
-    if (tiles <= 256) return {16, m > 8 ? 1 : 2, ks};
-    if (m > 8) return {cols == 12 ? 8 : 16, 1, 1};
-    return {8, cols == 12 ? 2 : 4, 1};
+    if (codes) {
+        while (tiles * ks < 96 && steps / (32 * ks) >= 3) ks *= 2;
+        return {tiles <= 256 ? 16 : 8, 1, ks};
+    }
+    while (tiles * ks <= 128 && steps / (16 * ks) >= (dual ? 6 : 12)) ks *= 2;
+    const int few = m > 8 ? 1 : 2;   // requests that the rows leave room for
+    if (tiles <= 256) return dual && (dtype == 2 || cols == 16) ? SkinnyPlan{8, 2, ks} : SkinnyPlan{16, few, ks};
+    if (cols == 12) return {8, few, 1};
+    if (tiles < 768) return m > 8 && !(dual && dtype == 0) ? SkinnyPlan{8, 1, 1} : SkinnyPlan{16, few, 1};
+    if (!dual && m > 8 && steps >= 64) return {16, 1, 1};
+    return {8, dtype == 0 && !dual && m <= 8 ? 4 : 2, 1};
 }
 static size_t skinny_part_bytes(int64_t n, bool dual, int cols, int ks) { return ks > 1 ? (size_t)cdiv_s(n, cols) * ks * (dual ? 2 : 1) * 256 * sizeof(float) : 0; }
 size_t skinny_workspace_bytes(int64_t k, int64_t n, bool dual) {
     // whichever of rows and codes splits more (f32 has the most steps), over the narrower tiles
-    return skinny_part_bytes(n, dual, 12, std::max(skinny_plan(1, k / 16, n, false).ks, skinny_plan(1, k / 64, n, true).ks));
+    return skinny_part_bytes(n, dual, 12, std::max(skinny_plan(0, 1, k / 16, n, dual, false).ks, skinny_plan(2, 1, k / 64, n, dual, true).ks));
 }
 bool skinny_quant_supported(int dtype, int64_t m, int64_t k, int64_t n, int qf) {
     if ((qf != 1 && qf != 2) || dtype != 2) return false;
@@ -437,7 +446,7 @@ void skinny_gemm(hipStream_t s, const SkinnyLinearArgs& a) {
     const bool dual = a.ws2 != nullptr;
     const int64_t steps = a.k / (a.quant == 1 ? 64 : a.quant == 2 ? 128 : a.dtype == 0 ? 16 : 32);
     const int cols = a.quant ? 16 : skinny_cols(a.n);
-    SkinnyPlan p = skinny_plan(a.m, steps, a.n, a.quant != 0);
+    SkinnyPlan p = skinny_plan(a.dtype, a.m, steps, a.n, dual, a.quant != 0);
     if (p.ks > 1 && (!a.part || !a.tickets || a.part_bytes < skinny_part_bytes(a.n, dual, cols, p.ks))) p.ks = 1;
     const dim3 grid((unsigned)cdiv_s(a.n, cols), (unsigned)p.ks);
     if (a.quant) {
@@ -466,14 +475,15 @@ void skinny_gemm(hipStream_t s, const SkinnyLinearArgs& a) {
         constexpr std::integral_constant<int, 8> I8{};
         constexpr std::integral_constant<int, 12> I12{};
         constexpr std::integral_constant<int, 16> I16{};
-        if (cols == 12) {
-            if (p.nw == 16) { if (p.depth == 1) go(type, pair, I16, I1, I12); else go(type, pair, I16, I2, I12); }
-            else { if (p.depth == 1) go(type, pair, I8, I1, I12); else go(type, pair, I8, I2, I12); }
-        } else {
-            if (p.depth == 1) go(type, pair, I16, I1, I16);
-            else if (p.nw == 16) go(type, pair, I16, I2, I16);
-            else go(type, pair, I8, I4, I16);
-        }
+        auto tile = [&](auto columns) {
+            if (p.nw == 16) { if (p.depth == 1) go(type, pair, I16, I1, columns); else go(type, pair, I16, I2, columns); }
+            else if (p.depth == 1) go(type, pair, I8, I1, columns);
+            else go(type, pair, I8, I2, columns);
+        };
+        if (cols == 12) return tile(I12);
+        if constexpr (std::is_same<decltype(type), float>::value && !decltype(pair)::value)
+            if (p.depth == 4) return go(type, pair, I8, I4, I16);
+        tile(I16);
     };
     auto types = [&](auto pair) { if (a.dtype == 0) shape(float(), pair); else shape(bf16_t(), pair); };
     if (dual) types(std::true_type{});

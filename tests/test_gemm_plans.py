@@ -58,3 +58,24 @@ def test_the_split_switch_reaches_every_type():
                                                (200, 1024, 2816, True, 1)])   # 31.9, in 2 38.7
 def test_f32_as_bf16_products_is_split_where_it_pays(m, k, n, dual, splits):
     assert lib()[1](0, m, k, n, dual, 0) == (splits > 1) * splits * m * n * 4 * (1 + dual)
+
+
+class SkinnyPlan(ctypes.Structure):
+    _fields_ = [("nw", ctypes.c_int), ("depth", ctypes.c_int), ("ks", ctypes.c_int)]
+
+
+# waves, requests of a wave and splits of layers of 2 to 16 rows where they were measured (us, and with the choice made before)
+@pytest.mark.parametrize("f32,m,k,n,dual,want", [(0, 12, 4096, 11008, True, (8, 1, 1)),    # 29.6, 16 waves of one 36.9
+                                                 (0, 12, 768, 50257, True, (8, 2, 1)),     # 26.2, 16 of one 32.2
+                                                 (0, 8, 512, 32000, False, (8, 2, 1)),     # 8.5, 8 of four 11.0
+                                                 (0, 12, 4096, 1024, True, (8, 2, 2)),     # 8.2, 16 of one, unsplit 11.9
+                                                 (1, 12, 2048, 8192, False, (8, 1, 1)),    # 14.9, 16 of one 16.9
+                                                 (1, 8, 3072, 576, True, (16, 2, 4)),      # 8.7, in two 10.7
+                                                 (1, 12, 4096, 11008, True, (16, 1, 1)),   # 62.3, 8 of one 67.3
+                                                 (0, 12, 3072, 32768, False, (16, 1, 1)),  # 37.1, 8 of two 40.4
+                                                 (0, 8, 9216, 3072, False, (16, 2, 1)), (1, 8, 3072, 768, False, (16, 2, 2)), (1, 7, 768, 50257, False, (8, 4, 1))])
+def test_layers_of_few_rows(f32, m, k, n, dual, want):
+    plan = backend.load_library()._ZN5gptrs1k11skinny_planEilllbb
+    plan.argtypes, plan.restype = [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_bool] * 2, SkinnyPlan
+    p = plan(0 if f32 else 2, m, k // (16 if f32 else 32), n, dual, False)
+    assert (p.nw, p.depth, p.ks) == want

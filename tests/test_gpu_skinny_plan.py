@@ -21,7 +21,9 @@ def bounds(x, w, dtype):
 
 SIZES = [(2, 32, 16), (3, 96, 130), (7, 3072, 40), (16, 1568, 700), (8, 9216, 304), (5, 288, 4096), (16, 544, 4112), (9, 160, 12272), (4, 192, 12304),
          # tiles of 12 columns: one to a CU, a last tile of 4, two to a CU; splits of 12 steps and more
-         (8, 96, 3072), (9, 64, 3064), (16, 224, 6144), (3, 352, 4108), (2, 12288, 36)]
+         (8, 96, 3072), (9, 64, 3064), (16, 224, 6144), (3, 352, 4108), (2, 12288, 36),
+         # tiles of 16 columns, two to a CU with up to 8 rows, and four with more
+         (6, 160, 8190), (13, 96, 12304)]
 
 
 @pytest.mark.parametrize("dtype", ["Bf16", "F32"])
