@@ -176,6 +176,7 @@ size_t skinny_workspace_bytes(int64_t k, int64_t n, bool dual);
 // waves of a workgroup, requests of a wave, workgroups of a tile; steps: of 16 (f32) or 32 k, words of codes
 struct SkinnyPlan { int nw, depth, ks; };
 SkinnyPlan skinny_plan(int dtype, int64_t m, int64_t steps, int64_t n, bool dual, bool codes);
+int skinny_pair_workgroups(int quant);
 bool skinny_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n);
 size_t skinny_weight_bytes(int dtype, int64_t k, int64_t n);
 void skinny_pack_weights(hipStream_t s, int dtype, const void* w, void* out, int64_t k, int64_t n);

@@ -262,9 +262,10 @@ __device__ __forceinline__ bf16x8_s nibbles_to_bf16(uint32_t w) {
                          (float)((lo >> 16) & 0xFFu), (float)((hi >> 16) & 0xFFu), (float)(lo >> 24), (float)(hi >> 24));
 }
 
-// QF 1: int8, per-column scales [N]; QF 2: int4 in groups of 128, scales [K/128, N].  A word covers KPW = 64 / 128 k.
+// QF 1: int8, per-column scales [N]; QF 2: int4 in groups of 128, scales [K/128, N].  A word covers KPW = 64 / 128 k.  Pairs in 8 waves, which wide layers take: three
+// workgroups to a CU (the compiler by itself uses 97 registers of int4's, room for two: K = 4096, N = 11008, 2 rows 19.2 us, this 15.0, 12 rows 23.0 and 16.8).
 template <int QF, bool DUAL, int NW, int U>
-__global__ __launch_bounds__(64 * NW) void skinny_gemm_quant_kernel(const bf16_t* __restrict__ x, const uint8_t* __restrict__ qs,
+__global__ __launch_bounds__(64 * NW, DUAL && NW == 8 ? 6 : 4) void skinny_gemm_quant_kernel(const bf16_t* __restrict__ x, const uint8_t* __restrict__ qs,
                                                                 const uint8_t* __restrict__ qs2, const bf16_t* __restrict__ sc,
                                                                 const bf16_t* __restrict__ sc2, const bf16_t* __restrict__ bias,
                                                                 const bf16_t* __restrict__ residual, bf16_t* __restrict__ y, int M, int K,
@@ -427,6 +428,12 @@ static size_t skinny_part_bytes(int64_t n, bool dual, int cols, int ks) { return
 size_t skinny_workspace_bytes(int64_t k, int64_t n, bool dual) {
     // whichever of rows and codes splits more (f32 has the most steps), over the narrower tiles
     return skinny_part_bytes(n, dual, 12, std::max(skinny_plan(0, 1, k / 16, n, dual, false).ks, skinny_plan(2, 1, k / 64, n, dual, true).ks));
+}
+// Workgroups of 8 waves of a pair of codes that fit a CU.
+int skinny_pair_workgroups(int quant) {
+    int n = 0;
+    const void* f = quant == 1 ? (const void*)skinny_gemm_quant_kernel<1, true, 8, 1> : (const void*)skinny_gemm_quant_kernel<2, true, 8, 1>;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, 512, 0) == hipSuccess ? n : -1;
 }
 bool skinny_quant_supported(int dtype, int64_t m, int64_t k, int64_t n, int qf) {
     if ((qf != 1 && qf != 2) || dtype != 2) return false;

@@ -6,7 +6,7 @@ import pytest
 
 from parity import hip_run
 from test_gpu_gemm_tiles import bf16, program
-from gptrs_amd import functional as F
+from gptrs_amd import backend, functional as F
 
 pytestmark = pytest.mark.gpu
 
@@ -66,3 +66,8 @@ def test_codes(hip, scheme, m, k, n):
     g = a / (1 + np.exp(-a))
     got = hip_run(hip, pair, [x, q, s, q2, s2])[0]
     assert (np.abs(got - g * b) <= 1.1 * ba * np.abs(b) + bb * np.abs(g) + 2.0 ** -7 * np.abs(g * b) + 1.1 * ba * bb + 1e-6).all()
+
+
+@pytest.mark.parametrize("quant", [1, 2])
+def test_pairs_of_codes_share_a_cu(hip, quant):
+    assert backend.load_library()._ZN5gptrs1k22skinny_pair_workgroupsEi(quant) >= 3
