@@ -944,10 +944,11 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* _
 // multiplies, 52 vector instructions for 8 values, so a wave takes one row of fragments and all of a large tile's columns: 256 x 96 in 8 waves of 32 x 96
 // (18 MFMAs per 52), two k-steps of 16 to a staged tile; 128 x 96 in 4, one k-step, two workgroups to a CU; and 64 x 64 in 4 waves of 32 x 32 for
 // launches of few rows (two k-steps: one barrier for 12 MFMAs, not 6; K = 768 in one round 19 -> 14.5 us).
-// What bounds it: with the chip full, the matrix pipes at the clock that random operands allow (256 x 96 at M = 8192, K = 3072, N = 768: 218
-// TFLOP/s = 1310 of bf16, the rate of the bf16 tiles); with K = 768 the tile's first loads and its epilogue.  us, M = 8192, weights from memory, f32 cores
-// and this: K = 768, N = 3072 288 -> 199, N = 2304 218 -> 151, N = 768 83 -> 51; K = 3072, N = 768 301 -> 177; M = 1000, K = 768, N = 3072 44 -> 35;
-// M = 512, N = 2304 27 -> 21; 16 prompts of 512 through GPT-2 small 13.9 -> 10.7 ms.  Dropped: 64 x 64 per wave (88 vector
+// What bounds it: with the chip full, the matrix pipes at the clock that random operands allow (256 x 96 at M = 8192, K = 3072, N = 768: 211
+// TFLOP/s = 1270 of bf16, the rate of the bf16 tiles); with K = 768 the tile's first loads and its epilogue.  us, programs of one layer, M = 8192, weights from memory, f32
+// cores and this: K = 768, N = 3072 291 -> 205, N = 2304 217 -> 154, N = 768 81 -> 52; K = 3072, N = 768 302 -> 183; M = 1000, K = 768, N = 3072 46 -> 41;
+// M = 512, N = 2304 29 -> 24.  Inside 16 prompts of 512 through GPT-2 small (14.07 -> 10.53 ms) the same layers take 241 (with GELU), 169 and, the last two in the
+// mean, 131.  Dropped: 64 x 64 per wave (88 vector
 // instructions per 24 MFMAs: 177 TFLOP/s against 193), 32 x 128 (the small products' own sums no longer fit the registers), fragments split a k tile
 // ahead of their use, a ring of six (no change).
 constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
@@ -1435,7 +1436,8 @@ static int tile_splits_f32(int64_t m, int64_t k, int64_t n, bool dual, size_t ro
 }
 
 // Up to two rows of 64 x 64 tiles the f32 cores keep up on 4 bytes a weight instead of 6 (M = 128, us, f32 and split: K = 768 and N = 2304, 768, 3072 11.8 and 12.9, 9.8 and 10.0,
-// 14.0 and 13.4, K = 3072, N = 768 15.1 and 14.6; M = 200: 16.2 and 15.3, 10.4 and 10.5, 17.2 and 15.7, 19.9 and 18.4).
+// 14.0 and 13.4, K = 3072, N = 768 15.1 and 14.6; M = 129: 14.1 and 14.0, 10.6 and 10.4, 17.4 and 16.8, 17.8 and 17.4; M = 200: 17.2 and 16.6,
+// 11.0 and 10.9, 18.1 and 17.7, 21.0 and 20.5).
 static bool mfma_splits_f32(int64_t m) { return m > 128; }
 // The split kernel's tiles and splits, by a cost fitted to measurements at M = 129 .. 8192 of 21 plain layers (K = 64 .. 5120, N = 256 .. 6144) and M = 129 .. 3000 of nine
 // pairs (K = 512 .. 4096, N = 768 .. 8192), 1 to 12 splits, weights from memory: rounds of workgroups, at one price where two share a CU and another

@@ -97,7 +97,7 @@ __device__ __forceinline__ float skinny_finish(float v, float v2, bool dual, int
 // c, so a wave's LDS reads meet no bank twice and a row's stores are neighbours.  What an output needs besides its sum is requested
 // before the first weight (the constructor) and has long arrived.  One output's code instead of four per lane of one wave, and no
 // round trip to memory at the end: 8 rows, us: K = 9216,
-// N = 3072 13.4 -> 12.8, N = 6144 9.9 -> 9.4, f32 K = 768, N = 768 4.7 -> 4.3; int4 pair of 9216 17 -> 12.
+// N = 3072 13.4 -> 12.8, N = 6144 9.9 -> 9.4, f32 K = 768, N = 768 4.7 -> 4.3; int4 pair of 9216 14.8 -> 12.8.
 template <typename T, bool DUAL, int NW, int COLS>
 struct SkinnyOut {
     static constexpr int NP = DUAL ? 2 : 1;
