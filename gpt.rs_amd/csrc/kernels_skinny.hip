@@ -161,13 +161,17 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const T* __restric
                                                           int out_f32, EpiExtra extra) {
     static_assert(COLS == 12 || COLS == 16, "columns of a tile");
     constexpr int KPC = SkinnyT<T>::KPC, KSTEP = 4 * KPC;
-    __shared__ float red[NW][DUAL ? 2 : 1][64][4];
+    // f32 over tiles of 16 columns, which 8 or 16 waves take by the rows: a wave of 8 adds its odd steps apart from its even ones, so that the sums are those of 16
+    // waves, in their order, as near to 64 bits.  R: with one request in flight the loop takes two steps at a time to tell them apart (16 rows, K = 2048, N = 8192
+    // 15.1 -> 15.4 us; over tiles of 12 columns, which 8 waves take whatever the rows, it would be 19.2 -> 21.1 for 12 rows of K = 3072, N = 4200).
+    constexpr int CH = std::is_same<T, float>::value && NW == 8 && COLS == 16 ? 2 : 1, R = CH > U ? CH : 1;
+    __shared__ float red[NW * CH][DUAL ? 2 : 1][64][4];
     __shared__ unsigned ticket;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));   // uniform: a matrix instruction does not look at the lane mask, so the tests of a step must be branches
     const int c = lane & 15, kg = lane >> 4;     // B: column c, k-group kg; A: row c, k-group kg
     const int tile = blockIdx.x;
-    SkinnyOut<T, DUAL, NW, COLS> out(tile, M, N, bias, residual, out_f32, extra.colscale);
+    SkinnyOut<T, DUAL, NW * CH, COLS> out(tile, M, N, bias, residual, out_f32, extra.colscale);
     const int ksplit = gridDim.y, ks = blockIdx.y;
     const int s_begin = (int)((int64_t)(K / KSTEP) * ks / ksplit), nsteps = (int)((int64_t)(K / KSTEP) * (ks + 1) / ksplit);
     const int bcol = c < COLS ? c : COLS - 1;    // columns beyond the tile re-read its last one; their sums are never stored
@@ -180,7 +184,9 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const T* __restric
     // A ring of U steps: a step's registers are asked to fetch the wave's next but U - 1 as soon as they have been multiplied, so
     // a wave has U - 1 or U requests on their way all the time.  (Rounds of U requests, all awaited before the next were made, left the memory
     // pipeline empty once a round: K = 9216, N = 3072, 8 rows 17.0 us; this 14.9, with tiles of 12 columns 11.8.)
-    f32x4_s acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
+    f32x4_s acc[CH], acc2[CH];
+#pragma unroll
+    for (int h = 0; h < CH; ++h) acc[h] = acc2[h] = f32x4_s{0.f, 0.f, 0.f, 0.f};
     u32x4_s b[U], b2[DUAL ? U : 1], a[U];
     auto fetch = [&](int u, int s) {
         b[u] = __builtin_nontemporal_load(bsrc + (int64_t)s * (4 * COLS));
@@ -190,23 +196,25 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const T* __restric
     if (s_begin + wave < nsteps) {
 #pragma unroll
         for (int u = 0; u < U; ++u) fetch(u, s_begin + wave + NW * u < nsteps ? s_begin + wave + NW * u : s_begin + wave);   // (a step past the end is not multiplied)
-        for (int s0 = s_begin + wave; s0 < nsteps; s0 += NW * U) {
+        for (int s0 = s_begin + wave; s0 < nsteps; s0 += NW * U * R) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int s = s0 + NW * u;
+            for (int i = 0; i < U * R; ++i) {
+                const int s = s0 + NW * i, u = i % U, h = i % CH;
                 if (s < nsteps) {
-                    acc = SkinnyT<T>::mma(a[u], b[u], acc);
-                    if (DUAL) acc2 = SkinnyT<T>::mma(a[u], b2[DUAL ? u : 0], acc2);
+                    acc[h] = SkinnyT<T>::mma(a[u], b[u], acc[h]);
+                    if (DUAL) acc2[h] = SkinnyT<T>::mma(a[u], b2[DUAL ? u : 0], acc2[h]);
                 }
                 if (s + NW * U < nsteps) fetch(u, s + NW * U);
             }
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        red[wave][0][lane][i] = acc[i];
-        if (DUAL) red[wave][DUAL ? 1 : 0][lane][i] = acc2[i];
-    }
+    for (int h = 0; h < CH; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            red[wave + NW * h][0][lane][i] = acc[h][i];
+            if (DUAL) red[wave + NW * h][DUAL ? 1 : 0][lane][i] = acc2[h][i];
+        }
     __syncthreads();
     float v[2];
     if (!out.sum(red, tile, part, tickets, &ticket, v)) return;

@@ -45,6 +45,15 @@ def test_plain_and_pair(hip, dtype, m, k, n):
     assert (np.abs(got[1] - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + (2.0 ** -7 if dtype == "Bf16" else 2.0 ** -20) * np.abs(g * t) + 1.1 * bs * bt + 1e-6).all()
 
 
+# f32 sums over tiles of 16 columns are those of 16 waves whatever the waves: rows by themselves (16 waves of two requests, 8 of four) and among 12 (8 of one, 16 of one)
+@pytest.mark.parametrize("k,n", [(1040, 8190), (1040, 12304), (2064, 8192)])
+def test_f32_sums_do_not_depend_on_the_waves(hip, k, n):
+    rng = np.random.default_rng(n)
+    x, w = rng.standard_normal((12, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    run = lambda rows: hip_run(hip, program([("F32", list(rows.shape)), ("F32", [k, n])], lambda a, b: [F.linear(a, b)]), [rows, w])[0]
+    assert np.array_equal(run(x)[:6], run(x[:6]))
+
+
 @pytest.mark.parametrize("scheme", ["w8", "w4g128"])
 @pytest.mark.parametrize("m,k,n", [(2, 128, 16), (7, 3072, 40), (16, 1664, 700), (8, 9216, 304), (5, 384, 4096), (16, 640, 4112), (9, 256, 12304)])
 def test_codes(hip, scheme, m, k, n):
