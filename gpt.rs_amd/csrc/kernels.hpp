@@ -228,7 +228,10 @@ struct ChainPhase {
     int kind, flags;
     const void* w; const void* x; const void* gamma; const void* bias; const void* residual;
     void* y;
-    int K, N, Kw, ntiles, wpt, units, upb, lds_bytes;
+    // C: words of a tile (1 KiB: 4 columns x 64 k-groups of the format).  Every workgroup has tlo tiles, the first trem one more.
+    // step_bytes: from one step of a wave to its next in the packed copy.  units: of an attention phase.
+    int K, N, C, tlo, trem, step_bytes, units, lds_bytes;
+    float inv_c;   // 1 / C
     float inv_n, eps;
     // quantised weights: wfmt 1 = int8 (16-byte word = 4 columns x 4 k, biased by 128; `scale`/`scale2` = the
     // per-column scale tensors of W and of the SwiGLU partner, as wscale/wscale2), wfmt 2 = int4 groups of 128 (word = 4 columns x 8 k,
@@ -263,7 +266,7 @@ void chain_unpack_weights(hipStream_t s, const void* packed, void* w, void* w2, 
 // int4 only: derived scale copy sc[tile][group][4] (bf16) from s [k/128, n] (and the partner's s2)
 size_t chain_scale_bytes(int64_t k, int64_t n, bool dual);
 void chain_pack_scales_w4(hipStream_t s, int dtype, const void* sc, const void* sc2, void* out, int64_t k, int64_t n);
-// fills K, N, Kw, ntiles, wpt, units, upb, lds_bytes, wfmt (and the dual flag); false when one workgroup would
+// fills K, N, C, tlo, trem, step_bytes, inv_c, lds_bytes, wfmt (and the dual flag); false when one workgroup would
 // own more bias/residual columns than the kernel stages
 bool chain_fill_phase(ChainPhase& p, int64_t k, int64_t n, bool dual, int wfmt = kChainW16);
 // Decode attention inside a chain: supported shapes, scratch for the per-chunk records, and the

@@ -5,20 +5,21 @@
 // every GEMV pays a launch gap, a cold start and a tail; here the whole run executes inside one
 // kernel of one workgroup per CU, phases separated by a grid-wide barrier:
 //
-//   * 8 compute waves per workgroup stream the workgroup's weight words from HBM straight into LDS
-//     (global_load_lds_dwordx4: no registers), each wave into a ring of its own (3 KiB per j-step: one 16-byte
-//     word per lane and tile of the unit), in the order they are consumed: phase by phase, unit by unit (TP
-//     tiles of 4 output columns for the whole of K), j-step by j-step.  Weights do not depend on activations,
-//     so a wave's requests run four or five j-steps ahead of its reads across unit AND phase boundaries: while the
-//     wave stands at the grid barrier, stages the next input or runs an attention phase, HBM keeps delivering
-//     the next phase's first words.  Loads of a wave return in order, so "j-step g has landed" is a wait on
-//     the count of loads in flight: a ring private to the wave needs no flags and no barrier.  The loop
-//     around a j-step is kept to a few dozen instructions (uniform bookkeeping in scalar registers, one vector
-//     add and clamp per request): with three waves per SIMD a longer loop body, not HBM, sets the pace.
-//   * the compute lanes read their words from the ring (lane t owns word t of each tile stream,
-//     Wc[tile][k/2][4 cols][2 k]) and issue v_dot2 (bf16 pairs) against the activation vector staged in LDS.
-//   * 1 control wave per workgroup sums the 8 waves' partial sums of a unit out of LDS, applies the
-//     epilogue (SwiGLU pair, bias, GELU, residual), stores through to memory, and runs the grid
+//   * A layer's output columns, in tiles of 4, are dealt evenly over the workgroups, and a workgroup's words (tile by tile, k by
+//     k; a word is 1 KiB, 16 bytes of each lane of a wave) evenly over its 8 compute waves, a run of consecutive words each:
+//     every wave finishes a phase at the same time, whatever K and N are.
+//   * The compute waves stream their words from HBM straight into LDS (global_load_lds_dwordx4: no registers), each wave into
+//     a ring of its own, three words (a step) at a time, in the order they are consumed, phase by phase.  Weights do not
+//     depend on activations, so a wave's requests run up to eight steps ahead of its reads across phase boundaries: while the
+//     wave stands at the grid barrier or stages the next input, HBM keeps delivering the next phase's first words.  Loads of a
+//     wave return in order, so "this step has landed" is a wait on the count of loads in flight: a ring private to the wave
+//     needs no flags and no barrier.  The packed copy holds the words in the order of their
+//     requests, step by step over all workgroups, so that what the whole chip asks for at one time is one run of memory: a
+//     head of 805 MB streams at 6.0 TB/s, where a run of its own for every workgroup streamed at 5.1.
+//   * The compute lanes read their words from the ring and multiply them by the activation vector staged in LDS (v_dot2 for
+//     bf16 pairs); at the end of a tile the wave leaves its part of the tile's 4 sums in LDS.
+//   * 1 control wave per workgroup adds the parts of a phase's tiles when all waves are done, a lane to each output column,
+//     applies the epilogue (SwiGLU pair, bias, GELU, residual), stores through to memory, and runs the grid
 //     barrier (16 striped arrival counters, one poll instruction).
 //   * Activations cross workgroups through agent-scope (sc1) loads and stores only, so no
 //     L2 write-back / invalidate is needed between phases; a phase's input vector is staged into
@@ -59,15 +60,21 @@ namespace {
 constexpr int NS = 512;          // compute threads
 constexpr int NT = NS + 64;      // + control wave: the threads that stage inputs and run attention phases
 constexpr int NWS = NS / 64;
-constexpr int TP = 3;            // tiles (of 4 columns) per unit
-constexpr int NSLOT = 4;         // unit hand-off slots between compute waves and control wave
+constexpr int SW = 3;            // words of a step: what a wave requests and consumes at a time
+constexpr int CW = 64;           // lanes, and 16-byte pieces, of a word
 constexpr int NC = kChainCounters;
 constexpr int EPI_MAX = 640;     // bias/residual values staged per workgroup and phase: N <= 160 * grid columns
 constexpr int MAXI = 8;          // 8-byte items per thread in the norm staging: K <= 4*MAXI*NT
-constexpr int SLOT_BYTES = TP * NS * 16;     // one j-step of a workgroup: a word per compute lane and tile
+constexpr int STEP_BYTES = SW * CW * 16;     // a step of a wave
+constexpr int SLOT_BYTES = NWS * STEP_BYTES; // ... of a workgroup
 constexpr int PARK_W4 = 1, PARK_W8 = 2;   // ... in the int4 and int8 kernels, whose step arithmetic and staging hold more registers (measured: one step more spills)
-constexpr int PARK = 3;             // j-steps a compute wave can hold in registers while it waits for a phase to open
-constexpr int RING_MIN = 4, RING_MAX = 5;    // j-steps a wave's ring holds (its requests run that far ahead of its reads): 5 where the staged activations leave room
+constexpr int PARK = 3;             // steps a compute wave can hold in registers while it waits for a phase to open
+constexpr int RING_MIN = 4, RING_MAX = 5;    // steps a wave's ring holds (its requests run that far ahead of its reads): 5 where the staged activations leave room
+// Steps a wave has in flight while it consumes a phase.  What is queued in a CU's memory pipeline stands in front of everything that
+// comes later, the control wave's stores, its arrival and its polls of the barrier among it, and more than 48 KiB of a CU under way
+// do not make HBM faster: long phases (the head) stream 134 us with two steps, 143 with three, 147 with five; phases of few steps
+// are shorter with three (K = 9216, N = 3072: 10.7 us against 11.5), since the next phase's first steps are then under way.
+constexpr int FLIGHT = 3, FLIGHT_LONG = 2, LONG_WORDS = 10 * SW;
 constexpr int LDS_BYTES = 160 * 1024;        // per workgroup on gfx950
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -126,15 +133,14 @@ template <typename P> __device__ __forceinline__ void lds_st(P p, int v) { __hip
 #define GPTRS_LDS_ACQUIRE() __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local")
 
 struct alignas(16) Shared {
-    float red[NSLOT][NWS][16];
+    float part[EPI_MAX / 2 + NWS][4];   // sums of a tile's 4 columns over a wave's words: tile t of the workgroup by wave w in row t + w
     float epi_bias[EPI_MAX];
     float epi_res[EPI_MAX];
     // int8: [0, EPI_MAX) scale of each owned output column (gate of a SwiGLU pair), [EPI_MAX, 2 EPI_MAX) the pair's
     // up column.  (int4 group scales are staged behind the activations, see stage_block.)
     float epi_s[2 * EPI_MAX];
     float ssq[32];   // per-wave sums of the norm statistics (LayerNorm takes two rounds: [0, 16) and [16, 32))
-    int red_cnt[NSLOT];
-    int go, consumed, abort, pad;
+    int go, done, abort, pad;   // done: waves that have left their sums of a linear phase, counted over the launch
 };
 
 // The table of phases is read-only for the whole launch: reading it through the constant address space lets the
@@ -156,7 +162,7 @@ __device__ __forceinline__ void wg_barrier() {
 // one vector load (a lane per dword) before it waits for the grid barrier and picks the fields out of the lanes.  Either
 // way nothing is fetched between the barrier and the first use.
 struct PhaseRegs {
-    int K, N, Kw, ntiles, upb, units, lds_bytes, flags, wfmt;
+    int K, N, C, tlo, trem, lds_bytes, flags, wfmt;
     float inv_n, eps, glu_limit, glu_alpha, glu_shift;   // (the last three: control wave only)
     const void *x, *gamma, *beta, *bias, *residual, *wscale, *wscale2, *colscale;
     void* y;
@@ -167,7 +173,7 @@ struct PhaseRegs {
 // that nobody reads is not kept)
 template <bool LN, bool POST>
 __device__ __forceinline__ void regs_from_table(PhaseRegs& R, const GPTRS_CONST ChainPhase* D) {
-    R.K = uni(D->K); R.N = uni(D->N); R.Kw = uni(D->Kw); R.ntiles = uni(D->ntiles); R.upb = uni(D->upb); R.units = uni(D->units);
+    R.K = uni(D->K); R.N = uni(D->N); R.C = uni(D->C); R.tlo = uni(D->tlo); R.trem = uni(D->trem);
     R.lds_bytes = uni(D->lds_bytes); R.flags = uni(D->flags); R.wfmt = uni(D->wfmt);
     R.inv_n = __int_as_float(uni(__float_as_int(D->inv_n))); R.eps = __int_as_float(uni(__float_as_int(D->eps)));
     R.x = uni_ptr(D->x); R.gamma = uni_ptr(D->gamma); R.beta = LN ? uni_ptr(D->beta) : nullptr; R.bias = uni_ptr(D->bias); R.residual = uni_ptr(D->residual);
@@ -182,8 +188,8 @@ __device__ __forceinline__ void regs_from_table(PhaseRegs& R, const GPTRS_CONST 
                                           (unsigned)__builtin_amdgcn_readlane(pd, (int)(offsetof(ChainPhase, field) / 4))))
 template <bool LN, bool POST>
 __device__ __forceinline__ void regs_from_lanes(PhaseRegs& R, int pd) {   // pd: dword `lane` of the descriptor
-    R.K = GPTRS_PD_INT(K); R.N = GPTRS_PD_INT(N); R.Kw = GPTRS_PD_INT(Kw); R.ntiles = GPTRS_PD_INT(ntiles); R.upb = GPTRS_PD_INT(upb);
-    R.units = GPTRS_PD_INT(units); R.lds_bytes = GPTRS_PD_INT(lds_bytes); R.flags = GPTRS_PD_INT(flags); R.wfmt = GPTRS_PD_INT(wfmt);
+    R.K = GPTRS_PD_INT(K); R.N = GPTRS_PD_INT(N); R.C = GPTRS_PD_INT(C); R.tlo = GPTRS_PD_INT(tlo); R.trem = GPTRS_PD_INT(trem);
+    R.lds_bytes = GPTRS_PD_INT(lds_bytes); R.flags = GPTRS_PD_INT(flags); R.wfmt = GPTRS_PD_INT(wfmt);
     R.inv_n = __int_as_float(GPTRS_PD_INT(inv_n)); R.eps = __int_as_float(GPTRS_PD_INT(eps));
     R.x = GPTRS_PD_PTR(x); R.gamma = GPTRS_PD_PTR(gamma); R.beta = LN ? GPTRS_PD_PTR(beta) : nullptr; R.bias = GPTRS_PD_PTR(bias); R.residual = GPTRS_PD_PTR(residual);
     R.wscale = GPTRS_PD_PTR(wscale); R.wscale2 = GPTRS_PD_PTR(wscale2); R.y = const_cast<void*>(GPTRS_PD_PTR(y));
@@ -194,6 +200,13 @@ __device__ __forceinline__ void regs_from_lanes(PhaseRegs& R, int pd) {   // pd:
         R.post_mult = __int_as_float(GPTRS_PD_INT(post_mult)); R.post_eps = __int_as_float(GPTRS_PD_INT(post_eps));
     }
 }
+
+// The tiles of a workgroup: the first `trem` workgroups take one more than `tlo`.
+__device__ __forceinline__ int tile_first(int blk, int tlo, int trem) { return blk * tlo + min(blk, trem); }
+__device__ __forceinline__ int tile_count(int blk, int tlo, int trem) { return tlo + (blk < trem ? 1 : 0); }
+// The first of a wave's words among the W of its workgroup: words [wave_first(W, w), wave_first(W, w + 1)) are wave w's.
+__host__ __device__ __forceinline__ int wave_first(int W, int w) { return (W * w) >> 3; }   // (W < 2^22)
+static_assert(NWS == 8, "wave_first");
 
 // ---------------------------------------------------------------------------- staging (all waves)
 // xs[j] = (x[2j], x[2j+1]) as a bf16 pair, zero beyond K; with norm: the value the stand-alone
@@ -215,10 +228,9 @@ __device__ __forceinline__ float stage_block(const PhaseRegs& P, unsigned* xs, f
     uint2* sc_dst = reinterpret_cast<uint2*>(xs + 2 * npad);
     uint2 sv[SB];
     if (FMT == kChainW4) {   // (every linear phase of a launch has the kernel's weight format)
-        const int G = P.Kw >> 4, upb = P.upb;
-        const int t0 = (int)blockIdx.x * upb * TP, t1 = min(min(t0 + upb * TP, P.units * TP), P.ntiles);
-        sc_n = max(t1 - t0, 0) * G;
-        sc_src = (const uint2*)P.wscale + (long)t0 * G;
+        const int G = 4 * P.C;
+        sc_n = tile_count(blockIdx.x, P.tlo, P.trem) * G;
+        sc_src = (const uint2*)P.wscale + (long)tile_first(blockIdx.x, P.tlo, P.trem) * G;
 #pragma unroll
         for (int u = 0; u < SB; ++u) {
             const int i = u * NT + t;
@@ -1219,15 +1231,14 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
     const int lane = threadIdx.x & 63;
     const int blk = blockIdx.x, per = gridDim.x / NC;
     const unsigned epoch = gload(bar + NC * 64);   // written by the previous launch, stable during this one
-    int ucount = 0;
+    int handed = 0;   // arrivals of compute waves that the phases up to this one bring
     for (int ph = 0; ph < nphases; ++ph) {
         // the phase's descriptor is requested before the wait for the barrier and lands in LDS after it, ahead of `go`
         const int pd = lane < kPhaseDwords ? gload(reinterpret_cast<const int*>(phases + ph) + lane) : 0;
         const GPTRS_CONST ChainPhase* D = table + ph;
         const int kind = uni(D->kind);
-        const int upb = uni(D->upb), units = uni(D->units);
-        const int u0 = kind == kChainLinear ? blk * upb : 0;
-        const int u1 = kind == kChainLinear ? min(u0 + upb, units) : 0;
+        const int units = uni(D->units);
+        const int T = kind == kChainLinear ? tile_count(blk, uni(D->tlo), uni(D->trem)) : 0;
         if (ph > 0) {
             // stall_phase (a test hook, -1 otherwise): one arrival more than the grid can deliver is expected at that
             // phase, so this wait runs out of time and the give-up path below is taken
@@ -1252,15 +1263,15 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
                 if (lane == 0) lds_st(&sh.go, ph);
                 run_attn_phase<FMT == kChainW32>(table + ph, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.go, (GPTRS_LDS int*)&sh.abort, ph, budget);
             }
-        } else if (u0 < u1) {
+        } else if (T > 0) {
             if (lane == 0) lds_st(&sh.go, ph);
             PhaseRegs P;
             regs_from_lanes<FMT == kChainW32 || FMT == kChainW16, FMT == kChainW16>(P, pd);
-            const int flags = P.flags, ntiles = P.ntiles, N = P.N;
+            const int flags = P.flags, N = P.N;
             const bool dual = flags & kChainDual;
             const int cpt = dual ? 2 : 4;              // output columns per tile
-            const int col0 = u0 * TP * cpt;
-            const int ncols = min((u1 - u0) * TP * cpt, EPI_MAX);
+            const int col0 = tile_first(blk, P.tlo, P.trem) * cpt;
+            const int ncols = min(T * cpt, EPI_MAX);
             // bias / residual / int8 scales of this workgroup's columns: the first round is requested before the
             // staging loads and written to LDS after the staging, so that its latency hides behind the staging
             // instead of holding up the workgroup's barrier inside it
@@ -1321,7 +1332,7 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
                 post_g = gload((const float*)P.post_gain + i);
             };
             if (post_y) {
-                const int active = (units + upb - 1) / upb, share = (P.K + active - 1) / active;
+                const int active = P.tlo > 0 ? (int)gridDim.x : P.trem, share = (P.K + active - 1) / active;
                 post_i = blk * share + lane;
                 post_end = min(blk * share + share, P.K);
                 if (post_i < post_end) post_load(post_i);
@@ -1343,87 +1354,70 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
                 }
             }
             char* out = (char*)P.y;
-            for (int u = u0; u < u1; ++u, ++ucount) {
-                const int slot = ucount % NSLOT;
-                Patience pat(8 * budget);
-                while (lds_ld(&sh.red_cnt[slot]) < NWS) {
-                    __builtin_amdgcn_s_sleep(1);
-                    if (pat.spent()) {
-                        lds_st(&sh.abort, 1);
-                        __hip_atomic_store(as_global(abort_flag), 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        return;
-                    }
+            handed += NWS;
+            const int W = T * P.C;
+            // A lane's column i: tile i / cpt of the workgroup, whose parts lie in the rows of the waves that hold its words.  All it
+            // needs besides the sums is read ahead of the wait for them.
+            for (int i0 = 0; i0 < ncols; i0 += 64) {
+                const int i = min(i0 + lane, ncols - 1), col = col0 + i;
+                const int tl = dual ? i >> 1 : i >> 2, c = dual ? (i & 1) * 2 : i & 3;
+                int w0 = 0, w1 = 0;   // the waves of the tile's first and last word
+#pragma unroll
+                for (int w = 1; w < NWS; ++w) {
+                    const int f = wave_first(W, w);
+                    w0 += f <= tl * P.C ? 1 : 0;
+                    w1 += f <= tl * P.C + P.C - 1 ? 1 : 0;
                 }
-                GPTRS_LDS_ACQUIRE();
-                float s[4] = {0.f, 0.f, 0.f, 0.f};
-                if (lane < TP) {
-#pragma unroll
-                    for (int w = 0; w < NWS; ++w) {
-                        const float4 v = *reinterpret_cast<const float4*>(&sh.red[slot][w][lane * 4]);
-                        s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
+                const float sc = (wfmt == kChainW8 || cscale) ? sh.epi_s[i] : 1.f;
+                const float su2 = (wfmt == kChainW8 && dual) ? sh.epi_s[EPI_MAX + i] : 1.f;
+                const bool add = flags & (kChainBias | kChainResidual);   // both arrays are staged when either is present
+                const float bi = add ? sh.epi_bias[i] : 0.f, re = add ? sh.epi_res[i] : 0.f;
+                if (i0 == 0) {
+                    Patience pat(8 * budget);
+                    while (lds_ld(&sh.done) < handed) {
+                        __builtin_amdgcn_s_sleep(1);
+                        if (pat.spent()) {
+                            lds_st(&sh.abort, 1);
+                            __hip_atomic_store(as_global(abort_flag), 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            return;
+                        }
                     }
+                    GPTRS_LDS_ACQUIRE();
                 }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
-                if (lane == 0) { lds_st(&sh.red_cnt[slot], 0); lds_st(&sh.consumed, ucount + 1); }
-                const int tile = u * TP + lane;
-                if (lane < TP && tile < ntiles) {
-                    const int e = min(((u - u0) * TP + lane) * cpt, EPI_MAX - 4);
-                    // the staged values of the tile's columns in one round of LDS reads, and only those the phase has
-                    float sc[4] = {1.f, 1.f, 1.f, 1.f}, bi[4] = {0.f, 0.f, 0.f, 0.f}, re[4] = {0.f, 0.f, 0.f, 0.f};
-                    if (wfmt == kChainW8) {
-                        if (dual) {
-                            const float2 a = *reinterpret_cast<const float2*>(&sh.epi_s[e]), b = *reinterpret_cast<const float2*>(&sh.epi_s[EPI_MAX + e]);
-                            sc[0] = a.x; sc[1] = b.x; sc[2] = a.y; sc[3] = b.y;
-                        } else {
-                            const float4 a = *reinterpret_cast<const float4*>(&sh.epi_s[e]);
-                            sc[0] = a.x; sc[1] = a.y; sc[2] = a.z; sc[3] = a.w;
-                        }
-                    }
-                    if (cscale) {   // (never a pair)
-                        const float4 a = *reinterpret_cast<const float4*>(&sh.epi_s[e]);
-                        sc[0] = a.x; sc[1] = a.y; sc[2] = a.z; sc[3] = a.w;
-                    }
-                    if (flags & (kChainBias | kChainResidual)) {   // both arrays are staged when either is present
-                        if (dual) {
-                            const float2 b = *reinterpret_cast<const float2*>(&sh.epi_bias[e]), r = *reinterpret_cast<const float2*>(&sh.epi_res[e]);
-                            bi[0] = b.x; bi[1] = b.y; re[0] = r.x; re[1] = r.y;
-                        } else {
-                            const float4 b = *reinterpret_cast<const float4*>(&sh.epi_bias[e]), r = *reinterpret_cast<const float4*>(&sh.epi_res[e]);
-                            bi[0] = b.x; bi[1] = b.y; bi[2] = b.z; bi[3] = b.w;
-                            re[0] = r.x; re[1] = r.y; re[2] = r.z; re[3] = r.w;
-                        }
-                    }
-                    if (wfmt == kChainW8) {
+                float s = 0.f, s2 = 0.f;   // s2: the up column of a pair
+                auto parts = [&](int u) {
+                    const int w = min(w0 + u, w1);
+                    const float2 v = *reinterpret_cast<const float2*>(&sh.part[tl + w][c & 2]);
+                    return w0 + u <= w1 ? v : make_float2(0.f, 0.f);
+                };
+                auto take = [&](float2 v) {   // (selected as values: a choice between the two members' addresses would put them in scratch memory)
+                    const float vx = v.x, vy = v.y;
+                    s += (c & 1) ? vy : vx;   // (a pair's c is even)
+                    s2 += vy;
+                };
+                {
+                    const float2 a = parts(0), b = parts(1);
+                    take(a); take(b);
+                }
+                if (T < NWS) {   // (with as many tiles as waves a tile's words are in two waves at most)
+                    float2 v[NWS - 2];
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) s[c] *= sc[c];
-                    }
-                    if (dual) {   // columns interleaved (gate, up, gate, up): activation.rs:141-162
-                        const int kind = flags & kChainClampedGlu ? 1 : 0;
-                        const float a0 = finish(glu_combine(s[0], s[1], kind, P.glu_limit, P.glu_alpha, P.glu_shift), flags, bi[0], re[0], 1.0f);
-                        const float a1 = finish(glu_combine(s[2], s[3], kind, P.glu_limit, P.glu_alpha, P.glu_shift), flags, bi[1], re[1], 1.0f);
-                        cstore4(out + 2 * (size_t)(tile * 2), pack_hw(a0, a1));
-                    } else {
-                        float o[4];
+                    for (int u = 2; u < NWS; ++u) v[u - 2] = parts(u);
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) o[c] = finish(s[c], flags, bi[c], re[c], sc[c]);
-                        if (wfmt == kChainW16 && (flags & kChainSoftcap)) {
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) o[c] = softcap_f32(o[c], P.glu_limit);   // (softcap shares the field)
-                        }
-                        if (tile * 4 + 4 > N) {   // the last tile of a width that is not a multiple of 4: its real columns one by one
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) {
-                                if (tile * 4 + c >= N) continue;
-                                if (out_f32) cstore4(out + 4 * (size_t)(tile * 4 + c), __float_as_uint(o[c]));
-                                else __hip_atomic_store(as_global((unsigned short*)out + (size_t)(tile * 4 + c)), (unsigned short)pack_hw(o[c], 0.f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            }
-                        } else if (out_f32) {
-                            cstore8(out + 4 * (size_t)(tile * 4), (unsigned long long)__float_as_uint(o[0]) | ((unsigned long long)__float_as_uint(o[1]) << 32));
-                            cstore8(out + 4 * (size_t)(tile * 4) + 8, (unsigned long long)__float_as_uint(o[2]) | ((unsigned long long)__float_as_uint(o[3]) << 32));
-                        } else {
-                            cstore8(out + 2 * (size_t)(tile * 4), (unsigned long long)pack_hw(o[0], o[1]) | ((unsigned long long)pack_hw(o[2], o[3]) << 32));
-                        }
-                    }
+                    for (int u = 2; u < NWS; ++u) take(v[u - 2]);
+                }
+                if (wfmt == kChainW8) { s *= sc; s2 *= su2; }
+                float o;
+                if (dual) {   // columns interleaved (gate, up, gate, up): activation.rs:141-162
+                    const int glu = flags & kChainClampedGlu ? 1 : 0;
+                    o = finish(glu_combine(s, s2, glu, P.glu_limit, P.glu_alpha, P.glu_shift), flags, bi, re, 1.0f);
+                } else {
+                    o = finish(s, flags, bi, re, sc);
+                    if (wfmt == kChainW16 && (flags & kChainSoftcap)) o = softcap_f32(o, P.glu_limit);   // (softcap shares the field)
+                }
+                if (i0 + lane < ncols && col < N) {   // (the last tile of a width that is not a multiple of 4 has columns that do not exist)
+                    if (out_f32) cstore4(out + 4 * (size_t)col, __float_as_uint(o));
+                    else __hip_atomic_store(as_global((unsigned short*)out + (size_t)col), (unsigned short)pack_hw(o, 0.f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
         }
@@ -1436,48 +1430,36 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
     if (blk == 0 && lane == 0) gstore(bar + NC * 64, epoch + (unsigned)nphases * per);
 }
 
-// Sums each of a wave's 12 per-lane accumulators (3 tiles x 4 columns) over its 64 lanes as a
-// reduce-scatter: exchanging half of the values with lane ^ 32 and then lane ^ 16 leaves every 16-lane row
-// with 3 values already summed over 4 lanes, which 4 row-wide DPP steps finish: 30 cross-lane operations where
-// 12 separate wave sums take 120.  Returns in lanes 16r + s (s < 3) the total of accumulator 3r + s, i.e.
-// element 3r + s of acc[p][c] taken as acc[0][0..3], acc[1][0..3], acc[2][0..3].
-__device__ __forceinline__ float reduce_unit(const float (&acc)[TP][4], int lane) {
-    static_assert(TP == 3, "12 accumulators per lane");
-    float v[12];
+// Sums each of a wave's 4 per-lane accumulators over its 64 lanes as a reduce-scatter: exchanging half of the values with lane ^ 32
+// and then lane ^ 16 leaves every 16-lane row with one value already summed over 4 lanes, which 4 row-wide DPP steps finish.
+// Returns the total of accumulator r in every lane of row r.
+__device__ __forceinline__ float reduce_tile(const float (&acc)[4]) {
+    float h[2];
 #pragma unroll
-    for (int p = 0; p < TP; ++p)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) v[p * 4 + c] = acc[p][c];
-    float h[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {   // lanes < 32 keep values 0..5, lanes >= 32 values 6..11
-        const u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[k]), __float_as_uint(v[k + 6]), false, false);
+    for (int k = 0; k < 2; ++k) {   // lanes < 32 keep values 0 and 1, lanes >= 32 values 2 and 3
+        const u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[k]), __float_as_uint(acc[k + 2]), false, false);
         h[k] = __uint_as_float(sw.x) + __uint_as_float(sw.y);
     }
-    float q[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {   // even rows keep values k, odd rows values k + 3 of their half
-        const u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[k]), __float_as_uint(h[k + 3]), false, false);
-        q[k] = __uint_as_float(sw.x) + __uint_as_float(sw.y);
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        int x = __float_as_int(q[k]);
+    const u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[0]), __float_as_uint(h[1]), false, false);
+    int x = __float_as_int(__uint_as_float(sw.x) + __uint_as_float(sw.y));
 #define GPTRS_DPP_ADD(ctrl) x = __float_as_int(__int_as_float(x) + __int_as_float(__builtin_amdgcn_update_dpp(0, x, (ctrl), 0xf, 0xf, false)))
-        GPTRS_DPP_ADD(0xB1);    // quad_perm [1,0,3,2]
-        GPTRS_DPP_ADD(0x4E);    // quad_perm [2,3,0,1]
-        GPTRS_DPP_ADD(0x141);   // row_half_mirror
-        GPTRS_DPP_ADD(0x140);   // row_mirror
+    GPTRS_DPP_ADD(0xB1);    // quad_perm [1,0,3,2]
+    GPTRS_DPP_ADD(0x4E);    // quad_perm [2,3,0,1]
+    GPTRS_DPP_ADD(0x141);   // row_half_mirror
+    GPTRS_DPP_ADD(0x140);   // row_mirror
 #undef GPTRS_DPP_ADD
-        q[k] = __int_as_float(x);
-    }
-    const int sidx = lane & 15;
-    return sidx == 0 ? q[0] : (sidx == 1 ? q[1] : q[2]);
+    return __int_as_float(x);
 }
 
 // ---------------------------------------------------------------------------- compute waves
 // s_waitcnt that waits until at most 3 * steps vector memory operations of the wave are in flight (and for nothing else);
 // the count is an immediate of the instruction
+// vector memory operations of the wave that are in flight, without waiting
+__device__ __forceinline__ int vm_in_flight() {
+    unsigned v;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_IB_STS)" : "=s"(v) : : "memory");
+    return (int)((v & 15u) | ((v >> 18) & 0x30u));
+}
 template <int N> __device__ __forceinline__ void wait_vm_imm() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }
 __device__ __forceinline__ void wait_vm_count(int n) {   // steps without loads in flight (padding, tiles that do not exist): rare
     switch (n) {
@@ -1490,315 +1472,284 @@ __device__ __forceinline__ void wait_vm_count(int n) {   // steps without loads 
     static_assert(3 * (RING_MAX - 1) <= 12, "cases above");
 }
 
+// what a lane reads of the staged activations for one word: its k-group's bf16 values, or one f32
+template <int FMT> struct Act { typedef unsigned type; };
+template <> struct Act<kChainW8> { typedef u32x2 type; };
+template <> struct Act<kChainW4> { typedef u32x4 type; };
+
 template <int FMT, int RING_D>
 __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, int nphases, const unsigned char* ring, unsigned long long budget) {
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, wave = uni(t >> 6);
     const int blk = blockIdx.x;
-    constexpr int kpw = FMT == kChainW32 ? 1 : (FMT == kChainW16 ? 2 : (FMT == kChainW8 ? 4 : 8));
-    constexpr unsigned STEP = NS * 16;   // bytes of a tile stream per j-step
 
-    // ---- request side: the wave's next j-step to ask for, in the order the steps are consumed.  Everything but r_off is
-    // uniform: a request costs one vector add and clamp, three scalar moves and three loads.
-    int r_phase = -1, r_unit = 0, r_unit_end = 0, r_j = 0, r_wpt = 1, r_ntiles = 1;
-    unsigned r_last = 0;              // byte offset of a tile stream's last weight word
-    unsigned r_tile_bytes = 0;        // bytes of a tile stream
-    unsigned long long r_w = 0, r_base[TP] = {0, 0, 0};   // tile streams of the unit
-    unsigned r_off = 0;               // this lane's byte offset in a tile stream at step r_j
-    const unsigned ring_lds = (unsigned)uni((int)((unsigned)(size_t)(GPTRS_LDS unsigned char*)ring + (unsigned)(wave * 1024)));
-    const unsigned ring_end = ring_lds + RING_D * SLOT_BYTES;
-    unsigned r_dst = ring_lds;        // LDS address of lane 0's word of tile 0 in the next slot to fill
-    int inflight = 0;                 // j-steps requested and not yet read
+    // ---- request side: the wave's next step to ask for, in the order the steps are consumed.  Everything but the lane's offset
+    // in a word is uniform.
+    int r_phase = -1, r_left = 0;     // words of the phase that are still to be asked for
+    unsigned r_step_bytes = 0;
+    unsigned long long r_base = 0;    // the next step's first word
+    const unsigned lane_off = (unsigned)lane * 16u;
+    const unsigned ring_lds = (unsigned)uni((int)((unsigned)(size_t)(GPTRS_LDS unsigned char*)ring + (unsigned)(wave * (RING_D * STEP_BYTES))));
+    int r_slot = 0;                   // slot of the ring to fill next
+    int inflight = 0;                 // steps requested and not yet read
     unsigned pend = 0u;               // bits 2i, 2i + 1: loads that the i-th oldest of them carries
     int loads = 0;                    // loads in flight
-    int r_tiles = TP;                 // tiles of the unit that exist
-    bool r_plain = false;             // the unit has all its tiles and its streams end with a j-step
-    auto r_unit_setup = [&]() {
-        // a phase's last tiles may not exist: nothing is fetched for them
-        r_tiles = min(TP, r_ntiles - r_unit * TP);
-        r_plain = r_tiles == TP && r_last + 16u == (unsigned)r_wpt * STEP;
-#pragma unroll
-        for (int p = 0; p < TP; ++p) r_base[p] = r_w + (unsigned long long)(unsigned)min(r_unit * TP + p, r_ntiles - 1) * r_tile_bytes;
-        r_off = (unsigned)t * 16u;
-        r_j = 0;
-    };
-    auto r_seek = [&]() -> bool {   // next linear phase in which this workgroup has units
+    auto r_seek = [&]() -> bool {     // next linear phase in which this wave has words
         for (;;) {
             ++r_phase;
             if (r_phase >= nphases) return false;
             const GPTRS_CONST ChainPhase* D = table + r_phase;
             if (uni(D->kind) != kChainLinear) continue;
-            const int upb = uni(D->upb);
-            r_unit = blk * upb;
-            r_unit_end = min(r_unit + upb, uni(D->units));
-            if (r_unit >= r_unit_end) continue;
-            r_wpt = uni(D->wpt);
-            r_ntiles = uni(D->ntiles);
-            r_tile_bytes = (unsigned)uni(D->Kw) * 16u;
-            r_last = (unsigned)((uni(D->K) + kpw - 1) / kpw - 1) * 16u;
-            r_w = (unsigned long long)uni_ptr(D->w);
-            r_unit_setup();
+            const int W = tile_count(blk, uni(D->tlo), uni(D->trem)) * uni(D->C);
+            r_left = wave_first(W, wave + 1) - wave_first(W, wave);
+            if (r_left == 0) continue;
+            r_step_bytes = (unsigned)uni(D->step_bytes);
+            r_base = (unsigned long long)uni_ptr(D->w) + (unsigned)(blk * SLOT_BYTES + wave * STEP_BYTES);
             return true;
         }
     };
     bool r_more = r_seek();
-    // Asks for one j-step: one load per tile of the unit that exists (three but for a phase's last unit), none when all of
-    // the wave's words of the step are padding behind K (the reader counts such words as zeros, and sums of tiles that do
-    // not exist are never stored); `pend` records how many loads each step in flight carries, two bits per step, oldest
-    // first.  Every load that is issued fetches weights never fetched before, so all of them take the same way through
-    // the memory system and return in the order of issue: a load that re-read words already in a cache was seen to
-    // complete ahead of older ones, which a count of loads in flight cannot express.  Lanes behind K in a partly filled
-    // wave issue nothing.
+    // Asks for one step: a load per word that exists (three but for a phase's last step).  `pend` records how many loads each step
+    // in flight carries, two bits per step, oldest first.  Every load fetches words never fetched before, so all of them take the
+    // same way through the memory system and return in the order of issue: a load that re-read words already in a cache was seen
+    // to complete ahead of older ones, which a count of loads in flight cannot express.  A step's words lie one behind the other
+    // in memory and in LDS, and the instruction's offset counts for both addresses.
     auto request = [&]() {
-        int cnt = TP;
-        if (__builtin_expect(r_plain, 1)) {   // three tiles, no padding: nothing to decide
-#pragma unroll
-            for (int p = 0; p < TP; ++p)   // M0: LDS address of lane 0's word
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(r_off), "s"((unsigned long long)uni_ptr((const char*)r_base[p])), "s"((unsigned)uni((int)(r_dst + (unsigned)(p * NS * 16)))) : "memory", "m0");
+        const unsigned dst = (unsigned)uni((int)(ring_lds + (unsigned)(r_slot * STEP_BYTES)));
+        const unsigned long long base = (unsigned long long)uni_ptr((const char*)r_base);
+        int cnt = SW;
+        if (__builtin_expect(r_left >= SW, 1)) {
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\tglobal_load_lds_dwordx4 %0, %1 offset:2048"
+                         : : "v"(lane_off), "s"(base), "s"(dst) : "memory", "m0");
         } else {
-            const bool any = (unsigned)((r_j * NS + wave * 64) * 16) <= r_last;   // the wave's first word of the step holds weights
-            cnt = any ? r_tiles : 0;
-            if (any) {
-                if (r_off <= r_last) {
-#pragma unroll
-                    for (int p = 0; p < TP; ++p)
-                        if (p < r_tiles)
-                            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(r_off), "s"((unsigned long long)uni_ptr((const char*)r_base[p])), "s"((unsigned)uni((int)(r_dst + (unsigned)(p * NS * 16)))) : "memory", "m0");
-                }
-            }
+            cnt = r_left;
+            if (cnt == 2)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024"
+                             : : "v"(lane_off), "s"(base), "s"(dst) : "memory", "m0");
+            else
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "s"(dst) : "memory", "m0");
         }
+        static_assert(SW == 3 && CW * 16 == 1024, "offsets above");
         pend |= (unsigned)cnt << (2 * inflight);
         loads += cnt;
-        r_off += STEP;
-        r_dst += SLOT_BYTES;
-        if (r_dst == ring_end) r_dst = ring_lds;
         ++inflight;
-        if (++r_j == r_wpt) {
-            if (++r_unit < r_unit_end) r_unit_setup();
-            else r_more = r_seek();
-        }
+        if (++r_slot == RING_D) r_slot = 0;
+        r_base += r_step_bytes;
+        r_left -= cnt;
+        if (r_left == 0) r_more = r_seek();
     };
     for (int i = 0; i < RING_D && r_more; ++i) request();
 
     // ---- read side
-    int c_phase = -1, c_unit = 0, c_unit_end = 0, c_j = 0, c_wpt = 1, c_sidx = 0, c_G = 0, c_soff = 0, c_Kv = 0, ucount = 0;
-    int c_consumed = 0;   // units the control wave has taken, as last read
+    int c_phase = -1, c_left = 0, c_k = 0, c_C = 1, c_row = 0, c_soff = 0, c_stile = 0;
     constexpr int c_fmt = FMT;
     PhaseRegs R;
-    // advance to this workgroup's next linear unit, taking part in attention phases on the way
+    // advance to the next linear phase in which this workgroup has tiles, taking part in attention phases on the way
     auto c_seek = [&]() -> bool {
         for (;;) {
             ++c_phase;
             if (c_phase >= nphases) return false;
             const GPTRS_CONST ChainPhase* D = table + c_phase;   // the fields that decide this workgroup's part, before the wait
-            const int units = uni(D->units);
             if (uni(D->kind) != kChainLinear) {
-                if (blk >= units) continue;
+                if (blk >= uni(D->units)) continue;
                 if (!run_attn_phase<FMT == kChainW32>(table + c_phase, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.go, (GPTRS_LDS int*)&sh.abort, c_phase,
                                     budget)) return false;
                 continue;
             }
-            const int upb = uni(D->upb);
-            c_unit = blk * upb;
-            c_unit_end = min(c_unit + upb, units);
-            if (c_unit >= c_unit_end) continue;
-            c_wpt = uni(D->wpt);
-            c_G = uni(D->Kw) >> 4;
-            c_Kv = (uni(D->K) + kpw - 1) / kpw;
-            c_sidx = 0;   // int4: entry of the unit's first tile and group in the staged scales ...
-            c_soff = uni(D->lds_bytes) >> 2;   // ... which sit behind the activations
+            const int T = tile_count(blk, uni(D->tlo), uni(D->trem));
+            if (T == 0) continue;
+            c_C = uni(D->C);
+            const int W = T * c_C, f0 = wave_first(W, wave);
+            c_left = wave_first(W, wave + 1) - f0;
+            // tile and k of the wave's first word (f0 + 1/2 over C is at least 1 / (2 C) away from a whole number: exact below 2^22 words)
+            const int tl = uni((int)(((float)f0 + 0.5f) * __int_as_float(uni(__float_as_int(D->inv_c)))));
+            c_k = f0 - tl * c_C;
+            c_row = tl + wave;
+            c_stile = tl * c_C * 4;             // int4: the tile's first entry in the staged scales ...
+            c_soff = uni(D->lds_bytes) >> 2;    // ... which sit behind the activations
             regs_from_table<FMT == kChainW32 || FMT == kChainW16, FMT == kChainW16>(R, D);
             return true;   // (the caller waits for the phase to open and stages its input)
         }
     };
 
-    float acc[TP][4];
+    // two chains per column, words in turn: half as many additions behind one another
+    float acc[2][4];
 #pragma unroll
-    for (int p = 0; p < TP; ++p)
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[p][c] = 0.f;
     int slot = 0;
-    const GPTRS_LDS u32x4* mine = (const GPTRS_LDS u32x4*)ring + t;   // this lane's word of tile 0 in slot 0
+    const GPTRS_LDS u32x4* mine = (const GPTRS_LDS u32x4*)ring + wave * (RING_D * SW * CW) + lane;   // this lane's piece of word 0 in slot 0
+
+    // this lane's activations for word k of a tile
+    auto activations = [&](int k) -> typename Act<FMT>::type {
+        return *reinterpret_cast<const typename Act<FMT>::type*>(&xs[(k * CW + lane) * (int)(sizeof(typename Act<FMT>::type) / 4)]);
+    };
+    // word k of its tile times the staged activations
+    auto multiply = [&](const u32x4& q4, const typename Act<FMT>::type& act, int k, float (&a)[4]) {
+        // element reads go through scalars: __builtin_bit_cast applied directly to `vec.y` of an
+        // ext-vector reads element 0 with this compiler
+        const unsigned q[4] = {q4.x, q4.y, q4.z, q4.w};
+        if constexpr (c_fmt == kChainW16) {
+            const unsigned xw = act;
+            const bf16x2 xv = __builtin_bit_cast(bf16x2, xw);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) a[c] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q[c]), xv, a[c], false);
+        } else if constexpr (c_fmt == kChainW32) {
+            const float xv = __uint_as_float(act);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) a[c] = __builtin_fmaf(__uint_as_float(q[c]), xv, a[c]);
+        } else if constexpr (c_fmt == kChainW8) {
+            const unsigned xa = act.x, xb = act.y;
+            const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
+            const float corr = -128.0f * ((x0 + x1) + (x2 + x3));
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                float v = a[c] + corr;
+                v = __builtin_fmaf((float)(q[c] & 0xFFu), x0, v);
+                v = __builtin_fmaf((float)((q[c] >> 8) & 0xFFu), x1, v);
+                v = __builtin_fmaf((float)((q[c] >> 16) & 0xFFu), x2, v);
+                v = __builtin_fmaf((float)(q[c] >> 24), x3, v);
+                a[c] = v;
+            }
+        } else {
+            const unsigned xa = act.x, xb = act.y, xc = act.z, xd = act.w;
+            const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
+            const float x4 = bf16lo(xc), x5 = bf16hi(xc), x6 = bf16lo(xd), x7 = bf16hi(xd);
+            const float corr = -8.0f * (((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7)));
+            const u32x2 sw = *reinterpret_cast<const u32x2*>(&xs[c_soff + 2 * (c_stile + k * 4 + (lane >> 4))]);
+            const unsigned sa = sw.x, sb = sw.y;
+            const float sc[4] = {bf16lo(sa), bf16hi(sa), bf16lo(sb), bf16hi(sb)};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                // byte i of a column's dword: k = 2i in the low nibble, k = 2i + 1 in the high one
+                const unsigned lo = q[c] & 0x0F0F0F0Fu, hi = (q[c] >> 4) & 0x0F0F0F0Fu;
+                float v = corr;
+                v = __builtin_fmaf((float)(lo & 0xFFu), x0, v);
+                v = __builtin_fmaf((float)(hi & 0xFFu), x1, v);
+                v = __builtin_fmaf((float)((lo >> 8) & 0xFFu), x2, v);
+                v = __builtin_fmaf((float)((hi >> 8) & 0xFFu), x3, v);
+                v = __builtin_fmaf((float)((lo >> 16) & 0xFFu), x4, v);
+                v = __builtin_fmaf((float)((hi >> 16) & 0xFFu), x5, v);
+                v = __builtin_fmaf((float)(lo >> 24), x6, v);
+                v = __builtin_fmaf((float)(hi >> 24), x7, v);
+                a[c] = __builtin_fmaf(sc[c], v, a[c]);
+            }
+        }
+    };
+    auto leave_tile = [&]() {   // the wave's part of a tile's 4 sums
+        float sum[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { sum[c] = acc[0][c] + acc[1][c]; acc[0][c] = 0.f; acc[1][c] = 0.f; }
+        const float v = reduce_tile(sum);
+        if ((lane & 15) == 0) sh.part[c_row][lane >> 4] = v;
+        ++c_row;
+        c_stile += 4 * c_C;
+        c_k = 0;
+    };
 
     // A request can hold its wave for a microsecond (the memory pipeline of a CU takes a limited number of requests, and one
     // beyond that waits for an older one to land), so the request that a read frees is made after the step's arithmetic
-    // and, at the end of a unit, after the partial sums are handed over: nothing the workgroup waits for stands behind it.
-    // phases (rare code: seek, attention, staging) around units around j-steps (the loop that has to be tight)
-    bool alive = true;
-    while (alive && c_seek()) {
-      // Until the phase opens the wave has nothing to do, its ring is full, and whatever of it has landed cannot be used
-      // yet: the memory system would idle through the barrier.  So the oldest steps that have landed move from the ring
-      // into registers (`park`), and the slots they leave are asked to fetch further ahead: up to PARK more j-steps of
-      // weights are on their way while the grid synchronises.  Parked steps are the phase's first ones and are read
-      // back first; the registers are free again before the next phase is looked for.
+    // and, at the end of a phase, after the sums are handed over: nothing the workgroup waits for stands behind it.
+    while (c_seek()) {
+      // Until the phase opens the wave has nothing to do, and what has landed cannot be used yet: the memory system would idle
+      // through the barrier.  So the ring is filled up, and then the oldest steps move from the ring into registers (`park`) and
+      // the slots they leave are asked to fetch further ahead.  A step is only asked for when nothing of the wave is in flight:
+      // the pipeline that the control wave polls the barrier through stays short.  Parked steps are the phase's first ones and
+      // are read back first; the registers are free again before the next phase is looked for.
       constexpr int PARKN = FMT == kChainW4 ? PARK_W4 : (FMT == kChainW8 ? PARK_W8 : PARK);   // (the int4 kernel stages its group scales through registers as well)
-      u32x4 park[PARKN][TP];
+      u32x4 park[PARKN][SW];
       int n_parked = 0, park_rd = 0;
       {
-        const int want = min(PARKN, min(c_wpt * (c_unit_end - c_unit), inflight));
+        auto closed = [&]() { return uni(lds_ld(&sh.go)) < c_phase && !uni(lds_ld(&sh.abort)); };
+        while (r_more && inflight < RING_D && closed()) {
+            if (vm_in_flight() == 0) request(); else __builtin_amdgcn_s_sleep(1);
+        }
+        const int want = min(PARKN, min((c_left + SW - 1) / SW, inflight));
 #pragma unroll
         for (int i = 0; i < PARKN; ++i) {
-            if (i < want && uni(lds_ld(&sh.go)) < c_phase) {
-                const GPTRS_LDS u32x4* wp = mine + slot * (SLOT_BYTES / 16);
-                // The wave has time, so it waits for everything it has in flight rather than for this step alone: the request
-                // it makes below then meets an empty queue and returns at once, and the wave is back at the test of `go`
-                // instead of held in the memory pipeline behind its own older requests when the phase opens.
-                if (loads) wait_vm_imm<0>();
-                pend = 0u;
-                loads = 0;
-                asm volatile("" ::: "memory");
+            if (i < want) {
+                while (vm_in_flight() > 0 && closed()) __builtin_amdgcn_s_sleep(1);
+                if (vm_in_flight() == 0 && closed()) {
+                    pend = 0u;
+                    loads = 0;
+                    const GPTRS_LDS u32x4* wp = mine + slot * (SW * CW);
+                    asm volatile("" ::: "memory");
 #pragma unroll
-                for (int p = 0; p < TP; ++p) park[i][p] = wp[p * NS];
-                --inflight;
-                if (++slot == RING_D) slot = 0;
-                __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the words are in registers before their slot is asked to take new ones
-                asm volatile("" ::: "memory");
-                if (r_more) request();
-                n_parked = i + 1;
+                    for (int p = 0; p < SW; ++p) park[i][p] = wp[p * CW];
+                    --inflight;
+                    if (++slot == RING_D) slot = 0;
+                    __builtin_amdgcn_s_waitcnt(0xC07F);
+                    asm volatile("" ::: "memory");
+                    if (r_more) request();
+                    n_parked = i + 1;
+                } else break;
             }
         }
       }
       if (!wait_go(&sh.go, &sh.abort, c_phase, budget)) break;
       if (FMT == kChainW32) stage_block_f32(R, const_cast<unsigned*>(xs), sh.ssq);
       else stage_block<FMT>(R, const_cast<unsigned*>(xs), sh.ssq);
+      // Every load of the wave is older than the row it has just staged and has landed with it.  The compiler is told so here: left
+      // to itself it waited for all loads in flight at the top of each pass of the loop below.
+      wait_vm_imm<0>();
       bool from_park = false;
-      for (; c_unit < c_unit_end; ++c_unit) {
-        for (c_j = 0; c_j < c_wpt; ++c_j) {
-        u32x4 cur[TP];
+      while (c_left > 0) {
+        u32x4 cur[SW];
         from_park = park_rd < n_parked;
         if (from_park) {
             switch (park_rd) {
-#define GPTRS_PARK(k) case k: _Pragma("unroll") for (int p = 0; p < TP; ++p) cur[p] = park[k < PARKN ? k : 0][p]; break;
+#define GPTRS_PARK(k) case k: _Pragma("unroll") for (int p = 0; p < SW; ++p) cur[p] = park[k < PARKN ? k : 0][p]; break;
                 GPTRS_PARK(0) GPTRS_PARK(1)
-                default: _Pragma("unroll") for (int p = 0; p < TP; ++p) cur[p] = park[PARKN - 1][p]; break;
+                default: _Pragma("unroll") for (int p = 0; p < SW; ++p) cur[p] = park[PARKN - 1][p]; break;
 #undef GPTRS_PARK
             }
             static_assert(PARK >= 1 && PARK <= 3 && PARK_W4 >= 1 && PARK_W4 <= 3 && PARK_W8 >= 1 && PARK_W8 <= 3, "cases above");
             ++park_rd;
         } else {
-        const GPTRS_LDS u32x4* wp = mine + slot * (SLOT_BYTES / 16);
-        // the loads of this j-step are the oldest in flight: they have landed once no more than the younger ones remain
-        {
-            const int oldest = (int)(pend & 3u), younger = loads - oldest;
-            if (oldest) {
-                if (__builtin_expect(younger == 3 * (RING_D - 1), 1)) wait_vm_imm<3 * (RING_D - 1)>();
-                else wait_vm_count(younger);
-            }
-            pend >>= 2;
-            loads = younger;
-        }
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int p = 0; p < TP; ++p) cur[p] = wp[p * NS];
-        --inflight;
-        if (++slot == RING_D) slot = 0;
-        }
-        if ((c_j + 1) * NS > c_Kv) {   // the stream's last step: lanes whose words are padding count as zeros
-            if (c_j * NS + t >= c_Kv) {
-#pragma unroll
-                for (int p = 0; p < TP; ++p) { cur[p].x = 0u; cur[p].y = 0u; cur[p].z = 0u; cur[p].w = 0u; }
-            }
-        }
-        // element reads go through scalars: __builtin_bit_cast applied directly to `vec.y` of an
-        // ext-vector reads element 0 with this compiler
-        if (c_fmt == kChainW16) {
-            const bf16x2 xv = __builtin_bit_cast(bf16x2, xs[c_j * NS + t]);
-#pragma unroll
-            for (int p = 0; p < TP; ++p) {
-                const unsigned q0 = cur[p].x, q1 = cur[p].y, q2 = cur[p].z, q3 = cur[p].w;
-                acc[p][0] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q0), xv, acc[p][0], false);
-                acc[p][1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q1), xv, acc[p][1], false);
-                acc[p][2] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q2), xv, acc[p][2], false);
-                acc[p][3] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q3), xv, acc[p][3], false);
-            }
-        } else if (c_fmt == kChainW32) {
-            const float xv = __uint_as_float(xs[c_j * NS + t]);
-#pragma unroll
-            for (int p = 0; p < TP; ++p) {
-                const unsigned q0 = cur[p].x, q1 = cur[p].y, q2 = cur[p].z, q3 = cur[p].w;
-                acc[p][0] = __builtin_fmaf(__uint_as_float(q0), xv, acc[p][0]);
-                acc[p][1] = __builtin_fmaf(__uint_as_float(q1), xv, acc[p][1]);
-                acc[p][2] = __builtin_fmaf(__uint_as_float(q2), xv, acc[p][2]);
-                acc[p][3] = __builtin_fmaf(__uint_as_float(q3), xv, acc[p][3]);
-            }
-        } else if (c_fmt == kChainW8) {
-            const u32x2 xw = *reinterpret_cast<const u32x2*>(&xs[2 * (c_j * NS + t)]);
-            const unsigned xa = xw.x, xb = xw.y;
-            const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
-            const float corr = -128.0f * ((x0 + x1) + (x2 + x3));
-#pragma unroll
-            for (int p = 0; p < TP; ++p) {
-                const unsigned q[4] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w};
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    float a = acc[p][c] + corr;
-                    a = __builtin_fmaf((float)(q[c] & 0xFFu), x0, a);
-                    a = __builtin_fmaf((float)((q[c] >> 8) & 0xFFu), x1, a);
-                    a = __builtin_fmaf((float)((q[c] >> 16) & 0xFFu), x2, a);
-                    a = __builtin_fmaf((float)(q[c] >> 24), x3, a);
-                    acc[p][c] = a;
-                }
-            }
-        } else {
-            const u32x4 xw = *reinterpret_cast<const u32x4*>(&xs[4 * (c_j * NS + t)]);
-            const unsigned xa = xw.x, xb = xw.y, xc = xw.z, xd = xw.w;
-            const float x0 = bf16lo(xa), x1 = bf16hi(xa), x2 = bf16lo(xb), x3 = bf16hi(xb);
-            const float x4 = bf16lo(xc), x5 = bf16hi(xc), x6 = bf16lo(xd), x7 = bf16hi(xd);
-            const float corr = -8.0f * (((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7)));
-#pragma unroll
-            for (int p = 0; p < TP; ++p) {
-                const unsigned q[4] = {cur[p].x, cur[p].y, cur[p].z, cur[p].w};
-                const u32x2 sw = *reinterpret_cast<const u32x2*>(&xs[c_soff + 2 * (c_sidx + p * c_G + c_j * (NS / 16) + (t >> 4))]);
-                const unsigned sa = sw.x, sb = sw.y;
-                const float sc[4] = {bf16lo(sa), bf16hi(sa), bf16lo(sb), bf16hi(sb)};
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    // byte i of a column's dword: k = 2i in the low nibble, k = 2i + 1 in the high one
-                    const unsigned lo = q[c] & 0x0F0F0F0Fu, hi = (q[c] >> 4) & 0x0F0F0F0Fu;
-                    float a = corr;
-                    a = __builtin_fmaf((float)(lo & 0xFFu), x0, a);
-                    a = __builtin_fmaf((float)(hi & 0xFFu), x1, a);
-                    a = __builtin_fmaf((float)((lo >> 8) & 0xFFu), x2, a);
-                    a = __builtin_fmaf((float)((hi >> 8) & 0xFFu), x3, a);
-                    a = __builtin_fmaf((float)((lo >> 16) & 0xFFu), x4, a);
-                    a = __builtin_fmaf((float)((hi >> 16) & 0xFFu), x5, a);
-                    a = __builtin_fmaf((float)(lo >> 24), x6, a);
-                    a = __builtin_fmaf((float)(hi >> 24), x7, a);
-                    acc[p][c] = __builtin_fmaf(sc[c], a, acc[p][c]);
-                }
-            }
-        }
-        if (!from_park && c_j + 1 < c_wpt && r_more) request();   // (the unit's last step: after the hand-over below; a parked step's slot was refilled when it was parked)
-        }   // j-steps
-        {
-            const int hslot = ucount % NSLOT;
-            const float v = reduce_unit(acc, lane);
-#pragma unroll
-            for (int p = 0; p < TP; ++p)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc[p][c] = 0.f;
-            // the hand-over slot is free once the control wave has taken the unit that used it last; its count only
-            // grows, so the LDS read is skipped while the last value seen says enough
-            if (c_consumed < ucount - NSLOT + 1) {
-                Patience pat(8 * budget);
-                while ((c_consumed = uni(lds_ld(&sh.consumed))) < ucount - NSLOT + 1) {
-                    __builtin_amdgcn_s_sleep(1);
-                    if (uni(lds_ld(&sh.abort)) || pat.spent()) { alive = false; break; }
-                }
-                if (!alive) break;
-            }
+            const GPTRS_LDS u32x4* wp = mine + slot * (SW * CW);
+            // the loads of this step are the oldest in flight: they have landed once no more than the younger ones remain
             {
-                // (index recomputed here: as a loop invariant it was kept in a register that the allocator spilled, and its
-                // reload waits for every load in flight)
-                const int t2 = local_tid(), l2 = t2 & 63;
-                if ((l2 & 15) < 3) sh.red[hslot][t2 >> 6][3 * (l2 >> 4) + (l2 & 15)] = v;
+                const int oldest = (int)(pend & 3u), younger = loads - oldest;
+                if (oldest) {
+                    if (__builtin_expect(younger == SW * (FLIGHT_LONG - 1), 1)) wait_vm_imm<SW * (FLIGHT_LONG - 1)>();
+                    else if (__builtin_expect(younger == SW * (FLIGHT - 1), 1)) wait_vm_imm<SW * (FLIGHT - 1)>();
+                    else if (__builtin_expect(younger == 0, 1)) wait_vm_imm<0>();
+                    else wait_vm_count(younger);
+                }
+                pend >>= 2;
+                loads = younger;
             }
-            GPTRS_LDS_RELEASE();
-            if (lane == 0) __hip_atomic_fetch_add(&sh.red_cnt[hslot], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            ++ucount;
-            c_sidx += TP * c_G;
-            if (!from_park && r_more) request();
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int p = 0; p < SW; ++p) cur[p] = wp[p * CW];
+            --inflight;
+            if (++slot == RING_D) slot = 0;
         }
-      }   // units
+        if (__builtin_expect(c_left >= SW && c_k + SW <= c_C, 1)) {   // three words of one tile
+            typename Act<FMT>::type x[SW];
+#pragma unroll
+            for (int p = 0; p < SW; ++p) x[p] = activations(c_k + p);
+#pragma unroll
+            for (int p = 0; p < SW; ++p) multiply(cur[p], x[p], c_k + p, acc[p & 1]);
+            c_k += SW;
+            c_left -= SW;
+            if (c_k == c_C) leave_tile();
+        } else {
+#pragma unroll
+            for (int p = 0; p < SW; ++p) {
+                if (c_left > 0) {
+                    multiply(cur[p], activations(c_k), c_k, acc[p & 1]);
+                    --c_left;
+                    if (++c_k == c_C) leave_tile();
+                }
+            }
+        }
+        if (c_left > 0 && r_more && inflight < (c_left > LONG_WORDS ? FLIGHT_LONG : FLIGHT)) request();   // (a parked step's slot was refilled when it was parked)
+      }
+      if (c_k > 0) leave_tile();
+      GPTRS_LDS_RELEASE();
+      if (lane == 0) __hip_atomic_fetch_add(&sh.done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (!from_park && r_more && inflight < FLIGHT) request();
     }
 }
 
@@ -1811,8 +1762,7 @@ __global__ __launch_bounds__(NT, 1) void chain_kernel(const ChainPhase* __restri
     unsigned char* ring = smem + sizeof(Shared) + xs_bytes;
     PhaseTable table = (PhaseTable)phases;
     {
-        if (threadIdx.x < NSLOT) sh.red_cnt[threadIdx.x] = 0;
-        if (threadIdx.x == 0) { sh.go = -1; sh.consumed = 0; sh.abort = 0; }
+        if (threadIdx.x == 0) { sh.go = -1; sh.done = 0; sh.abort = 0; }
         __syncthreads();
     }
     const int wave = threadIdx.x >> 6;
@@ -1825,74 +1775,96 @@ __global__ __launch_bounds__(NT, 1) void chain_kernel(const ChainPhase* __restri
 }
 
 // ---------------------------------------------------------------------------- weight layout
-// Wc[tile][j][c][h] = W[2j + h][column(tile, c)], zero outside [K) x [N).  Single: column = 4*tile + c.
-// Dual (SwiGLU pair): columns interleaved, c = 0,2 -> gate column 2*tile + c/2, c = 1,3 -> the same
-// column of up, so one tile finishes two outputs.
+// Single: column = 4 * tile + c.  Dual (SwiGLU pair): columns interleaved, c = 0, 2 -> gate column 2 * tile + c / 2, c = 1, 3 -> the
+// same column of up, so one tile finishes two outputs.  A word holds 64 k-groups of the tile's 4 columns, lane l (16 bytes) group
+// 64 chunk + l: 2 k of each column in bf16, 1 in f32, 4 int8 codes, 8 int4 codes.  Zero (of codes: the biased zero) outside the matrix.
+// Place of word (tile, chunk) in the copy, in words: [step][workgroup][wave][3], the order in which the chip asks for them.
+struct ChainOrder {
+    int64_t ntiles, C, grid, tlo, trem;
+    __host__ __device__ int64_t word(int64_t tile, int64_t chunk) const {
+        const int64_t big = trem * (tlo + 1);
+        const int64_t b = tile < big ? tile / (tlo + 1) : trem + (tile - big) / tlo;
+        const int64_t t0 = b * tlo + (b < trem ? b : trem), W = (tlo + (b < trem ? 1 : 0)) * C, f = (tile - t0) * C + chunk;
+        const int64_t w = (8 * f + 7) / W, i = f - wave_first((int)W, (int)w);
+        return (((i / SW) * grid + b) * NWS + w) * SW + i % SW;
+    }
+    int64_t steps() const { return (((tlo + (trem > 0 ? 1 : 0)) * C + NWS - 1) / NWS + SW - 1) / SW; }
+    int64_t words() const { return steps() * grid * NWS * SW; }
+};
+
+__device__ __forceinline__ const void* chain_column(const void* w, const void* w2, int64_t tile, int c, int64_t& col) {
+    if (w2) { col = tile * 2 + (c >> 1); return (c & 1) ? w2 : w; }
+    col = tile * 4 + c;
+    return w;
+}
 __global__ void chain_pack_kernel(const bf16_t* __restrict__ w, const bf16_t* __restrict__ w2, uint32_t* __restrict__ out,
-                                  int64_t K, int64_t N, int64_t Kw, int64_t ntiles) {
-    const int64_t total = ntiles * Kw * 4;
+                                  int64_t K, int64_t N, ChainOrder o) {
+    const int64_t total = o.ntiles * o.C * 256;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
         const int c = (int)(idx & 3);
-        const int64_t j = (idx >> 2) % Kw, tile = (idx >> 2) / Kw;
-        const bf16_t* src = w;
+        const int64_t j = (idx >> 2) % (o.C * CW), tile = (idx >> 2) / (o.C * CW);
         int64_t col;
-        if (w2) { col = tile * 2 + (c >> 1); if (c & 1) src = w2; }
-        else col = tile * 4 + c;
+        const bf16_t* src = (const bf16_t*)chain_column(w, w2, tile, c, col);
         uint32_t lo = 0, hi = 0;
         if (col < N) {
             if (2 * j < K) lo = src[(2 * j) * N + col];
             if (2 * j + 1 < K) hi = src[(2 * j + 1) * N + col];
         }
-        out[idx] = lo | (hi << 16);
+        out[o.word(tile, j / CW) * 256 + (j % CW) * 4 + c] = lo | (hi << 16);
     }
 }
-
-// Quantised codes: the same tile order with one byte per (column, code row): word j of a tile holds code rows
-// 4j .. 4j+3 of its 4 columns.  int8: a code row is one k, bytes stored as q + 128 (flip = 0x80).  int4: a code
-// row is a packed byte (k = 2r low nibble, 2r + 1 high nibble), both nibbles stored as q + 8 (flip = 0x88).
-// Bytes outside the matrix hold the biased zero.
-// f32 weights: word (tile, k) = the 4 columns of the tile at row k
-__global__ void chain_pack_f32_kernel(const float* __restrict__ w, float* __restrict__ out, int64_t K, int64_t N, int64_t Kw, int64_t ntiles) {
-    const int64_t total = ntiles * Kw * 4;
+__global__ void chain_pack_f32_kernel(const float* __restrict__ w, float* __restrict__ out, int64_t K, int64_t N, ChainOrder o) {
+    const int64_t total = o.ntiles * o.C * 256;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
         const int c = (int)(idx & 3);
-        const int64_t j = (idx >> 2) % Kw, tile = (idx >> 2) / Kw;
+        const int64_t j = (idx >> 2) % (o.C * CW), tile = (idx >> 2) / (o.C * CW);
         const int64_t col = tile * 4 + c;
-        out[idx] = (col < N && j < K) ? w[j * N + col] : 0.f;
+        out[o.word(tile, j / CW) * 256 + (j % CW) * 4 + c] = (col < N && j < K) ? w[j * N + col] : 0.f;
     }
 }
-
+// Quantised codes: one byte per (column, code row), group j of a tile holds code rows 4j .. 4j+3 of its 4 columns.  int8: a code
+// row is one k, bytes stored as q + 128 (flip = 0x80).  int4: a code row is a packed byte (k = 2r low nibble, 2r + 1 high
+// nibble), both nibbles stored as q + 8 (flip = 0x88).
 __global__ void chain_pack_codes_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2, uint32_t* __restrict__ out,
-                                        int64_t rows, int64_t N, int64_t Kw, int64_t ntiles, uint32_t flip) {
-    const int64_t total = ntiles * Kw * 4;
+                                        int64_t rows, int64_t N, ChainOrder o, uint32_t flip) {
+    const int64_t total = o.ntiles * o.C * 256;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
         const int c = (int)(idx & 3);
-        const int64_t j = (idx >> 2) % Kw, tile = (idx >> 2) / Kw;
-        const uint8_t* src = w;
+        const int64_t j = (idx >> 2) % (o.C * CW), tile = (idx >> 2) / (o.C * CW);
         int64_t col;
-        if (w2) { col = tile * 2 + (c >> 1); if (c & 1) src = w2; }
-        else col = tile * 4 + c;
+        const uint8_t* src = (const uint8_t*)chain_column(w, w2, tile, c, col);
         uint32_t v = 0;
         for (int h = 0; h < 4; ++h) {
             const int64_t r = 4 * j + h;
             const uint32_t b = (col < N && r < rows) ? ((uint32_t)src[r * N + col] ^ flip) : flip;
             v |= b << (8 * h);
         }
-        out[idx] = v;
+        out[o.word(tile, j / CW) * 256 + (j % CW) * 4 + c] = v;
     }
 }
-// int4 group scales in tile order: sc[tile][g][c] (bf16) for g < Kw / 16, zero outside the matrix
+// int4 group scales in tile order: sc[tile][g][c] (bf16) for g < 4 C, zero outside the matrix
 __global__ void chain_pack_scales_kernel(const bf16_t* __restrict__ sc, const bf16_t* __restrict__ sc2, bf16_t* __restrict__ out,
                                          int64_t groups, int64_t N, int64_t G, int64_t ntiles) {
     const int64_t total = ntiles * G * 4;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
         const int c = (int)(idx & 3);
         const int64_t g = (idx >> 2) % G, tile = (idx >> 2) / G;
-        const bf16_t* src = sc;
         int64_t col;
-        if (sc2) { col = tile * 2 + (c >> 1); if (c & 1) src = sc2; }
-        else col = tile * 4 + c;
+        const bf16_t* src = (const bf16_t*)chain_column(sc, sc2, tile, c, col);
         out[idx] = (col < N && g < groups) ? src[g * N + col] : (bf16_t)0;
+    }
+}
+// The inverse of the bf16 copy: the row-major [K, N] matrix back, exactly -- the copy is a permutation plus zero padding.  A matrix
+// whose packed copy exists need not stay resident in its row-major form; this brings it back when some other kernel family
+// asks for it.  second: the up matrix of a pair.
+__global__ void chain_unpack_kernel(const uint32_t* __restrict__ packed, bf16_t* __restrict__ w, int64_t K, int64_t N, ChainOrder o, int dual, int second) {
+    const int64_t total = (K + 1) / 2 * N;
+    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t col = idx % N, j = idx / N;
+        const int64_t tile = dual ? col >> 1 : col >> 2, c = dual ? ((col & 1) << 1) + second : col & 3;
+        const uint32_t v = packed[o.word(tile, j / CW) * 256 + (j % CW) * 4 + c];
+        w[(2 * j) * N + col] = (bf16_t)(v & 0xFFFFu);
+        if (2 * j + 1 < K) w[(2 * j + 1) * N + col] = (bf16_t)(v >> 16);
     }
 }
 
@@ -1916,7 +1888,8 @@ static inline int64_t cdiv64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 static inline int chain_kpw(int wfmt) { return wfmt == kChainW32 ? 1 : (wfmt == kChainW16 ? 2 : (wfmt == kChainW8 ? 4 : 8)); }   // k per column of a word
 // bytes of staged activations per weight word: kpw bf16 values, or one f32
 static inline int chain_xbytes(int wfmt) { return wfmt == kChainW32 ? 4 : chain_kpw(wfmt) * 2; }
-static inline int64_t chain_kw(int64_t k, int wfmt) { return cdiv64(cdiv64(k, chain_kpw(wfmt)), NS) * NS; }
+static inline int64_t chain_chunks(int64_t k, int wfmt) { return cdiv64(k, chain_kpw(wfmt) * CW); }   // words of a tile
+static inline int64_t chain_xs_bytes(int64_t k, int wfmt) { return chain_chunks(k, wfmt) * CW * chain_xbytes(wfmt); }   // staged activations
 
 bool chain_supported(int dtype, int64_t m, int64_t k, int64_t n, bool dual, bool norm, int wfmt, bool x_f32, bool plain) {
     if (m != 1 || k < 4 || n < 4) return false;
@@ -1926,43 +1899,59 @@ bool chain_supported(int dtype, int64_t m, int64_t k, int64_t n, bool dual, bool
     if (wfmt < kChainW16 || wfmt > kChainW32) return false;
     if (wfmt == kChainW32) {   // f32 weights, activations and output; no SwiGLU pair
         if (dtype != 0 || dual || k % 4 != 0 || (n % 4 != 0 && !ragged_ok) || k > 4 * (MAXI / 2) * NT) return false;
-        return chain_kw(k, wfmt) * chain_xbytes(wfmt) / 4 <= kChainMaxXsWords;
+        return chain_xs_bytes(k, wfmt) / 4 <= kChainMaxXsWords;
     }
     if (dtype != 2) return false;
     if (x_f32 && (!norm || k > 4 * (MAXI / 2) * NT)) return false;
     if (k % 4 != 0 || (n % (dual ? 2 : 4) != 0 && !ragged_ok)) return false;
     if (wfmt == kChainW4 && k % 128 != 0) return false;
     if (norm && k > 4 * MAXI * NT) return false;
-    if (chain_kw(k, wfmt) * chain_xbytes(wfmt) / 4 > kChainMaxXsWords) return false;
+    if (chain_xs_bytes(k, wfmt) / 4 > kChainMaxXsWords) return false;
     return true;
 }
 
-size_t chain_weight_bytes(int64_t k, int64_t n, bool dual, int wfmt) {
-    const int64_t ncols = dual ? 2 * n : n;
-    return (size_t)(cdiv64(ncols, 4) * chain_kw(k, wfmt) * 16);
+static ChainOrder chain_order(int64_t k, int64_t n, bool dual, int wfmt) {
+    ChainOrder o;
+    o.ntiles = cdiv64(dual ? 2 * n : n, 4);
+    o.C = chain_chunks(k, wfmt);
+    o.grid = chain_grid() > 0 ? chain_grid() : 256;
+    o.tlo = o.ntiles / o.grid;
+    o.trem = o.ntiles % o.grid;
+    return o;
 }
 
+size_t chain_weight_bytes(int64_t k, int64_t n, bool dual, int wfmt) { return (size_t)(chain_order(k, n, dual, wfmt).words() * CW * 16); }
+
 void chain_pack_weights(hipStream_t s, const void* w, const void* w2, void* out, int64_t k, int64_t n, int wfmt) {
-    const int64_t ncols = w2 ? 2 * n : n, ntiles = cdiv64(ncols, 4), kw = chain_kw(k, wfmt);
-    const int64_t total = ntiles * kw * 4;
+    const ChainOrder o = chain_order(k, n, w2 != nullptr, wfmt);
+    const int64_t total = o.ntiles * o.C * 256;
     if (total <= 0) return;
     const unsigned g = (unsigned)std::min<int64_t>(cdiv64(total, 256), 65536);
     if (wfmt == kChainW32)
-        chain_pack_f32_kernel<<<g, 256, 0, s>>>((const float*)w, (float*)out, k, n, kw, ntiles);
+        chain_pack_f32_kernel<<<g, 256, 0, s>>>((const float*)w, (float*)out, k, n, o);
     else if (wfmt == kChainW16)
-        chain_pack_kernel<<<g, 256, 0, s>>>((const bf16_t*)w, (const bf16_t*)w2, (uint32_t*)out, k, n, kw, ntiles);
+        chain_pack_kernel<<<g, 256, 0, s>>>((const bf16_t*)w, (const bf16_t*)w2, (uint32_t*)out, k, n, o);
     else
-        chain_pack_codes_kernel<<<g, 256, 0, s>>>((const uint8_t*)w, (const uint8_t*)w2, (uint32_t*)out, wfmt == kChainW8 ? k : k / 2, n, kw,
-                                                  ntiles, wfmt == kChainW8 ? 0x80u : 0x88u);
+        chain_pack_codes_kernel<<<g, 256, 0, s>>>((const uint8_t*)w, (const uint8_t*)w2, (uint32_t*)out, wfmt == kChainW8 ? k : k / 2, n, o,
+                                                  wfmt == kChainW8 ? 0x80u : 0x88u);
+}
+
+void chain_unpack_weights(hipStream_t s, const void* packed, void* w, void* w2, int64_t k, int64_t n, bool dual) {
+    const int64_t total = (k + 1) / 2 * n;
+    if (total <= 0) return;
+    const ChainOrder o = chain_order(k, n, dual, kChainW16);
+    const unsigned g = (unsigned)std::min<int64_t>(cdiv64(total, 256), 65536);
+    if (w) chain_unpack_kernel<<<g, 256, 0, s>>>((const uint32_t*)packed, (bf16_t*)w, k, n, o, dual ? 1 : 0, 0);
+    if (w2) chain_unpack_kernel<<<g, 256, 0, s>>>((const uint32_t*)packed, (bf16_t*)w2, k, n, o, dual ? 1 : 0, 1);
 }
 
 size_t chain_scale_bytes(int64_t k, int64_t n, bool dual) {
-    return (size_t)(cdiv64(dual ? 2 * n : n, 4) * (chain_kw(k, kChainW4) / 16) * 4 * sizeof(bf16_t));
+    return (size_t)(cdiv64(dual ? 2 * n : n, 4) * 4 * chain_chunks(k, kChainW4) * 4 * sizeof(bf16_t));
 }
 
 void chain_pack_scales_w4(hipStream_t s, int dtype, const void* sc, const void* sc2, void* out, int64_t k, int64_t n) {
     if (dtype != 2) return;   // the chain only takes bf16 activations and scales
-    const int64_t ntiles = cdiv64(sc2 ? 2 * n : n, 4), G = chain_kw(k, kChainW4) / 16;
+    const int64_t ntiles = cdiv64(sc2 ? 2 * n : n, 4), G = 4 * chain_chunks(k, kChainW4);
     const int64_t total = ntiles * G * 4;
     if (total <= 0) return;
     const unsigned g = (unsigned)std::min<int64_t>(cdiv64(total, 256), 65536);
@@ -1970,22 +1959,23 @@ void chain_pack_scales_w4(hipStream_t s, int dtype, const void* sc, const void* 
 }
 
 bool chain_fill_phase(ChainPhase& p, int64_t k, int64_t n, bool dual, int wfmt) {
-    const int grid = chain_grid();
+    const ChainOrder o = chain_order(k, n, dual, wfmt);
+    const int64_t most = o.tlo + (o.trem > 0 ? 1 : 0);   // tiles of a workgroup
     p.K = (int)k;
     p.N = (int)n;
-    p.Kw = (int)chain_kw(k, wfmt);
-    p.ntiles = (int)cdiv64(dual ? 2 * n : n, 4);
-    p.wpt = p.Kw / NS;
-    p.units = (p.ntiles + TP - 1) / TP;
-    p.upb = grid > 0 ? (p.units + grid - 1) / grid : p.units;
+    p.C = (int)o.C;
+    p.tlo = (int)o.tlo;
+    p.trem = (int)o.trem;
+    p.step_bytes = (int)(o.grid * SLOT_BYTES);
+    p.inv_c = 1.0f / (float)o.C;
     p.kind = kChainLinear;
     p.wfmt = wfmt;
-    p.lds_bytes = p.Kw * chain_xbytes(wfmt);
+    p.lds_bytes = (int)chain_xs_bytes(k, wfmt);
     // int4: the workgroup's group scales (8 bytes per tile and group) are staged behind the activations
-    const int64_t total = p.lds_bytes + (wfmt == kChainW4 ? (int64_t)p.upb * TP * (p.Kw / 16) * 8 : 0);
+    const int64_t total = p.lds_bytes + (wfmt == kChainW4 ? most * 4 * o.C * 8 : 0);
     p.lds_total = (int)std::min<int64_t>(total, INT32_MAX);
     if (dual) p.flags |= kChainDual;
-    return (int64_t)p.upb * TP * (dual ? 2 : 4) <= EPI_MAX && total <= (int64_t)kChainMaxXsWords * 4;
+    return most * (dual ? 2 : 4) <= EPI_MAX && most * o.C < (1 << 22) && total <= (int64_t)kChainMaxXsWords * 4;
 }
 
 bool chain_attn_supported(int dtype, int64_t t, int64_t n_q, int64_t n_kv, int64_t head_dim, int64_t rot_half) {

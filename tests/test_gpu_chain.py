@@ -78,6 +78,20 @@ def test_single_linear(hip, k, n):
     run_both(hip, lambda fb, a, b: a.matmul(b), [[1, k], [k, n]], [x, w], 2e-5, 2e-5)
 
 
+# 4-column tiles are dealt over 256 workgroups and a workgroup's 1 KiB words over 8 waves: one tile less than workgroups, as many, one
+# more; eight tiles and a few more to a workgroup (where a tile's parts change from up to eight waves to two); fewer words than
+# waves, words that do not divide by 8 or 3, a word that is mostly padding
+DEALT = [(132, 1020), (132, 1024), (132, 1028), (384, 3084), (260, 8204), (1156, 7172)]
+
+
+@pytest.mark.parametrize("k,n", DEALT)
+def test_tiles_dealt_over_workgroups(hip, k, n):
+    x, w, r = rnd(23, (1, k)), rnd(24, (k, n), 2.0 / np.sqrt(k)), rnd(25, (1, n))
+    # as above: the f32 dot, and the residual, rounded once
+    run_both(hip, lambda fb, a, b, c: a.matmul(b) + c, [[1, k], [k, n], [1, n]], [x, w, r], 2e-5, 2e-5, rtol=ULP)
+    run_both_f32(hip, lambda fb, a, b, c: a.matmul(b) + c, [[1, k], [k, n], [1, n]], [x, w, r])
+
+
 @pytest.mark.parametrize("k,n", [(3072, 6144), (1024, 256)])
 def test_norm_linear(hip, k, n):
     x, g, w = rnd(3, (1, k), 3.0), rnd(4, (k,)) + 1.5, rnd(5, (k, n), 2.0 / np.sqrt(k))

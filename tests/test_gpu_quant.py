@@ -116,6 +116,16 @@ def test_decode_linear_bf16(hip, scheme, k, n):
     run_linear(hip, lambda fb, a, b, c: F.linear_quantized(a, b, c), specs, [x, q, s], 2e-2, 2e-2, expect_chain=True)
 
 
+@pytest.mark.parametrize("scheme", ["w8", "w4g128"])
+@pytest.mark.parametrize("k,n", [(128, 1020), (640, 1028), (1152, 3084), (2176, 8204)])
+def test_decode_linear_tiles_dealt_over_workgroups(hip, scheme, k, n):
+    """Codes of the chain where tiles and words do not divide evenly over workgroups, waves and steps."""
+    x, w = bf16_round(rnd(16, (1, k))), rnd(17, (k, n), 2.0 / np.sqrt(k))
+    q, s = quantize(w, scheme)
+    specs = [("Bf16", [1, k]), code_spec(scheme, k, n), ("Bf16", scale_dims(scheme, k, n))]
+    run_linear(hip, lambda fb, a, b, c: F.linear_quantized(a, b, c), specs, [x, q, s], 2e-2, 2e-2, expect_chain=True)
+
+
 @pytest.mark.parametrize("scheme,k,n", [("w8", 3072, 32768), ("w4g128", 3072, 32768), ("w4g128", 2048, 155648)])
 def test_decode_linear_wide(hip, scheme, k, n):
     """Vocabulary-sized outputs: many units per workgroup, and (last case) more int4 group scales per workgroup
