@@ -322,6 +322,9 @@ bool mfma_gemm_supported(int dtype, int64_t m, int64_t k, int64_t n, int quant =
 // Dynamic LDS that mfma_gemm() asks for int4 codes when `room` bytes of workspace are there (0: the register-staged kernel runs):
 // never more than a CU has, however little room there is.
 size_t mfma_int4_lds_bytes(int64_t m, int64_t k, int64_t n, bool dual, size_t room);
+// launches that an unsplit bf16 layer takes (its workspace granted in full): 1, or 2 with out[8] = rows and columns of the first (0: all), first row and
+// column of the second, rows and columns of the first's tile, both tiles
+int mfma_bf16_regions(int64_t m, int64_t k, int64_t n, bool dual, int64_t* out);
 void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a);
 
 // Rotate-half RoPE on packed [T, Q|K|V] rows (ops/functional/rotary.rs:430-536).

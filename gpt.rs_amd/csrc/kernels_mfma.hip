@@ -625,7 +625,7 @@ __device__ __forceinline__ void gemm_finish8(const TileEpilogue<T>& p, int64_t m
 }
 template <typename T, int KG, int NST, int WM, int WN, int KW, int TM, int TN, bool DUAL, int QF>
 __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* __restrict__ x, const T* __restrict__ wk, const T* __restrict__ wk2,
-                                                                 int M, int K, int Npad, int NT, int MT, int splits, float* __restrict__ part, const T* __restrict__ scale, const T* __restrict__ scale2,
+                                                                 int M, int K, int Npad, int row0, int col0, int NT, int MT, int splits, float* __restrict__ part, const T* __restrict__ scale, const T* __restrict__ scale2,
                                                                  TileEpilogue<T> epi) {
     static_assert(KG == 4 || KG == 8, "k-groups of a k tile");
     typedef typename Mma<T>::frag frag_t;
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_tile_kernel(const T* _
         by = first + (v % gsz) % gm;
         bx = (v % gsz) / gm;
     }
-    const int m0 = by * BM, n0 = bx * NREAL;
+    const int m0 = row0 + by * BM, n0 = col0 + bx * NREAL;   // the tiles cover NT columns and MT rows of them from (row0, col0) on
     auto swz = [](int row) { return KG == 8 ? (row >> 1) & 7 : (row >> 2) & 3; };
     // what each of this wave's load instructions fetches, per lane
     unsigned a_off[LA], b_off[LB];
@@ -1330,14 +1330,18 @@ static void launch_reduce_norm(hipStream_t s, const MfmaLinearArgs& a, int split
 
 // The tiles, in the order of tile_cost's table.
 enum TileId { kT256x256, kT256x192, kT192x192, kT128x256, kT128x192, kT128x128, kT64x256, kT64x128, kTiles };
-struct TilePlan { int tile; int splits; };
+// The part of a layer's outputs that a launch forms: whole tiles from (row0, col0) on; no rows or columns: to the end.  (A layer whose k
+// is split is formed by one launch.)
+struct TileRegion { int64_t row0 = 0, col0 = 0, rows = 0, cols = 0; };
+// rest_tile >= 0 (bf16): the layer takes two launches, `tile` over `first` and `rest_tile` over `rest`.
+struct TilePlan { int tile; int splits; int rest_tile = -1; TileRegion first = {}, rest = {}; };
 constexpr int kTileLds = 160 * 1024;   // LDS of one CU
 
 // LDS of an int4 tile: a ring of three and, behind it, the scales of the groups of 128 k that a workgroup's share of K touches.
 static int64_t int4_lds_bytes(int64_t bm, int64_t bn, int64_t k, int64_t splits) { return 3 * (bm * 128 + bn * 32) + (cdiv(cdiv(k, 64), splits) / 2 + 2) * bn * 2; }
 
 template <typename T, int KG, int NST, int WM, int WN, int TM, int TN, bool DUAL, int QF = 0, int KW = 1>
-static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
+static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits, TileRegion at = {}) {
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NREAL = DUAL ? BN / 2 : BN;
     constexpr int ring = NST * (BM * KG * 16 + BN * KG * (QF == 0 ? 16 : QF == 1 ? 8 : 4)), area = WM * WN * KW * 32 * (32 * (DUAL && TN % 2 == 0 ? TN / 2 : TN) + 4) * 4;
     constexpr int rows = KW == 1 ? area : std::max(area, WM * WN * KW * (TM / KW) * TN * 16 * 64 * 4);   // what the epilogue puts where the ring was
@@ -1351,10 +1355,10 @@ static void launch_tile(hipStream_t s, const MfmaLinearArgs& a, int splits) {
         (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_most);
         configured = true;
     }
-    const int64_t nt = cdiv(a.n, NREAL), mt = cdiv(a.m, BM);
+    const int64_t nt = cdiv((at.cols ? at.cols : a.n - at.col0), NREAL), mt = cdiv((at.rows ? at.rows : a.m - at.row0), BM);
     TileEpilogue<T> epi{(const T*)a.bias, a.residual, a.y, a.n, a.act, a.out_f32, a.extra};
     kern<<<(unsigned)(cdiv(nt * mt * splits, 8) * 8), 64 * WM * WN * KW, lds_bytes, s>>>((const T*)a.x, (const T*)a.wk, (const T*)a.wk2, (int)a.m, (int)a.k,
-                                                                                   (int)mfma_padded_n(a.n), (int)nt, (int)mt, splits, (float*)a.part,
+                                                                                   (int)mfma_padded_n(a.n), (int)at.row0, (int)at.col0, (int)nt, (int)mt, splits, (float*)a.part,
                                                                                    (const T*)a.scale, (const T*)a.scale2, epi);
     if constexpr (std::is_same<T, bf16_t>::value && !DUAL)
         if (splits > 1 && norm_fits(a)) return launch_reduce_norm(s, a, splits);
@@ -1400,22 +1404,63 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t roo
             if (us < least) { least = us; best = {t, sp}; }
         }
     }
+    // Two launches: as many whole rows or columns of tiles as fill whole rounds, and the rest, which would leave most of a last round idle,
+    // in tiles that fill a round of their own.  Taken where the fit says 7.5 % or more: what it says less about came out level, since a
+    // last round that is partly empty runs at a higher clock.  us, weights from memory, measured against the best single launch: pair of
+    // 9216 M = 1000 126 -> 119, 2047 238 -> 218, 3000 340 -> 319; N = 6176 M = 3000 135 -> 123; K = 1536, N = 6144 M = 3064 75 -> 71.
+    // Over 160 shapes that the rule was tried on (M = 64 .. 7600, K = 576 .. 9216, N = 768 .. 14336) it gains 8.8 % in the mean; the losses, up to
+    // 7 %, are all at K of 1024 and less (M = 4758, K = 768, N = 5120 69 -> 74), where the second launch's start counts: those stay whole.
+    // Left alone too: N = 14432 M = 3064 (5.6 % by the fit, 265 and 262), K = 3072, N = 4096 M = 3064 (5.4 %, 86 and 85).
+    if (best.splits == 1 && least > 40.0 && k > 1024) {
+        const double one = least;
+        auto cost = [&](int t, int64_t rows, int64_t cols) {
+            const TileCost& c = kTileCost[t];
+            const int64_t tiles = cdiv(rows, c.bm) * cdiv(cols, dual ? c.bn / 2 : c.bn);
+            const double kt = (double)k / 64;
+            return (double)cdiv(tiles, c.slots) * (c.fixed + c.per_kt * kt) + c.full_kt * kt * (double)tiles / 256;
+        };
+        for (int t = 0; t < kTiles; ++t) {
+            if ((dual && (t == kT256x192 || t == kT192x192)) || (t == kT192x192 && k < 80 * 64)) continue;
+            const TileCost& c = kTileCost[t];
+            const int64_t bn = dual ? c.bn / 2 : c.bn, nt = cdiv(n, bn), mt = cdiv(m, c.bm), filled = nt * mt / c.slots * c.slots;
+            for (const bool by_columns : {true, false}) {
+                const int64_t whole = filled / (by_columns ? mt : nt);   // columns or rows of tiles
+                if (whole < 1 || whole >= (by_columns ? nt : mt)) continue;
+                TileRegion first, rest;
+                (by_columns ? first.cols : first.rows) = whole * (by_columns ? bn : c.bm);
+                (by_columns ? rest.col0 : rest.row0) = whole * (by_columns ? bn : c.bm);
+                const double us1 = cost(t, by_columns ? m : first.rows, by_columns ? first.cols : n);
+                for (int r = 0; us1 < least && r < kTiles; ++r) {
+                    if (r == kT192x192 || (dual && r == kT256x192)) continue;
+                    const double us = us1 + cost(r, m - rest.row0, n - rest.col0);
+                    if (us < least && us < 0.925 * one) { least = us; best = {t, 1, r, first, rest}; }
+                }
+            }
+        }
+    }
     return best;
 }
+int mfma_bf16_regions(int64_t m, int64_t k, int64_t n, bool dual, int64_t* out) {
+    const TilePlan p = tile_plan(m, k, n, dual);
+    if (p.rest_tile < 0) return 1;
+    const int64_t v[8] = {p.first.rows, p.first.cols, p.rest.row0, p.rest.col0, kTileCost[p.tile].bm, dual ? kTileCost[p.tile].bn / 2 : kTileCost[p.tile].bn, p.tile, p.rest_tile};
+    for (int i = 0; i < 8; ++i) out[i] = v[i];
+    return 2;
+}
 template <bool DUAL>
-static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p) {
+static void launch_tile_plan(hipStream_t s, const MfmaLinearArgs& a, TilePlan p, TileRegion at = {}) {
     typedef bf16_t T;
     switch (p.tile) {
-        case kT256x256: return launch_tile<T, 4, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits);
-        case kT256x192: if constexpr (!DUAL) return launch_tile<T, 8, 2, 4, 2, 2, 3, false>(s, a, p.splits); else return;
-        case kT192x192: if constexpr (!DUAL) return launch_tile<T, 8, 3, 2, 2, 3, 3, false>(s, a, p.splits); else return;
-        case kT128x256: return launch_tile<T, 8, 3, 2, 4, 2, 2, DUAL>(s, a, p.splits);
-        case kT128x192: return launch_tile<T, 8, 3, 2, 2, 2, 3, DUAL, 0, 2>(s, a, p.splits);
+        case kT256x256: return launch_tile<T, 4, 4, 2, 4, 4, 2, DUAL>(s, a, p.splits, at);
+        case kT256x192: if constexpr (!DUAL) return launch_tile<T, 8, 2, 4, 2, 2, 3, false>(s, a, p.splits, at); else return;
+        case kT192x192: if constexpr (!DUAL) return launch_tile<T, 8, 3, 2, 2, 3, 3, false>(s, a, p.splits, at); else return;
+        case kT128x256: return launch_tile<T, 8, 3, 2, 4, 2, 2, DUAL>(s, a, p.splits, at);
+        case kT128x192: return launch_tile<T, 8, 3, 2, 2, 2, 3, DUAL, 0, 2>(s, a, p.splits, at);
         case kT128x128:
-            if constexpr (DUAL) return launch_tile<T, 8, 4, 4, 2, 1, 2, true>(s, a, p.splits);
-            else return launch_tile<T, 8, 4, 2, 4, 2, 1, false>(s, a, p.splits);
-        case kT64x256: return launch_tile<T, 8, 3, 2, 4, 1, 2, DUAL>(s, a, p.splits);
-        default: return launch_tile<T, 8, 3, 2, 2, 1, 2, DUAL>(s, a, p.splits);
+            if constexpr (DUAL) return launch_tile<T, 8, 4, 4, 2, 1, 2, true>(s, a, p.splits, at);
+            else return launch_tile<T, 8, 4, 2, 4, 2, 1, false>(s, a, p.splits, at);
+        case kT64x256: return launch_tile<T, 8, 3, 2, 4, 1, 2, DUAL>(s, a, p.splits, at);
+        default: return launch_tile<T, 8, 3, 2, 2, 1, 2, DUAL>(s, a, p.splits, at);
     }
 }
 
@@ -1614,7 +1659,10 @@ void mfma_gemm(hipStream_t s, const MfmaLinearArgs& a) {
         return dual ? launch_tile<float, 8, 3, 2, 2, 1, 2, true>(s, a, sp) : launch_tile<float, 8, 3, 2, 2, 1, 1, false>(s, a, sp);
     }
     const TilePlan p = tile_plan(a.m, a.k, a.n, dual, room_of(a));
-    return dual ? launch_tile_plan<true>(s, a, p) : launch_tile_plan<false>(s, a, p);
+    dual ? launch_tile_plan<true>(s, a, p, p.first) : launch_tile_plan<false>(s, a, p, p.first);
+    if (p.rest_tile < 0) return;
+    const TilePlan r{p.rest_tile, 1};
+    dual ? launch_tile_plan<true>(s, a, r, p.rest) : launch_tile_plan<false>(s, a, r, p.rest);
 }
 
 }  // namespace k

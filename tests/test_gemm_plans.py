@@ -22,6 +22,32 @@ def lib():
     return lds, part
 
 
+def regions(m, k, n, dual):
+    """None for one launch, or (rows, columns) of the first, (row, column) of the second, the first's tile."""
+    f, out = backend.load_library()._ZN5gptrs1k17mfma_bf16_regionsElllbPl, (ctypes.c_int64 * 8)()   # mfma_bf16_regions
+    f.argtypes, f.restype = [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_void_p], ctypes.c_int
+    if f(m, k, n, dual, out) == 1:
+        return None
+    return (out[0], out[1]), (out[2], out[3]), (out[4], out[5])
+
+
+def test_two_launches_cover_a_layer_once():
+    """The first launch takes whole rows or whole columns of its tiles, the second what is left of the layer; short K stay whole."""
+    two = 0
+    for m in (17, 333, 600, 1000, 1713, 2047, 3000, 4758, 8188):
+        for k in (64, 768, 1024, 1088, 3072, 9216):
+            for n in (8, 768, 2304, 3075, 6176, 9216, 14432):
+                for dual in (False, True):
+                    r = regions(m, k, n, dual)
+                    if r is None:
+                        continue
+                    (rows, cols), at, (bm, bn) = r
+                    assert k > 1024 and (rows == 0) != (cols == 0) and at == (rows, cols)
+                    assert rows % bm == 0 and cols % bn == 0 and rows < m and cols < n
+                    two += 1
+    assert two > 40
+
+
 @pytest.mark.parametrize("dual", [False, True])
 def test_int4_tiles_fit_whatever_the_workspace(dual):
     """The scales of a workgroup's share of K lie in LDS: with the splits given up for want of room the share is all of K, and the tile has to be

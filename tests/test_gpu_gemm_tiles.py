@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from parity import hip_run, to_bytes
-from test_gemm_plans import lib
+from test_gemm_plans import lib, regions
 from gptrs_amd import functional as F
 from gptrs_amd.ptir import FunctionBuilder, Program, bf16_bits_to_f32, f32_to_bf16_bits
 
@@ -65,6 +65,13 @@ def test_tiles_and_splits(hip, m, k, n):
     assert (np.abs(got[2][rows] - s * sig * t) <= pair).all()
     for a, b in zip(got, staged):           # two orders of the same sums, one rounding apart in bf16
         assert (np.abs(a - b) <= 2.0 ** -6 * np.maximum(np.abs(a), np.abs(b)) + 4e-4 * np.sqrt(k) / 16).all()
+
+
+# layers that take two launches, of the layer itself or of the pair: split between columns and between rows, ragged in both
+@pytest.mark.parametrize("m,k,n", [(2824, 1088, 5398), (2075, 1088, 7699), (609, 1792, 6587), (1555, 1088, 5027), (857, 2624, 5157)])
+def test_two_launches(hip, m, k, n):
+    assert any(regions(m, k, n, dual) is not None for dual in (False, True))
+    test_tiles_and_splits(hip, m, k, n)
 
 
 # the same kernel in f32, of up to 128 rows (64 x 64 tiles): tile edges, columns that are no multiple of 8, one k tile, k tiles that do not divide among
