@@ -123,6 +123,10 @@ struct Step {
     // Prefill linear: the next step is an RMS norm of its f32 result, which the launch that adds its splits may do; the norm's result is then
     // given its storage together with this step's own.
     bool norm_next = false;
+    // Linear layers of 2 to 16 rows under one and the same norm: the first of them (norm_first) has a launch norm the rows and leaves them at
+    // norm_off for the others; -1: the step's own scratch holds them.
+    int norm_first = -1, norm_last = -1;
+    size_t norm_off = 0;
     // Sum of two gathers of program inputs: the gathers' steps are left out and this step reads the tables itself.
     int take_a = -1, take_b = -1;
     bool left_out = false;

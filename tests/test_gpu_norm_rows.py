@@ -26,3 +26,35 @@ def test_rows(hip, n):
     want = c / np.sqrt((c ** 2).mean(axis=1, keepdims=True) + 1e-5) * g + b
     # ... and a mean that is off by its own roundings
     assert (np.abs(ln - want) <= 2 * rel * (np.abs(want) + np.abs(b) + 4 * np.abs(g)) + 1e-6).all()
+
+
+@pytest.mark.parametrize("ln", [False, True])
+@pytest.mark.parametrize("m,k,n", [(2, 64, 48), (8, 3072, 576), (16, 512, 2304)])
+def test_one_norm_of_several_layers(hip, ln, m, k, n):
+    """Layers of a few rows under one norm read rows that were normed once: bit for bit what each gives in a program of its own, and a norm
+    with other gains, or of other rows, is another one."""
+    rng = np.random.default_rng(m + k + n)
+    x = rng.standard_normal((m, k), dtype=np.float32)
+    gs = [(1 + 0.1 * rng.standard_normal(k)).astype(np.float32) for _ in range(2)]
+    b = (0.1 * rng.standard_normal(k)).astype(np.float32)
+    ws = [rng.standard_normal((k, n), dtype=np.float32) * np.float32(k ** -0.5) for _ in range(4)]
+    norm = lambda a, g, c: (F.layer_norm(a, g, c, 1e-5) if ln else F.rms_norm(a, g, 1e-5))[0].cast("Bf16")   # noqa: E731
+    bodies = [lambda h, h2, w, a, g, c: F.linear(h, w[0], out_dtype="F32"),
+              lambda h, h2, w, a, g, c: F.linear(h2, w[1], out_dtype="F32"),
+              lambda h, h2, w, a, g, c: F.swiglu(F.linear(h, w[2]), F.linear(h, w[3])),
+              lambda h, h2, w, a, g, c: F.linear(norm(a + a, g, c), w[1], out_dtype="F32"),
+              lambda h, h2, w, a, g, c: F.linear(h, w[1], out_dtype="F32")]
+    specs = [("F32", [m, k]), ("F32", [k]), ("F32", [k]), ("F32", [k])] + [("Bf16", [k, n])] * 4
+    args = [x, *gs, b, *ws]
+
+    def run(which):
+        return hip_run(hip, program(specs, lambda a, g, g2, c, *w: [bodies[i](norm(a, g, c), norm(a, g2, c), w, a, g, c) for i in which]), args)
+
+    together = run(range(5))
+    for i, got in enumerate(together):
+        assert np.array_equal(np.asarray(got, np.float32), np.asarray(run([i])[0], np.float32)), i
+    h64 = x.astype(np.float64) - (x.astype(np.float64).mean(1, keepdims=True) if ln else 0)
+    h64 = h64 / np.sqrt((h64 ** 2).mean(1, keepdims=True) + 1e-5) * gs[0] + (b if ln else 0)
+    want = h64 @ ws[0].astype(np.float64)
+    # the normed row and the weights rounded to bf16: 2^-9 each, of the products' root mean square in the mean; ten times that
+    assert np.abs(together[0] - want).max() <= 10 * 2.0 ** -8.5 * np.sqrt((h64 ** 2).mean() * (ws[0] ** 2).mean() * k)
