@@ -113,6 +113,77 @@ __device__ __forceinline__ void split_bf16_hw(float a, float b, uint32_t& hi, ui
     hi = pack_bf16_hw(a, b);
     lo = pack_bf16_hw(a - bf16lo(hi), b - bf16hi(hi));
 }
+// One step of a bf16 prompt's attention: 64 staged keys, 16 queries of a wave.  Everything is transposed (scores: rows = keys, columns
+// = queries; result: rows = values), so a lane works on one query: softmax in f32 registers, weights as powers of two, and they go from
+// there into the product with the values, as a bf16 value and its remainder.  A maximum that is -inf has to end with a key that its query sees;
+// behind a finite one all keys may be hidden.  `hidden(key)`: the lane's query does not see the key; asked only where `edge`, which is a scalar: one
+// branch and selects (a branch around every score's test took 16 of them a step).
+// Keys [64][kPromptKeyStride] and values [64][kPromptValueStride] in LDS: rows 16 and 32 bytes longer than whole rounds of the banks, so a key fragment meets no
+// bank twice, nor do the eight pieces of rows that half a wave's transposing read takes (values 16 bytes longer: every bank twice).
+// What bounds it: LDS, 32 KiB a wave and step at 128 + 128 values beside 48 MFMAs and some 250 vector instructions; a CU takes 2.0 us for the 8 waves of a workgroup and gains
+// nothing from a second one.  Dropped: 32 queries a wave in 4 waves (half the LDS reads, but then two waves a SIMD wait on each other: chunks of 1024, 1 x 1000
+// 45 -> 55 us, 1 x 3000 90 against 87; keys of 192, 1 x 3000 207 -> 240).
+template <int KS> constexpr int kPromptKeyStride = KS * 32 + 8;
+template <int VT> constexpr int kPromptValueStride = VT * 16 + 16;
+template <int KS, int VT, typename F>
+__device__ __forceinline__ void prompt_attn_step(const bf16_t* kt, const bf16_t* vt, const u32x4_m (&q)[KS], f32x4_m (&o)[VT], float& m, float& l, float scale2, int k0, int lane,
+                                                 bool edge, const F& hidden) {
+    constexpr int KSTR = kPromptKeyStride<KS>, VSTR = kPromptValueStride<VT>;
+    const int c = lane & 15, kg = lane >> 4;
+    f32x4_m s[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        s[j] = f32x4_m{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) s[j] = mma16(*reinterpret_cast<const u32x4_m*>(kt + (16 * j + c) * KSTR + 32 * k + 8 * kg), q[k], s[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] *= scale2;
+    if (edge) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[j][e] = hidden(k0 + 16 * j + 4 * kg + e) ? -INFINITY : s[j][e];
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[j][e]);
+    const float mn = fmaxf(m, col4_max(mx));
+    float sum = 0.f;
+    u32x4_m ph[2], pl[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float u = __builtin_amdgcn_exp2f(s[j][2 * e] - mn), v = __builtin_amdgcn_exp2f(s[j][2 * e + 1] - mn);
+            sum += u + v;
+            uint32_t hi, lo;
+            split_bf16_hw(u, v, hi, lo);
+            ph[j / 2][2 * (j & 1) + e] = hi;
+            pl[j / 2][2 * (j & 1) + e] = lo;
+        }
+    sum = col4_sum(sum);
+    if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {                   // some column's maximum has moved
+        const float corr = __builtin_amdgcn_exp2f(m - mn);
+        l *= corr;
+#pragma unroll
+        for (int v = 0; v < VT; ++v)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[v][e] *= corr;
+        m = mn;
+    }
+    l += sum;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            const u32x4_m vv = lds_operand_t2(vt + 32 * k * VSTR + 16 * v, VSTR, lane);
+            o[v] = mma16(vv, ph[k], o[v]);
+            o[v] = mma16(vv, pl[k], o[v]);
+        }
+}
 // Sum / maximum over the 16 lanes of a row, in every lane of it
 __device__ __forceinline__ float row16_sum(float v) {
     int x = __float_as_int(v);

@@ -443,20 +443,22 @@ constexpr int kQTile = 128;      // queries per workgroup: 16 per wave
 constexpr int kKTile = 64;       // keys per step
 
 // Workgroup = 128 queries (16 per wave) x head x sequence; keys from the first query's chunk on.  Keys and values of a step in LDS,
-// the next step's words in registers meanwhile.  Queries come from the projection, rotated and normed on the way in.  Everything is
-// transposed (scores: rows = keys, columns = queries; result: rows = values), so a lane works on one query: softmax in f32
-// registers, started from the sink (maximum = sink, weight 1: always finite, also for a step of which a query sees nothing); the
-// weights go from there into the product with the values, as a bf16 value and its remainder.
+// the next step's words in registers meanwhile.  Queries come from the projection, rotated and normed on the way in.  The softmax
+// is started from the sink (maximum = sink, weight 1: always finite, also for a step of which a query sees nothing).
+// Times, us, 32 heads of 128 + 128, before and after: 1 x 3000 in chunks of 1024 104 -> 79 (the order of the workgroups 87 -> 79: by position two of one length
+// shared a CU), 4 x 1000 109 -> 93, 1 x 1000 47.6 -> 45.4, 1 x 128 10.0 -> 8.4.
 template <int KS, int VT>
-__global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, const bf16_t* __restrict__ kr, const bf16_t* __restrict__ vr) {
+__global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, const bf16_t* __restrict__ kr, const bf16_t* __restrict__ vr, int per_chunk) {
     extern __shared__ __align__(16) unsigned char chk_smem[];
-    constexpr int KSTR = KS * 32 + 8, VSTR = VT * 16 + 8;
+    constexpr int KSTR = kPromptKeyStride<KS>, VSTR = kPromptValueStride<VT>;
     bf16_t* kt = reinterpret_cast<bf16_t*>(chk_smem);                 // [64][KSTR]
     bf16_t* vt = kt + kKTile * KSTR;                                  // [64][VSTR]
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 15, kg = lane >> 4;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), c = lane & 15, kg = lane >> 4;
     const XcdTile at = xcd_tile();
     const int b = at.z, h = at.y, T = a.len[b], r0 = a.row0[b];
-    const int q0 = ((int)gridDim.x - 1 - (int)at.x) * kQTile;
+    // the longest workgroups first: all chunks' last tiles, then all chunks' last but one (per_chunk tiles in a chunk), or simply from the prompt's end
+    const int chunks = per_chunk ? (int)gridDim.x / per_chunk : 1, tile = (int)gridDim.x - 1 - (int)at.x;
+    const int q0 = (per_chunk ? tile % chunks * per_chunk + tile / chunks : tile) * kQTile;
     if (q0 >= T) return;
     const int H = (int)a.heads, G = (int)a.kv_heads, D = (int)a.dim, V = (int)a.vdim, rot = (int)a.rot, g = h / (H / G);
     const int chunk = a.chunk > 0 && a.chunk < T ? (int)a.chunk : T;
@@ -485,33 +487,48 @@ __global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, cons
     fetch(kbeg);
 
     const int64_t row = r0 + min(qi, T - 1);                          // queries behind the prompt repeat its last one and are not stored
+    const float gate = a.proj[row * a.ld + (int64_t)(H + G) * D + (int64_t)G * V + h];
     u32x4_m q[KS];
     {
         const float* src = a.proj + row * a.ld + (int64_t)h * D;
         const float* tab = a.table + row * rot;
-        f32x4_m x[KS][2];
+        // every load is made, of a clamped place, before the first value is used: with tests around them each pair of cosines was a trip to memory of its own
+        f32x4_m x[KS][2], cs[KS], sn[KS];
         float ss = 0.f;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-            const int d = 32 * k + 8 * kg;
-            x[k][0] = x[k][1] = f32x4_m{0.f, 0.f, 0.f, 0.f};
-            if (d < D) {
-                x[k][0] = *reinterpret_cast<const f32x4_u*>(src + d);
-                x[k][1] = *reinterpret_cast<const f32x4_u*>(src + d + 4);
+            const int d = min(32 * k + 8 * kg, D - 8);
+            x[k][0] = *reinterpret_cast<const f32x4_u*>(src + d);
+            x[k][1] = *reinterpret_cast<const f32x4_u*>(src + d + 4);
+        }
+        if (rot > 0) {
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int dd = d + 2 * e;
-                    if (dd < rot) {
-                        const float cs = tab[dd >> 1], sn = tab[rot / 2 + (dd >> 1)];
-                        const float u = x[k][e >> 1][2 * (e & 1)], v = x[k][e >> 1][2 * (e & 1) + 1];
-                        x[k][e >> 1][2 * (e & 1)] = u * cs - v * sn;
-                        x[k][e >> 1][2 * (e & 1) + 1] = v * cs + u * sn;
-                    }
+                    const int i = min(16 * k + 4 * kg + e, rot / 2 - 1);
+                    cs[k][e] = tab[i];
+                    sn[k][e] = tab[rot / 2 + i];
                 }
-            }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss += x[k][e >> 2][e & 3] * x[k][e >> 2][e & 3];
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool turned = 32 * k + 8 * kg + 2 * e < rot;
+                    const float u = x[k][e >> 1][2 * (e & 1)], v = x[k][e >> 1][2 * (e & 1) + 1];
+                    const float ut = u * cs[k][e] - v * sn[k][e], vt2 = v * cs[k][e] + u * sn[k][e];
+                    x[k][e >> 1][2 * (e & 1)] = turned ? ut : u;
+                    x[k][e >> 1][2 * (e & 1) + 1] = turned ? vt2 : v;
+                }
         }
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float v = 32 * k + 8 * kg < D ? x[k][e >> 2][e & 3] : 0.f;
+                x[k][e >> 2][e & 3] = v;
+                ss += v * v;
+            }
         const float inv = 1.0f / sqrtf(col4_sum(ss) / (float)D + a.eps);
 #pragma unroll
         for (int k = 0; k < KS; ++k)
@@ -538,61 +555,10 @@ __global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, cons
         __syncthreads();
         if (k0 + kKTile < kend) fetch(k0 + kKTile);
         if (k0 > myq + 15 || k0 + kKTile <= wlo) continue;            // no query of the wave sees a key of the step
-        f32x4_m s[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            s[j] = f32x4_m{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < KS; ++k) s[j] = mma16(*reinterpret_cast<const u32x4_m*>(kt + (16 * j + c) * KSTR + 32 * k + 8 * kg), q[k], s[j]);
-        }
-        const bool edge = k0 + kKTile - 1 > myq || k0 < whi;          // some query does not see some key
-        float mx = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int key = k0 + 16 * j + 4 * kg + e;
-                float x = s[j][e] * scale2;
-                if (edge && (key > qi || key < qlo)) x = -INFINITY;
-                s[j][e] = x;
-                mx = fmaxf(mx, x);
-            }
-        const float mn = fmaxf(m, col4_max(mx));
-        float sum = 0.f;
-        u32x4_m ph[2], pl[2];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float u = __builtin_amdgcn_exp2f(s[j][2 * e] - mn), v = __builtin_amdgcn_exp2f(s[j][2 * e + 1] - mn);
-                sum += u + v;
-                uint32_t hi, lo;
-                split_bf16_hw(u, v, hi, lo);
-                ph[j / 2][2 * (j & 1) + e] = hi;
-                pl[j / 2][2 * (j & 1) + e] = lo;
-            }
-        sum = col4_sum(sum);
-        if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {               // some column's maximum has moved
-            const float corr = __builtin_amdgcn_exp2f(m - mn);
-            l *= corr;
-#pragma unroll
-            for (int v = 0; v < VT; ++v)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[v][e] *= corr;
-            m = mn;
-        }
-        l += sum;
-#pragma unroll
-        for (int k = 0; k < kKTile / 32; ++k)
-#pragma unroll
-            for (int v = 0; v < VT; ++v) {
-                const u32x4_m vv = lds_operand_t2(vt + 32 * k * VSTR + 16 * v, VSTR, lane);
-                o[v] = mma16(vv, ph[k], o[v]);
-                o[v] = mma16(vv, pl[k], o[v]);
-            }
+        prompt_attn_step<KS, VT>(kt, vt, q, o, m, l, scale2, k0, lane, k0 + kKTile - 1 > myq || k0 < whi, [&](int key) { return key > qi || key < qlo; });
     }
     if (qi >= T) return;
-    const float f = sigmoid_f32(a.proj[row * a.ld + (int64_t)(H + G) * D + (int64_t)G * V + h]) / l;
+    const float f = sigmoid_f32(gate) / l;
     bf16_t* out = (bf16_t*)a.ctx + (row * H + h) * V + 4 * kg;
 #pragma unroll
     for (int v = 0; v < VT; ++v)
@@ -715,10 +681,12 @@ size_t chunk_prefill_scratch_bytes(int dtype, int64_t total, int64_t heads, int6
 }
 template <int KS, int VT>
 static void launch_prefill(hipStream_t s, const ChunkSeqArgs& a, const void* k, const void* v, int64_t longest) {
-    constexpr int lds = kKTile * (KS * 32 + 8 + VT * 16 + 8) * 2;
+    constexpr int lds = kKTile * (kPromptKeyStride<KS> + kPromptValueStride<VT>) * 2;
     static_assert(lds <= 160 * 1024, "LDS of one CU");
     with_lds(chunk_prefill_kernel<KS, VT>, lds);
-    chunk_prefill_kernel<KS, VT><<<dim3((unsigned)cdiv_c(longest, kQTile), (unsigned)a.heads, (unsigned)a.nseq), 512, lds, s>>>(a, (const bf16_t*)k, (const bf16_t*)v);
+    const int64_t per_chunk = a.chunk > 0 && a.chunk < longest && a.chunk % kQTile == 0 ? a.chunk / kQTile : 0;   // else tiles reach over a chunk's end, or there is one
+    const int64_t tiles = per_chunk ? per_chunk * cdiv_c(longest, a.chunk) : cdiv_c(longest, kQTile);
+    chunk_prefill_kernel<KS, VT><<<dim3((unsigned)tiles, (unsigned)a.heads, (unsigned)a.nseq), 512, lds, s>>>(a, (const bf16_t*)k, (const bf16_t*)v, (int)per_chunk);
 }
 template <int KS>
 static void launch_prefill_v(hipStream_t s, const ChunkSeqArgs& a, const void* k, const void* v, int64_t longest) {

@@ -15,6 +15,9 @@ namespace k {
 
 namespace {
 
+// 16 bytes at any 4-byte boundary
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+
 inline int64_t cdiv_l(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // the angle is formed and reduced in f64: at position 10^5 an f32 product is off by 0.004 rad
@@ -478,17 +481,17 @@ __global__ __launch_bounds__(256) void latent_combine_kernel(LatentDecodeArgs a,
 constexpr int kQTile = 128;      // queries per workgroup: 16 per wave
 constexpr int kKTile = 64;       // keys per step
 
-// Workgroup = 128 queries x head x sequence, 8 waves.  Keys [unrotated | shared rotated part] and values of a step in LDS, the
-// next step's words in registers meanwhile.  Everything is transposed (scores: rows = keys, columns = queries; result:
-// rows = values), so a lane works on one query: softmax in f32 registers, the weights go from there into the product with the
-// values, as a bf16 value and its remainder.  KS: dim + rot in steps of 32, VT: vdim in tiles of 16 (both zero padded).
+// Workgroup = 128 queries (16 per wave) x head x sequence.  Keys [unrotated | shared rotated part] and values of a step in LDS, the
+// next step's words in registers meanwhile.  KS: dim + rot in steps of 32, VT: vdim in tiles of 16 (both zero padded).
+// Times, us, 32 heads of 128 + 64 and 128, before and after scalar masks, conflict-free values and queries loaded at once: 4 x 1000 120 -> 110, 1 x 3000
+// 226 -> 208, 1 x 333 19.4 -> 17.9.
 template <int KS, int VT>
 __global__ __launch_bounds__(512) void latent_prefill_kernel(LatentPrefillArgs a) {
     extern __shared__ __align__(16) unsigned char lat_smem[];
-    constexpr int KSTR = KS * 32 + 8, VSTR = VT * 16 + 8;
+    constexpr int KSTR = kPromptKeyStride<KS>, VSTR = kPromptValueStride<VT>;
     bf16_t* kt = reinterpret_cast<bf16_t*>(lat_smem);                 // [64][KSTR]
     bf16_t* vt = kt + kKTile * KSTR;                                  // [64][VSTR]
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 15, kg = lane >> 4;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), c = lane & 15, kg = lane >> 4;
     const XcdTile at = xcd_tile();
     const int b = at.z, h = at.y, T = a.len[b], r0 = a.row0[b];
     const int q0 = ((int)gridDim.x - 1 - (int)at.x) * kQTile;   // the longest workgroups first
@@ -501,7 +504,7 @@ __global__ __launch_bounds__(512) void latent_prefill_kernel(LatentPrefillArgs a
     // one repeat it (their scores are masked), columns behind a row's end repeat its start (the queries are zero there, or the
     // result is not stored).
     constexpr int KW = KS * 4, VW = VT * 2;                           // 16-byte words per staged row
-    constexpr int KU = kKTile * KW / 512, VU = (kKTile * VW + 511) / 512;   // ... per thread
+    constexpr int KU = kKTile * KW / 512, VU = kKTile * VW / 512;   // ... per thread
     static_assert(kKTile * KW % 512 == 0 && kKTile * VW % 512 == 0, "whole rounds of the workgroup");
     u32x4_m rk[KU], rv[VU];
     const char* kbase = (const char*)a.k + ((int64_t)r0 * H + h) * dim * 2;
@@ -530,23 +533,33 @@ __global__ __launch_bounds__(512) void latent_prefill_kernel(LatentPrefillArgs a
         const int row = r0 + min(qi, T - 1);
         const bf16_t* src = (const bf16_t*)a.x + ((int64_t)row * H + h) * hd;
         const float* tab = a.table + (int64_t)row * rot;
+        // every load is made, of a clamped place, before the first value is used: with tests around them each pair of cosines was a trip to memory of its own
+        f32x4_m cs[KS], sn[KS];
 #pragma unroll
-        for (int k = 0; k < KS; ++k) {
-            const int d = 32 * k + 8 * kg;
-            u32x4_m v = {0u, 0u, 0u, 0u};
-            if (d < hd) {
-                v = *reinterpret_cast<const u32x4_m*>(src + d);
-                if (d >= dim) {
+        for (int k = 0; k < KS; ++k) q[k] = *reinterpret_cast<const u32x4_m*>(src + min(32 * k + 8 * kg, hd - 8));
+        if (rot > 0) {
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+                if (32 * k + 24 >= dim) {
+                    const int i = min(max(32 * k + 8 * kg - dim, 0), rot - 8) / 2;
+                    cs[k] = *reinterpret_cast<const f32x4_u*>(tab + i);
+                    sn[k] = *reinterpret_cast<const f32x4_u*>(tab + rot / 2 + i);
+                }
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+                if (32 * k + 24 >= dim) {
+                    const bool turned = 32 * k + 8 * kg >= dim;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float cs = tab[(d - dim) / 2 + e], sn = tab[rot / 2 + (d - dim) / 2 + e];
-                        const float x0 = bf16lo(v[e]), x1 = bf16hi(v[e]);
-                        v[e] = pack_bf16_hw(x0 * cs - x1 * sn, x1 * cs + x0 * sn);
+                        const float x0 = bf16lo(q[k][e]), x1 = bf16hi(q[k][e]);
+                        const uint32_t r = pack_bf16_hw(x0 * cs[k][e] - x1 * sn[k][e], x1 * cs[k][e] + x0 * sn[k][e]);
+                        q[k][e] = turned ? r : q[k][e];
                     }
                 }
-            }
-            q[k] = v;
         }
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+            if (32 * k + 8 * kg >= hd) q[k] = u32x4_m{0u, 0u, 0u, 0u};
     }
     f32x4_m o[VT];
     float m = -INFINITY, l = 0.f;
@@ -568,58 +581,8 @@ __global__ __launch_bounds__(512) void latent_prefill_kernel(LatentPrefillArgs a
         __syncthreads();
         if (k0 + kKTile < kend) fetch(k0 + kKTile);
         if (k0 > myq + 15) continue;                                  // all keys of the step lie ahead of the wave's queries
-        f32x4_m s[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            s[j] = f32x4_m{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < KS; ++k) s[j] = mma16(*reinterpret_cast<const u32x4_m*>(kt + (16 * j + c) * KSTR + 32 * k + 8 * kg), q[k], s[j]);
-        }
-        const bool edge = k0 + kKTile - 1 > myq;                      // some key lies ahead of some query
-        float mx = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float x = s[j][e] * scale2;
-                if (edge && k0 + 16 * j + 4 * kg + e > qi) x = -INFINITY;
-                s[j][e] = x;
-                mx = fmaxf(mx, x);
-            }
-        // k0 and myq are multiples of 16 and k0 <= myq + 15, so every query sees key k0: the maximum is finite
-        const float mn = fmaxf(m, col4_max(mx));
-        float sum = 0.f;
-        u32x4_m ph[2], pl[2];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float u = __builtin_amdgcn_exp2f(s[j][2 * e] - mn), v = __builtin_amdgcn_exp2f(s[j][2 * e + 1] - mn);
-                sum += u + v;
-                uint32_t hi, lo;
-                split_bf16_hw(u, v, hi, lo);
-                ph[j / 2][2 * (j & 1) + e] = hi;
-                pl[j / 2][2 * (j & 1) + e] = lo;
-            }
-        sum = col4_sum(sum);
-        if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {               // some column's maximum has moved
-            const float corr = __builtin_amdgcn_exp2f(m - mn);
-            l *= corr;
-#pragma unroll
-            for (int v = 0; v < VT; ++v)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[v][e] *= corr;
-            m = mn;
-        }
-        l += sum;
-#pragma unroll
-        for (int k = 0; k < kKTile / 32; ++k)
-#pragma unroll
-            for (int v = 0; v < VT; ++v) {
-                const u32x4_m vv = lds_operand_t2(vt + 32 * k * VSTR + 16 * v, VSTR, lane);
-                o[v] = mma16(vv, ph[k], o[v]);
-                o[v] = mma16(vv, pl[k], o[v]);
-            }
+        // the first step holds key 0, which every query sees: maxima are finite from there on
+        prompt_attn_step<KS, VT>(kt, vt, q, o, m, l, scale2, k0, lane, k0 + kKTile - 1 > myq, [&](int key) { return key > qi; });
     }
     if (qi >= T) return;
     const float inv = 1.0f / l;
@@ -753,7 +716,7 @@ size_t latent_prefill_scratch_bytes(int dtype, int64_t total, int64_t heads, int
 }
 template <int KS, int VT>
 static void launch_prefill(hipStream_t s, const LatentPrefillArgs& a, int64_t longest) {
-    constexpr int lds = kKTile * (KS * 32 + 8 + VT * 16 + 8) * 2;
+    constexpr int lds = kKTile * (kPromptKeyStride<KS> + kPromptValueStride<VT>) * 2;
     static_assert(lds <= 160 * 1024, "LDS of one CU");
     with_lds(latent_prefill_kernel<KS, VT>, lds);
     latent_prefill_kernel<KS, VT><<<dim3((unsigned)cdiv_l(longest, kQTile), (unsigned)a.heads, (unsigned)a.nseq), 512, lds, s>>>(a);

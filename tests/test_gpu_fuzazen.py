@@ -271,6 +271,12 @@ def test_prompt_and_single_keys(hip, dt, shape, lens, chunk):
             check(g, w, TOL[dt], (shape, lens, chunk, fusion, "cache"))
 
 
+@pytest.mark.parametrize("lens,chunk", [([129], 128), ([700, 256, 100, 513], 256), ([385, 384, 1], 384)])
+def test_prompts_over_chunks_of_whole_tiles(hip, lens, chunk):
+    """Tiles of 128 queries are taken chunk by chunk from the chunks' ends on: prompts that end at a chunk's end, behind it and inside the first."""
+    test_prompt_and_single_keys(hip, "Bf16", (4, 2, 64, 24, 16), lens, chunk)
+
+
 @pytest.mark.parametrize("dt", ["F32", "Bf16"])
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("pos,cap,chunk", [([0], 4, 9), ([63, 64, 65], 128, 1000), ([127, 128, 255, 0], 128, 128), ([2000, 2047, 2048, 5], 1024, 1024),
