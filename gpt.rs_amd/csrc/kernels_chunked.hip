@@ -222,10 +222,13 @@ constexpr int kDecHeads = 16;    // query heads per workgroup (of one key / valu
 // remainder) feed the product with the values from there.  The slices' records (sums, maximum in base 2, weight) meet through
 // `part`: the workgroup that draws the last ticket merges them, adds the sink to the denominator and applies the gate.  KS: dim
 // in steps of 32, VT: vdim in tiles of 16 (both zero padded).
+// Bound by trips to memory one after another, and by the fetching of code that other launches have put out of the instruction cache: 1 sequence, 900 rows,
+// 32 / 8 heads of 128 + 128, us between launches of the chain: 12.9 with queries, angles and keys loaded where they are used; 11.5 loaded ahead, with the first
+// records beside their weights (4100 instructions); 10.4 with loops that run once or twice left rolled (2700).
 template <int KS, int VT>
 __global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkSeqArgs a, float* __restrict__ part, unsigned* __restrict__ tickets, int ns) {
     extern __shared__ __align__(16) unsigned char chk_smem[];
-    constexpr int QS = KS * 32 + 8, VS = VT * 16 + 8, VW = VT * 2, VP = VT * 16;
+    constexpr int QS = KS * 32 + 8, VS = kPromptValueStride<VT>, VW = VT * 2, VP = VT * 16;
     bf16_t* qs = reinterpret_cast<bf16_t*>(chk_smem);                 // [16][QS]
     bf16_t* knew = qs + kDecHeads * QS;                               // [QS]
     bf16_t* vnew = knew + QS;                                         // [VS]
@@ -238,17 +241,41 @@ __global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkSeqArgs a, float
     const int ht = (per_kv + kDecHeads - 1) / kDecHeads;
     const int b = blockIdx.z, g = (int)blockIdx.y / ht, h0 = g * per_kv + (int)blockIdx.y % ht * kDecHeads, sp = blockIdx.x;
     const int nh = min(kDecHeads, (g + 1) * per_kv - h0);             // heads that exist
+    // what the step itself brings is requested first, all of it, from clamped places, since loads are answered in order: the thread's two of every 32 dims of its
+    // query (16 lanes to a head) and of the new key, their angles, a value, and a gate and a sink for whoever merges
+    const int l16 = t & 15, hl = min(t >> 4, nh - 1);
+    const float* prow = a.proj + (int64_t)(a.row0[b]) * a.ld;
+    const float* tab = a.table + (int64_t)a.row0[b] * rot;
+    const float* gate = prow + (int64_t)(H + G) * D + (int64_t)G * V;
+    float qx[KS][2], kx[KS][2], cs[KS], sn[KS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const int d = min(32 * k + 2 * l16, D - 2);
+        const float *xq = prow + (int64_t)(h0 + hl) * D + d, *xk = prow + (int64_t)(H + g) * D + d;
+        qx[k][0] = xq[0]; qx[k][1] = xq[1];
+        kx[k][0] = xk[0]; kx[k][1] = xk[1];
+        cs[k] = sn[k] = 0.f;
+    }
+    if (rot > 0) {
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            const int d2 = min(16 * k + l16, rot / 2 - 1);
+            cs[k] = tab[d2];
+            sn[k] = tab[rot / 2 + d2];
+        }
+    }
+    const float vx = prow[(int64_t)(H + G) * D + (int64_t)g * V + min(t, V - 1)];
+    static_assert(VP <= 256, "a thread to a value");
+    float gt = gate[h0 + min(wave, nh - 1)], sk = a.sink[h0 + min(wave, nh - 1)];
     const int C = (int)a.rows, p = max(a.pos[b], 0), upd = clamp_row(a.starts[3 * b + 1], C - 1);
     const int n = min((a.chunk > 0 ? (int)(p % a.chunk) : p) + 1, C);
     const int per = ((n + ns - 1) / ns + kDecTile - 1) / kDecTile * kDecTile;
     const int p0 = sp * per, p1 = min(p0 + per, n);
     const bool owner = upd >= p0 && (upd < p0 + per || sp == ns - 1); // this slice holds the new row (or the row lies behind the last seen one)
-    const float* prow = a.proj + (int64_t)(a.row0[b]) * a.ld;
-    const float* tab = a.table + (int64_t)a.row0[b] * rot;
     bf16_t* kc = (bf16_t*)a.kcache[b] + (int64_t)g * C * D;
     bf16_t* vc = (bf16_t*)a.vcache[b] + (int64_t)g * C * V;
 
-    // the first step's cache rows are requested ahead of everything else.  Rows behind the last one repeat it (weight zero),
+    // the first step's cache rows are on their way while those are worked on.  Rows behind the last one repeat it (weight zero),
     // columns behind a row's end repeat its start (the queries are zero there, or the sums are not used).
     u32x4_m kf[2][KS], vw[VT];
     auto fetch = [&](int r0) {
@@ -267,39 +294,30 @@ __global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkSeqArgs a, float
     const int r_first = p0 + wave * kDecTile;
     if (r_first < p1) fetch(r_first);
 
-    // queries: 16 lanes to a head, and once more for the new key
-    auto prepare = [&](const float* x, bf16_t* to, bool live) {
-        const int l16 = t & 15;
+    auto prepare = [&](const float (&x)[KS][2], bf16_t* to, bool live, bool store) {
         float u[KS], v[KS], q = 0.f;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
             const int d = 32 * k + 2 * l16;
-            u[k] = v[k] = 0.f;
-            if (live && d < D) {
-                const float x0 = x[d], x1 = x[d + 1];
-                u[k] = x0; v[k] = x1;
-                if (d < rot) {
-                    const float cs = tab[d >> 1], sn = tab[rot / 2 + (d >> 1)];
-                    u[k] = x0 * cs - x1 * sn;
-                    v[k] = x1 * cs + x0 * sn;
-                }
-            }
+            const float ut = x[k][0] * cs[k] - x[k][1] * sn[k], vt2 = x[k][1] * cs[k] + x[k][0] * sn[k];
+            u[k] = live && d < D ? (d < rot ? ut : x[k][0]) : 0.f;
+            v[k] = live && d < D ? (d < rot ? vt2 : x[k][1]) : 0.f;
             q += u[k] * u[k] + v[k] * v[k];
         }
         const float inv = 1.0f / sqrtf(row16_sum(q) / (float)D + a.eps);
+        if (!store) return;
 #pragma unroll
         for (int k = 0; k < KS; ++k) *reinterpret_cast<uint32_t*>(to + 32 * k + 2 * l16) = pack_bf16_hw(u[k] * inv, v[k] * inv);
     };
-    prepare(prow + (int64_t)(h0 + min(t >> 4, nh - 1)) * D, qs + (t >> 4) * QS, (t >> 4) < nh);
+    prepare(qx, qs + (t >> 4) * QS, (t >> 4) < nh, true);
     if (owner) {
-        if (t < 16) prepare(prow + (int64_t)(H + g) * D, knew, true);
-        const float* xv = prow + (int64_t)(H + G) * D + (int64_t)g * V;
-        for (int d = t; d < VP; d += 256) vnew[d] = d < V ? f32_to_bf16(xv[d]) : (bf16_t)0;
+        prepare(kx, knew, true, t < 16);
+        if (t < VP) vnew[t] = t < V ? f32_to_bf16(vx) : (bf16_t)0;
     }
     __syncthreads();
     if (owner && (int)blockIdx.y % ht == 0) {
-        for (int d = t; d < D; d += 256) kc[(int64_t)upd * D + d] = knew[d];
-        for (int d = t; d < V; d += 256) vc[(int64_t)upd * V + d] = vnew[d];
+        if (t < D) kc[(int64_t)upd * D + t] = knew[t];
+        if (t < V) vc[(int64_t)upd * V + t] = vnew[t];
     }
 
     f32x4_m o[VT];                                                    // rows: values, column: head c
@@ -373,31 +391,31 @@ __global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkSeqArgs a, float
     if (kg == 0) { sm[wave][c] = m_run; sl[wave][c] = l_run; }
     __syncthreads();
 
-    const float* gate = prow + (int64_t)(H + G) * D + (int64_t)G * V;
     bf16_t* ctx = (bf16_t*)a.ctx + (int64_t)a.row0[b] * H * V;
-    const int rs = V + 2;
-    float* rec = part + ((int64_t)b * H + h0) * ns * rs;              // of head h0: [ns][rs]
-    for (int i = t; i < nh * V; i += 256) {
-        const int h = i / V, d = i % V;
+    const int rs = V + 2, pairs = nh * (V / 2);                       // a thread takes two values that are neighbours
+    float* rec = part + ((int64_t)b * H + h0) * ns * rs;              // of head h0: [ns][rs], 8-byte aligned
+#pragma unroll 1
+    for (int i = t; i < pairs; i += 256) {
+        const int h = i / (V / 2), d = i % (V / 2) * 2;
         const float mm = fmaxf(fmaxf(sm[0][h], sm[1][h]), fmaxf(sm[2][h], sm[3][h]));
-        float L = 0.f, O = 0.f;
+        float L = 0.f;
+        float2 O = make_float2(0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             const float f = sm[w][h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sm[w][h] - mm);
+            const float2 x = *reinterpret_cast<const float2*>(so + (w * kDecHeads + h) * VP + d);
             L += f * sl[w][h];
-            O += f * so[(w * kDecHeads + h) * VP + d];
+            O.x += f * x.x;
+            O.y += f * x.y;
         }
         if (ns == 1) {
             const float s2 = a.sink[h0 + h] * 1.44269504f, mt = fmaxf(mm, s2);
-            const float f = __builtin_amdgcn_exp2f(mm - mt), den = L * f + __builtin_amdgcn_exp2f(s2 - mt);
-            ctx[(int64_t)(h0 + h) * V + d] = f32_to_bf16(O * f / den * sigmoid_f32(gate[h0 + h]));
+            const float f = __builtin_amdgcn_exp2f(mm - mt), den = L * f + __builtin_amdgcn_exp2f(s2 - mt), sg = sigmoid_f32(gate[h0 + h]);
+            *reinterpret_cast<uint32_t*>(ctx + (int64_t)(h0 + h) * V + d) = pack_bf16_hw(O.x * f / den * sg, O.y * f / den * sg);
         } else {
             float* r = rec + ((int64_t)h * ns + sp) * rs;
-            __hip_atomic_store(r + d, O, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (d == 0) {
-                __hip_atomic_store(r + V, mm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(r + V + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            __hip_atomic_store(reinterpret_cast<uint64_t*>(r + d), __builtin_bit_cast(uint64_t, O), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (d == 0) __hip_atomic_store(reinterpret_cast<uint64_t*>(r + V), __builtin_bit_cast(uint64_t, make_float2(mm, L)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     if (ns == 1) return;
@@ -411,30 +429,55 @@ __global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkSeqArgs a, float
     if (drawn + 1 != (unsigned)ns) return;
     asm volatile("" ::: "memory");
     if (t == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // zero for the next launch
+    // the first records of the thread's outputs are requested with the slices' weights
+    constexpr int U = 8;
+    float2 x[U];
+    auto records = [&](int i, int s0) {
+        const float* r = rec + (int64_t)(i / (V / 2)) * ns * rs + i % (V / 2) * 2;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            x[u] = __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(r + (int64_t)min(s0 + u, ns - 1) * rs), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    };
+    auto slices = [&](int h) {                                        // ns <= 64: a lane per slice
+        return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(rec + ((int64_t)min(h, nh - 1) * ns + min(lane, ns - 1)) * rs + V),
+                                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    };
+    float2 ml = slices(wave);
+    records(min(t, pairs - 1), 0);
     float* wgt = so;                                                  // [16][ns], with the denominator and the gate in it
-    for (int h = wave; h < nh; h += 4) {                              // ns <= 64: a lane per slice
-        const float* r = rec + ((int64_t)h * ns + min(lane, ns - 1)) * rs + V;
-        const float mv = __hip_atomic_load(r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), lv = __hip_atomic_load(r + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const float s2 = a.sink[h0 + h] * 1.44269504f;
-        const float mt = fmaxf(wave_max(lane < ns ? mv : -INFINITY), s2);
-        const float f = lane < ns && mv != -INFINITY ? __builtin_amdgcn_exp2f(mv - mt) : 0.f;
-        const float den = wave_sum(f * lv) + __builtin_amdgcn_exp2f(s2 - mt);
-        if (lane < ns) wgt[h * ns + lane] = f / den * sigmoid_f32(gate[h0 + h]);
+#pragma unroll 1
+    for (int h = wave; h < nh;) {
+        const float s2 = sk * 1.44269504f;
+        const float mt = fmaxf(wave_max(lane < ns ? ml.x : -INFINITY), s2);
+        const float f = lane < ns && ml.x != -INFINITY ? __builtin_amdgcn_exp2f(ml.x - mt) : 0.f;
+        const float den = wave_sum(f * ml.y) + __builtin_amdgcn_exp2f(s2 - mt);
+        if (lane < ns) wgt[h * ns + lane] = f / den * sigmoid_f32(gt);
+        h += 4;
+        if (h < nh) {
+            ml = slices(h);
+            gt = gate[h0 + h];
+            sk = a.sink[h0 + h];
+        }
     }
     __syncthreads();
-    for (int i = t; i < nh * V; i += 256) {
-        const int h = i / V, d = i % V;
-        const float* r = rec + (int64_t)h * ns * rs + d;
-        float v = 0.f;
-        constexpr int U = 8;
-        for (int s0 = 0; s0 < ns; s0 += U) {
-            float x[U];
+    float2 v = make_float2(0.f, 0.f);
+#pragma unroll 1
+    for (int i = t, s0 = 0; i < pairs;) {
+        const int h = i / (V / 2);
 #pragma unroll
-            for (int u = 0; u < U; ++u) x[u] = __hip_atomic_load(r + (int64_t)min(s0 + u, ns - 1) * rs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-            for (int u = 0; u < U; ++u) v += s0 + u < ns ? wgt[h * ns + s0 + u] * x[u] : 0.f;
+        for (int u = 0; u < U; ++u) {
+            const float f = s0 + u < ns ? wgt[h * ns + s0 + u] : 0.f;
+            v.x += s0 + u < ns ? f * x[u].x : 0.f;
+            v.y += s0 + u < ns ? f * x[u].y : 0.f;
         }
-        ctx[(int64_t)(h0 + h) * V + d] = f32_to_bf16(v);
+        s0 += U;
+        if (s0 >= ns) {
+            *reinterpret_cast<uint32_t*>(ctx + (int64_t)(h0 + h) * V + i % (V / 2) * 2) = pack_bf16_hw(v.x, v.y);
+            v = make_float2(0.f, 0.f);
+            i += 256;
+            s0 = 0;
+        }
+        if (i < pairs) records(i, s0);
     }
 }
 
@@ -624,10 +667,10 @@ size_t chunk_decode_scratch_bytes(int dtype, int64_t nseq, int64_t rows, int64_t
 }
 template <int KS, int VT>
 static void launch_decode(hipStream_t s, const ChunkSeqArgs& a) {
-    constexpr size_t rows = (size_t)4 * kDecTile * (VT * 16 + 8) * 2, sums = (size_t)4 * kDecHeads * VT * 16 * 4;
-    constexpr size_t lds = (size_t)(kDecHeads * (KS * 32 + 8) + KS * 32 + 8 + VT * 16 + 8) * 2 + (rows > sums ? rows : sums);
+    constexpr size_t rows = (size_t)4 * kDecTile * kPromptValueStride<VT> * 2, sums = (size_t)4 * kDecHeads * VT * 16 * 4;
+    constexpr size_t lds = (size_t)(kDecHeads * (KS * 32 + 8) + KS * 32 + 8 + kPromptValueStride<VT>) * 2 + (rows > sums ? rows : sums);
     static_assert(lds + 1024 <= 160 * 1024, "LDS of one CU");
-    static_assert(((KS * 32 + 8) * 2) % 16 == 0 && ((VT * 16 + 8) * 2) % 16 == 0, "16-byte rows");
+    static_assert(((KS * 32 + 8) * 2) % 16 == 0 && (kPromptValueStride<VT> * 2) % 16 == 0, "16-byte rows");
     with_lds(chunk_decode_kernel<KS, VT>, lds);
     const int64_t ns = chunk_nsplit(a.nseq, a.rows, a.heads, a.kv_heads);
     const dim3 grid((unsigned)ns, (unsigned)(a.kv_heads * cdiv_c(a.heads / a.kv_heads, kDecHeads)), (unsigned)a.nseq);

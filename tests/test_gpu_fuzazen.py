@@ -320,6 +320,12 @@ def test_decode_of_a_batch_and_single_rows(hip, dt, shape, pos, cap, chunk):
             check(g, w, TOL[dt], (shape, pos, fusion, "cache"))
 
 
+@pytest.mark.parametrize("shape,pos,cap", [((5, 1, 64, 136, 16), [1199, 130], 1280), ((16, 1, 32, 64, 0), [1023, 0], 1152), ((4, 2, 128, 128, 128), [128, 1152], 1153)])
+def test_merge_of_many_slices_heads_and_values(hip, shape, pos, cap):
+    """More slices than a thread's records at a time (nine and ten of 128 rows), more heads than waves, more pairs of values than threads."""
+    test_decode_of_a_batch_and_single_rows(hip, "Bf16", shape, pos, cap, 2000)
+
+
 # ------------------------------------------------------------------------------------------ whole models
 def load(hip, tmp_path, name, dt, seed=0, **kw):
     cfg = U.STACKS[name]
