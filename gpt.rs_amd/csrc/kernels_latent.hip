@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void latent_attn_x_kernel(LatentAttnXArgs a) {
 
 // ---------------------------------------------------------------------------- decode (bf16)
 constexpr int kPrepRows = 64;    // latent dimensions per workgroup of the query part
-constexpr int kTileP = 64;       // cache rows per step of the attention part
+constexpr int kTileP = 32;       // cache rows per step of the attention part
 constexpr int kHeadTile = 16;
 
 // Blocks [0, heads * rank / 64): W_uk^T q_n of one head and 64 latent dimensions, for every sequence (the first of a head
@@ -276,9 +276,13 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentDecodeArgs a, bf
 }
 
 // Workgroup = slice of the positions x sequence x up to 4 waves; a wave = 16 heads and 16 RT latent dimensions of their result, and
-// all waves share the cache rows, 64 at a time in LDS.  Scores transposed (rows: positions, columns: heads), so a lane holds 16
+// all waves share the cache rows, 32 at a time in LDS.  Scores transposed (rows: positions, columns: heads), so a lane holds 8
 // positions of one head: softmax in registers, and the weights (a bf16 value and its remainder) feed the product with the
 // cached latents from there.  part f32 [nseq][heads][nsplit][rank + 2]: sums, maximum (base 2), weight.
+// Bound by its chain of trips to memory and LDS and by the code it fetches (other launches put it out of the instruction cache), not by bytes: 32 heads, rank 512 + 64, us,
+// with 64 rows to a step and a slice and the rows requested behind the queries' stores, and now: 8 x 71 positions 11.9 -> 8.9, 8 x 246 12.5 -> 9.7,
+// 2 x 906 13.9 -> 11.1, 1 x 2906 20.7 -> 18.1.  Dropped: steps of 64 rows over slices of 32, with a shorter form for the last 32 (10.6, 11.3, 12.5, 19.8), slices of 16
+// (9.1, 10.6, 11.0, 18.2).
 template <int RT>
 __global__ __launch_bounds__(256) void latent_partial_kernel(LatentDecodeArgs a, const bf16_t* __restrict__ ql, float* __restrict__ part, int nsplit) {
     extern __shared__ __align__(16) unsigned char lat_smem[];
@@ -305,27 +309,31 @@ __global__ __launch_bounds__(256) void latent_partial_kernel(LatentDecodeArgs a,
     const int wv = w / 8;                                             // 16-byte words per row (a multiple of 4)
     const bf16_t* cache = (const bf16_t*)a.cache[b];
     // 8 threads to a row: a thread takes every eighth word of it
-    auto stage = [&](const bf16_t* src, bf16_t* dst, int nrows, int last) {   // rows behind `last` repeat it
-        constexpr int R = 2, U = 10;                                  // rows x words per thread requested before the first is stored
-        for (int r0 = tid >> 3; r0 < nrows; r0 += 8 * W * R)
+    constexpr int U = 10;                                             // words per thread requested before the first is stored
+    auto request = [&](u32x4_m (&v)[U], const bf16_t* src, int r, int k0, int last) {   // rows behind `last` repeat it
+        const u32x4_m* from = reinterpret_cast<const u32x4_m*>(src + (int64_t)min(r, last) * w);
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = from[min(k0 + 8 * u, wv - 1)];
+    };
+    auto stage = [&](u32x4_m (&v)[U], bool first, const bf16_t* src, bf16_t* dst, int nrows, int last) {   // first: v holds the first round's words
+        for (int r = tid >> 3; r < nrows; r += 8 * W)
             for (int k0 = tid & 7; k0 < wv; k0 += 8 * U) {
-                u32x4_m v[R][U];
+                if (!first) request(v, src, r, k0, last);
+                first = false;
+                u32x4_m* to = reinterpret_cast<u32x4_m*>(dst + r * ws);
 #pragma unroll
-                for (int i = 0; i < R; ++i) {
-                    const u32x4_m* from = reinterpret_cast<const u32x4_m*>(src + (int64_t)min(r0 + 8 * W * i, last) * w);
-#pragma unroll
-                    for (int u = 0; u < U; ++u) v[i][u] = from[min(k0 + 8 * u, wv - 1)];
-                }
-#pragma unroll
-                for (int i = 0; i < R; ++i) {
-                    u32x4_m* to = reinterpret_cast<u32x4_m*>(dst + (r0 + 8 * W * i) * ws);
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (r0 + 8 * W * i < nrows && k0 + 8 * u < wv) to[k0 + 8 * u] = v[i][u];
-                }
+                for (int u = 0; u < U; ++u)
+                    if (k0 + 8 * u < wv) to[k0 + 8 * u] = v[u];
             }
     };
-    stage(ql + ((int64_t)b * H + ht0 * kHeadTile) * w, q0s, (ht1 - ht0 + 1) * kHeadTile, H - 1 - ht0 * kHeadTile);
+    u32x4_m rw[U];                                                    // the first rows are requested with the queries
+    {
+        u32x4_m qw[U];
+        const bf16_t* from = ql + ((int64_t)b * H + ht0 * kHeadTile) * w;
+        request(qw, from, tid >> 3, tid & 7, H - 1 - ht0 * kHeadTile);
+        request(rw, cache + (int64_t)p0 * w, tid >> 3, tid & 7, min(kTileP, p1 - p0) - 1);
+        stage(qw, true, from, q0s, (ht1 - ht0 + 1) * kHeadTile, H - 1 - ht0 * kHeadTile);
+    }
     const bf16_t* qs = q0s + (ht - ht0) * kHeadTile * ws;
     f32x4_m acc[RT];                                                  // rows: latent dimensions, column: head c
 #pragma unroll
@@ -335,7 +343,7 @@ __global__ __launch_bounds__(256) void latent_partial_kernel(LatentDecodeArgs a,
     for (int q0 = p0; q0 < p1; q0 += kTileP) {
         const int np = min(kTileP, p1 - q0);
         __syncthreads();
-        stage(cache + (int64_t)q0 * w, rows, kTileP, np - 1);
+        stage(rw, q0 == p0, cache + (int64_t)q0 * w, rows, kTileP, np - 1);
         __syncthreads();
         constexpr int PT = kTileP / 16;
         f32x4_m sc[PT];
@@ -430,7 +438,7 @@ __global__ __launch_bounds__(256) void latent_combine_kernel(LatentDecodeArgs a,
         for (int u = 0; u < SU; ++u) dst[u] = *reinterpret_cast<const float2*>(rec + (int64_t)min(s0 + u, nsplit - 1) * rs + min(r, rank - 2));
     };
     records(2 * t, 0, y[0]);
-    records(2 * t, SU, y[1]);
+    if (nsplit > SU) records(2 * t, SU, y[1]);
     {   // every wave finds the weights of the (at most 32) slices; wave 0 leaves them in LDS
         const float m = wave_max(mv), e = __builtin_amdgcn_exp2f(mv - m);
         const float l = wave_sum(e * lv);
@@ -438,16 +446,21 @@ __global__ __launch_bounds__(256) void latent_combine_kernel(LatentDecodeArgs a,
     }
     __syncthreads();
     for (int r = 2 * t; r < rank; r += 512) {
-        if (r != 2 * t) { records(r, 0, y[0]); records(r, SU, y[1]); }
+        if (r != 2 * t) {
+            records(r, 0, y[0]);
+            if (nsplit > SU) records(r, SU, y[1]);
+        }
         float2 v = make_float2(0.f, 0.f);
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < 2; ++q) {
+            if (q * SU >= nsplit) break;
 #pragma unroll
             for (int u = 0; u < SU; ++u) {
                 const float f = wgt[q * SU + u];   // zero behind the last slice, and for an empty one, whose sums are unset
                 v.x += f != 0.f ? f * y[q][u].x : 0.f;
                 v.y += f != 0.f ? f * y[q][u].y : 0.f;
             }
+        }
         lat[r] = v.x;
         lat[r + 1] = v.y;
     }
@@ -644,7 +657,7 @@ void latent_attn_expanded(hipStream_t s, const LatentAttnXArgs& a) {
 
 
 static size_t lat_align(size_t n) { return (n + 255) / 256 * 256; }
-// slices of the positions: 64 rows each up to 32 of them, fewer where the batch fills the chip by itself
+// slices of the positions: 32 rows each up to 32 of them, fewer where the batch fills the chip by itself
 static int latent_nsplit(int64_t nseq, int64_t capacity, int64_t heads) {
     const int64_t blocks = nseq * cdiv_l(heads, kHeadTile);
     int64_t n = std::min<int64_t>(cdiv_l(capacity, kTileP), 32);
@@ -656,7 +669,7 @@ static size_t latent_partial_lds(int64_t w, int64_t head_tiles = 1) {
 }
 static bool latent_fast(int dtype, int64_t heads, int64_t dim, int64_t rot, int64_t rank, int64_t vdim) {
     return dtype == 2 && heads >= 1 && dim % 8 == 0 && vdim % 8 == 0 && rot % 2 == 0 && rank % 16 == 0 && (rank + rot) % 32 == 0 && rank <= 1024 && dim <= 512 &&
-           latent_partial_lds(rank + rot) <= 160 * 1024;
+           (64 + kHeadTile) * (rank + rot + 8) * 2 <= 160 * 1024;
 }
 size_t latent_decode_scratch_bytes(int dtype, int64_t nseq, int64_t capacity, int64_t heads, int64_t dim, int64_t rot, int64_t rank, int64_t vdim) {
     if (latent_fast(dtype, heads, dim, rot, rank, vdim))

@@ -181,6 +181,13 @@ def test_decode_attention_of_a_batch(hip, dt, shape, lens):
             check(got[2 + b], want[2 + b], TOL[dt], "cache")
 
 
+@pytest.mark.parametrize("shape", [(33, 16, 32, 64, 24), (3, 16, 16, 976, 8)])
+@pytest.mark.parametrize("lens", [[511, 33, 481], [512]])
+def test_decode_attention_over_full_slices(hip, shape, lens):
+    """Slices of 32 rows that are full, one short and one over; three tiles of heads, and latents that take a thread several rounds to stage."""
+    test_decode_attention_of_a_batch(hip, "Bf16", shape, lens)
+
+
 @pytest.mark.parametrize("dt", ["F32", "Bf16"])
 @pytest.mark.parametrize("H,G,N,V,K,ng", [(4, 2, 16, 16, 4, 2), (3, 1, 12, 20, 2, 3), (8, 4, 64, 48, 4, 4), (2, 1, 128, 64, 3, 1), (2, 2, 200, 24, 4, 1), (6, 3, 8, 40, 5, 1)])
 @pytest.mark.parametrize("lens", [[1], [1, 1, 1], [2], [63], [64], [65, 1, 129], [16, 17]])
