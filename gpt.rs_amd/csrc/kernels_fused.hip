@@ -71,12 +71,72 @@ __global__ void layer_norm_long_kernel(const T* __restrict__ x, const T* __restr
         stf(out, i, ((ldf(row, i) - mean) * inv_std) * ldf(gamma, i) + ldf(beta, i));
 }
 
+// f32 rows, many of them: W waves to a row, 16 bytes a lane and instruction.  n % 4 == 0, at most 256 V4 W values, 16-byte aligned operands.
+// Four sums a lane, by place, put together in pairs: distance from 64 bits, values of mean 1 and spread 1, 768 of them 8.1e-8 (the kernel above 8.5e-8), 3072 8.6e-8 (1.0e-7).
+// Bound by memory, and at few rows by its one trip there.  us a launch, with a value at a time, and now, f32 rows of 768: 7 rows 3.2 -> 2.8, 512 4.8 -> 4.8, 2048
+// 6.4 -> 5.9, 8192 13.9 -> 10.1; rows of 3072 into bf16: 512 6.4 -> 5.9, 1000 11.2 -> 8.3, 3000 22.8 -> 12.2.  Dropped: a wave to a row of 3072 (7 rows 9.1, 1000 13.6, 3000 16.6).
+template <typename TO, int V4, int W>
+__global__ __launch_bounds__(256) void layer_norm_rows_kernel(const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta, TO* __restrict__ y,
+                                                              int64_t rows, int n, float inv_n, float eps) {
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    static_assert(W == 1 || W == 4, "waves of a workgroup of 256 threads to a row");
+    __shared__ float red[16];
+    const int t = threadIdx.x % (64 * W);
+    const int64_t r = W == 4 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= rows) return;
+    const auto total = [&](const f32x4_t& a) {
+        const float p = (a[0] + a[1]) + (a[2] + a[3]);
+        return W == 4 ? block_sum(p, red) : wave_sum(p);
+    };
+    const float* row = x + r * n;
+    f32x4_t v[V4], ga[V4], be[V4], s = {0.f, 0.f, 0.f, 0.f}, q = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < V4; ++j) v[j] = *reinterpret_cast<const f32x4_t*>(row + min(4 * (64 * W * j + t), n - 4));
+#pragma unroll
+    for (int j = 0; j < V4; ++j) {
+        ga[j] = *reinterpret_cast<const f32x4_t*>(gamma + min(4 * (64 * W * j + t), n - 4));
+        be[j] = *reinterpret_cast<const f32x4_t*>(beta + min(4 * (64 * W * j + t), n - 4));
+    }
+#pragma unroll
+    for (int j = 0; j < V4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += 4 * (64 * W * j + t) < n ? v[j][e] : 0.f;
+    const float mean = total(s) * inv_n;
+#pragma unroll
+    for (int j = 0; j < V4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[j][e] -= mean;
+            q[e] += 4 * (64 * W * j + t) < n ? v[j][e] * v[j][e] : 0.f;
+        }
+    const float inv_std = 1.0f / sqrtf(total(q) * inv_n + eps);
+#pragma unroll
+    for (int j = 0; j < V4; ++j) {
+        const int i = 4 * (64 * W * j + t);
+        const f32x4_t o = (v[j] * inv_std) * ga[j] + be[j];
+        if (i >= n) continue;
+        if constexpr (sizeof(TO) == 4) *reinterpret_cast<f32x4_t*>(y + r * n + i) = o;
+        else *reinterpret_cast<uint2*>(y + r * n + i) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+    }
+}
+
+// From how many rows of more than 768 values on four waves to a row beat sixteen, which have less to do each (us, 3072 values: 7 rows 4.0 and 4.2, 128 4.3 and 4.2, 256 4.9 and 4.9, 512
+// 6.4 and 5.9); shorter rows take a wave each, however few.
+constexpr int64_t kNormRows = 256;
+
 template <typename T, typename TO>
 static void layer_norm_t(hipStream_t s, const T* x, const T* g, const T* b, TO* y, int64_t rows, int64_t n, float inv_n,
                          float eps) {
     const int block = n <= 256 ? 64 : (n <= 1024 ? 256 : 1024);  // decode has ONE row: spread it over many lanes
     const int64_t per = cdiv(n, block);
     const unsigned grid = (unsigned)rows;
+    if constexpr (sizeof(T) == 4)
+        if ((n <= 768 || rows >= kNormRows) && n % 4 == 0 && n <= 4096 && (((uintptr_t)x | (uintptr_t)g | (uintptr_t)b | (uintptr_t)y) & 15u) == 0) {
+            if (n <= 768) layer_norm_rows_kernel<TO, 3, 1><<<(unsigned)cdiv(rows, 4), 256, 0, s>>>(x, g, b, y, rows, (int)n, inv_n, eps);
+            else if (n <= 3072) layer_norm_rows_kernel<TO, 3, 4><<<grid, 256, 0, s>>>(x, g, b, y, rows, (int)n, inv_n, eps);
+            else layer_norm_rows_kernel<TO, 4, 4><<<grid, 256, 0, s>>>(x, g, b, y, rows, (int)n, inv_n, eps);
+            return;
+        }
     if (per <= 4) layer_norm_kernel<T, TO, 4><<<grid, block, 0, s>>>(x, g, b, y, n, inv_n, eps);
     else if (per <= 16) layer_norm_kernel<T, TO, 16><<<grid, block, 0, s>>>(x, g, b, y, n, inv_n, eps);
     else layer_norm_long_kernel<T, TO><<<grid, 1024, 0, s>>>(x, g, b, y, n, inv_n, eps);

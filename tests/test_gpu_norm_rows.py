@@ -28,6 +28,27 @@ def test_rows(hip, n):
     assert (np.abs(ln - want) <= 2 * rel * (np.abs(want) + np.abs(b) + 4 * np.abs(g)) + 1e-6).all()
 
 
+@pytest.mark.parametrize("n", [4, 252, 256, 260, 764, 768, 772, 1024, 1028, 3072, 3076, 4096, 4100])
+@pytest.mark.parametrize("rows", [1, 255, 257])
+def test_layer_norm_of_many_rows(hip, rows, n):
+    """Rows that waves take 16 bytes at a time, on both sides of each line between the kernels and the last workgroup partly filled; f32 results and
+    bf16 ones; some rows far from zero."""
+    rng = np.random.default_rng(rows + n)
+    x, g, b = (rng.standard_normal(s, dtype=np.float32) for s in ((rows, n), (n,), (n,)))
+    x += (np.arange(rows) % 3)[:, None].astype(np.float32)
+    f32 = lambda *d: ("F32", list(d))   # noqa: E731
+    norm = lambda a, c, d: F.layer_norm(a, c, d, 1e-5)[0]   # noqa: E731
+    y = hip_run(hip, program([f32(rows, n), f32(n), f32(n)], lambda a, c, d: [norm(a, c, d)]), [x, g, b])[0]
+    y16 = hip_run(hip, program([f32(rows, n), f32(n), f32(n)], lambda a, c, d: [norm(a, c, d).cast("Bf16")]), [x, g, b])[0]
+    x64 = x.astype(np.float64)
+    c = x64 - x64.mean(axis=1, keepdims=True)
+    want = c / np.sqrt((c ** 2).mean(axis=1, keepdims=True) + 1e-5) * g + b
+    # as in test_rows; the mean's own roundings are those of values up to 2 + 4 in size, of rows whose spread is 1 (four values: down to a tenth)
+    tol = 2 * (np.sqrt(n) * 2.0 ** -24 + 2.0 ** -21) * (np.abs(want) + np.abs(b) + 4 * np.abs(g) * np.maximum(1, 3 / np.sqrt((c ** 2).mean(axis=1, keepdims=True) + 1e-5))) + 1e-6
+    assert (np.abs(y - want) <= tol).all()
+    assert (np.abs(np.asarray(y16, np.float32) - want) <= tol + 2.0 ** -8 * np.abs(want)).all()
+
+
 @pytest.mark.parametrize("ln", [False, True])
 @pytest.mark.parametrize("m,k,n", [(2, 64, 48), (8, 3072, 576), (16, 512, 2304)])
 def test_one_norm_of_several_layers(hip, ln, m, k, n):
