@@ -1452,14 +1452,15 @@ __device__ __forceinline__ float reduce_tile(const float (&acc)[4]) {
 }
 
 // ---------------------------------------------------------------------------- compute waves
-// s_waitcnt that waits until at most 3 * steps vector memory operations of the wave are in flight (and for nothing else);
-// the count is an immediate of the instruction
-// vector memory operations of the wave that are in flight, without waiting
+// vector memory operations of the wave that are in flight, without waiting: says when it is worth while to look.  That words have
+// landed is what the wait below says, and nothing is read out of the ring without it.
 __device__ __forceinline__ int vm_in_flight() {
     unsigned v;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_IB_STS)" : "=s"(v) : : "memory");
     return (int)((v & 15u) | ((v >> 18) & 0x30u));
 }
+// s_waitcnt that waits until at most N vector memory operations of the wave are in flight (and for nothing else); the count is
+// an immediate of the instruction
 template <int N> __device__ __forceinline__ void wait_vm_imm() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }
 __device__ __forceinline__ void wait_vm_count(int n) {   // steps without loads in flight (padding, tiles that do not exist): rare
     switch (n) {
@@ -1670,6 +1671,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
             if (i < want) {
                 while (vm_in_flight() > 0 && closed()) __builtin_amdgcn_s_sleep(1);
                 if (vm_in_flight() == 0 && closed()) {
+                    wait_vm_imm<0>();   // (of no length: nothing is in flight)
                     pend = 0u;
                     loads = 0;
                     const GPTRS_LDS u32x4* wp = mine + slot * (SW * CW);

@@ -19,7 +19,7 @@ exceeds."""
 import numpy as np
 import pytest
 
-from parity import FunctionBuilder, Program, assert_close, hip_run, oracle_run
+from parity import FunctionBuilder, Program, assert_close, hip_run, oracle_run, po
 from gptrs_amd import functional as F
 from gptrs_amd.ptir import f32_to_bf16_bits
 
@@ -254,6 +254,43 @@ def test_padded_steps_and_missing_tiles_are_stable(hip, k, n):
         got = np.asarray(hip_run(hip, p, [x, w])[0], np.float32)
         assert_close(got, plain, atol=2e-5, rtol=ULP, what=f"run {rep} vs per-linear kernel")
     assert hip.counter("chain_launches") == before + 25
+
+
+@pytest.mark.parametrize("fmt", ["f32", "bf16", "w8", "w4g128"])
+@pytest.mark.parametrize("k", [768, 2560])
+def test_steps_parked_before_a_phase_opens(hip, fmt, k):
+    """While a wave waits for a phase to open it moves the phase's first weights from its ring into registers.  Eight dependent layers in one launch, whose
+    later phases start from such words, give bit for bit what each layer gives in a launch of its own (the same sums in the same order), every time."""
+    x, ws = rnd(80, (1, k)), [rnd(81 + i, (k, k), 2.0 / np.sqrt(k)) for i in range(8)]
+    dt = "F32" if fmt == "f32" else "Bf16"
+    if fmt in ("f32", "bf16"):
+        specs, args, per = [(dt, [k, k])] * 8, ws, 1
+        layer = lambda a, w: a.matmul(w[0])   # noqa: E731
+    else:
+        quant = po.quantize_int8_per_channel if fmt == "w8" else po.quantize_int4_g128
+        args, per = [t for w in ws for t in quant(w)], 2
+        specs = [("Si8", [k, k]), (dt, [k])] * 8 if fmt == "w8" else [("Ui8", [k // 2, k]), (dt, [k // 128, k])] * 8
+        layer = lambda a, w: F.linear_quantized(a, *w)   # noqa: E731
+
+    def build(fb, a, *w):
+        for i in range(8):
+            a = layer(a, w[i * per:i * per + per])
+        return a
+
+    hip.set_option("chain_f32_min_kb", 0)
+    try:
+        want = x
+        for i in range(8):
+            one = prog(lambda fb, a, *w: layer(a, w), [(dt, [1, k]), *specs[i * per:i * per + per]])
+            want = np.asarray(hip_run(hip, one, [want, *args[i * per:i * per + per]])[0], np.float32)
+        p = prog(build, [(dt, [1, k]), *specs])
+        for rep in range(10):
+            before, phases = hip.counter("chain_launches"), hip.counter("chain_phases")
+            got = np.asarray(hip_run(hip, p, [x, *args])[0], np.float32)
+            assert (hip.counter("chain_launches") - before, hip.counter("chain_phases") - phases) == (1, 8)
+            assert np.array_equal(got, want), rep
+    finally:
+        hip.set_option("chain_f32_min_kb", 4096)
 
 
 # ------------------------------------------------------------------------------ f32 phases (GPT-2)
