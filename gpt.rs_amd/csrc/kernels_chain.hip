@@ -1352,6 +1352,9 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
                     epi_load(i, e_bw, e_rw, e_ga, e_gb);
                     epi_store(i, e_bw, e_rw, e_ga, e_gb);
                 }
+                // below a lane reads what other lanes of the wave have stored (no instruction: LDS serves a wave in order, the compiler has to as well)
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
             char* out = (char*)P.y;
             handed += NWS;

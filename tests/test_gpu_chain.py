@@ -125,6 +125,15 @@ def test_bias_gelu_residual(hip, k, n):
     run_both(hip, lambda fb, a, c, d, e: F.linear(a, c, d) + e, [[1, k], [k, n], [n], [1, n]], [x, w, b, r], 2e-5, 2e-5)
 
 
+@pytest.mark.parametrize("n", [16384, 33796])
+def test_bias_and_residual_of_many_columns(hip, n):
+    """64 columns to a workgroup, one round of the control wave's lanes, and 132: two rounds of staging biases and residuals, two columns a lane, and three
+    of reading them, a column a lane."""
+    x, w, b, r = rnd(42, (1, 64)), rnd(43, (64, n), 0.25), rnd(44, (n,)), rnd(45, (1, n))
+    run_both(hip, lambda fb, a, c, d, e: F.linear(a, c, d) + e, [[1, 64], [64, n], [n], [1, n]], [x, w, b, r], 2e-5, 2e-5)
+    run_both_f32(hip, lambda fb, a, c, d, e: F.linear(a, c, d) + e, [[1, 64], [64, n], [n], [1, n]], [x, w, b, r])
+
+
 @pytest.mark.parametrize("d,f", [(3072, 9216), (256, 640)])
 def test_block_tail_chain(hip, d, f):
     """out-proj (+residual) -> RMSNorm -> gate/up SwiGLU -> down (+residual) -> RMSNorm -> next
