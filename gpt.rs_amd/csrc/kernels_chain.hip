@@ -15,7 +15,8 @@
 //     wave return in order, so "this step has landed" is a wait on the count of loads in flight: a ring private to the wave
 //     needs no flags and no barrier.  The packed copy holds the words in the order of their
 //     requests, step by step over all workgroups, so that what the whole chip asks for at one time is one run of memory: a
-//     head of 805 MB streams at 6.0 TB/s, where a run of its own for every workgroup streamed at 5.1.
+//     head of 805 MB streams at 6.0 TB/s, where a run of its own for every workgroup streamed at 5.1.  What a wave has
+//     beyond the whole steps that all waves have (a step at most where tiles divide evenly) stands behind them.
 //   * The compute lanes read their words from the ring and multiply them by the activation vector staged in LDS (v_dot2 for
 //     bf16 pairs); at the end of a tile the wave leaves its part of the tile's 4 sums in LDS.
 //   * 1 control wave per workgroup adds the parts of a phase's tiles when all waves are done, a lane to each output column,
@@ -207,6 +208,11 @@ __device__ __forceinline__ int tile_count(int blk, int tlo, int trem) { return t
 // The first of a wave's words among the W of its workgroup: words [wave_first(W, w), wave_first(W, w + 1)) are wave w's.
 __host__ __device__ __forceinline__ int wave_first(int W, int w) { return (W * w) >> 3; }   // (W < 2^22)
 static_assert(NWS == 8, "wave_first");
+// Where the packed copy of a phase holds what wave `w` of workgroup `blk` asks for behind the `whole` steps that every wave has: its rest, a run of words.  All
+// workgroups' rests lie one behind the other, behind the whole steps; counted in words from there.  f0: wave_first.
+__host__ __device__ __forceinline__ int wave_rest(int blk, int w, int f0, int C, int tlo, int trem, int whole) {
+    return (blk * tlo + (blk < trem ? blk : trem)) * C + f0 - whole * (SW * (NWS * blk + w));   // the words of the workgroups and waves before, less what they have in whole steps
+}
 
 // ---------------------------------------------------------------------------- staging (all waves)
 // xs[j] = (x[2j], x[2j+1]) as a bf16 pair, zero beyond K; with norm: the value the stand-alone
@@ -1488,7 +1494,8 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
 
     // ---- request side: the wave's next step to ask for, in the order the steps are consumed.  Everything but the lane's offset
     // in a word is uniform.
-    int r_phase = -1, r_left = 0;     // words of the phase that are still to be asked for
+    int r_phase = -1, r_left = 0;     // words of the phase's whole steps, then of its rest, that are still to be asked for
+    int r_rest = 0, r_jump = 0;       // the rest that follows, and how many words further on it stands
     unsigned r_step_bytes = 0;
     unsigned long long r_base = 0;    // the next step's first word
     const unsigned lane_off = (unsigned)lane * 16u;
@@ -1503,16 +1510,22 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
             if (r_phase >= nphases) return false;
             const GPTRS_CONST ChainPhase* D = table + r_phase;
             if (uni(D->kind) != kChainLinear) continue;
-            const int W = tile_count(blk, uni(D->tlo), uni(D->trem)) * uni(D->C);
-            r_left = wave_first(W, wave + 1) - wave_first(W, wave);
-            if (r_left == 0) continue;
-            r_step_bytes = (unsigned)uni(D->step_bytes);
-            r_base = (unsigned long long)uni_ptr(D->w) + (unsigned)(blk * SLOT_BYTES + wave * STEP_BYTES);
+            const int tlo = uni(D->tlo), trem = uni(D->trem), C = uni(D->C), whole = uni(D->whole);
+            const int W = tile_count(blk, tlo, trem) * C, f0 = wave_first(W, wave);
+            const int words = wave_first(W, wave + 1) - f0;
+            if (words == 0) continue;
+            const int at = blk * (NWS * SW) + wave * SW, rest = wave_rest(blk, wave, f0, C, tlo, trem, whole);
+            r_left = whole > 0 ? SW * whole : words;
+            r_rest = words - r_left;
+            r_jump = rest - at;
+            r_step_bytes = whole > 0 ? (unsigned)uni(D->step_bytes) : (unsigned)STEP_BYTES;
+            r_base = (unsigned long long)uni_ptr(D->w) + ((unsigned long long)(unsigned)(whole > 0 ? at : rest) << 10);
             return true;
         }
     };
+    static_assert(CW * 16 == 1 << 10, "bytes of a word");
     bool r_more = r_seek();
-    // Asks for one step: a load per word that exists (three but for a phase's last step).  `pend` records how many loads each step
+    // Asks for one step: a load per word that exists (three but for the last step of a wave's rest).  `pend` records how many loads each step
     // in flight carries, two bits per step, oldest first.  Every load fetches words never fetched before, so all of them take the
     // same way through the memory system and return in the order of issue: a load that re-read words already in a cache was seen
     // to complete ahead of older ones, which a count of loads in flight cannot express.  A step's words lie one behind the other
@@ -1539,7 +1552,16 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
         if (++r_slot == RING_D) r_slot = 0;
         r_base += r_step_bytes;
         r_left -= cnt;
-        if (r_left == 0) r_more = r_seek();
+        if (r_left == 0) {
+            if (r_rest > 0) {
+                r_base += (long long)r_jump * (CW * 16);
+                r_step_bytes = (unsigned)STEP_BYTES;
+                r_left = r_rest;
+                r_rest = 0;
+            } else {
+                r_more = r_seek();
+            }
+        }
     };
     for (int i = 0; i < RING_D && r_more; ++i) request();
 
@@ -1783,18 +1805,22 @@ __global__ __launch_bounds__(NT, 1) void chain_kernel(const ChainPhase* __restri
 // Single: column = 4 * tile + c.  Dual (SwiGLU pair): columns interleaved, c = 0, 2 -> gate column 2 * tile + c / 2, c = 1, 3 -> the
 // same column of up, so one tile finishes two outputs.  A word holds 64 k-groups of the tile's 4 columns, lane l (16 bytes) group
 // 64 chunk + l: 2 k of each column in bf16, 1 in f32, 4 int8 codes, 8 int4 codes.  Zero (of codes: the biased zero) outside the matrix.
-// Place of word (tile, chunk) in the copy, in words: [step][workgroup][wave][3], the order in which the chip asks for them.
+// Place of word (tile, chunk) in the copy, in words: [step][workgroup][wave][3] for the steps that every wave of a workgroup with tiles has in full, the
+// order in which the chip asks for them, and behind those [workgroup][wave][rest].  Every word of the matrix once and nothing else.  (With the waves' last steps padded
+// to three words, and room in a step for workgroups without tiles, 3072 x 64 took 6.3 MB for 0.39, and the layers of GPT-2 small 528 MB for 340.)
 struct ChainOrder {
     int64_t ntiles, C, grid, tlo, trem;
+    __host__ __device__ int64_t active() const { return tlo > 0 ? grid : trem; }   // workgroups that have tiles
+    __host__ __device__ int64_t whole() const { return (tlo > 0 ? tlo : 1) * C / NWS / SW; }
     __host__ __device__ int64_t word(int64_t tile, int64_t chunk) const {
         const int64_t big = trem * (tlo + 1);
         const int64_t b = tile < big ? tile / (tlo + 1) : trem + (tile - big) / tlo;
         const int64_t t0 = b * tlo + (b < trem ? b : trem), W = (tlo + (b < trem ? 1 : 0)) * C, f = (tile - t0) * C + chunk;
-        const int64_t w = (8 * f + 7) / W, i = f - wave_first((int)W, (int)w);
-        return (((i / SW) * grid + b) * NWS + w) * SW + i % SW;
+        const int64_t w = (8 * f + 7) / W, f0 = wave_first((int)W, (int)w), i = f - f0, n = whole();
+        if (i < SW * n) return (((i / SW) * active() + b) * NWS + w) * SW + i % SW;
+        return n * active() * (NWS * SW) + wave_rest((int)b, (int)w, (int)f0, (int)C, (int)tlo, (int)trem, (int)n) + i - SW * n;
     }
-    int64_t steps() const { return (((tlo + (trem > 0 ? 1 : 0)) * C + NWS - 1) / NWS + SW - 1) / SW; }
-    int64_t words() const { return steps() * grid * NWS * SW; }
+    int64_t words() const { return ntiles * C; }
 };
 
 __device__ __forceinline__ const void* chain_column(const void* w, const void* w2, int64_t tile, int c, int64_t& col) {
@@ -1926,6 +1952,7 @@ static ChainOrder chain_order(int64_t k, int64_t n, bool dual, int wfmt) {
 }
 
 size_t chain_weight_bytes(int64_t k, int64_t n, bool dual, int wfmt) { return (size_t)(chain_order(k, n, dual, wfmt).words() * CW * 16); }
+int64_t chain_weight_word(int64_t k, int64_t n, bool dual, int wfmt, int64_t tile, int64_t chunk) { return chain_order(k, n, dual, wfmt).word(tile, chunk); }
 
 void chain_pack_weights(hipStream_t s, const void* w, const void* w2, void* out, int64_t k, int64_t n, int wfmt) {
     const ChainOrder o = chain_order(k, n, w2 != nullptr, wfmt);
@@ -1971,7 +1998,8 @@ bool chain_fill_phase(ChainPhase& p, int64_t k, int64_t n, bool dual, int wfmt) 
     p.C = (int)o.C;
     p.tlo = (int)o.tlo;
     p.trem = (int)o.trem;
-    p.step_bytes = (int)(o.grid * SLOT_BYTES);
+    p.whole = (int)o.whole();
+    p.step_bytes = (int)(o.active() * SLOT_BYTES);
     p.inv_c = 1.0f / (float)o.C;
     p.kind = kChainLinear;
     p.wfmt = wfmt;
