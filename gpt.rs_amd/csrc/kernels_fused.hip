@@ -120,8 +120,11 @@ __global__ __launch_bounds__(256) void layer_norm_rows_kernel(const float* __res
     }
 }
 
-// From how many rows of more than 768 values on four waves to a row beat sixteen, which have less to do each (us, 3072 values: 7 rows 4.0 and 4.2, 128 4.3 and 4.2, 256 4.9 and 4.9, 512
-// 6.4 and 5.9); shorter rows take a wave each, however few.
+// Rows of up to 768 values take a wave each, however few (us inside a graph, with the kernel above and now: 7 rows of 64 2.0 and 1.9, of 256 2.4 and 2.0, of 768 2.4 and 2.1; 8192 rows of
+// 64 4.3 and 4.2, of 256 5.5 and 5.0, of 640 11.4 and 7.2, of 768 12.3 and 8.1).  Rows of 772 to 1024 stay with that kernel, which takes them with 4 waves: the 12 values a lane of the
+// form below are 4 then, and lose (772: 512 rows 2.9 and 3.0, 2048 4.7 and 5.5, 8192 12.6 and 13.5; 1024: 2.9 and 3.1, 5.0 and 5.8, 14.0 and 14.7).  For longer rows it takes 16 waves, which
+// have less to do each: four beat them from kNormRows rows on (3072 values between other launches: 7 rows 4.0 and 4.2, 128 4.3 and 4.2, 256 4.9 and 4.9, 512 6.4 and 5.9; inside a graph
+// 256 rows 3.6 and 3.0, 512 4.8 and 3.8, 8192 46.4 and 29.8; 1028 values 3.1 and 2.6, 4.2 and 3.2, 36.5 and 14.9; 4096 4.0 and 3.4, 5.4 and 4.4, 51.7 and 39.4).
 constexpr int64_t kNormRows = 256;
 
 template <typename T, typename TO>
@@ -131,7 +134,7 @@ static void layer_norm_t(hipStream_t s, const T* x, const T* g, const T* b, TO* 
     const int64_t per = cdiv(n, block);
     const unsigned grid = (unsigned)rows;
     if constexpr (sizeof(T) == 4)
-        if ((n <= 768 || rows >= kNormRows) && n % 4 == 0 && n <= 4096 && (((uintptr_t)x | (uintptr_t)g | (uintptr_t)b | (uintptr_t)y) & 15u) == 0) {
+        if ((n <= 768 || (n > 1024 && rows >= kNormRows)) && n % 4 == 0 && n <= 4096 && (((uintptr_t)x | (uintptr_t)g | (uintptr_t)b | (uintptr_t)y) & 15u) == 0) {
             if (n <= 768) layer_norm_rows_kernel<TO, 3, 1><<<(unsigned)cdiv(rows, 4), 256, 0, s>>>(x, g, b, y, rows, (int)n, inv_n, eps);
             else if (n <= 3072) layer_norm_rows_kernel<TO, 3, 4><<<grid, 256, 0, s>>>(x, g, b, y, rows, (int)n, inv_n, eps);
             else layer_norm_rows_kernel<TO, 4, 4><<<grid, 256, 0, s>>>(x, g, b, y, rows, (int)n, inv_n, eps);

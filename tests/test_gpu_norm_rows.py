@@ -49,6 +49,16 @@ def test_layer_norm_of_many_rows(hip, rows, n):
     assert (np.abs(np.asarray(y16, np.float32) - want) <= tol + 2.0 ** -8 * np.abs(want)).all()
 
 
+@pytest.mark.parametrize("n", [772, 900, 1024])
+def test_layer_norm_of_772_to_1024_values_takes_one_way(hip, n):
+    """However many rows there are: bit for bit what each gives in a program of few rows (sums in the same order)."""
+    rng = np.random.default_rng(n)
+    x, g, b = (rng.standard_normal(s, dtype=np.float32) for s in ((300, n), (n,), (n,)))
+    f32 = lambda *d: ("F32", list(d))   # noqa: E731
+    run = lambda a: hip_run(hip, program([f32(*a.shape), f32(n), f32(n)], lambda a, c, d: [F.layer_norm(a, c, d, 1e-5)[0]]), [a, g, b])[0]   # noqa: E731
+    assert np.array_equal(run(x), np.concatenate([run(x[i:i + 100]) for i in range(0, 300, 100)]))
+
+
 @pytest.mark.parametrize("ln", [False, True])
 @pytest.mark.parametrize("m,k,n", [(2, 64, 48), (8, 3072, 576), (16, 512, 2304)])
 def test_one_norm_of_several_layers(hip, ln, m, k, n):
