@@ -3,7 +3,7 @@ the first length that is read again instead, lengths that are no multiple of eig
 import numpy as np
 import pytest
 
-from parity import hip_run
+from parity import hip_run, po
 from test_gpu_gemm_tiles import program
 from gptrs_amd import functional as F
 
@@ -79,13 +79,56 @@ def test_one_norm_of_several_layers(hip, ln, m, k, n):
     args = [x, *gs, b, *ws]
 
     def run(which):
-        return hip_run(hip, program(specs, lambda a, g, g2, c, *w: [bodies[i](norm(a, g, c), norm(a, g2, c), w, a, g, c) for i in which]), args)
+        got = hip_run(hip, program(specs, lambda a, g, g2, c, *w: [bodies[i](norm(a, g, c), norm(a, g2, c), w, a, g, c) for i in which]), args)
+        launches.append(hip.counter("last_program_launches"))
+        return got
 
+    launches = []
     together = run(range(5))
     for i, got in enumerate(together):
         assert np.array_equal(np.asarray(got, np.float32), np.asarray(run([i])[0], np.float32)), i
+    assert launches[0] == sum(launches[1:]) - 2, launches   # three layers under one norm
     h64 = x.astype(np.float64) - (x.astype(np.float64).mean(1, keepdims=True) if ln else 0)
     h64 = h64 / np.sqrt((h64 ** 2).mean(1, keepdims=True) + 1e-5) * gs[0] + (b if ln else 0)
     want = h64 @ ws[0].astype(np.float64)
     # the normed row and the weights rounded to bf16: 2^-9 each, of the products' root mean square in the mean; ten times that
     assert np.abs(together[0] - want).max() <= 10 * 2.0 ** -8.5 * np.sqrt((h64 ** 2).mean() * (ws[0] ** 2).mean() * k)
+
+
+@pytest.mark.parametrize("scheme,ln", [("bf16", False), ("bf16", True), ("w8", False), ("w4g128", False)])   # (a layer of codes takes no layer norm in)
+@pytest.mark.parametrize("m,k,n", [(2, 128, 48), (8, 1024, 576), (16, 512, 2304)])
+def test_one_norm_of_layers_with_operands(hip, scheme, ln, m, k, n):
+    """The same of layers that have a bias, a residual, both or neither, between their weights and the norm's gains, and of int8 and int4 codes with their
+    scales; a layer under other gains stands between them."""
+    rng = np.random.default_rng(m + k + n)
+    x, r = (rng.standard_normal((m, d), dtype=np.float32) for d in (k, n))
+    gs = [(1 + 0.1 * rng.standard_normal(k)).astype(np.float32) for _ in range(2)]
+    b = (0.1 * rng.standard_normal(k)).astype(np.float32)
+    bias = rng.standard_normal(n, dtype=np.float32)
+    ws = [rng.standard_normal((k, n), dtype=np.float32) * np.float32(k ** -0.5) for _ in range(5)]
+    norm = lambda a, g, c: (F.layer_norm(a, g, c, 1e-5) if ln else F.rms_norm(a, g, 1e-5))[0].cast("Bf16")   # noqa: E731
+    if scheme == "bf16":
+        weights, per, wspecs = ws, 1, [("Bf16", [k, n])] * 5
+        layer = lambda h, w, *more: F.linear(h, *w, *more)   # noqa: E731
+    else:
+        weights = [t for w in ws for t in (po.quantize_int8_per_channel if scheme == "w8" else po.quantize_int4_g128)(w)]
+        per, wspecs = 2, ([("Si8", [k, n]), ("Bf16", [n])] if scheme == "w8" else [("Ui8", [k // 2, n]), ("Bf16", [k // 128, n])]) * 5
+        layer = lambda h, w, *more: F.linear_quantized(h, *w, *more)   # noqa: E731
+    bodies = [lambda h, h2, w, d, e: layer(h, w[0], d),
+              lambda h, h2, w, d, e: layer(h, w[1]) + e,
+              lambda h, h2, w, d, e: layer(h2, w[2], d),
+              lambda h, h2, w, d, e: layer(h, w[3], d) + e,
+              lambda h, h2, w, d, e: layer(h, w[4])]
+    specs = [("F32", [m, k]), ("F32", [k]), ("F32", [k]), ("F32", [k]), ("Bf16", [n]), ("Bf16", [m, n])] + wspecs
+    args = [x, *gs, b, bias, r, *weights]
+
+    def run(which):
+        got = hip_run(hip, program(specs, lambda a, g, g2, c, d, e, *w: [bodies[i](norm(a, g, c), norm(a, g2, c), [w[per * j:per * j + per] for j in range(5)], d, e) for i in which]), args)
+        launches.append(hip.counter("last_program_launches"))
+        return got
+
+    launches = []
+    together = run(range(5))
+    for i, got in enumerate(together):
+        assert np.array_equal(np.asarray(got, np.float32), np.asarray(run([i])[0], np.float32)), i
+    assert launches[0] == sum(launches[1:]) - 3, launches   # four layers under one norm
