@@ -229,9 +229,9 @@ struct ChainPhase {
     const void* w; const void* x; const void* gamma; const void* bias; const void* residual;
     void* y;
     // C: words of a tile (1 KiB: 4 columns x 64 k-groups of the format).  Every workgroup has tlo tiles, the first trem one more.
-    // whole: steps of three words that every wave of a workgroup with tiles has; step_bytes: from one of them to the wave's next in the packed copy.
-    // units: of an attention phase.
-    int K, N, C, tlo, trem, whole, step_bytes, units, lds_bytes;
+    // whole: steps of three words that every wave of a workgroup with tiles has; step_bytes: from one of them to the wave's next in the packed copy;
+    // behind: words of all of them.  (An attention phase: none.)  units: of an attention phase.
+    int K, N, C, tlo, trem, whole, step_bytes, behind, units, lds_bytes;
     float inv_c;   // 1 / C
     float inv_n, eps;
     // quantised weights: wfmt 1 = int8 (16-byte word = 4 columns x 4 k, biased by 128; `scale`/`scale2` = the
@@ -261,6 +261,8 @@ bool chain_supported(int dtype, int64_t m, int64_t k, int64_t n, bool dual, bool
 size_t chain_weight_bytes(int64_t k, int64_t n, bool dual, int wfmt = kChainW16);
 // place of word `chunk` of a tile in the copy, in words of 1 KiB
 int64_t chain_weight_word(int64_t k, int64_t n, bool dual, int wfmt, int64_t tile, int64_t chunk);
+// the places of the words that a wave asks for, in its order, at most `most` of them; how many
+int chain_wave_words(int64_t k, int64_t n, bool dual, int wfmt, int blk, int wave, int64_t* out, int most);
 // w2 != nullptr: SwiGLU pair, columns of w (gate) and w2 (up) interleaved.  wfmt 0: w is bf16 [k,n];
 // 1: si8 [k,n]; 2: packed int4, ui8 [k/2,n]; 3: f32 [k,n] (no pair)
 void chain_pack_weights(hipStream_t s, const void* w, const void* w2, void* out, int64_t k, int64_t n, int wfmt = kChainW16);
@@ -269,7 +271,7 @@ void chain_unpack_weights(hipStream_t s, const void* packed, void* w, void* w2, 
 // int4 only: derived scale copy sc[tile][group][4] (bf16) from s [k/128, n] (and the partner's s2)
 size_t chain_scale_bytes(int64_t k, int64_t n, bool dual);
 void chain_pack_scales_w4(hipStream_t s, int dtype, const void* sc, const void* sc2, void* out, int64_t k, int64_t n);
-// fills K, N, C, tlo, trem, whole, step_bytes, inv_c, lds_bytes, wfmt (and the dual flag); false when one workgroup would
+// fills K, N, C, tlo, trem, whole, step_bytes, behind, inv_c, lds_bytes, wfmt (and the dual flag); false when one workgroup would
 // own more bias/residual columns than the kernel stages
 bool chain_fill_phase(ChainPhase& p, int64_t k, int64_t n, bool dual, int wfmt = kChainW16);
 // Decode attention inside a chain: supported shapes, scratch for the per-chunk records, and the

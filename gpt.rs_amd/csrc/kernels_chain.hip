@@ -203,15 +203,19 @@ __device__ __forceinline__ void regs_from_lanes(PhaseRegs& R, int pd) {   // pd:
 }
 
 // The tiles of a workgroup: the first `trem` workgroups take one more than `tlo`.
-__device__ __forceinline__ int tile_first(int blk, int tlo, int trem) { return blk * tlo + min(blk, trem); }
-__device__ __forceinline__ int tile_count(int blk, int tlo, int trem) { return tlo + (blk < trem ? 1 : 0); }
+__host__ __device__ __forceinline__ int tile_first(int blk, int tlo, int trem) { return blk * tlo + (blk < trem ? blk : trem); }
+__host__ __device__ __forceinline__ int tile_count(int blk, int tlo, int trem) { return tlo + (blk < trem ? 1 : 0); }
 // The first of a wave's words among the W of its workgroup: words [wave_first(W, w), wave_first(W, w + 1)) are wave w's.
 __host__ __device__ __forceinline__ int wave_first(int W, int w) { return (W * w) >> 3; }   // (W < 2^22)
 static_assert(NWS == 8, "wave_first");
-// Where the packed copy of a phase holds what wave `w` of workgroup `blk` asks for behind the `whole` steps that every wave has: its rest, a run of words.  All
-// workgroups' rests lie one behind the other, behind the whole steps; counted in words from there.  f0: wave_first.
-__host__ __device__ __forceinline__ int wave_rest(int blk, int w, int f0, int C, int tlo, int trem, int whole) {
-    return (blk * tlo + (blk < trem ? blk : trem)) * C + f0 - whole * (SW * (NWS * blk + w));   // the words of the workgroups and waves before, less what they have in whole steps
+// A wave asks for a phase's words in two parts: the `whole` steps of three words that every wave of a workgroup with tiles has, which lie in the order in which the
+// chip asks for them, [step][workgroup][wave][3], and its rest, a run of words; all workgroups' rests lie one behind the other from word `behind` on.
+struct WavePart { int words, at, run, more; };   // words, place of the first, whether they are one run, words of the phase that follow them
+__host__ __device__ __forceinline__ WavePart wave_part(int blk, int w, bool rest, int C, int tlo, int trem, int whole, int behind) {
+    const int W = tile_count(blk, tlo, trem) * C, f0 = wave_first(W, w), words = wave_first(W, w + 1) - f0, at = SW * (NWS * blk + w), in_steps = words > 0 ? SW * whole : 0;
+    const bool run = rest || whole == 0;
+    // of a run: the words of the workgroups and waves before, less what they have in whole steps
+    return WavePart{run ? words - in_steps : in_steps, run ? behind + tile_first(blk, tlo, trem) * C + f0 - whole * at : at, run, run ? 0 : words - in_steps};
 }
 
 // ---------------------------------------------------------------------------- staging (all waves)
@@ -1494,8 +1498,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
 
     // ---- request side: the wave's next step to ask for, in the order the steps are consumed.  Everything but the lane's offset
     // in a word is uniform.
-    int r_phase = -1, r_left = 0;     // words of the phase's whole steps, then of its rest, that are still to be asked for
-    int r_rest = 0, r_jump = 0;       // the rest that follows, and how many words further on it stands
+    int r_part = -1, r_left = 0;      // part of a phase (2 phase: its whole steps, 2 phase + 1: the rest), words of it that are still to be asked for
     unsigned r_step_bytes = 0;
     unsigned long long r_base = 0;    // the next step's first word
     const unsigned lane_off = (unsigned)lane * 16u;
@@ -1504,22 +1507,17 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
     int inflight = 0;                 // steps requested and not yet read
     unsigned pend = 0u;               // bits 2i, 2i + 1: loads that the i-th oldest of them carries
     int loads = 0;                    // loads in flight
-    auto r_seek = [&]() -> bool {     // next linear phase in which this wave has words
+    auto r_seek = [&]() -> bool {     // next part of a linear phase in which this wave has words (an attention phase has no tiles)
         for (;;) {
-            ++r_phase;
-            if (r_phase >= nphases) return false;
-            const GPTRS_CONST ChainPhase* D = table + r_phase;
-            if (uni(D->kind) != kChainLinear) continue;
-            const int tlo = uni(D->tlo), trem = uni(D->trem), C = uni(D->C), whole = uni(D->whole);
-            const int W = tile_count(blk, tlo, trem) * C, f0 = wave_first(W, wave);
-            const int words = wave_first(W, wave + 1) - f0;
-            if (words == 0) continue;
-            const int at = blk * (NWS * SW) + wave * SW, rest = wave_rest(blk, wave, f0, C, tlo, trem, whole);
-            r_left = whole > 0 ? SW * whole : words;
-            r_rest = words - r_left;
-            r_jump = rest - at;
-            r_step_bytes = whole > 0 ? (unsigned)uni(D->step_bytes) : (unsigned)STEP_BYTES;
-            r_base = (unsigned long long)uni_ptr(D->w) + ((unsigned long long)(unsigned)(whole > 0 ? at : rest) << 10);
+            ++r_part;
+            if (r_part >> 1 >= nphases) return false;
+            const GPTRS_CONST ChainPhase* D = table + (r_part >> 1);
+            const WavePart p = wave_part(blk, wave, r_part & 1, uni(D->C), uni(D->tlo), uni(D->trem), uni(D->whole), uni(D->behind));
+            r_left = p.words;
+            if (p.more == 0) r_part |= 1;
+            if (r_left == 0) continue;
+            r_step_bytes = p.run ? (unsigned)STEP_BYTES : (unsigned)uni(D->step_bytes);
+            r_base = (unsigned long long)uni_ptr(D->w) + ((unsigned long long)(unsigned)p.at << 10);
             return true;
         }
     };
@@ -1552,16 +1550,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
         if (++r_slot == RING_D) r_slot = 0;
         r_base += r_step_bytes;
         r_left -= cnt;
-        if (r_left == 0) {
-            if (r_rest > 0) {
-                r_base += (long long)r_jump * (CW * 16);
-                r_step_bytes = (unsigned)STEP_BYTES;
-                r_left = r_rest;
-                r_rest = 0;
-            } else {
-                r_more = r_seek();
-            }
-        }
+        if (r_left == 0) r_more = r_seek();
     };
     for (int i = 0; i < RING_D && r_more; ++i) request();
 
@@ -1805,21 +1794,25 @@ __global__ __launch_bounds__(NT, 1) void chain_kernel(const ChainPhase* __restri
 // Single: column = 4 * tile + c.  Dual (SwiGLU pair): columns interleaved, c = 0, 2 -> gate column 2 * tile + c / 2, c = 1, 3 -> the
 // same column of up, so one tile finishes two outputs.  A word holds 64 k-groups of the tile's 4 columns, lane l (16 bytes) group
 // 64 chunk + l: 2 k of each column in bf16, 1 in f32, 4 int8 codes, 8 int4 codes.  Zero (of codes: the biased zero) outside the matrix.
-// Place of word (tile, chunk) in the copy, in words: [step][workgroup][wave][3] for the steps that every wave of a workgroup with tiles has in full, the
-// order in which the chip asks for them, and behind those [workgroup][wave][rest].  Every word of the matrix once and nothing else.  (With the waves' last steps padded
-// to three words, and room in a step for workgroups without tiles, 3072 x 64 took 6.3 MB for 0.39, and the layers of GPT-2 small 528 MB for 340.)
+// Every word of the matrix has one place (WavePart), and there is nothing else: with the waves' last steps padded to three words, and room in a step for workgroups
+// without tiles, 3072 x 64 took 6.3 MB for 0.39, and the layers of GPT-2 small 528 MB for 340.
 struct ChainOrder {
     int64_t ntiles, C, grid, tlo, trem;
     __host__ __device__ int64_t active() const { return tlo > 0 ? grid : trem; }   // workgroups that have tiles
-    __host__ __device__ int64_t whole() const { return (tlo > 0 ? tlo : 1) * C / NWS / SW; }
+    // Under two steps a wave asks for all of its words at once, whatever their order: they are one run, which saves the second look into the table.
+    __host__ __device__ int64_t whole() const {
+        const int64_t least = (tlo > 0 ? tlo : 1) * C / NWS;   // words of a wave
+        return least < 2 * SW ? 0 : least / SW;
+    }
     __host__ __device__ int64_t word(int64_t tile, int64_t chunk) const {
         const int64_t big = trem * (tlo + 1);
         const int64_t b = tile < big ? tile / (tlo + 1) : trem + (tile - big) / tlo;
         const int64_t t0 = b * tlo + (b < trem ? b : trem), W = (tlo + (b < trem ? 1 : 0)) * C, f = (tile - t0) * C + chunk;
-        const int64_t w = (8 * f + 7) / W, f0 = wave_first((int)W, (int)w), i = f - f0, n = whole();
-        if (i < SW * n) return (((i / SW) * active() + b) * NWS + w) * SW + i % SW;
-        return n * active() * (NWS * SW) + wave_rest((int)b, (int)w, (int)f0, (int)C, (int)tlo, (int)trem, (int)n) + i - SW * n;
+        const int64_t w = (8 * f + 7) / W, i = f - wave_first((int)W, (int)w), n = whole();   // word i of wave w
+        const WavePart p = wave_part((int)b, (int)w, i >= SW * n, (int)C, (int)tlo, (int)trem, (int)n, (int)behind());
+        return p.run ? p.at + i - SW * n : p.at + (i / SW) * active() * (NWS * SW) + i % SW;
     }
+    __host__ __device__ int64_t behind() const { return whole() * active() * (NWS * SW); }
     int64_t words() const { return ntiles * C; }
 };
 
@@ -1952,6 +1945,18 @@ static ChainOrder chain_order(int64_t k, int64_t n, bool dual, int wfmt) {
 }
 
 size_t chain_weight_bytes(int64_t k, int64_t n, bool dual, int wfmt) { return (size_t)(chain_order(k, n, dual, wfmt).words() * CW * 16); }
+int chain_wave_words(int64_t k, int64_t n, bool dual, int wfmt, int blk, int wave, int64_t* out, int most) {
+    const ChainOrder o = chain_order(k, n, dual, wfmt);
+    int got = 0;
+    for (int part = 0; part < 2; ++part) {
+        const WavePart p = wave_part(blk, wave, part & 1, (int)o.C, (int)o.tlo, (int)o.trem, (int)o.whole(), (int)o.behind());
+        if (p.more == 0) part |= 1;
+        int64_t base = p.at;
+        for (int left = p.words; left > 0; left -= SW, base += p.run ? (int64_t)SW : o.active() * NWS * SW)
+            for (int i = 0; i < (left < SW ? left : SW) && got < most; ++i) out[got++] = base + i;
+    }
+    return got;
+}
 int64_t chain_weight_word(int64_t k, int64_t n, bool dual, int wfmt, int64_t tile, int64_t chunk) { return chain_order(k, n, dual, wfmt).word(tile, chunk); }
 
 void chain_pack_weights(hipStream_t s, const void* w, const void* w2, void* out, int64_t k, int64_t n, int wfmt) {
@@ -1999,6 +2004,7 @@ bool chain_fill_phase(ChainPhase& p, int64_t k, int64_t n, bool dual, int wfmt) 
     p.tlo = (int)o.tlo;
     p.trem = (int)o.trem;
     p.whole = (int)o.whole();
+    p.behind = (int)o.behind();
     p.step_bytes = (int)(o.active() * SLOT_BYTES);
     p.inv_c = 1.0f / (float)o.C;
     p.kind = kChainLinear;
