@@ -488,8 +488,8 @@ constexpr int kKTile = 64;       // keys per step
 // Workgroup = 128 queries (16 per wave) x head x sequence; keys from the first query's chunk on.  Keys and values of a step in LDS,
 // the next step's words in registers meanwhile.  Queries come from the projection, rotated and normed on the way in.  The softmax
 // is started from the sink (maximum = sink, weight 1: always finite, also for a step of which a query sees nothing).
-// Times, us, 32 heads of 128 + 128, before and after: 1 x 3000 in chunks of 1024 104 -> 79 (the order of the workgroups 87 -> 79: by position two of one length
-// shared a CU), 4 x 1000 109 -> 93, 1 x 1000 47.6 -> 45.4, 1 x 128 10.0 -> 8.4.
+// Times, us, 32 heads of 128 + 128, before the workgroups' order, scalar masks and queries loaded at once, and now: 1 x 3000 in chunks of 1024 104 -> 67 (the order of
+// the workgroups 87 -> 79: by position two of one length shared a CU), 4 x 1000 108 -> 79, 1 x 1000 47.5 -> 41, 1 x 128 17.9 -> 12.7.
 template <int KS, int VT>
 __global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, const bf16_t* __restrict__ kr, const bf16_t* __restrict__ vr, int per_chunk) {
     extern __shared__ __align__(16) unsigned char chk_smem[];
@@ -535,35 +535,54 @@ __global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, cons
     {
         const float* src = a.proj + row * a.ld + (int64_t)h * D;
         const float* tab = a.table + row * rot;
-        // every load is made, of a clamped place, before the first value is used: with tests around them each pair of cosines was a trip to memory of its own
-        f32x4_m x[KS][2], cs[KS], sn[KS];
+        // All of a query is requested at once, then the cosines and sines of KG steps of 32 values at a time, four of each to a lane and load, of steps that turn any: with a
+        // test and a trip to memory for each pair a workgroup spent about 5 us here, with single values for every step, turned or not, up to 16.  KG: two of eight steps,
+        // whose registers otherwise leave room for one workgroup to a CU instead of two (`if`, not `break`, and no branch around the last pairs, for the same reason).
+        // us, with pairs behind tests, with single values at once and now: 192 + 64 values 1 x 128 16.0, 26.0, 14.0, 4 x 1000 107, 167, 95; 96 + 128 1 x 128 12.0, 17.9, 12.3; 128 + 128 17.9, 17.8, 12.7.
+        constexpr int KG = KS > 4 ? 2 : KS;
+        const int even = rot & ~7;   // whole fours of pairs
+        f32x4_m x[KS][2];
         float ss = 0.f;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-            const int d = min(32 * k + 8 * kg, D - 8);
-            x[k][0] = *reinterpret_cast<const f32x4_u*>(src + d);
-            x[k][1] = *reinterpret_cast<const f32x4_u*>(src + d + 4);
+            x[k][0] = x[k][1] = f32x4_m{0.f, 0.f, 0.f, 0.f};
+            if (32 * k >= D) continue;
+            const float* from = 32 * k + 32 <= D ? src + 32 * k + 8 * kg : src + min(32 * k + 8 * kg, D - 8);
+            x[k][0] = *reinterpret_cast<const f32x4_u*>(from);
+            x[k][1] = *reinterpret_cast<const f32x4_u*>(from + 4);
         }
-        if (rot > 0) {
 #pragma unroll
-            for (int k = 0; k < KS; ++k)
+        for (int k0 = 0; k0 < KS; k0 += KG)
+            if (32 * k0 < even) {
+                f32x4_m cs[KG], sn[KG];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int i = min(16 * k + 4 * kg + e, rot / 2 - 1);
-                    cs[k][e] = tab[i];
-                    sn[k][e] = tab[rot / 2 + i];
+                for (int k = 0; k < KG; ++k) {
+                    const float* from = tab + (32 * (k0 + k) + 8 * kg < even ? 16 * (k0 + k) + 4 * kg : 0);
+                    cs[k] = *reinterpret_cast<const f32x4_u*>(from);
+                    sn[k] = *reinterpret_cast<const f32x4_u*>(from + rot / 2);
                 }
 #pragma unroll
-            for (int k = 0; k < KS; ++k)
+                for (int k = 0; k < KG; ++k) {
+                    const bool turned = 32 * (k0 + k) + 8 * kg < even;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const bool turned = 32 * k + 8 * kg + 2 * e < rot;
+                    for (int e = 0; e < 4; ++e) {
+                        const float u = x[k0 + k][e >> 1][2 * (e & 1)], v = x[k0 + k][e >> 1][2 * (e & 1) + 1];
+                        const float ut = u * cs[k][e] - v * sn[k][e], vt2 = v * cs[k][e] + u * sn[k][e];
+                        x[k0 + k][e >> 1][2 * (e & 1)] = turned ? ut : u;
+                        x[k0 + k][e >> 1][2 * (e & 1) + 1] = turned ? vt2 : v;
+                    }
+                }
+            }
+#pragma unroll
+        for (int k = 0; k < KS; ++k)   // up to three pairs more, of one lane of a query's four
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (32 * k + 8 * kg == even && 2 * e < rot - even) {
+                    const float cs = tab[16 * k + 4 * kg + e], sn = tab[rot / 2 + 16 * k + 4 * kg + e];
                     const float u = x[k][e >> 1][2 * (e & 1)], v = x[k][e >> 1][2 * (e & 1) + 1];
-                    const float ut = u * cs[k][e] - v * sn[k][e], vt2 = v * cs[k][e] + u * sn[k][e];
-                    x[k][e >> 1][2 * (e & 1)] = turned ? ut : u;
-                    x[k][e >> 1][2 * (e & 1) + 1] = turned ? vt2 : v;
+                    x[k][e >> 1][2 * (e & 1)] = u * cs - v * sn;
+                    x[k][e >> 1][2 * (e & 1) + 1] = v * cs + u * sn;
                 }
-        }
 #pragma unroll
         for (int k = 0; k < KS; ++k)
 #pragma unroll

@@ -271,6 +271,12 @@ def test_prompt_and_single_keys(hip, dt, shape, lens, chunk):
             check(g, w, TOL[dt], (shape, lens, chunk, fusion, "cache"))
 
 
+@pytest.mark.parametrize("shape", [(2, 1, 256, 64, 2), (2, 1, 256, 64, 254), (4, 2, 192, 24, 70), (3, 1, 96, 128, 36), (2, 1, 136, 16, 136), (2, 1, 64, 16, 8), (1, 1, 8, 8, 6)])
+def test_prompts_of_heads_turned_in_part(hip, shape):
+    """Turned parts of whole fours of pairs and one to three pairs more, at the first and the last of up to eight steps of 32 values; heads that end inside a step."""
+    test_prompt_and_single_keys(hip, "Bf16", shape, [129, 40], 100)
+
+
 @pytest.mark.parametrize("lens,chunk", [([129], 128), ([700, 256, 100, 513], 256), ([385, 384, 1], 384)])
 def test_prompts_over_chunks_of_whole_tiles(hip, lens, chunk):
     """Tiles of 128 queries are taken chunk by chunk from the chunks' ends on: prompts that end at a chunk's end, behind it and inside the first."""
