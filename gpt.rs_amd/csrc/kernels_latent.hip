@@ -546,30 +546,35 @@ __global__ __launch_bounds__(512) void latent_prefill_kernel(LatentPrefillArgs a
         const int row = r0 + min(qi, T - 1);
         const bf16_t* src = (const bf16_t*)a.x + ((int64_t)row * H + h) * hd;
         const float* tab = a.table + (int64_t)row * rot;
-        // every load is made, of a clamped place, before the first value is used: with tests around them each pair of cosines was a trip to memory of its own
-        f32x4_m cs[KS], sn[KS];
+        // all of a query is requested at once, then the cosines and sines of KG steps of 32 values, of steps that turn any: with tests around them each pair of cosines was a trip to
+        // memory of its own.  Eight steps two at a time: all of them at once left registers for one workgroup to a CU instead of two (192 + 64 and 64 values, 1 x 3000, us: behind tests
+        // 175-184, all at once 207, now 160)
+        constexpr int KG = KS < 8 ? KS : 2;
 #pragma unroll
         for (int k = 0; k < KS; ++k) q[k] = *reinterpret_cast<const u32x4_m*>(src + min(32 * k + 8 * kg, hd - 8));
-        if (rot > 0) {
 #pragma unroll
-            for (int k = 0; k < KS; ++k)
-                if (32 * k + 24 >= dim) {
-                    const int i = min(max(32 * k + 8 * kg - dim, 0), rot - 8) / 2;
+        for (int k0 = 0; k0 < KS; k0 += KG)
+            if (rot > 0 && 32 * (k0 + KG - 1) + 24 >= dim) {
+                f32x4_m cs[KG], sn[KG];
+#pragma unroll
+                for (int k = 0; k < KG; ++k) {
+                    if (32 * (k0 + k) + 24 < dim) continue;
+                    const int i = min(max(32 * (k0 + k) + 8 * kg - dim, 0), rot - 8) / 2;
                     cs[k] = *reinterpret_cast<const f32x4_u*>(tab + i);
                     sn[k] = *reinterpret_cast<const f32x4_u*>(tab + rot / 2 + i);
                 }
 #pragma unroll
-            for (int k = 0; k < KS; ++k)
-                if (32 * k + 24 >= dim) {
-                    const bool turned = 32 * k + 8 * kg >= dim;
+                for (int k = 0; k < KG; ++k) {
+                    if (32 * (k0 + k) + 24 < dim) continue;
+                    const bool turned = 32 * (k0 + k) + 8 * kg >= dim;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float x0 = bf16lo(q[k][e]), x1 = bf16hi(q[k][e]);
+                        const float x0 = bf16lo(q[k0 + k][e]), x1 = bf16hi(q[k0 + k][e]);
                         const uint32_t r = pack_bf16_hw(x0 * cs[k][e] - x1 * sn[k][e], x1 * cs[k][e] + x0 * sn[k][e]);
-                        q[k][e] = turned ? r : q[k][e];
+                        q[k0 + k][e] = turned ? r : q[k0 + k][e];
                     }
                 }
-        }
+            }
 #pragma unroll
         for (int k = 0; k < KS; ++k)
             if (32 * k + 8 * kg >= hd) q[k] = u32x4_m{0u, 0u, 0u, 0u};
