@@ -282,7 +282,8 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentDecodeArgs a, bf
 // Bound by its chain of trips to memory and LDS and by the code it fetches (other launches put it out of the instruction cache), not by bytes: 32 heads, rank 512 + 64, us,
 // with 64 rows to a step and a slice and the rows requested behind the queries' stores, and now: 8 x 71 positions 11.9 -> 8.9, 8 x 246 12.5 -> 9.7,
 // 2 x 906 13.9 -> 11.1, 1 x 2906 20.7 -> 18.1.  Dropped: steps of 64 rows over slices of 32, with a shorter form for the last 32 (10.6, 11.3, 12.5, 19.8), slices of 16
-// (9.1, 10.6, 11.0, 18.2).
+// (9.1, 10.6, 11.0, 18.2).  Steps of 32 rows wait twice as often for memory, so the next step's rows are requested while one is computed: slices of 125 rows and more, with steps of 64,
+// of 32 and now: 8 x 4000 23.0, 23.4, 21.2; 32 x 4000 73.6, 77.2, 69.0; 64 x 2000 96.5, 98.5, 90.0; 1 x 16000 51.5, 56.5, 52.5.
 template <int RT>
 __global__ __launch_bounds__(256) void latent_partial_kernel(LatentDecodeArgs a, const bf16_t* __restrict__ ql, float* __restrict__ part, int nsplit) {
     extern __shared__ __align__(16) unsigned char lat_smem[];
@@ -315,7 +316,8 @@ __global__ __launch_bounds__(256) void latent_partial_kernel(LatentDecodeArgs a,
 #pragma unroll
         for (int u = 0; u < U; ++u) v[u] = from[min(k0 + 8 * u, wv - 1)];
     };
-    auto stage = [&](u32x4_m (&v)[U], bool first, const bf16_t* src, bf16_t* dst, int nrows, int last) {   // first: v holds the first round's words
+    auto stage = [&](u32x4_m (&v)[U], const bf16_t* src, bf16_t* dst, int nrows, int last) {   // v holds the first round's words
+        bool first = true;
         for (int r = tid >> 3; r < nrows; r += 8 * W)
             for (int k0 = tid & 7; k0 < wv; k0 += 8 * U) {
                 if (!first) request(v, src, r, k0, last);
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(256) void latent_partial_kernel(LatentDecodeArgs a,
         const bf16_t* from = ql + ((int64_t)b * H + ht0 * kHeadTile) * w;
         request(qw, from, tid >> 3, tid & 7, H - 1 - ht0 * kHeadTile);
         request(rw, cache + (int64_t)p0 * w, tid >> 3, tid & 7, min(kTileP, p1 - p0) - 1);
-        stage(qw, true, from, q0s, (ht1 - ht0 + 1) * kHeadTile, H - 1 - ht0 * kHeadTile);
+        stage(qw, from, q0s, (ht1 - ht0 + 1) * kHeadTile, H - 1 - ht0 * kHeadTile);
     }
     const bf16_t* qs = q0s + (ht - ht0) * kHeadTile * ws;
     f32x4_m acc[RT];                                                  // rows: latent dimensions, column: head c
@@ -343,8 +345,10 @@ __global__ __launch_bounds__(256) void latent_partial_kernel(LatentDecodeArgs a,
     for (int q0 = p0; q0 < p1; q0 += kTileP) {
         const int np = min(kTileP, p1 - q0);
         __syncthreads();
-        stage(rw, q0 == p0, cache + (int64_t)q0 * w, rows, kTileP, np - 1);
+        stage(rw, cache + (int64_t)q0 * w, rows, kTileP, np - 1);
         __syncthreads();
+        const int q1 = q0 + kTileP;                                   // the next step's first rows are on their way meanwhile
+        if (q1 < p1) request(rw, cache + (int64_t)q1 * w, tid >> 3, tid & 7, min(kTileP, p1 - q1) - 1);
         constexpr int PT = kTileP / 16;
         f32x4_m sc[PT];
 #pragma unroll
