@@ -1408,11 +1408,17 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t roo
     // in tiles that fill a round of their own.  Taken where the fit says 7.5 % or more: what it says less about came out level, since a
     // last round that is partly empty runs at a higher clock.  us, weights from memory, measured against the best single launch: pair of
     // 9216 M = 1000 126 -> 119, 2047 238 -> 218, 3000 340 -> 319; N = 6176 M = 3000 135 -> 123; K = 1536, N = 6144 M = 3064 75 -> 71.
-    // Over 160 shapes that the rule was tried on (M = 64 .. 7600, K = 576 .. 9216, N = 768 .. 14336) it gains 8.8 % in the mean; the losses, up to
-    // 7 %, are all at K of 1024 and less (M = 4758, K = 768, N = 5120 69 -> 74), where the second launch's start counts: those stay whole.
+    // Over 160 shapes that the rule was tried on first (M = 64 .. 7600, K = 576 .. 9216, N = 768 .. 14336) it gains 8.8 % in the mean; losses of up to
+    // 7 % at K of 1024 and less (M = 4758, K = 768, N = 5120 69 -> 74), where the second launch's start counts: those stay whole.  A second launch over
+    // a few rows more is bound by the weights, which it reads again, where they are more than the last cache holds: priced without, pairs of
+    // K = 9216 .. 14336, N = 14336 lost up to 8 % (M = 563, K = 9216, N = 14432 317 -> 337; M = 270, K = 11008, N = 14336 254 -> 275).  With it they are one launch
+    // (317) or are split by columns (M = 352, K = 9216, N = 14432 242, 246, 216; M = 359, K = 14336 378, 376, 332).  Over 180 shapes that take two launches (K up to 14336,
+    // N up to 18432) the mean gain is 5.5 %, the largest loss 3 % (M = 2756, K = 14336, N = 6144 442 -> 456: the fit gives 128 x 192 tiles 10 % too much at long K).
     // Left alone too: N = 14432 M = 3064 (5.6 % by the fit, 265 and 262), K = 3072, N = 4096 M = 3064 (5.4 %, 86 and 85).
     if (best.splits == 1 && least > 40.0 && k > 1024) {
         const double one = least;
+        // a second launch over further rows reads all weights again; what is left of 256 MB and less is still in the last cache
+        const double weights = (double)k * n * (dual ? 2 : 1) * 2, again = weights > 256e6 ? weights / 5.0e6 : 0.0;
         auto cost = [&](int t, int64_t rows, int64_t cols) {
             const TileCost& c = kTileCost[t];
             const int64_t tiles = cdiv(rows, c.bm) * cdiv(cols, dual ? c.bn / 2 : c.bn);
@@ -1432,7 +1438,7 @@ static TilePlan tile_plan(int64_t m, int64_t k, int64_t n, bool dual, size_t roo
                 const double us1 = cost(t, by_columns ? m : first.rows, by_columns ? first.cols : n);
                 for (int r = 0; us1 < least && r < kTiles; ++r) {
                     if (r == kT192x192 || (dual && r == kT256x192)) continue;
-                    const double us = us1 + cost(r, m - rest.row0, n - rest.col0);
+                    const double us = us1 + std::max(cost(r, m - rest.row0, n - rest.col0), by_columns ? 0.0 : again);
                     if (us < least && us < 0.925 * one) { least = us; best = {t, 1, r, first, rest}; }
                 }
             }

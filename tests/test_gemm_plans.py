@@ -48,6 +48,13 @@ def test_two_launches_cover_a_layer_once():
     assert two > 40
 
 
+@pytest.mark.parametrize("m,k,n", [(563, 9216, 14432), (542, 11008, 14336), (352, 9216, 14432), (260, 9216, 14336), (270, 11008, 14336)])
+def test_weights_that_no_cache_holds_are_not_read_again_for_a_few_rows(m, k, n):
+    """Pairs of 0.5 GB of weights: one launch, or two that read half of them each."""
+    r = regions(m, k, n, True)
+    assert r is None or r[0][0] == 0   # (no split between rows)
+
+
 @pytest.mark.parametrize("dual", [False, True])
 def test_int4_tiles_fit_whatever_the_workspace(dual):
     """The scales of a workgroup's share of K lie in LDS: with the splits given up for want of room the share is all of K, and the tile has to be
