@@ -64,7 +64,7 @@ constexpr int NWS = NS / 64;
 constexpr int SW = 3;            // words of a step: what a wave requests and consumes at a time
 constexpr int CW = 64;           // lanes, and 16-byte pieces, of a word
 constexpr int NC = kChainCounters;
-constexpr int EPI_MAX = 640;     // bias/residual values staged per workgroup and phase: N <= 160 * grid columns
+constexpr int EPI_MAX = 640;     // output columns of a workgroup, staged values among them: N <= 640 * grid (tiles that do not divide evenly: up to 4 fewer)
 constexpr int MAXI = 8;          // 8-byte items per thread in the norm staging: K <= 4*MAXI*NT
 constexpr int STEP_BYTES = SW * CW * 16;     // a step of a wave
 constexpr int SLOT_BYTES = NWS * STEP_BYTES; // ... of a workgroup
@@ -567,32 +567,11 @@ __device__ __forceinline__ void unpack8(unsigned long long a, unsigned long long
     o[0] = bf16lo(a0); o[1] = bf16hi(a0); o[2] = bf16lo(a1); o[3] = bf16hi(a1);
     o[4] = bf16lo(b0); o[5] = bf16hi(b0); o[6] = bf16lo(b1); o[7] = bf16hi(b1);
 }
-// 8 consecutive bf16: coherent (written earlier in this launch) / plain (older than the launch)
-__device__ __forceinline__ void cload_bf16x8(const bf16_t* p, float (&o)[8]) { unpack8(cload8(p), cload8(p + 4), o); }
+// 8 consecutive bf16, older than the launch
 __device__ __forceinline__ void load_bf16x8(const bf16_t* p, float (&o)[8]) {
     const uint4 v = gload4(p);
     o[0] = bf16lo(v.x); o[1] = bf16hi(v.x); o[2] = bf16lo(v.y); o[3] = bf16hi(v.y);
     o[4] = bf16lo(v.z); o[5] = bf16hi(v.z); o[6] = bf16lo(v.w); o[7] = bf16hi(v.w);
-}
-// Rotate-half RoPE (ops/functional/rotary.rs:430-536) while loading dims [c0, c0+8) of one head of
-// the packed projection: dims below `half` pair with dim+half, the next `half` dims with dim-half,
-// the rest pass through; the result is rounded to bf16 like a stored post-RoPE row.
-__device__ __forceinline__ void cload_roped(const bf16_t* head, int c0, int half, const bf16_t* cs, const bf16_t* sn, float (&out)[8]) {
-    float own[8];
-    cload_bf16x8(head + c0, own);
-    if (cs == nullptr || c0 >= 2 * half) {
-#pragma unroll
-        for (int v = 0; v < 8; ++v) out[v] = own[v];
-        return;
-    }
-    const bool first = c0 < half;
-    float other[8], c[8], sv[8];
-    cload_bf16x8(head + (first ? c0 + half : c0 - half), other);
-    const int j0 = first ? c0 : c0 - half;
-    load_bf16x8(cs + j0, c);
-    load_bf16x8(sn + j0, sv);
-#pragma unroll
-    for (int v = 0; v < 8; ++v) out[v] = rbf(first ? own[v] * c[v] - other[v] * sv[v] : own[v] * c[v] + other[v] * sv[v]);
 }
 __device__ __forceinline__ long clampl(long v, long lo, long hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
@@ -1475,7 +1454,7 @@ __device__ __forceinline__ int vm_in_flight() {
 // s_waitcnt that waits until at most N vector memory operations of the wave are in flight (and for nothing else); the count is
 // an immediate of the instruction
 template <int N> __device__ __forceinline__ void wait_vm_imm() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }
-__device__ __forceinline__ void wait_vm_count(int n) {   // steps without loads in flight (padding, tiles that do not exist): rare
+__device__ __forceinline__ void wait_vm_count(int n) {   // a step of fewer than three words in flight behind the oldest one, or a full ring
     switch (n) {
 #define GPTRS_VM(k) case k: wait_vm_imm<k>(); break;
         GPTRS_VM(1) GPTRS_VM(2) GPTRS_VM(3) GPTRS_VM(4) GPTRS_VM(5) GPTRS_VM(6) GPTRS_VM(7) GPTRS_VM(8)
@@ -1705,8 +1684,9 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
       if (!wait_go(&sh.go, &sh.abort, c_phase, budget)) break;
       if (FMT == kChainW32) stage_block_f32(R, const_cast<unsigned*>(xs), sh.ssq);
       else stage_block<FMT>(R, const_cast<unsigned*>(xs), sh.ssq);
-      // Every load of the wave is older than the row it has just staged and has landed with it.  The compiler is told so here: left
-      // to itself it waited for all loads in flight at the top of each pass of the loop below.
+      // All loads of the wave have landed from here on.  A wave that has staged a part of the row has waited for them with it, since loads return in order; one
+      // that has not (f32 rows of 768 take three waves) waits here for the words it has under way.  The compiler is told by it too: left to itself it
+      // waited for all loads in flight at the top of each pass of the loop below.
       wait_vm_imm<0>();
       bool from_park = false;
       while (c_left > 0) {

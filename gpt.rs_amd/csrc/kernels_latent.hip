@@ -676,6 +676,7 @@ static int latent_nsplit(int64_t nseq, int64_t capacity, int64_t heads) {
 static size_t latent_partial_lds(int64_t w, int64_t head_tiles = 1) {
     return (size_t)(kTileP + head_tiles * kHeadTile) * (w + 8) * 2;
 }
+// (64 + 16 rows in LDS, rank + rot up to 992: what these kernels needed with steps of 64 rows.  Longer rows would fit now; they stay with the plain kernels, as before.)
 static bool latent_fast(int dtype, int64_t heads, int64_t dim, int64_t rot, int64_t rank, int64_t vdim) {
     return dtype == 2 && heads >= 1 && dim % 8 == 0 && vdim % 8 == 0 && rot % 2 == 0 && rank % 16 == 0 && (rank + rot) % 32 == 0 && rank <= 1024 && dim <= 512 &&
            (64 + kHeadTile) * (rank + rot + 8) * 2 <= 160 * 1024;

@@ -1,6 +1,6 @@
 """GPU parity of the persistent decode chain (one launch for a run of M = 1 bf16 linears and decode
 attentions) against the CPU oracle, at the widths of the Ministral-3B-shaped decoder: several
-words per lane and tile (K 3072..9216), several units per workgroup, RMSNorm prologue, SwiGLU pair,
+words per lane and tile (K 3072..9216), several tiles per workgroup, RMSNorm prologue, SwiGLU pair,
 bias + exact GELU, residual, and chains of dependent phases.
 
 Reference: the oracle run in F32 on the same bf16-representable inputs (the reference's CPU backends
@@ -246,11 +246,10 @@ def test_grid_barrier_gives_up_and_the_backend_goes_on(hip):
 
 @pytest.mark.parametrize("k,n", [(2560, 32768), (1536, 32768), (3072, 32776), (200, 4100)])
 def test_padded_steps_and_missing_tiles_are_stable(hip, k, n):
-    """Shapes whose tile streams end inside a j-step (K = 2560, 1536: the last step's upper waves hold nothing but padding;
-    K = 200: a wave that is partly padding) or whose last unit lacks tiles (N = 32776 -> 8194 tiles = 2731 units + 1 tile;
-    N = 4100 -> 1025 tiles), run many times: a wave asks for weights several steps ahead and tells by the count of its loads
-    in flight which step has landed, which holds only while every load it issues returns in order.  (Loads that re-read
-    cached words in place of padding did not, and whole units came out wrong now and then.)"""
+    """Shapes whose tiles end inside a word (K = 200: 128 and 72 of its values in two words), whose waves end inside a step of three words (K = 2560: 80 words a wave), have
+    one word or none (N = 4100: 1025 tiles of two words) or unequal shares (N = 32776: 96 and 99), run many times: a wave asks for weights several steps ahead
+    and tells by the count of its loads in flight which step has landed, which holds only while every load it issues returns in order.  (Loads that
+    re-read cached words in place of padding did not, and sums came out wrong now and then.)"""
     x, w = rnd(70, (1, k)), rnd(71, (k, n), 2.0 / np.sqrt(k))
     p = prog(lambda fb, a, b: a.matmul(b), [("Bf16", [1, k]), ("Bf16", [k, n])])
     hip.set_option("chain", 0)

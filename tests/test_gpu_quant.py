@@ -128,7 +128,7 @@ def test_decode_linear_tiles_dealt_over_workgroups(hip, scheme, k, n):
 
 @pytest.mark.parametrize("scheme,k,n", [("w8", 3072, 32768), ("w4g128", 3072, 32768), ("w4g128", 2048, 155648)])
 def test_decode_linear_wide(hip, scheme, k, n):
-    """Vocabulary-sized outputs: many units per workgroup, and (last case) more int4 group scales per workgroup
+    """Vocabulary-sized outputs: many tiles per workgroup, and (last case) more int4 group scales per workgroup
     than one round of the cooperative staging loads."""
     x = bf16_round(rnd(14, (1, k)))
     w = np.random.default_rng(15).standard_normal((k, n), dtype=np.float32)
