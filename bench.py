@@ -365,8 +365,8 @@ README_GPT2_TOKENS_PER_S = 74.71   # reference README.md:18-25: GPT-2 small f32,
 
 def chain_floor_record(be, phases: int = 157, reps: int = 20):
     """What a decode chain of `phases` phases costs when there is next to nothing to stream: a persistent launch over
-    dependent bf16 linears alternating [1, 64] x [64, 3072] (every workgroup takes part: staging, a step or two of words, epilogue,
-    barrier) and [1, 3072] x [3072, 64] (six workgroups work, all meet at the barrier), 393 KB of weights per phase.  The
+    dependent bf16 linears alternating [1, 64] x [64, 3072] (every workgroup takes part: staging, a step of words at most, epilogue,
+    barrier) and [1, 3072] x [3072, 64] (sixteen workgroups work, all meet at the barrier), 393 KB of weights per phase.  The
     launch time (HIP events of the library's "profile" option around the launch) over the number of phases is the
     synchronisation cost per phase that a real chain pays on top of its streaming."""
     from gptrs_amd.ptir import FunctionBuilder, Program, f32_to_bf16_bits
@@ -400,7 +400,7 @@ def chain_floor_record(be, phases: int = 157, reps: int = 20):
     us = t_ns / calls / 1e3
     return {"phases": phases, "us_per_launch": round(us, 1), "us_per_phase": round(us / phases, 2),
             "what": "persistent launch over %d dependent bf16 linears with 393 KB of weights each (alternating 64 -> 3072 and 3072 -> 64): "
-                    "grid barrier, staging, a step or two of words, epilogue and store acknowledgement per phase, nothing to stream" % phases}
+                    "grid barrier, staging, a step of words at most, epilogue and store acknowledgement per phase, nothing to stream" % phases}
 
 
 def quant_record(be, cfg, quant: str, prompt, capacity: int, steps: int = 64, warmup: int = 8, prof_steps: int = 16):
