@@ -68,8 +68,9 @@ constexpr int EPI_MAX = 640;     // output columns of a workgroup, staged values
 constexpr int MAXI = 8;          // 8-byte items per thread in the norm staging: K <= 4*MAXI*NT
 constexpr int STEP_BYTES = SW * CW * 16;     // a step of a wave
 constexpr int SLOT_BYTES = NWS * STEP_BYTES; // ... of a workgroup
-constexpr int PARK_W4 = 1, PARK_W8 = 2;   // ... in the int4 and int8 kernels, whose step arithmetic and staging hold more registers (measured: one step more spills)
-constexpr int PARK = 3;             // steps a compute wave can hold in registers while it waits for a phase to open
+// Steps a compute wave can hold in registers while it waits for a phase to open: bf16, and fewer in the int4 and int8 kernels, whose step arithmetic and staging hold more registers (one step
+// more spills), and in f32, whose short phases lose more to a longer text than three parked steps give (GPT-2 call of 64 tokens, us: one 26690, two 27560, three 27720).
+constexpr int PARK = 3, PARK_W8 = 2, PARK_W4 = 1, PARK_W32 = 1;
 constexpr int RING_MIN = 4, RING_MAX = 5;    // steps a wave's ring holds (its requests run that far ahead of its reads): 5 where the staged activations leave room
 // Steps a wave has in flight while it consumes a phase.  What is queued in a CU's memory pipeline stands in front of everything that
 // comes later, the control wave's stores, its arrival and its polls of the barrier among it, and more than 48 KiB of a CU under way
@@ -1529,7 +1530,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
         if (++r_slot == RING_D) r_slot = 0;
         r_base += r_step_bytes;
         r_left -= cnt;
-        if (r_left == 0) r_more = r_seek();
+        if (__builtin_expect(r_left == 0, 0)) r_more = r_seek();
     };
     for (int i = 0; i < RING_D && r_more; ++i) request();
 
@@ -1650,7 +1651,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
       // the slots they leave are asked to fetch further ahead.  A step is only asked for when nothing of the wave is in flight:
       // the pipeline that the control wave polls the barrier through stays short.  Parked steps are the phase's first ones and
       // are read back first; the registers are free again before the next phase is looked for.
-      constexpr int PARKN = FMT == kChainW4 ? PARK_W4 : (FMT == kChainW8 ? PARK_W8 : PARK);   // (the int4 kernel stages its group scales through registers as well)
+      constexpr int PARKN = FMT == kChainW4 ? PARK_W4 : FMT == kChainW8 ? PARK_W8 : FMT == kChainW32 ? PARK_W32 : PARK;   // (the int4 kernel stages its group scales through registers as well)
       u32x4 park[PARKN][SW];
       int n_parked = 0, park_rd = 0;
       {
@@ -1699,7 +1700,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
                 default: _Pragma("unroll") for (int p = 0; p < SW; ++p) cur[p] = park[PARKN - 1][p]; break;
 #undef GPTRS_PARK
             }
-            static_assert(PARK >= 1 && PARK <= 3 && PARK_W4 >= 1 && PARK_W4 <= 3 && PARK_W8 >= 1 && PARK_W8 <= 3, "cases above");
+            static_assert(PARKN >= 1 && PARKN <= 3, "cases above");
             ++park_rd;
         } else {
             const GPTRS_LDS u32x4* wp = mine + slot * (SW * CW);
