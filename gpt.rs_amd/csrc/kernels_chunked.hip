@@ -488,7 +488,7 @@ constexpr int kKTile = 64;       // keys per step
 // Workgroup = 128 queries (16 per wave) x head x sequence; keys from the first query's chunk on.  Keys and values of a step in LDS,
 // the next step's words in registers meanwhile.  Queries come from the projection, rotated and normed on the way in.  The softmax
 // is started from the sink (maximum = sink, weight 1: always finite, also for a step of which a query sees nothing).
-// Times, us, 32 heads of 128 + 128, before the workgroups' order, scalar masks and queries loaded at once, and now: 1 x 3000 in chunks of 1024 104 -> 67 (the order of
+// Times, us, 32 heads of 128 + 128, before the workgroups' order, scalar masks and queries loaded at once, and now: 1 x 3000 in chunks of 1024 104 -> 67 (71 inside a call; the order of
 // the workgroups 87 -> 79: by position two of one length shared a CU), 4 x 1000 108 -> 79, 1 x 1000 47.5 -> 41, 1 x 128 17.9 -> 12.7.
 template <int KS, int VT>
 __global__ __launch_bounds__(512) void chunk_prefill_kernel(ChunkSeqArgs a, const bf16_t* __restrict__ kr, const bf16_t* __restrict__ vr, int per_chunk) {
