@@ -31,7 +31,7 @@
 //     the moment its barrier is seen.
 //
 // Decode attention (T = 1 over the KV cache) runs inside the same launch as two more phase kinds,
-// executed by all 9 waves of a workgroup together: "partial" (one workgroup per kv head and
+// executed by the 8 compute waves of a workgroup together: "partial" (one workgroup per kv head and
 // position chunk: append this step's K/V row, online softmax over the chunk for the query heads
 // of the group) and "combine" (one workgroup per query head merges the chunk records).
 //
@@ -561,25 +561,7 @@ __device__ __forceinline__ void stage_block_f32(const PhaseRegs& P, unsigned* xs
 }
 
 // ---------------------------------------------------------------------------- decode attention
-constexpr int NW = NT / 64;
-
-__device__ __forceinline__ void unpack8(unsigned long long a, unsigned long long b, float (&o)[8]) {
-    const unsigned a0 = (unsigned)a, a1 = (unsigned)(a >> 32), b0 = (unsigned)b, b1 = (unsigned)(b >> 32);
-    o[0] = bf16lo(a0); o[1] = bf16hi(a0); o[2] = bf16lo(a1); o[3] = bf16hi(a1);
-    o[4] = bf16lo(b0); o[5] = bf16hi(b0); o[6] = bf16lo(b1); o[7] = bf16hi(b1);
-}
-// 8 consecutive bf16, older than the launch
-__device__ __forceinline__ void load_bf16x8(const bf16_t* p, float (&o)[8]) {
-    const uint4 v = gload4(p);
-    o[0] = bf16lo(v.x); o[1] = bf16hi(v.x); o[2] = bf16lo(v.y); o[3] = bf16hi(v.y);
-    o[4] = bf16lo(v.z); o[5] = bf16hi(v.z); o[6] = bf16lo(v.w); o[7] = bf16hi(v.w);
-}
-__device__ __forceinline__ long clampl(long v, long lo, long hi) { return v < lo ? lo : (v > hi ? hi : v); }
-
-__device__ __forceinline__ void unpack_u4(const uint4& v, float (&o)[8]) {
-    o[0] = bf16lo(v.x); o[1] = bf16hi(v.x); o[2] = bf16lo(v.y); o[3] = bf16hi(v.y);
-    o[4] = bf16lo(v.z); o[5] = bf16hi(v.z); o[6] = bf16lo(v.w); o[7] = bf16hi(v.w);
-}
+__device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 // Waits inside the kernel are bounded by wall-clock time (wall_clock64 ticks at 100 MHz): the control wave's wait for the
 // grid barrier by the launch's budget, the waits on it inside the workgroup by a multiple of that, so that the control
 // wave is the one to give up and say why.
@@ -607,567 +589,360 @@ __device__ __forceinline__ bool wait_go(IP go, IP abort, int phase, unsigned lon
 
 // exp through v_exp_f32 (2^x): softmax weights only, about one ulp, exp(-inf) = 0
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896f); }
-// sum over the lpr (8, 16 or 32) consecutive lanes of a lane group, result in each of them
-__device__ __forceinline__ float group_sum(float v, int lpr) {
-    int x = __float_as_int(v);
-#define GPTRS_DPP_ADD(ctrl) x = __float_as_int(__int_as_float(x) + __int_as_float(__builtin_amdgcn_update_dpp(0, x, (ctrl), 0xf, 0xf, false)))
-    GPTRS_DPP_ADD(0xB1);    // quad_perm [1,0,3,2]
-    GPTRS_DPP_ADD(0x4E);    // quad_perm [2,3,0,1]
-    GPTRS_DPP_ADD(0x141);   // row_half_mirror: 8 lanes
-    if (lpr >= 16) GPTRS_DPP_ADD(0x140);  // row_mirror: 16 lanes
-#undef GPTRS_DPP_ADD
-    float r = __int_as_float(x);
+template <int CTRL> __device__ __forceinline__ float dpp(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false)); }
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140, DPP_ROR8 = 0x128;
+// sums over the lpr (8, 16 or 32) consecutive lanes of a lane group, in each of them; N values at a time, so that one value's steps stand between another's
+template <int N> __device__ __forceinline__ void group_sums(float (&v)[N], int lpr) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] += dpp<DPP_XOR1>(v[j]);
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] += dpp<DPP_XOR2>(v[j]);
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] += dpp<DPP_HALF_MIRROR>(v[j]);
+    if (lpr >= 16) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) v[j] += dpp<DPP_MIRROR>(v[j]);
+    }
     if (lpr == 32) {
-        const u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(r), __float_as_uint(r), false, false);
-        r = __uint_as_float(sw.x) + __uint_as_float(sw.y);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[j]), __float_as_uint(v[j]), false, false);
+            v[j] = __uint_as_float(sw.x) + __uint_as_float(sw.y);
+        }
     }
-    return r;
 }
-// the values of v held by this lane and by its partner lane ^ off (off = 8, 16 or 32), in an order
-// that is the same for both partners of a pair up to a swap: for symmetric merges only
-__device__ __forceinline__ void lane_pair(float v, int off, float& a, float& b) {
-    if (off == 8) {
-        a = v;
-        b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));  // row_ror:8
-    } else if (off == 16) {
-        const u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        a = __uint_as_float(sw.x); b = __uint_as_float(sw.y);
-    } else {
-        const u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        a = __uint_as_float(sw.x); b = __uint_as_float(sw.y);
-    }
+// Two values of every lane, lane ^ 32 (16) exchanged: the lanes below keep a, those above b, each added up over the pair.
+__device__ __forceinline__ float halves32(float a, float b) {
+    const u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(sw.x) + __uint_as_float(sw.y);
+}
+__device__ __forceinline__ float halves16(float a, float b) {
+    const u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(sw.x) + __uint_as_float(sw.y);
+}
+__device__ __forceinline__ float pair_max32(float a) {
+    const u32x2 sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+    return fmaxf(__uint_as_float(sw.x), __uint_as_float(sw.y));
+}
+__device__ __forceinline__ float pair_max16(float a) {
+    const u32x2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+    return fmaxf(__uint_as_float(sw.x), __uint_as_float(sw.y));
 }
 
-// unit = kv head * nch + chunk.  Each of the 8 streaming waves serves ONE query head of the kv
-// head's group (wave w: head w % G, position subset w / G of 8 / G), so a lane carries a single
-// online-softmax state; a cache row (head_dim bf16) is read by head_dim/8 lanes, 16 bytes each, and
-// the waves of different heads re-read the same rows out of the caches.  Cache rows older than
-// this launch are requested BEFORE the grid barrier is awaited (they do not depend on the
-// previous phase); only the query row and this step's K/V row are read after it.
+// What a maximum of nothing but hidden scores (-inf) is subtracted as: exp(-inf - 0) = 0, where exp(-inf + inf) is none.
+__device__ __forceinline__ float finite_max(float m) { return m == -INFINITY ? 0.f : m; }
+
+// Merge of the records (max m, sum l, N weighted values) of the N_REC waves w = first, first + step, ... of a head, left in LDS.
+template <int N_REC>
+__device__ __forceinline__ void merge_waves(const GPTRS_LDS float* sm, const GPTRS_LDS float* sl, const GPTRS_LDS float* so, int first, int step, int dh, int d,
+                                            float& m, float& l, float& o) {
+    float mm[N_REC], ll[N_REC], oo[N_REC];
+#pragma unroll
+    for (int u = 0; u < N_REC; ++u) { const int w = first + u * step; mm[u] = sm[w]; ll[u] = sl[w]; oo[u] = so[w * dh + d]; }
+    m = mm[0];
+#pragma unroll
+    for (int u = 1; u < N_REC; ++u) m = fmaxf(m, mm[u]);
+    const float ref = finite_max(m);
+    l = 0.f; o = 0.f;
+#pragma unroll
+    for (int u = 0; u < N_REC; ++u) { const float c = fast_exp(mm[u] - ref); l += ll[u] * c; o += oo[u] * c; }
+}
+
+// The two phases are run by the 8 compute waves.  Nothing in them is long: a phase is a chain of latencies (the query row out of
+// other workgroups' hands, scores, softmax, sums over lanes and waves, stores and their acknowledgement), so what counts is how
+// many instructions stand behind one another between the barrier and the arrival.  With one online-softmax step for each row, a
+// branch on the head's size in every exchange between lanes (1.6 us of two exchanges), 64-bit divisions and the control wave among the
+// readers the two phases took, us: bf16 behind 1008 positions of 32 / 8 heads of 128 7.3 + 5.7, in the int8 kernel 7.4 + 4.8, f32 behind 80
+// positions of 12 heads of 64 (one phase) 6.2.  With all rows of a lane in one step, one branch for each round of exchanges, and exchanges
+// that leave each half of the lanes with half of the values 4.9 + 5.0, 4.6 + 3.9 and 3.3.
+//
+// unit = kv head * nch + chunk.  Each wave serves ONE query head of the kv head's group (wave w: head w % G, position subset
+// w / G of 8 / G), so a lane carries a single softmax state; a cache row is read by head_dim / 8 lanes, 8 values each, and
+// the waves of different heads re-read the same rows out of the caches.  Cache rows older than this launch, and the
+// RoPE rows, are requested BEFORE the grid barrier is awaited (they do not depend on the previous phase); only the query
+// row and this step's K/V row are read after it.
+template <bool F32>
 __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int unit, int phase,
                              unsigned long long budget) {
-    constexpr int PP = 5;   // positions per lane group requested ahead of the barrier (32 chunks x 8 lane groups x 5 = 1280 positions)
-    const int t = local_tid(), lane = t & 63, wave = uni(t >> 6);
-    const bool control = wave == NWS;
-    const int dh = P.head_dim, n_q = P.n_q, n_kv = P.n_kv, nch = P.nch, half = P.rot_half;
-    const int G = n_q / n_kv, nparts = NWS / G;
-    const long cap = P.capacity;
-    const int lpr = dh >> 3, rpw = 64 / lpr, sub = lane / lpr, li = lane % lpr;
-    const int g = wave % G, part = wave / G;
-    const int stride = nparts * rpw, sid = part * rpw + sub;   // position slots of this head's waves
-    const int kvh = unit / nch, c = unit - kvh * nch;
-    const bf16_t* qkv = (const bf16_t*)P.x;
-    bf16_t* kc = (bf16_t*)P.k_cache;
-    bf16_t* vc = (bf16_t*)P.v_cache;
-    const bf16_t* cs = (const bf16_t*)P.cos;
-    const bf16_t* sn = (const bf16_t*)P.sin;
-    const long qpos = clampl(uni(gload(P.query_start)), 0, cap - 1);       // DynamicSlice clamp (cpu.rs:804-820)
-    const long upd = clampl(uni(gload(P.update_starts + 1)), 0, cap - 1);  // DynamicUpdateSlice clamp
-    const float scale = P.scale;
-    const long L = qpos + 1, CL = (L + nch - 1) / nch;
-    const long p0 = c * CL, p1 = min(L, p0 + CL);
-    const int owner = (int)min(upd / CL, (long)nch - 1);
-    const bf16_t* knew = qkv + (long)n_q * dh + (long)kvh * dh;
-    const bf16_t* vnew = qkv + (long)(n_q + n_kv) * dh + (long)kvh * dh;
-    const int c0 = li * 8;
-    uint4 kraw[PP], vraw[PP];
-#pragma unroll
-    for (int j = 0; j < PP; ++j) {
-        const long p = p0 + sid + (long)j * stride;
-        if (!control && p < p1 && p != upd) {
-            const long row = ((long)kvh * cap + p) * dh + c0;
-            kraw[j] = gload4(kc + row);
-            vraw[j] = gload4(vc + row);
-        } else {
-            kraw[j] = make_uint4(0, 0, 0, 0);
-            vraw[j] = make_uint4(0, 0, 0, 0);
-        }
-    }
-    if (!control && !wait_go(go, abort, phase, budget)) return false;
-
-    float m = -INFINITY, l = 0.f, o[8];
-#pragma unroll
-    for (int v = 0; v < 8; ++v) o[v] = 0.f;
-    if (!control) {
-        // the wave's query head (RoPE applied on the fly) and, in the first lane group of each head's
-        // first wave of the workgroup that owns position `upd`, this step's K/V row: all requested
-        // before any is consumed
-        const bool rot = cs != nullptr && c0 < 2 * half;
-        const bool first = c0 < half;
-        const int j0 = first ? c0 : c0 - half, co = first ? c0 + half : c0 - half;
-        float cosv[8], sinv[8];
-        if (rot) { load_bf16x8(cs + j0, cosv); load_bf16x8(sn + j0, sinv); }
-        const bf16_t* head = qkv + (long)(kvh * G + g) * dh;
-        unsigned long long qa[2], qb[2] = {0ull, 0ull};
-        qa[0] = cload8(head + c0); qa[1] = cload8(head + c0 + 4);
-        if (rot) { qb[0] = cload8(head + co); qb[1] = cload8(head + co + 4); }
-        const bool fresh = c == owner && sid == 0;           // this lane group handles the new row
-        unsigned long long ka[2] = {0ull, 0ull}, kb[2] = {0ull, 0ull}, va[2] = {0ull, 0ull};
-        if (fresh) {
-            ka[0] = cload8(knew + c0); ka[1] = cload8(knew + c0 + 4);
-            if (rot) { kb[0] = cload8(knew + co); kb[1] = cload8(knew + co + 4); }
-            va[0] = cload8(vnew + c0); va[1] = cload8(vnew + c0 + 4);
-        }
-        auto rope = [&](const unsigned long long (&own2)[2], const unsigned long long (&oth2)[2], float (&out)[8]) {
-            float own[8], other[8];
-            unpack8(own2[0], own2[1], own);
-            if (!rot) {
-#pragma unroll
-                for (int v = 0; v < 8; ++v) out[v] = own[v];
-                return;
-            }
-            unpack8(oth2[0], oth2[1], other);
-#pragma unroll
-            for (int v = 0; v < 8; ++v)
-                out[v] = rbf(first ? own[v] * cosv[v] - other[v] * sinv[v] : own[v] * cosv[v] + other[v] * sinv[v]);
-        };
-        float qf[8];
-        rope(qa, qb, qf);
-
-        auto visit = [&](const float (&kf)[8], const float (&vf)[8]) {
-            float sc = 0.f;
-#pragma unroll
-            for (int v = 0; v < 8; ++v) sc += qf[v] * kf[v];
-            sc = group_sum(sc, lpr) * scale;
-            const float mn = fmaxf(m, sc);
-            const float corr = fast_exp(m - mn);
-            const float pe = fast_exp(sc - mn);
-            l = l * corr + pe;
-#pragma unroll
-            for (int v = 0; v < 8; ++v) o[v] = o[v] * corr + pe * vf[v];
-            m = mn;
-        };
-#pragma unroll
-        for (int j = 0; j < PP; ++j) {
-            const long p = p0 + sid + (long)j * stride;
-            if (p < p1 && p != upd) {
-                float kf[8], vf[8];
-                unpack_u4(kraw[j], kf);
-                unpack_u4(vraw[j], vf);
-                visit(kf, vf);
-            }
-        }
-        for (long p = p0 + sid + (long)PP * stride; p < p1; p += stride) {
-            if (p == upd) continue;
-            float kf[8], vf[8];
-            const long row = ((long)kvh * cap + p) * dh + c0;
-            load_bf16x8(kc + row, kf);
-            load_bf16x8(vc + row, vf);
-            visit(kf, vf);
-        }
-        if (fresh) {   // this step's row: attended to when in range; appended once (by head 0's wave)
-            float kf[8], vf[8];
-            rope(ka, kb, kf);
-            unpack8(va[0], va[1], vf);
-            if (g == 0) {
-                const long row = ((long)kvh * cap + upd) * dh + c0;
-                gstore4(kc + row, make_uint4(pack_bf16x2(kf[0], kf[1]), pack_bf16x2(kf[2], kf[3]), pack_bf16x2(kf[4], kf[5]), pack_bf16x2(kf[6], kf[7])));
-                gstore4(vc + row, make_uint4((unsigned)va[0], (unsigned)(va[0] >> 32), (unsigned)va[1], (unsigned)(va[1] >> 32)));
-            }
-            if (upd >= p0 && upd < p1) visit(kf, vf);
-        }
-        // merge the lane groups of this wave
-        for (int off = lpr; off < 64; off <<= 1) {
-            float ma, mb, la, lb;
-            lane_pair(m, off, ma, mb);
-            lane_pair(l, off, la, lb);
-            const float mn = fmaxf(ma, mb);
-            const float ca = mn == -INFINITY ? 0.f : fast_exp(ma - mn);
-            const float cb = mn == -INFINITY ? 0.f : fast_exp(mb - mn);
-            l = la * ca + lb * cb;
-#pragma unroll
-            for (int v = 0; v < 8; ++v) {
-                float oa, ob;
-                lane_pair(o[v], off, oa, ob);
-                o[v] = oa * ca + ob * cb;
-            }
-            m = mn;
-        }
-    }
-    // merge the waves of each head through LDS and leave one record per query head
-    GPTRS_LDS float* sm = lds;
-    GPTRS_LDS float* sl = lds + NWS;
-    GPTRS_LDS float* so = lds + 2 * NWS;
-    if (!control && sub == 0) {
-        if (li == 0) { sm[wave] = m; sl[wave] = l; }
-#pragma unroll
-        for (int v = 0; v < 8; ++v) so[wave * dh + c0 + v] = o[v];
-    }
-    wg_barrier();
-    float* partp = P.part;
-    const bool final = P.flags & kChainAttnFinal;
-    for (int idx = t; idx < G * dh; idx += NT) {
-        const int gg = idx / dh, d = idx - gg * dh;
-        float mn = -INFINITY;
-        for (int w = gg; w < NWS; w += G) mn = fmaxf(mn, sm[w]);
-        float Ls = 0.f, O = 0.f;
-        if (mn != -INFINITY) {
-            for (int w = gg; w < NWS; w += G) {
-                const float cw = fast_exp(sm[w] - mn);
-                Ls += sl[w] * cw;
-                O += so[w * dh + d] * cw;
-            }
-        }
-        if (final) {
-            // one chunk per kv head: its record is the whole softmax, and the context row is written here (what the merge of
-            // a single record gives: O / L)
-            __hip_atomic_store(as_global((unsigned short*)P.y + (long)(kvh * G + gg) * dh + d), (unsigned short)pack_bf16x2(O / Ls, 0.f),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            continue;
-        }
-        float* rec = partp + ((long)(kvh * G + gg) * nch + c) * (dh + 2);
-        if (d == 0) { cstore4(rec, __float_as_uint(mn)); cstore4(rec + 1, __float_as_uint(Ls)); }
-        cstore4(rec + 2 + d, __float_as_uint(O));
-    }
-    // every lane's stores (record words, the appended cache row) have left the CU before the control wave, which passes
-    // this barrier last of all it executes here, reports the workgroup's arrival
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    wg_barrier();
-    return true;
-}
-
-// unit = query head: softmax-merge of its nch chunk records into the context row.  Thread
-// (sg, d2) reads the records of the chunks s = sg, sg + NW, ... for the dims (2 d2, 2 d2 + 1) in
-// one round of loads and merges them locally; the NW subsets meet in LDS.
-__device__ bool attn_combine(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq, int phase,
-                             unsigned long long budget) {
-    constexpr int MAXC = 8;   // chunks per thread: nch <= MAXC * NW
-    const int t = local_tid(), wave = uni(t >> 6);
-    const int dh = P.head_dim, nch = P.nch;
-    if (wave != NWS && !wait_go(go, abort, phase, budget)) return false;
-    const float* base = P.part + (long)hq * nch * (dh + 2);
-    bf16_t* ctx = (bf16_t*)P.y;
-    const int h2 = dh / 2;
-    for (int d0 = 0; d0 < h2; d0 += 64) {
-        const int d2 = d0 + (t & 63);
-        const bool act = d2 < h2;
-        unsigned long long ml[MAXC], ov[MAXC];
-#pragma unroll
-        for (int u = 0; u < MAXC; ++u) {
-            const int s = wave + u * NW;
-            const bool ok = act && s < nch;
-            ml[u] = ok ? cload8(base + (long)s * (dh + 2)) : 0ull;
-            ov[u] = ok ? cload8(base + (long)s * (dh + 2) + 2 + 2 * d2) : 0ull;
-        }
-        float mn = -INFINITY;
-#pragma unroll
-        for (int u = 0; u < MAXC; ++u)
-            if (wave + u * NW < nch) mn = fmaxf(mn, __uint_as_float((unsigned)ml[u]));
-        float Ls = 0.f, o0 = 0.f, o1 = 0.f;
-#pragma unroll
-        for (int u = 0; u < MAXC; ++u) {
-            if (wave + u * NW < nch) {
-                const float ms = __uint_as_float((unsigned)ml[u]);
-                const float cw = ms == -INFINITY ? 0.f : fast_exp(ms - mn);
-                Ls += __uint_as_float((unsigned)(ml[u] >> 32)) * cw;
-                o0 += __uint_as_float((unsigned)ov[u]) * cw;
-                o1 += __uint_as_float((unsigned)(ov[u] >> 32)) * cw;
-            }
-        }
-        GPTRS_LDS f32x4* rec = (GPTRS_LDS f32x4*)lds;
-        { f32x4 r4; r4.x = mn; r4.y = Ls; r4.z = o0; r4.w = o1; rec[wave * 64 + (t & 63)] = r4; }
-        wg_barrier();
-        if (wave == 0 && act) {
-            float M = -INFINITY;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) M = fmaxf(M, rec[w * 64 + t].x);
-            float Lt = 0.f, a0 = 0.f, a1 = 0.f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const f32x4 r = rec[w * 64 + t];
-                const float cw = r.x == -INFINITY ? 0.f : fast_exp(r.x - M);
-                Lt += r.y * cw; a0 += r.z * cw; a1 += r.w * cw;
-            }
-            cstore4(ctx + (long)hq * dh + 2 * d2, pack_bf16x2(a0 / Lt, a1 / Lt));
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the context words are out before the arrival is reported
-        wg_barrier();
-    }
-    return true;
-}
-
-// The two attention phases once more with the element type as a parameter, instantiated for f32 rows and caches only (a
-// lane's 8 values are then two 16-byte words; no RoPE): written this way the bf16 phases above lost a microsecond each
-// to the compiler, so they keep their own text.
-template <bool F32>
-__device__ bool attn_partial_t(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int unit, int phase,
-                             unsigned long long budget) {
     typedef typename std::conditional<F32, float, bf16_t>::type E;
-    constexpr int PP = F32 ? 2 : 4;   // positions per lane group requested ahead of the barrier
+    constexpr int PP = F32 ? 2 : 5;   // rows of a lane in one step; the first step's are requested ahead of the barrier (32 chunks x 8 lane groups x 5 = 1280 positions)
     constexpr int RW = F32 ? 2 : 1;   // 16-byte words of a lane's 8 values
     const int t = local_tid(), lane = t & 63, wave = uni(t >> 6);
-    const bool control = wave == NWS;
     const int dh = P.head_dim, n_q = P.n_q, n_kv = P.n_kv, nch = P.nch, half = P.rot_half;
-    const int G = n_q / n_kv, nparts = NWS / G;
-    const long cap = P.capacity;
-    const int lpr = dh >> 3, rpw = 64 / lpr, sub = lane / lpr, li = lane % lpr;
-    const int g = wave % G, part = wave / G;
-    const int stride = nparts * rpw, sid = part * rpw + sub;   // position slots of this head's waves
+    const int G = n_q / n_kv, nparts = NWS / G, cap = P.capacity;   // G = 1, 2, 4 or 8
+    const int lpr = dh >> 3, lsh = lpr == 8 ? 3 : lpr == 16 ? 4 : 5, sub = lane >> lsh, li = lane & (lpr - 1);
+    const int g = wave & (G - 1), part = wave / G;
+    const int stride = nparts * (64 >> lsh), sid = part * (64 >> lsh) + sub;   // position slots of this head's waves
     const int kvh = unit / nch, c = unit - kvh * nch;
     const E* qkv = (const E*)P.x;
-    E* kc = (E*)P.k_cache;
-    E* vc = (E*)P.v_cache;
-    const bf16_t* cs = F32 ? nullptr : (const bf16_t*)P.cos;
-    const bf16_t* sn = F32 ? nullptr : (const bf16_t*)P.sin;
-    const long qpos = clampl(uni(gload(P.query_start)), 0, cap - 1);       // DynamicSlice clamp (cpu.rs:804-820)
-    const long upd = clampl(uni(gload(P.update_starts + 1)), 0, cap - 1);  // DynamicUpdateSlice clamp
+    E* kc = (E*)P.k_cache + (long)kvh * cap * dh;
+    E* vc = (E*)P.v_cache + (long)kvh * cap * dh;
+    const bool rotate = !F32 && P.cos != nullptr;
+    const int qpos = clampi(uni(gload(P.query_start)), 0, cap - 1);       // DynamicSlice clamp (cpu.rs:804-820)
+    const int upd = clampi(uni(gload(P.update_starts + 1)), 0, cap - 1);  // DynamicUpdateSlice clamp
     const float scale = P.scale;
-    const long L = qpos + 1, CL = (L + nch - 1) / nch;
-    const long p0 = c * CL, p1 = min(L, p0 + CL);
-    const int owner = (int)min(upd / CL, (long)nch - 1);
-    const E* knew = qkv + (long)n_q * dh + (long)kvh * dh;
-    const E* vnew = qkv + (long)(n_q + n_kv) * dh + (long)kvh * dh;
+    const int L = qpos + 1, CL = (L + nch - 1) / nch;
+    const int p0 = c * CL, p1 = min(L, p0 + CL);
+    const bool owner = c == min(upd / CL, nch - 1);
     const int c0 = li * 8;
-    uint4 kraw[PP][RW], vraw[PP][RW];
-#pragma unroll
-    for (int j = 0; j < PP; ++j) {
-        const long p = p0 + sid + (long)j * stride;
-        const bool take = !control && p < p1 && p != upd;
-        const long row = ((long)kvh * cap + p) * dh + c0;
-#pragma unroll
-        for (int r = 0; r < RW; ++r) {
-            kraw[j][r] = take ? gload4(kc + row + 4 * r) : make_uint4(0, 0, 0, 0);
-            vraw[j][r] = take ? gload4(vc + row + 4 * r) : make_uint4(0, 0, 0, 0);
-        }
-    }
-    // a lane's 8 values of a row: unpacked from bf16 or taken as they are
-    auto row_values = [&](const uint4 (&raw)[RW], float (&f)[8]) {
-        if (F32) {
-            f[0] = __uint_as_float(raw[0].x); f[1] = __uint_as_float(raw[0].y); f[2] = __uint_as_float(raw[0].z); f[3] = __uint_as_float(raw[0].w);
-            f[4] = __uint_as_float(raw[RW - 1].x); f[5] = __uint_as_float(raw[RW - 1].y); f[6] = __uint_as_float(raw[RW - 1].z); f[7] = __uint_as_float(raw[RW - 1].w);
-        } else {
-            unpack_u4(raw[0], f);
-        }
-    };
-    auto load_row = [&](const E* p, float (&f)[8]) {   // plain loads (cache rows older than this launch)
-        uint4 raw[RW];
-#pragma unroll
-        for (int r = 0; r < RW; ++r) raw[r] = gload4(p + 4 * r);
-        row_values(raw, f);
-    };
-    auto cload_row = [&](const E* p, unsigned long long (&w)[2 * RW]) {   // agent-scope loads (rows written by the phase before)
-#pragma unroll
-        for (int r = 0; r < 2 * RW; ++r) w[r] = cload8(p + (F32 ? 2 : 4) * r);
-    };
-    auto words_values = [&](const unsigned long long (&w)[2 * RW], float (&f)[8]) {
-        if (F32) {
-#pragma unroll
-            for (int r = 0; r < 2 * RW; ++r) { f[(2 * r) & 7] = __uint_as_float((unsigned)w[r]); f[(2 * r + 1) & 7] = __uint_as_float((unsigned)(w[r] >> 32)); }
-        } else {
-            unpack8(w[0], w[1], f);
-        }
-    };
-    if (!control && !wait_go(go, abort, phase, budget)) return false;
-
-    float m = -INFINITY, l = 0.f, o[8];
-#pragma unroll
-    for (int v = 0; v < 8; ++v) o[v] = 0.f;
-    if (!control) {
-        // the wave's query head (RoPE applied on the fly) and, in the first lane group of each head's
-        // first wave of the workgroup that owns position `upd`, this step's K/V row: all requested
-        // before any is consumed
-        const bool rot = cs != nullptr && c0 < 2 * half;
-        const bool first = c0 < half;
-        const int j0 = first ? c0 : c0 - half, co = first ? c0 + half : c0 - half;
-        float cosv[8], sinv[8];
-        if (rot) { load_bf16x8(cs + j0, cosv); load_bf16x8(sn + j0, sinv); }
-        const E* head = qkv + (long)(kvh * G + g) * dh;
-        unsigned long long qa[2 * RW], qb[2 * RW];
-#pragma unroll
-        for (int r = 0; r < 2 * RW; ++r) qb[r] = 0ull;
-        cload_row(head + c0, qa);
-        if (rot) cload_row(head + co, qb);
-        const bool fresh = c == owner && sid == 0;           // this lane group handles the new row
-        unsigned long long ka[2 * RW], kb[2 * RW], va[2 * RW];
-#pragma unroll
-        for (int r = 0; r < 2 * RW; ++r) { ka[r] = 0ull; kb[r] = 0ull; va[r] = 0ull; }
-        if (fresh) {
-            cload_row(knew + c0, ka);
-            if (rot) cload_row(knew + co, kb);
-            cload_row(vnew + c0, va);
-        }
-        auto rope = [&](const unsigned long long (&own2)[2 * RW], const unsigned long long (&oth2)[2 * RW], float (&out)[8]) {
-            float own[8], other[8];
-            words_values(own2, own);
-            if (!rot) {
-#pragma unroll
-                for (int v = 0; v < 8; ++v) out[v] = own[v];
-                return;
-            }
-            words_values(oth2, other);
-#pragma unroll
-            for (int v = 0; v < 8; ++v)
-                out[v] = rbf(first ? own[v] * cosv[v] - other[v] * sinv[v] : own[v] * cosv[v] + other[v] * sinv[v]);
-        };
-        float qf[8];
-        rope(qa, qb, qf);
-
-        auto visit = [&](const float (&kf)[8], const float (&vf)[8]) {
-            float sc = 0.f;
-#pragma unroll
-            for (int v = 0; v < 8; ++v) sc += qf[v] * kf[v];
-            sc = group_sum(sc, lpr) * scale;
-            const float mn = fmaxf(m, sc);
-            const float corr = fast_exp(m - mn);
-            const float pe = fast_exp(sc - mn);
-            l = l * corr + pe;
-#pragma unroll
-            for (int v = 0; v < 8; ++v) o[v] = o[v] * corr + pe * vf[v];
-            m = mn;
-        };
+    u32x4 kraw[PP][RW], vraw[PP][RW];
+    auto request_rows = [&](u32x4 (&raw)[PP][RW], const E* cache, int base) {
 #pragma unroll
         for (int j = 0; j < PP; ++j) {
-            const long p = p0 + sid + (long)j * stride;
-            if (p < p1 && p != upd) {
-                float kf[8], vf[8];
-                row_values(kraw[j], kf);
-                row_values(vraw[j], vf);
-                visit(kf, vf);
-            }
-        }
-        for (long p = p0 + sid + (long)PP * stride; p < p1; p += stride) {
-            if (p == upd) continue;
-            float kf[8], vf[8];
-            const long row = ((long)kvh * cap + p) * dh + c0;
-            load_row(kc + row, kf);
-            load_row(vc + row, vf);
-            visit(kf, vf);
-        }
-        if (fresh) {   // this step's row: attended to when in range; appended once (by head 0's wave)
-            float kf[8], vf[8];
-            rope(ka, kb, kf);
-            words_values(va, vf);
-            if (g == 0) {
-                const long row = ((long)kvh * cap + upd) * dh + c0;
-                if (F32) {
+            const int p = base + sid + j * stride;
+            const bool take = p < p1 && p != upd;
 #pragma unroll
-                    for (int r = 0; r < RW; ++r) {
-                        gstore4(kc + row + 4 * r, make_uint4((unsigned)ka[2 * r], (unsigned)(ka[2 * r] >> 32), (unsigned)ka[(2 * r + 1) % (2 * RW)], (unsigned)(ka[(2 * r + 1) % (2 * RW)] >> 32)));
-                        gstore4(vc + row + 4 * r, make_uint4((unsigned)va[2 * r], (unsigned)(va[2 * r] >> 32), (unsigned)va[(2 * r + 1) % (2 * RW)], (unsigned)(va[(2 * r + 1) % (2 * RW)] >> 32)));
-                    }
-                } else {
-                    gstore4(kc + row, make_uint4(pack_bf16x2(kf[0], kf[1]), pack_bf16x2(kf[2], kf[3]), pack_bf16x2(kf[4], kf[5]), pack_bf16x2(kf[6], kf[7])));
-                    gstore4(vc + row, make_uint4((unsigned)va[0], (unsigned)(va[0] >> 32), (unsigned)va[1], (unsigned)(va[1] >> 32)));
-                }
-            }
-            if (upd >= p0 && upd < p1) visit(kf, vf);
+            for (int r = 0; r < RW; ++r) raw[j][r] = take ? *(const GPTRS_GLOBAL u32x4*)(cache + (long)p * dh + c0 + 4 * r) : u32x4{0u, 0u, 0u, 0u};
         }
-        // merge the lane groups of this wave
-        for (int off = lpr; off < 64; off <<= 1) {
-            float ma, mb, la, lb;
-            lane_pair(m, off, ma, mb);
-            lane_pair(l, off, la, lb);
-            const float mn = fmaxf(ma, mb);
-            const float ca = mn == -INFINITY ? 0.f : fast_exp(ma - mn);
-            const float cb = mn == -INFINITY ? 0.f : fast_exp(mb - mn);
-            l = la * ca + lb * cb;
+    };
+    auto row_values = [&](const u32x4 (&raw)[RW], float (&f)[8]) {
+        const unsigned w[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[RW - 1].x, raw[RW - 1].y, raw[RW - 1].z, raw[RW - 1].w};
 #pragma unroll
-            for (int v = 0; v < 8; ++v) {
-                float oa, ob;
-                lane_pair(o[v], off, oa, ob);
-                o[v] = oa * ca + ob * cb;
-            }
-            m = mn;
+        for (int v = 0; v < 8; ++v) f[v] = F32 ? __uint_as_float(w[v]) : ((v & 1) ? bf16hi(w[v >> 1]) : bf16lo(w[v >> 1]));
+    };
+    // a row that the phase before has written: agent-scope loads
+    auto request_new = [&](const E* p, u32x4 (&raw)[RW]) {
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            const unsigned long long a = cload8(p + (F32 ? 4 : 8) * r), b = cload8(p + (F32 ? 4 : 8) * r + (F32 ? 2 : 4));
+            raw[r].x = (unsigned)a; raw[r].y = (unsigned)(a >> 32); raw[r].z = (unsigned)b; raw[r].w = (unsigned)(b >> 32);
+        }
+    };
+    request_rows(kraw, kc, p0);
+    request_rows(vraw, vc, p0);
+    const bool rot = rotate && c0 < 2 * half, first = c0 < half;
+    u32x4 cosr[1], sinr[1];
+    if (rot) {
+        const int j0 = first ? c0 : c0 - half;
+        cosr[0] = *(const GPTRS_GLOBAL u32x4*)((const bf16_t*)P.cos + j0);
+        sinr[0] = *(const GPTRS_GLOBAL u32x4*)((const bf16_t*)P.sin + j0);
+    }
+    if (!wait_go(go, abort, phase, budget)) return false;
+
+    // The wave's query head and, in the first position subset of the workgroup that owns position `upd`, this step's K and V rows
+    // (for the first lane group), all requested before any is consumed; RoPE on the fly.
+    const bool new_row = owner && part == 0;
+    u32x4 qa[RW], qb[RW], ka[RW], kb[RW], va[RW];
+    {
+        const int co = first ? c0 + half : c0 - half;
+        const E* head = qkv + (long)(kvh * G + g) * dh;
+        const E* knew = qkv + (long)(n_q + kvh) * dh;
+        request_new(head + c0, qa);
+        if (rot) request_new(head + co, qb);
+        if (new_row) {
+            request_new(knew + c0, ka);
+            if (rot) request_new(knew + co, kb);
+            request_new(knew + (long)n_kv * dh + c0, va);
         }
     }
-    // merge the waves of each head through LDS and leave one record per query head
+    auto rope = [&](const u32x4 (&own_raw)[RW], const u32x4 (&other_raw)[RW], float (&out)[8]) {
+        row_values(own_raw, out);
+        if constexpr (!F32) {
+            if (rot) {
+                float other[8], cosv[8], sinv[8];
+                row_values(other_raw, other);
+                row_values(cosr, cosv);
+                row_values(sinr, sinv);
+#pragma unroll
+                for (int v = 0; v < 8; ++v) out[v] = rbf(first ? out[v] * cosv[v] - other[v] * sinv[v] : out[v] * cosv[v] + other[v] * sinv[v]);
+            }
+        }
+    };
+    float qf[8], m = -INFINITY, l = 0.f, o[8];
+    rope(qa, qb, qf);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) o[v] = 0.f;
+    auto score = [&](const float (&kf)[8]) {
+        float s = qf[0] * kf[0];
+#pragma unroll
+        for (int v = 1; v < 8; ++v) s = __builtin_fmaf(qf[v], kf[v], s);
+        return s;
+    };
+    if (new_row) {   // this step's row: attended to when in range, appended once (by head 0's wave)
+        float kf[8], vf[8], s[1];
+        rope(ka, kb, kf);
+        row_values(va, vf);
+        if (sub == 0 && g == 0) {
+            E* kd = kc + (long)upd * dh + c0;
+            E* vd = vc + (long)upd * dh + c0;
+            if constexpr (F32) {
+#pragma unroll
+                for (int r = 0; r < RW; ++r) { *(GPTRS_GLOBAL u32x4*)(kd + 4 * r) = ka[r]; *(GPTRS_GLOBAL u32x4*)(vd + 4 * r) = va[r]; }
+            } else {
+                u32x4 kw;
+                kw.x = pack_bf16x2(kf[0], kf[1]); kw.y = pack_bf16x2(kf[2], kf[3]); kw.z = pack_bf16x2(kf[4], kf[5]); kw.w = pack_bf16x2(kf[6], kf[7]);
+                *(GPTRS_GLOBAL u32x4*)kd = kw;
+                *(GPTRS_GLOBAL u32x4*)vd = va[0];
+            }
+        }
+        s[0] = score(kf);
+        group_sums(s, lpr);
+        if (sub == 0 && upd >= p0 && upd < p1) {
+            m = s[0] * scale;
+            l = 1.f;
+#pragma unroll
+            for (int v = 0; v < 8; ++v) o[v] = vf[v];
+        }
+    }
+    for (int base = p0;;) {
+        float s[PP], mn = m;
+#pragma unroll
+        for (int j = 0; j < PP; ++j) {
+            float kf[8];
+            row_values(kraw[j], kf);
+            s[j] = score(kf);
+        }
+        group_sums(s, lpr);
+#pragma unroll
+        for (int j = 0; j < PP; ++j) {
+            const int p = base + sid + j * stride;
+            s[j] = p < p1 && p != upd ? s[j] * scale : -INFINITY;
+            mn = fmaxf(mn, s[j]);
+        }
+        const int next = base + PP * stride;
+        const bool more = next < p1;
+        if (more) request_rows(kraw, kc, next);
+        const float ref = finite_max(mn), corr = fast_exp(m - ref);
+        m = mn;
+        l *= corr;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) o[v] *= corr;
+#pragma unroll
+        for (int j = 0; j < PP; ++j) {
+            float vf[8];
+            row_values(vraw[j], vf);
+            s[j] = fast_exp(s[j] - ref);
+            l += s[j];
+#pragma unroll
+            for (int v = 0; v < 8; ++v) o[v] = __builtin_fmaf(s[j], vf[v], o[v]);
+        }
+        if (!more) break;
+        request_rows(vraw, vc, next);
+        base = next;
+    }
+    // The lane groups of the wave: one maximum, then sums in which each half of the lanes goes on with half of the values.
+    // Which of its 8 a lane ends up with: bits 5, 4 and 3 of its number, as many of them as there are lane groups.
+    float mw = m;
+    if (lpr == 8) mw = fmaxf(mw, dpp<DPP_ROR8>(mw));
+    if (lpr <= 16) mw = pair_max16(mw);
+    mw = pair_max32(mw);
+    const float cw = fast_exp(m - finite_max(mw));
+    l *= cw;
+    l = halves32(l, l);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) o[v] *= cw;
+    float h4[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) h4[v] = halves32(o[v], o[v + 4]);
     GPTRS_LDS float* sm = lds;
     GPTRS_LDS float* sl = lds + NWS;
     GPTRS_LDS float* so = lds + 2 * NWS;
-    if (!control && sub == 0) {
-        if (li == 0) { sm[wave] = m; sl[wave] = l; }
-#pragma unroll
-        for (int v = 0; v < 8; ++v) so[wave * dh + c0 + v] = o[v];
-    }
-    wg_barrier();
-    float* partp = P.part;
-    const bool final = P.flags & kChainAttnFinal;
-    for (int idx = t; idx < G * dh; idx += NT) {
-        const int gg = idx / dh, d = idx - gg * dh;
-        float mn = -INFINITY;
-        for (int w = gg; w < NWS; w += G) mn = fmaxf(mn, sm[w]);
-        float Ls = 0.f, O = 0.f;
-        if (mn != -INFINITY) {
-            for (int w = gg; w < NWS; w += G) {
-                const float cw = fast_exp(sm[w] - mn);
-                Ls += sl[w] * cw;
-                O += so[w * dh + d] * cw;
-            }
+    GPTRS_LDS float* mine = so + wave * dh + c0 + (lane >> 5) * 4;
+    if (lpr == 32) {
+        GPTRS_LDS f32x4* d4 = (GPTRS_LDS f32x4*)mine;
+        *d4 = f32x4{h4[0], h4[1], h4[2], h4[3]};
+    } else {
+        l = halves16(l, l);
+        const float h0 = halves16(h4[0], h4[2]), h1 = halves16(h4[1], h4[3]);
+        mine += ((lane >> 4) & 1) * 2;
+        if (lpr == 16) {
+            mine[0] = h0;
+            mine[1] = h1;
+        } else {
+            l += dpp<DPP_ROR8>(l);
+            const bool up = lane & 8;
+            const float keep = up ? h1 : h0, give = up ? h0 : h1;
+            mine[up ? 1 : 0] = keep + dpp<DPP_ROR8>(give);
         }
+    }
+    if (lane == 0) { sm[wave] = mw; sl[wave] = l; }
+    wg_barrier();
+    // the waves of each head: one record per query head
+    const bool final = P.flags & kChainAttnFinal;
+    for (int idx = t; idx < G * dh; idx += NS) {
+        const int gg = idx >> (lsh + 3), d = idx & (dh - 1);
+        float mr, lr, orr;
+        if (nparts == 2) merge_waves<2>(sm, sl, so, gg, 4, dh, d, mr, lr, orr);
+        else if (nparts == 8) merge_waves<8>(sm, sl, so, gg, 1, dh, d, mr, lr, orr);
+        else if (nparts == 4) merge_waves<4>(sm, sl, so, gg, 2, dh, d, mr, lr, orr);
+        else merge_waves<1>(sm, sl, so, gg, 8, dh, d, mr, lr, orr);
         if (final) {
             // one chunk per kv head: its record is the whole softmax, and the context row is written here (what the merge of
             // a single record gives: O / L)
             const long at = (long)(kvh * G + gg) * dh + d;
-            if (F32) cstore4((float*)P.y + at, __float_as_uint(O / Ls));
-            else __hip_atomic_store(as_global((unsigned short*)P.y + at), (unsigned short)pack_bf16x2(O / Ls, 0.f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (F32) cstore4((float*)P.y + at, __float_as_uint(orr / lr));
+            else __hip_atomic_store(as_global((unsigned short*)P.y + at), (unsigned short)pack_bf16x2(orr / lr, 0.f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             continue;
         }
-        float* rec = partp + ((long)(kvh * G + gg) * nch + c) * (dh + 2);
-        if (d == 0) { cstore4(rec, __float_as_uint(mn)); cstore4(rec + 1, __float_as_uint(Ls)); }
-        cstore4(rec + 2 + d, __float_as_uint(O));
+        float* rec = P.part + ((long)(kvh * G + gg) * nch + c) * (dh + 2);
+        cstore4(rec + 2 + d, __float_as_uint(orr));
+        if (d == 0) cstore8(rec, (unsigned long long)__float_as_uint(mr) | ((unsigned long long)__float_as_uint(lr) << 32));
     }
     // every lane's stores (record words, the appended cache row) have left the CU before the control wave, which passes
-    // this barrier last of all it executes here, reports the workgroup's arrival
+    // this barrier as well, reports the workgroup's arrival
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     wg_barrier();
     return true;
 }
 
-// unit = query head: softmax-merge of its nch chunk records into the context row.  Thread
-// (sg, d2) reads the records of the chunks s = sg, sg + NW, ... for the dims (2 d2, 2 d2 + 1) in
-// one round of loads and merges them locally; the NW subsets meet in LDS.
+// unit = query head: softmax-merge of its nch chunk records into the context row.  A lane has the dims 2 d2, 2 d2 + 1 of the chunks
+// wave, wave + 8, ...: all requested at once, merged, and the 8 waves' parts meet in LDS.
+template <int N_REC>
+__device__ __forceinline__ void merge_chunks(const float* base, int wave, int nch, int dh, int d2, bool act, float& m, float& l, float& o0, float& o1) {
+    unsigned long long ml[N_REC], ov[N_REC];
+#pragma unroll
+    for (int u = 0; u < N_REC; ++u) {
+        const int s = wave + u * NWS;
+        const bool ok = act && s < nch;
+        const float* rec = base + (long)s * (dh + 2);
+        ml[u] = ok ? cload8(rec) : 0xff800000ull;   // (-inf, 0)
+        ov[u] = ok ? cload8(rec + 2 + 2 * d2) : 0ull;
+    }
+    m = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < N_REC; ++u) m = fmaxf(m, __uint_as_float((unsigned)ml[u]));
+    const float ref = finite_max(m);
+    l = 0.f; o0 = 0.f; o1 = 0.f;
+#pragma unroll
+    for (int u = 0; u < N_REC; ++u) {
+        const float c = fast_exp(__uint_as_float((unsigned)ml[u]) - ref);
+        l += __uint_as_float((unsigned)(ml[u] >> 32)) * c;
+        o0 += __uint_as_float((unsigned)ov[u]) * c;
+        o1 += __uint_as_float((unsigned)(ov[u] >> 32)) * c;
+    }
+}
 template <bool F32>
-__device__ bool attn_combine_t(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq, int phase,
+__device__ bool attn_combine(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq, int phase,
                              unsigned long long budget) {
-    constexpr int MAXC = 8;   // chunks per thread: nch <= MAXC * NW
-    const int t = local_tid(), wave = uni(t >> 6);
-    const int dh = P.head_dim, nch = P.nch;
-    if (wave != NWS && !wait_go(go, abort, phase, budget)) return false;
+    const int t = local_tid(), wave = uni(t >> 6), lane = t & 63;
+    const int dh = P.head_dim, nch = P.nch, h2 = dh / 2;   // nch <= 64
     const float* base = P.part + (long)hq * nch * (dh + 2);
-    bf16_t* ctx = (bf16_t*)P.y;
-    const int h2 = dh / 2;
+    if (!wait_go(go, abort, phase, budget)) return false;
     for (int d0 = 0; d0 < h2; d0 += 64) {
-        const int d2 = d0 + (t & 63);
+        const int d2 = d0 + lane;
         const bool act = d2 < h2;
-        unsigned long long ml[MAXC], ov[MAXC];
-#pragma unroll
-        for (int u = 0; u < MAXC; ++u) {
-            const int s = wave + u * NW;
-            const bool ok = act && s < nch;
-            ml[u] = ok ? cload8(base + (long)s * (dh + 2)) : 0ull;
-            ov[u] = ok ? cload8(base + (long)s * (dh + 2) + 2 + 2 * d2) : 0ull;
-        }
-        float mn = -INFINITY;
-#pragma unroll
-        for (int u = 0; u < MAXC; ++u)
-            if (wave + u * NW < nch) mn = fmaxf(mn, __uint_as_float((unsigned)ml[u]));
-        float Ls = 0.f, o0 = 0.f, o1 = 0.f;
-#pragma unroll
-        for (int u = 0; u < MAXC; ++u) {
-            if (wave + u * NW < nch) {
-                const float ms = __uint_as_float((unsigned)ml[u]);
-                const float cw = ms == -INFINITY ? 0.f : fast_exp(ms - mn);
-                Ls += __uint_as_float((unsigned)(ml[u] >> 32)) * cw;
-                o0 += __uint_as_float((unsigned)ov[u]) * cw;
-                o1 += __uint_as_float((unsigned)(ov[u] >> 32)) * cw;
-            }
-        }
+        float m, l, o0, o1;
+        if (nch <= 4 * NWS) merge_chunks<4>(base, wave, nch, dh, d2, act, m, l, o0, o1);
+        else merge_chunks<8>(base, wave, nch, dh, d2, act, m, l, o0, o1);
         GPTRS_LDS f32x4* rec = (GPTRS_LDS f32x4*)lds;
-        { f32x4 r4; r4.x = mn; r4.y = Ls; r4.z = o0; r4.w = o1; rec[wave * 64 + (t & 63)] = r4; }
+        rec[wave * 64 + lane] = f32x4{m, l, o0, o1};
         wg_barrier();
         if (wave == 0 && act) {
-            float M = -INFINITY;
+            f32x4 v[NWS];
 #pragma unroll
-            for (int w = 0; w < NW; ++w) M = fmaxf(M, rec[w * 64 + t].x);
+            for (int w = 0; w < NWS; ++w) v[w] = rec[w * 64 + lane];
+            float M = v[0].x;
+#pragma unroll
+            for (int w = 1; w < NWS; ++w) M = fmaxf(M, v[w].x);
+            const float ref = finite_max(M);
             float Lt = 0.f, a0 = 0.f, a1 = 0.f;
 #pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const f32x4 r = rec[w * 64 + t];
-                const float cw = r.x == -INFINITY ? 0.f : fast_exp(r.x - M);
-                Lt += r.y * cw; a0 += r.z * cw; a1 += r.w * cw;
+            for (int w = 0; w < NWS; ++w) {
+                const float cw = fast_exp(v[w].x - ref);
+                Lt += v[w].y * cw; a0 += v[w].z * cw; a1 += v[w].w * cw;
             }
             if (F32) cstore8((float*)P.y + (long)hq * dh + 2 * d2, (unsigned long long)__float_as_uint(a0 / Lt) | ((unsigned long long)__float_as_uint(a1 / Lt) << 32));
-            else cstore4(ctx + (long)hq * dh + 2 * d2, pack_bf16x2(a0 / Lt, a1 / Lt));
+            else cstore4((bf16_t*)P.y + (long)hq * dh + 2 * d2, pack_bf16x2(a0 / Lt, a1 / Lt));
         }
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the context words are out before the arrival is reported
         wg_barrier();
@@ -1175,11 +950,12 @@ __device__ bool attn_combine_t(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Ch
     return true;
 }
 
-// The 9 compute and control waves of the workgroup: the units blk, blk + grid, ... of an attention phase.  Kept out of
-// line (its register needs must not leak into the compute loop); the LDS operands travel as explicit
+// The compute waves of the workgroup: the units blk, blk + grid, ... of an attention phase.  The LDS operands travel as explicit
 // local-address-space pointers so their accesses stay ds_* instructions.
-// The descriptor comes straight from the table in memory (scalar loads): the compute waves enter an attention phase, and
-// request the cache rows it needs, before the control wave has seen the barrier and filled the LDS copy.
+// The descriptor comes straight from the table in memory (scalar loads): the waves enter an attention phase, and
+// request the cache rows it needs, before the control wave has seen the barrier.
+// The control wave only takes part in the workgroup barriers (attn_barriers of them to a unit).
+__device__ __forceinline__ int attn_barriers(int kind, int head_dim) { return kind == kChainAttnCombine && head_dim > 128 ? 4 : 2; }
 template <bool F32>
 __device__ __forceinline__ bool run_attn_phase(const GPTRS_CONST ChainPhase* php, GPTRS_LDS float* lds, GPTRS_LDS int* go, GPTRS_LDS int* abort, int phase,
                                                unsigned long long budget) {
@@ -1192,14 +968,7 @@ __device__ __forceinline__ bool run_attn_phase(const GPTRS_CONST ChainPhase* php
     }
     const int kind = P.kind, units = P.units;
     for (int u = blockIdx.x; u < units; u += gridDim.x) {
-        bool ok;
-        if (F32) {
-            if (kind == kChainAttnCombine) ok = attn_combine_t<true>(go, abort, P, lds, u, phase, budget);
-            else ok = attn_partial_t<true>(go, abort, P, lds, u, phase, budget);
-        } else {
-            if (kind == kChainAttnCombine) ok = attn_combine(go, abort, P, lds, u, phase, budget);
-            else ok = attn_partial(go, abort, P, lds, u, phase, budget);
-        }
+        const bool ok = kind == kChainAttnCombine ? attn_combine<F32>(go, abort, P, lds, u, phase, budget) : attn_partial<F32>(go, abort, P, lds, u, phase, budget);
         if (!ok) return false;
     }
     return true;
@@ -1227,7 +996,7 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
         const int pd = lane < kPhaseDwords ? gload(reinterpret_cast<const int*>(phases + ph) + lane) : 0;
         const GPTRS_CONST ChainPhase* D = table + ph;
         const int kind = uni(D->kind);
-        const int units = uni(D->units);
+        const int units = uni(D->units), barriers = attn_barriers(kind, uni(D->head_dim));
         const int T = kind == kChainLinear ? tile_count(blk, uni(D->tlo), uni(D->trem)) : 0;
         if (ph > 0) {
             // stall_phase (a test hook, -1 otherwise): one arrival more than the grid can deliver is expected at that
@@ -1251,7 +1020,7 @@ __device__ void control_wave(Shared& sh, unsigned* xs, const ChainPhase* phases,
         if (kind != kChainLinear) {
             if (blk < units) {
                 if (lane == 0) lds_st(&sh.go, ph);
-                run_attn_phase<FMT == kChainW32>(table + ph, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.go, (GPTRS_LDS int*)&sh.abort, ph, budget);
+                for (int n = barriers * ((units - 1 - blk) / (int)gridDim.x + 1); n > 0; --n) wg_barrier();
             }
         } else if (T > 0) {
             if (lane == 0) lds_st(&sh.go, ph);
@@ -2031,7 +1800,7 @@ void chain_fill_attn(ChainPhase& partial, ChainPhase& combine, int64_t n_q, int6
     partial.lds_bytes = partial.lds_total = (int)((2 * NWS + NWS * head_dim) * sizeof(float));
     combine.kind = kChainAttnCombine;
     combine.units = (int)n_q;
-    combine.lds_bytes = combine.lds_total = (int)(NW * 64 * sizeof(float4));
+    combine.lds_bytes = combine.lds_total = (int)(NWS * 64 * sizeof(float4));
 }
 
 bool chain_launch(hipStream_t s, const ChainPhase* dev_table, int nphases, int lds_bytes, unsigned* bar, int* abort_flag, int wfmt,

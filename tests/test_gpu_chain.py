@@ -204,6 +204,28 @@ def test_decode_attention_in_chain(hip, hq, hkv, dh, rope, cap):
             assert_close(g[:, pos], w[:, pos], atol=2e-2, rtol=2e-2, what=f"appended row of cache {i} at pos {pos}")
 
 
+@pytest.mark.parametrize("hq,hkv,dh,cap", [(8, 1, 256, 2048), (8, 2, 128, 1024), (4, 4, 64, 128)])
+def test_decode_attention_appends_elsewhere_than_it_looks(hip, hq, hkv, dh, cap):
+    """The row is written at one position and the query stands at another: the new row counts only where it is in range, a chunk
+    may hold nothing else, and lanes take several steps of rows (one kv head of 256: two rows of a chunk at a time)."""
+    d = 128
+    cfg = F.AttentionConfig(embed_dim=d, num_query_heads=hq, num_key_value_heads=hkv, head_dim=dh)
+    tp, qp = cfg.total_projection_dim, cfg.query_projection_dim
+    arrays = [rnd(40, (1, d)), rnd(41, (d, tp), 2.0 / np.sqrt(d)), rnd(42, (qp, d), 2.0 / np.sqrt(qp)), rnd(43, (hkv, cap, dh)), rnd(44, (hkv, cap, dh))]
+
+    def build(fb, a, w1, w2, k, v, us, qs):
+        c, k2, v2 = F.attention_decode_cache(cfg, a.matmul(w1), k, v, us, qs)
+        return [c.matmul(w2), k2, v2]
+
+    specs, ints = [list(a.shape) for a in arrays], [("Si32", [3]), ("Si32", [1])]
+    pb, pf = (prog(build, [(t, s) for s in specs] + ints) for t in ("Bf16", "F32"))
+    for qpos, upd in [(0, 0), (0, 5), (40, 100), (100, 40), (cap - 1, cap // 2), (cap // 2, cap - 1)]:
+        us, qs = np.array([0, upd, 0], np.int32), np.array([qpos], np.int32)
+        got = hip_run(hip, pb, arrays + [us, qs])
+        want = oracle_run(pf, [bf16_round(a) for a in arrays] + [us, qs])
+        assert_close(got[0], want[0], atol=3e-2, rtol=2e-2, what=f"context projection, query at {qpos}, row at {upd}")
+
+
 def test_grid_barrier_gives_up_and_the_backend_goes_on(hip):
     """A grid barrier that cannot complete must end in an execution error, not in a hang: the host option
     "chain_stall_phase" makes every workgroup of the next launch expect one arrival more than the grid can deliver at that
