@@ -205,9 +205,12 @@ void dequant_w4g128(hipStream_t s, int dtype, const uint8_t* packed, const void*
 // copy), bias, exact-erf GELU, residual.  x, residual and y may be produced by earlier phases of
 // the same launch.
 constexpr int kChainCounters = 16;        // striped arrival counters of the grid barrier
+constexpr int kChainGroups = 8;           // workgroups b, b + 8, b + 16, ... of a launch: on this card they share an L2 cache
+constexpr int kChainLine = 64;            // words from one barrier word to the next: lines of their own
 constexpr int kChainMaxPhases = 192;
 constexpr int kChainMaxXsWords = 12288;   // staged activation words (48 KiB): K <= 24576 for bf16 weights
-constexpr size_t kChainBarrierBytes = (kChainCounters * 64 + 64) * sizeof(unsigned);  // zero-initialised once
+// striped counters, arrivals of each group, notes from group to group [to][from], the counts that the next launch starts from; zero-initialised once
+constexpr size_t kChainBarrierBytes = (kChainCounters + kChainGroups + kChainGroups * kChainGroups + 1) * kChainLine * sizeof(unsigned);
 // kChainOutF32: y and the residual are f32.  kChainXF32 (with kChainNorm): x and gamma are f32, the normalised row is
 // rounded to bf16 once as it is staged.
 // kChainLayerNorm (with kChainNorm, f32 phases or kChainXF32): LayerNorm with gains `gamma` and offsets `beta` instead of RMSNorm.

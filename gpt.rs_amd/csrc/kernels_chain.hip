@@ -21,7 +21,7 @@
 //     bf16 pairs); at the end of a tile the wave leaves its part of the tile's 4 sums in LDS.
 //   * 1 control wave per workgroup adds the parts of a phase's tiles when all waves are done, a lane to each output column,
 //     applies the epilogue (SwiGLU pair, bias, GELU, residual), stores through to memory, and runs the grid
-//     barrier (16 striped arrival counters, one poll instruction).
+//     barrier (16 striped arrival counters, or counters of groups and notes between them; one poll instruction).
 //   * Activations cross workgroups through agent-scope (sc1) loads and stores only, so no
 //     L2 write-back / invalidate is needed between phases; a phase's input vector is staged into
 //     LDS by the 9 compute and control waves together right after the barrier (RMSNorm statistics
@@ -63,7 +63,7 @@ constexpr int NT = NS + 64;      // + control wave: the threads that stage input
 constexpr int NWS = NS / 64;
 constexpr int SW = 3;            // words of a step: what a wave requests and consumes at a time
 constexpr int CW = 64;           // lanes, and 16-byte pieces, of a word
-constexpr int NC = kChainCounters;
+constexpr int NC = kChainCounters, NG = kChainGroups, LINE = kChainLine;
 constexpr int EPI_MAX = 640;     // output columns of a workgroup, staged values among them: N <= 640 * grid (tiles that do not divide evenly: up to 4 fewer)
 constexpr int MAXI = 8;          // 8-byte items per thread in the norm staging: K <= 4*MAXI*NT
 constexpr int STEP_BYTES = SW * CW * 16;     // a step of a wave
@@ -998,8 +998,19 @@ __device__ __forceinline__ void control_wave(GPTRS_LDS Shared& sh, GPTRS_LDS uns
                              unsigned long long budget, int stall_phase) {
     PhaseTable table = (PhaseTable)phases;
     const int lane = threadIdx.x & 63;
-    const int blk = blockIdx.x, per = gridDim.x / NC;
-    const unsigned epoch = gload(bar + NC * 64);   // written by the previous launch, stable during this one
+    // The grid barrier.  Striped: a workgroup adds one to one of NC counters, and everybody polls all of them.  With notes: it adds one to its group's counter and
+    // is told how many came before it; the last of a group leaves a note for every group, and everybody polls the eight notes for its own group, which
+    // the group's L2 holds between two of them.  Two hops for one, but the arrivals meet nobody's polls.  By themselves 1.72 and 2.10 us (with values out and in 2.53 and 2.91);
+    // 61 phases of GPT-2 305 and 327 us, 157 of bf16 1510 and 1545.  Where codes are streamed the wait for the answer costs more than that (int8 1121
+    // and 1111, int4 1090 and 1060).  Every access is of agent scope: that a group shares a cache makes the notes fast, not right.
+    constexpr bool NOTES = FMT == kChainW16 || FMT == kChainW32;
+    const int blk = blockIdx.x, grp = blk % NG;
+    const unsigned per = gridDim.x / NC, members = gridDim.x / NG;
+    unsigned* const group_count = bar + (NC + grp) * LINE;
+    unsigned* const notes = bar + (NC + NG) * LINE;
+    unsigned* const counted = bar + (NC + NG + NG * NG) * LINE + (NOTES ? 1 : 0);   // phases that launches with this barrier have had
+    const unsigned epoch = gload(counted);   // written by the previous launch, stable during this one
+    const GPTRS_GLOBAL unsigned* const word = as_global(NOTES ? notes + (grp * NG + lane) * LINE : bar + lane * LINE);
     int handed = 0;   // arrivals of compute waves that the phases up to this one bring
     for (int ph = 0; ph < nphases; ++ph) {
         // the phase's descriptor is requested before the wait for the barrier and lands in LDS after it, ahead of `go`
@@ -1011,11 +1022,11 @@ __device__ __forceinline__ void control_wave(GPTRS_LDS Shared& sh, GPTRS_LDS uns
         if (ph > 0) {
             // stall_phase (a test hook, -1 otherwise): one arrival more than the grid can deliver is expected at that
             // phase, so this wait runs out of time and the give-up path below is taken
-            const unsigned target = epoch + (unsigned)ph * per + (ph == stall_phase ? 1u : 0u);
+            const unsigned target = (epoch + (unsigned)ph) * (NOTES ? 1u : per) + (ph == stall_phase ? 1u : 0u);
             Patience pat(budget);
             bool ok = true;
             for (;;) {
-                const unsigned v = lane < NC ? __hip_atomic_load(as_global(bar) + lane * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : target;
+                const unsigned v = lane < (NOTES ? NG : NC) ? __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : target;
                 if (__builtin_amdgcn_ballot_w64((int)(v - target) < 0) == 0) break;
                 __builtin_amdgcn_s_sleep(1);
                 if (pat.spent() || ((pat.spins & 63u) == 0 && __hip_atomic_load(as_global(abort_flag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) { ok = false; break; }
@@ -1191,10 +1202,18 @@ __device__ __forceinline__ void control_wave(GPTRS_LDS Shared& sh, GPTRS_LDS uns
         // this workgroup's outputs have left the CU before it arrives at the barrier
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
         asm volatile("" ::: "memory");
-        if (lane == 0) __hip_atomic_fetch_add(as_global(bar) + (blk % NC) * 64, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (NOTES) {
+            unsigned before = 0u;
+            if (lane == 0) before = __hip_atomic_fetch_add(as_global(group_count), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned done = epoch + (unsigned)ph + 1u;
+            if ((unsigned)uni((int)before) + 1u == done * members && lane < NG)
+                __hip_atomic_store(as_global(notes) + (lane * NG + grp) * LINE, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (lane == 0) {
+            __hip_atomic_fetch_add(as_global(bar) + (blk % NC) * LINE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
-    // every launch advances each counter by nphases * per: the next launch starts from there
-    if (blk == 0 && lane == 0) gstore(bar + NC * 64, epoch + (unsigned)nphases * per);
+    // every launch counts its phases: the next launch starts from there
+    if (blk == 0 && lane == 0) gstore(counted, epoch + (unsigned)nphases);
 }
 
 // In the bf16 kernel, where requests ahead fill what the barriers leave, the compute waves' registers are dealt better beside a function of its own (157 phases 1542 us,
