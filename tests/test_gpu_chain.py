@@ -356,6 +356,16 @@ def test_f32_single_linear(hip, k, n):
 
 @pytest.mark.parametrize("k,n", [(768, 2304), (3072, 768), (100, 40)])
 def test_f32_layer_norm_linear_bias(hip, k, n):
+    run_f32_layer_norm_linear_bias(hip, k, n)
+
+
+@pytest.mark.parametrize("k,n", [(4, 8), (60, 40), (256, 40), (260, 40), (1020, 40), (1024, 40), (1028, 40)])
+def test_f32_layer_norm_of_rows_that_one_wave_reads(hip, k, n):
+    """Up to 1024 values each wave finds a row's mean and variance by itself; lengths at the edges of its loads and of that rule."""
+    run_f32_layer_norm_linear_bias(hip, k, n)
+
+
+def run_f32_layer_norm_linear_bias(hip, k, n):
     x, g, bt = rnd(33, (1, k), 3.0) + 0.7, rnd(34, (k,)) + 1.5, rnd(35, (k,))
     w, b = rnd(36, (k, n), 2.0 / np.sqrt(k)), rnd(37, (n,))
     run_both_f32(hip, lambda fb, a, gm, be, c, d: F.linear(F.layer_norm(a, gm, be, 1e-5)[0], c, d),
