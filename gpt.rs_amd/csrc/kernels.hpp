@@ -167,7 +167,11 @@ struct SkinnyLinearArgs {
     int quant; const void* scale; const void* scale2;
     int out_f32 = 0;   // bf16 only: y and residual are f32
     EpiExtra extra;    // unquantised only
+    // x are rows that the launch brings to LayerNorm itself (skinny_norm_fits): gains and offsets, f32
+    const float* gamma = nullptr; const float* beta = nullptr;
+    float inv_n = 0.f, eps = 0.f;
 };
+bool skinny_norm_fits(const SkinnyLinearArgs& a, const void* gamma, const void* beta);
 bool skinny_quant_supported(int dtype, int64_t m, int64_t k, int64_t n, int qf);
 size_t skinny_codes_bytes(int64_t k, int64_t n, int qf);
 void skinny_pack_codes(hipStream_t s, const void* codes, void* out, int64_t k, int64_t n, int qf);

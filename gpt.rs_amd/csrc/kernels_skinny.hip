@@ -223,6 +223,69 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const T* __restric
     out.store(y, out_f32, o);
 }
 
+// An f32 layer whose rows are normed first (LayerNorm), a tile for each CU at most.  Every workgroup norms all rows, wave r row r, while its weights, all of them asked
+// for before, are on their way from memory; the normed rows are the A operand in LDS, a row 16 bytes longer than it is, so that 16 rows' reads meet no bank twice.
+// Asked for ahead of the rows the weights held them up (loads return in order): 7 rows of 768, N = 2304 5.11 us, so 4.75, the norm's launch in front 6.43 and the layer
+// alone 4.21; N = 3072 4.96, 6.55 and 4.32; 16 rows 5.74 and 6.95, 5.85 and 7.09.  A tile for each CU at most, since every workgroup norms all rows.
+constexpr int kNormSteps = 4;                     // steps of 16 k of a wave: K <= 1008, where 16 rows are 64 KB
+template <int COLS>
+__global__ __launch_bounds__(1024) void skinny_norm_kernel(const float* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta, const float* __restrict__ ws,
+                                                           const float* __restrict__ bias, const float* __restrict__ residual, float* __restrict__ y, int M, int K, int N, int act,
+                                                           float inv_n, float eps, EpiExtra extra) {
+    constexpr int NW = 16;
+    extern __shared__ __align__(16) float rows[];   // [M][K + 4], then the waves' sums
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int c = lane & 15, kg = lane >> 4, nsteps = K / 16, tile = blockIdx.x;
+    const int items = K / 4;                      // of 16 bytes
+    f32x4_s v[4], g[4], o[4];
+    if (wave < M) {                               // (loads return in order: what is nearer is asked for first)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = reinterpret_cast<const f32x4_s*>(x + (int64_t)wave * K)[min(64 * j + lane, items - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            g[j] = reinterpret_cast<const f32x4_s*>(gamma)[min(64 * j + lane, items - 1)];
+            o[j] = reinterpret_cast<const f32x4_s*>(beta)[min(64 * j + lane, items - 1)];
+        }
+    }
+    const u32x4_s* bsrc = reinterpret_cast<const u32x4_s*>(ws) + (int64_t)tile * (K / 4) * COLS + kg * COLS + (c < COLS ? c : COLS - 1);
+    u32x4_s b[kNormSteps];
+#pragma unroll
+    for (int u = 0; u < kNormSteps; ++u)
+        if (wave + NW * u < nsteps) b[u] = __builtin_nontemporal_load(bsrc + (int64_t)(wave + NW * u) * (4 * COLS));
+    SkinnyOut<float, false, NW, COLS> out(tile, M, N, bias, residual, 0, extra.colscale);
+    if (wave < M) {
+        float s = 0.f, q = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s += 64 * j + lane < items ? (v[j].x + v[j].y) + (v[j].z + v[j].w) : 0.f;
+        const float mean = wave_sum(s) * inv_n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[j] -= mean;
+            q += 64 * j + lane < items ? (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w) : 0.f;
+        }
+        const float inv_std = 1.0f / sqrtf(wave_sum(q) * inv_n + eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (64 * j + lane < items) *reinterpret_cast<f32x4_s*>(&rows[wave * (K + 4) + 4 * (64 * j + lane)]) = (v[j] * inv_std) * g[j] + o[j];
+    }
+    __syncthreads();
+    f32x4_s acc = {0.f, 0.f, 0.f, 0.f};
+    const float* a = &rows[(c < M ? c : M - 1) * (K + 4) + 4 * kg];   // rows beyond M re-read the last one; their products are never stored
+#pragma unroll
+    for (int u = 0; u < kNormSteps; ++u) {
+        const int s = wave + NW * u;
+        if (s < nsteps) acc = SkinnyT<float>::mma(*reinterpret_cast<const u32x4_s*>(a + 16 * s), b[u], acc);
+    }
+    __syncthreads();
+    float (*red)[1][64][4] = reinterpret_cast<float (*)[1][64][4]>(rows);
+    *reinterpret_cast<f32x4_s*>(red[wave][0][lane]) = acc;
+    __syncthreads();
+    float sum[2];
+    if (!out.sum(red, tile, nullptr, nullptr, nullptr, sum)) return;
+    out.store(y, 0, skinny_finish(sum[0], 0.f, false, act, out.bias, residual != nullptr, out.res, extra.glu, out.colscale));
+}
+
 // Qs[tile][S][lane = 16 kg + c][16 bytes]: byte i = code row (RPW S + RPL kg + i) of column 16 tile + c, xor flip.  int8:
 // code rows are k, RPL = 16 rows per lane, flip 0x80.  int4: a code row is a packed byte of two k, RPL = 16 rows (32 k)
 // per lane, flip 0x88.  Rows and columns outside the matrix hold the biased zero.
@@ -457,8 +520,22 @@ void skinny_pack_codes(hipStream_t s, const void* codes, void* out, int64_t k, i
                                                qf == 1 ? 0x80u : 0x88u);
 }
 
+bool skinny_norm_fits(const SkinnyLinearArgs& a, const void* gamma, const void* beta) {
+    return a.dtype == 0 && !a.quant && !a.ws2 && a.extra.softcap == 0.f && a.k <= 1008 && cdiv_s(a.n, skinny_cols(a.n)) <= 256 &&
+           (((uintptr_t)a.x | (uintptr_t)gamma | (uintptr_t)beta) & 15) == 0;
+}
+
 void skinny_gemm(hipStream_t s, const SkinnyLinearArgs& a) {
     const bool dual = a.ws2 != nullptr;
+    if (a.gamma) {   // (the caller has asked skinny_norm_fits)
+        const int cols = skinny_cols(a.n);
+        const unsigned grid = (unsigned)cdiv_s(a.n, cols);
+        const size_t lds = std::max<size_t>((size_t)a.m * (a.k + 4) * sizeof(float), 16 * 64 * 4 * sizeof(float));
+        const auto fn = cols == 12 ? skinny_norm_kernel<12> : skinny_norm_kernel<16>;
+        fn<<<grid, 1024, lds, s>>>((const float*)a.x, a.gamma, a.beta, (const float*)a.ws, (const float*)a.bias, (const float*)a.residual, (float*)a.y, (int)a.m, (int)a.k,
+                                   (int)a.n, a.act, a.inv_n, a.eps, a.extra);
+        return;
+    }
     const int64_t steps = a.k / (a.quant == 1 ? 64 : a.quant == 2 ? 128 : a.dtype == 0 ? 16 : 32);
     const int cols = a.quant ? 16 : skinny_cols(a.n);
     SkinnyPlan p = skinny_plan(a.dtype, a.m, steps, a.n, dual, a.quant != 0);

@@ -1319,6 +1319,13 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
                     void* xn = cx.ws + (shared ? st.norm_off : st.scratch_off);
                     if (shared && &plan.steps[st.norm_first] != &st) {
                         oi += in.norm_ln ? 2 : 1;   // the first of the layers has left the rows there
+                    } else if (in.norm_ln && !shared && !in.x_f32 && k::skinny_norm_fits(sa, src_ptr(st, cx, oi), src_ptr(st, cx, oi + 1))) {
+                        sa.gamma = (const float*)src_ptr(st, cx, oi);
+                        sa.beta = (const float*)src_ptr(st, cx, oi + 1);
+                        sa.inv_n = in.scale;
+                        sa.eps = in.eps;
+                        xn = const_cast<void*>(sa.x);
+                        oi += 2;
                     } else if (in.norm_ln) {
                         if (in.x_f32) k::layer_norm_f32_to_bf16(s, sa.x, src_ptr(st, cx, oi), src_ptr(st, cx, oi + 1), xn, sa.m, sa.k, in.scale, in.eps);
                         else k::layer_norm(s, (int)ldt, sa.x, src_ptr(st, cx, oi), src_ptr(st, cx, oi + 1), xn, sa.m, sa.k, in.scale, in.eps);

@@ -143,6 +143,15 @@ def test_f32(hip, case):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("case", [(1, 7, 12, 12, 64, False, 16, 0), (3, 16, 4, 2, 64, False, 20, 3), (2, 15, 4, 1, 128, False, 15, 0), (16, 2, 2, 2, 128, False, 9, -1),
+                                  (1, 16, 8, 8, 128, False, 16, 5), (1, 17, 12, 12, 64, False, 17, 0), (2, 16, 8, 2, 64, True, 16, 0)])
+def test_f32_of_few_rows(hip, case):
+    """Up to 16 rows without rotation a wave takes each row by itself; one row more, and rotated rows, go another way."""
+    B, T, hq, hkv, dh, rot, cap, first = case
+    check_program(hip, program("F32", B, T, hq, hkv, dh, rot, cap), inputs(B, T, hq, hkv, dh, rot, cap, first, 11), what=str(case))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("donate", [False, True])
 @pytest.mark.parametrize("case", CASES[:-1])
 def test_bf16(hip, case, donate):

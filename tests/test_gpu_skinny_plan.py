@@ -45,6 +45,26 @@ def test_plain_and_pair(hip, dtype, m, k, n):
     assert (np.abs(got[1] - g * t) <= 1.1 * bs * np.abs(t) + bt * np.abs(g) + (2.0 ** -7 if dtype == "Bf16" else 2.0 ** -20) * np.abs(g * t) + 1.1 * bs * bt + 1e-6).all()
 
 
+@pytest.mark.parametrize("m,k,n", [(2, 16, 16), (7, 768, 2304), (16, 1008, 700), (9, 240, 3073), (16, 256, 4096), (3, 1008, 50), (16, 1024, 40), (5, 768, 4112)])
+def test_f32_layer_norm_inside(hip, m, k, n):
+    """LayerNorm, layer, bias and GELU in one launch (up to 1008 values and a tile for each CU), at the edges of that rule, against float64.  A normed value is off by
+    the rounding of its mean, its difference from it and two products: 8 units of 1 + |value|; a sum as in `bounds`."""
+    rng = np.random.default_rng(m + k + n)
+    x = rng.standard_normal((m, k), dtype=np.float32) * 2 + 1
+    g, b = rng.standard_normal(k, dtype=np.float32) * 0.1 + 1, rng.standard_normal(k, dtype=np.float32)
+    w, bias = rng.standard_normal((k, n), dtype=np.float32) * np.float32(k ** -0.5), rng.standard_normal(n, dtype=np.float32)
+    args = [("F32", list(a.shape)) for a in (x, g, b, w, bias)]
+    p = program(args, lambda a, gg, bb, ww, c: [F.linear(F.layer_norm(a, gg, bb, 1e-5)[0], ww, c)])
+    got = hip_run(hip, p, [x, g, b, w, bias])[0]
+    x64 = x.astype(np.float64)
+    c = x64 - x64.mean(1, keepdims=True)
+    z = c / np.sqrt((c * c).mean(1, keepdims=True) + 1e-5)
+    xn = z * g + b
+    s, bound = bounds(xn, w, "F32")
+    off = 8 * 2.0 ** -24 * (((1 + np.abs(z)) * np.abs(g) + np.abs(b)) @ np.abs(w).astype(np.float64))
+    assert (np.abs(got - (s + bias)) <= bound + off + 2.0 ** -23 * np.abs(bias)).all()
+
+
 # f32 sums over tiles of 16 columns are those of 16 waves whatever the waves: rows by themselves (16 waves of two requests, 8 of four) and among 12 (8 of one, 16 of one)
 @pytest.mark.parametrize("k,n", [(1040, 8190), (1040, 12304), (2064, 8192)])
 def test_f32_sums_do_not_depend_on_the_waves(hip, k, n):
