@@ -264,7 +264,9 @@ __device__ __forceinline__ float half_sum(float x) {
 // bf16 decode attention with the scores on the matrix cores.  grid (n_kv, nsplit, batch), 256 threads; wave w of a
 // workgroup takes the 32-key tiles w, w+4, ... of the workgroup's share, the rows of its next tile in flight while it works on one.
 // Bound by the caches' rows; 8 sequences of 1000 positions of 8 kv heads of 128 (33 MB), capacity 2048: 18.1 -> 14.5 us since the
-// attended tiles, not the capacity, are shared out and all workgroups are resident at once.  Per tile
+// attended tiles, not the capacity, are shared out and all workgroups are resident at once; with the merge of the records behind it 18.9 -> 16.8 us (2 x 3000 18.8 -> 17.1, 8 x 30
+// 9.3 -> 8.4) with fused multiply-adds, four weights to an LDS read and exchanges that halve the values.  The merge by the workgroup that draws a kv head's last ticket instead of
+// a launch: 19.5, 33.1 and 9.7.  Per tile
 //   S^T[key, q] = K[key, :] . Q[q, :]   v_mfma_f32_32x32x16_bf16, A = cache rows, read whole and turned in LDS (lane = key row),
 //                                       B = the group's G query heads in columns 0..G-1 (other columns repeat them)
 // so a lane owns ONE query: its 16 scores, the running maximum and sum (log2 domain) are per-lane values and the
@@ -273,6 +275,13 @@ __device__ __forceinline__ float half_sum(float x) {
 // lanes, 16 bytes of a V row each) accumulates O[g, :] over its keys of the tile.  States are merged across
 // lane-groups by shuffles, across waves through LDS, across splits by attn_decode_combine_kernel (same records as
 // attn_decode_kernel, maxima in natural-log units).
+// Two values of every lane, lane ^ OFF exchanged: the lanes below keep a, those above b, each added up over the pair.
+template <int OFF> __device__ __forceinline__ float lane_halves(float a, float b) {
+    static_assert(OFF == 16 || OFF == 32, "swaps that the hardware has");
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                             : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
 template <int DH, int G>
 __global__ __launch_bounds__(256, DH * G == 1024 ? 1 : 2) void attn_decode_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ kc,
                                                                bf16_t* __restrict__ vc, const int32_t* __restrict__ us,
@@ -436,15 +445,22 @@ __global__ __launch_bounds__(256, DH * G == 1024 ? 1 : 2) void attn_decode_mfma_
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[g][e] *= c;
         }
+        float pr[G][NV];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int j = 0; j < NV; j += 4) {
+                const float4 p4 = *reinterpret_cast<const float4*>(&p_lds[wave][g][NV * sub + j]);
+                pr[g][j] = p4.x; pr[g][j + 1] = p4.y; pr[g][j + 2] = p4.z; pr[g][j + 3] = p4.w;
+            }
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const float vf[8] = {bf16lo(vreg[j][0]), bf16hi(vreg[j][0]), bf16lo(vreg[j][1]), bf16hi(vreg[j][1]),
                                  bf16lo(vreg[j][2]), bf16hi(vreg[j][2]), bf16lo(vreg[j][3]), bf16hi(vreg[j][3])};
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const float pj = p_lds[wave][g][NV * sub + j];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o[g][e] += pj * vf[e];
+                for (int e = 0; e < 8; ++e) o[g][e] = __builtin_fmaf(pr[g][j], vf[e], o[g][e]);
             }
         }
         if (t + 4 < ntiles) load_v(k0 + 128);
@@ -452,18 +468,27 @@ __global__ __launch_bounds__(256, DH * G == 1024 ? 1 : 2) void attn_decode_mfma_
         __builtin_amdgcn_wave_barrier();
     }
 
-    // merge the lane-groups of this wave (they share the wave's maximum), then the four waves through LDS
+    // merge the lane-groups of this wave (they share the wave's maximum), then the four waves through LDS.  The lanes exchanged with go on with half of the values
+    // each time (o[g][e] in a row: bits 5, 4 and 3 of the lane say which), so 32 values take 24 exchanges, not 64
+    float w0[G * 8], w1[G * 4], w2[G * 2];
 #pragma unroll
-    for (int off = LPR; off < 64; off <<= 1)
+    for (int i = 0; i < G * 8; ++i) w0[i] = o[i >> 3][i & 7];
 #pragma unroll
-        for (int g = 0; g < G; ++g)
+    for (int i = 0; i < G * 4; ++i) w1[i] = lane_halves<32>(w0[i], w0[i + G * 4]);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[g][e] += __shfl_xor(o[g][e], off, 64);
-    if (sub == 0) {
+    for (int i = 0; i < G * 2; ++i) w2[i] = lane_halves<16>(w1[i], w1[i + G * 2]);
+    const int first_value = (lane >> 5) * (G * 4) + ((lane >> 4) & 1) * (G * 2);
+    if constexpr (NSUB == 4) {
 #pragma unroll
-        for (int g = 0; g < G; ++g)
+        for (int i = 0; i < G * 2; ++i) so[wave][(first_value + i) >> 3][li * 8 + ((first_value + i) & 7)] = w2[i];
+    } else {
+        const bool up = lane & 8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) so[wave][g][li * 8 + e] = o[g][e];
+        for (int i = 0; i < G; ++i) {
+            const float keep = up ? w2[i + G] : w2[i], give = up ? w2[i] : w2[i + G];
+            const int at = first_value + (up ? G : 0) + i;
+            so[wave][at >> 3][li * 8 + (at & 7)] = keep + dpp_move<0x128>(give);   // row_ror:8
+        }
     }
     if (lane < G) { sm[wave][lane] = m_run; sl[wave][lane] = l_run; }
     __syncthreads();
