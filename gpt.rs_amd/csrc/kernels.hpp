@@ -24,8 +24,21 @@ struct CopyDesc {
     int dyn_rank = 0;
     int64_t dyn_max[kMaxRank] = {};
     int64_t dyn_stride[kMaxRank] = {};
+    bool operator==(const CopyDesc& o) const {
+        bool same = rank == o.rank && dyn == o.dyn && total == o.total && dst_off == o.dst_off && src_off == o.src_off && dyn_rank == o.dyn_rank;
+        for (int i = 0; i < kMaxRank; ++i)
+            same = same && dims[i] == o.dims[i] && dst_stride[i] == o.dst_stride[i] && src_stride[i] == o.src_stride[i] && dyn_max[i] == o.dyn_max[i] && dyn_stride[i] == o.dyn_stride[i];
+        return same;
+    }
 };
 void copy_strided(hipStream_t s, void* dst, const void* src, int elem_size, const CopyDesc& d, const int32_t* starts);
+// the same copy between up to kMost pairs of tensors in one launch
+struct CopyPairs {
+    static constexpr int kMost = 64;
+    void* dst[kMost];
+    const void* src[kMost];
+};
+void copy_strided_pairs(hipStream_t s, const CopyPairs& pairs, int count, int elem_size, const CopyDesc& d, const int32_t* starts);
 
 // Up to 256 payload bytes travel as kernel arguments: an upload with no staging buffer and
 // no host synchronisation (token ids, positions, update_starts, RoPE rows).

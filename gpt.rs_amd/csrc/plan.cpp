@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cstring>
 #include <functional>
+#include <set>
 
 #include "runtime.hpp"
 
@@ -855,6 +856,24 @@ void Builder::build() {
     }
     plan.workspace_bytes = high;
 
+    // runs of equal copies
+    for (int s = 0; s < n_steps;) {
+        const Step& first = plan.steps[s];
+        int e = s + 1;
+        auto copies = [&](const Step& st) { return st.in.op == OpKind::DynamicUpdateSlice && st.copies.size() == 1 && !st.left_out; };
+        if (copies(first)) {
+            std::set<int> written(first.dst.begin(), first.dst.end());
+            for (; e < n_steps; ++e) {
+                const Step& st = plan.steps[e];
+                if (!copies(st) || !(st.copies[0] == first.copies[0]) || st.elem_size != first.elem_size || st.src[2] != first.src[2] || st.src_const[2] != first.src_const[2]) break;
+                if (written.count(st.src[0]) || written.count(st.src[1]) || written.count(st.src[2])) break;
+                written.insert(st.dst.begin(), st.dst.end());
+            }
+            plan.steps[s].copy_run = e - s;
+        }
+        s = e;
+    }
+
     // runs of consecutive decode linears / decode attentions -> one persistent launch each
     auto chain_phases = [&](const Step& st) -> int {   // phases the step takes in a chain, 0: not chainable
         const Instr& in = st.in;
@@ -1104,7 +1123,24 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
             ++cx.launches;
             break;
         case OpKind::DynamicUpdateSlice: {
+            if (st.copy_run == 0 && &st < cx.copied_end) break;
+            cx.copied_end = nullptr;
             const void* base = src_ptr(st, cx, 0);
+            if (st.copy_run > 1) {
+                bool in_place = true;
+                for (int i = 0; i < st.copy_run; ++i) in_place = in_place && cx.ptr[(&st)[i].dst[0]] == src_ptr((&st)[i], cx, 0);
+                if (in_place) {
+                    for (int i0 = 0; i0 < st.copy_run; i0 += k::CopyPairs::kMost) {
+                        const int n = std::min(st.copy_run - i0, k::CopyPairs::kMost);
+                        k::CopyPairs pairs{};
+                        for (int i = 0; i < n; ++i) { pairs.dst[i] = cx.ptr[(&st)[i0 + i].dst[0]]; pairs.src[i] = src_ptr((&st)[i0 + i], cx, 1); }
+                        k::copy_strided_pairs(s, pairs, n, st.elem_size, st.copies[0], (const int32_t*)src_ptr(st, cx, 2));
+                        ++cx.launches;
+                    }
+                    cx.copied_end = &st + st.copy_run;
+                    break;
+                }
+            }
             if (dst != base && out.bytes()) {
                 GPTRS_HIP_CHECK(hipMemcpyAsync(dst, base, out.bytes(), hipMemcpyDeviceToDevice, s));
                 ++cx.launches;

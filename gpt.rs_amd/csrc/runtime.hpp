@@ -130,6 +130,9 @@ struct Step {
     // Sum of two gathers of program inputs: the gathers' steps are left out and this step reads the tables itself.
     int take_a = -1, take_b = -1;
     bool left_out = false;
+    // DynamicUpdateSlices behind one another that copy the same way between tensors of their own: the first of them has their number, and one launch does them
+    // all where each updates its base in place; 0: a step behind the first (or no such step).
+    int copy_run = 0;
     k::CopyDesc pack_l{}, pack_r{};
     size_t pack_l_off = 0, pack_r_off = 0;
 };
@@ -374,6 +377,7 @@ struct ExecCtx {
     bool chain = false;               // run decode linears as persistent chain launches
     std::vector<BufferP> input_bufs;  // per input position
     const Step* done_ahead = nullptr; // a step whose work the step before it has done
+    const Step* copied_end = nullptr; // the steps before this one whose copies an earlier step's launch has made
 };
 void run_step(const Plan& plan, const Step& st, ExecCtx& cx);
 

@@ -33,6 +33,9 @@ def decode_cache_capacity(required_len: int, max_len: int) -> int:
     return min(bucket, max_len)
 
 
+GROW_SLOTS = 32   # layers' caches that one program copies into larger ones
+
+
 @dataclass
 class DecodeKvCache:
     """ops/functional/attention.rs:100-126: fixed-capacity [Hkv, capacity, Dh] + active len."""
@@ -280,6 +283,21 @@ class _ModelBase:
             self._programs[key] = (Program(fb), {})
         return self.backend.run_program(self._programs[key][0], [self._zeros([heads, capacity, width]), handle, self._upload_i32([0, 0, 0])],
                                         [True, False, False])[0]
+
+    def _grow_many(self, handles: list, dims, capacity: int) -> list:
+        """`_grow_rows` of several tensors of one shape in one program."""
+        heads, old_cap, width = dims
+        n = len(handles)
+        key = ("grow", n, heads, old_cap, width, capacity)
+        if key not in self._programs:
+            fb = FunctionBuilder("main", self.dtype)
+            bases = [fb.param(self.dtype, [heads, capacity, width]) for _ in range(n)]
+            olds = [fb.param(self.dtype, [heads, old_cap, width]) for _ in range(n)]
+            st = fb.param("Si32", [3])
+            fb.set_results([F.dynamic_update_slice_into(base, old, st) for base, old in zip(bases, olds)])
+            self._programs[key] = (Program(fb), {})
+        return self.backend.run_program(self._programs[key][0], [*self._zeros_many([heads, capacity, width], n), *handles, self._upload_i32([0, 0, 0])],
+                                        [True] * n + [False] * (n + 1))
 
     def _run(self, program: Program, args: list, donate: Optional[list] = None):
         if self.front_end:
@@ -594,9 +612,12 @@ class Gpt(_ModelBase):
     def _grow_caches(self, caches, capacity: int):
         """model/gpt.rs:626-657: copy each layer's cache into a larger zero buffer."""
         dims = (self.attn.num_key_value_heads, caches[0][0].capacity, self.attn.kv_head_dim)
-        for c in caches:
-            for i, slot in enumerate(c):
-                c[i] = DecodeKvCache(self._grow_rows(slot.keys, dims, capacity), self._grow_rows(slot.values, dims, capacity), slot.len, capacity)
+        slots = [(c, i) for c in caches for i in range(len(c))]
+        for lo in range(0, len(slots), GROW_SLOTS):      # what a program has copied is dropped before the next is run
+            part = slots[lo:lo + GROW_SLOTS]
+            grown = iter(self._grow_many([h for c, i in part for h in (c[i].keys, c[i].values)], dims, capacity))
+            for c, i in part:
+                c[i] = DecodeKvCache(next(grown), next(grown), c[i].len, capacity)
 
 
 # ================================================================================ Ministral

@@ -25,6 +25,27 @@ def prog(build, param_specs):
     return Program(fb)
 
 
+@pytest.mark.parametrize("n,donated", [(2, 2), (5, 0), (5, 3), (64, 64), (70, 70)])
+def test_equal_updates_behind_one_another(hip, n, donated):
+    """Updates that copy the same way are one launch where all of them write in place, and one each where a base is kept; one that updates
+    what another of them has written, and one at another place, are not among them.  Twice and three times the same program: a recorded launch as well."""
+    base, upd = [2, 9, 4], [2, 5, 4]
+
+    def build(fb, *a):
+        st, st2, bases, upds = a[0], a[1], a[2:2 + n], a[2 + n:]
+        out = [F.dynamic_update_slice_into(b, u, st) for b, u in zip(bases, upds)]
+        again = F.dynamic_update_slice_into(out[0], upds[1], st2)
+        return [*out[1:], again]
+
+    p = prog(build, [("Si32", [3])] * 2 + [("F32", base)] * n + [("F32", upd)] * n)
+    args = [np.array([0, 3, 0], np.int32), np.array([0, 1, 0], np.int32)]
+    args += [rng_uniform(900 + i, base) for i in range(n)] + [rng_uniform(990 + i, upd) for i in range(n)]
+    want = oracle_run(p, args)
+    for _ in range(3):
+        got = hip_run(hip, p, args, [False, False] + [i < donated for i in range(n)] + [False] * n)
+        assert all(np.array_equal(g, w) for g, w in zip(got, want))
+
+
 # ------------------------------------------------------------------ reference-held vectors
 def test_smoke_matmul_golden(hip):
     # crates/gpt-rs-backend-tests/src/smoke.rs:12-24
