@@ -303,11 +303,16 @@ size_t chain_attn_part_bytes(int64_t n_q, int64_t n_kv, int64_t head_dim);
 int chain_attn_phases(int64_t capacity);
 void chain_fill_attn(ChainPhase& partial, ChainPhase& combine, int64_t n_q, int64_t n_kv, int64_t head_dim, int64_t capacity,
                      int64_t rot_half, float scale);
+// The same for one sequence of the chunked design: x is the f32 projection [(n_q + n_kv) dim + n_kv dim + n_q gates], `cos` the f32 row of angles [rot / 2 cosines, rot / 2 sines], `query_start`
+// the position; of `combine`, `gamma` the sinks [n_q] and `bias` the gates.
+bool chain_chunk_attn_supported(int64_t n_q, int64_t n_kv, int64_t dim, int64_t vdim, int64_t rot);
+void chain_fill_chunk_attn(ChainPhase& partial, ChainPhase& combine, int64_t n_q, int64_t n_kv, int64_t dim, int64_t capacity, int64_t rot, int64_t chunk, float scale, float eps);
 // bar: kChainBarrierBytes of device memory zeroed once; abort_flag: raised when a barrier wait
 // gives up (every wave then leaves the kernel).  false: launch not possible (caller falls back).
 // stall_phase >= 0 (tests of the give-up path): every workgroup expects one arrival too many at that phase's barrier.
 bool chain_launch(hipStream_t s, const ChainPhase* dev_table, int nphases, int lds_bytes, unsigned* bar, int* abort_flag,
-                  int wfmt = kChainW16, int stall_phase = -1);   // wfmt: the weight format of EVERY linear phase of the table
+                  int wfmt = kChainW16, int stall_phase = -1,   // wfmt: the weight format of EVERY linear phase of the table
+                  bool chunk_rows = false);                     // the attention phases are those of chain_fill_chunk_attn (bf16 weights)
 
 // Prefill GEMM (M > 16, bf16) on the matrix cores over a k-grouped copy of the weights,
 // Wk8[K/8][Npad][8] (kernels_mfma.hip).  wk2 != nullptr: SwiGLU pair.

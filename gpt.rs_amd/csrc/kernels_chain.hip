@@ -711,10 +711,17 @@ __device__ __forceinline__ void merge_waves(const GPTRS_LDS float* sm, const GPT
 // the waves of different heads re-read the same rows out of the caches.  Cache rows older than this launch, and the
 // RoPE rows, are requested BEFORE the grid barrier is awaited (they do not depend on the previous phase); only the query
 // row and this step's K/V row are read after it.
-template <bool F32>
+//
+// Rows of the chunked design (ROWS == kRowsChunk): the projection's row is f32, queries and the new key are turned pair by pair (f32 angles), brought to unit
+// mean square over the head and rounded to bf16 once, a value is rounded once; the caches hold the current chunk.
+enum : int { kRowsBf16 = 0, kRowsF32 = 1, kRowsChunk = 2 };
+template <int ROWS>
 __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int unit, int phase,
                              unsigned long long budget) {
-    typedef typename std::conditional<F32, float, bf16_t>::type E;
+    constexpr bool F32 = ROWS == kRowsF32, CHUNK = ROWS == kRowsChunk;
+    typedef typename std::conditional<F32, float, bf16_t>::type E;       // of the caches
+    typedef typename std::conditional<ROWS == kRowsBf16, bf16_t, float>::type X;   // of the projection's row
+    constexpr int XW = ROWS == kRowsBf16 ? 1 : 2;                         // 16-byte words of a lane's 8 values there
     constexpr int PP = F32 ? 2 : 5;   // rows of a lane in one step; the first step's are requested ahead of the barrier (32 chunks x 8 lane groups x 5 = 1280 positions)
     constexpr int RW = F32 ? 2 : 1;   // 16-byte words of a lane's 8 values
     const int t = local_tid(), lane = t & 63, wave = uni(t >> 6);
@@ -724,11 +731,13 @@ __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
     const int g = wave & (G - 1), part = wave / G;
     const int stride = nparts * (64 >> lsh), sid = part * (64 >> lsh) + sub;   // position slots of this head's waves
     const int kvh = unit / nch, c = unit - kvh * nch;
-    const E* qkv = (const E*)P.x;
+    const X* qkv = (const X*)P.x;
     E* kc = (E*)P.k_cache + (long)kvh * cap * dh;
     E* vc = (E*)P.v_cache + (long)kvh * cap * dh;
-    const bool rotate = !F32 && P.cos != nullptr;
-    const int qpos = clampi(uni(gload(P.query_start)), 0, cap - 1);       // DynamicSlice clamp (cpu.rs:804-820)
+    const bool rotate = ROWS == kRowsBf16 && P.cos != nullptr;
+    int qpos = uni(gload(P.query_start));
+    if (CHUNK) qpos = max(qpos, 0) % P.N;                                 // (N: positions of a chunk)
+    qpos = clampi(qpos, 0, cap - 1);                                      // DynamicSlice clamp (cpu.rs:804-820)
     const int upd = clampi(uni(gload(P.update_starts + 1)), 0, cap - 1);  // DynamicUpdateSlice clamp
     const float scale = P.scale;
     const int L = qpos + 1, CL = (L + nch - 1) / nch;
@@ -751,10 +760,10 @@ __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
         for (int v = 0; v < 8; ++v) f[v] = F32 ? __uint_as_float(w[v]) : ((v & 1) ? bf16hi(w[v >> 1]) : bf16lo(w[v >> 1]));
     };
     // a row that the phase before has written: agent-scope loads
-    auto request_new = [&](const E* p, u32x4 (&raw)[RW]) {
+    auto request_new = [&](const X* p, u32x4 (&raw)[XW]) {
 #pragma unroll
-        for (int r = 0; r < RW; ++r) {
-            const unsigned long long a = cload8(p + (F32 ? 4 : 8) * r), b = cload8(p + (F32 ? 4 : 8) * r + (F32 ? 2 : 4));
+        for (int r = 0; r < XW; ++r) {
+            const unsigned long long a = cload8(p + (XW == 2 ? 4 : 8) * r), b = cload8(p + (XW == 2 ? 4 : 8) * r + (XW == 2 ? 2 : 4));
             raw[r].x = (unsigned)a; raw[r].y = (unsigned)(a >> 32); raw[r].z = (unsigned)b; raw[r].w = (unsigned)(b >> 32);
         }
     };
@@ -762,6 +771,11 @@ __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
     request_rows(vraw, vc, p0);
     const bool rot = rotate && c0 < 2 * half, first = c0 < half;
     u32x4 cosr[1], sinr[1];
+    const bool turn = CHUNK && c0 < 2 * half;
+    if (turn) {   // the angles of a lane's four pairs: [rot / 2] cosines, as many sines
+        cosr[0] = *(const GPTRS_GLOBAL u32x4*)((const float*)P.cos + (c0 >> 1));
+        sinr[0] = *(const GPTRS_GLOBAL u32x4*)((const float*)P.cos + half + (c0 >> 1));
+    }
     if (rot) {
         const int j0 = first ? c0 : c0 - half;
         cosr[0] = *(const GPTRS_GLOBAL u32x4*)((const bf16_t*)P.cos + j0);
@@ -772,11 +786,11 @@ __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
     // The wave's query head and, in the first position subset of the workgroup that owns position `upd`, this step's K and V rows
     // (for the first lane group), all requested before any is consumed; RoPE on the fly.
     const bool new_row = owner && part == 0;
-    u32x4 qa[RW], qb[RW], ka[RW], kb[RW], va[RW];
+    u32x4 qa[XW], qb[XW], ka[XW], kb[XW], va[XW];
     {
         const int co = first ? c0 + half : c0 - half;
-        const E* head = qkv + (long)(kvh * G + g) * dh;
-        const E* knew = qkv + (long)(n_q + kvh) * dh;
+        const X* head = qkv + (long)(kvh * G + g) * dh;
+        const X* knew = qkv + (long)(n_q + kvh) * dh;
         request_new(head + c0, qa);
         if (rot) request_new(head + co, qb);
         if (new_row) {
@@ -785,14 +799,33 @@ __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
             request_new(knew + (long)n_kv * dh + c0, va);
         }
     }
-    auto rope = [&](const u32x4 (&own_raw)[RW], const u32x4 (&other_raw)[RW], float (&out)[8]) {
-        row_values(own_raw, out);
-        if constexpr (!F32) {
+    auto new_values = [&](const u32x4 (&raw)[XW], float (&f)[8]) {
+        const unsigned w[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[XW - 1].x, raw[XW - 1].y, raw[XW - 1].z, raw[XW - 1].w};
+#pragma unroll
+        for (int v = 0; v < 8; ++v) f[v] = XW == 2 ? __uint_as_float(w[v]) : ((v & 1) ? bf16hi(w[v >> 1]) : bf16lo(w[v >> 1]));
+    };
+    auto rope = [&](const u32x4 (&own_raw)[XW], const u32x4 (&other_raw)[XW], float (&out)[8]) {
+        new_values(own_raw, out);
+        if constexpr (CHUNK) {
+            const unsigned cw[4] = {cosr[0].x, cosr[0].y, cosr[0].z, cosr[0].w}, sw[4] = {sinr[0].x, sinr[0].y, sinr[0].z, sinr[0].w};
+            float q[1] = {0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float a = out[2 * i], b = out[2 * i + 1], cv = __uint_as_float(cw[i]), sv = __uint_as_float(sw[i]);
+                if (turn) { out[2 * i] = a * cv - b * sv; out[2 * i + 1] = b * cv + a * sv; }
+                q[0] += out[2 * i] * out[2 * i] + out[2 * i + 1] * out[2 * i + 1];
+            }
+            group_sums(q, lpr);
+            const float inv = 1.0f / sqrtf(q[0] / (float)dh + P.eps);
+#pragma unroll
+            for (int v = 0; v < 8; ++v) out[v] = rbf(out[v] * inv);
+        }
+        if constexpr (ROWS == kRowsBf16) {
             if (rot) {
                 float other[8], cosv[8], sinv[8];
-                row_values(other_raw, other);
-                row_values(cosr, cosv);
-                row_values(sinr, sinv);
+                new_values(other_raw, other);
+                new_values(cosr, cosv);
+                new_values(sinr, sinv);
 #pragma unroll
                 for (int v = 0; v < 8; ++v) out[v] = rbf(first ? out[v] * cosv[v] - other[v] * sinv[v] : out[v] * cosv[v] + other[v] * sinv[v]);
             }
@@ -811,7 +844,11 @@ __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
     if (new_row) {   // this step's row: attended to when in range, appended once (by head 0's wave)
         float kf[8], vf[8], s[1];
         rope(ka, kb, kf);
-        row_values(va, vf);
+        new_values(va, vf);
+        if (CHUNK) {
+#pragma unroll
+            for (int v = 0; v < 8; ++v) vf[v] = rbf(vf[v]);
+        }
         if (sub == 0 && g == 0) {
             E* kd = kc + (long)upd * dh + c0;
             E* vd = vc + (long)upd * dh + c0;
@@ -822,7 +859,9 @@ __device__ bool attn_partial(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
                 u32x4 kw;
                 kw.x = pack_bf16x2(kf[0], kf[1]); kw.y = pack_bf16x2(kf[2], kf[3]); kw.z = pack_bf16x2(kf[4], kf[5]); kw.w = pack_bf16x2(kf[6], kf[7]);
                 *(GPTRS_GLOBAL u32x4*)kd = kw;
-                *(GPTRS_GLOBAL u32x4*)vd = va[0];
+                u32x4 vw = va[0];
+                if constexpr (CHUNK) { vw.x = pack_hw(vf[0], vf[1]); vw.y = pack_hw(vf[2], vf[3]); vw.z = pack_hw(vf[4], vf[5]); vw.w = pack_hw(vf[6], vf[7]); }
+                *(GPTRS_GLOBAL u32x4*)vd = vw;
             }
         }
         s[0] = score(kf);
@@ -961,13 +1000,18 @@ __device__ __forceinline__ void merge_chunks(const float* base, int wave, int nc
         o1 += __uint_as_float((unsigned)(ov[u] >> 32)) * c;
     }
 }
-template <bool F32>
+template <int ROWS>
 __device__ bool attn_combine(GPTRS_LDS int* go, GPTRS_LDS int* abort, const ChainPhase& P, GPTRS_LDS float* lds, int hq, int phase,
                              unsigned long long budget) {
     const int t = local_tid(), wave = uni(t >> 6), lane = t & 63;
+    constexpr bool F32 = ROWS == kRowsF32;
     const int dh = P.head_dim, nch = P.nch, h2 = dh / 2;   // nch <= 64
     const float* base = P.part + (long)hq * nch * (dh + 2);
+    float sink = 0.f;   // chunked rows: one more term of the head's denominator, and a gate over the head (a value of the projection's row)
+    if (ROWS == kRowsChunk) sink = gload((const float*)P.gamma + hq);
     if (!wait_go(go, abort, phase, budget)) return false;
+    float gate = 0.f;
+    if (ROWS == kRowsChunk) gate = __uint_as_float(cload4((const float*)P.bias + hq));
     for (int d0 = 0; d0 < h2; d0 += 64) {
         const int d2 = d0 + lane;
         const bool act = d2 < h2;
@@ -984,6 +1028,7 @@ __device__ bool attn_combine(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
             float M = v[0].x;
 #pragma unroll
             for (int w = 1; w < NWS; ++w) M = fmaxf(M, v[w].x);
+            if (ROWS == kRowsChunk) M = fmaxf(M, sink);
             const float ref = finite_max(M);
             float Lt = 0.f, a0 = 0.f, a1 = 0.f;
 #pragma unroll
@@ -991,6 +1036,7 @@ __device__ bool attn_combine(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
                 const float cw = fast_exp(v[w].x - ref);
                 Lt += v[w].y * cw; a0 += v[w].z * cw; a1 += v[w].w * cw;
             }
+            if (ROWS == kRowsChunk) { Lt += fast_exp(sink - ref); Lt *= 1.0f + expf(-gate); }   // (times the gate's sigmoid)
             if (F32) cstore8((float*)P.y + (long)hq * dh + 2 * d2, (unsigned long long)__float_as_uint(a0 / Lt) | ((unsigned long long)__float_as_uint(a1 / Lt) << 32));
             else cstore4((bf16_t*)P.y + (long)hq * dh + 2 * d2, pack_bf16x2(a0 / Lt, a1 / Lt));
         }
@@ -1006,7 +1052,7 @@ __device__ bool attn_combine(GPTRS_LDS int* go, GPTRS_LDS int* abort, const Chai
 // request the cache rows it needs, before the control wave has seen the barrier.
 // The control wave only takes part in the workgroup barriers (attn_barriers of them to a unit).
 __device__ __forceinline__ int attn_barriers(int kind, int head_dim) { return kind == kChainAttnCombine && head_dim > 128 ? 4 : 2; }
-template <bool F32>
+template <int ROWS>
 __device__ __forceinline__ bool run_attn_phase(const GPTRS_CONST ChainPhase* php, GPTRS_LDS float* lds, GPTRS_LDS int* go, GPTRS_LDS int* abort, int phase,
                                                unsigned long long budget) {
     ChainPhase P;
@@ -1018,7 +1064,7 @@ __device__ __forceinline__ bool run_attn_phase(const GPTRS_CONST ChainPhase* php
     }
     const int kind = P.kind, units = P.units;
     for (int u = blockIdx.x; u < units; u += gridDim.x) {
-        const bool ok = kind == kChainAttnCombine ? attn_combine<F32>(go, abort, P, lds, u, phase, budget) : attn_partial<F32>(go, abort, P, lds, u, phase, budget);
+        const bool ok = kind == kChainAttnCombine ? attn_combine<ROWS>(go, abort, P, lds, u, phase, budget) : attn_partial<ROWS>(go, abort, P, lds, u, phase, budget);
         if (!ok) return false;
     }
     return true;
@@ -1315,7 +1361,7 @@ template <int FMT> struct Act { typedef unsigned type; };
 template <> struct Act<kChainW8> { typedef u32x2 type; };
 template <> struct Act<kChainW4> { typedef u32x4 type; };
 
-template <int FMT, int RING_D>
+template <int FMT, int RING_D, int ROWS>
 __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, int nphases, const unsigned char* ring, unsigned long long budget) {
     const int t = threadIdx.x, lane = t & 63, wave = uni(t >> 6);
     const int blk = blockIdx.x;
@@ -1390,7 +1436,7 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
             const GPTRS_CONST ChainPhase* D = table + c_phase;   // the fields that decide this workgroup's part, before the wait
             if (uni(D->kind) != kChainLinear) {
                 if (blk >= uni(D->units)) continue;
-                if (!run_attn_phase<FMT == kChainW32>(table + c_phase, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.go, (GPTRS_LDS int*)&sh.abort, c_phase,
+                if (!run_attn_phase<ROWS>(table + c_phase, (GPTRS_LDS float*)xs, (GPTRS_LDS int*)&sh.go, (GPTRS_LDS int*)&sh.abort, c_phase,
                                     budget)) return false;
                 continue;
             }
@@ -1593,7 +1639,8 @@ __device__ void compute_waves(Shared& sh, const unsigned* xs, PhaseTable table, 
     }
 }
 
-template <int FMT, int RING_D>
+// ROWS: what the launch's attention phases read
+template <int FMT, int RING_D, int ROWS = FMT == kChainW32 ? kRowsF32 : kRowsBf16>
 __global__ __launch_bounds__(NT, 1) void chain_kernel(const ChainPhase* __restrict__ phases, int nphases, unsigned* bar, int* abort_flag,
                                                         int xs_bytes, unsigned long long budget, int stall_phase) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1607,7 +1654,7 @@ __global__ __launch_bounds__(NT, 1) void chain_kernel(const ChainPhase* __restri
     }
     const int wave = threadIdx.x >> 6;
     if (wave < NWS) {
-        compute_waves<FMT, RING_D>(sh, xs, table, nphases, ring, budget);
+        compute_waves<FMT, RING_D, ROWS>(sh, xs, table, nphases, ring, budget);
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): no load may land in LDS after the workgroup has gone
     } else {
         if constexpr (FMT == kChainW16) {
@@ -1723,7 +1770,7 @@ __global__ void chain_unpack_kernel(const uint32_t* __restrict__ packed, bf16_t*
 }
 
 static int g_grid = 0;
-static int g_occupancy_ok[8] = {-1, -1, -1, -1, -1, -1, -1, -1};   // per kernel: does a workgroup fit a CU with the LDS it asks for
+static int g_occupancy_ok[10] = {-1, -1, -1, -1, -1, -1, -1, -1, -1, -1};   // per kernel: does a workgroup fit a CU with the LDS it asks for
 
 }  // namespace
 
@@ -1883,22 +1930,35 @@ void chain_fill_attn(ChainPhase& partial, ChainPhase& combine, int64_t n_q, int6
     combine.lds_bytes = combine.lds_total = (int)(NWS * 64 * sizeof(float4));
 }
 
+bool chain_chunk_attn_supported(int64_t n_q, int64_t n_kv, int64_t dim, int64_t vdim, int64_t rot) {
+    return dim == vdim && rot % 8 == 0 && rot <= dim && chain_attn_supported(2, 1, n_q, n_kv, dim, 0);
+}
+void chain_fill_chunk_attn(ChainPhase& partial, ChainPhase& combine, int64_t n_q, int64_t n_kv, int64_t dim, int64_t capacity, int64_t rot, int64_t chunk, float scale, float eps) {
+    chain_fill_attn(partial, combine, n_q, n_kv, dim, std::max<int64_t>(capacity, 129), rot / 2, scale);   // (two phases whatever the capacity: the merge adds the sink)
+    for (ChainPhase* p : {&partial, &combine}) {
+        p->capacity = (int)capacity;
+        p->N = chunk > 0 ? (int)std::min<int64_t>(chunk, INT32_MAX) : INT32_MAX;
+        p->eps = eps;
+    }
+}
+
 bool chain_launch(hipStream_t s, const ChainPhase* dev_table, int nphases, int lds_bytes, unsigned* bar, int* abort_flag, int wfmt,
-                  int stall_phase) {
+                  int stall_phase, bool chunk_rows) {
     const int grid = chain_grid();
     if (grid <= 0 || nphases <= 0 || nphases > kChainMaxPhases || lds_bytes > kChainMaxXsWords * 4) return false;
-    if (wfmt < kChainW16 || wfmt > kChainW32) return false;
+    if (wfmt < kChainW16 || wfmt > kChainW32 || (chunk_rows && wfmt != kChainW16)) return false;
     const int xs_bytes = (lds_bytes + 1023) / 1024 * 1024;
     static const int max_depth = [] { const char* e = getenv("GPTRS_HIP_CHAIN_RING"); return e ? std::max(RING_MIN, std::min(RING_MAX, atoi(e))) : RING_MAX; }();
     const int depth = sizeof(Shared) + (size_t)xs_bytes + (size_t)max_depth * SLOT_BYTES <= (size_t)LDS_BYTES ? max_depth : RING_MIN;
     const size_t smem = sizeof(Shared) + (size_t)xs_bytes + (size_t)depth * SLOT_BYTES;
     if (smem > (size_t)LDS_BYTES) return false;
     static_assert(RING_MAX == RING_MIN + 1, "two kernels per weight format");
-    const int variant = wfmt * 2 + (depth - RING_MIN);
+    const int variant = (chunk_rows ? 4 : wfmt) * 2 + (depth - RING_MIN);
     typedef void (*Kernel)(const ChainPhase*, int, unsigned*, int*, int, unsigned long long, int);
-    static const Kernel kernels[8] = {chain_kernel<kChainW16, RING_MIN>, chain_kernel<kChainW16, RING_MAX>, chain_kernel<kChainW8, RING_MIN>,
+    static const Kernel kernels[10] = {chain_kernel<kChainW16, RING_MIN>, chain_kernel<kChainW16, RING_MAX>, chain_kernel<kChainW8, RING_MIN>,
                                       chain_kernel<kChainW8, RING_MAX>,  chain_kernel<kChainW4, RING_MIN>,  chain_kernel<kChainW4, RING_MAX>,
-                                      chain_kernel<kChainW32, RING_MIN>, chain_kernel<kChainW32, RING_MAX>};
+                                      chain_kernel<kChainW32, RING_MIN>, chain_kernel<kChainW32, RING_MAX>,
+                                       chain_kernel<kChainW16, RING_MIN, kRowsChunk>, chain_kernel<kChainW16, RING_MAX, kRowsChunk>};
     static_assert(kChainW16 == 0 && kChainW8 == 1 && kChainW4 == 2 && kChainW32 == 3, "index of a kernel");
     const Kernel fn = kernels[variant];
     if (g_occupancy_ok[variant] < 0) {

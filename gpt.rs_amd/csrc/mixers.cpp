@@ -244,7 +244,14 @@ void lower_mixer_calls(Function& fn) {
 }
 
 // operands of Mix::ChunkDecode / ChunkPrefill: proj, sink, pos, starts, [table,] keys_0, values_0, keys_1, ..
-static size_t chunk_cache_operand(const Instr& in, int64_t b) { return (size_t)(4 + (in.mx.rot > 0 ? 1 : 0) + 2 * b); }
+size_t chunk_cache_operand(const Instr& in, int64_t b) { return (size_t)(4 + (in.mx.rot > 0 ? 1 : 0) + 2 * b); }
+
+// a step of one sequence's attention that a decode chain can take
+bool chain_chunk_attn(const Instr& in) {
+    const Instr::MixAttrs& m = in.mx;
+    return in.op == OpKind::FMixer && in.mix == Mix::ChunkDecode && in.lens.size() == 1 && in.out_specs[0].dtype == DType::BF16 && in.out_specs[0].dims[0] == 1 &&
+           k::chain_chunk_attn_supported(m.heads, m.groups, m.dim, m.vdim, m.rot);
+}
 
 size_t mixer_scratch_bytes(const Instr& in, const std::vector<const Spec*>& operands) {
     const Instr::MixAttrs& m = in.mx;
@@ -255,7 +262,8 @@ size_t mixer_scratch_bytes(const Instr& in, const std::vector<const Spec*>& oper
         return k::latent_decode_scratch_bytes(dt, std::min<int64_t>(rows, k::kMixerBatch), operands[in.append ? 8 : 5]->dims[1], m.heads, m.dim, m.rot, m.rank, m.vdim);
     if (in.mix == Mix::LatentPrefill) return k::latent_prefill_scratch_bytes(dt, rows, m.heads, m.dim, m.rot, m.vdim);
     if (in.mix == Mix::ChunkDecode)
-        return k::chunk_decode_scratch_bytes(dt, std::min<int64_t>(rows, k::kMixerBatch), operands[chunk_cache_operand(in, 0)]->dims[1], m.heads, m.groups, m.dim, m.vdim);
+        return std::max(k::chunk_decode_scratch_bytes(dt, std::min<int64_t>(rows, k::kMixerBatch), operands[chunk_cache_operand(in, 0)]->dims[1], m.heads, m.groups, m.dim, m.vdim),
+                        chain_chunk_attn(in) ? k::chain_attn_part_bytes(m.heads, m.groups, m.dim) : (size_t)0);
     if (in.mix == Mix::ChunkPrefill) return k::chunk_prefill_scratch_bytes(dt, rows, m.heads, m.groups, m.dim, m.vdim);
     return 0;
 }

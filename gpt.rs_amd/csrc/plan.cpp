@@ -877,6 +877,7 @@ void Builder::build() {
     // runs of consecutive decode linears / decode attentions -> one persistent launch each
     auto chain_phases = [&](const Step& st) -> int {   // phases the step takes in a chain, 0: not chainable
         const Instr& in = st.in;
+        if (in.op == OpKind::FMixer) return chain_chunk_attn(in) ? 2 : 0;
         if (in.op == OpKind::FAttnDecode) {
             if (in.batch > 1) return 0;
             const Spec& x = plan.values[st.src[0]].spec;
@@ -904,6 +905,7 @@ void Builder::build() {
     };
     // f32 linears and f32 attentions go together (the launch's kernel reads f32 rows and caches), the others likewise
     auto f32_class = [&](const Step& st) {
+        if (st.in.op == OpKind::FMixer) return false;
         if (st.in.op == OpKind::FAttnDecode) return plan.values[st.src[0]].spec.dtype == DType::F32;
         return step_format(st) == k::kChainW32;
     };
@@ -914,11 +916,16 @@ void Builder::build() {
         bool has_linear = plan.steps[s].in.op == OpKind::FLinear;
         int fmt = has_linear ? step_format(plan.steps[s]) : -1;   // one weight format per launch
         const bool cls = f32_class(plan.steps[s]);
+        OpKind att = has_linear ? OpKind::FLinear : plan.steps[s].in.op;   // one kind of attention per launch; the chunked one beside bf16 weights only
         while (e < n_steps) {
             const Step& nx = plan.steps[e];
             const int q = chain_phases(nx);
             if (!q || np + q > k::kChainMaxPhases) break;
             if (f32_class(nx) != cls) break;
+            if (nx.in.op != OpKind::FLinear && att != OpKind::FLinear && att != nx.in.op) break;
+            if (nx.in.op == OpKind::FMixer && fmt > k::kChainW16) break;
+            if (nx.in.op == OpKind::FLinear && att == OpKind::FMixer && step_format(nx) != k::kChainW16) break;
+            if (nx.in.op != OpKind::FLinear) att = nx.in.op;
             if (nx.in.op == OpKind::FLinear) {
                 if (fmt >= 0 && step_format(nx) != fmt) break;
                 fmt = step_format(nx);
@@ -982,9 +989,39 @@ static bool run_chain(const Plan& plan, const Step& head, ExecCtx& cx) {
         }
         if (f32_linears > 0 && f32_bytes < cx.be->chain_f32_min_bytes * f32_linears) { cx.chain = false; return false; }
     }
+    bool chunk_rows = false;
     for (int i = 0; i < head.chain_len; ++i) {
         const Step& st = (&head)[i];
         const Instr& in = st.in;
+        if (in.op == OpKind::FMixer) {   // operands: proj, sink, pos, starts, [table,] keys, values
+            const Instr::MixAttrs& m = in.mx;
+            const size_t ci = chunk_cache_operand(in, 0);
+            const Spec& ck = plan.values[st.src[ci]].spec;
+            void* caches[2];
+            for (int kv = 0; kv < 2; ++kv) {
+                const void* from = cx.ptr[st.src[ci + kv]];
+                caches[kv] = cx.ptr[st.dst[1 + kv]];
+                if (caches[kv] != from) { GPTRS_HIP_CHECK(hipMemcpyAsync(caches[kv], from, ck.bytes(), hipMemcpyDeviceToDevice, cx.stream)); ++cx.launches; }
+            }
+            k::ChainPhase pa{}, pc{};
+            k::chain_fill_chunk_attn(pa, pc, m.heads, m.groups, m.dim, ck.dims[1], m.rot, m.chunk, in.scale, in.eps);
+            pa.x = cx.ptr[st.src[0]];
+            pa.k_cache = caches[0]; pa.v_cache = caches[1];
+            pa.update_starts = (const int32_t*)cx.ptr[st.src[3]];
+            pa.query_start = (const int32_t*)cx.ptr[st.src[2]];
+            if (m.rot > 0) pa.cos = cx.ptr[st.src[4]];
+            pa.part = pc.part = (float*)(cx.ws + st.scratch_off);
+            pc.gamma = cx.ptr[st.src[1]];
+            pc.bias = (const float*)pa.x + (m.heads + 2 * m.groups) * m.dim;
+            pc.y = pa.y = cx.ptr[st.dst[0]];
+            aligned8({pa.x, pa.part, pc.y});
+            if (((uintptr_t)caches[0] | (uintptr_t)caches[1] | (uintptr_t)pa.cos) & 15) fail_exec("decode chain: cache and angle buffers must be 16-byte aligned");
+            lds_bytes = std::max(lds_bytes, std::max(pa.lds_total, pc.lds_total));
+            phases.push_back(pa);
+            phases.push_back(pc);
+            chunk_rows = true;
+            continue;
+        }
         if (in.op == OpKind::FAttnDecode) {
             const Spec& ck = plan.values[st.src[1]].spec;
             void* kout = cx.ptr[st.dst[1]];
@@ -1078,7 +1115,7 @@ static bool run_chain(const Plan& plan, const Step& head, ExecCtx& cx) {
         cx.be->chain_stall_phase = -1;
         cx.be->chain_stall_fired = true;
     }
-    if (!k::chain_launch(cx.stream, table, (int)phases.size(), lds_bytes, cx.be->chain_barrier(), cx.be->chain_abort_flag(), wfmt, stall)) {
+    if (!k::chain_launch(cx.stream, table, (int)phases.size(), lds_bytes, cx.be->chain_barrier(), cx.be->chain_abort_flag(), wfmt, stall, chunk_rows)) {
         if (e0) { (void)hipEventDestroy(e0); (void)hipEventDestroy(e1); }
         cx.chain = false;
         return false;
@@ -1617,6 +1654,8 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
             break;
         }
         case OpKind::FMixer:
+            if (cx.chain && st.chain_member) break;  // executed by the launch of the run's first step
+            if (cx.chain && st.chain_len > 0 && run_chain(plan, st, cx)) break;
             run_mixer(plan, st, cx);
             break;
         default:

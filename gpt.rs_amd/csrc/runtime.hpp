@@ -353,6 +353,8 @@ void lower_norm_calls(Function& fn);
 void lower_mixer_calls(Function& fn);
 // mixers.cpp: scratch of one launch, and the launch itself.  mixer_inplace_pairs: (operand slot, output slot) of the state
 // that the call may update in place when the caller donates it.
+size_t chunk_cache_operand(const Instr& in, int64_t b);   // position of sequence b's keys among the operands of ChunkDecode / ChunkPrefill
+bool chain_chunk_attn(const Instr& in);                  // ... a step that a decode chain can take
 size_t mixer_scratch_bytes(const Instr& in, const std::vector<const Spec*>& operands);
 std::vector<std::pair<int, int>> mixer_inplace_pairs(const Instr& in);
 struct Plan;

@@ -332,6 +332,42 @@ def test_merge_of_many_slices_heads_and_values(hip, shape, pos, cap):
     test_decode_of_a_batch_and_single_rows(hip, "Bf16", shape, pos, cap, 2000)
 
 
+@pytest.mark.parametrize("shape,taken", [((4, 2, 64, 64, 64), True), ((8, 1, 128, 128, 32), True), ((2, 2, 256, 256, 256), True), ((8, 8, 64, 64, 0), True), ((32, 8, 128, 128, 128), True),
+                                         ((3, 1, 64, 64, 8), False), ((4, 2, 64, 64, 12), False), ((4, 2, 64, 128, 8), False)])
+@pytest.mark.parametrize("pos,cap,chunk", [(0, 4, 9), (5, 6, 0), (63, 64, 100), (128, 129, 1000), (2000, 1024, 1024), (1023, 1024, 1024)])
+def test_decode_inside_a_chain(hip, shape, taken, pos, cap, chunk):
+    """One sequence's step in front of a layer: with 1, 2, 4 or 8 query heads to a key head of 64, 128 or 256 and as wide values the attention is two phases of the
+    layer's launch.  Against the oracle, the launches apart, and rows behind the current place that would stand out."""
+    H, G, D, V, rot = shape
+    place = min(pos % chunk if chunk else pos, cap - 1)
+    q, k = rn(3, 1, H, D).astype(np.float64), 0.5 * rn(4, 1, G, D).astype(np.float64)
+    kc, vc = 0.3 * rn(60, G, cap, D), rn(80, G, cap, V)
+    lead = unit(q.reshape(1, G, H // G, D)[:, :, 0])[0]
+    kc[:, place // 2] = lead * D ** 0.5
+    kc[:, place + 1:] = 2 * lead[:, None] * D ** 0.5
+    vc[:, place + 1:] += 50.0
+    sink = rn(2, H)
+    sink[0] = 6.0
+    w = rn(5, H * V, 96) * (H * V) ** -0.5
+    args = [(projection(1, np.array([pos]), H, G, D, V, rot, 30.0, q, k), "F32"), (sink, "F32"), (np.array([pos], np.int32), "Si32"), (np.array([0, place, 0], np.int32), "Si32"),
+            (F.pair_frequencies(rot, 30.0) if rot else np.zeros(1, np.float32), "F32"), (kc, "Bf16"), (vc, "Bf16"), (w, "Bf16")]
+    mixer = emit_mixer("Bf16", [1], H, G, D, V, rot, chunk, 9.0 / D, True)
+
+    def emit(fb, *a):
+        ctx, *caches = mixer(fb, *a[:-1])
+        return [ctx.matmul(a[-1]), *caches]
+
+    prog = build(emit, args)
+    want = on_oracle(prog, args)
+    for opts, phases in (({}, 3 if taken else 1), ({"chain": 0}, 0)):
+        before = hip.counter("chain_phases")
+        got = on_device(hip, prog, args, **opts)
+        assert hip.counter("chain_phases") - before == phases, (shape, opts)
+        check(got[0], want[0], 3e-2, (shape, pos, opts))
+        for g, c in zip(got[1:], want[1:]):
+            check(g, c, TOL["Bf16"], (shape, pos, opts, "cache"))
+
+
 # ------------------------------------------------------------------------------------------ whole models
 def load(hip, tmp_path, name, dt, seed=0, **kw):
     cfg = U.STACKS[name]
