@@ -4,6 +4,7 @@
 // Both compute softmax((q.k) * scale + mask) . v with the additive -1e9 mask replaced by its
 // exact f32 effect: masked positions contribute exactly 0 (exp underflows), so only positions
 // <= the query position are visited.  GQA: query head h reads kv head h / group.
+#include <algorithm>
 #include <cstdlib>
 
 #include <type_traits>
@@ -808,6 +809,10 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const T* __restrict__
 // 2 s + g (it stages them itself, into its own LDS buffers), and the two online-softmax states meet through LDS at the
 // end.  A row tile then takes half as many steps, and a SIMD holds two waves whose matrix and vector phases overlap
 // (the launch has one wave-sized task per SIMD otherwise).
+// KG = 4, HW = 2: four groups of two waves, two query heads to a workgroup: half the steps again, and twice the workgroups, for launches that leave
+// most CUs idle (143 KB of LDS, one workgroup to a CU).  What is left of 333 rows' 13.6 us is 9 that two steps also take: the start, the
+// first rows' arrival and code that no launch before has brought.  Filling the caches on the way, which saves attn_prefill_kv_kernel's 4.8 us,
+// was level at best: keys are turned again by every row tile (13.6 + 4.9 -> 20.8).  Asking for the first tile ahead of turning the queries gave 14.6.
 // V^T as the A operand of a 32 x 32 x 16 product, out of 16 rows of V from v on (keys down, 32 d across): lane 32 h + c holds, of d = c, the
 // keys 4 h .. 4 h + 3 and 8 + 4 h .. 8 + 4 h + 3, the order in which the scores' lanes hold theirs.  Two transposing reads: lane i of 16 gets
 // column i of four rows, lane 4 e + j of the 16 names columns 4 j .. 4 j + 3 of row e.
@@ -823,8 +828,8 @@ __device__ __forceinline__ bf16x8_v v_fragment(const bf16_t* v, int stride, int 
     return __builtin_bit_cast(bf16x8_v, r);
 }
 
-template <int DH, int KG, bool FILL>
-__global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ ctx, int T,
+template <int DH, int KG, int HW, bool FILL>
+__global__ __launch_bounds__(64 * HW * KG, KG > 1 ? 1 : FILL ? 2 : 3) void attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ ctx, int T,
                                                                 int n_q, int n_kv, float scale_log2e, int zgroups, PrefillKv<bf16_t> kv) {
     constexpr int KT = 32;            // keys per tile
     constexpr int KS = DH + 8;        // K tile row stride in elements (16 bytes of padding)
@@ -832,17 +837,19 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_pre
     constexpr int ND = DH / 32;       // 32-row blocks of d in O^T
     constexpr int NK = DH / 16;       // k-steps of the score product
     constexpr int CH = KT * DH / 8;   // 16-byte chunks of a K (or V) tile
-    constexpr int CPT = (CH + 255) / 256;
+    constexpr int TPG = 64 * HW;      // threads of a key group
+    constexpr int CPT = (CH + TPG - 1) / TPG;
     __shared__ __align__(16) bf16_t smem[KG * 2 * KT * (KS + VS)];
 
-    const int kg = threadIdx.x / 256;                     // key group of this wave
-    const int tid = threadIdx.x % 256, lane = tid & 63, wave = tid >> 6;
+    static_assert(!FILL || KG == 1, "a workgroup that fills the caches sees every tile once");
+    const int kg = KG == 4 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / TPG) : (int)threadIdx.x / TPG;   // key group of this wave
+    const int tid = threadIdx.x % TPG, lane = tid & 63, wave = tid >> 6;
     bf16_t (*ksm)[KT * KS] = reinterpret_cast<bf16_t (*)[KT * KS]>(smem + kg * 2 * KT * KS);
     bf16_t (*vsm)[KT * VS] = reinterpret_cast<bf16_t (*)[KT * VS]>(smem + KG * 2 * KT * KS + kg * 2 * KT * VS);
     const int col = lane & 31, half = lane >> 5;
     const int G = n_q / n_kv;
-    const int gw = G >= 4 ? 4 : G;                 // query heads of the group in this workgroup
-    const int rtpb = 4 / gw;                       // 32-row tiles per workgroup
+    const int gw = G >= HW ? HW : G;               // query heads of the group in this workgroup
+    const int rtpb = HW / gw;                      // 32-row tiles per workgroup
     const XcdTile at = xcd_tile();
     const int kvh = at.y;
     const int seq = at.z / zgroups, zg = at.z % zgroups;
@@ -897,7 +904,7 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_pre
     auto gload = [&](int t) {
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
-            const int c = min(tid + 256 * j, CH - 1);
+            const int c = min(tid + TPG * j, CH - 1);
             const int r = c / (DH / 8), ch = c % (DH / 8);
             const int64_t key = min(t * KT + r, T - 1);
             kreg[j] = *reinterpret_cast<const u32x4_s*>(kp + key * kpitch + ch * 8);
@@ -913,8 +920,8 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_pre
     auto lwrite = [&](int buf, int t) {
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
-            const int c = tid + 256 * j;
-            if (CH % 256 == 0 || c < CH) {
+            const int c = tid + TPG * j;
+            if (CH % TPG == 0 || c < CH) {
                 const int r = c / (DH / 8), ch = c % (DH / 8);
                 if (FILL) {
                     if (kv.cos) kreg[j] = rotated_chunk<bf16_t>(kreg[j], kother[FILL ? j : 0], kcos[FILL ? j : 0], ksin[FILL ? j : 0], ch >= DH / 16);
@@ -1010,7 +1017,7 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_pre
         // that saw no tile has m = -inf, l = 0, O = 0 and drops out.  The tiles in LDS are dead (the loop ended on a
         // barrier); the exchange area is 66 floats per lane of the second group.
         float* xch = reinterpret_cast<float*>(smem) + (wave * 64 + lane);
-        static_assert(KG == 1 || (ND * 16 + 2) * 256 * 4 <= (int)sizeof(smem), "exchange area fits the tiles");
+        static_assert(KG != 2 || (ND * 16 + 2) * 256 * 4 <= (int)sizeof(smem), "exchange area fits the tiles");
         if (kg == 1) {
 #pragma unroll
             for (int db = 0; db < ND; ++db)
@@ -1030,11 +1037,50 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_pre
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc_o[db][v] = acc_o[db][v] * c0 + xch[(db * 16 + v) * 256] * c1;
     }
+    if (KG == 4) {
+        // four states, likewise; group g finishes the 32 d of block g, so every wave writes and reads as much
+        constexpr int SLOTS = ND * 16 + 2;
+        static_assert(KG != 4 || (SLOTS * KG * TPG * 4 <= (int)sizeof(smem) && ND <= KG), "exchange area fits the tiles");
+        float* xch = reinterpret_cast<float*>(smem) + wave * 64 + lane;
+        auto at_slot = [&](int g, int slot) -> float& { return xch[(g * SLOTS + slot) * TPG]; };
+#pragma unroll
+        for (int db = 0; db < ND; ++db)
+            if (db != kg) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) at_slot(kg, db * 16 + v) = acc_o[db][v];
+            }
+        at_slot(kg, ND * 16) = m_run;
+        at_slot(kg, ND * 16 + 1) = l_run;
+        __syncthreads();
+        float mm = m_run, c[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) mm = fmaxf(mm, at_slot(g, ND * 16));
+        const float own = __builtin_amdgcn_exp2f(m_run - mm);
+        l_run = 0.f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            c[g] = __builtin_amdgcn_exp2f(at_slot(g, ND * 16) - mm);
+            l_run += at_slot(g, ND * 16 + 1) * c[g];
+        }
+#pragma unroll
+        for (int db = 0; db < ND; ++db)
+            if (db == kg) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    float o = acc_o[db][v] * own;
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        if (g != db) o = __builtin_fmaf(at_slot(g, db * 16 + v), c[g], o);
+                    acc_o[db][v] = o;
+                }
+            }
+    }
     if (active && q0 + col < T) {
         const float inv = 1.0f / l_run;
         bf16_t* op = ctx + (int64_t)(q0 + col) * n_q * DH + (int64_t)head * DH;
 #pragma unroll
-        for (int db = 0; db < ND; ++db)
+        for (int db = 0; db < ND; ++db) {
+            if (KG == 4 && db != kg) continue;
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int d = db * 32 + 8 * g4 + 4 * half;
@@ -1042,6 +1088,7 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 1 : FILL ? 2 : 3) void attn_pre
                 const uint32_t hi = pack_bf16x2(acc_o[db][4 * g4 + 2] * inv, acc_o[db][4 * g4 + 3] * inv);
                 *reinterpret_cast<uint2*>(op + d) = make_uint2(lo, hi);
             }
+        }
     }
 }
 
@@ -1335,8 +1382,14 @@ static int attn_prefill_mfma(hipStream_t s, const AttnPrefillArgs& a) {
     kv.starts = a.starts;
     kv.capacity = a.capacity;
     if (a.rot_half) { kv.cos = (const T*)a.cos; kv.sin = (const T*)a.sin; }
-    const int g = (int)(a.n_q / a.n_kv), gw = g >= 4 ? 4 : g, zg = g >= 4 ? g / 4 : 1;
-    const dim3 grid((unsigned)cdiv(cdiv(a.t, 32), 4 / gw), (unsigned)a.n_kv, (unsigned)(zg * a.batch));
+    // four key groups (bf16) while the launch is one workgroup to a CU at most and rows see more than two tiles.  us, four and two groups (one, under 128
+    // rows), 32 / 8 heads of 128: 100 rows 11.3 and 13.5, 128 11.2 and 13.8, 200 11.7 and 14.2, 333 13.6 and 17.1, 512 (256 workgroups) 16.9 and 21.6, 2 x 256
+    // 13.7 and 17.1; beyond: 2 x 333 23.5 and 19.0, 1000 37 and 35; 64 rows 12 and 11
+    static const bool allow_kg = [] { const char* e = getenv("GPTRS_HIP_ATTN_KEYGROUPS"); return !(e && e[0] == '0'); }();
+    const int64_t g = a.n_q / a.n_kv;
+    const bool kg4 = std::is_same<T, bf16_t>::value && allow_kg && a.t > 64 && cdiv(cdiv(a.t, 32), g == 1 ? 2 : 1) * a.n_kv * (g == 1 ? 1 : g / 2) * a.batch <= 256;
+    const int64_t hw = kg4 ? 2 : 4, gw = std::min(g, hw), zg = g / gw;   // waves of a key group; query heads of a workgroup, workgroups of a key head
+    const dim3 grid((unsigned)cdiv(cdiv(a.t, 32), hw / gw), (unsigned)a.n_kv, (unsigned)(zg * a.batch));
     const float sl = a.scale * 1.44269504088896f;
     if constexpr (std::is_same<T, float>::value)
         if (a.t <= kShortRows && !kv.cos && (a.head_dim == 64 || a.head_dim == 128)) {
@@ -1347,10 +1400,9 @@ static int attn_prefill_mfma(hipStream_t s, const AttnPrefillArgs& a) {
         }
     // two key groups per workgroup once the launch is smaller than three workgroups per CU and rows are long
     // enough to split (bf16)
-    static const bool allow_kg = [] { const char* e = getenv("GPTRS_HIP_ATTN_KEYGROUPS"); return !(e && e[0] == '0'); }();
-    const bool kg2 = std::is_same<T, bf16_t>::value && allow_kg && a.t >= 128 && (int64_t)grid.x * grid.y * grid.z < 768;
+    const bool kg2 = !kg4 && std::is_same<T, bf16_t>::value && allow_kg && a.t >= 128 && (int64_t)grid.x * grid.y * grid.z < 768;
     // one row tile: the attention fills the caches itself (us: 7 rows, 12 heads of 64 in f32 8.9 -> 6.4, 16 x 100 rows 22.7 -> 17.9; 20 rows, 32 / 8 heads of 128 in bf16 11.5 -> 9.4)
-    const bool fill = a.starts && grid.x == 1 && !kg2;
+    const bool fill = a.starts && grid.x == 1 && !kg2 && !kg4;
     int launches = 1;
     if (a.starts && !fill) {
         const int64_t chunks = a.batch * a.t * 2 * a.n_kv * a.head_dim / (16 / (int64_t)sizeof(T));
@@ -1359,14 +1411,15 @@ static int attn_prefill_mfma(hipStream_t s, const AttnPrefillArgs& a) {
     }
     auto go = [&](auto dh) {
         constexpr int D = decltype(dh)::value;
-        auto launch = [&](auto kernel, int threads) { kernel<<<grid, threads, 0, s>>>((const T*)a.qkv, (T*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, zg, kv); };
+        auto launch = [&](auto kernel, int threads) { kernel<<<grid, threads, 0, s>>>((const T*)a.qkv, (T*)a.ctx, (int)a.t, (int)a.n_q, (int)a.n_kv, sl, (int)zg, kv); };
         if constexpr (std::is_same<T, float>::value) {
             if (fill) launch(attn_prefill_mfma_f32_kernel<D, true>, 256);
             else launch(attn_prefill_mfma_f32_kernel<D, false>, 256);
         } else {
-            if (kg2) launch(attn_prefill_mfma_kernel<D, 2, false>, 512);
-            else if (fill) launch(attn_prefill_mfma_kernel<D, 1, true>, 256);
-            else launch(attn_prefill_mfma_kernel<D, 1, false>, 256);
+            if (kg4) launch(attn_prefill_mfma_kernel<D, 4, 2, false>, 512);
+            else if (kg2) launch(attn_prefill_mfma_kernel<D, 2, 4, false>, 512);
+            else if (fill) launch(attn_prefill_mfma_kernel<D, 1, 4, true>, 256);
+            else launch(attn_prefill_mfma_kernel<D, 1, 4, false>, 256);
         }
     };
     if (a.head_dim == 32) go(std::integral_constant<int, 32>{});

@@ -32,3 +32,11 @@ def test_every_row(hip, dtype, hq, hkv, dh, t):
         score = 2.0 ** -24 * 2 * np.sqrt(dh) * (np.abs(q[:, h]) @ np.abs(k[:, h * hkv // hq]).T).max() * dh ** -0.5
         tol = (2.0 ** -8 if dtype == "Bf16" else 0) + 2 * score + 2.0 ** -24 * (2 * np.sqrt(t) + 16)
         assert (np.abs(got[:, h] - w @ vh) <= tol * (mags + np.abs(w @ vh)) + 1e-6).all(), h
+
+
+# 65 to 128 keys: a wave group of four without a tile, one with a part of one; groups of 1, 2, 4 and 8 query heads; the last launch of four key
+# groups (256 workgroups) and the first beyond
+@pytest.mark.parametrize("hq,hkv,dh,t", [(4, 4, 32, 65), (5, 5, 128, 96), (8, 4, 64, 97), (8, 4, 32, 128), (16, 2, 32, 129), (16, 2, 128, 65),
+                                         (32, 8, 128, 100), (32, 8, 128, 512), (32, 8, 128, 513), (8, 8, 64, 2000)])
+def test_four_key_groups(hip, hq, hkv, dh, t):
+    test_every_row(hip, "Bf16", hq, hkv, dh, t)
