@@ -13,8 +13,10 @@ materialize / to_literal / run_program / param_resolver / sample_decode_token.
 """
 from __future__ import annotations
 
+import copy
 import itertools
 import os
+from array import array
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -81,6 +83,28 @@ def _np_to_bytes(arr: np.ndarray, dtype: str) -> bytes:
     if dtype == "Si32":
         return np.ascontiguousarray(arr, dtype="<i4").tobytes()
     raise ValueError(dtype)
+
+
+def _int_rows(rows) -> Optional[np.ndarray]:
+    """Lists of integers behind one another as int32 (8192 of them, checked, 0.19 ms, item by item 0.77); None: something else is in them."""
+    flat = array("i")
+    try:
+        for row in rows:
+            flat.fromlist(row)
+    except (TypeError, OverflowError):
+        return None
+    return np.frombuffer(flat, np.intc) if len(flat) else np.empty(0, np.intc)
+
+
+def _checked_tokens(rows, vocab_size: int):
+    """The tokens of all rows, each inside the vocabulary."""
+    flat = _int_rows(rows)
+    if flat is None or (flat.size and (flat.min() < 0 or flat.max() >= vocab_size)):
+        for row in rows:
+            for t in row:
+                if not 0 <= t < vocab_size:
+                    raise ValueError(f"token index {t} out of range")
+    return flat if flat is not None else [t for row in rows for t in row]
 
 
 def base_param_id(name: str) -> int:
@@ -328,6 +352,15 @@ class _ModelBase:
             opt = FE.optimize(program, roles, stable, self.backend, self.backend.param_resolver(), **hooks)
             entry = self._optimized[program.key] = (opt, {}, tuple(names), self.backend_pipeline)
         opt, held = entry[0], entry[1]
+        if held.get("complete") and not self._lazy:   # every parameter has been found: only the arguments change from run to run
+            inputs, don = list(held["inputs"]), None
+            for pos, src in held["args"]:
+                inputs[pos] = args[src]
+            if donate is not None:
+                don = [False] * len(inputs)
+                for pos, src in held["args"]:
+                    don[pos] = bool(donate[src])
+            return self.backend.run_program(opt.program, inputs, don)
         inputs, don = [], []
         resolver = self.backend.param_resolver()
         for pos, (p, src) in enumerate(zip(opt.inputs, opt.source_index)):
@@ -346,6 +379,10 @@ class _ModelBase:
                 held[pos] = h
             inputs.append(h)
             don.append(False)
+        if not self._lazy:
+            held["args"] = [(pos, src) for pos, (p, src) in enumerate(zip(opt.inputs, opt.source_index)) if p.role == FE.ARG]
+            held["inputs"] = [None if p.role == FE.ARG else h for p, h in zip(opt.inputs, inputs)]
+            held["complete"] = True
         return self.backend.run_program(opt.program, inputs, don if donate is not None else None)
 
 
@@ -565,10 +602,7 @@ class Gpt(_ModelBase):
         if total > cfg.context_length:
             raise ValueError(f"token sequence length {total} exceeds model context length {cfg.context_length}")
         if token_handle is None:
-            for row in token_rows:
-                for t in row:
-                    if not 0 <= t < cfg.vocab_size:
-                        raise ValueError(f"token index {t} out of range")
+            tokens = _checked_tokens(token_rows, cfg.vocab_size)
         elif seq != 1:
             raise ValueError("device tokens feed one step (one token per sequence)")
         if any(len(c) != cfg.num_layers for c in caches):
@@ -586,8 +620,8 @@ class Gpt(_ModelBase):
             raise ValueError("decode with an existing cache supports one token per sequence")
         L = cfg.num_layers
         prog, _ = self._build(seq, capacity, have, batch, last_logits_only)
-        poss = [position_offset + j for _ in range(batch) for j in range(seq)]
-        tok_arg = token_handle if token_handle is not None else self._upload_i32([t for row in token_rows for t in row])
+        poss = [position_offset] * batch if seq == 1 else np.tile(np.arange(position_offset, total, dtype=np.int32), batch)
+        tok_arg = token_handle if token_handle is not None else self._upload_i32(tokens)
         args = [tok_arg, self._upload_i32(poss)]
         if have:
             for c in caches:
@@ -659,6 +693,7 @@ class Ministral(_ModelBase):
         self.config = config
         self.attn = config.attention_config()
         self.rope = F.RopeConfig(config.rotary_dim, config.rope_theta, config.rope_scaling)
+        self._rope_table: Dict[str, object] = {}
         if residual_dtype is not None and residual_dtype not in ("F32",):
             raise ValueError("residual_dtype must be None or 'F32'")
         self.residual_dtype = residual_dtype if (residual_dtype and residual_dtype != dtype) else None
@@ -889,6 +924,23 @@ class Ministral(_ModelBase):
         self._programs[key] = (prog, layout)
         return prog, layout
 
+    def _rope_rows(self, start: int, end: int):
+        """Bytes of the cosines and sines of positions start .. end - 1.  The rows of positions seen so far are kept with the model, to a power of
+        two (they are constants of its rotation; 333 rows anew 0.13 ms in front of the first launch)."""
+        if start < 0:
+            return tuple(_np_to_bytes(x, self.dtype) for x in F.rotary_cos_sin_cache_slice(start, end - start, self.rope))
+        table = self._rope_table
+        if table.get("rope") != self.rope:
+            table = {"rope": copy.deepcopy(self.rope), "rows": 0, "cos": b"", "sin": b""}
+        have = table["rows"]
+        if have < end:
+            rows = max(decode_cache_capacity(end, self.config.context_length), end)
+            cos, sin = F.rotary_cos_sin_cache_slice(have, rows - have, self.rope)
+            table = {"rope": table["rope"], "rows": rows, "cos": table["cos"] + _np_to_bytes(cos, self.dtype), "sin": table["sin"] + _np_to_bytes(sin, self.dtype)}
+            self._rope_table = table
+        row = len(table["cos"]) // table["rows"]
+        return table["cos"][start * row:end * row], table["sin"][start * row:end * row]
+
     def forward_with_decode_cache(self, tokens, position_offset, caches, fixed_capacity=None, last_logits_only=False):
         """model/ministral.rs:613-766.  last_logits_only: see Gpt.forward_with_decode_cache."""
         return self.forward_batch([list(tokens)], position_offset, [caches], fixed_capacity, last_logits_only=last_logits_only)
@@ -922,12 +974,14 @@ class Ministral(_ModelBase):
             raise ValueError("decode with an existing cache supports one token per sequence")
         L = cfg.num_layers
         prog, _ = self._build(seq, capacity, have, batch, last_logits_only)
-        cos, sin = F.rotary_cos_sin_cache_slice(position_offset, seq, self.rope)   # ministral.rs:253-261
-        half = cfg.rotary_dim // 2
-        tok_arg = token_handle if token_handle is not None else self._upload_i32([t for row in token_rows for t in row])
-        args = [tok_arg,
-                self.backend.materialize(TensorSpec(self.dtype, [seq, half]), _np_to_bytes(cos, self.dtype)),
-                self.backend.materialize(TensorSpec(self.dtype, [seq, half]), _np_to_bytes(sin, self.dtype))]
+        cos, sin = self._rope_rows(position_offset, total)   # ministral.rs:253-261
+        if token_handle is not None:
+            tok_arg = token_handle
+        else:
+            tokens = _int_rows(token_rows)
+            tok_arg = self._upload_i32(tokens if tokens is not None else [t for row in token_rows for t in row])
+        table = TensorSpec(self.dtype, [seq, cfg.rotary_dim // 2])
+        args = [tok_arg, self.backend.materialize(table, cos), self.backend.materialize(table, sin)]
         if have:
             args += [self._upload_i32([0, position_offset, 0]), self._upload_i32([position_offset])]
             kv = [h for c in caches for slot in c for h in (slot.keys, slot.values)]
@@ -1029,10 +1083,7 @@ class _RaggedModel(_ModelBase):
         if token_handle is not None and max(lens) != 1:
             raise ValueError("device tokens feed one step (one token per sequence)")
         if token_handle is None:
-            for row in token_rows:
-                for t in row:
-                    if not 0 <= t < cfg.vocab_size:
-                        raise ValueError(f"token index {t} out of range")
+            tokens = _checked_tokens(token_rows, cfg.vocab_size)
         totals = [o + n for o, n in zip(offs, lens)]
         need = max(totals)
         if need > cfg.context_length:
@@ -1056,8 +1107,9 @@ class _RaggedModel(_ModelBase):
         if logit_rows is not None and list(logit_rows) == list(range(sum(lens))):
             logit_rows = None
         prog, _ = self._build(lens, capacity, have, last_logits_only and logit_rows is None, None if logit_rows is None else len(logit_rows))
-        tok_arg = token_handle if token_handle is not None else self._upload_i32([t for row in token_rows for t in row])
-        args = [tok_arg, self._upload_i32([o + j for o, n in zip(offs, lens) for j in range(n)])] + self._position_args(offs)
+        tok_arg = token_handle if token_handle is not None else self._upload_i32(tokens)
+        poss = offs if max(lens) == 1 else np.concatenate([np.arange(o, o + n, dtype=np.int32) for o, n in zip(offs, lens)])
+        args = [tok_arg, self._upload_i32(poss)] + self._position_args(offs)
         if logit_rows is not None:
             args.append(self._upload_i32(logit_rows))
         held = [h for c in caches for i, slot in enumerate(c) for h in (self._slot_handles(slot) if have else self._fresh_slot(i, capacity))]
@@ -1862,7 +1914,6 @@ class Generator:
         # the loop only ever samples from the last row: prefill runs the head on that row alone (`self.logits` is then
         # [1, V] after a prefill as after a decode step); False keeps every row as the reference's forward does
         self.last_logits_only = bool(last_logits_only)
-        self._rng = np.random.default_rng(seed)
         can_pipeline = device_sampling and hasattr(model.backend, "sample_decode_token_begin") and \
             hasattr(model, "forward_decode_device_token")
         if pipelined and not can_pipeline:
@@ -1873,6 +1924,7 @@ class Generator:
         context = self.tokens[self.window_start:]
         self.logits = self._prefill(context)
         self.processed_len = len(context)
+        self._rng = np.random.default_rng(seed)   # (while the device reads the prompt)
 
     def _sample(self) -> int:
         be = self.model.backend

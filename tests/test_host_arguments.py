@@ -1,0 +1,55 @@
+"""What the models prepare on the host ahead of a program: tokens and positions as arrays, rotation tables kept with the model, inputs of a
+program whose parameters have been found."""
+import numpy as np
+import pytest
+
+from oracle_backend import OracleBackend
+from gptrs_amd import functional as F
+from gptrs_amd import models
+
+
+@pytest.mark.parametrize("rows", [[[0]], [[5, 99, 0]], [[1, 2], [3, 4]], [[np.int64(7), True], [np.int32(98)]], [[3.0, 4.5]], [(1, 2)], [np.array([8, 9])]])
+def test_tokens(rows):
+    got = np.asarray(models._checked_tokens(rows, 100), np.int32)
+    np.testing.assert_array_equal(got, np.asarray([t for r in rows for t in r], np.int32))
+
+
+@pytest.mark.parametrize("rows", [[[100]], [[-1]], [[0, 1], [2, 100]], [[1 << 40]], [[-(1 << 70)]], [[float("nan")]], [[-0.5]]])
+def test_tokens_outside(rows):
+    with pytest.raises(ValueError, match="out of range"):
+        models._checked_tokens(rows, 100)
+
+
+@pytest.mark.parametrize("dtype", ["F32", "Bf16"])
+@pytest.mark.parametrize("scaling", [None, ("linear", 4.0)])
+def test_rotation_rows_are_those_of_their_positions(dtype, scaling):
+    cfg = models.MinistralConfig(vocab_size=32, context_length=96, embed_dim=32, num_layers=1, num_heads=4, num_kv_heads=2, head_dim=8, ffn_dim=32,
+                                 rotary_dim=8, rope_scaling=scaling)
+    m = models.Ministral(cfg, OracleBackend(), dtype)
+
+    def rows(start, end):
+        return tuple(models._np_to_bytes(x, dtype) for x in F.rotary_cos_sin_cache_slice(start, end - start, m.rope))
+
+    for start, end in ((0, 7), (7, 8), (8, 9), (0, 33), (95, 96), (0, 96), (-2, 3)):
+        assert m._rope_rows(start, end) == rows(start, end)
+    m.rope.theta = 500.0
+    assert m._rope_rows(3, 9) == rows(3, 9)
+
+
+def test_runs_behind_the_first_see_new_arguments_and_new_parameters():
+    cfg = models.GptConfig(vocab_size=24, context_length=16, embed_dim=16, num_layers=1, num_heads=2, mlp_ratio=2)
+    be = OracleBackend()
+    m = models.Gpt.random(cfg, be, seed=3)
+
+    def logits(tokens):
+        return be.to_numpy(m.forward_with_decode_cache(tokens, 0, [None]))
+
+    first, other, again = logits([1, 2, 3]), logits([4, 5, 6]), logits([1, 2, 3])
+    np.testing.assert_array_equal(first, again)
+    assert not np.array_equal(first, other)
+    head = np.random.default_rng(1).standard_normal((16, 24)).astype(np.float32)
+    m.set_param("lm_head", head)
+    assert not np.array_equal(logits([1, 2, 3]), first)
+    fresh = models.Gpt.random(cfg, OracleBackend(), seed=3)
+    fresh.set_param("lm_head", head)
+    np.testing.assert_array_equal(logits([1, 2, 3]), fresh.backend.to_numpy(fresh.forward_with_decode_cache([1, 2, 3], 0, [None])))
