@@ -6,6 +6,8 @@
 
 #include <mutex>
 
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "device_utils.hpp"
 
@@ -445,7 +447,7 @@ void dot_generic(hipStream_t s, int dtype, const void* a, const void* b, void* c
 // (out64, one row, or out32) and, with `host`, straight into the pinned slot that the caller waits for, with the device's error flags beside
 // it: host[0] the token of a single row, host[1] the flags, from host + 2 on the tokens of several.  Between two decode steps
 // that is one launch of 6 us where two stages and two copies took 19.  A ticket is zero before and after every launch.
-template <typename T>
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void argmax_kernel(const T* __restrict__ logits, int64_t n, float* pv, int32_t* pi, unsigned* tickets, int64_t* out64, int32_t* out32,
                                                      int64_t* host, const int64_t* err_flags) {
     constexpr int U = 4;
@@ -463,14 +465,21 @@ __global__ __launch_bounds__(256) void argmax_kernel(const T* __restrict__ logit
             better(ov, oi);
         }
     };
-    const int64_t stride = (int64_t)gridDim.x * 256;
-    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += U * stride) {
-        float v[U];
+    typedef T vec_t __attribute__((ext_vector_type(VEC)));
+    const int64_t stride = (int64_t)gridDim.x * 256, whole = n / VEC;
+    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < whole; i0 += U * stride) {
+        vec_t v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = ldf(row, i0 + u * stride < n ? i0 + u * stride : i0);
+        for (int u = 0; u < U; ++u) v[u] = reinterpret_cast<const vec_t*>(row)[i0 + u * stride < whole ? i0 + u * stride : i0];
 #pragma unroll
-        for (int u = 0; u < U; ++u) better(v[u], (int32_t)(i0 + u * stride < n ? i0 + u * stride : i0));
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                const T x = v[u][e];
+                better(ldf(&x, 0), (int32_t)((i0 + u * stride < whole ? i0 + u * stride : i0) * VEC + e));
+            }
     }
+    if (blockIdx.x == 0 && threadIdx.x < n - whole * VEC) better(ldf(row, whole * VEC + threadIdx.x), (int32_t)(whole * VEC + threadIdx.x));
     over_wave();
     if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = best; si[threadIdx.x >> 6] = bidx; }
     __syncthreads();
@@ -503,12 +512,19 @@ __global__ __launch_bounds__(256) void argmax_kernel(const T* __restrict__ logit
 }
 void argmax_tokens(hipStream_t s, int dtype, const void* logits, int64_t rows, int64_t vocab, int64_t* out64, int32_t* out32, const ArgmaxScratch& w, int64_t* host) {
     if (rows <= 0) return;
+    // Up to 256 workgroups of four loads of a value each; beyond, 16 bytes a load and 256 workgroups, since all of them meet at tickets that share a line (us: 8 rows
+    // of 131072 by 1024 workgroups 16.9, so 9.0; one row of 50257 5.7, with 16 bytes a load in 50 workgroups 6.1, in 13 5.9)
+    const int vec = dtype == 0 ? 4 : 8;
     int64_t nb = cdiv(vocab, 256 * 4);
+    const bool wide = rows * nb > 256 && ((uintptr_t)logits & 15u) == 0 && (rows == 1 || vocab % vec == 0);
+    if (wide) nb = std::min<int64_t>(cdiv(vocab, 256 * vec), std::max<int64_t>(256 / rows, 1));
     if (nb > w.parts / rows) nb = w.parts / rows;
     if (nb < 1) nb = 1;
     const dim3 grid((unsigned)nb, (unsigned)rows);
-    if (dtype == 0) argmax_kernel<float><<<grid, 256, 0, s>>>((const float*)logits, vocab, w.val, w.idx, w.tickets, out64, out32, host, w.err_flags);
-    else argmax_kernel<bf16_t><<<grid, 256, 0, s>>>((const bf16_t*)logits, vocab, w.val, w.idx, w.tickets, out64, out32, host, w.err_flags);
+    auto go = [&](auto kernel, auto* x) { kernel<<<grid, 256, 0, s>>>(x, vocab, w.val, w.idx, w.tickets, out64, out32, host, w.err_flags); };
+    if (dtype == 0) { if (wide) go(argmax_kernel<float, 4>, (const float*)logits); else go(argmax_kernel<float, 1>, (const float*)logits); }
+    else if (wide) go(argmax_kernel<bf16_t, 8>, (const bf16_t*)logits);
+    else go(argmax_kernel<bf16_t, 1>, (const bf16_t*)logits);
 }
 
 // The same in two stages without tickets, for callers that may overlap (argmax_rows_noalloc): per-block partials, then one block per row; out[r] as si32.

@@ -8,7 +8,7 @@ import pytest
 from parity import FunctionBuilder, Program, assert_close, check_program, hip_run, oracle_run, to_bytes
 from gptrs_amd import functional as F
 from gptrs_amd.backend import HipBackend
-from gptrs_amd.ptir import Tensor, bf16_bits_to_f32, f32_to_bf16_bits
+from gptrs_amd.ptir import Tensor, TensorSpec, bf16_bits_to_f32, f32_to_bf16_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -789,3 +789,21 @@ def test_gathers_left_out_take_no_memory():
     out = be.run_program(p, args)
     assert be.counter("bytes_allocated") - before < 1.5 * rows * inner * 4, "the sum alone"
     del out
+
+
+@pytest.mark.parametrize("dtype", ["F32", "Bf16"])
+@pytest.mark.parametrize("rows,vocab", [(1, 1), (1, 3), (1, 4097), (1, 50257), (1, 131072), (2, 4096), (3, 5003), (8, 32768), (16, 8191), (16, 70000)])
+def test_greedy_tokens_of_every_place(hip, dtype, rows, vocab):
+    """The largest value at the first, a middle and the last place, several equal ones (the first counts), rows without any finite value."""
+    rng = np.random.default_rng(vocab + rows)
+    for at in (0, vocab // 2, vocab - 1, None):
+        x = rng.integers(-40, 40, (rows, vocab)).astype(np.float32)   # whole numbers: exact in bf16, many equal
+        if at is not None:
+            x[:, at] = 64.0
+        x[rows - 1] = -np.inf if at is None else x[rows - 1]
+        want = x.argmax(1)
+        h = hip.materialize(TensorSpec(dtype, (rows, vocab)), to_bytes(x, dtype))
+        if rows == 1:
+            assert hip.sample_decode_token(h) == want[0]
+        else:
+            assert list(hip.sample_decode_rows_wait(hip.sample_decode_rows_begin(h), rows)) == list(want)
