@@ -1754,6 +1754,29 @@ struct Fuser {
         }
     }
 
+    // The last rows of several prompts, sliced out of the stacked rows and put behind one another: the concatenation reads the slices' sources.
+    void pass_concat_slices() {
+        const std::vector<int> uses = count_uses();
+        for (auto& in : fn.body) {
+            if (in.dead || in.op != OpKind::Concat || !in.part_starts.empty()) continue;
+            std::vector<std::vector<int64_t>> starts(in.operands.size()), sizes(in.operands.size());
+            bool any = false;
+            for (size_t i = 0; i < in.operands.size(); ++i) {
+                const int v = in.operands[i].value;
+                const Instr* p = v >= 0 ? producer(v) : nullptr;
+                if (!p || p->op != OpKind::Slice || uses[v] != 1 || p->operands[0].value < 0) continue;
+                starts[i] = p->a;
+                sizes[i] = p->b;
+                in.operands[i].value = p->operands[0].value;
+                any = true;
+            }
+            if (!any) continue;
+            in.part_starts = std::move(starts);
+            in.part_sizes = std::move(sizes);
+            ++fused;
+        }
+    }
+
     void dce() {
         std::vector<bool> live(fn.max_value_id + 1, false);
         for (int r : fn.result_ids) live[r] = true;
@@ -1945,6 +1968,7 @@ int fuse_function(Function& fn) {
     f.pass_scalar_rhs();
     f.dce();
     f.pass_update_views();
+    f.pass_concat_slices();
     f.dce();
     f.toposort();
     return f.fused;

@@ -239,12 +239,14 @@ void Builder::validate(Instr& in) {
             const Spec& x0 = spec_of(in, 0);
             in.axis = norm_axis(in.axis, x0.rank(), "concat");
             int64_t total = 0;
+            // (after fusion an operand may be the tensor that its part is a slice of)
+            auto part = [&](size_t i) -> const std::vector<int64_t>& { return i < in.part_sizes.size() && !in.part_sizes[i].empty() ? in.part_sizes[i] : spec_of(in, i).dims; };
             for (size_t i = 0; i < in.operands.size(); ++i) {
                 const Spec& x = spec_of(in, i);
                 expect(x.dtype == x0.dtype && x.rank() == x0.rank(), "concat dtype/rank mismatch");
                 for (int d = 0; d < x.rank(); ++d)
-                    if (d != in.axis) expect(x.dims[d] == x0.dims[d], "concat shape mismatch off the concat axis");
-                total += x.dims[in.axis];
+                    if (d != in.axis) expect(part(i)[d] == part(0)[d], "concat shape mismatch off the concat axis");
+                total += part(i)[in.axis];
             }
             expect(out.dtype == x0.dtype && out.rank() == x0.rank() && out.dims[in.axis] == total, "concat output shape mismatch");
             break;
@@ -448,10 +450,21 @@ void Builder::describe(Step& st) {
             int64_t along = 0;
             for (size_t i = 0; i < in.operands.size(); ++i) {
                 const Spec& x = spec_of(in, i);
-                st.copies.push_back(make_copy(x.dims, out_strides, row_major_strides(x.dims), along * out_strides[in.axis], 0));
-                along += x.dims[in.axis];
+                const auto xs = row_major_strides(x.dims);
+                const bool part = i < in.part_sizes.size() && !in.part_sizes[i].empty();
+                int64_t off = 0;
+                for (int d = 0; part && d < x.rank(); ++d) off += in.part_starts[i][d] * xs[d];
+                const std::vector<int64_t>& dims = part ? in.part_sizes[i] : x.dims;
+                st.copies.push_back(make_copy(dims, out_strides, xs, along * out_strides[in.axis], off));
+                along += dims[in.axis];
             }
             st.elem_size = widen_copies(st.copies, es_of(out));
+            st.copies_alike = st.copies.size() > 1;
+            for (k::CopyDesc c : st.copies) {
+                c.dst_off = st.copies[0].dst_off;
+                c.src_off = st.copies[0].src_off;
+                st.copies_alike = st.copies_alike && c == st.copies[0];
+            }
             break;
         }
         case OpKind::DynamicSlice: {
@@ -1150,6 +1163,21 @@ void run_step(const Plan& plan, const Step& st, ExecCtx& cx) {
             ++cx.launches;
             break;
         case OpKind::Concat:
+            if (st.copies_alike) {   // parts of one shape: a launch for up to 64 of them
+                k::CopyDesc c = st.copies[0];
+                c.dst_off = c.src_off = 0;
+                for (size_t i0 = 0; i0 < st.copies.size(); i0 += k::CopyPairs::kMost) {
+                    const int n = (int)std::min<size_t>(st.copies.size() - i0, k::CopyPairs::kMost);
+                    k::CopyPairs pairs{};
+                    for (int i = 0; i < n; ++i) {
+                        pairs.dst[i] = (char*)dst + st.copies[i0 + i].dst_off * st.elem_size;
+                        pairs.src[i] = (const char*)src_ptr(st, cx, i0 + i) + st.copies[i0 + i].src_off * st.elem_size;
+                    }
+                    k::copy_strided_pairs(s, pairs, n, st.elem_size, c, nullptr);
+                    ++cx.launches;
+                }
+                break;
+            }
             for (size_t i = 0; i < st.copies.size(); ++i) {
                 k::copy_strided(s, dst, src_ptr(st, cx, i), st.elem_size, st.copies[i], nullptr);
                 ++cx.launches;

@@ -128,6 +128,8 @@ struct Instr {
     // and its element strides and offset inside operand 1; empty when operand 1 is the update itself
     std::vector<int64_t> view_dims, view_strides;
     int64_t view_off = 0;
+    // Concat whose operand i is a Slice of the tensor that it names now: where the part starts there, and its size; empty: the operand is the part
+    std::vector<std::vector<int64_t>> part_starts, part_sizes;
     bool mfma = false;                       // FLinear: prefill GEMM over the k-grouped weight copy
     bool tiled = false;                      // FLinear: decode GEMV over the column-tiled weight copy
     bool norm = false;                       // FLinear: RMSNorm of x fused in (last operand = gamma; eps, scale)

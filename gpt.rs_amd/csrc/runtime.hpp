@@ -106,6 +106,7 @@ struct Step {
     std::vector<int> dst;          // output value ids
     // precomputed launch descriptors
     std::vector<k::CopyDesc> copies;  // strided copies (one per concat operand, etc.)
+    bool copies_alike = false;        // Concat: they differ in their offsets only
     int elem_size = 0;
     k::DotDesc dot{};
     int64_t outer = 0, axis_len = 0, inner = 0;

@@ -46,6 +46,31 @@ def test_equal_updates_behind_one_another(hip, n, donated):
         assert all(np.array_equal(g, w) for g, w in zip(got, want))
 
 
+@pytest.mark.parametrize("dtype,width", [("F32", 8), ("F32", 3), ("Bf16", 4)])
+@pytest.mark.parametrize("n,alike", [(2, True), (3, False), (65, True)])
+def test_slices_put_behind_one_another(hip, dtype, width, n, alike):
+    """The last rows of several sequences: slices of one tensor, of a result, of an input that is updated in place between the slice and the
+    concatenation, of a slice that is read elsewhere too, and a whole tensor.  Parts of one shape are a launch for up to 64 of them."""
+    rows = 3 * n + 2
+
+    def build(fb, x, y, upd, st):
+        z = x + x
+        mine = [y.slice([1, 0], [1, width]), y.slice([3, 0], [1, width])]
+        new = F.dynamic_update_slice_into(y, upd, st)
+        part = lambda t, b: t.slice([3 * b + b % 2, 0], [1 if alike else 1 + b % 2, width])
+        kept = part(x, 0)
+        cat = type(x).concat
+        return [cat(0, [part(z, b) for b in range(n)]), cat(0, mine), new, cat(0, [kept] + [part(x, b) for b in range(1, n)]), kept + kept,
+                cat(1, [x, x.slice([0, 0], [rows, 1])])]
+
+    p = prog(build, [(dtype, [rows, width]), (dtype, [5, width]), (dtype, [2, width]), ("Si32", [2])])
+    args = [rng_uniform(31, [rows, width]), rng_uniform(32, [5, width]), rng_uniform(33, [2, width]), np.array([0, 0], np.int32)]
+    want = oracle_run(p, args)
+    for _ in range(3):
+        got = hip_run(hip, p, args, [False, True, False, False])
+        assert all(np.array_equal(g, w) for g, w in zip(got, want))
+
+
 # ------------------------------------------------------------------ reference-held vectors
 def test_smoke_matmul_golden(hip):
     # crates/gpt-rs-backend-tests/src/smoke.rs:12-24
