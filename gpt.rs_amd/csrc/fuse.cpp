@@ -361,7 +361,7 @@ struct Fuser {
     }
 
     // The f32 rows of an embedding, taken, widened and scaled, and the same rounded to bf16 -> Mix::EmbedRows (table, indices) ->
-    // (rows f32[, rows bf16]).  Only where it saves something besides the widening: a scale or the rounded copy.
+    // (rows f32[, rows bf16]).  f32 tables: only with a scale or the rounded copy, without them it is the gather.
     void pass_embed() {
         for (size_t i = 0; i < fn.body.size(); ++i) {
             const Instr take = fn.body[i];
@@ -397,7 +397,7 @@ struct Fuser {
             int low = -1;
             for (size_t j = 0; j < fn.body.size() && low < 0; ++j)
                 if (!fn.body[j].dead && fn.body[j].op == OpKind::Cast && fn.body[j].operands[0].value == root && fn.body[j].out_specs[0].dtype == DType::BF16) low = (int)j;
-            if (!scaled && low < 0) continue;
+            if (!scaled && low < 0 && take.out_specs[0].dtype == DType::F32) continue;
             Instr ni = make(OpKind::FMixer, "fused.embed_rows", {take.operands[0].value, take.operands[1].value}, root, *spec_of(root));
             ni.mix = Mix::EmbedRows;
             ni.scale = scale;

@@ -121,8 +121,11 @@ void post_norm_add(hipStream_t s, const float* x, const float* y, const float* g
                    float inv_n, float eps);
 void softcap(hipStream_t s, const float* x, float* y, int64_t n, float cap);
 // rows of `table` [vocab, n] by index, as f32 times scale; out16 (may be null): the same rounded to bf16.  Indices as in take().
+// A table of cosines and sines [rows, cos of half | sin of half] of positions[r] * freqs[c], times a magnitude.
+struct RopeTableArgs { const int32_t* positions = nullptr; const float* freqs = nullptr; float magnitude = 0.f; float* out = nullptr; int64_t rows = 0, half = 0; };
+// (with `rope`: that table in the same launch)
 void embed_rows(hipStream_t s, int dtype, const void* table, const int32_t* idx, float* out, void* out16, int64_t n_idx, int64_t vocab, int64_t n,
-                float scale, int* err_flag);
+                float scale, int* err_flag, const RopeTableArgs& rope = RopeTableArgs());
 void softmax_rows(hipStream_t s, int dtype, const void* x, void* y, int64_t rows, int64_t n);
 void gelu(hipStream_t s, int dtype, const void* x, void* y, int64_t n, float half, float inv_div, float one);
 void swiglu(hipStream_t s, int dtype, const void* gate, const void* up, void* y, int64_t n);  // up==nullptr: silu
@@ -424,7 +427,7 @@ void attn_concat(hipStream_t s, const AttnConcatArgs& a);
 // dtype: 0 f32, 2 bf16, of the tensors called "T" below; everything else is f32.
 
 // cos | sin of positions[r] * freqs[i], times `magnitude`: out f32 [rows, 2 * half]
-void rope_table(hipStream_t s, const int32_t* positions, const float* freqs, float magnitude, float* out, int64_t rows, int64_t half);
+void rope_table(hipStream_t s, const RopeTableArgs& a);
 // rotates the pairs (offset + 2i, offset + 2i + 1), i < half, of every head of x T [rows, heads * head_dim]; the rest is copied
 void rope_pairs(hipStream_t s, int dtype, const void* x, const float* table, void* y, int64_t rows, int64_t heads, int64_t head_dim,
                 int64_t offset, int64_t half);

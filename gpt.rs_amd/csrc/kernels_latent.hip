@@ -20,17 +20,7 @@ typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 
 inline int64_t cdiv_l(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// the angle is formed and reduced in f64: at position 10^5 an f32 product is off by 0.004 rad
-__global__ __launch_bounds__(256) void rope_table_kernel(const int32_t* __restrict__ pos, const float* __restrict__ freqs, float mag,
-                                                         float* __restrict__ out, int64_t rows, int64_t half) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * half) return;
-    const int64_t r = i / half, c = i % half;
-    double sn, cs;
-    sincos((double)pos[r] * (double)freqs[c], &sn, &cs);
-    out[r * 2 * half + c] = (float)cs * mag;
-    out[r * 2 * half + half + c] = (float)sn * mag;
-}
+__global__ __launch_bounds__(256) void rope_table_kernel(RopeTableArgs a) { rope_table_entry(a, (int64_t)blockIdx.x * 256 + threadIdx.x); }
 
 template <typename T>
 __global__ __launch_bounds__(256) void rope_pairs_kernel(const T* __restrict__ x, const float* __restrict__ table, T* __restrict__ y, int64_t pairs,
@@ -620,9 +610,9 @@ void with_lds(F kern, size_t bytes) { (void)hipFuncSetAttribute((const void*)ker
 
 }  // namespace
 
-void rope_table(hipStream_t s, const int32_t* positions, const float* freqs, float magnitude, float* out, int64_t rows, int64_t half) {
-    if (rows <= 0 || half <= 0) return;
-    rope_table_kernel<<<(unsigned)cdiv_l(rows * half, 256), 256, 0, s>>>(positions, freqs, magnitude, out, rows, half);
+void rope_table(hipStream_t s, const RopeTableArgs& a) {
+    if (a.rows <= 0 || a.half <= 0) return;
+    rope_table_kernel<<<(unsigned)cdiv_l(a.rows * a.half, 256), 256, 0, s>>>(a);
 }
 void rope_pairs(hipStream_t s, int dtype, const void* x, const float* table, void* y, int64_t rows, int64_t heads, int64_t head_dim, int64_t offset,
                 int64_t half) {

@@ -289,9 +289,37 @@ void run_mixer(const Plan& plan, const Step& st, ExecCtx& cx) {
     auto spec = [&](size_t i) -> const Spec& { return plan.values[st.src[i]].spec; };
     void* dst = cx.ptr[st.dst[0]];
     const int dt = (int)out.dtype;
+    // A step's embedding and its rotation table, whichever comes first, are one launch: neither reads the other.  Up to 16 rows (beyond, a launch is a small
+    // part of either, and the table's f64 arithmetic would take the embedding's registers).
+    auto beside = [&](Mix other) -> const Step* {
+        const Step* nx = &st + 1;
+        if (nx >= plan.steps.data() + plan.steps.size() || nx->in.op != OpKind::FMixer || nx->in.mix != other || nx->left_out || out.dims[0] > 16) return nullptr;
+        for (const Step* one : {&st, nx})   // what both read is there before and after: neither may write over the other's operands
+            for (int v : one->src) {
+                if (v < 0) return nullptr;
+                while (plan.values[v].root != v) v = plan.values[v].root;
+                if (plan.storage[v].kind != Storage::Input && plan.storage[v].kind != Storage::Const) return nullptr;
+            }
+        return nx;
+    };
+    auto table_of = [&](const Step& t) {
+        const Spec& o = t.in.out_specs[0];
+        return k::RopeTableArgs{(const int32_t*)cx.ptr[t.src[0]], (const float*)cx.ptr[t.src[1]], t.in.scale, (float*)cx.ptr[t.dst[0]], o.dims[0], o.dims[1] / 2};
+    };
+    auto embed = [&](const Step& e, const k::RopeTableArgs& rope) {
+        const Spec &o = e.in.out_specs[0], &table = plan.values[e.src[0]].spec;
+        k::embed_rows(s, (int)table.dtype, cx.ptr[e.src[0]], (const int32_t*)cx.ptr[e.src[1]], (float*)cx.ptr[e.dst[0]], e.dst.size() > 1 ? cx.ptr[e.dst[1]] : nullptr, o.dims[0],
+                      table.dims[0], o.dims[1], e.in.scale, cx.err_flag, rope);
+        ++cx.launches;
+    };
     switch (in.mix) {
         case Mix::RopeTable:
-            k::rope_table(s, (const int32_t*)ptr(0), f(1), in.scale, (float*)dst, out.dims[0], out.dims[1] / 2);
+            if (const Step* nx = beside(Mix::EmbedRows)) {
+                embed(*nx, table_of(st));
+                cx.done_ahead = nx;
+                break;
+            }
+            k::rope_table(s, table_of(st));
             ++cx.launches;
             break;
         case Mix::RopePairs:
@@ -496,9 +524,12 @@ void run_mixer(const Plan& plan, const Step& st, ExecCtx& cx) {
             ++cx.launches;
             break;
         case Mix::EmbedRows:
-            k::embed_rows(s, (int)spec(0).dtype, ptr(0), (const int32_t*)ptr(1), (float*)dst, st.dst.size() > 1 ? cx.ptr[st.dst[1]] : nullptr, out.dims[0],
-                          spec(0).dims[0], out.dims[1], in.scale, cx.err_flag);
-            ++cx.launches;
+            if (const Step* nx = beside(Mix::RopeTable)) {
+                embed(st, table_of(*nx));
+                cx.done_ahead = nx;
+                break;
+            }
+            embed(st, k::RopeTableArgs());
             break;
         case Mix::Softcap:
             k::softcap(s, f(0), (float*)dst, out.count(), in.softcap);
