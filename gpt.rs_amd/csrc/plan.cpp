@@ -875,12 +875,15 @@ void Builder::build() {
         int e = s + 1;
         auto copies = [&](const Step& st) { return st.in.op == OpKind::DynamicUpdateSlice && st.copies.size() == 1 && !st.left_out; };
         if (copies(first)) {
-            std::set<int> written(first.dst.begin(), first.dst.end());
+            std::set<int> written;   // roots: a reshape of what one of them writes is the same memory
+            auto writes = [&](const Step& st) { for (int v : st.dst) written.insert(root(v)); };
+            auto reads_it = [&](int v) { return v >= 0 && written.count(root(v)) != 0; };
+            writes(first);
             for (; e < n_steps; ++e) {
                 const Step& st = plan.steps[e];
                 if (!copies(st) || !(st.copies[0] == first.copies[0]) || st.elem_size != first.elem_size || st.src[2] != first.src[2] || st.src_const[2] != first.src_const[2]) break;
-                if (written.count(st.src[0]) || written.count(st.src[1]) || written.count(st.src[2])) break;
-                written.insert(st.dst.begin(), st.dst.end());
+                if (reads_it(st.src[0]) || reads_it(st.src[1]) || reads_it(st.src[2])) break;
+                writes(st);
             }
             plan.steps[s].copy_run = e - s;
         }

@@ -46,6 +46,22 @@ def test_equal_updates_behind_one_another(hip, n, donated):
         assert all(np.array_equal(g, w) for g, w in zip(got, want))
 
 
+def test_an_update_by_a_reshaped_result_waits_for_it(hip):
+    """The second update copies as the first does and takes, reshaped twice, what the first has written in place."""
+    dims = [2, 5, 4]
+
+    def build(fb, st, b0, b1, u0):
+        first = F.dynamic_update_slice_into(b0, u0, st)
+        return [first, F.dynamic_update_slice_into(b1, first.reshape([10, 4]).reshape(dims), st)]
+
+    p = prog(build, [("Si32", [3])] + [("F32", dims)] * 3)
+    args = [np.zeros(3, np.int32)] + [rng_uniform(70 + i, dims) for i in range(3)]
+    want = oracle_run(p, args)
+    for _ in range(3):
+        got = hip_run(hip, p, args, [False, True, True, False])
+        assert all(np.array_equal(g, w) for g, w in zip(got, want))
+
+
 @pytest.mark.parametrize("dtype,width", [("F32", 8), ("F32", 3), ("Bf16", 4)])
 @pytest.mark.parametrize("n,alike", [(2, True), (3, False), (65, True)])
 def test_slices_put_behind_one_another(hip, dtype, width, n, alike):
