@@ -42,8 +42,8 @@ MFMA_PEAK_TFLOPS = 2500.0   # MI355X dense bf16 MFMA
 # rocprofv3 FETCH_SIZE + WRITE_SIZE scaled by a copy kernel of known size (commands and raw figures: `profile`).  The
 # figure belongs to ONE version of the kernel: `source_sha256` is the hash of gpt.rs_amd/csrc/kernels_chain.hip it was
 # measured on, and `roofline.traffic` is null whenever the file in the tree hashes differently.
-CHAIN_TRAFFIC = {"bytes": 7.0127e9 + 0.0230e9, "w8_bytes": 3.5908e9 + 0.0245e9,
-                 "source_sha256": "b6f5ccf9ac05763ee3f562699f6df2338a2460fa1f0e2110e5afa19f937f8903",
+CHAIN_TRAFFIC = {"bytes": 7.0073e9 + 0.0216e9, "w8_bytes": 3.5865e9 + 0.0198e9,
+                 "source_sha256": "bb4f06fa915ba4a69c895f8845e231f16698ece285841fba83738fcdf3cc08ac",
                  "profile": "profiles/chain_kernel_ministral3b_bf16_b1_decode.md"}
 
 
