@@ -925,9 +925,37 @@ void Builder::build() {
         if (st.in.op == OpKind::FAttnDecode) return plan.values[st.src[0]].spec.dtype == DType::F32;
         return step_format(st) == k::kChainW32;
     };
+    // What a launch reads ahead of its barriers, copies ahead of itself or loads as constant (caches, angles, positions, sinks, gains, biases, scales) is older than the
+    // launch: a run ends where a step would take such an operand from a step of the run.  Rows and residuals pass from phase to phase (agent-scope stores and loads).
+    auto passes = [&](const Step& st, size_t i) {
+        if (i == 0) return true;
+        const Instr& in = st.in;
+        if (in.op != OpKind::FLinear) return false;
+        size_t at = linear_extra_pos(in) + (in.has_bias ? 1 : 0) + (in.has_scale ? 1 : 0);
+        if (in.has_residual && i == at++) return true;
+        at += (in.norm ? 1 : 0) + (in.norm && in.norm_ln ? 1 : 0);
+        return in.post && i == at + 1;   // (gain, residual)
+    };
+    // A cache that is not updated in place is copied ahead of the launch, into an output of its own or, behind a run's first step, into workspace that the steps before may still use.
+    auto copies_over_others = [&](const Step& st) {
+        if (st.in.op == OpKind::FLinear) return false;
+        for (size_t o = 1; o < st.dst.size(); ++o)
+            if (plan.storage[st.dst[o]].kind == Storage::Temp) return true;
+        return false;
+    };
     for (int s = 0; s < n_steps;) {
         int np = chain_phases(plan.steps[s]);
         if (!np) { ++s; continue; }
+        std::set<int> written, kept;   // roots: rows, and caches (plain stores: nothing of the launch may read them)
+        auto writes = [&](const Step& st) {
+            for (size_t o = 0; o < st.dst.size(); ++o) (st.in.op != OpKind::FLinear && o > 0 ? kept : written).insert(root(st.dst[o]));
+        };
+        auto reads_ahead = [&](const Step& st) {
+            for (size_t i = 0; i < st.src.size(); ++i)
+                if (st.src[i] >= 0 && (kept.count(root(st.src[i])) || (written.count(root(st.src[i])) && !passes(st, i)))) return true;
+            return false;
+        };
+        writes(plan.steps[s]);
         int e = s + 1;
         bool has_linear = plan.steps[s].in.op == OpKind::FLinear;
         int fmt = has_linear ? step_format(plan.steps[s]) : -1;   // one weight format per launch
@@ -938,6 +966,7 @@ void Builder::build() {
             const int q = chain_phases(nx);
             if (!q || np + q > k::kChainMaxPhases) break;
             if (f32_class(nx) != cls) break;
+            if (reads_ahead(nx) || copies_over_others(nx)) break;
             if (nx.in.op != OpKind::FLinear && att != OpKind::FLinear && att != nx.in.op) break;
             if (nx.in.op == OpKind::FMixer && fmt > k::kChainW16) break;
             if (nx.in.op == OpKind::FLinear && att == OpKind::FMixer && step_format(nx) != k::kChainW16) break;
@@ -948,6 +977,7 @@ void Builder::build() {
                 has_linear = true;
             }
             np += q;
+            writes(nx);
             ++e;
         }
         if (has_linear) {   // an attention on its own keeps its stand-alone kernels
@@ -1044,7 +1074,7 @@ static bool run_chain(const Plan& plan, const Step& head, ExecCtx& cx) {
             void* vout = cx.ptr[st.dst[2]];
             const void* kin = src_ptr(st, cx, 1);
             const void* vin = src_ptr(st, cx, 2);
-            // caches that were not donated are copied ahead of the launch (they are inputs of the run)
+            // caches that are not updated in place are copied ahead of the launch (no step of the run writes them: build)
             if (kout != kin) { GPTRS_HIP_CHECK(hipMemcpyAsync(kout, kin, ck.bytes(), hipMemcpyDeviceToDevice, cx.stream)); ++cx.launches; }
             if (vout != vin) { GPTRS_HIP_CHECK(hipMemcpyAsync(vout, vin, ck.bytes(), hipMemcpyDeviceToDevice, cx.stream)); ++cx.launches; }
             k::ChainPhase pa{}, pc{};

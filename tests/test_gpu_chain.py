@@ -226,6 +226,72 @@ def test_decode_attention_appends_elsewhere_than_it_looks(hip, hq, hkv, dh, cap)
         assert_close(got[0], want[0], atol=3e-2, rtol=2e-2, what=f"context projection, query at {qpos}, row at {upd}")
 
 
+@pytest.mark.parametrize("cap", [16, 2048])
+@pytest.mark.parametrize("between", [False, True])
+def test_a_second_step_on_the_caches_of_the_first(hip, cap, between):
+    """Two steps of attention one behind the other on one pair of caches, each in front of a layer: the second one's cache holds what the first has
+    written, so a launch ends between them."""
+    d, cfg = 128, F.AttentionConfig(embed_dim=128, num_query_heads=4, num_key_value_heads=2, head_dim=64)
+    tp, qp = cfg.total_projection_dim, cfg.query_projection_dim
+    arrays = [rnd(50, (1, d)), rnd(51, (d, tp), 2.0 / np.sqrt(d)), rnd(52, (qp, tp), 4.0 / np.sqrt(qp)), rnd(53, (qp, d), 2.0 / np.sqrt(qp)), rnd(54, (2, cap, 64)), rnd(55, (2, cap, 64))]
+
+    def build(fb, a, w1, w2, w3, k, v, us, qs, us2, qs2):
+        c, k, v = F.attention_decode_cache(cfg, a.matmul(w1), k, v, us, qs)
+        kept = [k, v] if between else []
+        c, k, v = F.attention_decode_cache(cfg, c.matmul(w2), k, v, us2, qs2)
+        return [c.matmul(w3), k, v, *kept]
+
+    specs, ints = [list(a.shape) for a in arrays], [("Si32", [3]), ("Si32", [1])] * 2
+    pb, pf = (prog(build, [(t, s) for s in specs] + ints) for t in ("Bf16", "F32"))
+    at = [np.array([0, 3, 0], np.int32), np.array([3], np.int32), np.array([0, 4, 0], np.int32), np.array([4], np.int32)]
+    before = hip.counter("chain_launches")
+    got = hip_run(hip, pb, arrays + at)
+    assert hip.counter("chain_launches") - before == (2 if between else 3)   # (caches that nobody keeps are copied by a launch of their own steps)
+    want = oracle_run(pf, [bf16_round(a) for a in arrays] + at)
+    for i, (g, w) in enumerate(zip(got, want)):   # (rows of a cache come out of two layers, each rounded once)
+        assert_close(g, w, atol=3e-2, rtol=2e-2, what=f"result {i}")
+
+
+def test_caches_that_nobody_keeps_are_copied_behind_the_steps_before(hip):
+    """A cache that is no result lies in the workspace, here where the rows of the layer in front were: its copy waits for that layer."""
+    d, cfg = 8192, F.AttentionConfig(embed_dim=8192, num_query_heads=1, num_key_value_heads=1, head_dim=64)
+    arrays = [rnd(56, (1, d)), rnd(57, (d, 192), 2.0 / np.sqrt(d)), rnd(58, (64, 40), 0.25), rnd(59, (1, 48, 64)), rnd(60, (1, 48, 64))]
+
+    def build(fb, a, w1, w2, k, v, us, qs):
+        return F.attention_decode_cache(cfg, (a + a).matmul(w1), k, v, us, qs)[0].matmul(w2)
+
+    specs, ints = [list(a.shape) for a in arrays], [("Si32", [3]), ("Si32", [1])]
+    at = [np.array([0, 2, 0], np.int32), np.array([2], np.int32)]
+    got = hip_run(hip, prog(build, [("Bf16", s) for s in specs] + ints), arrays + at)
+    want = oracle_run(prog(build, [("F32", s) for s in specs] + ints), [bf16_round(a) for a in arrays] + at)
+    assert_close(got[0], want[0], atol=3e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("what", ["bias", "gain", "cache"])
+def test_a_layer_whose_vector_a_step_before_has_written(hip, what):
+    """Biases and gains are loaded as constants of the launch, and a cache's rows are stored as such: a layer that takes one of them from a step of the run
+    begins another launch."""
+    n, cap = 256, 4
+    cfg = F.AttentionConfig(embed_dim=n, num_query_heads=1, num_key_value_heads=1, head_dim=64)
+    arrays = [rnd(61, (1, n)), rnd(62, (n, n), 2.0 / np.sqrt(n)), rnd(63, (n, n), 2.0 / np.sqrt(n)), rnd(64, (n, 192), 2.0 / np.sqrt(n)), rnd(65, (1, cap, 64)), rnd(66, (1, cap, 64))]
+
+    def build(fb, a, w1, w2, w3, k, v, us, qs):
+        if what == "cache":
+            c, k, v = F.attention_decode_cache(cfg, a.matmul(w3), k, v, us, qs)
+            return [v.reshape([1, n]).matmul(w1), c, k, v]
+        vec = a.matmul(w1).reshape([n])
+        return [F.linear(a, w2, vec) if what == "bias" else F.rms_norm(a, vec, 1e-5)[0].matmul(w2), vec]
+
+    specs, ints = [list(a.shape) for a in arrays], [("Si32", [3]), ("Si32", [1])]
+    at = [np.array([0, 3, 0], np.int32), np.array([3], np.int32)]
+    before = hip.counter("chain_launches")
+    got = hip_run(hip, prog(build, [("Bf16", s) for s in specs] + ints), arrays + at)
+    assert hip.counter("chain_launches") - before == 2
+    want = oracle_run(prog(build, [("F32", s) for s in specs] + ints), [bf16_round(a) for a in arrays] + at)
+    for i, (g, w) in enumerate(zip(got, want)):
+        assert_close(g, w, atol=3e-2, rtol=2e-2, what=f"result {i}")
+
+
 def test_grid_barrier_gives_up_and_the_backend_goes_on(hip):
     """A grid barrier that cannot complete must end in an execution error, not in a hang: the host option
     "chain_stall_phase" makes every workgroup of the next launch expect one arrival more than the grid can deliver at that

@@ -368,6 +368,30 @@ def test_decode_inside_a_chain(hip, shape, taken, pos, cap, chunk):
             check(g, c, TOL["Bf16"], (shape, pos, opts, "cache"))
 
 
+@pytest.mark.parametrize("kept", [False, True])
+@pytest.mark.parametrize("cap,rot", [(5, 0), (300, 0), (300, 16)])
+def test_a_second_step_on_the_caches_of_the_first(hip, cap, rot, kept):
+    """Two steps on one pair of caches, each in front of a layer: the second one sees and returns the first one's row."""
+    H, G, D = 4, 2, 64
+    q, k = rn(3, 2, H, D).astype(np.float64), 0.5 * rn(4, 2, G, D).astype(np.float64)
+    args = [(projection(1, np.array([p]), H, G, D, D, rot, 30.0, q[i:i + 1], k[i:i + 1]), "F32") for i, p in enumerate((3, 4))] + [(rn(2, H), "F32")]
+    args += [(np.array([p], np.int32), "Si32") for p in (3, 4)] + [(np.array([0, p, 0], np.int32), "Si32") for p in (3, 4)]
+    args += [(F.pair_frequencies(rot, 30.0) if rot else np.zeros(1, np.float32), "F32"), (0.3 * rn(60, G, cap, D), "Bf16"), (rn(80, G, cap, D), "Bf16"),
+             (rn(5, H * D, 96) * (H * D) ** -0.5, "Bf16")]
+    mixer = emit_mixer("Bf16", [1], H, G, D, D, rot, 0, 9.0 / D, True)
+
+    def emit(fb, p1, p2, sink, pos1, pos2, at1, at2, freqs, kc, vc, w):
+        c1, k1, v1 = mixer(fb, p1, sink, pos1, at1, freqs, kc, vc)
+        c2, k2, v2 = mixer(fb, p2, sink, pos2, at2, freqs, k1, v1)
+        return [c1.matmul(w), c2.matmul(w), k2, v2] + ([k1, v1] if kept else [])
+
+    before = hip.counter("chain_launches")
+    got, want = both(hip, emit, args)
+    assert hip.counter("chain_launches") > before
+    for g, w, tol in zip(got, want, [3e-2] * 2 + [TOL["Bf16"]] * 4):
+        check(g, w, tol, (cap, rot, kept))
+
+
 # ------------------------------------------------------------------------------------------ whole models
 def load(hip, tmp_path, name, dt, seed=0, **kw):
     cfg = U.STACKS[name]
