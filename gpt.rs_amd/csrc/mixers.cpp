@@ -300,6 +300,11 @@ void run_mixer(const Plan& plan, const Step& st, ExecCtx& cx) {
                 while (plan.values[v].root != v) v = plan.values[v].root;
                 if (plan.storage[v].kind != Storage::Input && plan.storage[v].kind != Storage::Const) return nullptr;
             }
+        for (int a : st.dst)   // rows that nobody reads give their memory back at once, and the other step's output may lie there
+            for (int b : nx->dst) {
+                const RootStorage &x = plan.storage[a], &y = plan.storage[b];
+                if (x.kind == Storage::Temp && y.kind == Storage::Temp && x.offset < y.offset + y.bytes && y.offset < x.offset + x.bytes) return nullptr;
+            }
         return nx;
     };
     auto table_of = [&](const Step& t) {

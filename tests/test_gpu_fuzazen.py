@@ -80,6 +80,23 @@ def test_head_norm(hip, dt, out, rows, heads, hd):
     check(got[0], want[0], TOL[out])
 
 
+@pytest.mark.parametrize("table_first", [False, True])
+@pytest.mark.parametrize("rows", [1, 16, 17])
+def test_embedding_read_in_bf16_only_beside_a_rotation_table(hip, rows, table_first):
+    """Nobody reads the embedding's f32 rows: their memory is free again behind their step, and the rotation table may lie there.  Up to 16 rows the two steps
+    are one launch where their outputs lie apart."""
+    pos, ids = np.arange(rows, dtype=np.int32) * 700, (np.arange(rows, dtype=np.int32) * 13) % 40
+
+    def emit(fb, table, i, p, f):
+        angles = F.rope_table(p, f) if table_first else None
+        x = table.take(i).cast("F32")
+        x = (x * fb.scalar_broadcast(1.5, list(x.dims), "F32")).cast("Bf16")
+        return F.rope_pairs(x, angles if table_first else F.rope_table(p, f), 16, 0)
+
+    got, want = both(hip, emit, [(rn(1, 40, 1024), "Bf16"), (ids, "Si32"), (pos, "Si32"), (F.pair_frequencies(64, 100.0), "F32")])
+    check(got[0], want[0], TOL["Bf16"])
+
+
 @pytest.mark.parametrize("dt", ["F32", "Bf16"])
 @pytest.mark.parametrize("rows,heads,vd", [(1, 1, 1), (7, 3, 5), (40, 8, 64)])
 def test_head_gate(hip, dt, rows, heads, vd):
