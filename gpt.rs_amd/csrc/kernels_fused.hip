@@ -386,7 +386,7 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const T* __restrict__ t
 }
 void embed_rows(hipStream_t s, int dtype, const void* table, const int32_t* idx, float* out, void* out16, int64_t n_idx, int64_t vocab, int64_t n,
                 float scale, int* err_flag, const RopeTableArgs& rope) {
-    if (n_idx <= 0 || n <= 0) return;
+    if (n_idx <= 0 || n <= 0) return rope_table(s, rope);
     const bool with_rope = rope.rows > 0 && rope.half > 0;
     const unsigned grid = (unsigned)(n_idx + (with_rope ? cdiv(rope.rows * rope.half, 256) : 0));
     auto go = [&](auto kernel, auto* t) { kernel<<<grid, 256, 0, s>>>(t, idx, out, (bf16_t*)out16, vocab, n, scale, err_flag, (int)n_idx, rope); };

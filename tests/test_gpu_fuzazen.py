@@ -97,6 +97,16 @@ def test_embedding_read_in_bf16_only_beside_a_rotation_table(hip, rows, table_fi
     check(got[0], want[0], TOL["Bf16"])
 
 
+def test_embedding_of_nothing_beside_a_rotation_table(hip):
+    """No rows are embedded: the table beside them is formed all the same."""
+    def emit(fb, table, i, p, f):
+        return [table.take(i).cast("F32"), F.rope_table(p, f)]
+
+    got, want = both(hip, emit, [(rn(1, 40, 64), "Bf16"), (np.zeros(0, np.int32), "Si32"), (np.array([3, 70, 9], np.int32), "Si32"), (F.pair_frequencies(8, 100.0), "F32")])
+    assert got[0].shape == (0, 64)
+    check(got[1], want[1], TOL["F32"])
+
+
 @pytest.mark.parametrize("dt", ["F32", "Bf16"])
 @pytest.mark.parametrize("rows,heads,vd", [(1, 1, 1), (7, 3, 5), (40, 8, 64)])
 def test_head_gate(hip, dt, rows, heads, vd):
