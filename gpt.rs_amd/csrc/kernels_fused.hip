@@ -360,16 +360,16 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const T* __restrict__ t
     const bool ok = id >= 0 && (int64_t)id < vocab;
     if (!ok && threadIdx.x == 0) atomicExch(err_flag, 1);
     const T* src = table + (int64_t)(ok ? id : 0) * n;
-    const float f = ok ? scale : 0.f;
     if (sizeof(T) == 2 && n % 8 == 0) {   // (rows of a tensor: 16-byte aligned)
         for (int64_t i = (int64_t)threadIdx.x * 8; i < n; i += 2048) {
-            const fused_u32x4_t w = *reinterpret_cast<const fused_u32x4_t*>(src + i);
+            fused_u32x4_t w = {0, 0, 0, 0};
+            if (ok) w = *reinterpret_cast<const fused_u32x4_t*>(src + i);
             fused_u32x4_t o;
             float v[8];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[2 * e] = bf16lo(w[e]) * f;
-                v[2 * e + 1] = bf16hi(w[e]) * f;
+                v[2 * e] = bf16lo(w[e]) * scale;
+                v[2 * e + 1] = bf16hi(w[e]) * scale;
                 o[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
             }
             *reinterpret_cast<float4*>(out + r * n + i) = make_float4(v[0], v[1], v[2], v[3]);
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const T* __restrict__ t
         return;
     }
     for (int64_t i = threadIdx.x; i < n; i += 256) {
-        const float v = Elem<T>::ld(src, i) * f;
+        const float v = ok ? Elem<T>::ld(src, i) * scale : 0.f;
         out[r * n + i] = v;
         if (out16) out16[r * n + i] = f32_to_bf16(v);
     }

@@ -9,6 +9,7 @@ import fuzazen_util as U
 import __graft_entry__ as entry
 from oracle.fuzazen_reference import Reference
 from gptrs_amd import functional as F, loader, models, trace
+from gptrs_amd.backend import BackendError
 from gptrs_amd.ptir import FunctionBuilder, Program, TensorSpec, f32_to_bf16_bits
 
 pytestmark = pytest.mark.gpu
@@ -105,6 +106,18 @@ def test_embedding_of_nothing_beside_a_rotation_table(hip):
     got, want = both(hip, emit, [(rn(1, 40, 64), "Bf16"), (np.zeros(0, np.int32), "Si32"), (np.array([3, 70, 9], np.int32), "Si32"), (F.pair_frequencies(8, 100.0), "F32")])
     assert got[0].shape == (0, 64)
     check(got[1], want[1], TOL["F32"])
+
+
+@pytest.mark.parametrize("width", [64, 20])
+@pytest.mark.parametrize("vocab", [0, 1])
+def test_embedding_outside_its_table(hip, vocab, width):
+    """An index outside the table is an error, and no row of the table is read for it: a table may have none."""
+    prog = build(lambda fb, table, i: table.take(i).cast("F32"), [(rn(1, vocab, width), "Bf16"), (np.array([1, -1], np.int32), "Si32")])
+    with pytest.raises(BackendError):
+        on_device(hip, prog, [(rn(1, vocab, width), "Bf16"), (np.array([1, -1], np.int32), "Si32")])
+    again = [(rn(2, 3, width), "Bf16"), (np.array([2, 0], np.int32), "Si32")]   # the backend goes on
+    got, want = both(hip, lambda fb, table, i: table.take(i).cast("F32"), again)
+    check(got[0], want[0], TOL["F32"])
 
 
 @pytest.mark.parametrize("dt", ["F32", "Bf16"])
