@@ -1384,10 +1384,12 @@ static int attn_prefill_mfma(hipStream_t s, const AttnPrefillArgs& a) {
     if (a.rot_half) { kv.cos = (const T*)a.cos; kv.sin = (const T*)a.sin; }
     // four key groups (bf16) while the launch is one workgroup to a CU at most and rows see more than two tiles.  us, four and two groups (one, under 128
     // rows), 32 / 8 heads of 128: 100 rows 11.3 and 13.5, 128 11.2 and 13.8, 200 11.7 and 14.2, 333 13.6 and 17.1, 512 (256 workgroups) 16.9 and 21.6, 2 x 256
-    // 13.7 and 17.1; beyond: 2 x 333 23.5 and 19.0, 1000 37 and 35; 64 rows 12 and 11
+    // 13.7 and 17.1; beyond: 2 x 333 23.5 and 19.0, 1000 37 and 35; 64 rows 12 and 11.  Not where one group's launch is one row tile that fills the caches itself (a query
+    // head to a key head, under 128 rows), which saves a launch: us with the rows into the caches, four groups and one, 12 heads of 64: 65 rows 8.0 and 6.6, 100 8.1 and 7.6, 127
+    // 8.4 and 7.8; 16 heads of 128: 10.1 and 9.0, 10.7 and 10.5, 11.4 and 11.6; 4 heads of 32: 7.1 and 5.6, 7.2 and 6.4; 32 heads of 128: 10.7 and 9.9, 10.9 and 11.5
     static const bool allow_kg = [] { const char* e = getenv("GPTRS_HIP_ATTN_KEYGROUPS"); return !(e && e[0] == '0'); }();
     const int64_t g = a.n_q / a.n_kv;
-    const bool kg4 = std::is_same<T, bf16_t>::value && allow_kg && a.t > 64 && cdiv(cdiv(a.t, 32), g == 1 ? 2 : 1) * a.n_kv * (g == 1 ? 1 : g / 2) * a.batch <= 256;
+    const bool kg4 = std::is_same<T, bf16_t>::value && allow_kg && a.t > 64 && !(a.starts && g == 1 && a.t < 128) && cdiv(cdiv(a.t, 32), g == 1 ? 2 : 1) * a.n_kv * (g == 1 ? 1 : g / 2) * a.batch <= 256;
     const int64_t hw = kg4 ? 2 : 4, gw = std::min(g, hw), zg = g / gw;   // waves of a key group; query heads of a workgroup, workgroups of a key head
     const dim3 grid((unsigned)cdiv(cdiv(a.t, 32), hw / gw), (unsigned)a.n_kv, (unsigned)(zg * a.batch));
     const float sl = a.scale * 1.44269504088896f;

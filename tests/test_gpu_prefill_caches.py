@@ -152,6 +152,20 @@ def test_f32_of_few_rows(hip, case):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("case,launches", [((1, 65, 4, 4, 64, True, 70, 0), 1), ((2, 100, 2, 2, 128, False, 100, 0), 1), ((1, 127, 12, 12, 32, True, 128, 1), 1),
+                                           ((1, 128, 4, 4, 64, True, 130, 0), 2), ((1, 65, 4, 2, 64, True, 70, 0), 2), ((1, 64, 4, 2, 64, True, 70, 0), 1)])
+def test_one_row_tile_fills_the_caches_itself(hip, case, launches):
+    """Where a workgroup sees every row of its key head the caches are filled on the way: no launch for them, and no key groups, of which each sees a part."""
+    B, T, hq, hkv, dh, rot, cap, first = case
+    p, args = program("Bf16", B, T, hq, hkv, dh, rot, cap), inputs(B, T, hq, hkv, dh, rot, cap, first, 12)
+    got = hip_run(hip, p, args, [False] * (len(args) - 2 * B) + [True] * 2 * B)
+    assert hip.counter("last_program_launches") == launches
+    want = oracle_run(program("F32", B, T, hq, hkv, dh, rot, cap), [a if a.dtype == np.int32 else bf16_bits_to_f32(f32_to_bf16_bits(a)).reshape(a.shape) for a in args])
+    for i, (g, w) in enumerate(zip(got, want)):   # rotated rows and the attention's output are rounded once or twice
+        assert_close(g, w, atol=2e-2, rtol=2e-2, what=f"{case} result {i}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("donate", [False, True])
 @pytest.mark.parametrize("case", CASES[:-1])
 def test_bf16(hip, case, donate):
