@@ -16,6 +16,7 @@ from __future__ import annotations
 import copy
 import itertools
 import os
+import threading
 from array import array
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -694,6 +695,7 @@ class Ministral(_ModelBase):
         self.attn = config.attention_config()
         self.rope = F.RopeConfig(config.rotary_dim, config.rope_theta, config.rope_scaling)
         self._rope_table: Dict[str, object] = {}
+        self._rope_lock = threading.Lock()
         if residual_dtype is not None and residual_dtype not in ("F32",):
             raise ValueError("residual_dtype must be None or 'F32'")
         self.residual_dtype = residual_dtype if (residual_dtype and residual_dtype != dtype) else None
@@ -925,21 +927,29 @@ class Ministral(_ModelBase):
         return prog, layout
 
     def _rope_rows(self, start: int, end: int):
-        """Bytes of the cosines and sines of positions start .. end - 1.  The rows of positions seen so far are kept with the model, to a power of
-        two (they are constants of its rotation; 333 rows anew 0.13 ms in front of the first launch)."""
-        if start < 0:
-            return tuple(_np_to_bytes(x, self.dtype) for x in F.rotary_cos_sin_cache_slice(start, end - start, self.rope))
-        table = self._rope_table
-        if table.get("rope") != self.rope:
-            table = {"rope": copy.deepcopy(self.rope), "rows": 0, "cos": b"", "sin": b""}
-        have = table["rows"]
-        if have < end:
-            rows = max(decode_cache_capacity(end, self.config.context_length), end)
-            cos, sin = F.rotary_cos_sin_cache_slice(have, rows - have, self.rope)
-            table = {"rope": table["rope"], "rows": rows, "cos": table["cos"] + _np_to_bytes(cos, self.dtype), "sin": table["sin"] + _np_to_bytes(sin, self.dtype)}
-            self._rope_table = table
-        row = len(table["cos"]) // table["rows"]
-        return table["cos"][start * row:end * row], table["sin"][start * row:end * row]
+        """Bytes of the cosines and sines of positions start .. end - 1.  The rows from position 0 on that calls have asked for are kept with the model (they
+        are constants of its rotation; 333 rows 0.14 ms in front of the first launch, 5 us when kept); no call forms rows that a call by itself would not,
+        but for a step at the end of the kept rows, which forms those of the steps behind it (64: 0.05 ms, one 0.03)."""
+        def rows(a, b):
+            return tuple(_np_to_bytes(x, self.dtype) for x in F.rotary_cos_sin_cache_slice(a, b - a, self.rope))
+
+        with self._rope_lock:
+            table = self._rope_table
+            if table.get("rope") != self.rope:
+                table.update(rope=copy.deepcopy(self.rope), rows=0, cos=bytearray(), sin=bytearray())
+            have = table["rows"]
+            if start < 0 or start > have or end <= start:   # behind a gap
+                return rows(start, end)
+            if end > have:
+                upto = end if end - start > 1 else max(end, min(end + 63, self.config.context_length))
+                new = rows(have, upto)
+                table["cos"] += new[0]
+                table["sin"] += new[1]
+                table["rows"] = upto
+                if start == have and upto == end:
+                    return new
+            row = len(table["cos"]) // table["rows"]
+            return tuple(bytes(memoryview(table[k])[start * row:end * row]) for k in ("cos", "sin"))
 
     def forward_with_decode_cache(self, tokens, position_offset, caches, fixed_capacity=None, last_logits_only=False):
         """model/ministral.rs:613-766.  last_logits_only: see Gpt.forward_with_decode_cache."""

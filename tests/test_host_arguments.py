@@ -36,6 +36,28 @@ def test_rotation_rows_are_those_of_their_positions(dtype, scaling):
     assert m._rope_rows(3, 9) == rows(3, 9)
 
 
+def test_rotation_rows_formed_by_a_call_are_those_it_asks_for(monkeypatch):
+    """A prompt forms its own rows and no more, a step at the end of the kept rows those of the next steps too, and rows behind a gap (caches of an earlier
+    program, say) are formed alone: position 100000 does not bring 100000 rows with it."""
+    cfg = models.MinistralConfig(vocab_size=32, context_length=1 << 18, embed_dim=32, num_layers=1, num_heads=4, num_kv_heads=2, head_dim=8, ffn_dim=32, rotary_dim=8)
+    m = models.Ministral(cfg, OracleBackend(), "Bf16")
+    formed = []
+
+    def slice_(start, length, rope, plain=F.rotary_cos_sin_cache_slice):
+        formed.append((start, length))
+        return plain(start, length, rope)
+
+    def rows(start, end, plain=F.rotary_cos_sin_cache_slice):
+        return tuple(models._np_to_bytes(x, "Bf16") for x in plain(start, end - start, m.rope))
+
+    monkeypatch.setattr(F, "rotary_cos_sin_cache_slice", slice_)
+    for (start, end), new in (((100000, 100001), [(100000, 1)]), ((0, 333), [(0, 333)]), ((0, 200), []), ((0, 700), [(333, 367)]), ((700, 701), [(700, 64)]), ((701, 702), []),
+                              ((763, 764), []), ((764, 765), [(764, 64)]), ((5000, 5001), [(5000, 1)])):
+        formed.clear()
+        assert m._rope_rows(start, end) == rows(start, end)
+        assert formed == new, (start, end)
+
+
 def test_runs_behind_the_first_see_new_arguments_and_new_parameters():
     cfg = models.GptConfig(vocab_size=24, context_length=16, embed_dim=16, num_layers=1, num_heads=2, mlp_ratio=2)
     be = OracleBackend()
