@@ -36,7 +36,8 @@ def decode_cache_capacity(required_len: int, max_len: int) -> int:
     return min(bucket, max_len)
 
 
-GROW_SLOTS = 32   # layers' caches that one program copies into larger ones
+GROW_SLOTS = 32        # layers' caches that one program copies into larger ones, at most
+GROW_BYTES = 1 << 28   # ... and bytes of the larger ones, beyond one layer's: old and new caches are there together while it runs
 
 
 @dataclass
@@ -648,8 +649,10 @@ class Gpt(_ModelBase):
         """model/gpt.rs:626-657: copy each layer's cache into a larger zero buffer."""
         dims = (self.attn.num_key_value_heads, caches[0][0].capacity, self.attn.kv_head_dim)
         slots = [(c, i) for c in caches for i in range(len(c))]
-        for lo in range(0, len(slots), GROW_SLOTS):      # what a program has copied is dropped before the next is run
-            part = slots[lo:lo + GROW_SLOTS]
+        pair = 2 * dims[0] * capacity * dims[2] * (2 if self.dtype == "Bf16" else 4)
+        most = max(1, min(GROW_SLOTS, GROW_BYTES // max(pair, 1)))
+        for lo in range(0, len(slots), most):      # what a program has copied is dropped before the next is run
+            part = slots[lo:lo + most]
             grown = iter(self._grow_many([h for c, i in part for h in (c[i].keys, c[i].values)], dims, capacity))
             for c, i in part:
                 c[i] = DecodeKvCache(next(grown), next(grown), c[i].len, capacity)

@@ -75,3 +75,25 @@ def test_runs_behind_the_first_see_new_arguments_and_new_parameters():
     fresh = models.Gpt.random(cfg, OracleBackend(), seed=3)
     fresh.set_param("lm_head", head)
     np.testing.assert_array_equal(logits([1, 2, 3]), fresh.backend.to_numpy(fresh.forward_with_decode_cache([1, 2, 3], 0, [None])))
+
+
+@pytest.mark.parametrize("layers,budget,runs", [(3, 1 << 28, [6]), (5, 2 * 2 * 2 * 32 * 8 * 4, [4, 4, 2]), (3, 1, [2, 2, 2]), (40, 1 << 28, [64, 16])])
+def test_growing_caches_hold_little_beside_them(monkeypatch, layers, budget, runs):
+    """Caches grow a program at a time, and a program holds no more new bytes than it is allowed, or one layer's."""
+    cfg = models.GptConfig(vocab_size=24, context_length=64, embed_dim=16, num_layers=layers, num_heads=2, mlp_ratio=2)
+    be = OracleBackend()
+    m = models.Gpt.random(cfg, be, seed=3)
+    caches = [None] * layers
+    m.forward_with_decode_cache([1, 2, 3], 0, caches)
+    before = [be.to_numpy(h) for s in caches for h in (s.keys, s.values)]
+    monkeypatch.setattr(models, "GROW_BYTES", budget)
+    grown, plain = [], m._grow_many
+    monkeypatch.setattr(m, "_grow_many", lambda handles, *a: grown.append(len(handles)) or plain(handles, *a))
+    rows = [caches]
+    m._grow_caches(rows, 32)
+    assert grown == runs
+    for s, h, old in zip([s for s in caches for _ in (0, 1)], [h for s in caches for h in (s.keys, s.values)], before):
+        new = be.to_numpy(h)
+        assert s.capacity == 32 and new.shape[1] == 32
+        np.testing.assert_array_equal(new[:, :old.shape[1]], old)
+        assert not new[:, old.shape[1]:].any()
