@@ -1927,6 +1927,8 @@ class Generator:
         # the loop only ever samples from the last row: prefill runs the head on that row alone (`self.logits` is then
         # [1, V] after a prefill as after a decode step); False keeps every row as the reference's forward does
         self.last_logits_only = bool(last_logits_only)
+        # (any other seed is looked at before the prompt is read, and may be refused)
+        self._rng = None if type(seed) is int and seed >= 0 else np.random.default_rng(seed)
         can_pipeline = device_sampling and hasattr(model.backend, "sample_decode_token_begin") and \
             hasattr(model, "forward_decode_device_token")
         if pipelined and not can_pipeline:
@@ -1937,7 +1939,8 @@ class Generator:
         context = self.tokens[self.window_start:]
         self.logits = self._prefill(context)
         self.processed_len = len(context)
-        self._rng = np.random.default_rng(seed)   # (while the device reads the prompt)
+        if self._rng is None:   # (while the device reads the prompt)
+            self._rng = np.random.default_rng(seed)
 
     def _sample(self) -> int:
         be = self.model.backend

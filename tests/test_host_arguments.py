@@ -97,3 +97,17 @@ def test_growing_caches_hold_little_beside_them(monkeypatch, layers, budget, run
         assert s.capacity == 32 and new.shape[1] == 32
         np.testing.assert_array_equal(new[:, :old.shape[1]], old)
         assert not new[:, old.shape[1]:].any()
+
+
+def test_a_seed_that_is_none_is_refused_before_the_prompt_is_read():
+    cfg = models.GptConfig(vocab_size=24, context_length=16, embed_dim=16, num_layers=1, num_heads=2, mlp_ratio=2)
+    m = models.Gpt.random(cfg, OracleBackend(), seed=3)
+    read = []
+    forward, m.forward_with_decode_cache = m.forward_with_decode_cache, lambda *a, **k: read.append(a) or forward(*a, **k)
+    for seed, error in ((-1, ValueError), ("seven", TypeError), (1.5, TypeError)):
+        with pytest.raises(error):
+            models.Generator(m, [1, 2, 3], seed=seed)
+        assert not read
+    for seed in (0, 7, np.int64(7), [1, 2], np.random.SeedSequence(5)):
+        gen = models.Generator(m, [1, 2, 3], seed=seed)
+        assert gen._rng.random() == np.random.default_rng(seed if not isinstance(seed, np.random.SeedSequence) else np.random.SeedSequence(5)).random()
